@@ -356,6 +356,18 @@ int niti_relu_i8_bwd(const int8_t* act, const int8_t* dy, int8_t* dx, int64_t n,
 int niti_quantize_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* absmax_bits,
                          int32_t* exp_out, void* stream);
 
+/* The same quantiser without a zeroed word in front of it: parts is scratch of at least 256 words with any contents.  Also
+   copies `targets` class indices (int64) from target_in to target_out, for callers whose step reads them from a buffer of
+   its own (0: none). */
+int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
+                               int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, void* stream);
+
+/* Display metrics of a step (main.py:156-163, meters.py:56-70) in one launch: sums[0..2] (double) += n x { mean cross entropy of
+   softmax(out_val 2^out_exp), top-1 %, top-5 % }.  out_val: [n,classes] int8, target: int64 [n], classes >= 5.  Ties count as
+   torch.topk orders them. */
+int niti_batch_metrics_i8(const int8_t* out_val, const int32_t* out_exp, const int64_t* target, int n, int classes, double* sums,
+                          void* stream);
+
 /* TiDropout (ti_torch.py:439-455): y[m][f] = x[m][f] * mask[f] with one keep (1) / drop (0) byte per feature, and - when
    exp_out is given - exp_out = exp_in + exp_add (the layer raises the exponent by one; exp_in NULL counts as 0), as one
    launch.  The backward pass is the same product on the error (exp_out NULL).  features % 16 == 0, 16-byte aligned. */

@@ -138,12 +138,66 @@ __global__ __launch_bounds__(256) void absmax_f32_kernel(const float* __restrict
   if (threadIdx.x < 64) fold_absmax(out, threadIdx.x < 4 ? wmax[threadIdx.x] : 0u);
 }
 
+// Largest |x| per workgroup, stored (not folded into a zeroed word: no fill in front, no atomics on one address - with a
+// thousand workgroups folding into one word the pass took 9.5 us for 1.5 MB and 18.5 us for 3 MB, memory-bound it is
+// about 2).  Also copies the batch's class indices where the caller keeps them in a buffer of its own.
+constexpr int kQuantParts = 256;   // partial maxima: one per thread of the workgroups that read them
+__global__ __launch_bounds__(256) void absmax_parts_f32_kernel(const float* __restrict__ x, int64_t n, uint32_t* __restrict__ parts,
+                                                               const int64_t* __restrict__ t_in, int64_t* __restrict__ t_out, int nt) {
+  __shared__ uint32_t wmax[4];
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  for (int64_t i = t0; i < nt; i += stride) t_out[i] = t_in[i];
+  uint32_t m = 0;
+  const int64_t nv = aligned16_dev(x) ? n >> 2 : 0;
+  for (int64_t i = t0; i < nv; i += stride) {
+    const v4i v = reinterpret_cast<const v4i*>(x)[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t b = static_cast<uint32_t>(v[e]) & 0x7FFFFFFFu;
+      m = b > m ? b : m;
+    }
+  }
+  for (int64_t i = (nv << 2) + t0; i < n; i += stride) {
+    const uint32_t b = __float_as_uint(x[i]) & 0x7FFFFFFFu;
+    m = b > m ? b : m;
+  }
+  m = wave_max_u32(m);
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t g = wmax[0];
+    for (int i = 1; i < 4; ++i) g = wmax[i] > g ? wmax[i] : g;
+    parts[blockIdx.x] = g;
+  }
+}
+
 // bw = ceil(log2 r); y = int8(clamp(round_half_even(x * 2^(bits - bw)), -128, 127)), float NCHW -> int8 NHWC with the
 // channels zero-padded to cpad; exp_out = bw - bits.  The product and the rounding are the reference's float32 operations.
+// r = the largest of nparts partial maxima (one word: the caller's absmax_bits); nparts == 0 (a batch of a few images):
+// every workgroup takes the maximum over the whole batch itself, which saves the launch in front of this one.
 __global__ __launch_bounds__(256) void quantize_f32_i8_kernel(const float* __restrict__ x, int8_t* __restrict__ y, int64_t pixels,
-                                                              int C, int HW, int cpad, const uint32_t* __restrict__ absmax_bits,
-                                                              int32_t* exp_out, int bits) {
-  const float r = __uint_as_float(*absmax_bits);
+                                                              int C, int HW, int cpad, const uint32_t* __restrict__ parts, int nparts,
+                                                              int32_t* exp_out, int bits, const int64_t* __restrict__ t_in,
+                                                              int64_t* __restrict__ t_out, int nt) {
+  __shared__ uint32_t wmax[4];
+  uint32_t m = 0;
+  if (nparts > 0) {
+    if (static_cast<int>(threadIdx.x) < nparts) m = parts[threadIdx.x];
+  } else {
+    for (int64_t i = threadIdx.x; i < pixels * C; i += 256) {
+      const uint32_t b = __float_as_uint(x[i]) & 0x7FFFFFFFu;
+      m = b > m ? b : m;
+    }
+    if (blockIdx.x == 0)
+      for (int i = threadIdx.x; i < nt; i += 256) t_out[i] = t_in[i];
+  }
+  m = wave_max_u32(m);
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = wmax[i] > m ? wmax[i] : m;
+  const float r = __uint_as_float(m);
   // ceil(log2 r) from the exponent and mantissa of r = m 2^e, 0.5 <= m < 1 (exact; a library log2f rounds k + log2(1 + d)
   // back to k for the first float32 values above 2^k, k >= 4, and differs between platforms there)
   int fe = 0;
@@ -151,24 +205,35 @@ __global__ __launch_bounds__(256) void quantize_f32_i8_kernel(const float* __res
   const int bw = fm == 0.5f ? fe - 1 : fe;
   const float scale = ldexpf(1.0f, bits - bw);
   if (blockIdx.x == 0 && threadIdx.x == 0 && exp_out != nullptr) *exp_out = r > 0.0f ? bw - bits : 0;
+  auto quad = [&](const float* src, int c0) {   // four channels of a pixel as one word
+    uint32_t word = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int c = c0 + e;
+      int q = 0;
+      if (c < C && r > 0.0f) {
+        const float v = fminf(fmaxf(rintf(src[static_cast<int64_t>(c) * HW] * scale), -128.0f), 127.0f);
+        q = static_cast<int>(v);
+      }
+      word |= (static_cast<uint32_t>(q) & 0xFFu) << (8 * e);
+    }
+    return word;
+  };
+  const bool wide = cpad % 16 == 0 && aligned16_dev(y);
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < pixels; p += stride) {
     const int64_t n = p / HW, hw = p - n * HW;
     const float* src = x + n * C * HW + hw;
     int8_t* dst = y + p * cpad;
-    for (int c0 = 0; c0 < cpad; c0 += 4) {
-      uint32_t word = 0;
+    if (wide) {
+      for (int c0 = 0; c0 < cpad; c0 += 16) {
+        v4i o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = c0 + e;
-        int q = 0;
-        if (c < C && r > 0.0f) {
-          const float v = fminf(fmaxf(rintf(src[static_cast<int64_t>(c) * HW] * scale), -128.0f), 127.0f);
-          q = static_cast<int>(v);
-        }
-        word |= (static_cast<uint32_t>(q) & 0xFFu) << (8 * e);
+        for (int d = 0; d < 4; ++d) o[d] = static_cast<int>(quad(src, c0 + 4 * d));
+        *reinterpret_cast<v4i*>(dst + c0) = o;
       }
-      *reinterpret_cast<uint32_t*>(dst + c0) = word;
+    } else {
+      for (int c0 = 0; c0 < cpad; c0 += 4) *reinterpret_cast<uint32_t*>(dst + c0) = quad(src, c0);
     }
   }
 }
@@ -330,9 +395,31 @@ extern "C" int niti_quantize_f32_i8(const float* x, int8_t* y, int N, int C, int
   const int64_t pixels = static_cast<int64_t>(N) * H * W, n = pixels * C;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(absmax_f32_kernel, dim3(grid_for(n, 256, 1024)), dim3(256), 0, s, x, n, absmax_bits);
-  hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad, absmax_bits,
-                     exp_out, bits);
+  hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad, absmax_bits, 1,
+                     exp_out, bits, static_cast<const int64_t*>(nullptr), static_cast<int64_t*>(nullptr), 0);
   return check_launch("quantize");
+}
+
+extern "C" int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
+                                          int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, void* stream) {
+  clear_error();
+  if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || cpad < C || cpad % 4 != 0 || bits < 1 || bits > 7 || targets < 0)
+    return fail(NITI_ERR_INVALID_ARG, "quantize_batch: N=%d C=%d H=%d W=%d cpad=%d bits=%d targets=%d", N, C, H, W, cpad, bits, targets);
+  if (x == nullptr || y == nullptr || parts == nullptr || (targets > 0 && (target_in == nullptr || target_out == nullptr)))
+    return fail(NITI_ERR_INVALID_ARG, "quantize_batch: null pointer");
+  if (reinterpret_cast<uintptr_t>(y) % 4 != 0) return fail(NITI_ERR_INVALID_ARG, "quantize_batch: output must be 4-byte aligned");
+  const int64_t pixels = static_cast<int64_t>(N) * H * W, n = pixels * C;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // up to 12 Ki values (four CIFAR images, 48 loads a thread) a workgroup reads the batch in less time than a launch takes
+  const bool solo = n <= 12288;
+  int nparts = 0;
+  if (!solo) {
+    nparts = grid_for((n + 3) / 4, 1024, kQuantParts);
+    hipLaunchKernelGGL(absmax_parts_f32_kernel, dim3(nparts), dim3(256), 0, s, x, n, parts, target_in, target_out, targets);
+  }
+  hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad, parts, nparts,
+                     exp_out, bits, target_in, target_out, solo ? targets : 0);
+  return check_launch("quantize_batch");
 }
 
 extern "C" int niti_mask_features_i8(const int8_t* x, const int8_t* mask, int8_t* y, int64_t rows, int features,

@@ -271,10 +271,12 @@ def scratch(nbytes: int, device) -> torch.Tensor:
 
 class _SyncArena:
     """Zeroed int32 words for the single-launch kernels of one training step: one fill per step instead of one
-    per kernel.  ``reset`` zeroes the arena and starts handing out slices from its beginning; ``take`` returns the
-    next zeroed slice.  Slices are handed out once per reset, so a kernel never sees words another kernel of the
-    same step wrote.  An arena that runs out (or was never reset) grows by another zeroed chunk, which later
-    resets zero as well, so ``timed_out`` covers every slice handed out since the last reset."""
+    per kernel.  ``reset`` starts handing out slices from the arena's beginning; ``take`` returns the next slice, zeroed: a
+    chunk is filled when its first slice since the reset is taken, so a step pays for the chunks it uses and not for
+    those that earlier callers made the arena grow to, and a step captured into a graph contains the fill of every
+    chunk it uses.  Slices are handed out once per reset, so a kernel never sees words another kernel of the
+    same step wrote.  An arena that runs out (or was never reset) grows by another chunk; ``timed_out`` covers every
+    slice handed out since the last reset."""
 
     WORDS = 1 << 16
     MAX_CHUNKS = 8
@@ -287,10 +289,7 @@ class _SyncArena:
     def reset(self, device):
         key = str(device)
         if key not in self.chunks:
-            self.chunks[key] = [torch.zeros(self.WORDS, dtype=torch.int32, device=device)]
-        else:
-            for c in self.chunks[key]:
-                c.zero_()
+            self.chunks[key] = [torch.empty(self.WORDS, dtype=torch.int32, device=device)]
         self.pos[key] = (0, 0)
         self.taken[key] = []
 
@@ -311,7 +310,9 @@ class _SyncArena:
                     self.reset(device)
                     ci, off, chunks = 0, 0, self.chunks[key]
                     break
-                chunks.append(torch.zeros(max(self.WORDS, words), dtype=torch.int32, device=device))
+                chunks.append(torch.empty(max(self.WORDS, words), dtype=torch.int32, device=device))
+        if off == 0:
+            chunks[ci].zero_()
         self.pos[key] = (ci, off + (words + 31) // 32 * 32)
         self.taken[key].append((ci, off))
         return chunks[ci][off:off + words]
@@ -484,20 +485,42 @@ def relu_fwd(x):
     return y
 
 
-def quantize_input(x, bits=7, cpad=16):
+def quantize_input(x, bits=7, cpad=16, out=None, exp_out=None, target=None, target_out=None):
     """Float NCHW batch -> (int8 NHWC batch with the channels zero-padded to ``cpad``, exponent as a 1-element int32
-    tensor): the reference's input quantiser and the layout change behind it in two launches."""
-    _chk_dev(x)
+    tensor): the reference's input quantiser and the layout change behind it in two launches (one for a few images).
+    ``out`` / ``exp_out``: tensors to write instead of new ones; ``target`` (int64) is copied to ``target_out`` on the way."""
+    _chk_dev(x, out, exp_out, target, target_out)
     if x.dtype != torch.float32 or x.dim() != 4 or not x.is_contiguous():
         raise RuntimeError("quantize_input: contiguous float32 [N,C,H,W] tensor expected")
     N, C, H, W = x.shape
     cpad = max(cpad, (C + 3) // 4 * 4)
-    y = torch.empty((N, H, W, cpad), dtype=torch.int8, device=x.device)
-    am = torch.zeros(1, dtype=torch.int32, device=x.device)
-    exp_out = torch.empty(1, dtype=torch.int32, device=x.device)
-    L.check(L.lib().niti_quantize_f32_i8(_ptr(x), _ptr(y), N, C, H, W, cpad, bits, _ptr(am), _ptr(exp_out), _stream(x)),
-            "niti_quantize_f32_i8")
-    return y, exp_out
+    if out is None:
+        out = torch.empty((N, H, W, cpad), dtype=torch.int8, device=x.device)
+    elif out.dtype != torch.int8 or tuple(out.shape) != (N, H, W, cpad):
+        raise RuntimeError("quantize_input: out must be a contiguous int8 [N,H,W,%d] tensor" % cpad)
+    if exp_out is None:
+        exp_out = torch.empty(1, dtype=torch.int32, device=x.device)
+    targets = 0
+    if target is not None:
+        targets = target.numel()
+        if target.dtype != torch.int64 or target_out is None or target_out.dtype != torch.int64 or target_out.numel() != targets:
+            raise RuntimeError("quantize_input: target and target_out must be int64 tensors of one size")
+    parts = torch.empty(256, dtype=torch.int32, device=x.device)
+    L.check(L.lib().niti_quantize_batch_f32_i8(_ptr(x), _ptr(out), N, C, H, W, cpad, bits, _ptr(parts), _ptr(exp_out), _ptr(target),
+                                               _ptr(target_out), targets, _stream(x)), "niti_quantize_batch_f32_i8")
+    return out, exp_out
+
+
+def batch_metrics(out_val, out_exp, target, sums):
+    """sums (float64 [3]) += batch size x (display loss, top-1 %, top-5 %) of int8 logits [n, classes >= 5] with exponent
+    ``out_exp`` (1-element int32 device tensor), in one launch."""
+    _chk_dev(out_val, out_exp, target, sums)
+    n, classes = out_val.shape
+    if (out_val.dtype != torch.int8 or out_exp.dtype != torch.int32 or target.dtype != torch.int64 or target.numel() != n
+            or sums.dtype != torch.float64 or sums.numel() != 3):
+        raise RuntimeError("batch_metrics: int8 logits [n, classes], int32 exponent, int64 targets [n] and float64 sums [3] expected")
+    L.check(L.lib().niti_batch_metrics_i8(_ptr(out_val), _ptr(out_exp), _ptr(target), n, classes, _ptr(sums), _stream(out_val)),
+            "niti_batch_metrics_i8")
 
 
 def mask_features(x, mask, exp_in=None, exp_add=None):

@@ -21,6 +21,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ops, ti_torch
+from .ti_net import TiNet
 from .ti_vgg import TiVGG_cifar
 
 
@@ -43,7 +44,13 @@ def apply_regime(regime, epoch):
 
 
 def _add_metrics(output, output_exp, target, sums):
-    """Adds batch size x (display loss, top-1, top-5) to ``sums`` (main.py:156-163)."""
+    """Adds batch size x (display loss, top-1, top-5) to ``sums`` (main.py:156-163): one launch for the integer logits of a
+    network, the same as tensor operations for anything else."""
+    if (output.is_cuda and output.dtype == torch.int8 and output.dim() == 2 and output.size(0) > 0 and output.size(1) >= 5
+            and output.is_contiguous() and isinstance(output_exp, torch.Tensor) and output_exp.dtype == torch.int32
+            and output_exp.numel() == 1 and output_exp.is_cuda and target.dtype == torch.int64 and target.is_contiguous()):
+        ops.batch_metrics(output, output_exp.reshape(1), target, sums)
+        return
     scale = torch.exp2(torch.as_tensor(output_exp, device=output.device).float().reshape(()))
     loss = F.cross_entropy(output.float() * scale, target)
     prec1, prec5 = accuracy(output.detach(), target, topk=(1, 5))
@@ -61,9 +68,8 @@ def _one_step(model, training, inputs, target, sums):
 class StepGraph:
     """The integer part of a training (or evaluation) step replayed from a captured HIP graph: a step is some forty
     short launches, and issuing them one by one from Python takes about twice as long as the device needs for them.
-    Only the library's own kernels, fills and random-number kernels are captured.  The input quantisation and the
-    display metrics - tensor-library reductions, whose multi-block forms clear their scratch words with memset
-    nodes that do not replay reliably here - run eagerly before and after each replay, on static buffers.  The
+    Only the library's own kernels, fills and random-number kernels are captured.  The input quantisation, which reads the
+    caller's batch, and the display metrics, which add to the caller's sums, run eagerly before and after each replay.  The
     first ``eager_steps`` batches run eagerly (ordinary steps: nothing is run twice), the next one is captured, from
     then on batches are replays.  Falls back to eager steps if the capture is refused."""
 
@@ -71,6 +77,8 @@ class StepGraph:
         self.model, self.training = model, training
         x_data, _ = model.quantize_input(inputs)
         self.x8 = torch.empty_like(x_data)                                               # quantised batch, NHWC
+        # the library's quantiser can write it: the network has no quantiser of its own, and the layout is that one's
+        self.direct = type(model).quantize_input is TiNet.quantize_input and x_data.dim() == 4 and x_data.shape[3] % 16 == 0
         self.x_exp = torch.empty(1, dtype=torch.int32, device=inputs.device)
         self.target = torch.empty_like(target)
         self.graph, self.failed, self.eager_left = None, False, eager_steps
@@ -83,10 +91,15 @@ class StepGraph:
             self.model.backward(self.target)
 
     def __call__(self, inputs, target, sums):
-        x_data, x_exp = self.model.quantize_input(inputs)       # ti_net.py:17-19
-        self.x8.copy_(x_data)
-        self.x_exp.copy_(x_exp.reshape(1))
-        self.target.copy_(target, non_blocking=True)
+        if (self.direct and inputs.is_cuda and inputs.dtype == torch.float32 and inputs.is_contiguous() and ti_torch.BW_MODE == "int"
+                and target.is_cuda and target.dtype == torch.int64 and target.is_contiguous()):
+            # ti_net.py:17-19 straight into the step's own buffers
+            ops.quantize_input(inputs, ti_torch.BITWIDTH, out=self.x8, exp_out=self.x_exp, target=target, target_out=self.target)
+        else:
+            x_data, x_exp = self.model.quantize_input(inputs)
+            self.x8.copy_(x_data)
+            self.x_exp.copy_(x_exp.reshape(1))
+            self.target.copy_(target, non_blocking=True)
         if self.graph is not None:
             self.graph.replay()
         elif self.eager_left > 0 or self.failed:

@@ -532,3 +532,22 @@ except train.GridWaitTimeout:
     sticky = [l for l in out.stdout.splitlines() if l.startswith("STICKY")][0].split()
     assert sticky[1:] == ["0", "1", "1", "0"], sticky
     assert "RAISED 1" in out.stdout
+
+
+@pytest.mark.parametrize("n,classes", [(1, 10), (80, 10), (1024, 10), (1025, 5), (3000, 33), (37, 600)])
+def test_batch_metrics(tt, n, classes):
+    """Display loss, top-1 and top-5 of a step in one launch against the tensor operations, ties of the largest and of the
+    fifth largest logit included (few distinct values)."""
+    from niti_amd import ops, train
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(n + classes)
+    for hi, e in ((1, -1), (3, 0), (127, -5), (127, 3)):
+        out = ri8(g, n, classes, lo=-hi, hi=hi).to(dev)
+        exp = torch.tensor([e], dtype=torch.int32, device=dev)
+        target = torch.randint(0, classes, (n,), generator=g).to(dev)
+        sums = torch.full((3,), 7.0, dtype=torch.float64, device=dev)
+        ops.batch_metrics(out, exp, target, sums)
+        loss = torch.nn.functional.cross_entropy(out.float() * 2.0 ** e, target)
+        prec1, prec5 = train.accuracy(out, target, topk=(1, 5))
+        ref = torch.stack([loss.double(), prec1.double(), prec5.double()]) * n + 7.0
+        assert torch.allclose(sums, ref, rtol=1e-6, atol=1e-6), (hi, e, sums.tolist(), ref.tolist())
