@@ -93,6 +93,8 @@ int niti_fill_u32(uint32_t* dst, int64_t n, uint32_t value, void* stream);
 size_t niti_conv2d_i8_filter_workspace(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad);
 int niti_conv2d_i8_filter_prepare(const int8_t* w, int8_t* dst, size_t dst_bytes, int N, int H, int W, int C, int K,
                                   int R, int S, int stride, int pad, int dgrad, void* stream);
+/* 1 when a data gradient of this convolution can read the forward pass's copy (NITI_CONV_FILTER_FORWARD_COPY) */
+int niti_conv2d_i8_forward_copy_ok(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 
 /*
  * Convolution forward (cross-correlation), replaces cutlassconv_cuda.sp_conv and

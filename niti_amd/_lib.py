@@ -35,6 +35,7 @@ SIGNATURES = {
     "niti_fill_u32": (_i, [_vp, _i64, C.c_uint32, _vp]),
     "niti_conv2d_i8_filter_workspace": (_sz, [_i] * 10),
     "niti_conv2d_i8_filter_prepare": (_i, [_vp, _vp, _sz] + [_i] * 10 + [_vp]),
+    "niti_conv2d_i8_forward_copy_ok": (_i, [_i] * 9),
     "niti_conv2d_i8_fprop": (_i, [_vp, _vp, _vp] + [_i] * 9 + [_u, _vp, _vp, _sz, _vp]),
     "niti_conv2d_i8_dgrad": (_i, [_vp, _vp, _vp] + [_i] * 9 + [_u, _vp, _vp, _sz, _vp]),
     "niti_conv2d_i8_requant_sync_words": (_sz, [_i] * 10),
@@ -110,6 +111,24 @@ def lib() -> C.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The tensor front end (csrc/host): argument checks, output allocation, sync words and the calls into the library."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise ImportError("niti_amd: the tensor front end cannot be loaded (%s); build it with `python -m niti_amd.build` "
+                              "(there is no fallback implementation)" % e)
+        module.set_error(NitiError)
+        _host = module
+    return _host
 
 
 def check(status: int, what: str) -> None:

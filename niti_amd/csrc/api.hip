@@ -113,9 +113,14 @@ static int check_forward_copy_flag(const char* who, int dgrad, unsigned flags, i
   if (!dgrad) return fail(NITI_ERR_INVALID_ARG, "%s: NITI_CONV_FILTER_FORWARD_COPY is a data-gradient flag", who);
   if (!(flags & NITI_CONV_FILTER_PREPARED))
     return fail(NITI_ERR_INVALID_ARG, "%s: NITI_CONV_FILTER_FORWARD_COPY needs NITI_CONV_FILTER_PREPARED", who);
-  if (filter_copy_kind(N, H, W, C, K, R, S, stride, pad, 0) != 2 || filter_copy_kind(N, H, W, C, K, R, S, stride, pad, 1) != 3)
+  if (niti_conv2d_i8_forward_copy_ok(N, H, W, C, K, R, S, stride, pad) == 0)
     return fail(NITI_ERR_UNSUPPORTED, "%s: the forward filter copy serves the data gradient only where both run the 3x3 kernel", who);
   return NITI_OK;
+}
+
+extern "C" int niti_conv2d_i8_forward_copy_ok(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0) return 0;
+  return filter_copy_kind(N, H, W, C, K, R, S, stride, pad, 0) == 2 && filter_copy_kind(N, H, W, C, K, R, S, stride, pad, 1) == 3 ? 1 : 0;
 }
 
 extern "C" int niti_pad_rows_i8(const int8_t* src, int8_t* dst, int64_t rows, int k, int kpad, void* stream) {

@@ -1,0 +1,528 @@
+// Convolution entries of niti_amd._host (see host.h).
+#include "host.h"
+
+#include <ATen/ops/slice.h>
+
+namespace niti_host {
+namespace {
+
+struct Dims {
+  int N, H, W, C, K, R, S;   // the forward convolution's extents
+};
+int out_extent(int in, int r, int stride, int pad) {
+  const int t = in + 2 * pad - r;
+  return stride <= 0 || t < 0 ? 0 : t / stride + 1;
+}
+Dims forward_dims(const at::Tensor& x, const at::Tensor& w, const char* who) {
+  if (x.dim() != 4 || w.dim() != 4) refuse(std::string(who) + ": [N,H,W,C] and [K,R,S,C] tensors expected");
+  const Dims d{static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), static_cast<int>(x.size(2)), static_cast<int>(x.size(3)),
+               static_cast<int>(w.size(0)), static_cast<int>(w.size(1)), static_cast<int>(w.size(2))};
+  if (w.size(3) != d.C)
+    refuse(std::string(who) + ": channel mismatch " + std::to_string(d.C) + " vs " + std::to_string(w.size(3)));
+  return d;
+}
+// extents of the convolution whose error map is `err`
+Dims gradient_dims(const at::Tensor& err, const at::Tensor& w, int pad, const char* who) {
+  if (err.dim() != 4 || w.dim() != 4) refuse(std::string(who) + ": [N,P,Q,K] and [K,R,S,C] tensors expected");
+  const int R = static_cast<int>(w.size(1)), S = static_cast<int>(w.size(2));
+  if (w.size(0) != err.size(3)) refuse(std::string(who) + ": channel mismatch");
+  return Dims{static_cast<int>(err.size(0)), static_cast<int>(err.size(1)) - 2 * pad + R - 1, static_cast<int>(err.size(2)) - 2 * pad + S - 1,
+              static_cast<int>(w.size(3)), static_cast<int>(w.size(0)), R, S};
+}
+
+struct Rounding {
+  int bits, method, div, bw;
+};
+Rounding rounding_of(Args& a) {
+  Rounding r;
+  r.bits = a.i();
+  r.method = a.i();
+  r.div = a.i();
+  r.bw = a.i();
+  return r;
+}
+
+bool is_i8(const at::Tensor& t) { return t.scalar_type() == at::kChar; }
+
+// ---- int32 results -----------------------------------------------------------------------------------------------
+at::Tensor fprop_i32(const at::Tensor& x, const at::Tensor& w, int stride, int pad, unsigned flags, uint32_t* absmax, Opt prepared) {
+  const char* who = "conv2d_fprop";
+  if (!is_i8(x) || !is_i8(w)) refuse(std::string(who) + ": int8 tensors expected");
+  const Dims d = forward_dims(x, w, who);
+  at::Tensor y = empty32({d.N, out_extent(d.H, d.R, stride, pad), out_extent(d.W, d.S, stride, pad), d.K}, x);
+  at::Tensor ws;
+  size_t bytes = 0;
+  const int8_t* wp = prepared != nullptr ? ptr<int8_t>(*prepared) : ptr<int8_t>(w);
+  if (prepared != nullptr) {
+    flags |= NITI_CONV_FILTER_PREPARED;
+  } else {
+    bytes = niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, stride, pad, 0);
+    if (bytes > 0) ws = empty8({static_cast<int64_t>(bytes)}, x);
+  }
+  check(niti_conv2d_i8_fprop(ptr<int8_t>(x), wp, ptr<int32_t>(y), d.N, d.H, d.W, d.C, d.K, d.R, d.S, stride, pad, flags, absmax,
+                             bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(x)),
+        "niti_conv2d_i8_fprop");
+  return y;
+}
+
+// `prepared`: a kernel-ready filter copy; `forward_copy`: it is the forward pass's
+at::Tensor dgrad_i32(const at::Tensor& err, const at::Tensor& w, int stride, int pad, unsigned flags, uint32_t* absmax, Opt prepared,
+                     bool forward_copy) {
+  const Dims d = gradient_dims(err, w, pad, "conv2d_dgrad");
+  if (d.H < 0 || d.W < 0) refuse("conv2d_dgrad: filter larger than the padded input");
+  at::Tensor dx = empty32({d.N, d.H, d.W, d.C}, err);
+  at::Tensor ws;
+  size_t bytes = 0;
+  const int8_t* wp = ptr<int8_t>(w);
+  if (prepared != nullptr) {
+    flags |= NITI_CONV_FILTER_PREPARED | (forward_copy ? NITI_CONV_FILTER_FORWARD_COPY : 0u);
+    wp = ptr<int8_t>(*prepared);
+  } else {
+    bytes = niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, stride, pad, 1);
+    ws = empty8({static_cast<int64_t>(bytes > 16 ? bytes : 16)}, err);
+  }
+  check(niti_conv2d_i8_dgrad(ptr<int8_t>(err), wp, ptr<int32_t>(dx), d.N, d.H, d.W, d.C, d.K, d.R, d.S, stride, pad, flags, absmax,
+                             prepared != nullptr ? nullptr : ws.data_ptr(), bytes, stream_of(err)),
+        "niti_conv2d_i8_dgrad");
+  return dx;
+}
+
+at::Tensor wgrad_i32(const at::Tensor& act, const at::Tensor& err, int R, int S, int stride, int pad, unsigned flags, uint32_t* absmax, Opt workspace) {
+  if (act.dim() != 4 || err.dim() != 4) refuse("conv2d_wgrad: [N,H,W,C] and [N,P,Q,K] tensors expected");
+  const int N = static_cast<int>(act.size(0)), H = static_cast<int>(act.size(1)), W = static_cast<int>(act.size(2)),
+            C = static_cast<int>(act.size(3)), K = static_cast<int>(err.size(3));
+  const size_t bytes = niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, pad);
+  at::Tensor ws = workspace != nullptr ? *workspace : scratch(bytes, act);
+  if (static_cast<size_t>(ws.numel()) < bytes)
+    refuse("conv2d_wgrad: workspace of " + std::to_string(bytes) + " bytes needed, got " + std::to_string(ws.numel()));
+  at::Tensor dw = empty32({K, R, S, C}, act);
+  check(niti_conv2d_i8_wgrad(ptr<int8_t>(act), ptr<int8_t>(err), ptr<int32_t>(dw), N, H, W, C, K, R, S, stride, pad, flags, absmax, ws.data_ptr(),
+                             bytes, stream_of(act)),
+        "niti_conv2d_i8_wgrad");
+  return dw;
+}
+
+// fprop(x, w, stride, pad, flags, absmax, prepared) -> y
+PyObject* fprop(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 7, "conv2d_fprop");
+    const at::Tensor& x = a.tensor();
+    const at::Tensor& w = a.tensor();
+    const int stride = a.i(), pad = a.i();
+    const unsigned flags = static_cast<unsigned>(a.integer());
+    Opt am = a.opt();
+    return wrap(fprop_i32(x, w, stride, pad, flags, ptr<uint32_t>(am), a.opt()));
+  });
+}
+
+// sp_conv(x, w, stride, pad): the drop-in convolution, results through float32 (cutlassconv_kernel.cu:180-319)
+PyObject* sp_conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 4) refuse("sp_conv: 4 arguments expected");
+    const char* names[2] = {"input", "weight"};
+    for (int i = 0; i < 2; ++i) {
+      if (!THPVariable_Check(args[i])) refuse(std::string(names[i]) + " must be a tensor");
+      const at::Tensor& t = THPVariable_Unpack(args[i]);
+      if (!t.is_cuda()) refuse(std::string(names[i]) + " must be a CUDA tensor");
+      if (!t.is_contiguous()) refuse(std::string(names[i]) + " must be contiguous");
+      if (!is_i8(t)) refuse(std::string("expected scalar type Char but found ") + c10::toString(t.scalar_type()));
+    }
+    Args a(args, n, 4, "sp_conv");
+    const at::Tensor& x = a.tensor();
+    const at::Tensor& w = a.tensor();
+    const int stride = a.i(), pad = a.i();
+    return wrap(fprop_i32(x, w, stride, pad, NITI_EPI_F32_ROUNDTRIP, nullptr, nullptr));
+  });
+}
+
+// dgrad(err, w, stride, pad, flags, absmax, prepared, forward_copy) -> dx
+PyObject* dgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 8, "conv2d_dgrad");
+    const at::Tensor& err = a.tensor();
+    const at::Tensor& w = a.tensor();
+    const int stride = a.i(), pad = a.i();
+    const unsigned flags = static_cast<unsigned>(a.integer());
+    Opt am = a.opt(), prepared = a.opt();
+    return wrap(dgrad_i32(err, w, stride, pad, flags, ptr<uint32_t>(am), prepared, a.flag()));
+  });
+}
+
+// wgrad(act, err, R, S, stride, pad, flags, absmax, workspace) -> dw
+PyObject* wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 9, "conv2d_wgrad");
+    const at::Tensor& act = a.tensor();
+    const at::Tensor& err = a.tensor();
+    const int R = a.i(), S = a.i(), stride = a.i(), pad = a.i();
+    const unsigned flags = static_cast<unsigned>(a.integer());
+    Opt am = a.opt();
+    return wrap(wgrad_i32(act, err, R, S, stride, pad, flags, ptr<uint32_t>(am), a.opt()));
+  });
+}
+
+// ---- results rounded to int8 in the launch -------------------------------------------------------------------------
+struct Fused {
+  bool dgrad = false, f32 = false, relu = false, hint = false, forward_copy = false;
+  int stride = 1, pad = 1, ties = 0;
+  Rounding r{};
+  Opt sync = nullptr, shift = nullptr, exp_a = nullptr, exp_b = nullptr, exp_out = nullptr, prepared = nullptr, mask = nullptr, pool_out = nullptr,
+      pool_in = nullptr, rand = nullptr;
+};
+
+// Convolution + requantisation.  `soft` (a layer asking): returns false, with nothing launched, where the single-launch
+// kernels do not cover the call or the device is too small for them.
+bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const Fused& f, bool soft, at::Tensor* y, at::Tensor* shift,
+                  at::Tensor* sync_view, const char* who) {
+  const int dg = f.dgrad ? 1 : 0;
+  const bool sto = f.r.method == NITI_ROUND_STOCHASTIC;
+  std::vector<int64_t> shape = f.dgrad ? std::vector<int64_t>{d.N, d.H, d.W, d.C}
+                                       : std::vector<int64_t>{d.N, out_extent(d.H, d.R, f.stride, f.pad), out_extent(d.W, d.S, f.stride, f.pad), d.K};
+  if (soft && sto && (f.pool_in != nullptr || d.H == 2)) return false;
+  if (sto) {
+    if (f.rand == nullptr || f.rand->scalar_type() != at::kInt || !has_shape(*f.rand, shape)) {
+      if (soft) return false;
+      refuse(std::string(who) + ": stochastic rounding needs `rand`, a contiguous int32 tensor shaped like the output");
+    }
+    if (f.pool_in != nullptr) refuse_niti(std::string(who) + ": stochastic rounding is not folded in together with the pooling's backward pass");
+  } else if (f.rand != nullptr) {
+    refuse(std::string(who) + ": `rand` is only used by method='sto'");
+  }
+  if (f.mask != nullptr && (!is_i8(*f.mask) || !has_shape(*f.mask, shape))) refuse(std::string(who) + ": relu_mask must be int8 and shaped like the output");
+  if (f.pool_in != nullptr) {   // the result is written at the pooling input's size
+    const std::vector<int64_t> big{shape[0], 2 * shape[1], 2 * shape[2], shape[3]};
+    if (f.mask == nullptr || !is_i8(*f.pool_in) || !has_shape(*f.pool_in, big))
+      refuse(std::string(who) + ": unpool needs relu_mask (the pooled map) and a contiguous int8 [N,2H,2W,C] pooling input");
+    shape = big;
+  }
+  if (!is_i8(x) || !is_i8(w)) refuse(std::string(who) + ": int8 tensors expected");
+  const size_t words = niti_conv2d_i8_requant_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
+  if (words == 0) {
+    if (soft) return false;
+    refuse_niti(std::string(who) + ": shape not covered by the single-launch path");
+  }
+  size_t have = 0;
+  uint32_t* sync = sync_words(f.sync, words, x, sync_view, &have, who);
+  *y = empty8(shape, x);
+  if (f.hint && f.shift == nullptr) refuse(std::string(who) + ": shift_hint needs shift_out, holding the predicted shift");
+  *shift = f.shift != nullptr ? *f.shift : scalar32(x);
+  unsigned flags = f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u;
+  at::Tensor ws;
+  size_t bytes = 0;
+  const int8_t* wp = ptr<int8_t>(w);
+  if (f.prepared != nullptr) {
+    flags |= NITI_CONV_FILTER_PREPARED | (f.forward_copy ? NITI_CONV_FILTER_FORWARD_COPY : 0u);
+    wp = ptr<int8_t>(*f.prepared);
+  } else {
+    bytes = niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
+    ws = empty8({static_cast<int64_t>(bytes > 16 ? bytes : 16)}, x);
+  }
+  void* wsp = f.prepared != nullptr ? nullptr : ws.data_ptr();
+  const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u);
+  const int8_t* xp = ptr<int8_t>(x);
+  int8_t* yp = ptr<int8_t>(*y);
+  int32_t* sp = ptr<int32_t>(*shift);
+  const int32_t *ea = ptr<int32_t>(f.exp_a), *eb = ptr<int32_t>(f.exp_b);
+  int32_t* eo = ptr<int32_t>(f.exp_out);
+  void* st = stream_of(x);
+  int rc;
+  if (sto && !f.dgrad)
+    rc = niti_conv2d_i8_fprop_requant_sto(xp, wp, yp, ptr<int8_t>(f.pool_out), ptr<int32_t>(f.rand), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride,
+                                          f.pad, flags, f.r.bits, f.r.div, f.r.bw, rq, sync, have, sp, ea, eb, eo, wsp, bytes, st);
+  else if (sto)
+    rc = niti_conv2d_i8_dgrad_requant_sto(xp, wp, yp, ptr<int32_t>(f.rand), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, flags, f.r.bits,
+                                          f.r.div, f.r.bw, rq, ptr<int8_t>(f.mask), sync, have, sp, ea, eb, eo, wsp, bytes, st);
+  else if (f.pool_in != nullptr)
+    rc = niti_conv2d_i8_dgrad_requant_unpool(xp, wp, yp, ptr<int8_t>(f.mask), ptr<int8_t>(f.pool_in), f.ties, d.N, d.H, d.W, d.C, d.K, d.R, d.S,
+                                             f.stride, f.pad, flags, f.r.bits, f.r.method, f.r.div, f.r.bw, rq, sync, have, sp, ea, eb, eo, wsp,
+                                             bytes, st);
+  else if (f.dgrad)
+    rc = niti_conv2d_i8_dgrad_requant(xp, wp, yp, d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, flags, f.r.bits, f.r.method, f.r.div, f.r.bw,
+                                      rq, ptr<int8_t>(f.mask), sync, have, sp, ea, eb, eo, wsp, bytes, st);
+  else if (f.pool_out != nullptr)
+    rc = niti_conv2d_i8_fprop_requant_pool(xp, wp, yp, ptr<int8_t>(f.pool_out), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, flags, f.r.bits,
+                                           f.r.method, f.r.div, f.r.bw, rq, sync, have, sp, ea, eb, eo, wsp, bytes, st);
+  else
+    rc = niti_conv2d_i8_fprop_requant(xp, wp, yp, d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, flags, f.r.bits, f.r.method, f.r.div, f.r.bw,
+                                      rq, sync, have, sp, ea, eb, eo, wsp, bytes, st);
+  if (soft) return check_fits(rc, who);
+  check(rc, who);
+  return true;
+}
+
+// int32 sums -> int8, for the shapes outside the single-launch kernels
+at::Tensor requant_i32(const at::Tensor& acc, const uint32_t* absmax, const Rounding& r, Opt rand, bool relu, int32_t* shift, Opt exp_a, Opt exp_b,
+                       int32_t* exp_out) {
+  if (rand != nullptr && (rand->scalar_type() != at::kInt || rand->numel() != acc.numel()))
+    refuse("requant: rand must be int32 with one entry per element");
+  at::Tensor y = empty8(acc.sizes(), acc);
+  check(niti_requant_i32_i8(ptr<int32_t>(acc), ptr<int8_t>(y), acc.numel(), absmax, r.bits, r.method, r.div, r.bw, ptr<int32_t>(rand),
+                            relu ? NITI_RQ_RELU : 0u, shift, ptr<int32_t>(exp_a), ptr<int32_t>(exp_b), exp_out, stream_of(acc)),
+        "niti_requant_i32_i8");
+  return y;
+}
+
+// requant_op(who, x, w, stride, pad, f32, bits, method, div, bw, relu, hint, sync, shift, exp_a, exp_b, exp_out, prepared,
+//            forward_copy, mask, pool_out, pool_in, ties, rand) -> (y, shift, sync): ops.conv2d_*_requant
+PyObject* requant_op(PyObject* const* args, Py_ssize_t n, bool dg) {
+  return guarded([&]() -> PyObject* {
+    const char* who = dg ? "niti_conv2d_i8_dgrad_requant" : "niti_conv2d_i8_fprop_requant";
+    Args a(args, n, 23, who);
+    const at::Tensor& x = a.tensor();
+    const at::Tensor& w = a.tensor();
+    Fused f;
+    f.dgrad = dg;
+    f.stride = a.i();
+    f.pad = a.i();
+    f.f32 = a.flag();
+    f.r = rounding_of(a);
+    f.relu = a.flag();
+    f.hint = a.flag();
+    f.sync = a.opt();
+    f.shift = a.opt();
+    f.exp_a = a.opt();
+    f.exp_b = a.opt();
+    f.exp_out = a.opt();
+    f.prepared = a.opt();
+    f.forward_copy = a.flag();
+    f.mask = a.opt();
+    f.pool_out = a.opt();
+    f.pool_in = a.opt();
+    f.ties = a.i();
+    f.rand = a.opt();
+    const Dims d = dg ? gradient_dims(x, w, f.pad, who) : forward_dims(x, w, who);
+    if (f.pool_out != nullptr &&
+        (!is_i8(*f.pool_out) || !has_shape(*f.pool_out, {d.N, out_extent(d.H, d.R, f.stride, f.pad) / 2, out_extent(d.W, d.S, f.stride, f.pad) / 2, d.K})))
+      refuse("conv2d_fprop_requant: pool_out must be a contiguous int8 [N,P/2,Q/2,K] tensor");
+    at::Tensor y, shift, sync;
+    conv_requant(x, w, d, f, false, &y, &shift, &sync, who);
+    return tuple_of({y, shift, sync});
+  });
+}
+PyObject* fprop_requant(PyObject*, PyObject* const* args, Py_ssize_t n) { return requant_op(args, n, false); }
+PyObject* dgrad_requant(PyObject*, PyObject* const* args, Py_ssize_t n) { return requant_op(args, n, true); }
+
+// layer_forward(fuse, x, w, stride, pad, f32, bits, method, div, bw, relu, shift state, exp_a, exp_b, prepared, pool, rand)
+//   -> (y, exponent, pooled map or None)
+// TiConv2d.forward: convolution, act_calc and where asked the ReLU and the 2x2 max-pool behind it (`pool`), in one launch
+// where the single-launch kernels cover the shape; otherwise convolution, then requantisation (nothing pooled).
+PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 17, "conv layer forward");
+    const bool fuse = a.flag();
+    const at::Tensor& x = a.tensor();
+    const at::Tensor& w = a.tensor();
+    Fused f;
+    f.stride = a.i();
+    f.pad = a.i();
+    f.f32 = a.flag();
+    f.r = rounding_of(a);
+    f.relu = a.flag();
+    f.shift = a.opt();
+    f.hint = f.shift != nullptr;
+    f.exp_a = a.opt();
+    f.exp_b = a.opt();
+    f.prepared = a.opt();
+    const bool pool = a.flag();
+    f.rand = a.opt();
+    const Dims d = forward_dims(x, w, "conv layer");
+    at::Tensor y, shift, pooled, e = scalar32(x);
+    f.exp_out = &e;
+    if (fuse) {
+      if (pool && f.relu && f.stride == 1 && f.pad == 1 && d.R == 3 && d.S == 3 && d.H == d.W && d.H >= 2 && d.H % 2 == 0) {
+        pooled = empty8({d.N, d.H / 2, d.W / 2, d.K}, x);
+        f.pool_out = &pooled;
+      }
+      if (conv_requant(x, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_fprop_requant")) return tuple_of({y, e, pooled});
+    }
+    uint32_t* am = arena_take(1, x, nullptr);
+    at::Tensor acc = fprop_i32(x, w, f.stride, f.pad, f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u, am, f.prepared);
+    y = requant_i32(acc, am, f.r, f.rand, f.relu, nullptr, f.exp_a, f.exp_b, ptr<int32_t>(e));
+    return tuple_of({y, e, at::Tensor()});
+  });
+}
+
+// layer_dgrad(fuse, err, w, stride, pad, f32, bits, method, div, bw, shift state, exp_a, exp_b, forward copy, mask, pool_in,
+//             ties, rand) -> (error, exponent, unpooled?)
+// TiConv2d.backward's data gradient: err_calc(conv_dgrad(err, w)), zeroed where `mask` (the layer's input) is not positive,
+// and - `pool_in` given - routed through the 2x2 max-pool in front of the layer, one launch where the kernels cover it.
+PyObject* layer_dgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 18, "conv layer data gradient");
+    const bool fuse = a.flag();
+    const at::Tensor& err = a.tensor();
+    const at::Tensor& w = a.tensor();
+    Fused f;
+    f.dgrad = true;
+    f.stride = a.i();
+    f.pad = a.i();
+    f.f32 = a.flag();
+    f.r = rounding_of(a);
+    f.shift = a.opt();
+    f.hint = f.shift != nullptr;
+    f.exp_a = a.opt();
+    f.exp_b = a.opt();
+    f.prepared = a.opt();
+    f.mask = a.opt();
+    Opt pool_in = a.opt();
+    f.ties = a.i();
+    f.rand = a.opt();
+    const Dims d = gradient_dims(err, w, f.pad, "conv layer");
+    // the forward pass's copy serves the data gradient only where both run the 3x3 kernel
+    f.forward_copy = f.prepared != nullptr;
+    if (f.forward_copy && niti_conv2d_i8_forward_copy_ok(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad) == 0) {
+      f.forward_copy = false;
+      f.prepared = nullptr;
+    }
+    at::Tensor y, shift, e = scalar32(err);
+    f.exp_out = &e;
+    PyObject* unpooled = Py_False;
+    bool done = false;
+    if (fuse && pool_in != nullptr) {
+      f.pool_in = pool_in;
+      done = conv_requant(err, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant_unpool");
+      if (done) unpooled = Py_True;
+      f.pool_in = nullptr;
+    }
+    if (fuse && !done) done = conv_requant(err, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant");
+    if (!done) {
+      uint32_t* am = arena_take(1, err, nullptr);
+      at::Tensor dx = dgrad_i32(err, w, f.stride, f.pad, f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u, am, f.prepared, f.forward_copy);
+      y = requant_i32(dx, am, f.r, f.rand, false, nullptr, f.exp_a, f.exp_b, ptr<int32_t>(e));
+      if (f.mask != nullptr)
+        check(niti_relu_i8_bwd(ptr<int8_t>(*f.mask), ptr<int8_t>(y), ptr<int8_t>(y), y.numel(), stream_of(err)), "niti_relu_i8_bwd");
+    }
+    PyObject* out = PyTuple_New(3);
+    if (out == nullptr) throw python_error();
+    PyTuple_SET_ITEM(out, 0, wrap(y));
+    PyTuple_SET_ITEM(out, 1, wrap(e));
+    Py_INCREF(unpooled);
+    PyTuple_SET_ITEM(out, 2, unpooled);
+    return out;
+  });
+}
+
+struct Update {
+  at::Tensor g8, dw, shift;
+};
+// weight gradient + grad_calc + update in one call; `soft` as in conv_requant
+bool wgrad_update_fused(const at::Tensor& act, const at::Tensor& err, const at::Tensor& w, int stride, int pad, unsigned flags, const Rounding& r,
+                        bool want_grad, bool want_dw, Opt sync, Opt shift, Opt exp_a, Opt exp_b, int32_t* exp_out, Opt workspace, Opt prepared,
+                        bool soft, Update* u, at::Tensor* sync_view) {
+  const char* who = "niti_conv2d_i8_wgrad_update";
+  if (!is_i8(act) || !is_i8(err) || !is_i8(w)) refuse("conv2d_wgrad_update: int8 tensors expected");
+  if (act.dim() != 4 || err.dim() != 4 || w.dim() != 4) refuse("conv2d_wgrad_update: four-dimensional tensors expected");
+  const int N = static_cast<int>(act.size(0)), H = static_cast<int>(act.size(1)), W = static_cast<int>(act.size(2)), C = static_cast<int>(act.size(3));
+  const int K = static_cast<int>(w.size(0)), R = static_cast<int>(w.size(1)), S = static_cast<int>(w.size(2)), Cw = static_cast<int>(w.size(3));
+  if (err.size(3) != K) refuse("conv2d_wgrad_update: channel mismatch");
+  const size_t words = niti_conv2d_i8_wgrad_update_sync_words(N, H, W, C, K, R, S, stride, pad);
+  if (words == 0) {
+    if (soft) return false;
+    refuse_niti("conv2d_wgrad_update: shape not covered by the single-pass path");
+  }
+  if (!has_shape(err, {N, out_extent(H, R, 1, pad), out_extent(W, S, 1, pad), K})) refuse("conv2d_wgrad_update: error map does not match the activations");
+  size_t have = 0;
+  uint32_t* sp = sync_words(sync, words, act, sync_view, &have, "conv2d_wgrad_update");
+  const size_t bytes = niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, pad);
+  at::Tensor ws = workspace != nullptr ? *workspace : scratch(bytes, act);
+  if (static_cast<size_t>(ws.numel()) < bytes)
+    refuse("conv2d_wgrad_update: workspace of " + std::to_string(bytes) + " bytes needed, got " + std::to_string(ws.numel()));
+  if (want_grad) u->g8 = empty8(w.sizes(), w);
+  if (want_dw) u->dw = empty32({K, R, S, C}, w);
+  u->shift = shift != nullptr ? *shift : scalar32(w);
+  const int rc = niti_conv2d_i8_wgrad_update(
+      ptr<int8_t>(act), ptr<int8_t>(err), ptr<int8_t>(w), Cw, N, H, W, C, K, R, S, stride, pad, flags, r.bits, r.method, r.div, r.bw, sp, have,
+      want_grad ? ptr<int8_t>(u->g8) : nullptr, want_dw ? ptr<int32_t>(u->dw) : nullptr, ptr<int8_t>(prepared), ptr<int32_t>(u->shift),
+      ptr<int32_t>(exp_a), ptr<int32_t>(exp_b), exp_out, ws.data_ptr(), bytes, stream_of(act));
+  if (soft) return check_fits(rc, who);
+  check(rc, who);
+  return true;
+}
+
+// wgrad_update(act, err, w, stride, pad, flags, mu, method, div, bw, sync, want_grad, want_dw, shift, exp_a, exp_b, exp_out,
+//              workspace, prepared) -> (g8, dw, shift, sync)
+PyObject* wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 19, "conv2d_wgrad_update");
+    const at::Tensor& act = a.tensor();
+    const at::Tensor& err = a.tensor();
+    const at::Tensor& w = a.tensor();
+    const int stride = a.i(), pad = a.i();
+    const unsigned flags = static_cast<unsigned>(a.integer());
+    const Rounding r = rounding_of(a);
+    Opt sync = a.opt();
+    const bool want_grad = a.flag(), want_dw = a.flag();
+    Opt shift = a.opt(), exp_a = a.opt(), exp_b = a.opt(), exp_out = a.opt(), workspace = a.opt(), prepared = a.opt();
+    Update u;
+    at::Tensor view;
+    wgrad_update_fused(act, err, w, stride, pad, flags, r, want_grad, want_dw, sync, shift, exp_a, exp_b, ptr<int32_t>(exp_out), workspace, prepared,
+                       false, &u, &view);
+    return tuple_of({u.g8, u.dw, u.shift, view});
+  });
+}
+
+// layer_wgrad_update(fuse, act, err, w, stride, pad, f32, mu, method, div, bw, want_grad, want_dw, shift state, exp_a, exp_b,
+//                    prepared, rand) -> (g8, dw, shift, exponent, one call?)
+// TiConv2d.backward's weight gradient, grad_calc and update of w in place; without a one-call form the int32 gradient (its
+// zero-padded channels dropped) is rounded and applied in a second step and returned.
+PyObject* layer_wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 18, "conv layer weight gradient");
+    const bool fuse = a.flag();
+    const at::Tensor& act = a.tensor();
+    const at::Tensor& err = a.tensor();
+    const at::Tensor& w = a.tensor();
+    const int stride = a.i(), pad = a.i();
+    const unsigned flags = a.flag() ? NITI_EPI_F32_ROUNDTRIP : 0u;
+    const Rounding r = rounding_of(a);
+    const bool want_grad = a.flag(), want_dw = a.flag();
+    Opt shift = a.opt(), exp_a = a.opt(), exp_b = a.opt(), prepared = a.opt(), rand = a.opt();
+    at::Tensor e = scalar32(act);
+    Update u;
+    bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, flags | (shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), r, want_grad, want_dw,
+                                          nullptr, shift, exp_a, exp_b, ptr<int32_t>(e), nullptr, prepared, true, &u, nullptr);
+    if (one) {
+      if (want_dw && u.dw.size(3) != w.size(3)) u.dw = u.dw.slice(3, 0, w.size(3)).contiguous();
+    } else {
+      uint32_t* am = arena_take(1, act, nullptr);
+      u.dw = wgrad_i32(act, err, static_cast<int>(w.size(1)), static_cast<int>(w.size(2)), stride, pad, flags, am, nullptr);
+      // zero-padded input channels give zero gradient columns (they cannot raise the range)
+      if (u.dw.size(3) != w.size(3)) u.dw = u.dw.slice(3, 0, w.size(3)).contiguous();
+      if (rand != nullptr && (rand->scalar_type() != at::kInt || rand->numel() != u.dw.numel()))
+        refuse("grad_update: rand must be int32 with one entry per element");
+      if (want_grad) u.g8 = empty8(w.sizes(), w);
+      u.shift = scalar32(w);
+      check(niti_grad_update_i8(ptr<int32_t>(u.dw), ptr<int8_t>(w), u.dw.numel(), am, r.bits, r.method, r.div, r.bw, ptr<int32_t>(rand),
+                                want_grad ? ptr<int8_t>(u.g8) : nullptr, ptr<int32_t>(u.shift), ptr<int32_t>(exp_a), ptr<int32_t>(exp_b),
+                                ptr<int32_t>(e), stream_of(act)),
+            "niti_grad_update_i8");
+    }
+    PyObject* out = PyTuple_New(5);
+    if (out == nullptr) throw python_error();
+    PyTuple_SET_ITEM(out, 0, wrap(u.g8));
+    PyTuple_SET_ITEM(out, 1, wrap(u.dw));
+    PyTuple_SET_ITEM(out, 2, wrap(u.shift));
+    PyTuple_SET_ITEM(out, 3, wrap(e));
+    PyObject* b = one ? Py_True : Py_False;
+    Py_INCREF(b);
+    PyTuple_SET_ITEM(out, 4, b);
+    return out;
+  });
+}
+
+#define FAST(name) reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(name)), METH_FASTCALL, nullptr
+}  // namespace
+
+PyMethodDef kConvMethods[] = {{"conv_fprop", FAST(fprop)},
+                              {"sp_conv", FAST(sp_conv)},
+                              {"conv_dgrad", FAST(dgrad)},
+                              {"conv_wgrad", FAST(wgrad)},
+                              {"conv_fprop_requant", FAST(fprop_requant)},
+                              {"conv_dgrad_requant", FAST(dgrad_requant)},
+                              {"conv_layer_forward", FAST(layer_forward)},
+                              {"conv_layer_dgrad", FAST(layer_dgrad)},
+                              {"conv_wgrad_update", FAST(wgrad_update)},
+                              {"conv_layer_wgrad_update", FAST(layer_wgrad_update)},
+                              {nullptr, nullptr, 0, nullptr}};
+
+}  // namespace niti_host

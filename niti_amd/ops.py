@@ -1,6 +1,7 @@
 """Tensor-level front end of the C ABI: takes torch device tensors, allocates outputs and
 workspaces with the torch allocator, launches on torch's current stream.  Nothing here
-computes: every function is one (or a few) calls into libniti_gfx950.so."""
+computes: every function is one (or a few) calls into libniti_gfx950.so - those that a layer makes on every
+step through the native module _host (csrc/host), the others through ctypes."""
 from __future__ import annotations
 
 from typing import Optional, Tuple
@@ -56,123 +57,22 @@ def conv2d_fprop(x, w, stride=1, padding=1, f32_epilogue=False, absmax: Optional
                  prepared_filter=None):
     """x [N,H,W,C] int8, w [K,R,S,C] int8 -> [N,P,Q,K] int32.  ``prepared_filter``: the output of
     conv_filter_prepare(w, N, H, W, stride, padding), to keep the filter copy out of the call."""
-    _chk_dev(x, w, absmax, prepared_filter)
-    if x.dtype != torch.int8 or w.dtype != torch.int8:
-        raise RuntimeError("conv2d_fprop: int8 tensors expected")
-    N, H, W, C = x.shape
-    K, R, S, C2 = w.shape
-    if C2 != C:
-        raise RuntimeError("conv2d_fprop: channel mismatch %d vs %d" % (C, C2))
-    P = (H + 2 * padding - R) // stride + 1
-    Q = (W + 2 * padding - S) // stride + 1
-    y = torch.empty((N, max(P, 0), max(Q, 0), K), dtype=torch.int32, device=x.device)
-    flags = _flags(f32_epilogue)
-    if prepared_filter is not None:
-        st = L.lib().niti_conv2d_i8_fprop(_ptr(x), _ptr(prepared_filter), _ptr(y), N, H, W, C, K, R, S, stride, padding,
-                                          flags | L.CONV_FILTER_PREPARED, _ptr(absmax), None, 0, _stream(x))
-    else:
-        nbytes = L.lib().niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, padding, 0)
-        ws = torch.empty(nbytes, dtype=torch.int8, device=x.device) if nbytes else None
-        st = L.lib().niti_conv2d_i8_fprop(_ptr(x), _ptr(w), _ptr(y), N, H, W, C, K, R, S, stride, padding, flags,
-                                          _ptr(absmax), _ptr(ws), nbytes, _stream(x))
-    L.check(st, "niti_conv2d_i8_fprop")
-    return y
+    return L.host().conv_fprop(x, w, stride, padding, L.EPI_F32_ROUNDTRIP if f32_epilogue else 0, absmax, prepared_filter)
 
 
 def conv2d_dgrad(err, w, stride=1, padding=1, f32_epilogue=False, absmax=None, prepared_filter=None, forward_filter=None):
     """err [N,P,Q,K] int8, w [K,R,S,C] int8 -> dx [N,H,W,C] int32 (stride 1).  ``prepared_filter``:
     the output of conv_filter_prepare(w, N, H, W, stride, padding, dgrad=True).  ``forward_filter``: the copy the
     FORWARD pass reads (conv_filter_prepare(.., dgrad=False)), for shapes where both passes run the 3x3 kernel."""
-    _chk_dev(err, w, absmax, prepared_filter, forward_filter)
-    N, P, Q, K = err.shape
-    K2, R, S, C = w.shape
-    if K2 != K:
-        raise RuntimeError("conv2d_dgrad: channel mismatch")
-    H = P - 2 * padding + R - 1
-    W = Q - 2 * padding + S - 1
-    dx = torch.empty((N, H, W, C), dtype=torch.int32, device=err.device)
-    flags = _flags(f32_epilogue)
-    if forward_filter is not None:
-        prepared_filter, flags = forward_filter, flags | L.CONV_FILTER_FORWARD_COPY
-    if prepared_filter is not None:
-        st = L.lib().niti_conv2d_i8_dgrad(_ptr(err), _ptr(prepared_filter), _ptr(dx), N, H, W, C, K, R, S, stride, padding,
-                                          flags | L.CONV_FILTER_PREPARED, _ptr(absmax), None, 0, _stream(err))
-    else:
-        nbytes = L.lib().niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, padding, 1)
-        ws = torch.empty(max(nbytes, 16), dtype=torch.int8, device=err.device)
-        st = L.lib().niti_conv2d_i8_dgrad(_ptr(err), _ptr(w), _ptr(dx), N, H, W, C, K, R, S, stride, padding,
-                                          flags, _ptr(absmax), _ptr(ws), nbytes, _stream(err))
-    L.check(st, "niti_conv2d_i8_dgrad")
-    return dx
+    forward = forward_filter is not None
+    return L.host().conv_dgrad(err, w, stride, padding, L.EPI_F32_ROUNDTRIP if f32_epilogue else 0, absmax,
+                               forward_filter if forward else prepared_filter, forward)
 
 
 def conv_requant_sync_words(N, H, W, C, K, R=3, S=3, stride=1, padding=1, dgrad=False) -> int:
     """uint32 words of the sync buffer conv2d_fprop_requant / conv2d_dgrad_requant need for a convolution with
     INPUT [N,H,W,C] and filter [K,R,S,C]; 0 when only the two-pass path (conv2d_* then requant) covers the shape."""
     return int(L.lib().niti_conv2d_i8_requant_sync_words(N, H, W, C, K, R, S, stride, padding, int(dgrad)))
-
-
-def _conv_requant(entry, dgrad, x, w, out_shape, dims, stride, padding, f32_epilogue, target_bits, method, div_mode,
-                  bw_mode, relu, sync, shift_out, exp_a, exp_b, exp_out, prepared_filter, relu_mask=None, forward_filter=None,
-                  shift_hint=False, pool_out=None, unpool=None, rand=None):
-    _chk_dev(x, w, sync, shift_out, exp_a, exp_b, exp_out, prepared_filter, relu_mask, forward_filter, rand)
-    if method == "sto":
-        # StoShift folded in: one random integer per output element (its low `shift` bits are used)
-        if rand is None or rand.dtype != torch.int32 or tuple(rand.shape) != tuple(out_shape) or not rand.is_contiguous():
-            raise RuntimeError("%s: stochastic rounding needs `rand`, a contiguous int32 tensor shaped like the output" % entry)
-        if unpool is not None:
-            raise L.NitiError("%s: stochastic rounding is not folded in together with the pooling's backward pass" % entry)
-    elif rand is not None:
-        raise RuntimeError("%s: `rand` is only used by method='sto'" % entry)
-    if relu_mask is not None and (relu_mask.dtype != torch.int8 or tuple(relu_mask.shape) != tuple(out_shape)):
-        raise RuntimeError("%s: relu_mask must be int8 and shaped like the output" % entry)
-    if unpool is not None:      # (pooling input [N,2H,2W,C], tie rule): the result is written at that size
-        pool_in, ties = unpool
-        _chk_dev(x, pool_in)
-        n_, h_, w_, c_ = out_shape
-        if relu_mask is None or pool_in.dtype != torch.int8 or tuple(pool_in.shape) != (n_, 2 * h_, 2 * w_, c_) or not pool_in.is_contiguous():
-            raise RuntimeError("%s: unpool needs relu_mask (the pooled map) and a contiguous int8 [N,2H,2W,C] pooling input" % entry)
-        entry = "niti_conv2d_i8_dgrad_requant_unpool"
-        out_shape = tuple(pool_in.shape)
-    if x.dtype != torch.int8 or w.dtype != torch.int8:
-        raise RuntimeError("%s: int8 tensors expected" % entry)
-    N, H, W, C, K, R, S = dims
-    words = conv_requant_sync_words(N, H, W, C, K, R, S, stride, padding, dgrad)
-    if words == 0:
-        raise L.NitiError("%s: shape not covered by the single-launch path" % entry)
-    if sync is None:
-        sync = sync_arena.take(words, x.device)
-    elif sync.dtype != torch.int32 or sync.numel() < words:
-        raise RuntimeError("%s: sync must be a zeroed int32 tensor of at least %d words" % (entry, words))
-    y = torch.empty(out_shape, dtype=torch.int8, device=x.device)
-    if shift_out is None:
-        if shift_hint:
-            raise RuntimeError("%s: shift_hint needs shift_out, holding the predicted shift" % entry)
-        shift_out = torch.empty(1, dtype=torch.int32, device=x.device)
-    flags = _flags(f32_epilogue)
-    if forward_filter is not None:
-        prepared_filter, flags = forward_filter, flags | L.CONV_FILTER_FORWARD_COPY
-    if prepared_filter is not None:
-        wptr, ws, nbytes, flags = _ptr(prepared_filter), None, 0, flags | L.CONV_FILTER_PREPARED
-    else:
-        nbytes = L.lib().niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, padding, int(dgrad))
-        ws = torch.empty(max(nbytes, 16), dtype=torch.int8, device=x.device)
-        wptr = _ptr(w)
-    head = (_ptr(x), wptr, _ptr(y), N, H, W, C, K, R, S, stride, padding, flags, target_bits, L.ROUND[method],
-            L.DIV[div_mode], L.BW[bw_mode], (L.RQ_RELU if relu else 0) | (L.RQ_SHIFT_HINT if shift_hint else 0))
-    tail = (_ptr(sync), sync.numel(), _ptr(shift_out), _ptr(exp_a), _ptr(exp_b), _ptr(exp_out), _ptr(ws), nbytes, _stream(x))
-    if method == "sto":         # entries of their own: (pooled output,) random integers behind the output, no method argument
-        entry = "niti_conv2d_i8_dgrad_requant_sto" if dgrad else "niti_conv2d_i8_fprop_requant_sto"
-        head = head[:3] + ((_ptr(rand),) if dgrad else (_ptr(pool_out), _ptr(rand))) + head[3:14] + head[15:]
-    elif pool_out is not None:    # the entry with the pooled output takes it right after the output
-        head = head[:3] + (_ptr(pool_out),) + head[3:]
-    if unpool is not None:
-        head = head[:3] + (_ptr(relu_mask), _ptr(unpool[0]), L.TIES[unpool[1]]) + head[3:]
-        st = getattr(L.lib(), entry)(*(head + tail))
-    else:
-        st = getattr(L.lib(), entry)(*(head + ((_ptr(relu_mask),) if dgrad else ()) + tail))
-    L.check(st, entry)
-    return y, shift_out, sync
 
 
 def conv2d_fprop_requant(x, w, stride=1, padding=1, f32_epilogue=False, target_bits=7, method="round", div_mode="floor",
@@ -183,20 +83,9 @@ def conv2d_fprop_requant(x, w, stride=1, padding=1, f32_epilogue=False, target_b
     given, must hold conv_requant_sync_words(...) zeroed int32 words.  ``shift_hint``: ``shift_out`` holds a
     predicted shift on entry (e.g. this tensor's shift of the previous training step); a good prediction saves the
     kernel a second store pass, the results do not depend on it."""
-    N, H, W, C = x.shape
-    K, R, S, C2 = w.shape
-    if C2 != C:
-        raise RuntimeError("conv2d_fprop_requant: channel mismatch %d vs %d" % (C, C2))
-    P = (H + 2 * padding - R) // stride + 1
-    Q = (W + 2 * padding - S) // stride + 1
-    if pool_out is not None:
-        _chk_dev(x, pool_out)
-        if pool_out.dtype != torch.int8 or tuple(pool_out.shape) != (N, P // 2, Q // 2, K) or not pool_out.is_contiguous():
-            raise RuntimeError("conv2d_fprop_requant: pool_out must be a contiguous int8 [N,P/2,Q/2,K] tensor")
-    entry = "niti_conv2d_i8_fprop_requant_pool" if pool_out is not None else "niti_conv2d_i8_fprop_requant"
-    return _conv_requant(entry, False, x, w, (N, P, Q, K), (N, H, W, C, K, R, S), stride, padding,
-                         f32_epilogue, target_bits, method, div_mode, bw_mode, relu, sync, shift_out, exp_a, exp_b, exp_out,
-                         prepared_filter, shift_hint=shift_hint, pool_out=pool_out, rand=rand)
+    return L.host().conv_fprop_requant(x, w, stride, padding, f32_epilogue, target_bits, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode],
+                                       relu, shift_hint, sync, shift_out, exp_a, exp_b, exp_out, prepared_filter, False, None, pool_out,
+                                       None, 0, rand)
 
 
 def conv2d_fprop_requant_static(x, w, stride=1, padding=1, f32_epilogue=False, target_bits=7, method="round", div_mode="floor",
@@ -242,31 +131,24 @@ def conv2d_dgrad_requant(err, w, stride=1, padding=1, f32_epilogue=False, target
     ``relu_mask`` (int8 [N,H,W,C]): results whose mask element is not positive are stored as zero, after range
     and rounding were taken from the unmasked sums (the backward pass of a ReLU in front of the layer).
     ``forward_filter``: the copy the forward pass reads, in place of ``prepared_filter`` (see conv2d_dgrad)."""
-    N, P, Q, K = err.shape
-    K2, R, S, C = w.shape
-    if K2 != K:
-        raise RuntimeError("conv2d_dgrad_requant: channel mismatch")
-    H = P - 2 * padding + R - 1
-    W = Q - 2 * padding + S - 1
-    return _conv_requant("niti_conv2d_i8_dgrad_requant", True, err, w, (N, H, W, C), (N, H, W, C, K, R, S), stride, padding,
-                         f32_epilogue, target_bits, method, div_mode, bw_mode, False, sync, shift_out, exp_a, exp_b, exp_out,
-                         prepared_filter, relu_mask, forward_filter, shift_hint, unpool=unpool, rand=rand)
+    forward = forward_filter is not None
+    pool_in, ties = unpool if unpool is not None else (None, "first")
+    return L.host().conv_dgrad_requant(err, w, stride, padding, f32_epilogue, target_bits, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode],
+                                       False, shift_hint, sync, shift_out, exp_a, exp_b, exp_out,
+                                       forward_filter if forward else prepared_filter, forward, relu_mask, None, pool_in, L.TIES[ties], rand)
 
 
-_scratch = {}
+def _index(device) -> int:
+    dev = torch.device(device)
+    return torch.cuda.current_device() if dev.index is None else dev.index
 
 
 def scratch(nbytes: int, device) -> torch.Tensor:
-    """One grow-only int8 buffer per device for kernel workspaces that live only inside a call.  Calls on one
+    """One grow-only int8 buffer per stream for kernel workspaces that live only inside a call.  Calls on one
     stream run in order, so they can all use the same memory - which also keeps the partial sums of
     consecutive weight-gradient launches in the same cache-resident region instead of walking through fresh
-    allocations.  Not for use from several streams at once."""
-    key = str(device)
-    buf = _scratch.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.int8, device=device)
-        _scratch[key] = buf
-    return buf
+    allocations.  Under graph capture: memory of the graph."""
+    return L.host().scratch(nbytes, _index(device))
 
 
 class _SyncArena:
@@ -276,56 +158,23 @@ class _SyncArena:
     those that earlier callers made the arena grow to, and a step captured into a graph contains the fill of every
     chunk it uses.  Slices are handed out once per reset, so a kernel never sees words another kernel of the
     same step wrote.  An arena that runs out (or was never reset) grows by another chunk; ``timed_out`` covers every
-    slice handed out since the last reset."""
-
-    WORDS = 1 << 16
-    MAX_CHUNKS = 8
-
-    def __init__(self):
-        self.chunks = {}    # device -> list of int32 tensors
-        self.pos = {}       # device -> (chunk index, offset)
-        self.taken = {}     # device -> list of (chunk index, offset)
+    slice handed out since the last reset.  Every stream, and every stream capture, has an arena of its own
+    (csrc/host/host.cpp); reset and take work on the current stream's."""
 
     def reset(self, device):
-        key = str(device)
-        if key not in self.chunks:
-            self.chunks[key] = [torch.empty(self.WORDS, dtype=torch.int32, device=device)]
-        self.pos[key] = (0, 0)
-        self.taken[key] = []
+        L.host().arena_reset(_index(device))
 
     def take(self, words, device):
-        key = str(device)
-        if key not in self.chunks:
-            self.reset(device)
-        ci, off = self.pos[key]
-        chunks = self.chunks[key]
-        while off + words > chunks[ci].numel():
-            ci, off = ci + 1, 0
-            if ci == len(chunks):
-                if torch.cuda.is_current_stream_capturing():
-                    raise RuntimeError("sync arena: out of words while a graph is being captured; run one step eagerly first")
-                if len(chunks) >= self.MAX_CHUNKS and words <= self.WORDS:
-                    # a caller that never resets: start over (the fill is ordered behind the launches that used the
-                    # words; their flags are gone from here but stay in the device-wide word, see sync_timeouts)
-                    self.reset(device)
-                    ci, off, chunks = 0, 0, self.chunks[key]
-                    break
-                chunks.append(torch.empty(max(self.WORDS, words), dtype=torch.int32, device=device))
-        if off == 0:
-            chunks[ci].zero_()
-        self.pos[key] = (ci, off + (words + 31) // 32 * 32)
-        self.taken[key].append((ci, off))
-        return chunks[ci][off:off + words]
+        return L.host().arena_take(words, _index(device))
 
     def timed_out(self, device) -> bool:
         """True if a single-launch kernel that used a slice since the last reset flagged that its grid-wide wait ran
         into the time limit (its output is then invalid).  Copies the flags to the host: for the end of a step or an
         epoch, not for the inner loop."""
-        key = str(device)
-        flags = [self.chunks[key][ci][off + 1] for ci, off in self.taken.get(key, [])]
+        flags = L.host().arena_flags(_index(device))
         if not flags:
             return False
-        return bool(torch.stack(flags).ne(0).any().item())
+        return bool(torch.cat(flags).ne(0).any().item())
 
 
 def sync_timeouts(device=None, clear=True) -> bool:
@@ -346,19 +195,8 @@ sync_arena = _SyncArena()
 
 def conv2d_wgrad(act, err, R, S, stride=1, padding=1, f32_epilogue=False, absmax=None, workspace=None):
     """act [N,H,W,C] int8, err [N,P,Q,K] int8 -> dw [K,R,S,C] int32 (stride 1).  ``workspace``: int8 tensor of
-    at least niti_conv2d_i8_wgrad_workspace bytes (default: a fresh allocation)."""
-    _chk_dev(act, err, absmax, workspace)
-    N, H, W, C = act.shape
-    K = err.shape[3]
-    dw = torch.empty((K, R, S, C), dtype=torch.int32, device=act.device)
-    nbytes = L.lib().niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, padding)
-    ws = workspace if workspace is not None else torch.empty(max(nbytes, 16), dtype=torch.int8, device=act.device)
-    if ws.numel() < nbytes:
-        raise RuntimeError("conv2d_wgrad: workspace of %d bytes needed, got %d" % (nbytes, ws.numel()))
-    st = L.lib().niti_conv2d_i8_wgrad(_ptr(act), _ptr(err), _ptr(dw), N, H, W, C, K, R, S, stride, padding,
-                                      _flags(f32_epilogue), _ptr(absmax), _ptr(ws), nbytes, _stream(act))
-    L.check(st, "niti_conv2d_i8_wgrad")
-    return dw
+    at least niti_conv2d_i8_wgrad_workspace bytes (default: the stream's scratch buffer)."""
+    return L.host().conv_wgrad(act, err, R, S, stride, padding, L.EPI_F32_ROUNDTRIP if f32_epilogue else 0, absmax, workspace)
 
 
 def wgrad_update_sync_words(N, H, W, C, K, R=3, S=3, stride=1, padding=1) -> int:
@@ -376,64 +214,19 @@ def conv2d_wgrad_update(act, err, w, stride=1, padding=1, f32_epilogue=False, mu
     on entry (the previous step's): the update's stores then overlap the wait for the tensor's range."""
     if shift_hint and shift_out is None:
         raise RuntimeError("conv2d_wgrad_update: shift_hint needs shift_out, holding the predicted shift")
-    _chk_dev(act, err, w, sync, shift_out, exp_a, exp_b, exp_out, workspace, prepared_filter)
-    if act.dtype != torch.int8 or err.dtype != torch.int8 or w.dtype != torch.int8:
-        raise RuntimeError("conv2d_wgrad_update: int8 tensors expected")
-    N, H, W, C = act.shape
-    K, R, S, Cw = w.shape
-    if err.shape[3] != K:
-        raise RuntimeError("conv2d_wgrad_update: channel mismatch")
-    words = wgrad_update_sync_words(N, H, W, C, K, R, S, stride, padding)
-    if words == 0:
-        raise L.NitiError("conv2d_wgrad_update: shape not covered by the single-pass path")
-    if sync is None:
-        sync = sync_arena.take(words, act.device)
-    elif sync.dtype != torch.int32 or sync.numel() < words:
-        raise RuntimeError("conv2d_wgrad_update: sync must be a zeroed int32 tensor of at least %d words" % words)
-    nbytes = L.lib().niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, padding)
-    ws = workspace if workspace is not None else torch.empty(max(nbytes, 16), dtype=torch.int8, device=act.device)
-    if ws.numel() < nbytes:
-        raise RuntimeError("conv2d_wgrad_update: workspace of %d bytes needed, got %d" % (nbytes, ws.numel()))
-    g8 = torch.empty(w.shape, dtype=torch.int8, device=w.device) if want_grad else None
-    dw = torch.empty((K, R, S, C), dtype=torch.int32, device=w.device) if want_dw else None
-    if shift_out is None:
-        shift_out = torch.empty(1, dtype=torch.int32, device=w.device)
-    st = L.lib().niti_conv2d_i8_wgrad_update(_ptr(act), _ptr(err), _ptr(w), Cw, N, H, W, C, K, R, S, stride, padding,
-                                             _flags(f32_epilogue) | (L.CONV_SHIFT_HINT if shift_hint else 0), mu, L.ROUND[method],
-                                             L.DIV[div_mode], L.BW[bw_mode],
-                                             _ptr(sync), sync.numel(), _ptr(g8), _ptr(dw), _ptr(prepared_filter), _ptr(shift_out), _ptr(exp_a),
-                                             _ptr(exp_b), _ptr(exp_out), _ptr(ws), nbytes, _stream(act))
-    L.check(st, "niti_conv2d_i8_wgrad_update")
-    return g8, dw, shift_out, sync
+    flags = (L.EPI_F32_ROUNDTRIP if f32_epilogue else 0) | (L.CONV_SHIFT_HINT if shift_hint else 0)
+    return L.host().conv_wgrad_update(act, err, w, stride, padding, flags, mu, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode], sync,
+                                      want_grad, want_dw, shift_out, exp_a, exp_b, exp_out, workspace, prepared_filter)
 
 
 def gemm(a, b, trans_a=False, trans_b=False, absmax=None, out=None, f32_epilogue=False):
     """c[m,n] = op(a) @ op(b), int8 x int8 -> int32.  trans_a: a stored [k,m]; trans_b: b stored [n,k].
     f32_epilogue: every sum takes the int32 -> float32 -> int32 round trip of the reference's convolution epilogue."""
-    _chk_dev(a, b, absmax, out)
-    if a.dtype != torch.int8 or b.dtype != torch.int8:
-        raise RuntimeError("gemm: int8 tensors expected")
-    m, k = (a.shape[1], a.shape[0]) if trans_a else (a.shape[0], a.shape[1])
-    n, k2 = (b.shape[0], b.shape[1]) if trans_b else (b.shape[1], b.shape[0])
-    if k != k2:
-        raise RuntimeError("gemm: inner extents differ (%d vs %d)" % (k, k2))
-    c = out if out is not None else torch.empty((m, n), dtype=torch.int32, device=a.device)
-    nbytes = L.lib().niti_gemm_i8_workspace(int(trans_a), int(trans_b), m, n, k)
-    ws = torch.empty(nbytes, dtype=torch.int8, device=a.device) if nbytes else None
-    st = L.lib().niti_gemm_i8(int(trans_a), int(trans_b), _ptr(a), _ptr(b), _ptr(c), m, n, k,
-                              L.EPI_F32_ROUNDTRIP if f32_epilogue else 0, _ptr(absmax),
-                              _ptr(ws), nbytes, _stream(a))
-    L.check(st, "niti_gemm_i8")
-    return c
+    return L.host().gemm(a, b, trans_a, trans_b, absmax, out, L.EPI_F32_ROUNDTRIP if f32_epilogue else 0)
 
 
 def absmax_i32(x, absmax=None):
-    _chk_dev(x, absmax)
-    if absmax is None:
-        absmax = new_scalar_u32(x.device)
-    st = L.lib().niti_absmax_i32(_ptr(x), x.numel(), _ptr(absmax), _stream(x))
-    L.check(st, "niti_absmax_i32")
-    return absmax
+    return L.host().absmax_i32(x, absmax)
 
 
 def requant(x, absmax, target_bits=7, method="round", div_mode="floor", bw_mode="int", rand=None, relu=False,
@@ -489,26 +282,7 @@ def quantize_input(x, bits=7, cpad=16, out=None, exp_out=None, target=None, targ
     """Float NCHW batch -> (int8 NHWC batch with the channels zero-padded to ``cpad``, exponent as a 1-element int32
     tensor): the reference's input quantiser and the layout change behind it in two launches (one for a few images).
     ``out`` / ``exp_out``: tensors to write instead of new ones; ``target`` (int64) is copied to ``target_out`` on the way."""
-    _chk_dev(x, out, exp_out, target, target_out)
-    if x.dtype != torch.float32 or x.dim() != 4 or not x.is_contiguous():
-        raise RuntimeError("quantize_input: contiguous float32 [N,C,H,W] tensor expected")
-    N, C, H, W = x.shape
-    cpad = max(cpad, (C + 3) // 4 * 4)
-    if out is None:
-        out = torch.empty((N, H, W, cpad), dtype=torch.int8, device=x.device)
-    elif out.dtype != torch.int8 or tuple(out.shape) != (N, H, W, cpad):
-        raise RuntimeError("quantize_input: out must be a contiguous int8 [N,H,W,%d] tensor" % cpad)
-    if exp_out is None:
-        exp_out = torch.empty(1, dtype=torch.int32, device=x.device)
-    targets = 0
-    if target is not None:
-        targets = target.numel()
-        if target.dtype != torch.int64 or target_out is None or target_out.dtype != torch.int64 or target_out.numel() != targets:
-            raise RuntimeError("quantize_input: target and target_out must be int64 tensors of one size")
-    parts = torch.empty(256, dtype=torch.int32, device=x.device)
-    L.check(L.lib().niti_quantize_batch_f32_i8(_ptr(x), _ptr(out), N, C, H, W, cpad, bits, _ptr(parts), _ptr(exp_out), _ptr(target),
-                                               _ptr(target_out), targets, _stream(x)), "niti_quantize_batch_f32_i8")
-    return out, exp_out
+    return L.host().quantize_input(x, bits, cpad, out, exp_out, target, target_out)
 
 
 def batch_metrics(out_val, out_exp, target, sums):
@@ -917,27 +691,12 @@ def mfma_probe(operands, workgroups=512, iters=1200):
 
 
 def maxpool_fwd(x, kernel_size=2, stride=2, padding=0):
-    _chk_dev(x)
-    if x.dtype != torch.int8:
-        raise RuntimeError("maxpool_fwd: int8 tensor expected")
-    N, H, W, C = x.shape
-    P = (H + 2 * padding - kernel_size) // stride + 1
-    Q = (W + 2 * padding - kernel_size) // stride + 1
-    y = torch.empty((N, max(P, 0), max(Q, 0), C), dtype=torch.int8, device=x.device)
-    st = L.lib().niti_maxpool_i8_fwd(_ptr(x), _ptr(y), N, H, W, C, kernel_size, stride, padding, _stream(x))
-    L.check(st, "niti_maxpool_i8_fwd")
-    return y
+    return L.host().maxpool_fwd(x, kernel_size, stride, padding)
 
 
 def maxpool_bwd(y, dy, x, kernel_size=2, stride=2, padding=0, ties="first", relu=False):
     """``relu``: also zero the gradient where x <= 0 (the backward pass of a ReLU whose output x is)."""
-    _chk_dev(y, dy, x)
-    N, H, W, C = x.shape
-    dx = torch.empty_like(x)
-    st = L.lib().niti_maxpool_i8_bwd(_ptr(y), _ptr(dy), _ptr(x), _ptr(dx), N, H, W, C, kernel_size, stride, padding,
-                                     L.TIES[ties] | (L.POOL_BWD_RELU if relu else 0), _stream(x))
-    L.check(st, "niti_maxpool_i8_bwd")
-    return dx
+    return L.host().maxpool_bwd(y, dy, x, kernel_size, stride, padding, L.TIES[ties] | (L.POOL_BWD_RELU if relu else 0))
 
 
 def group_conv_f32(x, w, stride, padding, dilation, groups):

@@ -1,24 +1,14 @@
 """Stand-in for the reference's ``cutlassconv_cuda`` extension
 (pytorch/cutlass-extension/cutlassconv.cpp:105-113)."""
-import torch
-
-from .. import ops
-
-
-def _check(t, name):
-    from . import check_input
-    check_input(t, name)
-    if t.dtype != torch.int8:
-        raise RuntimeError("expected scalar type Char but found %s" % t.dtype)  # what .data<int8_t>() raises
+from .. import _lib as L
+from .. import ops  # noqa: F401  (brings torch in before the native module)
 
 
 def sp_conv(input, weight, stride_h, padding_h):
     """cutlassconv.cpp:57-64 -> cutlassconv_kernel.cu:180-319: NHWC int8 x KRSC int8 -> new NPQK
     int32 tensor, cross-correlation, same stride/padding in both dimensions, results passed through
     fp32 as the CUTLASS epilogue does."""
-    _check(input, "input")
-    _check(weight, "weight")
-    return ops.conv2d_fprop(input, weight, int(stride_h), int(padding_h), f32_epilogue=True)
+    return L.host().sp_conv(input, weight, int(stride_h), int(padding_h))
 
 
 def sp_conv_optimized(input, weight, stride_h, padding_h):

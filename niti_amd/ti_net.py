@@ -29,7 +29,7 @@ class TiNet(Module):
         for a, b, c in zip(layers, layers[1:], layers[2:]):
             if (isinstance(a, ti_torch.TiConv2d) and isinstance(b, ti_torch.TiReLU) and b.fused and isinstance(c, ti_torch.TiMaxpool2d)
                     and (c.kernel_size, c.stride, c.padding) == (2, 2, 0)):
-                a.pool_after = c
+                a.__dict__["pool_after"] = c      # plain attributes, not sub-modules: the pooling has its own place in the network
         # ReLU [-> max-pool] -> TiConv2d: the convolution zeroes its data gradient where its own input (the ReLU's
         # possibly pooled output) is not positive, which is that ReLU's backward pass (a max-pool routes gradients
         # only to elements equal to the pooled maximum, so masking before or after its backward is the same)
@@ -44,7 +44,7 @@ class TiNet(Module):
                 l.bwd_folded = True
                 if j == i + 2 and (layers[i + 1].kernel_size, layers[i + 1].stride, layers[i + 1].padding) == (2, 2, 0):
                     # ... and the data gradient writes its result through that max-pool's backward pass as well
-                    layers[j].pool_below = layers[i + 1]
+                    layers[j].__dict__["pool_below"] = layers[i + 1]
             elif j == i + 2:
                 # ReLU -> max-pool -> anything else: the pooling's backward pass applies the mask to its own output
                 layers[i + 1].relu_below = True

@@ -24,7 +24,7 @@ import torch
 import torch.nn.functional as F
 from torch.nn.modules import Module
 
-from . import ops
+from . import _lib, ops
 
 GPU = "cuda"
 BITWIDTH = 7
@@ -48,9 +48,11 @@ def _exp_tensor(e, device) -> torch.Tensor:
     (which also keeps a step capturable into a HIP graph)."""
     if isinstance(e, torch.Tensor):
         if e.is_cuda:
+            if e.dtype == torch.int32 and e.dim() == 1:
+                return e
             return e.reshape(1) if e.dtype == torch.int32 else e.reshape(1).to(torch.int32)
         e = int(e)
-    key = (int(e), str(device))
+    key = (int(e), device)
     t = _EXP_CONSTANTS.get(key)
     if t is None:
         t = torch.tensor([int(e)], dtype=torch.int32, device=device)
@@ -101,14 +103,24 @@ ERROR_ROUND_METHOD = RoundShift
 GRAD_ROUND_METHOD = PstoShift
 
 
+_METHODS = {RoundShift: "round", StoShift: "sto", PstoShift: "psto"}
+_METHOD_CODES = {fn: _lib.ROUND[name] for fn, name in _METHODS.items()}
+_STO = _lib.ROUND["sto"]
+
+
 def _method_name(fn) -> str:
-    if fn is RoundShift:
-        return "round"
-    if fn is StoShift:
-        return "sto"
-    if fn is PstoShift:
-        return "psto"
-    raise ValueError("rounding method must be RoundShift, StoShift or PstoShift")
+    try:
+        return _METHODS[fn]
+    except KeyError:
+        raise ValueError("rounding method must be RoundShift, StoShift or PstoShift") from None
+
+
+def _method_code(fn) -> int:
+    """The library's number of a rounding method."""
+    try:
+        return _METHOD_CODES[fn]
+    except KeyError:
+        raise ValueError("rounding method must be RoundShift, StoShift or PstoShift") from None
 
 
 def _rand_bits_like(x: torch.Tensor) -> torch.Tensor:
@@ -138,7 +150,6 @@ def roundoff4(size):
 # ------------------------------------------------------------------------------------------
 def TensorBitwidth(val):
     """ti_torch.py:366-367 (host value; synchronises)."""
-    from . import _lib
     return int(_lib.lib().niti_bitwidth(int(val), _lib.BW[BW_MODE]))
 
 
@@ -184,60 +195,16 @@ def grad_calc(int32_acc, mu, absmax=None, rand=None):
     return y, shift
 
 
-FUSE_CONV_REQUANT = True     # run convolution + requantisation as one launch where the library covers the shape
+FUSE_CONV_REQUANT = True     # run a product + requantisation as one launch where the library covers the shape
 KEEP_INT32_GRAD = False      # also store layer.grad_int32acc when the weight gradient is rounded and applied in one call
-_fused_refused = set()       # (dgrad, input shape, filter shape, stride, padding) the device turned out too small for
 
 
-def _conv_requant_fused(dgrad, x, w, stride, padding, fn, rand, relu, exp_a, exp_b, relu_mask=None, prepared_filter=None,
-                        forward_filter=None, shift_state=None, pool_out=None, unpool=None):
-    """conv (forward or data gradient) + act_calc / err_calc as one launch.  Returns (int8 tensor, shift,
-    exp_out) or None when the call needs the two-pass path: a shape outside the single-launch kernel, more
-    workgroups than the device holds at once, or StoShift (ti_torch.py:33-46) on a 2 x 2 map or together with the
-    pooling's backward pass.  StoShift otherwise runs inside the launch on ``rand`` (int32, shaped like the output;
-    drawn here when the caller gives none)."""
-    method = _method_name(fn)
-    if not FUSE_CONV_REQUANT or (method != "sto" and rand is not None):
+def _sto_rand(method, rand, shape, dev):
+    """Random integers (int32, contiguous) for a rounding of a tensor of ``shape``: the caller's or 31 random bits each,
+    of which a kernel keeps the low `shift` ones; None where the method takes none."""
+    if method != _STO:
         return None
-    key = (dgrad, tuple(x.shape), tuple(w.shape), stride, padding, unpool is not None)
-    if key in _fused_refused:
-        return None
-    N = x.shape[0]
-    K, R, S, C = w.shape
-    H, W = (x.shape[1] - 2 * padding + R - 1, x.shape[2] - 2 * padding + S - 1) if dgrad else (x.shape[1], x.shape[2])
-    if ops.conv_requant_sync_words(N, H, W, C, K, R, S, stride, padding, dgrad) == 0:
-        _fused_refused.add(key)
-        return None
-    if method == "sto":
-        if unpool is not None or H == 2:
-            return None
-        out_shape = (N, H, W, C) if dgrad else (N, (H + 2 * padding - R) // stride + 1, (W + 2 * padding - S) // stride + 1, K)
-        if rand is None:
-            rand = torch.randint(0, 2 ** 31 - 1, out_shape, dtype=torch.int32, device=x.device)
-        elif rand.dtype != torch.int32 or tuple(rand.shape) != out_shape:
-            return None
-        rand = rand.contiguous()
-    from ._lib import NitiError
-    exp_out = torch.empty(1, dtype=torch.int32, device=x.device)
-    call = ops.conv2d_dgrad_requant if dgrad else ops.conv2d_fprop_requant
-    kw = dict(relu=relu, prepared_filter=prepared_filter) if not dgrad else dict(relu_mask=relu_mask, forward_filter=forward_filter)
-    if pool_out is not None:
-        kw.update(pool_out=pool_out)
-    if unpool is not None:
-        kw.update(unpool=unpool)
-    if shift_state is not None:     # the tensor's shift of the previous step: the kernel's prediction for this one
-        kw.update(shift_out=shift_state, shift_hint=True)
-    if method == "sto":
-        kw.update(rand=rand)
-    try:
-        y, shift, _ = call(x, w, stride, padding, f32_epilogue=F32_EPILOGUE, target_bits=BITWIDTH, method=method,
-                           div_mode=DIV_MODE, bw_mode=BW_MODE, exp_a=exp_a, exp_b=exp_b, exp_out=exp_out, **kw)
-    except NitiError as e:
-        if "do not fit" not in str(e):
-            raise
-        _fused_refused.add(key)
-        return None
-    return y, shift, exp_out
+    return torch.randint(0, 2 ** 31 - 1, shape, dtype=torch.int32, device=dev) if rand is None else rand.contiguous()
 
 
 # ------------------------------------------------------------------------------------------
@@ -400,171 +367,116 @@ class TiConv2d(UpdateWeight):
         self.pool_below = None      # the 2x2 / stride-2 TiMaxpool2d in front of this layer, if its backward pass is folded in
 
     def forward(self, input, rand=None):
-        self.act, self.act_in_exp = input
-        dev = self.act.device
-        self.act16 = _pad_channels16(self.act).contiguous()      # channel-padded copy, reused by the weight gradient
+        d = self.__dict__       # plain attributes: Module.__setattr__ looks for parameters first
+        act, act_exp = input
+        d["act"], d["act_in_exp"] = act, act_exp
+        dev = act.device
+        # channel-padded copy, reused by the weight gradient
+        act16 = d["act16"] = act if act.shape[3] % 16 == 0 and act.is_contiguous() else _pad_channels16(act).contiguous()
+        weight = self.weight
         # With an up-to-date kernel-ready filter copy the padded weights are passed for their shape only: the first
         # layer then reuses the padded tensor the copy was made from instead of padding the weights again every step.
-        key = (self.weight.data_ptr(), self.weight._version, tuple(self.act16.shape))
-        shape_only = (self.weight.shape[3] % 16 != 0 and getattr(self, "_wprep_key", None) == key
-                      and getattr(self, "_wprep", None) is not None and getattr(self, "_w16_kept", None) is not None)
-        w16 = self._w16_kept if shape_only else _pad_channels16(self.weight).contiguous()
-        self._w16_kept = w16 if self.weight.shape[3] % 16 != 0 else None
-        exp_a, exp_b = _exp_tensor(self.act_in_exp, dev), self._wexp()
-        pooled = None
-        N, H, W, _ = self.act16.shape
-        if self.pool_after is not None and self.fuse_relu and self.stride == 1 and self.padding == 1 and H == W and H >= 2 and H % 2 == 0:
-            pooled = torch.empty((N, H // 2, W // 2, self.weight.shape[0]), dtype=torch.int8, device=dev)
-        fused = _conv_requant_fused(False, self.act16, w16, self.stride, self.padding, ACT_ROUND_METHOD, rand,
-                                    self.fuse_relu, exp_a, exp_b, prepared_filter=self._forward_filter(w16),
-                                    shift_state=self._shift_state("act", dev), pool_out=pooled)
-        if fused is not None:
-            if pooled is not None:      # the pooling layer finds its result ready when it sees this tensor
-                self.pool_after.preset = (fused[0], pooled)
-            return fused[0], fused[2]
-        if shape_only:
-            w16 = self._w16_kept = _pad_channels16(self.weight).contiguous()
-        am = ops.new_scalar_u32(dev)
-        acc = ops.conv2d_fprop(self.act16, w16, self.stride, self.padding, f32_epilogue=F32_EPILOGUE, absmax=am)
-        act_out, _, exp_out = _requant(acc, BITWIDTH, ACT_ROUND_METHOD, am, rand, relu=self.fuse_relu,
-                                       exp_a=exp_a, exp_b=exp_b, want_exp=True)
-        return act_out, exp_out
+        key = (weight.data_ptr(), weight._version, act16.shape)
+        fresh = d.get("_wprep_key") == key
+        if weight.shape[3] % 16 == 0:
+            w16, shape_only = (weight if weight.is_contiguous() else weight.contiguous()), False
+            d["_w16_kept"] = None
+        else:
+            shape_only = fresh and d.get("_wprep") is not None and d.get("_w16_kept") is not None
+            w16 = d["_w16_kept"] = self._w16_kept if shape_only else _pad_channels16(weight).contiguous()
+        if not fresh:
+            # kernel-ready copy of the filter: made when the weight tensor was replaced or modified through torch; the
+            # fused weight update keeps it in step with its own changes
+            N, H, W, _ = act16.shape
+            d["_wprep"] = ops.conv_filter_prepare(w16, N, H, W, self.stride, self.padding)
+            d["_wprep_key"] = key
+        method = _method_code(ACT_ROUND_METHOD)
+        if method == _STO:
+            R, S = w16.shape[1:3]
+            N, H, W, _ = act16.shape
+            rand = _sto_rand(method, rand, (N, (H + 2 * self.padding - R) // self.stride + 1, (W + 2 * self.padding - S) // self.stride + 1,
+                                            w16.shape[0]), dev)
+        elif rand is not None:
+            rand = None
+        y, exp_out, pooled = _lib.host().conv_layer_forward(
+            FUSE_CONV_REQUANT, act16, w16, self.stride, self.padding, F32_EPILOGUE, BITWIDTH, method, _lib.DIV[DIV_MODE], _lib.BW[BW_MODE],
+            self.fuse_relu, self._shift_state("act", dev), _exp_tensor(act_exp, dev), self._wexp(), d["_wprep"],
+            self.pool_after is not None, rand)
+        if pooled is not None:      # the pooling layer finds its result ready when it sees this tensor
+            self.pool_after.__dict__["preset"] = (y, pooled)
+        return y, exp_out
 
     def backward(self, input, rand=None, grad_rand=None):
+        d = self.__dict__
         err_in, err_exp = input
-        err_in = err_in.contiguous()
+        if not err_in.is_contiguous():
+            err_in = err_in.contiguous()
         dev = err_in.device
-        self.err_exp_in = _exp_tensor(err_exp, dev)
-        self.err_exp = self.err_exp_in
+        host = _lib.host()
+        div, bw = _lib.DIV[DIV_MODE], _lib.BW[BW_MODE]
+        d["err_exp_in"] = d["err_exp"] = _exp_tensor(err_exp, dev)
+        act, act16, weight = d["act"], d["act16"], self.weight
+        if not weight.is_contiguous():
+            weight = self.weight = weight.contiguous()
+        prepared = self._synced_filter()
         if not self.first_layer:
             # data gradient with the weights as they were in the forward pass
             # relu_below: the ReLU in front of this layer (possibly with a max-pool in between) leaves its backward
             # pass to this layer, whose input is that ReLU's (pooled) output
-            from ._lib import NitiError
-            mask = self.act.contiguous() if self.relu_below else None
-            try:
-                err_out, new_exp = self._data_gradient(err_in, rand, mask, self._dgrad_filter())
-            except NitiError as e:
-                if "forward filter copy" not in str(e):
-                    raise
-                self._dgrad_own_copy = True     # this shape's data gradient runs a kernel that needs its own copy
-                err_out, new_exp = self._data_gradient(err_in, rand, mask, None)
-            self.err_exp = new_exp
-        K, R, S, C = self.weight.shape
-        if self._wgrad_update_fused(err_in, grad_rand):
-            if not self.first_layer:
-                return err_out, self.err_exp
-            return None
-        amg = ops.new_scalar_u32(dev)
-        dw = ops.conv2d_wgrad(self.act16, err_in, R, S, self.stride, self.padding,
-                              f32_epilogue=F32_EPILOGUE and not self.first_layer, absmax=amg,
-                              workspace=self._wgrad_workspace(err_in))
-        # zero-padded input channels give zero gradient columns: drop them (they cannot raise the range)
-        self.grad_int32acc = dw if dw.shape[3] == C else dw[..., :C].contiguous()
-        self.weight_update(amg, grad_rand)
+            mask = pool_in = None
+            if self.relu_below:
+                mask = act if act.is_contiguous() else act.contiguous()
+                pool = self.pool_below
+                # the max-pool in front of this layer: its backward pass is written by this launch's epilogue
+                if pool is not None and err_in.shape[1] >= 2:
+                    pooled, whole = pool.__dict__.get("act_out"), pool.__dict__.get("act_in")
+                    if pooled is not None and pooled.data_ptr() == mask.data_ptr() and whole.is_contiguous():
+                        pool_in = whole
+            method = _method_code(ERROR_ROUND_METHOD)
+            if method == _STO:
+                N, P, Q, _ = err_in.shape
+                _, R, S, C = weight.shape
+                rand = _sto_rand(method, rand, (N, P - 2 * self.padding + R - 1, Q - 2 * self.padding + S - 1, C), dev)
+            elif rand is not None:
+                rand = None
+            err_out, new_exp, unpooled = host.conv_layer_dgrad(
+                FUSE_CONV_REQUANT, err_in, weight, self.stride, self.padding, F32_EPILOGUE, BITWIDTH, method, div, bw,
+                self._shift_state("err", dev), d["err_exp_in"], self._wexp(),
+                prepared if act16.shape[3] == weight.shape[3] else None, mask, pool_in, _lib.TIES[POOL_TIES], rand)
+            if unpooled:
+                pool.__dict__["bwd_done"] = err_out
+            d["err_exp"] = new_exp
+        method = _method_code(GRAD_ROUND_METHOD)
+        grad_rand = _sto_rand(method, grad_rand, tuple(weight.shape), dev)
+        d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"], one = host.conv_layer_wgrad_update(
+            FUSE_CONV_REQUANT and grad_rand is None, act16, err_in, weight, self.stride, self.padding,
+            F32_EPILOGUE and not self.first_layer, GRAD_BITWIDTH, method, div, bw, self.keep_grad, KEEP_INT32_GRAD,
+            self._shift_state("grad", dev), d["err_exp"], _exp_tensor(d["act_in_exp"], dev), prepared, grad_rand)
+        if not one:
+            d["_wprep_key"] = None      # any kernel-ready copy of the old weights is stale now
         if not self.first_layer:
-            return err_out, self.err_exp
+            return err_out, d["err_exp"]
 
     def _shift_state(self, which, device):
         """1-element int32 device tensor that keeps the requantisation shift of this layer's activations ("act") or
         errors ("err") from one step to the next; the single-launch kernels take it as their prediction."""
-        states = self.__dict__.setdefault("_shift_states", {})
-        key = (which, str(device))
-        if key not in states:
-            states[key] = torch.zeros(1, dtype=torch.int32, device=device)
-        return states[key]
-
-    def _dgrad_filter(self):
-        """The forward pass's kernel-ready filter copy, which the data gradient can read in place of a copy of its
-        own while it matches the weights, or None."""
-        if getattr(self, "_dgrad_own_copy", False) or self.act16.shape[3] != self.weight.shape[3]:
-            return None
-        return self._synced_filter()
-
-    def _data_gradient(self, err_in, rand, mask, forward_filter):
-        """err_calc(conv_dgrad(err_in, weight)) (ti_torch.py:422-427), the ReLU mask applied; -> (int8 error, exponent)."""
-        pool = self.pool_below
-        if (pool is not None and mask is not None and err_in.shape[1] >= 2 and getattr(pool, "act_out", None) is not None
-                and pool.act_out.data_ptr() == mask.data_ptr() and pool.act_in.is_contiguous()):
-            # the max-pool in front of this layer: its backward pass is written by this launch's epilogue
-            fused = _conv_requant_fused(True, err_in, self.weight, self.stride, self.padding, ERROR_ROUND_METHOD, rand,
-                                        False, self.err_exp_in, self._wexp(), relu_mask=mask, forward_filter=forward_filter,
-                                        shift_state=self._shift_state("err", err_in.device), unpool=(pool.act_in, POOL_TIES))
-            if fused is not None:
-                pool.bwd_done = fused[0]
-                return fused[0], fused[2]
-        fused = _conv_requant_fused(True, err_in, self.weight, self.stride, self.padding, ERROR_ROUND_METHOD, rand,
-                                    False, self.err_exp_in, self._wexp(), relu_mask=mask, forward_filter=forward_filter,
-                                    shift_state=self._shift_state("err", err_in.device))
-        if fused is not None:
-            err_out, _, new_exp = fused
-            return err_out, new_exp
-        am = ops.new_scalar_u32(err_in.device)
-        dx = ops.conv2d_dgrad(err_in, self.weight, self.stride, self.padding, f32_epilogue=F32_EPILOGUE, absmax=am,
-                              forward_filter=forward_filter)
-        err_out, _, new_exp = _requant(dx, BITWIDTH, ERROR_ROUND_METHOD, am, rand,
-                                       exp_a=self.err_exp_in, exp_b=self._wexp(), want_exp=True)
-        if mask is not None:
-            err_out = ops.relu_bwd(mask, err_out)
-        return err_out, new_exp
-
-    def _forward_filter(self, w16):
-        """Kernel-ready copy of the (channel-padded) filter for the forward pass.  Made when the weight tensor was
-        replaced or modified through torch; the fused weight update keeps it in step with its own changes."""
-        key = (self.weight.data_ptr(), self.weight._version, tuple(self.act16.shape))
-        if getattr(self, "_wprep_key", None) != key:
-            N, H, W, _ = self.act16.shape
-            self._wprep = ops.conv_filter_prepare(w16, N, H, W, self.stride, self.padding)
-            self._wprep_key = key
-        return self._wprep
-
-    def _wgrad_workspace(self, err_in):
-        from . import _lib
-        N, H, W, C16 = self.act16.shape
-        K, R, S, _ = self.weight.shape
-        return ops.scratch(_lib.lib().niti_conv2d_i8_wgrad_workspace(N, H, W, C16, K, R, S, self.padding), err_in.device)
+        states = self.__dict__.get("_shift_states")
+        if states is None:
+            states = self.__dict__["_shift_states"] = {}
+        key = (which, device)
+        state = states.get(key)
+        if state is None:
+            state = states[key] = torch.zeros(1, dtype=torch.int32, device=device)
+        return state
 
     def _synced_filter(self):
         """The forward filter copy if it matches the weights as they are now (then the update maintains it)."""
-        key = getattr(self, "_wprep_key", None)
-        if key is None or self._wprep is None or key[:2] != (self.weight.data_ptr(), self.weight._version):
-            self._wprep_key = None
+        d = self.__dict__
+        key, weight = d.get("_wprep_key"), self.weight
+        if key is None or key[0] != weight.data_ptr() or key[1] != weight._version:
+            d["_wprep_key"] = None
             return None
-        return self._wprep
-
-    def _wgrad_update_fused(self, err_in, grad_rand):
-        """Weight gradient, grad_calc and the weight update as one call into the library (no int32 gradient in
-        memory unless KEEP_INT32_GRAD).  False when the call needs the separate steps."""
-        method = _method_name(GRAD_ROUND_METHOD)
-        if not FUSE_CONV_REQUANT or method == "sto" or grad_rand is not None or not self.weight.is_contiguous():
-            return False
-        N, H, W, C16 = self.act16.shape
-        K, R, S, C = self.weight.shape
-        if ops.wgrad_update_sync_words(N, H, W, C16, K, R, S, self.stride, self.padding) == 0:
-            return False
-        dev = err_in.device
-        key = ("wgrad_update", tuple(self.act16.shape), tuple(self.weight.shape))
-        if key in _fused_refused:
-            return False
-        from ._lib import NitiError
-        self.grad_exp = torch.empty(1, dtype=torch.int32, device=dev)
-        try:
-            return self._wgrad_update_call(err_in, method, dev, C)
-        except NitiError as e:
-            if "do not fit" not in str(e):
-                raise
-            _fused_refused.add(key)     # a device too small for the finishing kernel's grid: separate steps from now on
-            return False
-
-    def _wgrad_update_call(self, err_in, method, dev, C):
-        self.grad, dw, self.grad_shift, _ = ops.conv2d_wgrad_update(
-            self.act16, err_in, self.weight, self.stride, self.padding, f32_epilogue=F32_EPILOGUE and not self.first_layer,
-            mu=GRAD_BITWIDTH, method=method, div_mode=DIV_MODE, bw_mode=BW_MODE, want_grad=self.keep_grad,
-            want_dw=KEEP_INT32_GRAD, exp_a=_exp_tensor(self.err_exp, dev), exp_b=_exp_tensor(self.act_in_exp, dev),
-            exp_out=self.grad_exp, workspace=self._wgrad_workspace(err_in), prepared_filter=self._synced_filter(),
-            shift_out=self._shift_state("grad", dev), shift_hint=True)
-        self.grad_int32acc = None if dw is None else (dw if dw.shape[3] == C else dw[..., :C].contiguous())
-        return True
+        return d["_wprep"]
 
 
 class TiLinear(UpdateWeight):
@@ -580,170 +492,92 @@ class TiLinear(UpdateWeight):
         self.loss_grad = None       # (targets, loss gradient) left by that forward
         self._dropped = None        # dropout mask the last forward applied itself
 
-    def _head(self, which, M, methods, rands):
-        """The pass runs as one of the classifier-head kernels (dropout, loss gradient, both backward products and the
-        update folded in) when the shape is inside them and no rounding needs random input."""
-        O, F = self.weight.shape
-        return (FUSE_CONV_REQUANT and all(r is None for r in rands) and all(_method_name(m) != "sto" for m in methods)
-                and self.weight.is_contiguous() and ("head", which, M, O, F) not in _fused_refused
-                and ops.head_sync_words(which, M, O, F) > 0)
-
     def _rng_state(self, dev):
         return self.rng.state(dev) if self.rng is not None else ops.rng_state(dev)
 
-    def _one_launch(self, which, M, fn, rand):
-        """The pass runs as one of the library's kernels for few output features (operands read as stored,
-        requantisation folded in) when the shape is inside them and the rounding needs no random input."""
-        O, F = self.weight.shape
-        return (FUSE_CONV_REQUANT and rand is None and _method_name(fn) != "sto" and self.weight.is_contiguous()
-                and (which, M, O, F) not in _fused_refused and ops.fc_sync_words(which, M, O, F) > 0)
-
-    def _wide(self, which, M):
-        """The pass runs as one of the library's any-width kernels (operands as stored, requantisation folded in, random
-        rounding included) when the shape is inside them and the layer has more than a few output features."""
-        O, F = self.weight.shape
-        return (FUSE_CONV_REQUANT and O > 16 and self.weight.is_contiguous() and ("wide", which, M, O, F) not in _fused_refused
-                and ops.linear_sync_words(which, M, O, F) > 0)
-
-    @staticmethod
-    def _sto_rand(fn, rand, shape, dev):
-        """Random integers for a stochastic rounding of a tensor of ``shape`` (the caller's, or drawn here)."""
-        if _method_name(fn) != "sto":
-            return None
-        return rand if rand is not None else torch.randint(0, 2 ** 31 - 1, shape, dtype=torch.int32, device=dev)
-
-    def _try(self, which, M, call):
-        """``call()``, or None when the device turned out too small to hold the kernel's grid at once."""
-        from ._lib import NitiError
-        try:
-            return call()
-        except NitiError as e:
-            if "do not fit" not in str(e):
-                raise
-            _fused_refused.add((which, M) + tuple(self.weight.shape))
-            return None
-
     def forward(self, input, rand=None):
-        self.act_in = input
+        d = self.__dict__
+        d["act_in"] = input
         act_in, exp_in = input
-        act_in = act_in.contiguous()
+        if not act_in.is_contiguous():
+            act_in = act_in.contiguous()
         dev = act_in.device
-        drop, self._dropped, self.loss_grad = self.drop_below, None, None
+        weight = self.weight if self.weight.is_contiguous() else self.weight.contiguous()
+        host = _lib.host()
+        method, div, bw = _method_code(ACT_ROUND_METHOD), _lib.DIV[DIV_MODE], _lib.BW[BW_MODE]
+        drop = self.drop_below
+        d["_dropped"] = d["loss_grad"] = None
         pending = drop is not None and drop.pending is not None and drop.pending[0] is input[0]
-        want_loss, self.next_target = self.next_target, None
-        if (pending or want_loss is not None) and self._head("forward", act_in.shape[0], (ACT_ROUND_METHOD,), (rand,)):
-            M = act_in.shape[0]
-            exp_out = torch.empty(1, dtype=torch.int32, device=dev)
+        want_loss, d["next_target"] = self.next_target, None
+        # the classifier-head kernel: dropout and loss gradient folded in, where no rounding needs random input
+        if (pending or want_loss is not None) and FUSE_CONV_REQUANT and rand is None and method != _STO:
+            target, loss_rand = want_loss if want_loss is not None else (None, None)
             given = drop.pending[1] if pending else None
-            draws = (pending and given is None) or (want_loss is not None and want_loss[1] is None)
-            done = self._try("head-forward", M, lambda: ops.head_forward(
-                act_in, self.weight, BITWIDTH, _method_name(ACT_ROUND_METHOD), DIV_MODE, BW_MODE,
-                dropout=None if not pending else ("draw" if given is None else "given"), drop_mask=given,
-                rng=self._rng_state(dev) if draws else None, exp_bias=1 if pending else 0,
-                target=want_loss[0] if want_loss is not None else None, loss_rand=want_loss[1] if want_loss is not None else None,
-                exp_a=_exp_tensor(exp_in, dev), exp_b=self._wexp(), exp_out=exp_out))
+            draws = (pending and given is None) or (want_loss is not None and loss_rand is None)
+            done = host.head_forward(act_in, weight, BITWIDTH, method, div, bw, 0 if not pending else (2 if given is None else 1), given,
+                                     self._rng_state(dev) if draws else None, 1 if pending else 0, target, loss_rand,
+                                     _exp_tensor(exp_in, dev), self._wexp())
             if done is not None:
                 if pending:
-                    drop.drop_mask = self._dropped = done[1]
-                    drop.pending = None
+                    drop.__dict__["drop_mask"] = d["_dropped"] = done[2]
+                    drop.__dict__["pending"] = None
                 if want_loss is not None:
-                    self.loss_grad = (want_loss[0], done[2])
-                return done[0], exp_out
+                    d["loss_grad"] = (target, done[3])
+                return done[0], done[1]
         if pending:   # the dropout left its work to this layer, which cannot take it: do it now
             act_in, exp_in = drop.apply_now(act_in, exp_in)
-            self.act_in = (act_in, exp_in)
-        if self._one_launch("forward", act_in.shape[0], ACT_ROUND_METHOD, rand):
-            exp_out = torch.empty(1, dtype=torch.int32, device=dev)
-            act_out, _, _ = ops.fc_fwd_requant(act_in, self.weight, BITWIDTH, _method_name(ACT_ROUND_METHOD), DIV_MODE, BW_MODE,
-                                               exp_a=_exp_tensor(exp_in, dev), exp_b=self._wexp(), exp_out=exp_out)
-            return act_out, exp_out
-        if self._wide("forward", act_in.shape[0]):
-            exp_out = torch.empty(1, dtype=torch.int32, device=dev)
-            M, O = act_in.shape[0], self.weight.shape[0]
-            done = self._try("wide-forward", M, lambda: ops.linear_fwd_requant(
-                act_in, self.weight, BITWIDTH, _method_name(ACT_ROUND_METHOD), DIV_MODE, BW_MODE,
-                rand=self._sto_rand(ACT_ROUND_METHOD, rand, (M, O), dev), exp_a=_exp_tensor(exp_in, dev), exp_b=self._wexp(),
-                exp_out=exp_out))
-            if done is not None:
-                return done[0], exp_out
-        am = ops.new_scalar_u32(dev)
-        acc = ops.gemm(act_in, self.weight, trans_b=True, absmax=am)            # act @ W^T, W read as stored
-        act_out, _, exp_out = _requant(acc, BITWIDTH, ACT_ROUND_METHOD, am, rand,
-                                       exp_a=_exp_tensor(exp_in, dev), exp_b=self._wexp(), want_exp=True)
-        return act_out, exp_out
+            d["act_in"] = (act_in, exp_in)
+        rand = _sto_rand(method, rand, (act_in.shape[0], weight.shape[0]), dev)
+        return host.linear_forward(FUSE_CONV_REQUANT, act_in, weight, BITWIDTH, method, div, bw, _exp_tensor(exp_in, dev), self._wexp(), rand)
 
     def backward(self, input, rand=None, grad_rand=None):
+        d = self.__dict__
         err_in, err_exp = input
-        err_in = err_in.contiguous()
+        if not err_in.is_contiguous():
+            err_in = err_in.contiguous()
         dev = err_in.device
-        act, self.act_in_exp = self.act_in
-        act = act.contiguous()
-        M = err_in.shape[0]
-        self.err_exp_in = _exp_tensor(err_exp, dev)
+        act, d["act_in_exp"] = d["act_in"]
+        if not act.is_contiguous():
+            act = act.contiguous()
+        weight = self.weight
+        if not weight.is_contiguous():
+            weight = self.weight = weight.contiguous()
+        host = _lib.host()
+        e_method, g_method = _method_code(ERROR_ROUND_METHOD), _method_code(GRAD_ROUND_METHOD)
+        div, bw = _lib.DIV[DIV_MODE], _lib.BW[BW_MODE]
+        d["err_exp_in"] = _exp_tensor(err_exp, dev)
         mask = self._dropped     # the forward pass read ``act`` through this mask: act_in is the tensor in front of the dropout
-        if not KEEP_INT32_GRAD and self._head("backward", M, (ERROR_ROUND_METHOD, GRAD_ROUND_METHOD), (rand, grad_rand)):
-            exps = torch.empty(2, dtype=torch.int32, device=dev)
+        if not KEEP_INT32_GRAD and FUSE_CONV_REQUANT and rand is None and grad_rand is None and e_method != _STO and g_method != _STO:
             # the 2x2 max-pool whose flattened output this layer read (TiNet.fuse): its backward pass in the same launch
-            pool = self.__dict__.get("pool_below")
-            unpool = None
-            if (pool is not None and getattr(pool, "act_out", None) is not None and pool.act_out.data_ptr() == act.data_ptr()
-                    and pool.act_out.numel() == act.numel() and pool.act_in.dim() == 4 and pool.act_in.is_contiguous()
-                    and pool.act_in.dtype == torch.int8 and pool.act_in.shape[3] % 64 == 0):
-                unpool = (pool.act_in, POOL_TIES, pool.relu_below)
-            done = self._try("head-backward", M, lambda: ops.head_backward(
-                err_in, act, self.weight, BITWIDTH, _method_name(ERROR_ROUND_METHOD), GRAD_BITWIDTH, _method_name(GRAD_ROUND_METHOD),
-                DIV_MODE, BW_MODE, drop_mask=mask, want_grad=self.keep_grad, exp_err=self.err_exp_in, exp_w=self._wexp(),
-                exp_act=_exp_tensor(self.act_in_exp, dev), exp_act_bias=1 if mask is not None else 0,
-                err_exp_out=exps[0:1], grad_exp_out=exps[1:2], unpool=unpool))
+            pool = d.get("pool_below")
+            pool_in = None
+            if pool is not None:
+                pooled, whole = pool.__dict__.get("act_out"), pool.__dict__.get("act_in")
+                if (pooled is not None and pooled.data_ptr() == act.data_ptr() and pooled.numel() == act.numel() and whole.dim() == 4
+                        and whole.is_contiguous() and whole.dtype == torch.int8 and whole.shape[3] % 64 == 0):
+                    pool_in = whole
+            done = host.head_backward(
+                err_in, act, weight, BITWIDTH, e_method, GRAD_BITWIDTH, g_method, div, bw, mask, self.keep_grad, d["err_exp_in"],
+                self._wexp(), _exp_tensor(d["act_in_exp"], dev), 1 if mask is not None else 0, pool_in,
+                _lib.TIES[POOL_TIES] | (_lib.POOL_BWD_RELU if pool_in is not None and pool.relu_below else 0))
             if done is not None:
-                self.err_exp, self.grad_exp = exps[0:1], exps[1:2]
-                self.grad, self.grad_shift, self.grad_int32acc = done[1], done[3], None
+                err_out, d["grad"], d["grad_shift"], d["err_exp"], d["grad_exp"], routed = done
+                d["grad_int32acc"] = None
                 if mask is not None:
-                    self.drop_below.bwd_done = done[0]     # masked already
-                if unpool is not None:
-                    pool.bwd_routed = (done[0], done[5])
-                return done[0], self.err_exp
+                    self.drop_below.__dict__["bwd_done"] = err_out     # masked already
+                if routed is not None:
+                    pool.__dict__["bwd_routed"] = (err_out, routed)
+                return err_out, d["err_exp"]
         if mask is not None:     # the separate passes want the masked activations and their exponent
-            act, self.act_in_exp = ops.mask_features(act, mask, _exp_tensor(self.act_in_exp, dev), 1)
-        done = None
-        if self._one_launch("dgrad", M, ERROR_ROUND_METHOD, rand):
-            new_exp = torch.empty(1, dtype=torch.int32, device=dev)
-            done = self._try("dgrad", M, lambda: ops.fc_dgrad_requant(
-                err_in, self.weight, BITWIDTH, _method_name(ERROR_ROUND_METHOD), DIV_MODE, BW_MODE,
-                exp_a=self.err_exp_in, exp_b=self._wexp(), exp_out=new_exp))
-        if done is None and self._wide("dgrad", M):
-            new_exp = torch.empty(1, dtype=torch.int32, device=dev)
-            done = self._try("wide-dgrad", M, lambda: ops.linear_dgrad_requant(
-                err_in, self.weight, BITWIDTH, _method_name(ERROR_ROUND_METHOD), DIV_MODE, BW_MODE,
-                rand=self._sto_rand(ERROR_ROUND_METHOD, rand, (M, self.weight.shape[1]), dev), exp_a=self.err_exp_in,
-                exp_b=self._wexp(), exp_out=new_exp))
-        if done is not None:
-            err_out, self.err_exp = done[0], new_exp
-        else:
-            am = ops.new_scalar_u32(dev)
-            dx = ops.gemm(err_in, self.weight, absmax=am)                             # err @ W
-            err_out, _, self.err_exp = _requant(dx, BITWIDTH, ERROR_ROUND_METHOD, am, rand,
-                                                exp_a=self.err_exp_in, exp_b=self._wexp(), want_exp=True)
-        done = None
-        if not KEEP_INT32_GRAD and self._one_launch("wgrad", M, GRAD_ROUND_METHOD, grad_rand):
-            self.grad_exp = torch.empty(1, dtype=torch.int32, device=dev)
-            done = self._try("wgrad", M, lambda: ops.fc_wgrad_update(
-                err_in, act, self.weight, GRAD_BITWIDTH, _method_name(GRAD_ROUND_METHOD), DIV_MODE, BW_MODE,
-                want_grad=self.keep_grad, exp_a=_exp_tensor(self.err_exp, dev), exp_b=_exp_tensor(self.act_in_exp, dev),
-                exp_out=self.grad_exp))
-        if done is None and not KEEP_INT32_GRAD and self._wide("wgrad", M):
-            self.grad_exp = torch.empty(1, dtype=torch.int32, device=dev)
-            done = self._try("wide-wgrad", M, lambda: ops.linear_wgrad_update(
-                err_in, act, self.weight, GRAD_BITWIDTH, _method_name(GRAD_ROUND_METHOD), DIV_MODE, BW_MODE,
-                rand=self._sto_rand(GRAD_ROUND_METHOD, grad_rand, tuple(self.weight.shape), dev), want_grad=self.keep_grad,
-                exp_a=_exp_tensor(self.err_exp, dev), exp_b=_exp_tensor(self.act_in_exp, dev), exp_out=self.grad_exp))
-        if done is not None:
-            self.grad, self.grad_shift, self.grad_int32acc = done[0], done[1], None
-        else:
-            amg = ops.new_scalar_u32(dev)
-            self.grad_int32acc = ops.gemm(err_in, act, trans_a=True, absmax=amg)     # err^T @ act
-            self.weight_update(amg, grad_rand)
-        return err_out, self.err_exp
+            act, d["act_in_exp"] = ops.mask_features(act, mask, _exp_tensor(d["act_in_exp"], dev), 1)
+        rand = _sto_rand(e_method, rand, tuple(act.shape), dev)
+        err_out, d["err_exp"] = host.linear_dgrad(FUSE_CONV_REQUANT, err_in, weight, BITWIDTH, e_method, div, bw, d["err_exp_in"],
+                                                  self._wexp(), rand)
+        grad_rand = _sto_rand(g_method, grad_rand, tuple(weight.shape), dev)
+        d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"] = host.linear_wgrad_update(
+            FUSE_CONV_REQUANT, err_in, act, weight, GRAD_BITWIDTH, g_method, div, bw, self.keep_grad, KEEP_INT32_GRAD, d["err_exp"],
+            _exp_tensor(d["act_in_exp"], dev), grad_rand)
+        return err_out, d["err_exp"]
 
 
 class TiReLU(Module):
@@ -756,7 +590,7 @@ class TiReLU(Module):
         self.bwd_folded = False
 
     def forward(self, input):
-        self.act_in = input
+        self.__dict__["act_in"] = input      # a plain attribute: Module.__setattr__ looks for parameters first
         act_in, exp_in = input
         if self.fused:
             return input
@@ -784,25 +618,27 @@ class TiMaxpool2d(Module):
         self.bwd_routed = None      # (error tensor, routed result) left by the classifier behind this layer
 
     def forward(self, input):
-        self.act_in, exp_in = input
-        preset, self.preset = self.preset, None
-        if preset is not None and preset[0] is self.act_in:
-            self.act_out = preset[1]
-            return self.act_out, exp_in
-        self.act_in = self.act_in.contiguous()
-        self.act_out = ops.maxpool_fwd(self.act_in, self.kernel_size, self.stride, self.padding)
-        return self.act_out, exp_in
+        d = self.__dict__       # plain attributes: Module.__setattr__ looks for parameters first
+        act_in, exp_in = input
+        preset, d["preset"] = d["preset"], None
+        if preset is not None and preset[0] is act_in:
+            d["act_in"], d["act_out"] = act_in, preset[1]
+            return preset[1], exp_in
+        d["act_in"] = act_in = act_in.contiguous()
+        d["act_out"] = _lib.host().maxpool_fwd(act_in, self.kernel_size, self.stride, self.padding)
+        return d["act_out"], exp_in
 
     def backward(self, input):
         err_in, err_exp = input
-        done, self.bwd_done = self.bwd_done, None
+        d = self.__dict__
+        done, d["bwd_done"] = d["bwd_done"], None
         if done is not None and done is err_in:
             return input        # the data gradient behind this layer wrote its result through this pooling already
-        routed, self.bwd_routed = self.bwd_routed, None
+        routed, d["bwd_routed"] = d["bwd_routed"], None
         if routed is not None and routed[0].data_ptr() == err_in.data_ptr() and routed[0].numel() == err_in.numel():
             return routed[1], err_exp     # the classifier's backward launch has run this pass
-        err_out = ops.maxpool_bwd(self.act_out, err_in.contiguous(), self.act_in, self.kernel_size, self.stride,
-                                  self.padding, POOL_TIES, relu=self.relu_below)
+        err_out = _lib.host().maxpool_bwd(d["act_out"], err_in.contiguous(), d["act_in"], self.kernel_size, self.stride, self.padding,
+                                          _lib.TIES[POOL_TIES] | (_lib.POOL_BWD_RELU if self.relu_below else 0))
         return err_out, err_exp
 
 
@@ -810,7 +646,7 @@ class TiFlat(Module):
     """ti_torch.py:318-332."""
 
     def forward(self, input):
-        self.act_in = input
+        self.__dict__["act_in"] = input
         act_in, exp_in = input
         return act_in.view(-1, act_in.nelement() // act_in.size(0)), exp_in
 
@@ -838,10 +674,10 @@ class TiDropout(Module):
                 mask = mask.to(act_in.device)
             if (self.head is not None and FUSE_CONV_REQUANT and act_in.is_cuda and act_in.dtype == torch.int8 and act_in.dim() == 2
                     and act_in.is_contiguous() and (mask is None or (mask.dtype == torch.int8 and mask.is_contiguous()))):
-                self.pending = (act_in, mask)
+                self.__dict__["pending"] = (act_in, mask)
                 return input
             return self.apply_now(act_in, exp_in, mask)
-        self.pending = None
+        self.__dict__["pending"] = None
         return input
 
     def apply_now(self, act_in, exp_in, mask=None):
@@ -862,7 +698,7 @@ class TiDropout(Module):
 
     def backward(self, input):
         err_in, err_exp = input
-        done, self.bwd_done = self.bwd_done, None
+        done, self.__dict__["bwd_done"] = self.bwd_done, None
         if done is not None and done is err_in:
             return input        # the layer behind this one masked its data gradient already
         if self._one_launch(err_in):
