@@ -292,16 +292,11 @@ int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err, int8_t* w,
  * (pytorch/int8mm-extension/int8mm.cpp:9-14, int8mm_kernel.cu:8-34):
  *   c[m,n] = sum_k opA[m,k] * opB[k,n],  c row-major with leading dimension n.
  * trans_a == 0: a is [m,k] row-major; 1: a is [k,m].  trans_b == 0: b is [k,n]; 1: b is [n,k].
- * Operands are read as stored, no operand copy: (trans_a=0, trans_b=1) with k % 16 == 0;
- * trans_b=0 - the form the reference's extension receives (trans_a=0) and the one with both
- * reduction indices slow (trans_a=1, m % 16 == 0) - with n % 32 == 0 and k % 32 == 0, through
- * transposing LDS reads; (trans_a=1, trans_b=1) with m % 32 == 0 and k % 32 == 0 the same way
- * (it fills the [n,m] buffer behind the transposed view that int8_mm returns, from lhs and rhs
- * as the reference passes them).  One launch - except that the forms with trans_a == trans_b
- * whose result has few tiles and whose reduction is long (n, k multiples of 128; in the doubly
- * transposed form m, k) split the reduction over workgroups: the int32 parts go to the workspace
- * and a second small launch adds them.  Other shapes first re-lay the operand(s) into the
- * workspace.  niti_gemm_i8_workspace() reports the bytes either way (0 when none are needed).
+ * Operands are read as stored, whatever the extents and the alignment, in one launch - except that the forms with
+ * trans_a == trans_b whose result has few tiles and whose reduction is very long (n, k multiples of 128; in the doubly
+ * transposed form m, k) split the reduction over workgroups: the int32 parts go to the workspace and a second small
+ * launch adds them.  Matrices of about 2 GiB and more are re-laid into the workspace first.
+ * niti_gemm_i8_workspace() reports the bytes a call may need (0 when none).
  */
 size_t niti_gemm_i8_workspace(int trans_a, int trans_b, int m, int n, int k);
 int niti_gemm_i8(int trans_a, int trans_b, const int8_t* a, const int8_t* b, int32_t* c, int m, int n, int k,
@@ -419,9 +414,9 @@ int niti_fc_i8_wgrad_update(const int8_t* err, const int8_t* act, int8_t* w, int
  * act [M][F], w [O][F], err [M][O], int8; no operand is re-laid and no int32 product is written to memory.
  * Rounding: NITI_ROUND_NEAREST, NITI_ROUND_PSEUDO_STOCHASTIC, or NITI_ROUND_STOCHASTIC with `rand` (one int32 per
  * OUTPUT element - [M][O], [M][F], [O][F] - low `shift` bits used, as in niti_requant_i32_i8; NULL otherwise).
- * Shapes: forward F % 16 == 0, O % 4 == 0; dgrad O % 32 == 0, F % 32 == 0, O <= 4096; wgrad O % 16 == 0, F % 16 == 0;
- * 16-byte aligned operands.  niti_linear_i8_sync_words returns 0 for shapes outside that or whose workgroups the
- * current device does not hold at once (then use niti_gemm_i8 + niti_requant_i32_i8 / niti_grad_update_i8).
+ * Any shape; operands of forward F % 16 == 0, O % 4 == 0, dgrad O % 32 == 0, F % 32 == 0 and wgrad O % 16 == 0, F % 16 == 0
+ * must be 16-byte aligned, others need no alignment.  niti_linear_i8_sync_words returns 0 for results whose workgroups the
+ * current device does not hold at once (about 8 M values; then use niti_gemm_i8 + niti_requant_i32_i8 / niti_grad_update_i8).
  * sync, shift_out, exp_* as in niti_fc_i8_*.
  */
 size_t niti_linear_i8_sync_words(int which, int M, int O, int F);

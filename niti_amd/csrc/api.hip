@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "gemm_any.h"
 
 namespace niti {
 namespace {
@@ -588,7 +589,7 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
 
 extern "C" size_t niti_gemm_i8_workspace(int trans_a, int trans_b, int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  if (gemm_kmajor_shape(trans_a, trans_b, m, n, k)) return gemm_kmajor_workspace(trans_a, trans_b, m, n, k);   // read as stored; partial sums of a split reduction
+  if (gemm_kmajor_shape(trans_a, trans_b, m, n, k) && gemm_any_shape(m, n, k)) return gemm_lines_workspace(trans_a, trans_b, m, n, k);   // read as stored; partial sums of a split reduction
   const size_t kp = static_cast<size_t>(round16(k));
   size_t bytes = 0;
   if (trans_a || k % 16 != 0) bytes += round256(static_cast<size_t>(m) * kp);
@@ -607,11 +608,20 @@ extern "C" int niti_gemm_i8(int trans_a, int trans_b, const int8_t* a, const int
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)))
     return fail(NITI_ERR_WORKSPACE, "gemm: needs %zu workspace bytes (16-byte aligned), got %zu", need, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // reduction index slow in b (and in a): one launch, both operands read as stored
-  if (gemm_kmajor_shape(trans_a, trans_b, m, n, k)) {
-    if (!aligned16(a) || !aligned16(b)) return fail(NITI_ERR_INVALID_ARG, "gemm: operands must be 16-byte aligned");
-    return launch_gemm_kmajor(trans_a, trans_b, a, b, c, m, n, k, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
+  // whole-line kernel: few, long rows of tiles (gemm_lines.hip says where it is the faster one)
+  if (gemm_lines_shape(trans_a, trans_b, m, n, k) && aligned16(a) && aligned16(b))
+    return launch_gemm_lines(trans_b, a, b, c, m, n, k, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
+  // Operands with the reduction index fast in both and 16-byte rows are implicit-GEMM tiles as they stand; on results that
+  // fill the chip that kernel's LDS-DMA ring is the faster one (4000 x 2000 x 8192 85 us against 97)
+  const bool direct = trans_a == 0 && trans_b != 0 && k % 16 == 0 && aligned16(a) && aligned16(b) && gemm_any_large(m, n);
+  if (!direct && gemm_any_shape(m, n, k)) {
+    AnyArgs g{a, b, m, n, k};
+    g.c = c;
+    g.absmax = absmax;
+    g.roundtrip = (flags & NITI_EPI_F32_ROUNDTRIP) != 0 ? 1 : 0;
+    return launch_gemm_any(trans_a, trans_b, g, s);
   }
+  // that, and matrices of about 2 GiB and more: a 1 x 1 convolution over operands re-laid with the reduction index fast
   const int kp = round16(k);
   int8_t* ws = static_cast<int8_t*>(workspace);
   const int8_t* a_use = a;  // [m][kp]
@@ -640,19 +650,5 @@ extern "C" int niti_gemm_i8(int trans_a, int trans_b, const int8_t* a, const int
   if (!aligned16(a_use) || !aligned16(b_use)) return fail(NITI_ERR_INVALID_ARG, "gemm: operands must be 16-byte aligned");
   // a 1x1 convolution over an m x 1 x 1 "image" with kp channels and n filters
   ConvProblem p{a_use, b_use, c, absmax, m, 1, 1, kp, n, 1, 1, 1, 0, n, n, n, 1, 1, flags};
-  // few output tiles and a long reduction (a fully connected layer on a batch): split the reduction over
-  // workgroups that add into the zeroed output (integer addition: any split gives the same bits), then one
-  // pass for the range
-  const long long tiles = static_cast<long long>((m + 127) / 128) * ((n + 127) / 128);
-  const int split = tiles >= 128 ? 1 : pick_split(tiles, (kp + 63) / 64);
-  if (split > 1) {
-    const int64_t nout = static_cast<int64_t>(m) * n;
-    if ((st = launch_fill_u32(reinterpret_cast<uint32_t*>(c), nout, 0u, s)) != NITI_OK) return st;
-    p.absmax = nullptr;
-    p.split_k = split;
-    if ((st = launch_conv_igemm(p, s)) != NITI_OK) return st;
-    if (absmax == nullptr && !(flags & NITI_EPI_F32_ROUNDTRIP)) return NITI_OK;
-    return launch_post_i32(c, nout, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, s);
-  }
   return launch_conv_igemm(p, s);
 }

@@ -20,14 +20,14 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm_any.h"
+#include "grid_range.h"
 #include "lds_asm.h"
 #include "nn_lines.h"
 #include "requant_math.h"
 
 namespace niti {
 namespace {
-
-constexpr int kSlot0 = 16;   // sync words: 0 range out, 1 wait gave up, 16.. one slot per workgroup
 
 struct FcwArgs {
   const int8_t* act;     // [M][F]
@@ -47,52 +47,6 @@ struct FcwArgs {
   const int32_t* exp_b;
   int32_t* exp_out;
 };
-
-__device__ inline int round_any(int x, int shift, int method, bool trunc, int u) {
-  if (shift < 1) return wrap_to_i8(x);
-  if (method == NITI_ROUND_STOCHASTIC) return round_one<NITI_ROUND_STOCHASTIC>(x, shift, trunc, u & ((1 << shift) - 1));
-  return method == NITI_ROUND_PSEUDO_STOCHASTIC ? round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(x, shift, trunc)
-                                                : round_one32<NITI_ROUND_NEAREST>(x, shift, trunc);
-}
-
-__device__ inline void write_scalars(const FcwArgs& a, uint32_t gmax, int shift) {
-  const int sh = shift > 0 ? shift : 0;
-  a.sync[0] = gmax;
-  if (a.shift_out != nullptr) *a.shift_out = sh;
-  if (a.exp_out != nullptr) *a.exp_out = sh + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
-}
-
-// Called by wavefront 0 of every workgroup with the workgroup's largest magnitude: the largest over the grid.
-__device__ inline uint32_t exchange_range(const FcwArgs& a, uint32_t bmax) {
-  const int lane = threadIdx.x & 63;
-  const int nb = gridDim.x * gridDim.y;
-  const int b = blockIdx.y * gridDim.x + blockIdx.x;
-  uint32_t* const slots = a.sync + kSlot0;
-  if (lane == 0) __hip_atomic_store(slot_word(slots, b), bmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
-  return g != 0u ? g - 1u : 0u;
-}
-
-// the workgroup's shift from every wavefront's largest magnitude: wmax[] holds one word per wavefront, gshare the result
-template <int NWAVES>
-__device__ inline int grid_shift(const FcwArgs& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare) {
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  lmax = wave_max_u32(lmax);
-  if (lane == 0) wmax[wave] = lmax;
-  __syncthreads();
-  if (wave == 0) {
-    uint32_t b = lane < NWAVES ? wmax[lane] : 0u;
-    b = wave_max_u32(b);
-    const uint32_t g = exchange_range(a, b);
-    if (lane == 0) *gshare = g;
-  }
-  __syncthreads();
-  const uint32_t gmax = *gshare;
-  const int shift = bitwidth_of(gmax, a.bw_mode) - a.target_bits;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) write_scalars(a, gmax, shift);
-  return shift;
-}
 
 // barrier that the compiler also treats as a fence for the hand-written LDS reads around it
 __device__ inline void sync_mem() {
@@ -174,11 +128,10 @@ __global__ __launch_bounds__(1024) void fcw_fwd_kernel(const FcwArgs a) {
   const long long at = static_cast<long long>(m) * a.O + ob;
   v4i u = zero;
   if (a.method == NITI_ROUND_STOCHASTIC) u = *reinterpret_cast<const v4i*>(a.rand + at);
-  int r[4];
+  v4i r = round4_any(fin, shift, a.method, trunc, u);
+  if (relu) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    r[i] = round_any(fin[i], shift, a.method, trunc, u[i]);
-    if (relu && r[i] < 0) r[i] = 0;
+    for (int i = 0; i < 4; ++i) r[i] = max(r[i], 0);
   }
   *reinterpret_cast<uint32_t*>(a.out8 + at) = pack4_i8(r[0], r[1], r[2], r[3]);
 }
@@ -298,11 +251,10 @@ __global__ __launch_bounds__(512) void fcw_fwd_lds_kernel(const FcwArgs a) {
   const long long at = static_cast<long long>(m) * a.O + ob;
   v4i u = zero;
   if (a.method == NITI_ROUND_STOCHASTIC) u = *reinterpret_cast<const v4i*>(a.rand + at);
-  int r[4];
+  v4i r = round4_any(fin, shift, a.method, trunc, u);
+  if (relu) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    r[i] = round_any(fin[i], shift, a.method, trunc, u[i]);
-    if (relu && r[i] < 0) r[i] = 0;
+    for (int i = 0; i < 4; ++i) r[i] = max(r[i], 0);
   }
   *reinterpret_cast<uint32_t*>(a.out8 + at) = pack4_i8(r[0], r[1], r[2], r[3]);
 }
@@ -381,9 +333,7 @@ __global__ __launch_bounds__(512) void fcw_dgrad_kernel(const FcwArgs a) {
     const long long at = static_cast<long long>(m) * a.F + f0 + 8 * g + 4 * lk;
     v4i u = zero;
     if (a.method == NITI_ROUND_STOCHASTIC) u = *reinterpret_cast<const v4i*>(a.rand + at);
-    int r[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = round_any(acc[4 * g + e], shift, a.method, trunc, u[e]);
+    const v4i r = round4_any(v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]}, shift, a.method, trunc, u);
     *reinterpret_cast<uint32_t*>(a.out8 + at) = pack4_i8(r[0], r[1], r[2], r[3]);
   }
 }
@@ -440,9 +390,7 @@ __global__ __launch_bounds__(512) void fcw_dgrad_lds_kernel(const FcwArgs a) {
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const v4i sum = *reinterpret_cast<const v4i*>(patch + row * kPitch + (q * 64 + p16 * 4) * 4);
-    int r[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = round_any(sum[e], shift, a.method, trunc, u[q][e]);
+    const v4i r = round4_any(sum, shift, a.method, trunc, u[q]);
     *reinterpret_cast<uint32_t*>(a.out8 + at + q * 64) = pack4_i8(r[0], r[1], r[2], r[3]);
   }
 }
@@ -558,10 +506,10 @@ __global__ __launch_bounds__(512) void fcw_wgrad_kernel(const FcwArgs a) {
         const long long at = static_cast<long long>(o) * a.F + f;
         const uint32_t wold = *reinterpret_cast<const uint32_t*>(a.w + at);
         const v4i u = *reinterpret_cast<const v4i*>(a.rand + at);
-        int r[4], wn[4];
+        const v4i r = round4_any(v4i{fin[t][4 * q], fin[t][4 * q + 1], fin[t][4 * q + 2], fin[t][4 * q + 3]}, shift, NITI_ROUND_STOCHASTIC, trunc, u);
+        int wn[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          r[e] = round_any(fin[t][4 * q + e], shift, NITI_ROUND_STOCHASTIC, trunc, u[e]);
           const int wo = static_cast<int>(static_cast<int8_t>((wold >> (8 * e)) & 0xFFu));
           wn[e] = clip127(wo - r[e]);
         }
@@ -582,10 +530,10 @@ __global__ __launch_bounds__(512) void fcw_wgrad_kernel(const FcwArgs a) {
     v4i wnew, g8;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      int r[4], wn[4];
+      const v4i r = round4_any(v4i{fin[t][4 * q], fin[t][4 * q + 1], fin[t][4 * q + 2], fin[t][4 * q + 3]}, shift, a.method, trunc, v4i{0, 0, 0, 0});
+      int wn[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        r[e] = round_any(fin[t][4 * q + e], shift, a.method, trunc, 0);
         const int wo = static_cast<int>(static_cast<int8_t>((static_cast<uint32_t>(wold[q]) >> (8 * e)) & 0xFFu));
         wn[e] = clip127(wo - r[e]);
       }
@@ -604,8 +552,6 @@ int resident_blocks(const void* kernel, int threads, size_t lds) {
     return 0;
   return cus * per_cu;
 }
-
-constexpr int kMaxSlots = 4096;
 
 // forward: reduction elements per wavefront (a multiple of 256), sixteen wavefronts per tile
 int fwd_chunk(int F) { return ((F + 15) / 16 + 255) / 256 * 256; }
@@ -678,11 +624,26 @@ int dgrad_resident(int O) {
   return resident_blocks(reinterpret_cast<const void*>(fcw_dgrad_kernel), 512, lds);
 }
 
+// Workgroups of the launch that takes any extents and alignment (gemm_any.hip); 0: none fits
+long long any_blocks(int which, int M, int O, int F) {
+  switch (which) {
+    case NITI_FC_FORWARD: return gemm_any_round_blocks(kAnyForward, M, O, F);
+    case NITI_FC_DGRAD: return gemm_any_round_blocks(kAnyDgrad, M, F, O);
+    case NITI_FC_WGRAD: return gemm_any_round_blocks(kAnyUpdate, O, F, M);
+    default: return 0;
+  }
+}
+
 // Workgroups of the launch on the current device and the per-workgroup tile count (MT / T); 0 when the shape is outside
 // the kernels or no variant's grid fits on the device at once.
 long long plan(int which, int M, int O, int F, int* tiles) {
   *tiles = 0;
   if (!shape_ok(which, M, O, F)) return 0;
+  // Where both sets of kernels cover the shape the ones for any extents take every weight gradient they fit (they share a
+  // 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512 8.6 -> 7.1) and the
+  // forward passes of large batches (512 x 4096 -> 1024 15.2 -> 13.0 us; 128 x 8192 -> 1024 takes them 12.3 instead of 8.3)
+  if (which == NITI_FC_WGRAD && any_blocks(which, M, O, F) > 0) return 0;
+  if (which == NITI_FC_FORWARD && M > 160 && any_blocks(which, M, O, F) > 0) return 0;
   if (which == NITI_FC_DGRAD) {
     if (const long long nl = dgrad_lds_blocks(M, O, F)) {
       *tiles = 1;
@@ -714,6 +675,26 @@ long long plan(int which, int M, int O, int F, int* tiles) {
   return best;
 }
 
+int launch_any(AnyRound what, const FcwArgs& f, const int8_t* a, const int8_t* b, int m, int n, int k, hipStream_t s) {
+  AnyArgs g{a, b, m, n, k};
+  g.out8 = f.out8;
+  g.w = f.w;
+  g.rand = f.rand;
+  g.sync = f.sync;
+  g.target_bits = f.target_bits;
+  g.method = f.method;
+  g.trunc = f.trunc;
+  g.bw_mode = f.bw_mode;
+  g.rq_flags = f.rq_flags;
+  g.spin_limit = f.spin_limit;
+  g.sticky = f.sticky;
+  g.shift_out = f.shift_out;
+  g.exp_a = f.exp_a;
+  g.exp_b = f.exp_b;
+  g.exp_out = f.exp_out;
+  return launch_gemm_any_round(what, g, s);
+}
+
 }  // namespace
 }  // namespace niti
 
@@ -721,7 +702,8 @@ using namespace niti;
 
 extern "C" size_t niti_linear_i8_sync_words(int which, int M, int O, int F) {
   int tiles = 0;
-  const long long nb = plan(which, M, O, F, &tiles);
+  long long nb = plan(which, M, O, F, &tiles);
+  if (nb == 0) nb = any_blocks(which, M, O, F);
   return nb == 0 ? 0 : static_cast<size_t>(kSlot0) + slot_words(static_cast<int>(nb));
 }
 
@@ -734,11 +716,10 @@ static int fcw_common(const char* who, int which, FcwArgs& a, int M, int O, int 
   if (target_bits < 1 || target_bits > 7) return fail(NITI_ERR_INVALID_ARG, "%s: target_bits=%d outside 1..7", who, target_bits);
   if (method != NITI_ROUND_NEAREST && method != NITI_ROUND_PSEUDO_STOCHASTIC && method != NITI_ROUND_STOCHASTIC)
     return fail(NITI_ERR_INVALID_ARG, "%s: rounding method %d", who, method);
-  if (method == NITI_ROUND_STOCHASTIC && (rand == nullptr || !aligned16(rand)))
-    return fail(NITI_ERR_INVALID_ARG, "%s: stochastic rounding needs `rand` (16-byte aligned, one int32 per output element)", who);
+  if (method == NITI_ROUND_STOCHASTIC && (rand == nullptr || reinterpret_cast<uintptr_t>(rand) % 4 != 0))
+    return fail(NITI_ERR_INVALID_ARG, "%s: stochastic rounding needs `rand` (one int32 per output element)", who);
   if (div_mode != NITI_DIV_FLOOR && div_mode != NITI_DIV_TRUNC) return fail(NITI_ERR_INVALID_ARG, "%s: div_mode=%d", who, div_mode);
   if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
-  if (!shape_ok(which, M, O, F)) return fail(NITI_ERR_UNSUPPORTED, "%s: M=%d O=%d F=%d outside these kernels; use the GEMM entry point", who, M, O, F);
   const size_t need = niti_linear_i8_sync_words(which, M, O, F);
   if (need == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: the workgroups of M=%d O=%d F=%d do not fit on the device at once", who, M, O, F);
   if (sync_words < need) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, need, sync_words);
@@ -770,7 +751,6 @@ extern "C" int niti_linear_i8_fwd_requant(const int8_t* act, const int8_t* w, in
                       exp_a, exp_b, exp_out);
   if (st != NITI_OK) return st;
   if (act == nullptr || w == nullptr || out8 == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: null pointer", who);
-  if (!aligned16(act) || !aligned16(w) || reinterpret_cast<uintptr_t>(out8) % 4 != 0) return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   if ((rq_flags & ~NITI_RQ_RELU) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
   a.act = act;
   a.w = const_cast<int8_t*>(w);
@@ -778,7 +758,9 @@ extern "C" int niti_linear_i8_fwd_requant(const int8_t* act, const int8_t* w, in
   a.rq_flags = rq_flags;
   a.kchunk = fwd_chunk(F);
   int mt = 0;
-  plan(NITI_FC_FORWARD, M, O, F, &mt);
+  if (plan(NITI_FC_FORWARD, M, O, F, &mt) == 0) return launch_any(kAnyForward, a, act, w, M, O, F, static_cast<hipStream_t>(stream));
+  if (!aligned16(act) || !aligned16(w) || !aligned16(rand) || reinterpret_cast<uintptr_t>(out8) % 4 != 0)
+    return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   const dim3 grid((O + 15) / 16, (M + 16 * mt - 1) / (16 * mt));
   hipStream_t s = static_cast<hipStream_t>(stream);
   // whole lines through LDS where the rows are whole lines (NITI_FC_LDS=0 pins the direct-fragment kernel)
@@ -805,10 +787,13 @@ extern "C" int niti_linear_i8_dgrad_requant(const int8_t* err, const int8_t* w, 
                       exp_a, exp_b, exp_out);
   if (st != NITI_OK) return st;
   if (err == nullptr || w == nullptr || dx8 == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: null pointer", who);
-  if (!aligned16(err) || !aligned16(w) || reinterpret_cast<uintptr_t>(dx8) % 4 != 0) return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   a.err = err;
   a.w = const_cast<int8_t*>(w);
   a.out8 = dx8;
+  int tiles = 0;
+  if (plan(NITI_FC_DGRAD, M, O, F, &tiles) == 0) return launch_any(kAnyDgrad, a, err, w, M, F, O, static_cast<hipStream_t>(stream));
+  if (!aligned16(err) || !aligned16(w) || !aligned16(rand) || reinterpret_cast<uintptr_t>(dx8) % 4 != 0)
+    return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   if (dgrad_lds_blocks(M, O, F) != 0) {
     if (!aligned16(dx8)) return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
     hipLaunchKernelGGL(fcw_dgrad_lds_kernel, dim3(F / 128, (M + 31) / 32), dim3(512), static_cast<size_t>(kDgLdsBytes),
@@ -830,13 +815,14 @@ extern "C" int niti_linear_i8_wgrad_update(const int8_t* err, const int8_t* act,
                       exp_out);
   if (st != NITI_OK) return st;
   if (err == nullptr || act == nullptr || w == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: null pointer", who);
-  if (!aligned16(err) || !aligned16(act) || !aligned16(w) || !aligned16(g8_out)) return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   a.err = err;
   a.act = act;
   a.w = w;
   a.out8 = g8_out;
   int t_use = 0;
-  plan(NITI_FC_WGRAD, M, O, F, &t_use);
+  if (plan(NITI_FC_WGRAD, M, O, F, &t_use) == 0) return launch_any(kAnyUpdate, a, err, act, O, F, M, static_cast<hipStream_t>(stream));
+  if (!aligned16(err) || !aligned16(act) || !aligned16(w) || !aligned16(g8_out) || !aligned16(rand))
+    return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   const dim3 grid((F + 255) / 256, (O + 32 * t_use - 1) / (32 * t_use));
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (t_use == 1) hipLaunchKernelGGL(fcw_wgrad_kernel<1>, grid, dim3(512), wgrad_lds(1), s, a);

@@ -1,0 +1,38 @@
+// int8 products of matrices with any extents, in any of the four operand layouts, read as stored (gemm_any.hip).
+#pragma once
+#include "common.h"
+
+namespace niti {
+
+struct AnyArgs {
+  const int8_t* a;       // [m][k], or [k][m] when transposed
+  const int8_t* b;       // [n][k] when transposed, or [k][n]
+  int m, n, k;
+  // int32 result
+  int32_t* c = nullptr;  // [m][n]
+  uint32_t* absmax = nullptr;
+  int roundtrip = 0;
+  // result rounded to int8, or rounded and subtracted from the weights
+  int8_t* out8 = nullptr;   // [m][n]; weight update: the rounded gradient, may be null
+  int8_t* w = nullptr;      // [m][n], weight update only
+  const int32_t* rand = nullptr;
+  uint32_t* sync = nullptr;
+  int target_bits = 7, method = 0, trunc = 0, bw_mode = 0;
+  unsigned rq_flags = 0;
+  long long spin_limit = 0;
+  uint32_t* sticky = nullptr;
+  int32_t* shift_out = nullptr;
+  const int32_t* exp_a = nullptr;
+  const int32_t* exp_b = nullptr;
+  int32_t* exp_out = nullptr;
+};
+
+bool gemm_any_shape(int m, int n, int k);                       // extents within the kernels' index arithmetic
+bool gemm_any_large(int m, int n);                              // the result fills the chip with 128 x 128 tiles
+int launch_gemm_any(int trans_a, int trans_b, const AnyArgs& a, hipStream_t stream);
+// workgroups of the launch that rounds (= sync slots), 0 when no variant's grid fits on the current device at once
+enum AnyRound { kAnyForward = 0, kAnyDgrad = 1, kAnyUpdate = 2 };   // layouts NT, NN, TN
+long long gemm_any_round_blocks(AnyRound what, int m, int n, int k);
+int launch_gemm_any_round(AnyRound what, const AnyArgs& a, hipStream_t stream);
+
+}  // namespace niti

@@ -25,7 +25,7 @@ enum Path { kFew, kWide, kSeparate };
 Path path_of(Pass pass, bool fuse, const Shape& s, int method, Opt rand, size_t* words) {
   if (!fuse) return kSeparate;
   if (rand == nullptr && method != NITI_ROUND_STOCHASTIC && (*words = niti_fc_i8_sync_words(pass, s.M, s.O, s.F)) > 0) return kFew;
-  if (s.O > 16 && (*words = niti_linear_i8_sync_words(pass, s.M, s.O, s.F)) > 0) return kWide;
+  if ((*words = niti_linear_i8_sync_words(pass, s.M, s.O, s.F)) > 0) return kWide;
   return kSeparate;
 }
 

@@ -5,6 +5,7 @@
 
 namespace niti {
 
+__device__ inline int clip127(int v) { return min(max(v, -127), 127); }
 __device__ inline int clip127(long long v) { return static_cast<int>(v > 127 ? 127 : (v < -127 ? -127 : v)); }
 
 // quotient and magnitude of the remainder of x / 2^s: floor division or truncation

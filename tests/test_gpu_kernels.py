@@ -1164,3 +1164,56 @@ def test_whole_line_kernels_on_drawn_shapes(dev, seed):
             ref, _ = po.act_calc(acc, 0, method, "floor", rand=low(uf, acc) if sto else None)
             y, _, sync = ops.linear_fwd_requant(act.to(dev), w.to(dev), 7, method, "floor", rand=uf.to(dev) if sto else None)
             assert torch.equal(y.cpu(), ref) and int(sync.cpu()[1]) == 0, (M, Fi, O, method)
+
+
+# edges of the 32 / 64 / 128 tiles, of the reduction chunks (512 / 256 / 128) and of 16-byte rows; single rows, columns and steps
+ANY_CASES = [(1, 1, 1), (2, 4, 152), (31, 33, 513), (32, 32, 512), (33, 65, 511), (64, 64, 256), (65, 129, 1025), (128, 128, 128),
+             (129, 130, 127), (77, 300, 31), (200, 3, 1000), (5, 701, 48), (300, 259, 257)]
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", ""])
+@pytest.mark.parametrize("case", ANY_CASES)
+def test_products_of_any_extents(dev, case, tile, monkeypatch):
+    """The kernel for operands of any extents and alignment: int32 products in all four layouts, TiLinear's three passes
+    with each rounding, every tile pinned and the dispatch's own choice ('')."""
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    if tile:
+        monkeypatch.setenv("NITI_ANY_TILE", tile)
+    m, n, k = case
+    _say("products_of_any_extents", case, tile)
+    g = torch.Generator().manual_seed(8100 + m + n + k)
+    A, B = ri8(g, m, k), ri8(g, k, n)
+    ref = po.int8mm(A, B)
+    for ta in (False, True):
+        for tb in (False, True):
+            a = (A.t().contiguous() if ta else A).to(dev)
+            b = (B.t().contiguous() if tb else B).to(dev)
+            am = ops.new_scalar_u32(dev)
+            assert torch.equal(ops.gemm(a, b, ta, tb, absmax=am).cpu(), ref), (ta, tb)
+            assert int(am.cpu()) == po.absmax(ref), (ta, tb)
+    M, O, F = m, n, k
+    act, w, err = ri8(g, M, F), ri8(g, O, F), ri8(g, M, O, lo=-60, hi=60)
+    for method in ("round", "psto", "sto"):
+        sto = method == "sto"
+
+        def drawn(acc, bits):    # wide random integers for the kernel, their low bits for the oracle
+            u = torch.randint(0, 1 << 24, acc.shape, generator=g, dtype=torch.int32)
+            s = max(po.bitwidth_int(po.absmax(acc)) - bits, 0)
+            return (u.to(dev), u & ((1 << s) - 1)) if sto else (None, None)
+        acc = po.int8mm(act, w.t().contiguous())
+        ud, u = drawn(acc, 7)
+        y, _, sync = ops.linear_fwd_requant(act.to(dev), w.to(dev), 7, method, rand=ud)
+        assert torch.equal(y.cpu(), po.act_calc(acc, 0, method, "floor", rand=u)[0]) and int(sync.cpu()[1]) == 0, method
+        acc = po.int8mm(err, w)
+        ud, u = drawn(acc, 7)
+        y, sh, _ = ops.linear_dgrad_requant(err.to(dev), w.to(dev), 7, method, rand=ud)
+        ref8, sh_ref = po.err_calc(acc, method, "floor", rand=u)
+        assert torch.equal(y.cpu(), ref8) and int(sh.cpu()) == sh_ref, method
+        acc = po.int8mm(err.t().contiguous(), act)
+        ud, u = drawn(acc, 5)
+        wd = w.to(dev)
+        g8, sh, _ = ops.linear_wgrad_update(err.to(dev), act.to(dev), wd, 5, method, rand=ud, want_grad=True)
+        g8_ref, sh_ref = po.grad_calc(acc, 5, method, "floor", rand=u)
+        assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref, method
+        assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref)), method
