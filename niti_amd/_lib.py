@@ -39,6 +39,7 @@ SIGNATURES = {
     "niti_conv2d_i8_fprop": (_i, [_vp, _vp, _vp] + [_i] * 9 + [_u, _vp, _vp, _sz, _vp]),
     "niti_conv2d_i8_dgrad": (_i, [_vp, _vp, _vp] + [_i] * 9 + [_u, _vp, _vp, _sz, _vp]),
     "niti_conv2d_i8_requant_sync_words": (_sz, [_i] * 10),
+    "niti_conv2d_i8_requant_sync_words_any": (_sz, [_i] * 10),
     "niti_conv2d_i8_fprop_requant": (_i, [_vp, _vp, _vp] + [_i] * 9 + [_u, _i, _i, _i, _i, _u, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "niti_conv2d_i8_fprop_requant_pool": (_i, [_vp, _vp, _vp, _vp] + [_i] * 9 + [_u, _i, _i, _i, _i, _u, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "niti_static_scratch_bytes": (_sz, []),

@@ -282,8 +282,10 @@ extern "C" int niti_sync_timeouts(uint32_t* flag_out, int clear, void* stream) {
   return NITI_OK;
 }
 
-static int fused_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad) {
+// `any`: also batches that are no whole tiles (the entry points refuse those unless NITI_RQ_ANY_SHAPE asks for them)
+static int fused_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad, bool any) {
   if (halo_off()) return 0;
+  if (!any && !(H == 2 && W == 2) && static_cast<long long>(N) * H * W % 256 != 0) return 0;
   if (!dgrad) return conv3x3_halo_requant_blocks(N, H, W, C, K, R, S, stride, pad);
   if (stride != 1 || R != S || pad > R - 1) return 0;
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
@@ -293,7 +295,14 @@ static int fused_blocks(int N, int H, int W, int C, int K, int R, int S, int str
 extern "C" size_t niti_conv2d_i8_requant_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad,
                                                     int dgrad) {
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0) return 0;
-  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad);
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, false);
+  return nb > 0 ? conv3x3_halo_sync_words(nb) : 0;
+}
+
+extern "C" size_t niti_conv2d_i8_requant_sync_words_any(int N, int H, int W, int C, int K, int R, int S, int stride, int pad,
+                                                        int dgrad) {
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0) return 0;
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, true);
   return nb > 0 ? conv3x3_halo_sync_words(nb) : 0;
 }
 
@@ -316,8 +325,8 @@ static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_
   if (rand != nullptr && !aligned16(rand)) return fail(NITI_ERR_INVALID_ARG, "%s: rand must be 16-byte aligned", who);
   if (div_mode != NITI_DIV_FLOOR && div_mode != NITI_DIV_TRUNC) return fail(NITI_ERR_INVALID_ARG, "%s: div_mode=%d", who, div_mode);
   if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
-  if ((rq_flags & ~(NITI_RQ_RELU | NITI_RQ_SHIFT_HINT)) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
-  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad);
+  if ((rq_flags & ~(NITI_RQ_RELU | NITI_RQ_SHIFT_HINT | NITI_RQ_ANY_SHAPE)) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, (rq_flags & NITI_RQ_ANY_SHAPE) != 0u);
   if (nb == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: shape not covered by the single-launch path; use the two-pass path", who);
   st = check_forward_copy_flag(who, dgrad, flags, N, H, W, C, K, R, S, stride, pad);
   if (st != NITI_OK) return st;
@@ -454,7 +463,7 @@ extern "C" int niti_conv2d_i8_fprop_requant_static(const int8_t* x, const int8_t
   const char* who = "conv_fprop_requant_static";
   int st = check_conv_dims(who, N, H, W, C, K, R, S, stride, pad);
   if (st != NITI_OK) return st;
-  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0);
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0, (rq_flags & NITI_RQ_ANY_SHAPE) != 0u);
   if (nb == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: shape not covered by the single-launch path", who);
   const size_t words = conv3x3_halo_sync_words(nb);
   if (words > kStaticSyncWords)

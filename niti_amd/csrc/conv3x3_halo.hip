@@ -1206,42 +1206,46 @@ __global__ __launch_bounds__(256) void halo_filter_prepare_kernel(const int8_t* 
   }
 }
 
-// Channel tile of a launch: 128 unless that leaves fewer workgroups than the device runs at once while
-// a tile of 64 would give it more to do.
-int halo_ktile(long long pix, int K, int H, int C) {
-  static int cus_of[kDeviceSlots] = {};
-  int& cus = cus_of[device_slot()];
+int compute_units() {
+  static int of[kDeviceSlots] = {};
+  int& cus = of[device_slot()];
   if (cus == 0) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       cus = 256;
   }
+  return cus;
+}
+
+// Channel tile of a launch: 128 unless that leaves fewer workgroups than the device runs at once while
+// a tile of 64 would give it more to do.
+int halo_ktile(long long pix, int K, int H, int C) {
+  const long long ptiles = (pix + 255) / 256;
+  const int cus = compute_units();
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
   if (forced == 128 || forced == 64) return forced;
   if (forced == 32 && H <= 16) return 32;
   // fewer 64-channel tiles than compute units on the small maps: tiles of 32 channels, twice as many workgroups
-  if (forced == 0 && H <= 8 && K > 32 && (pix / 256) * ((K + 63) / 64) < cus) return 32;
+  if (forced == 0 && H <= 8 && K > 32 && ptiles * ((K + 63) / 64) < cus) return 32;
   // exactly one 64-channel tile per compute unit and a short reduction: two 32-channel workgroups per unit overlap
   // each other's fill and epilogue (measured per launch: 128 -> 256 at 16 x 16 data gradient 14.5 -> 13.9 us, 256 -> 512
   // at 8 x 8 forward 13.9 -> 12.7 us; with 512 input channels the narrower tile's longer loop loses more than that)
-  if (forced == 0 && H <= 16 && K > 32 && C <= 256 && (pix / 256) * ((K + 63) / 64) == cus) return 32;
+  if (forced == 0 && H <= 16 && K > 32 && C <= 256 && ptiles * ((K + 63) / 64) == cus) return 32;
   if (K <= 64) return 64;   // nothing to gain from computing 128 channels
   // one slice of reduction (the first layer): the launch is all output stores, and the 64-channel tile's workgroups -
   // 512 pixels each where 256-pixel ones would not all fit - spread them better (3 -> 128 at 32 x 32: 9.9 -> 9.5 us)
   if (forced == 0 && C <= 32 && H == 32 && pix % 512 == 0) return 64;
-  const long long b128 = (pix / 256) * ((K + 127) / 128);
+  const long long b128 = ptiles * ((K + 127) / 128);
   return (b128 < 2LL * cus && K > 64) ? 64 : 128;
 }
 
 // The 64-channel tile with 512 pixels per workgroup: where 256-pixel workgroups would be more than the device holds
 // at once (a condition of the requantising variant), on the large maps where such launches occur.
 bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
-  if (ktile != 64 || (H != 32 && H != 16) || pix % 512 != 0) return false;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  return (pix / 256) * ((K + 63) / 64) > 2LL * cus;
+  if (ktile != 64 || (H != 32 && H != 16)) return false;
+  const int cus = compute_units();
+  return (pix + 255) / 256 * ((K + 63) / 64) > 2LL * cus;
 }
 
 template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto = false>
@@ -1387,8 +1391,9 @@ bool conv3x3_halo_supported(int N, int H, int W, int C, int K, int R, int S, int
   if (R != 3 || S != 3 || stride != 1 || pad != 1 || H != W) return false;
   if (H != 2 && H != 4 && H != 8 && H != 16 && H != 32) return false;
   if (C % 16 != 0 || K % 4 != 0) return false;
-  const long long pix = static_cast<long long>(N) * H * W;
-  if (H != 2 && pix % 256 != 0) return false;  // workgroups own whole rows / whole images (2 x 2 maps: any batch)
+  // workgroups own whole rows / whole images; images behind the last one (a batch that is no whole tile of the 4 x 4 and 8 x 8
+  // maps) read as zeros and are not stored
+  const long long pix = static_cast<long long>(N) * H * W + 512;
   if (pix * C >= 0x7fffffffLL || pix * K * 4 >= 0x7fffffffLL) return false;
   if (conv3x3_halo_filter_bytes(C, K) >= 0x7fffffffULL) return false;
   return true;
@@ -1423,7 +1428,7 @@ int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S,
   const long long pix = static_cast<long long>(N) * H * W;
   const int ktile = halo_ktile(pix, K, H, C);
   const long long px = halo_two_pixel_tiles(pix, K, H, ktile) ? 512 : 256;
-  const long long nb = H == 2 ? map2_blocks(N, K) : (pix / px) * ((K + ktile - 1) / ktile);
+  const long long nb = H == 2 ? map2_blocks(N, K) : ((pix + px - 1) / px) * ((K + ktile - 1) / ktile);
   return nb <= kMaxSlots ? static_cast<int>(nb) : 0;  // more than the device holds at once run as two launches
 }
 

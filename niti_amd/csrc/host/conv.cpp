@@ -163,7 +163,7 @@ PyObject* wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // ---- results rounded to int8 in the launch -------------------------------------------------------------------------
 struct Fused {
-  bool dgrad = false, f32 = false, relu = false, hint = false, forward_copy = false;
+  bool dgrad = false, f32 = false, relu = false, hint = false, forward_copy = false, any_shape = false;
   int stride = 1, pad = 1, ties = 0;
   Rounding r{};
   Opt sync = nullptr, shift = nullptr, exp_a = nullptr, exp_b = nullptr, exp_out = nullptr, prepared = nullptr, mask = nullptr, pool_out = nullptr,
@@ -196,7 +196,9 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
     shape = big;
   }
   if (!is_i8(x) || !is_i8(w)) refuse(std::string(who) + ": int8 tensors expected");
-  const size_t words = niti_conv2d_i8_requant_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
+  const bool any = soft || f.any_shape;
+  const size_t words = any ? niti_conv2d_i8_requant_sync_words_any(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg)
+                           : niti_conv2d_i8_requant_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
   if (words == 0) {
     if (soft) return false;
     refuse_niti(std::string(who) + ": shape not covered by the single-launch path");
@@ -218,7 +220,7 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
     ws = empty8({static_cast<int64_t>(bytes > 16 ? bytes : 16)}, x);
   }
   void* wsp = f.prepared != nullptr ? nullptr : ws.data_ptr();
-  const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u);
+  const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u) | (any ? NITI_RQ_ANY_SHAPE : 0u);
   const int8_t* xp = ptr<int8_t>(x);
   int8_t* yp = ptr<int8_t>(*y);
   int32_t* sp = ptr<int32_t>(*shift);
@@ -263,11 +265,11 @@ at::Tensor requant_i32(const at::Tensor& acc, const uint32_t* absmax, const Roun
 }
 
 // requant_op(who, x, w, stride, pad, f32, bits, method, div, bw, relu, hint, sync, shift, exp_a, exp_b, exp_out, prepared,
-//            forward_copy, mask, pool_out, pool_in, ties, rand) -> (y, shift, sync): ops.conv2d_*_requant
+//            forward_copy, mask, pool_out, pool_in, ties, rand, any_shape) -> (y, shift, sync): ops.conv2d_*_requant
 PyObject* requant_op(PyObject* const* args, Py_ssize_t n, bool dg) {
   return guarded([&]() -> PyObject* {
     const char* who = dg ? "niti_conv2d_i8_dgrad_requant" : "niti_conv2d_i8_fprop_requant";
-    Args a(args, n, 23, who);
+    Args a(args, n, 24, who);
     const at::Tensor& x = a.tensor();
     const at::Tensor& w = a.tensor();
     Fused f;
@@ -290,6 +292,7 @@ PyObject* requant_op(PyObject* const* args, Py_ssize_t n, bool dg) {
     f.pool_in = a.opt();
     f.ties = a.i();
     f.rand = a.opt();
+    f.any_shape = a.flag();
     const Dims d = dg ? gradient_dims(x, w, f.pad, who) : forward_dims(x, w, who);
     if (f.pool_out != nullptr &&
         (!is_i8(*f.pool_out) || !has_shape(*f.pool_out, {d.N, out_extent(d.H, d.R, f.stride, f.pad) / 2, out_extent(d.W, d.S, f.stride, f.pad) / 2, d.K})))

@@ -1007,13 +1007,11 @@ long long slice_stride_for(int C, int K) {
   return (n + 1023) / 1024 * 1024 + 1088;
 }
 
-// The narrow-tile arrangement needs whole stages of 256 pixels.  NITI_WGRAD_NARROW=0/1 pins the choice (tests).
+// The narrow-tile arrangement takes any batch (pixels behind the last image read as zeros).  NITI_WGRAD_NARROW=0 pins the wide
+// one, which needs whole bands of 128 pixels (tests).
 bool use_narrow_arrangement(int N, int Q) {
-  const bool fits = (static_cast<long long>(N) * Q * Q) % 256 == 0;
-  if (Q < 8) return true;   // the only arrangement for the small maps (the shape check requires whole stages)
   const char* e = getenv("NITI_WGRAD_NARROW");
-  if (e != nullptr) return e[0] == '1' && fits;
-  return fits;
+  return !(e != nullptr && e[0] == '0' && Q >= 8 && (static_cast<long long>(N) * Q * Q) % 128 == 0);
 }
 
 int pick_splits(int N, int Q, int C, int K) {
@@ -1021,7 +1019,7 @@ int pick_splits(int N, int Q, int C, int K) {
   int target = e != nullptr ? atoi(e) : 0;
   int bands, tiles;
   if (use_narrow_arrangement(N, Q)) {
-    bands = N * Q * Q / 256;
+    bands = (N * Q * Q + 255) / 256;
     tiles = ((K + 127) / 128) * ((C + 31) / 32);
     if (target < 1) target = 256;
   } else {
@@ -1108,10 +1106,7 @@ bool wgrad3x3_supported(int N, int H, int W, int C, int K, int R, int S, int str
   if (R != 3 || S != 3 || stride != 1 || pad != 1 || H != W) return false;
   if (H != 2 && H != 4 && H != 8 && H != 16 && H != 32) return false;
   if (C % 16 != 0 || K % 16 != 0) return false;
-  const long long pix = static_cast<long long>(N) * H * W;
-  if (pix % 128 != 0) return false;  // bands of 128 pixels: whole rows / whole images
-  if (H <= 4 && pix % 256 != 0) return false;  // small maps: only the arrangement with stages of 256 pixels
-  if (H == 8 && N % 2 != 0) return false;
+  const long long pix = static_cast<long long>(N) * H * W + 256;   // the last stage counted whole
   if (pix * C >= 0x7fffffffLL || pix * K >= 0x7fffffffLL) return false;
   return true;
 }
@@ -1131,7 +1126,7 @@ static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N,
   a.K = K;
   a.Cp = Cp;
   const bool narrow = use_narrow_arrangement(N, H);
-  a.bands = N * H * H / (narrow ? 256 : 128);
+  a.bands = narrow ? (N * H * H + 255) / 256 : N * H * H / 128;
   splits = pick_splits(N, H, C, K);
   a.bands_per_split = (a.bands + splits - 1) / splits;
   a.act_bytes = static_cast<long long>(N) * H * H * C;

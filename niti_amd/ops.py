@@ -77,15 +77,16 @@ def conv_requant_sync_words(N, H, W, C, K, R=3, S=3, stride=1, padding=1, dgrad=
 
 def conv2d_fprop_requant(x, w, stride=1, padding=1, f32_epilogue=False, target_bits=7, method="round", div_mode="floor",
                          bw_mode="int", relu=False, sync=None, shift_out=None, exp_a=None, exp_b=None, exp_out=None,
-                         prepared_filter=None, shift_hint=False, pool_out=None, rand=None):
+                         prepared_filter=None, shift_hint=False, pool_out=None, rand=None, any_shape=False):
     """conv2d_fprop + requant as one launch: x [N,H,W,C] int8, w [K,R,S,C] int8 -> ([N,P,Q,K] int8, device shift,
     sync).  method "sto" takes ``rand`` (int32, shaped like the output).  ``pool_out`` ([N,P/2,Q/2,K] int8): also receives the 2x2 / stride-2 maximum of the output.  sync[0] holds max|sum| afterwards, sync[1] != 0 flags a timed-out wait (invalid output).  ``sync``, if
     given, must hold conv_requant_sync_words(...) zeroed int32 words.  ``shift_hint``: ``shift_out`` holds a
     predicted shift on entry (e.g. this tensor's shift of the previous training step); a good prediction saves the
-    kernel a second store pass, the results do not depend on it."""
+    kernel a second store pass, the results do not depend on it.  ``any_shape``: also batches that are no whole tiles of 256
+    pixels (NITI_RQ_ANY_SHAPE)."""
     return L.host().conv_fprop_requant(x, w, stride, padding, f32_epilogue, target_bits, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode],
                                        relu, shift_hint, sync, shift_out, exp_a, exp_b, exp_out, prepared_filter, False, None, pool_out,
-                                       None, 0, rand)
+                                       None, 0, rand, any_shape)
 
 
 def conv2d_fprop_requant_static(x, w, stride=1, padding=1, f32_epilogue=False, target_bits=7, method="round", div_mode="floor",
@@ -123,7 +124,8 @@ def conv2d_fprop_requant_static(x, w, stride=1, padding=1, f32_epilogue=False, t
 
 def conv2d_dgrad_requant(err, w, stride=1, padding=1, f32_epilogue=False, target_bits=7, method="round", div_mode="floor",
                          bw_mode="int", sync=None, shift_out=None, exp_a=None, exp_b=None, exp_out=None,
-                         prepared_filter=None, relu_mask=None, forward_filter=None, shift_hint=False, unpool=None, rand=None):
+                         prepared_filter=None, relu_mask=None, forward_filter=None, shift_hint=False, unpool=None, rand=None,
+                         any_shape=False):
     """conv2d_dgrad + requant as one launch: err [N,P,Q,K] int8, w [K,R,S,C] int8 -> ([N,H,W,C] int8, shift, sync).
     method "sto" takes ``rand`` (int32, shaped like the output; not together with ``unpool``).
     ``unpool`` = (pool_in [N,2H,2W,C] int8, "first" | "all") with ``relu_mask`` = the pooled map: the backward pass of
@@ -135,7 +137,8 @@ def conv2d_dgrad_requant(err, w, stride=1, padding=1, f32_epilogue=False, target
     pool_in, ties = unpool if unpool is not None else (None, "first")
     return L.host().conv_dgrad_requant(err, w, stride, padding, f32_epilogue, target_bits, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode],
                                        False, shift_hint, sync, shift_out, exp_a, exp_b, exp_out,
-                                       forward_filter if forward else prepared_filter, forward, relu_mask, None, pool_in, L.TIES[ties], rand)
+                                       forward_filter if forward else prepared_filter, forward, relu_mask, None, pool_in, L.TIES[ties], rand,
+                                       any_shape)
 
 
 def _index(device) -> int:

@@ -1217,3 +1217,38 @@ def test_products_of_any_extents(dev, case, tile, monkeypatch):
         g8_ref, sh_ref = po.grad_calc(acc, 5, method, "floor", rand=u)
         assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref, method
         assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref)), method
+
+
+@pytest.mark.parametrize("case", [(1, 8, 64, 128), (3, 8, 96, 48), (5, 8, 512, 64), (25, 8, 32, 80), (1, 4, 64, 32), (17, 4, 48, 128), (515, 4, 16, 16),
+                                  (1, 16, 64, 64), (513, 16, 16, 144)])
+def test_conv_ragged_batches(dev, case):
+    """Batches that are no whole tile of 256 (512) pixels through the single-launch kernels: forward with ReLU and max-pool,
+    data gradient with the forward filter copy, weight gradient with update, and the int32 forms."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    _say("conv_ragged_batches", case)
+    g = torch.Generator().manual_seed(7700 + N + Q + C)
+    x, w, e = ri8(g, N, Q, Q, C), ri8(g, K, 3, 3, C), ri8(g, N, Q, Q, K, lo=-40, hi=40)
+    xd, wd, ed = x.to(dev), w.to(dev), e.to(dev)
+    acc = co.conv_fprop(x, w, 1, 1)
+    am = ops.new_scalar_u32(dev)
+    assert torch.equal(ops.conv2d_fprop(xd, wd, absmax=am).cpu(), acc) and int(am.cpu()) == po.absmax(acc)
+    prepared = ops.conv_filter_prepare(wd, N, Q, Q)
+    pool = torch.empty((N, Q // 2, Q // 2, K), dtype=torch.int8, device=dev)
+    y, sh, sync = ops.conv2d_fprop_requant(xd, wd, relu=True, prepared_filter=prepared, pool_out=pool, any_shape=True)
+    ref = torch.clamp(po.act_calc(acc, 0)[0], min=0)
+    assert torch.equal(y.cpu(), ref) and int(sync.cpu()[1]) == 0
+    assert torch.equal(pool.cpu(), po.maxpool_fwd(ref))
+    dacc = co.conv_dgrad(e, w, Q, Q, 1, 1)
+    y, sh, _ = ops.conv2d_dgrad_requant(ed, wd, forward_filter=prepared, any_shape=True)
+    dref, dsh = po.err_calc(dacc)
+    assert torch.equal(y.cpu(), dref) and int(sh.cpu()) == dsh
+    wacc = co.conv_wgrad(x, e, 3, 3, 1, 1)
+    assert torch.equal(ops.conv2d_wgrad(xd, ed, 3, 3).cpu(), wacc)
+    g8_ref, sh_ref = po.grad_calc(wacc, 5, "psto")
+    g8, _, sh, sync = ops.conv2d_wgrad_update(xd, ed, wd, want_grad=True, prepared_filter=prepared)
+    assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
+    assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref))
+    assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q))
