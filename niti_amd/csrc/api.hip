@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "conv_any.h"
 #include "gemm_any.h"
 
 namespace niti {
@@ -94,6 +95,12 @@ static bool halo_off() {
     return e != nullptr && e[0] == '1';
   }();
   return off;
+}
+
+// NITI_CONV_TILE pins a tile of the pipelined generic kernel (measurements)
+static int generic_pinned() {
+  const char* e = getenv("NITI_CONV_TILE");
+  return e != nullptr ? atoi(e) : 0;
 }
 
 // which filter copy a convolution of this shape uses: 0 none (w as stored), 1 flipped/transposed
@@ -190,6 +197,9 @@ extern "C" int niti_conv2d_i8_fprop(const int8_t* x, const int8_t* w, int32_t* y
   } else if (flags & NITI_CONV_FILTER_PREPARED) {
     // no copy exists for this shape: filter_prepare wrote nothing, so `w` must be the filter itself
   }
+  const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
+  if (generic_pinned() == 0 && conv_any_shape(kConvForward, shape))
+    return launch_conv_any(kConvForward, shape, x, w, y, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, s);
   const int P = (H + 2 * pad - R) / stride + 1, Q = (W + 2 * pad - S) / stride + 1;
   ConvProblem p{x, w, y, absmax, N, H, W, C, K, R, S, stride, pad,
                 static_cast<long long>(P) * Q * K, static_cast<long long>(Q) * K, K, 1, 1, flags};
@@ -218,6 +228,9 @@ extern "C" int niti_conv2d_i8_dgrad(const int8_t* err, const int8_t* w, int32_t*
     const size_t need = niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, pad, 1);
     if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))
       return fail(NITI_ERR_WORKSPACE, "conv_dgrad: needs %zu workspace bytes (16-byte aligned), got %zu", need, workspace_bytes);
+    const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
+    if (kind == 1 && generic_pinned() == 0 && aligned16(w) && conv_any_shape(kConvDgrad, shape))
+      return launch_conv_any(kConvDgrad, shape, err, w, dx, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, s);
     st = kind == 3 ? launch_halo_filter_prepare(w, static_cast<int8_t*>(workspace), C, K, 1, s)
                    : launch_filter_flip_transpose(w, static_cast<int8_t*>(workspace), K, R, S, C, s);
     if (st != NITI_OK) return st;
@@ -303,7 +316,7 @@ extern "C" size_t niti_conv2d_i8_requant_sync_words_any(int N, int H, int W, int
                                                         int dgrad) {
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0) return 0;
   const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, true);
-  return nb > 0 ? conv3x3_halo_sync_words(nb) : 0;
+  return nb > 0 ? conv3x3_halo_sync_words(nb) : conv_any_requant_words(dgrad ? kConvDgrad : kConvForward, {N, H, W, C, K, R, S, stride, pad});
 }
 
 static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_t* w, int8_t* y8, int N, int H, int W, int C,
@@ -327,6 +340,21 @@ static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_
   if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
   if ((rq_flags & ~(NITI_RQ_RELU | NITI_RQ_SHIFT_HINT | NITI_RQ_ANY_SHAPE)) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
   const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, (rq_flags & NITI_RQ_ANY_SHAPE) != 0u);
+  if (nb == 0 && (rq_flags & NITI_RQ_ANY_SHAPE) != 0u && pool_out == nullptr && pool_x == nullptr && (!dgrad || (flags & NITI_CONV_FILTER_PREPARED) == 0u)) {
+    // every other shape, read as stored
+    const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
+    const ConvPass pass = dgrad ? kConvDgrad : kConvForward;
+    const size_t words = conv_any_requant_words(pass, shape);
+    if (words != 0) {
+      if (sync_words < words) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, words, sync_words);
+      RequantSpec rq{target_bits, method, div_mode == NITI_DIV_TRUNC, bw_mode, rq_flags, sync_spin_limit(), timeout_word(), shift_out, exp_a, exp_b, exp_out,
+                     relu_mask, nullptr};
+      rq.rand = method == NITI_ROUND_STOCHASTIC ? rand : nullptr;
+      return launch_conv_any_requant(pass, shape, x, w, y8, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, static_cast<hipStream_t>(stream));
+    }
+  }
+  if (nb == 0 && (rq_flags & NITI_RQ_ANY_SHAPE) != 0u && (pool_out != nullptr || pool_x != nullptr))
+    return fail(NITI_ERR_UNSUPPORTED, "%s: a pooling is folded in by the 3x3 kernels only, which do not fit this call", who);
   if (nb == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: shape not covered by the single-launch path; use the two-pass path", who);
   st = check_forward_copy_flag(who, dgrad, flags, N, H, W, C, K, R, S, stride, pad);
   if (st != NITI_OK) return st;
@@ -507,7 +535,9 @@ extern "C" size_t niti_conv2d_i8_wgrad_workspace(int N, int H, int W, int C, int
   if (P <= 0 || Q <= 0) return 0;
   if (wgrad3x3_supported(N, H, W, C, K, R, S, 1, pad)) return round256(wgrad3x3_workspace(N, H, C, K));
   const size_t np = static_cast<size_t>(round16(N));
-  return round256(static_cast<size_t>(C) * H * W * np) + round256(static_cast<size_t>(K) * P * Q * np);
+  const size_t copies = round256(static_cast<size_t>(C) * H * W * np) + round256(static_cast<size_t>(K) * P * Q * np);
+  const size_t slices = round256(conv_any_wgrad_workspace({N, H, W, C, K, R, S, 1, pad}));
+  return slices > copies ? slices : copies;
 }
 
 extern "C" int niti_conv2d_i8_wgrad(const int8_t* act, const int8_t* err, int32_t* dw, int N, int H, int W, int C, int K,
@@ -529,6 +559,9 @@ extern "C" int niti_conv2d_i8_wgrad(const int8_t* act, const int8_t* err, int32_
     return launch_wgrad3x3(act, err, dw, N, H, C, K, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
   }
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
+  const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
+  if (conv_any_shape(kConvWgrad, shape) && aligned16(act) && aligned16(err) && aligned16(dw))
+    return launch_conv_any_wgrad(shape, act, err, dw, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
   const int np = round16(N);
   int8_t* act_t = static_cast<int8_t*>(workspace);                                 // [C][H*W][np]
   int8_t* err_t = act_t + round256(static_cast<size_t>(C) * H * W * np);           // [K][P*Q][np]
@@ -555,7 +588,8 @@ extern "C" int niti_conv2d_i8_wgrad(const int8_t* act, const int8_t* err, int32_
 
 extern "C" size_t niti_conv2d_i8_wgrad_update_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0) return 0;
-  if (!wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && !wgrad_small_shape(N, H, W, C, K, R, S, stride, pad)) return 0;
+  if (!wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && !wgrad_small_shape(N, H, W, C, K, R, S, stride, pad))
+    return conv_any_wgrad_update_words({N, H, W, C, K, R, S, stride, pad});
   const int nb = wgrad3x3_finish_blocks(C, K);
   return nb > 0 ? wgrad3x3_sync_words(nb) + wgrad_first_extra_words(H, C, K) : 0;
 }
@@ -592,6 +626,11 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
     return fail(NITI_ERR_UNSUPPORTED, "conv_wgrad_update: w_prepared needs a shape whose forward pass uses a kernel-ready filter copy, 4-byte aligned");
   RequantSpec rq{mu, method, div_mode == NITI_DIV_TRUNC, bw_mode, (flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u, sync_spin_limit(),
                  timeout_word(), shift_out, exp_a, exp_b, exp_out, nullptr, nullptr};
+  if (!wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && !wgrad_small_shape(N, H, W, C, K, R, S, stride, pad)) {
+    if (w_prepared != nullptr) return fail(NITI_ERR_UNSUPPORTED, "conv_wgrad_update: the kernels that keep a kernel-ready filter copy in step do not fit this shape");
+    return launch_conv_any_wgrad_update({N, H, W, C, K, R, S, stride, pad}, act, err, w, w_channels, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, g8_out,
+                                        dw_out, workspace, static_cast<hipStream_t>(stream));
+  }
   return launch_wgrad3x3_update(act, err, w, w_channels, N, H, C, K, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, g8_out,
                                 dw_out, w_prepared, workspace, static_cast<hipStream_t>(stream));
 }

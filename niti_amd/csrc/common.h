@@ -243,7 +243,14 @@ struct RequantSpec {
 long long sync_spin_limit();
 // this device's word that every grid-wide wait sets when it gives up (api.hip); nullptr if it cannot be looked up
 uint32_t* timeout_word();
+int wgrad_finish_blocks(long long elements);
 int wgrad3x3_finish_blocks(int C, int K);
+// partial sums in slices [K][R][S][C] -> int32 gradient, or -> rounded gradient -> updated weights (sync words: slots of
+// wgrad_finish_blocks workgroups)
+int launch_wgrad_reduce(const int32_t* partial, long long slice_stride, int splits, int32_t* dw, int64_t n, bool roundtrip, uint32_t* absmax,
+                        hipStream_t stream);
+int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, hipStream_t stream);
 size_t wgrad3x3_sync_words(int blocks);
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
                            bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep,

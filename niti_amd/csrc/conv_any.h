@@ -1,0 +1,31 @@
+// int8 convolutions of any map, filter and channel count (multiples of 16 where stated), read as stored (conv_any.hip).
+#pragma once
+#include "common.h"
+
+namespace niti {
+
+// the forward convolution's extents
+struct ConvShape {
+  int N, H, W, C, K, R, S, stride, pad;
+  int P() const { return (H + 2 * pad - R) / stride + 1; }
+  int Q() const { return (W + 2 * pad - S) / stride + 1; }
+};
+
+enum ConvPass { kConvForward = 0, kConvDgrad = 1, kConvWgrad = 2 };
+
+bool conv_any_shape(ConvPass pass, const ConvShape& s);   // extents and channel counts the kernels take (16-byte aligned pointers)
+// forward: a = x, b = w; data gradient: a = error map, b = w (stride 1).  int32 sums, range folded into absmax.
+int launch_conv_any(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int32_t* y, bool roundtrip, uint32_t* absmax, hipStream_t stream);
+// the same rounded to int8 in the launch: sync words, 0 when no tile's grid is resident at once
+size_t conv_any_requant_words(ConvPass pass, const ConvShape& s);
+int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int8_t* y, bool roundtrip, uint32_t* sync,
+                            const RequantSpec& rq, hipStream_t stream);
+// weight gradient (stride 1)
+size_t conv_any_wgrad_workspace(const ConvShape& s);
+int launch_conv_any_wgrad(const ConvShape& s, const int8_t* act, const int8_t* err, int32_t* dw, bool roundtrip, uint32_t* absmax, void* workspace,
+                          hipStream_t stream);
+size_t conv_any_wgrad_update_words(const ConvShape& s);
+int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const int8_t* err, int8_t* w, int w_channels, bool roundtrip, uint32_t* sync,
+                                 const RequantSpec& rq, int8_t* g8, int32_t* dw, void* workspace, hipStream_t stream);
+
+}  // namespace niti

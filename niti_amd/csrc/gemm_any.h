@@ -15,6 +15,7 @@ struct AnyArgs {
   // result rounded to int8, or rounded and subtracted from the weights
   int8_t* out8 = nullptr;   // [m][n]; weight update: the rounded gradient, may be null
   int8_t* w = nullptr;      // [m][n], weight update only
+  const int8_t* mask = nullptr;   // laid out like out8: results are zero where it is not positive (not for the weight update)
   const int32_t* rand = nullptr;
   uint32_t* sync = nullptr;
   int target_bits = 7, method = 0, trunc = 0, bw_mode = 0;

@@ -332,11 +332,16 @@ PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     at::Tensor y, shift, pooled, e = scalar32(x);
     f.exp_out = &e;
     if (fuse) {
-      if (pool && f.relu && f.stride == 1 && f.pad == 1 && d.R == 3 && d.S == 3 && d.H == d.W && d.H >= 2 && d.H % 2 == 0) {
+      // the 3x3 kernels' maps
+      if (pool && f.relu && f.stride == 1 && f.pad == 1 && d.R == 3 && d.S == 3 && d.H == d.W && d.H >= 2 && d.H <= 32 && (d.H & (d.H - 1)) == 0) {
         pooled = empty8({d.N, d.H / 2, d.W / 2, d.K}, x);
         f.pool_out = &pooled;
       }
       if (conv_requant(x, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_fprop_requant")) return tuple_of({y, e, pooled});
+      if (f.pool_out != nullptr) {
+        f.pool_out = nullptr;
+        if (conv_requant(x, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_fprop_requant")) return tuple_of({y, e, at::Tensor()});
+      }
     }
     uint32_t* am = arena_take(1, x, nullptr);
     at::Tensor acc = fprop_i32(x, w, f.stride, f.pad, f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u, am, f.prepared);
@@ -381,7 +386,7 @@ PyObject* layer_dgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
     f.exp_out = &e;
     PyObject* unpooled = Py_False;
     bool done = false;
-    if (fuse && pool_in != nullptr) {
+    if (fuse && pool_in != nullptr && d.H == d.W && d.H <= 32 && (d.H & (d.H - 1)) == 0) {
       f.pool_in = pool_in;
       done = conv_requant(err, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant_unpool");
       if (done) unpooled = Py_True;

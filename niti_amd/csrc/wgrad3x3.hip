@@ -1151,28 +1151,33 @@ static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N,
   return launch_geom<8, 8, 2>(a, splits, stream);
 }
 
+int launch_wgrad_reduce(const int32_t* partial, long long slice_stride, int splits, int32_t* dw, int64_t n, bool roundtrip, uint32_t* absmax,
+                        hipStream_t stream) {
+  int64_t g = (n / 4 + 63) / 64;
+  if (g < 1) g = 1;
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(static_cast<unsigned>(g)), dim3(256), 0, stream, partial, dw, n, static_cast<int64_t>(slice_stride), splits,
+                     roundtrip ? 1 : 0, absmax);
+  return check_launch("wgrad_reduce");
+}
+
 int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, int H, int C, int K, bool roundtrip,
                     uint32_t* absmax, void* workspace, hipStream_t stream) {
   WgradArgs a;
   int splits = 1;
   const int st = launch_wgrad3x3_partials(act, err, N, H, C, K, C, workspace, a, splits, stream);
   if (st != NITI_OK) return st;
-  const int64_t n = static_cast<int64_t>(K) * 9 * C;
-  int64_t g = (n / 4 + 63) / 64;
-  if (g < 1) g = 1;
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(static_cast<unsigned>(g)), dim3(256), 0, stream, a.partial, dw, n,
-                     static_cast<int64_t>(a.slice_stride), splits, roundtrip ? 1 : 0, absmax);
-  return check_launch("wgrad_reduce");
+  return launch_wgrad_reduce(a.partial, a.slice_stride, splits, dw, static_cast<int64_t>(K) * 9 * C, roundtrip, absmax, stream);
 }
 
-// Workgroups of the finishing kernel for a [K][9][C] gradient (= sync slots), or 0 when it is too large for
+// Workgroups of the finishing kernel for a gradient of that many elements (= sync slots), or 0 when it is too large for
 // the kernel's per-workgroup share.
-int wgrad3x3_finish_blocks(int C, int K) {
-  const long long groups = (static_cast<long long>(K) * 9 * C / 4 + 63) / 64;
+int wgrad_finish_blocks(long long elements) {
+  const long long groups = (elements / 4 + 63) / 64;
   const long long nb = groups < 1024 ? groups : 1024;
   if (groups > nb * kFinishV) return 0;
   return static_cast<int>(nb < 1 ? 1 : nb);
 }
+int wgrad3x3_finish_blocks(int C, int K) { return wgrad_finish_blocks(static_cast<long long>(K) * 9 * C); }
 
 // header, range slots (of the finishing launch or of the one-launch form, whichever has more workgroups), arrival slots
 static size_t range_slot_words(int blocks) { return slot_words(blocks > kArriveSlots ? blocks : kArriveSlots); }
@@ -1181,6 +1186,60 @@ size_t wgrad3x3_sync_words(int blocks) {
   return static_cast<size_t>(kFinishSlot0) + range_slot_words(blocks) + slot_words(kArriveSlots) + 16 + kArriveSlots;
 }
 static size_t wgrad3x3_arrive_offset(int C, int K) { return static_cast<size_t>(kFinishSlot0) + range_slot_words(wgrad3x3_finish_blocks(C, K)); }
+
+static FinishArgs finish_args(long long elements, int C, int8_t* w, int w_channels, bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8,
+                              int32_t* dw) {
+  FinishArgs f{};
+  f.nv = elements / 4;
+  f.C = C;
+  f.Cw = w_channels;
+  f.w = w;
+  f.g8 = g8;
+  f.dw = dw;
+  f.sync = sync;
+  f.roundtrip = roundtrip ? 1 : 0;
+  f.target_bits = rq.target_bits;
+  f.method = rq.method;
+  f.trunc = rq.trunc;
+  f.predict = (rq.flags & NITI_RQ_SHIFT_HINT) != 0 ? 1 : 0;
+  f.bw_mode = rq.bw_mode;
+  f.spin_limit = rq.spin_limit;
+  f.sticky = rq.sticky;
+  f.shift_out = rq.shift_out;
+  f.exp_a = rq.exp_a;
+  f.exp_b = rq.exp_b;
+  f.exp_out = rq.exp_out;
+  return f;
+}
+
+// the finishing launch on its own
+static int launch_finish(FinishArgs f, const int32_t* partial, long long slice_stride, int splits, hipStream_t stream) {
+  const int nb = wgrad_finish_blocks(f.nv * 4);
+  static int resident_of[kDeviceSlots][2] = {};   // workgroups of 4 / 16 wavefronts the device holds at once
+  int* const resident = resident_of[device_slot()];
+  if (resident[0] == 0) {
+    int dev = 0, cus = 0, per4 = 0, per16 = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per4, reinterpret_cast<const void*>(wgrad_finish_kernel<4>), 256, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per16, reinterpret_cast<const void*>(wgrad_finish_kernel<16>), 1024, 0) != hipSuccess)
+      return fail(NITI_ERR_LAUNCH, "wgrad_update: cannot query occupancy");
+    resident[0] = cus * per4;
+    resident[1] = cus * per16;
+  }
+  if (nb == 0 || nb > resident[0]) return fail(NITI_ERR_UNSUPPORTED, "wgrad_update: %d workgroups do not fit on the device at once (%d)", nb, resident[0]);
+  f.partial = partial;
+  f.slice_stride = slice_stride;
+  f.splits = splits;
+  // many slices and few columns per workgroup: sixteen wavefronts share the slices
+  if (splits >= 32 && nb <= resident[1]) hipLaunchKernelGGL(wgrad_finish_kernel<16>, dim3(nb), dim3(1024), 0, stream, f);
+  else hipLaunchKernelGGL(wgrad_finish_kernel<4>, dim3(nb), dim3(256), 0, stream, f);
+  return check_launch("wgrad_finish");
+}
+
+int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, hipStream_t stream) {
+  return launch_finish(finish_args(elements, C, w, w_channels, roundtrip, sync, rq, g8, dw), partial, slice_stride, splits, stream);
+}
 
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
                            bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep,
@@ -1207,43 +1266,12 @@ int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int 
   }
   if (!wgrad3x3_supported(N, H, H, C, K, 3, 3, 1, 1))
     return fail(NITI_ERR_UNSUPPORTED, "wgrad_update: %d pixels on %d x %d maps run only as the one-launch kernel, which this call cannot use", N * H * H, H, H);
-  static int resident_of[kDeviceSlots][2] = {};   // workgroups of 4 / 16 wavefronts the device holds at once
-  int* const resident = resident_of[device_slot()];
-  if (resident[0] == 0) {
-    int dev = 0, cus = 0, per4 = 0, per16 = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per4, reinterpret_cast<const void*>(wgrad_finish_kernel<4>), 256, 0) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per16, reinterpret_cast<const void*>(wgrad_finish_kernel<16>), 1024, 0) != hipSuccess)
-      return fail(NITI_ERR_LAUNCH, "wgrad_update: cannot query occupancy");
-    resident[0] = cus * per4;
-    resident[1] = cus * per16;
-  }
-  if (nb > resident[0]) return fail(NITI_ERR_UNSUPPORTED, "wgrad_update: %d workgroups do not fit on the device at once (%d)", nb, resident[0]);
-  WgradArgs a;
-  int splits = 1;
-  FinishArgs f{};
-  f.nv = static_cast<long long>(K) * 9 * Cp / 4;
-  f.C = Cp;
-  f.Cw = w_channels;
-  f.w = w;
-  f.g8 = g8;
-  f.dw = dw;
+  FinishArgs f = finish_args(static_cast<long long>(K) * 9 * Cp, Cp, w, w_channels, roundtrip, sync, rq, g8, dw);
   f.wprep = wprep;
-  f.sync = sync;
-  f.roundtrip = roundtrip ? 1 : 0;
-  f.target_bits = rq.target_bits;
-  f.method = rq.method;
-  f.trunc = rq.trunc;
-  f.predict = (rq.flags & NITI_RQ_SHIFT_HINT) != 0 ? 1 : 0;
-  f.bw_mode = rq.bw_mode;
-  f.spin_limit = rq.spin_limit;
-  f.sticky = rq.sticky;
-  f.shift_out = rq.shift_out;
-  f.exp_a = rq.exp_a;
-  f.exp_b = rq.exp_b;
-  f.exp_out = rq.exp_out;
   f.arrive = sync + wgrad3x3_arrive_offset(C, K);
   f.wide = f.arrive + slot_words(kArriveSlots);
+  WgradArgs a;
+  int splits = 1;
   {
     // main loop and finishing pass as one launch where its grid is resident at once (NITI_WGRAD_ONE_LAUNCH=0 pins the pair)
     const char* e = getenv("NITI_WGRAD_ONE_LAUNCH");
@@ -1254,13 +1282,7 @@ int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int 
   }
   const int st = launch_wgrad3x3_partials(act, err, N, H, C, K, Cp, workspace, a, splits, stream);
   if (st != NITI_OK) return st;
-  f.partial = a.partial;
-  f.slice_stride = a.slice_stride;
-  f.splits = splits;
-  // many slices and few columns per workgroup: sixteen wavefronts share the slices
-  if (splits >= 32 && nb <= resident[1]) hipLaunchKernelGGL(wgrad_finish_kernel<16>, dim3(nb), dim3(1024), 0, stream, f);
-  else hipLaunchKernelGGL(wgrad_finish_kernel<4>, dim3(nb), dim3(256), 0, stream, f);
-  return check_launch("wgrad_finish");
+  return launch_finish(f, a.partial, a.slice_stride, splits, stream);
 }
 
 }  // namespace niti

@@ -1252,3 +1252,59 @@ def test_conv_ragged_batches(dev, case):
     assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
     assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref))
     assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q))
+
+
+# (N, H, W, C, K, filter, stride, padding): edges of the 32 / 64 / 128 / 256 tiles and of the reduction's chunks, taps that fall
+# outside on every side, maps smaller than the filter, one pixel, strides, output channels that are no multiple of anything
+ANY_CONVS = [(1, 1, 1, 16, 16, 3, 1, 1), (1, 5, 5, 32, 48, 3, 1, 1), (3, 7, 9, 32, 48, 3, 1, 1), (2, 4, 5, 128, 144, 5, 1, 2), (5, 13, 6, 48, 32, 1, 1, 0),
+             (2, 6, 6, 16, 64, 5, 1, 0), (9, 14, 14, 96, 160, 3, 1, 1), (1, 20, 11, 80, 272, 3, 1, 2), (4, 28, 28, 64, 70, 3, 2, 1), (3, 9, 12, 48, 1, 3, 2, 0),
+             (2, 16, 16, 112, 21, 5, 2, 2), (7, 8, 8, 16, 33, 1, 2, 0), (2, 10, 3, 528, 32, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", "3", ""])
+@pytest.mark.parametrize("case", ANY_CONVS)
+def test_convolutions_of_any_shape(dev, case, tile, monkeypatch):
+    """The kernels for maps, filters and channel counts outside the 3x3 kernels: int32 sums, rounded results, data gradient and
+    weight gradient with update (split and whole), every tile pinned and the dispatch's own choice ('')."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, H, W, C, K, R, stride, pad = case
+    if tile:
+        monkeypatch.setenv("NITI_ANY_TILE", tile)
+    _say("convolutions_of_any_shape", case, tile)
+    g = torch.Generator().manual_seed(8800 + N + H + C + K)
+    x, w = ri8(g, N, H, W, C), ri8(g, K, R, R, C)
+    xd, wd = x.to(dev), w.to(dev)
+    acc = co.conv_fprop(x, w, stride, pad)
+    am = ops.new_scalar_u32(dev)
+    assert torch.equal(ops.conv2d_fprop(xd, wd, stride, pad, absmax=am).cpu(), acc) and int(am.cpu()) == po.absmax(acc)
+    rand = torch.randint(0, 1 << 20, acc.shape, generator=g, dtype=torch.int32)
+    for method in ("round", "psto", "sto"):
+        u = rand % (1 << max(po.RangeEstimate(acc, "int") - 7, 0)) if method == "sto" else None
+        y, sh, sync = ops.conv2d_fprop_requant(xd, wd, stride, pad, method=method, relu=True, any_shape=True, rand=None if u is None else u.to(torch.int32).to(dev))
+        assert torch.equal(y.cpu(), torch.clamp(po.act_calc(acc, 0, method, rand=u)[0], min=0)) and int(sync.cpu()[1]) == 0, method
+    if stride != 1 or K % 16 != 0:
+        return
+    P, Q = acc.shape[1:3]
+    e = ri8(g, N, P, Q, K, lo=-40, hi=40)
+    ed = e.to(dev)
+    dacc = co.conv_dgrad(e, w, H, W, 1, pad)
+    am = ops.new_scalar_u32(dev)
+    assert torch.equal(ops.conv2d_dgrad(ed, wd, 1, pad, absmax=am).cpu(), dacc) and int(am.cpu()) == po.absmax(dacc)
+    mask = ri8(g, N, H, W, C)
+    dref, dsh = po.err_calc(dacc)
+    y, sh, _ = ops.conv2d_dgrad_requant(ed, wd, 1, pad, relu_mask=mask.to(dev), any_shape=True)
+    assert torch.equal(y.cpu(), dref * (mask > 0)) and int(sh.cpu()) == dsh
+    wacc = co.conv_wgrad(x, e, R, R, 1, pad)
+    g8_ref, sh_ref = po.grad_calc(wacc, 5, "psto")
+    for slices in ("1", "3", ""):
+        monkeypatch.setenv("NITI_ANY_SLICES", slices) if slices else monkeypatch.delenv("NITI_ANY_SLICES")
+        am = ops.new_scalar_u32(dev)
+        assert torch.equal(ops.conv2d_wgrad(xd, ed, R, R, 1, pad, absmax=am).cpu(), wacc) and int(am.cpu()) == po.absmax(wacc)
+        for want_dw in (False, True):
+            wu = w.to(dev)
+            g8, dw, sh, sync = ops.conv2d_wgrad_update(xd, ed, wu, 1, pad, want_grad=True, want_dw=want_dw)
+            assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
+            assert torch.equal(wu.cpu(), po.weight_update(w, g8_ref))
+            assert not want_dw or torch.equal(dw.cpu(), wacc)
