@@ -38,6 +38,8 @@ enum {
                                         by niti_conv2d_i8_filter_prepare for the same shape; no workspace */
 #define NITI_CONV_SHIFT_HINT 8u /* niti_conv2d_i8_wgrad_update only: *shift_out holds a predicted shift on entry, see
                                    NITI_RQ_SHIFT_HINT */
+#define NITI_CONV_ANY_KERNEL 16u /* niti_conv2d_i8_wgrad_update only: a 3x3 gradient runs on the kernel for any shape where
+                                    the batch is too small for the 9-tap kernel to pay (same results) */
 #define NITI_CONV_FILTER_FORWARD_COPY 4u /* data gradient only, with NITI_CONV_FILTER_PREPARED: `w` is the
                                             copy that niti_conv2d_i8_filter_prepare(.., dgrad = 0) made of
                                             the same filter (the one the forward pass reads) */

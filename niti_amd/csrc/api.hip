@@ -533,7 +533,11 @@ extern "C" size_t niti_conv2d_i8_wgrad_workspace(int N, int H, int W, int C, int
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || pad < 0) return 0;
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
   if (P <= 0 || Q <= 0) return 0;
-  if (wgrad3x3_supported(N, H, W, C, K, R, S, 1, pad)) return round256(wgrad3x3_workspace(N, H, C, K));
+  if (wgrad3x3_supported(N, H, W, C, K, R, S, 1, pad)) {
+    const size_t own = wgrad3x3_workspace(N, H, C, K);
+    const size_t any = wgrad3x3_prefers_any(N, H, C, K) ? conv_any_wgrad_workspace({N, H, W, C, K, R, S, 1, pad}) : 0;
+    return round256(any > own ? any : own);
+  }
   const size_t np = static_cast<size_t>(round16(N));
   const size_t copies = round256(static_cast<size_t>(C) * H * W * np) + round256(static_cast<size_t>(K) * P * Q * np);
   const size_t slices = round256(conv_any_wgrad_workspace({N, H, W, C, K, R, S, 1, pad}));
@@ -591,7 +595,10 @@ extern "C" size_t niti_conv2d_i8_wgrad_update_sync_words(int N, int H, int W, in
   if (!wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && !wgrad_small_shape(N, H, W, C, K, R, S, stride, pad))
     return conv_any_wgrad_update_words({N, H, W, C, K, R, S, stride, pad});
   const int nb = wgrad3x3_finish_blocks(C, K);
-  return nb > 0 ? wgrad3x3_sync_words(nb) + wgrad_first_extra_words(H, C, K) : 0;
+  if (nb == 0) return 0;
+  const size_t own = wgrad3x3_sync_words(nb) + wgrad_first_extra_words(H, C, K);
+  const size_t any = wgrad3x3_prefers_any(N, H, C, K) ? conv_any_wgrad_update_words({N, H, W, C, K, R, S, stride, pad}) : 0;
+  return any > own ? any : own;
 }
 
 extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int W,
@@ -602,7 +609,7 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
                                            void* stream) {
   clear_error();
   int st = check_conv_dims("conv_wgrad_update", N, H, W, C, K, R, S, stride, pad);
-  if (st == NITI_OK) st = check_flags("conv_wgrad_update", flags, NITI_EPI_F32_ROUNDTRIP | NITI_CONV_SHIFT_HINT);
+  if (st == NITI_OK) st = check_flags("conv_wgrad_update", flags, NITI_EPI_F32_ROUNDTRIP | NITI_CONV_SHIFT_HINT | NITI_CONV_ANY_KERNEL);
   if (st != NITI_OK) return st;
   if (act == nullptr || err == nullptr || w == nullptr || sync == nullptr)
     return fail(NITI_ERR_INVALID_ARG, "conv_wgrad_update: null pointer");
@@ -624,12 +631,12 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
     return fail(NITI_ERR_INVALID_ARG, "conv_wgrad_update: w and g8_out must be 4-byte aligned");
   if (w_prepared != nullptr && (filter_copy_kind(N, H, W, C, K, R, S, stride, pad, 0) != 2 || reinterpret_cast<uintptr_t>(w_prepared) % 4 != 0))
     return fail(NITI_ERR_UNSUPPORTED, "conv_wgrad_update: w_prepared needs a shape whose forward pass uses a kernel-ready filter copy, 4-byte aligned");
-  RequantSpec rq{mu, method, div_mode == NITI_DIV_TRUNC, bw_mode, (flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u, sync_spin_limit(),
+  RequantSpec rq{mu, method, div_mode == NITI_DIV_TRUNC, bw_mode, ((flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u) | ((flags & NITI_CONV_ANY_KERNEL) ? NITI_RQ_ANY_SHAPE : 0u), sync_spin_limit(),
                  timeout_word(), shift_out, exp_a, exp_b, exp_out, nullptr, nullptr};
   if (!wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && !wgrad_small_shape(N, H, W, C, K, R, S, stride, pad)) {
     if (w_prepared != nullptr) return fail(NITI_ERR_UNSUPPORTED, "conv_wgrad_update: the kernels that keep a kernel-ready filter copy in step do not fit this shape");
     return launch_conv_any_wgrad_update({N, H, W, C, K, R, S, stride, pad}, act, err, w, w_channels, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, g8_out,
-                                        dw_out, workspace, static_cast<hipStream_t>(stream));
+                                        dw_out, nullptr, workspace, static_cast<hipStream_t>(stream));
   }
   return launch_wgrad3x3_update(act, err, w, w_channels, N, H, C, K, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, g8_out,
                                 dw_out, w_prepared, workspace, static_cast<hipStream_t>(stream));

@@ -212,6 +212,7 @@ int launch_post_i32(int32_t* v, int64_t n, bool roundtrip, uint32_t* absmax, hip
 // native 3x3 / stride 1 / pad 1 weight gradient (wgrad3x3.hip)
 bool wgrad3x3_supported(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 size_t wgrad3x3_workspace(int N, int H, int C, int K);
+bool wgrad3x3_prefers_any(int N, int H, int C, int K);   // few pixels: conv_any.hip's kernel is the faster one
 int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, int H, int C, int K, bool roundtrip,
                     uint32_t* absmax, void* workspace, hipStream_t stream);
 
@@ -250,7 +251,7 @@ int wgrad3x3_finish_blocks(int C, int K);
 int launch_wgrad_reduce(const int32_t* partial, long long slice_stride, int splits, int32_t* dw, int64_t n, bool roundtrip, uint32_t* absmax,
                         hipStream_t stream);
 int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
-                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, hipStream_t stream);
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream);
 size_t wgrad3x3_sync_words(int blocks);
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
                            bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep,

@@ -22,10 +22,11 @@ int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* a, 
                             const RequantSpec& rq, hipStream_t stream);
 // weight gradient (stride 1)
 size_t conv_any_wgrad_workspace(const ConvShape& s);
+double conv_any_wgrad_us(const ConvShape& s);   // estimated time with update, 0: not a shape of these kernels
 int launch_conv_any_wgrad(const ConvShape& s, const int8_t* act, const int8_t* err, int32_t* dw, bool roundtrip, uint32_t* absmax, void* workspace,
                           hipStream_t stream);
 size_t conv_any_wgrad_update_words(const ConvShape& s);
 int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const int8_t* err, int8_t* w, int w_channels, bool roundtrip, uint32_t* sync,
-                                 const RequantSpec& rq, int8_t* g8, int32_t* dw, void* workspace, hipStream_t stream);
+                                 const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, void* workspace, hipStream_t stream);
 
 }  // namespace niti

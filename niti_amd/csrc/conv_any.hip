@@ -15,25 +15,12 @@
 #include "conv_any.h"
 
 #include <stdlib.h>
+#include <string.h>
 
 #include "any_tile.h"
 
 namespace niti {
 namespace {
-
-// x / d for 0 <= x < 2^31: with 2^(s-1) < d <= 2^s and mul = floor(2^(31+s) / d) + 1, mul d exceeds 2^(31+s) by at most d <= 2^s,
-// hence x mul / 2^(31+s) exceeds x / d by less than 1 / d
-struct Reciprocal {
-  uint32_t mul, shift;   // mul 0: d = 1
-  explicit Reciprocal(int d = 1) : mul(0), shift(0) {
-    if (d < 2) return;
-    int s = 1;
-    while ((1LL << s) < d) ++s;
-    mul = static_cast<uint32_t>((1ULL << (31 + s)) / static_cast<unsigned>(d) + 1);
-    shift = static_cast<uint32_t>(s - 1);
-  }
-  __device__ int of(int x) const { return mul != 0u ? static_cast<int>(__umulhi(static_cast<uint32_t>(x), mul) >> shift) : x; }
-};
 
 struct ConvAnyArgs {
   AnyArgs g;
@@ -383,6 +370,7 @@ size_t words_for(long long blocks) { return static_cast<size_t>(kSlot0) + slot_w
 // ---- weight gradient: tile and slices of the reduction
 struct Split {
   int tile, slices, per;   // chunks of a slice
+  double us;               // estimated time
 };
 int chunk_of(int tile) { return tile == 0 ? TileS::BK : tile == 1 ? TileM::BK : TileL::BK; }
 long long slice_of(const ConvShape& s) {
@@ -391,17 +379,16 @@ long long slice_of(const ConvShape& s) {
 }
 // The tile and the number of slices with the least estimated time.  A compute unit's time is its rounds of workgroups times
 // their chunks; a tile costs its prologue and epilogue, and cutting the reduction costs the finishing launch and the partial
-// sums' way through memory.  The constants are a least-squares fit (12% rms) to 19 layers, 1 to 118 GOP, each with every tile
-// and 1 to 64 slices; the pick is within 1.2% of the best of them on the geometric mean.
-Split pick_split(const ConvShape& s) {
-  constexpr double kTile[4] = {5.2, 6.4, 7.3, 8.8}, kChunk[4] = {0.70, 0.64, 0.47, 0.68}, kRound[4] = {0.7, 1.8, 0.0, 0.0};   // us
-  constexpr double kFinish = 2.1, kMillionSums = 1.6;
+// sums' way through memory.  The constants are a least-squares fit (13% rms) to 46 layers, 0.1 to 23 GOP, each with every tile
+// and 1 to 48 slices; the pick is within 2% of the best of them on the geometric mean.
+Split estimate_split(const ConvShape& s) {
+  constexpr double kTile[4] = {6.4, 7.9, 8.7, 10.3}, kChunk[4] = {0.68, 0.61, 0.47, 0.68}, kRound[4] = {0.8, 2.0, 0.0, 0.0};   // us
+  constexpr double kFinish = 2.0, kMillionSums = 1.6;
   int m, n, k;
   product_of(kConvWgrad, s, &m, &n, &k);
   const int pin = pinned_tile();
   const char* e = getenv("NITI_ANY_SLICES");   // pins the number of slices (tests, measurements)
-  Split best{0, 0, 0};
-  double least = 0;
+  Split best{0, 0, 0, 0};
   for (int t = 0; t < 4; ++t) {
     if (pin >= 0 && t != pin) continue;
     const long long tiles = tiles_with(t, m, n);
@@ -415,13 +402,29 @@ Split pick_split(const ConvShape& s) {
       const double rounds = blocks > 512 ? blocks / 256 : blocks > 256 ? 2 : 1;
       double us = kTile[t] + rounds * per * kChunk[t] + (rounds - 1) * kRound[t];
       if (slices > 1 || blocks > 512) us += kFinish + kMillionSums * 1e-6 * slices * static_cast<double>(m) * n;
-      if (best.slices == 0 || us < least) {
-        least = us;
-        best = Split{t, slices, per};
-      }
+      if (best.slices == 0 || us < best.us) best = Split{t, slices, per, us};
     }
   }
   return best;
+}
+
+// the pick for a shape is asked for several times per call: each thread keeps the last few
+Split pick_split(const ConvShape& s) {
+  if (getenv("NITI_ANY_TILE") != nullptr || getenv("NITI_ANY_SLICES") != nullptr) return estimate_split(s);
+  struct Entry {
+    int key[6];
+    Split split;
+  };
+  static thread_local Entry kept[16] = {};
+  const int key[6] = {s.N, s.H * 65536 + s.W, s.C, s.K, s.R * 65536 + s.S, s.pad};
+  unsigned h = 0;
+  for (int v : key) h = h * 31u + static_cast<unsigned>(v);
+  Entry& e = kept[(h ^ (h >> 8)) & 15u];
+  if (memcmp(e.key, key, sizeof(key)) != 0) {
+    memcpy(e.key, key, sizeof(key));
+    e.split = estimate_split(s);
+  }
+  return e.split;
 }
 
 }  // namespace
@@ -478,6 +481,8 @@ size_t conv_any_wgrad_workspace(const ConvShape& s) {
   return static_cast<size_t>(pick_split(s).slices) * slice_of(s) * sizeof(int32_t);
 }
 
+double conv_any_wgrad_us(const ConvShape& s) { return conv_any_shape(kConvWgrad, s) ? pick_split(s).us : 0.0; }
+
 static int launch_slices(const ConvShape& s, const Split& p, const int8_t* act, const int8_t* err, void* workspace, hipStream_t stream) {
   ConvAnyArgs a = args_of(kConvWgrad, s, err, act, false);
   a.g.c = static_cast<int32_t*>(workspace);
@@ -514,7 +519,7 @@ size_t conv_any_wgrad_update_words(const ConvShape& s) {
 }
 
 int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const int8_t* err, int8_t* w, int w_channels, bool roundtrip, uint32_t* sync,
-                                 const RequantSpec& rq, int8_t* g8, int32_t* dw, void* workspace, hipStream_t stream) {
+                                 const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, void* workspace, hipStream_t stream) {
   const Split p = pick_split(s);
   int m, n, k;
   product_of(kConvWgrad, s, &m, &n, &k);
@@ -523,6 +528,9 @@ int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const in
     ConvAnyArgs a = args_of(kConvWgrad, s, err, act, roundtrip);
     set_rounding(a.g, rq, sync);
     a.g.w = w;
+    a.g.wprep = wprep;
+    a.g.channels = s.C;
+    a.g.by_channels = Reciprocal(s.C);
     a.g.out8 = g8;
     a.chunks_per_slice = p.per;
     return launch_tile<kConvWgrad, kUpdate>(p.tile, a, 1, stream);
@@ -530,7 +538,7 @@ int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const in
   const int st = launch_slices(s, p, act, err, workspace, stream);
   if (st != NITI_OK) return st;
   return launch_wgrad_finish(static_cast<const int32_t*>(workspace), slice_of(s), p.slices, static_cast<long long>(m) * n, s.C, w, w_channels, roundtrip, sync,
-                             rq, g8, dw, stream);
+                             rq, g8, dw, wprep, stream);
 }
 
 }  // namespace niti

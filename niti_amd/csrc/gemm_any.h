@@ -4,6 +4,20 @@
 
 namespace niti {
 
+// x / d for 0 <= x < 2^31: with 2^(s-1) < d <= 2^s and mul = floor(2^(31+s) / d) + 1, mul d exceeds 2^(31+s) by at most d <= 2^s,
+// hence x mul / 2^(31+s) exceeds x / d by less than 1 / d
+struct Reciprocal {
+  uint32_t mul, shift;   // mul 0: d = 1
+  explicit Reciprocal(int d = 1) : mul(0), shift(0) {
+    if (d < 2) return;
+    int s = 1;
+    while ((1LL << s) < d) ++s;
+    mul = static_cast<uint32_t>((1ULL << (31 + s)) / static_cast<unsigned>(d) + 1);
+    shift = static_cast<uint32_t>(s - 1);
+  }
+  __device__ int of(int x) const { return mul != 0u ? static_cast<int>(__umulhi(static_cast<uint32_t>(x), mul) >> shift) : x; }
+};
+
 struct AnyArgs {
   const int8_t* a;       // [m][k], or [k][m] when transposed
   const int8_t* b;       // [n][k] when transposed, or [k][n]
@@ -15,6 +29,9 @@ struct AnyArgs {
   // result rounded to int8, or rounded and subtracted from the weights
   int8_t* out8 = nullptr;   // [m][n]; weight update: the rounded gradient, may be null
   int8_t* w = nullptr;      // [m][n], weight update only
+  int8_t* wprep = nullptr;  // weight update of a [m][9][channels] filter: the 3x3 forward kernel's copy of it, kept in step
+  int channels = 0;
+  Reciprocal by_channels{};
   const int8_t* mask = nullptr;   // laid out like out8: results are zero where it is not positive (not for the weight update)
   const int32_t* rand = nullptr;
   uint32_t* sync = nullptr;

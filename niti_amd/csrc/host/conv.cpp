@@ -487,7 +487,7 @@ PyObject* layer_wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Opt shift = a.opt(), exp_a = a.opt(), exp_b = a.opt(), prepared = a.opt(), rand = a.opt();
     at::Tensor e = scalar32(act);
     Update u;
-    bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, flags | (shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), r, want_grad, want_dw,
+    bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, flags | NITI_CONV_ANY_KERNEL | (shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), r, want_grad, want_dw,
                                           nullptr, shift, exp_a, exp_b, ptr<int32_t>(e), nullptr, prepared, true, &u, nullptr);
     if (one) {
       if (want_dw && u.dw.size(3) != w.size(3)) u.dw = u.dw.slice(3, 0, w.size(3)).contiguous();

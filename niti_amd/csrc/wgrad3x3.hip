@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "conv_any.h"
 #include "lds_asm.h"
 #include "requant_math.h"
 
@@ -1115,6 +1116,22 @@ size_t wgrad3x3_workspace(int N, int H, int C, int K) {
   return static_cast<size_t>(pick_splits(N, H, C, K)) * slice_stride_for(C, K) * sizeof(int32_t);
 }
 
+// With few pixels most of this kernel's time is its 9-tap sums' way through memory, whatever the batch: 14.5 us + 1.55 per
+// band of 256 pixels a workgroup walks + 0.3 per MB of partial sums (within 15% over 1 to 200 images of 8 x 8 to 32 x 32, 128
+// to 512 channels).  The kernel for any shape starts lower and grows faster: 8 images of 16 x 16, 256 -> 256 channels 21.3
+// against 11.7 us, 24 images 25.8 / 21.0, 80 images 33.5 / 37.2 (a fifth is kept as margin: operands that the launch before
+// has just written cost its many tiles more).  NITI_WGRAD_ANY=0 / 1 pins the choice (tests), as do the other
+// pins of this file.
+bool wgrad3x3_prefers_any(int N, int H, int C, int K) {
+  const char* e = getenv("NITI_WGRAD_ANY");
+  const double any = conv_any_wgrad_us({N, H, H, C, K, 3, 3, 1, 1});
+  if (any == 0.0) return false;
+  if (e != nullptr) return e[0] != '0';
+  if (getenv("NITI_WGRAD_ONE_LAUNCH") != nullptr || getenv("NITI_WGRAD_BLOCKS") != nullptr || !use_narrow_arrangement(N, H)) return false;
+  const int splits = pick_splits(N, H, C, K), bands = (N * H * H + 255) / 256;
+  return any < 0.8 * (14.5 + 1.55 * ((bands + splits - 1) / splits) + 0.3e-6 * static_cast<double>(wgrad3x3_workspace(N, H, C, K)));
+}
+
 static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N, int H, int C, int K, int Cp, void* workspace,
                                     WgradArgs& a, int& splits, hipStream_t stream, FinishArgs* finish = nullptr) {
   a.act = act;
@@ -1162,6 +1179,7 @@ int launch_wgrad_reduce(const int32_t* partial, long long slice_stride, int spli
 
 int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, int H, int C, int K, bool roundtrip,
                     uint32_t* absmax, void* workspace, hipStream_t stream) {
+  if (wgrad3x3_prefers_any(N, H, C, K)) return launch_conv_any_wgrad({N, H, H, C, K, 3, 3, 1, 1}, act, err, dw, roundtrip, absmax, workspace, stream);
   WgradArgs a;
   int splits = 1;
   const int st = launch_wgrad3x3_partials(act, err, N, H, C, K, C, workspace, a, splits, stream);
@@ -1237,8 +1255,10 @@ static int launch_finish(FinishArgs f, const int32_t* partial, long long slice_s
 }
 
 int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
-                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, hipStream_t stream) {
-  return launch_finish(finish_args(elements, C, w, w_channels, roundtrip, sync, rq, g8, dw), partial, slice_stride, splits, stream);
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream) {
+  FinishArgs f = finish_args(elements, C, w, w_channels, roundtrip, sync, rq, g8, dw);
+  f.wprep = wprep;
+  return launch_finish(f, partial, slice_stride, splits, stream);
 }
 
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
@@ -1264,6 +1284,8 @@ int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int 
     if ((e == nullptr || e[0] != '0') && wgrad_small_supported(N, H, C, K, w_channels))
       return launch_wgrad_small_update(act, err, w, N, H, C, K, roundtrip, sync, rq, g8, dw, wprep, stream);
   }
+  if ((rq.flags & NITI_RQ_ANY_SHAPE) != 0 && w_channels == C && wgrad3x3_prefers_any(N, H, C, K))
+    return launch_conv_any_wgrad_update({N, H, H, C, K, 3, 3, 1, 1}, act, err, w, w_channels, roundtrip, sync, rq, g8, dw, wprep, workspace, stream);
   if (!wgrad3x3_supported(N, H, H, C, K, 3, 3, 1, 1))
     return fail(NITI_ERR_UNSUPPORTED, "wgrad_update: %d pixels on %d x %d maps run only as the one-launch kernel, which this call cannot use", N * H * H, H, H);
   FinishArgs f = finish_args(static_cast<long long>(K) * 9 * Cp, Cp, w, w_channels, roundtrip, sync, rq, g8, dw);

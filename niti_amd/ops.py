@@ -209,15 +209,16 @@ def wgrad_update_sync_words(N, H, W, C, K, R=3, S=3, stride=1, padding=1) -> int
 
 def conv2d_wgrad_update(act, err, w, stride=1, padding=1, f32_epilogue=False, mu=5, method="psto", div_mode="floor",
                         bw_mode="int", sync=None, want_grad=False, want_dw=False, shift_out=None, exp_a=None, exp_b=None,
-                        exp_out=None, workspace=None, prepared_filter=None, shift_hint=False):
+                        exp_out=None, workspace=None, prepared_filter=None, shift_hint=False, any_kernel=False):
     """Weight gradient + grad_calc + weight update: act [N,H,W,C] int8 (C may carry zero channel padding), err
     [N,H,W,K] int8, w [K,3,3,Cw] int8 updated in place.  Returns (g8 or None, dw int32 or None, device shift, sync).
     ``prepared_filter``: conv_filter_prepare(w padded to C channels, N, H, W) made earlier; it receives the updated
     weights too and stays valid for the next forward pass.  ``shift_hint``: ``shift_out`` holds a predicted shift
-    on entry (the previous step's): the update's stores then overlap the wait for the tensor's range."""
+    on entry (the previous step's): the update's stores then overlap the wait for the tensor's range.  ``any_kernel``: small
+    batches may run on the kernel for any shape (NITI_CONV_ANY_KERNEL)."""
     if shift_hint and shift_out is None:
         raise RuntimeError("conv2d_wgrad_update: shift_hint needs shift_out, holding the predicted shift")
-    flags = (L.EPI_F32_ROUNDTRIP if f32_epilogue else 0) | (L.CONV_SHIFT_HINT if shift_hint else 0)
+    flags = (L.EPI_F32_ROUNDTRIP if f32_epilogue else 0) | (L.CONV_SHIFT_HINT if shift_hint else 0) | (L.CONV_ANY_KERNEL if any_kernel else 0)
     return L.host().conv_wgrad_update(act, err, w, stride, padding, flags, mu, L.ROUND[method], L.DIV[div_mode], L.BW[bw_mode], sync,
                                       want_grad, want_dw, shift_out, exp_a, exp_b, exp_out, workspace, prepared_filter)
 

@@ -1308,3 +1308,29 @@ def test_convolutions_of_any_shape(dev, case, tile, monkeypatch):
             assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
             assert torch.equal(wu.cpu(), po.weight_update(w, g8_ref))
             assert not want_dw or torch.equal(dw.cpu(), wacc)
+
+
+@pytest.mark.parametrize("case", [(4, 32, 16, 32), (8, 16, 128, 64), (6, 8, 80, 144), (64, 8, 64, 256), (16, 16, 256, 128), (2, 8, 16, 16), (1, 8, 48, 208),
+                                  (3, 16, 32, 64)])
+def test_conv_wgrad_update_small_batches(dev, case, monkeypatch):
+    """3x3 weight gradients with update on the kernel for any shape (which small batches pick), the forward pass's filter copy
+    kept in step."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    monkeypatch.setenv("NITI_WGRAD_ANY", "1")
+    _say("conv_wgrad_update_small_batches", case)
+    g = torch.Generator().manual_seed(991 + C + K)
+    x, e, w = ri8(g, N, Q, Q, C), ri8(g, N, Q, Q, K, lo=-40, hi=40), ri8(g, K, 3, 3, C)
+    acc = co.conv_wgrad(x, e, 3, 3, 1, 1)
+    g8_ref, sh_ref = po.grad_calc(acc, 5, "psto")
+    for slices in ("1", "2", ""):
+        monkeypatch.setenv("NITI_ANY_SLICES", slices) if slices else monkeypatch.delenv("NITI_ANY_SLICES")
+        wd = w.to(dev)
+        prepared = ops.conv_filter_prepare(wd, N, Q, Q)
+        g8, _, sh, sync = ops.conv2d_wgrad_update(x.to(dev), e.to(dev), wd, want_grad=True, prepared_filter=prepared, any_kernel=True)
+        assert torch.equal(g8.cpu(), g8_ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
+        assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref))
+        assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q))
+    assert torch.equal(ops.conv2d_wgrad(x.to(dev), e.to(dev), 3, 3).cpu(), acc)
