@@ -437,6 +437,20 @@ int niti_linear_i8_wgrad_update(const int8_t* err, const int8_t* act, int8_t* w,
                                 int32_t* shift_out, const int32_t* exp_a, const int32_t* exp_b, int32_t* exp_out, void* stream);
 
 /*
+ * TiLinear.backward (ti_torch.py:249-266) as one launch: dx8 = err_calc(err @ w) with the weights as they are on entry, then
+ * w = clip(w - grad_calc(err^T @ act)).  err_exp_out = error shift + exp_err + exp_w, grad_exp_out = gradient shift +
+ * err_exp_out + exp_act.  Roundings as above, the random integers of the error [M][F] and of the gradient [O][F].  Any
+ * alignment; niti_linear_i8_backward_sync_words returns 0 where the workgroups of both do not fit on the current device at
+ * once (then: the two entry points above).
+ */
+size_t niti_linear_i8_backward_sync_words(int M, int O, int F);
+int niti_linear_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int M, int O, int F, int err_bits,
+                            int err_method, int grad_bits, int grad_method, int div_mode, int bw_mode, const int32_t* err_rand,
+                            const int32_t* grad_rand, uint32_t* sync, size_t sync_words, int8_t* g8_out, int32_t* err_shift_out,
+                            int32_t* grad_shift_out, const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act,
+                            int32_t* err_exp_out, int32_t* grad_exp_out, void* stream);
+
+/*
  * Integer cross-entropy gradient, TiLoss.forward (ti_loss.py:5-36), as one launch: out_val [n][classes] int8 logits
  * with exponent *out_exp (device scalar), target [n] int64 class indices, rand [n][classes] int32 random integers
  * (the low four bits stand in for the reference's torch.randint(0, 16)) -> grad [n][classes] int8 with exponent 0.

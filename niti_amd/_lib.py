@@ -78,6 +78,8 @@ SIGNATURES = {
     "niti_linear_i8_fwd_requant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _u, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "niti_linear_i8_dgrad_requant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "niti_linear_i8_wgrad_update": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "niti_linear_i8_backward_sync_words": (_sz, [_i] * 3),
+    "niti_linear_i8_backward": (_i, [_vp, _vp, _vp, _vp] + [_i] * 9 + [_vp, _vp, _vp, _sz] + [_vp] * 9),
     "niti_loss_grad_i8": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "niti_loss_grad_i8_rng": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "niti_rng_words_u32": (_i, [_vp, _u, _vp, _sz, _vp]),

@@ -27,7 +27,7 @@ struct Tile {
   static_assert(WM * WN * WK == 8 && BK % (32 * WK) == 0, "eight wavefronts");
 };
 using TileS = Tile<1, 1, 8, 1, 1, 512, 2, 2>;    //  32 x  32
-using TileM = Tile<2, 2, 2, 1, 1, 256, 2, 4>;    //  64 x  64
+using TileM = Tile<2, 2, 2, 1, 1, 256, 2, 2>;    //  64 x  64
 using TileH = Tile<4, 2, 1, 1, 1, 128, 2, 4>;    // 128 x  64
 using TileL = Tile<2, 4, 1, 2, 1, 128, 2, 2>;    // 128 x 128
 
@@ -132,10 +132,11 @@ struct DenseOperand {
 };
 
 // An operand's load(c, raw) is called for c = first, first + 1, ... in turn, piece(raw, i, c, last) once for each of its pieces.
-// Chunks first .. chunks - 1 of the tile at (m0, n0) of the [g.m][g.n] result; int32 sums go to `out`.
-template <class T, class OpA, class OpB, int MODE>
+// Chunks first .. chunks - 1 of the tile at (m0, n0) of the [g.m][g.n] result; int32 sums go to `out`.  shift_of(largest
+// magnitude of the lane, 32 words of LDS): the shift, for the modes that round.
+template <class T, class OpA, class OpB, int MODE, class ShiftOf>
 __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, OpA oa, OpB ob, const int m0, const int n0, const int first,
-                                         const int chunks, int8_t* const smem) {
+                                         const int chunks, int8_t* const smem, ShiftOf shift_of) {
   constexpr bool TA = !OpA::G::kFast, TB = OpB::G::kFast;
   constexpr int PA = OpA::G::PITCH, PB = OpB::G::PITCH;
   constexpr int BYTES_A = OpA::G::BYTES, BYTES_B = OpB::G::BYTES;
@@ -304,7 +305,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
       if (wave == 0) fold_absmax(g.absmax, lane < 8 ? words[lane] : 0u);
     }
   } else {
-    shift = grid_shift<8>(g, lmax, words, words + 8);
+    shift = shift_of(lmax, words);
   }
   const bool trunc = g.trunc != 0, relu = (g.rq_flags & NITI_RQ_RELU) != 0;
   // what the rounding reads is requested for all of the thread's results in front of the first store (the compiler keeps

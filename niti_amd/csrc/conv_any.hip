@@ -218,16 +218,17 @@ __global__ __launch_bounds__(512) void conv_any_kernel(const ConvAnyArgs a) {
   const int place = (id & 7) * (nb >> 3) + min(id & 7, nb & 7) + (id >> 3);
   const int slice = place / per, tile = place - slice * per;
   const int n0 = tile % nt * T::BN, m0 = tile / nt * T::BM;
+  auto shift_of = [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(a.g, lmax, words, words + 8); };
   if constexpr (PASS == kConvWgrad) {
     const int first = slice * a.chunks_per_slice;
     const int chunks = min((a.g.k + T::BK - 1) / T::BK, first + a.chunks_per_slice);
-    any_tile<T, A, B, MODE>(a.g, a.g.c + slice * a.slice, A(a.g.a, a.g.k, a.g.m, m0), B(a, n0, first), m0, n0, first, chunks, smem);
+    any_tile<T, A, B, MODE>(a.g, a.g.c + slice * a.slice, A(a.g.a, a.g.k, a.g.m, m0), B(a, n0, first), m0, n0, first, chunks, smem, shift_of);
   } else {
     const int chunks = (a.g.k + T::BK - 1) / T::BK;
     if constexpr (PASS == kConvForward)
-      any_tile<T, A, B, MODE>(a.g, a.g.c, A(a, m0), B(a.g.b, a.g.n, a.g.k, n0), m0, n0, 0, chunks, smem);
+      any_tile<T, A, B, MODE>(a.g, a.g.c, A(a, m0), B(a.g.b, a.g.n, a.g.k, n0), m0, n0, 0, chunks, smem, shift_of);
     else
-      any_tile<T, A, B, MODE>(a.g, a.g.c, A(a, m0), B(a, n0), m0, n0, 0, chunks, smem);
+      any_tile<T, A, B, MODE>(a.g, a.g.c, A(a, m0), B(a, n0), m0, n0, 0, chunks, smem, shift_of);
   }
 }
 

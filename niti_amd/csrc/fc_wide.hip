@@ -830,3 +830,64 @@ extern "C" int niti_linear_i8_wgrad_update(const int8_t* err, const int8_t* act,
   else hipLaunchKernelGGL(fcw_wgrad_kernel<4>, grid, dim3(512), wgrad_lds(4), s, a);
   return check_launch(who);
 }
+
+extern "C" size_t niti_linear_i8_backward_sync_words(int M, int O, int F) {
+  int nd = 0, nw = 0;
+  if (M <= 0 || O <= 0 || F <= 0 || !gemm_any_backward_blocks(M, O, F, &nd, &nw)) return 0;
+  return 2 * static_cast<size_t>(kSlot0) + slot_words(nd) + slot_words(nw);
+}
+
+extern "C" int niti_linear_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int M, int O, int F, int err_bits,
+                                       int err_method, int grad_bits, int grad_method, int div_mode, int bw_mode, const int32_t* err_rand,
+                                       const int32_t* grad_rand, uint32_t* sync, size_t sync_words, int8_t* g8_out, int32_t* err_shift_out,
+                                       int32_t* grad_shift_out, const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act,
+                                       int32_t* err_exp_out, int32_t* grad_exp_out, void* stream) {
+  clear_error();
+  const char* who = "linear_backward";
+  if (M <= 0 || O <= 0 || F <= 0) return fail(NITI_ERR_INVALID_ARG, "%s: non-positive extent", who);
+  if (err == nullptr || act == nullptr || w == nullptr || dx8 == nullptr || sync == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: null pointer", who);
+  if (err_bits < 1 || err_bits > 7 || grad_bits < 1 || grad_bits > 7)
+    return fail(NITI_ERR_INVALID_ARG, "%s: target bits %d, %d outside 1..7", who, err_bits, grad_bits);
+  for (int i = 0; i < 2; ++i) {
+    const int method = i == 0 ? err_method : grad_method;
+    const int32_t* const rand = i == 0 ? err_rand : grad_rand;
+    if (method != NITI_ROUND_NEAREST && method != NITI_ROUND_PSEUDO_STOCHASTIC && method != NITI_ROUND_STOCHASTIC)
+      return fail(NITI_ERR_INVALID_ARG, "%s: rounding method %d", who, method);
+    if (method == NITI_ROUND_STOCHASTIC && (rand == nullptr || reinterpret_cast<uintptr_t>(rand) % 4 != 0))
+      return fail(NITI_ERR_INVALID_ARG, "%s: stochastic rounding needs random integers (one int32 per output element)", who);
+  }
+  if (div_mode != NITI_DIV_FLOOR && div_mode != NITI_DIV_TRUNC) return fail(NITI_ERR_INVALID_ARG, "%s: div_mode=%d", who, div_mode);
+  if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
+  int nd = 0, nw = 0;
+  if (!gemm_any_backward_blocks(M, O, F, &nd, &nw))
+    return fail(NITI_ERR_UNSUPPORTED, "%s: the workgroups of M=%d O=%d F=%d do not fit on the device at once", who, M, O, F);
+  const size_t need = 2 * static_cast<size_t>(kSlot0) + slot_words(nd) + slot_words(nw);
+  if (sync_words < need) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, need, sync_words);
+  AnyArgs d{err, w, M, F, O};
+  d.out8 = dx8;
+  d.rand = err_rand;
+  d.sync = sync;
+  d.target_bits = err_bits;
+  d.method = err_method;
+  d.shift_out = err_shift_out;
+  d.exp_a = exp_err;
+  d.exp_b = exp_w;
+  d.exp_out = err_exp_out;
+  AnyArgs g{err, act, O, F, M};
+  g.out8 = g8_out;
+  g.w = w;
+  g.rand = grad_rand;
+  g.sync = sync + kSlot0 + slot_words(nd);
+  g.target_bits = grad_bits;
+  g.method = grad_method;
+  g.shift_out = grad_shift_out;
+  g.exp_b = exp_act;
+  g.exp_out = grad_exp_out;
+  for (AnyArgs* a : {&d, &g}) {
+    a->trunc = div_mode == NITI_DIV_TRUNC ? 1 : 0;
+    a->bw_mode = bw_mode;
+    a->spin_limit = sync_spin_limit();
+    a->sticky = timeout_word();
+  }
+  return launch_gemm_any_backward(d, g, static_cast<hipStream_t>(stream));
+}

@@ -52,5 +52,9 @@ int launch_gemm_any(int trans_a, int trans_b, const AnyArgs& a, hipStream_t stre
 enum AnyRound { kAnyForward = 0, kAnyDgrad = 1, kAnyUpdate = 2 };   // layouts NT, NN, TN
 long long gemm_any_round_blocks(AnyRound what, int m, int n, int k);
 int launch_gemm_any_round(AnyRound what, const AnyArgs& a, hipStream_t stream);
+// Both gradients of a [m][f] -> [m][o] layer as one launch: d = data gradient (NN: error, w), w = update (TN: error, act) whose
+// exponent builds on d's (w.exp_a is not read); workgroups of each = slots of each.  false: not resident together
+bool gemm_any_backward_blocks(int m, int o, int f, int* nd, int* nw);
+int launch_gemm_any_backward(const AnyArgs& d, const AnyArgs& w, hipStream_t stream);
 
 }  // namespace niti

@@ -21,18 +21,42 @@ template <class T, bool TB, bool kAligned> using OperandB = DenseOperand<Pieces<
 template <class T, bool TA, bool TB>
 constexpr int lds_bytes() { return any_lds_bytes<T, OperandA<T, TA, true>, OperandB<T, TB, true>>(); }
 
-template <class T, bool TA, bool TB, int MODE, bool kAligned>
-__global__ __launch_bounds__(512) void gemm_any_kernel(const AnyArgs g) {
-  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+// tile `id` of nt x mt
+template <class T, bool TA, bool TB, int MODE, bool kAligned, class ShiftOf>
+__device__ __forceinline__ void gemm_any_tile(const AnyArgs& g, int id, int nt, int mt, int8_t* smem, ShiftOf shift_of) {
   // Workgroups go to the eight dies in turn, and each die has its own L2: a die takes a run of neighbouring tiles, along the
   // side on which neighbours share the lines of an operand with the reduction index slow.
-  const int nt = gridDim.x, mt = gridDim.y, nb = nt * mt;
-  const int id = blockIdx.y * nt + blockIdx.x;
+  const int nb = nt * mt;
   const int tile = T::BM >= 128 ? id : (id & 7) * (nb >> 3) + min(id & 7, nb & 7) + (id >> 3);
   const int n0 = (TA ? tile / mt : tile % nt) * T::BN, m0 = (TA ? tile % mt : tile / nt) * T::BM;
   const OperandA<T, TA, kAligned> oa(g.a, TA ? g.k : g.m, TA ? g.m : g.k, m0);
   const OperandB<T, TB, kAligned> ob(g.b, TB ? g.n : g.k, TB ? g.k : g.n, n0);
-  any_tile<T, OperandA<T, TA, kAligned>, OperandB<T, TB, kAligned>, MODE>(g, g.c, oa, ob, m0, n0, 0, (g.k + T::BK - 1) / T::BK, smem);
+  any_tile<T, OperandA<T, TA, kAligned>, OperandB<T, TB, kAligned>, MODE>(g, g.c, oa, ob, m0, n0, 0, (g.k + T::BK - 1) / T::BK, smem, shift_of);
+}
+
+template <class T, bool TA, bool TB, int MODE, bool kAligned>
+__global__ __launch_bounds__(512) void gemm_any_kernel(const AnyArgs g) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  gemm_any_tile<T, TA, TB, MODE, kAligned>(g, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y, smem,
+                                           [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(g, lmax, words, words + 8); });
+}
+
+// TiLinear's backward pass as one launch: the first `nd` workgroups take the data gradient, the others the weight gradient and
+// its update, which waits until the old weights have been read.  The two have nothing else to do with each other and each
+// alone is the length of its latency chain on part of the chip: together they take little more than the longer one (100 x
+// 1000 -> 300: 12.9 -> 8.5 us).
+template <class TD, class TW, bool kAligned>
+__global__ __launch_bounds__(512, kAligned || TW::BM < 128 ? 4 : 2) void gemm_backward_kernel(const AnyArgs d, const AnyArgs w, const int nd) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  const int id = blockIdx.x;
+  if (id < nd) {
+    gemm_any_tile<TD, false, false, kRequant, kAligned>(d, id, (d.n + TD::BN - 1) / TD::BN, (d.m + TD::BM - 1) / TD::BM, smem,
+                                                        [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(d, lmax, words, words + 8, id, nd); });
+  } else {
+    const int nw = static_cast<int>(gridDim.x) - nd;
+    gemm_any_tile<TW, true, false, kUpdate, kAligned>(w, id - nd, (w.n + TW::BN - 1) / TW::BN, (w.m + TW::BM - 1) / TW::BM, smem,
+                                                      [&](uint32_t lmax, uint32_t* words) { return grid_shift_behind<8>(w, d, nd, lmax, words, words + 8, id - nd, nw); });
+  }
 }
 
 template <class T>
@@ -128,7 +152,83 @@ int launch_round(const AnyArgs& a, hipStream_t s) {
   }
 }
 
+// ---- data gradient and weight update together
+template <class TD, class TW>
+constexpr int backward_lds() { return lds_bytes<TD, false, false>() > lds_bytes<TW, true, false>() ? lds_bytes<TD, false, false>() : lds_bytes<TW, true, false>(); }
+
+// workgroups of the variant the device holds at once
+template <class TD, class TW, bool kAligned>
+int backward_resident() {
+  static int of[kDeviceSlots] = {};
+  int& r = of[device_slot()];
+  if (r == 0) {
+    auto k = gemm_backward_kernel<TD, TW, kAligned>;
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, backward_lds<TD, TW>()) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k), 512, backward_lds<TD, TW>()) != hipSuccess)
+      return 0;
+    r = cus * per_cu;
+  }
+  return r;
+}
+
+// calls f(data gradient's tile, weight gradient's tile) with the pair of tiles
+template <class F>
+auto with_tiles(int td, int tw, F f) {
+  if (td == 0) return tw == 0 ? f(TileS{}, TileS{}) : tw == 1 ? f(TileS{}, TileM{}) : f(TileS{}, TileL{});
+  return tw == 0 ? f(TileM{}, TileS{}) : tw == 1 ? f(TileM{}, TileM{}) : f(TileM{}, TileL{});
+}
+
+struct BackwardPlan {
+  int td, tw;         // tiles
+  long long nd, nw;   // workgroups, nd 0: not together
+};
+BackwardPlan plan_backward(int m, int o, int f) {
+  BackwardPlan p{pick_tile<false, false>(m, f), pick_tile<true, false>(o, f), 0, 0};
+  if (p.td > 1) return p;    // a data gradient that fills the chip on its own
+  with_tiles(p.td, p.tw, [&](auto d, auto w) {
+    using TD = decltype(d);
+    using TW = decltype(w);
+    const long long nd = tiles_of<TD>(m, f), nw = tiles_of<TW>(o, f);
+    const int fit = o % 16 == 0 && f % 16 == 0 ? backward_resident<TD, TW, true>() : backward_resident<TD, TW, false>();
+    if (nd > kMaxSlots || nw > kMaxSlots || nd + nw > fit) return 0;
+    p.nd = nd;
+    p.nw = nw;
+    return 0;
+  });
+  return p;
+}
+
 }  // namespace
+
+bool gemm_any_backward_blocks(int m, int o, int f, int* nd, int* nw) {
+  if (!gemm_any_shape(m, f, o) || !gemm_any_shape(o, f, m)) return false;
+  const BackwardPlan p = plan_backward(m, o, f);
+  *nd = static_cast<int>(p.nd);
+  *nw = static_cast<int>(p.nw);
+  return p.nd != 0;
+}
+
+int launch_gemm_any_backward(const AnyArgs& d, const AnyArgs& w, hipStream_t stream) {
+  const BackwardPlan p = plan_backward(d.m, d.k, d.n);
+  if (p.nd == 0) return fail(NITI_ERR_UNSUPPORTED, "gemm_any: the workgroups of both gradients do not fit on the device at once");
+  const bool aligned = aligned_rows<false, false>(d) && aligned_rows<true, false>(w);
+  const int nd = static_cast<int>(p.nd);
+  if (!aligned && d.k % 16 == 0 && d.n % 16 == 0) {   // planned with the rows' extents alone: pointers off 16 bytes
+    const long long fit = with_tiles(p.td, p.tw, [](auto dt, auto wt) { return static_cast<long long>(backward_resident<decltype(dt), decltype(wt), false>()); });
+    if (p.nd + p.nw > fit) return fail(NITI_ERR_UNSUPPORTED, "gemm_any: the workgroups of both gradients do not fit on the device at once");
+  }
+  return with_tiles(p.td, p.tw, [&](auto dt, auto wt) {
+    using TD = decltype(dt);
+    using TW = decltype(wt);
+    const dim3 grid(static_cast<unsigned>(p.nd + p.nw));
+    constexpr size_t lds = backward_lds<TD, TW>();
+    if (aligned) hipLaunchKernelGGL((gemm_backward_kernel<TD, TW, true>), grid, dim3(512), lds, stream, d, w, nd);
+    else hipLaunchKernelGGL((gemm_backward_kernel<TD, TW, false>), grid, dim3(512), lds, stream, d, w, nd);
+    return check_launch("gemm_backward");
+  });
+}
 
 bool gemm_any_large(int m, int n) { return tiles_of<TileL>(m, n) >= 160; }
 

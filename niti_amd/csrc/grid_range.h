@@ -41,36 +41,63 @@ __device__ inline void write_scalars(const Args& a, uint32_t gmax, int shift) {
   if (a.exp_out != nullptr) *a.exp_out = sh + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
 }
 
-// Called by wavefront 0 of every workgroup with the workgroup's largest magnitude: the largest over the grid.
-template <class Args>
-__device__ inline uint32_t exchange_range(const Args& a, uint32_t bmax) {
-  const int lane = threadIdx.x & 63;
-  const int nb = gridDim.x * gridDim.y;
-  const int b = blockIdx.y * gridDim.x + blockIdx.x;
-  uint32_t* const slots = a.sync + kSlot0;
-  if (lane == 0) __hip_atomic_store(slot_word(slots, b), bmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
-  return g != 0u ? g - 1u : 0u;
-}
-
-// the workgroup's shift from every wavefront's largest magnitude: wmax[] holds one word per wavefront, gshare the result
+// The workgroup's shift from every wavefront's largest magnitude: wmax[] holds one word per wavefront, gshare the result.
+// `block` of `blocks` workgroups take part.
 template <int NWAVES, class Args>
-__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare) {
+__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare, int block, int blocks) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   lmax = wave_max_u32(lmax);
   if (lane == 0) wmax[wave] = lmax;
   __syncthreads();
   if (wave == 0) {
-    uint32_t b = lane < NWAVES ? wmax[lane] : 0u;
-    b = wave_max_u32(b);
-    const uint32_t g = exchange_range(a, b);
-    if (lane == 0) *gshare = g;
+    const uint32_t b = wave_max_u32(lane < NWAVES ? wmax[lane] : 0u);
+    if (lane == 0) __hip_atomic_store(slot_word(a.sync + kSlot0, block), b + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &a.sync[1], a.sticky);
+    if (lane == 0) *gshare = g != 0u ? g - 1u : 0u;
   }
   __syncthreads();
   const uint32_t gmax = *gshare;
   const int shift = bitwidth_of(gmax, a.bw_mode) - a.target_bits;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) write_scalars(a, gmax, shift);
+  if (block == 0 && threadIdx.x == 0) write_scalars(a, gmax, shift);
+  return shift;
+}
+template <int NWAVES, class Args>
+__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare) {
+  return grid_shift<NWAVES>(a, lmax, wmax, gshare, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+}
+
+// A weight update next to the data gradient `first` that reads the old weights, in one launch: the update's workgroups wait for
+// both ranges - a workgroup of the data gradient fills its slot when it has read its weights - and the gradient's exponent
+// builds on the error's that comes out of this launch.  share: two words.
+template <int NWAVES, class Args>
+__device__ inline int grid_shift_behind(const Args& a, const Args& first, int first_blocks, uint32_t lmax, uint32_t* wmax, uint32_t* share, int block,
+                                        int blocks) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  lmax = wave_max_u32(lmax);
+  if (lane == 0) wmax[wave] = lmax;
+  __syncthreads();
+  if (wave == 0) {
+    const uint32_t b = wave_max_u32(lane < NWAVES ? wmax[lane] : 0u);
+    if (lane == 0) __hip_atomic_store(slot_word(a.sync + kSlot0, block), b + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t f = wait_slots(first.sync + kSlot0, first_blocks, a.spin_limit, &a.sync[1], a.sticky);
+    const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &a.sync[1], a.sticky);
+    if (lane == 0) {
+      share[0] = g != 0u ? g - 1u : 0u;
+      share[1] = f != 0u ? f - 1u : 0u;
+    }
+  }
+  __syncthreads();
+  const uint32_t gmax = share[0];
+  const int shift = bitwidth_of(gmax, a.bw_mode) - a.target_bits;
+  if (block == 0 && threadIdx.x == 0) {
+    const int sh = max(shift, 0), before = max(bitwidth_of(share[1], first.bw_mode) - first.target_bits, 0);
+    a.sync[0] = gmax;
+    if (a.shift_out != nullptr) *a.shift_out = sh;
+    if (a.exp_out != nullptr)
+      *a.exp_out = sh + before + (first.exp_a != nullptr ? *first.exp_a : 0) + (first.exp_b != nullptr ? *first.exp_b : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
+  }
   return shift;
 }
 

@@ -64,77 +64,98 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// linear_dgrad(fuse, err, w, bits, method, div, bw, exp_a, exp_b, rand) -> (error, exponent): err_calc(err @ w)
-PyObject* dgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return guarded([&]() -> PyObject* {
-    Args a(args, n, 10, "linear_dgrad");
-    const bool fuse = a.flag();
-    const at::Tensor& err = a.tensor();
-    const at::Tensor& w = a.tensor();
-    const int bits = a.i(), method = a.i(), div = a.i(), bw = a.i();
-    Opt ea = a.opt(), eb = a.opt(), rand = a.opt();
-    const Shape s = shape_of(err, w, 0, "linear_dgrad");
-    check_rand(rand, static_cast<int64_t>(s.M) * s.F, "linear_dgrad");
-    at::Tensor y, e = scalar32(err);
-    size_t words = 0;
-    void* st = stream_of(err);
-    const Path p = path_of(kDgrad, fuse, s, method, rand, &words);
-    if (p != kSeparate) {
-      y = empty8({s.M, s.F}, err);
-      uint32_t* sync = arena_take(static_cast<long>(words), err, nullptr);
-      const int rc = p == kFew ? niti_fc_i8_dgrad_requant(ptr<int8_t>(err), ptr<int8_t>(w), ptr<int8_t>(y), s.M, s.O, s.F, bits, method, div, bw, sync,
-                                                          words, nullptr, ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st)
-                               : niti_linear_i8_dgrad_requant(ptr<int8_t>(err), ptr<int8_t>(w), ptr<int8_t>(y), s.M, s.O, s.F, bits, method, div, bw,
-                                                              ptr<int32_t>(rand), sync, words, nullptr, ptr<int32_t>(ea), ptr<int32_t>(eb),
-                                                              ptr<int32_t>(e), st);
-      if (check_fits(rc, "niti_linear_i8_dgrad_requant")) return tuple_of({y, e});
-    }
-    uint32_t* am = arena_take(1, err, nullptr);
-    at::Tensor acc = gemm(err, w, false, false, am);
-    y = empty8({s.M, s.F}, err);
-    check(niti_requant_i32_i8(ptr<int32_t>(acc), ptr<int8_t>(y), acc.numel(), am, bits, method, div, bw, ptr<int32_t>(rand), 0u, nullptr,
-                              ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st),
-          "niti_requant_i32_i8");
-    return tuple_of({y, e});
-  });
+struct Rounding {
+  int bits, method, div, bw;
+  Opt rand;
+};
+
+// err_calc(err @ w) -> y, its exponent in e
+at::Tensor data_gradient(bool fuse, const at::Tensor& err, const at::Tensor& w, const Shape& s, const Rounding& r, Opt ea, Opt eb, const at::Tensor& e) {
+  at::Tensor y = empty8({s.M, s.F}, err);
+  size_t words = 0;
+  void* st = stream_of(err);
+  const Path p = path_of(kDgrad, fuse, s, r.method, r.rand, &words);
+  if (p != kSeparate) {
+    uint32_t* sync = arena_take(static_cast<long>(words), err, nullptr);
+    const int rc = p == kFew ? niti_fc_i8_dgrad_requant(ptr<int8_t>(err), ptr<int8_t>(w), ptr<int8_t>(y), s.M, s.O, s.F, r.bits, r.method, r.div, r.bw, sync,
+                                                        words, nullptr, ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st)
+                             : niti_linear_i8_dgrad_requant(ptr<int8_t>(err), ptr<int8_t>(w), ptr<int8_t>(y), s.M, s.O, s.F, r.bits, r.method, r.div, r.bw,
+                                                            ptr<int32_t>(r.rand), sync, words, nullptr, ptr<int32_t>(ea), ptr<int32_t>(eb),
+                                                            ptr<int32_t>(e), st);
+    if (check_fits(rc, "niti_linear_i8_dgrad_requant")) return y;
+  }
+  uint32_t* am = arena_take(1, err, nullptr);
+  at::Tensor acc = gemm(err, w, false, false, am);
+  check(niti_requant_i32_i8(ptr<int32_t>(acc), ptr<int8_t>(y), acc.numel(), am, r.bits, r.method, r.div, r.bw, ptr<int32_t>(r.rand), 0u, nullptr,
+                            ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st),
+        "niti_requant_i32_i8");
+  return y;
 }
 
-// linear_wgrad_update(fuse, err, act, w, mu, method, div, bw, want_grad, keep_acc, exp_a, exp_b, rand)
-//   -> (g8, int32 gradient, shift, exponent): grad_calc(err^T @ act), w updated in place
-PyObject* wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
+// grad_calc(err^T @ act), w updated in place; returns the int32 gradient where there was one
+at::Tensor weight_gradient(bool fuse, const at::Tensor& err, const at::Tensor& act, const at::Tensor& w, const Shape& s, const Rounding& r, int8_t* g8, Opt ea,
+                           Opt eb, const at::Tensor& shift, const at::Tensor& e) {
+  size_t words = 0;
+  void* st = stream_of(err);
+  const Path p = path_of(kWgrad, fuse, s, r.method, r.rand, &words);
+  if (p != kSeparate) {
+    uint32_t* sync = arena_take(static_cast<long>(words), err, nullptr);
+    const int rc = p == kFew ? niti_fc_i8_wgrad_update(ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), s.M, s.O, s.F, r.bits, r.method, r.div, r.bw, sync,
+                                                       words, g8, ptr<int32_t>(shift), ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st)
+                             : niti_linear_i8_wgrad_update(ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), s.M, s.O, s.F, r.bits, r.method, r.div, r.bw,
+                                                           ptr<int32_t>(r.rand), sync, words, g8, ptr<int32_t>(shift), ptr<int32_t>(ea),
+                                                           ptr<int32_t>(eb), ptr<int32_t>(e), st);
+    if (check_fits(rc, "niti_linear_i8_wgrad_update")) return at::Tensor();
+  }
+  uint32_t* am = arena_take(1, err, nullptr);
+  at::Tensor acc = gemm(err, act, true, false, am);   // err^T @ act
+  check(niti_grad_update_i8(ptr<int32_t>(acc), ptr<int8_t>(w), acc.numel(), am, r.bits, r.method, r.div, r.bw, ptr<int32_t>(r.rand), g8, ptr<int32_t>(shift),
+                            ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st),
+        "niti_grad_update_i8");
+  return acc;
+}
+
+// linear_backward(fuse, err, act, w, error bits, error method, gradient bits, gradient method, div, bw, want_grad, keep_acc, exp_err,
+//                 exp_w, exp_act, error rand, gradient rand) -> (error, error exponent, g8, int32 gradient, shift, exponent)
+// TiLinear.backward: both gradients in one launch where they fit on the device together, one after the other otherwise.
+PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    Args a(args, n, 13, "linear_wgrad_update");
+    Args a(args, n, 17, "linear_backward");
     const bool fuse = a.flag();
     const at::Tensor& err = a.tensor();
     const at::Tensor& act = a.tensor();
     const at::Tensor& w = a.tensor();
-    const int mu = a.i(), method = a.i(), div = a.i(), bw = a.i();
+    Rounding re{}, rg{};
+    re.bits = a.i();
+    re.method = a.i();
+    rg.bits = a.i();
+    rg.method = a.i();
+    re.div = rg.div = a.i();
+    re.bw = rg.bw = a.i();
     const bool want_grad = a.flag(), keep = a.flag();
-    Opt ea = a.opt(), eb = a.opt(), rand = a.opt();
-    const Shape s = shape_of(err, w, 0, "linear_wgrad_update");
-    if (act.dim() != 2 || act.size(0) != s.M || act.size(1) != s.F || act.scalar_type() != at::kChar) refuse("linear_wgrad_update: int8 act [M,F] expected");
-    check_rand(rand, static_cast<int64_t>(s.O) * s.F, "linear_wgrad_update");
-    at::Tensor g8, acc, shift = scalar32(w), e = scalar32(w);
+    Opt exp_err = a.opt(), exp_w = a.opt(), exp_act = a.opt();
+    re.rand = a.opt();
+    rg.rand = a.opt();
+    const Shape s = shape_of(err, w, 0, "linear_backward");
+    if (act.dim() != 2 || act.size(0) != s.M || act.size(1) != s.F || act.scalar_type() != at::kChar) refuse("linear_backward: int8 act [M,F] expected");
+    check_rand(re.rand, static_cast<int64_t>(s.M) * s.F, "linear_backward");
+    check_rand(rg.rand, static_cast<int64_t>(s.O) * s.F, "linear_backward");
+    at::Tensor g8, acc, y, ee = scalar32(err), shift = scalar32(w), ge = scalar32(w);
     if (want_grad) g8 = empty8({s.O, s.F}, w);
     int8_t* gp = want_grad ? ptr<int8_t>(g8) : nullptr;
-    size_t words = 0;
-    void* st = stream_of(err);
-    const Path p = path_of(kWgrad, fuse && !keep, s, method, rand, &words);
-    if (p != kSeparate) {
+    const size_t words = fuse && !keep ? niti_linear_i8_backward_sync_words(s.M, s.O, s.F) : 0;
+    if (words > 0) {
+      y = empty8({s.M, s.F}, err);
       uint32_t* sync = arena_take(static_cast<long>(words), err, nullptr);
-      const int rc = p == kFew ? niti_fc_i8_wgrad_update(ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), s.M, s.O, s.F, mu, method, div, bw, sync,
-                                                         words, gp, ptr<int32_t>(shift), ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st)
-                               : niti_linear_i8_wgrad_update(ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), s.M, s.O, s.F, mu, method, div, bw,
-                                                             ptr<int32_t>(rand), sync, words, gp, ptr<int32_t>(shift), ptr<int32_t>(ea),
-                                                             ptr<int32_t>(eb), ptr<int32_t>(e), st);
-      if (check_fits(rc, "niti_linear_i8_wgrad_update")) return tuple_of({g8, acc, shift, e});
+      const int rc = niti_linear_i8_backward(ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), ptr<int8_t>(y), s.M, s.O, s.F, re.bits, re.method, rg.bits,
+                                             rg.method, re.div, re.bw, ptr<int32_t>(re.rand), ptr<int32_t>(rg.rand), sync, words, gp, nullptr,
+                                             ptr<int32_t>(shift), ptr<int32_t>(exp_err), ptr<int32_t>(exp_w), ptr<int32_t>(exp_act), ptr<int32_t>(ee),
+                                             ptr<int32_t>(ge), stream_of(err));
+      if (check_fits(rc, "niti_linear_i8_backward")) return tuple_of({y, ee, g8, acc, shift, ge});
     }
-    uint32_t* am = arena_take(1, err, nullptr);
-    acc = gemm(err, act, true, false, am);   // err^T @ act
-    check(niti_grad_update_i8(ptr<int32_t>(acc), ptr<int8_t>(w), acc.numel(), am, mu, method, div, bw, ptr<int32_t>(rand), gp, ptr<int32_t>(shift),
-                              ptr<int32_t>(ea), ptr<int32_t>(eb), ptr<int32_t>(e), st),
-          "niti_grad_update_i8");
-    return tuple_of({g8, acc, shift, e});
+    y = data_gradient(fuse, err, w, s, re, exp_err, exp_w, ee);
+    acc = weight_gradient(fuse && !keep, err, act, w, s, rg, gp, &ee, exp_act, shift, ge);
+    return tuple_of({y, ee, g8, acc, shift, ge});
   });
 }
 
@@ -220,8 +241,7 @@ PyObject* head_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }  // namespace
 
 PyMethodDef kLinearMethods[] = {{"linear_forward", FAST(forward)},
-                                {"linear_dgrad", FAST(dgrad)},
-                                {"linear_wgrad_update", FAST(wgrad_update)},
+                                {"linear_backward", FAST(backward)},
                                 {"head_forward", FAST(head_forward)},
                                 {"head_backward", FAST(head_backward)},
                                 {nullptr, nullptr, 0, nullptr}};

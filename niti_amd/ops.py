@@ -476,6 +476,16 @@ def linear_wgrad_update(err, act, w, mu=5, method="psto", div_mode="floor", bw_m
     return g8, shift_out, sync
 
 
+def linear_backward(err, act, w, err_bits=7, err_method="round", mu=5, grad_method="psto", div_mode="floor", bw_mode="int", err_rand=None,
+                    grad_rand=None, want_grad=False, exp_err=None, exp_w=None, exp_act=None):
+    """TiLinear.backward (ti_torch.py:249-266): err [M,O], act [M,F], w [O,F] int8, w updated in place behind the data gradient that
+    reads it; one launch where both gradients' workgroups fit on the device together.  Returns (error [M,F] int8, its exponent,
+    int8 gradient or None, int32 gradient or None, gradient shift, gradient exponent)."""
+    _chk_dev(err, act, w, err_rand, grad_rand, exp_err, exp_w, exp_act)
+    return L.host().linear_backward(True, err, act, w, err_bits, L.ROUND[err_method], mu, L.ROUND[grad_method], L.DIV[div_mode], L.BW[bw_mode],
+                                    want_grad, False, exp_err, exp_w, exp_act, err_rand, grad_rand)
+
+
 def pad_last_dim(t, multiple=16):
     """``t`` with zeros appended along its last dimension up to a multiple of ``multiple`` (``t`` itself when it
     already is one): the channel padding of conv2d_int8 (ti_torch.py:182-187) as one launch."""

@@ -571,12 +571,10 @@ class TiLinear(UpdateWeight):
         if mask is not None:     # the separate passes want the masked activations and their exponent
             act, d["act_in_exp"] = ops.mask_features(act, mask, _exp_tensor(d["act_in_exp"], dev), 1)
         rand = _sto_rand(e_method, rand, tuple(act.shape), dev)
-        err_out, d["err_exp"] = host.linear_dgrad(FUSE_CONV_REQUANT, err_in, weight, BITWIDTH, e_method, div, bw, d["err_exp_in"],
-                                                  self._wexp(), rand)
         grad_rand = _sto_rand(g_method, grad_rand, tuple(weight.shape), dev)
-        d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"] = host.linear_wgrad_update(
-            FUSE_CONV_REQUANT, err_in, act, weight, GRAD_BITWIDTH, g_method, div, bw, self.keep_grad, KEEP_INT32_GRAD, d["err_exp"],
-            _exp_tensor(d["act_in_exp"], dev), grad_rand)
+        err_out, d["err_exp"], d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"] = host.linear_backward(
+            FUSE_CONV_REQUANT, err_in, act, weight, BITWIDTH, e_method, GRAD_BITWIDTH, g_method, div, bw, self.keep_grad, KEEP_INT32_GRAD,
+            d["err_exp_in"], self._wexp(), _exp_tensor(d["act_in_exp"], dev), rand, grad_rand)
         return err_out, d["err_exp"]
 
 

@@ -1334,3 +1334,34 @@ def test_conv_wgrad_update_small_batches(dev, case, monkeypatch):
         assert torch.equal(wd.cpu(), po.weight_update(w, g8_ref))
         assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q))
     assert torch.equal(ops.conv2d_wgrad(x.to(dev), e.to(dev), 3, 3).cpu(), acc)
+
+
+@pytest.mark.parametrize("tile", ["0", "1", ""])
+@pytest.mark.parametrize("case", ANY_CASES)
+def test_linear_backward_together(dev, case, tile, monkeypatch):
+    """Data gradient and weight update as one launch: the error comes from the old weights, the exponents add up."""
+    from niti_amd import _lib, ops
+    from oracle import niti_oracle as po
+    if tile:
+        monkeypatch.setenv("NITI_ANY_TILE", tile)
+    M, O, F = case
+    _say("linear_backward_together", case, tile)
+    if tile != "0":
+        assert _lib.lib().niti_linear_i8_backward_sync_words(M, O, F) > 0
+    g = torch.Generator().manual_seed(9100 + M + O + F)
+    act, w, err = ri8(g, M, F), ri8(g, O, F), ri8(g, M, O, lo=-40, hi=40)
+    dacc, wacc = po.int8mm(err, w), po.int8mm(err.t().contiguous(), act)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    for e_method, g_method in (("round", "psto"), ("sto", "sto"), ("psto", "round")):
+        er, gr = (torch.randint(0, 1 << 20, t.shape, generator=g, dtype=torch.int32) for t in (dacc, wacc))
+        low = lambda u, acc, bits: u % (1 << max(po.RangeEstimate(acc, "int") - bits, 0))
+        dref, dsh = po.err_calc(dacc, e_method, rand=low(er, dacc, 7))
+        gref, gsh = po.grad_calc(wacc, 5, g_method, rand=low(gr, wacc, 5))
+        wd = w.to(dev)
+        dx, de, g8, _, sh, ge = ops.linear_backward(err.to(dev), act.to(dev), wd, err_method=e_method, grad_method=g_method,
+                                                    err_rand=er.to(dev) if e_method == "sto" else None, grad_rand=gr.to(dev) if g_method == "sto" else None,
+                                                    want_grad=True, exp_err=scalar(-4), exp_w=scalar(-3), exp_act=scalar(2))
+        assert torch.equal(dx.cpu(), dref) and int(de.cpu()) == dsh - 7, (e_method, g_method)
+        assert torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh and int(ge.cpu()) == gsh + dsh - 7 + 2
+        assert torch.equal(wd.cpu(), po.weight_update(w, gref))
+    assert not ops.sync_arena.timed_out(dev)
