@@ -451,6 +451,28 @@ int niti_linear_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int
                             int32_t* err_exp_out, int32_t* grad_exp_out, void* stream);
 
 /*
+ * TiConv2d.backward (ti_torch.py:404-437, stride 1) as one launch - two where the reduction over the pixels is cut: dx8 =
+ * err_calc(conv_dgrad(err, w)) with the weights as they are on entry, then w = clip(w - grad_calc(conv_wgrad(act, err))).
+ * err [N][P][Q][K], act [N][H][W][C], w [K][R][S][C], all 16-byte aligned, C and K multiples of 16.  relu_mask (may be NULL):
+ * laid out like dx8, which is zero where the mask is not positive.  pool_in (may be NULL, needs relu_mask = the pooled map): dx8
+ * is the [N][2H][2W][C] gradient of the 2x2 / stride-2 max-pool's input pool_in (ties as in niti_maxpool_i8_bwd).
+ * err_method may be NITI_ROUND_STOCHASTIC with err_rand, one int32 per element of [N][H][W][C] (not with pool_in); grad_method
+ * NITI_ROUND_NEAREST or NITI_ROUND_PSEUDO_STOCHASTIC.  w_prepared (may be NULL): the forward pass's kernel-ready copy of w, kept in
+ * step.  err_exp_out = error shift + exp_err + exp_w, grad_exp_out = gradient shift + err_exp_out + exp_act.
+ * NITI_CONV_SHIFT_HINT: *grad_shift_out holds a predicted shift on entry.
+ * niti_conv2d_i8_backward_sync_words returns 0 where the two do not fit on the device at once or are faster one by one
+ * (niti_conv2d_i8_dgrad_requant, niti_conv2d_i8_wgrad_update).
+ */
+size_t niti_conv2d_i8_backward_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad);
+size_t niti_conv2d_i8_backward_workspace(int N, int H, int W, int C, int K, int R, int S, int pad);
+int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+                            int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
+                            const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
+                            size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
+                            const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
+                            int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Integer cross-entropy gradient, TiLoss.forward (ti_loss.py:5-36), as one launch: out_val [n][classes] int8 logits
  * with exponent *out_exp (device scalar), target [n] int64 class indices, rand [n][classes] int32 random integers
  * (the low four bits stand in for the reference's torch.randint(0, 16)) -> grad [n][classes] int8 with exponent 0.

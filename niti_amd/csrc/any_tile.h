@@ -27,7 +27,7 @@ struct Tile {
   static_assert(WM * WN * WK == 8 && BK % (32 * WK) == 0, "eight wavefronts");
 };
 using TileS = Tile<1, 1, 8, 1, 1, 512, 2, 2>;    //  32 x  32
-using TileM = Tile<2, 2, 2, 1, 1, 256, 2, 2>;    //  64 x  64
+using TileM = Tile<2, 2, 2, 1, 1, 256, 2, 4>;    //  64 x  64
 using TileH = Tile<4, 2, 1, 1, 1, 128, 2, 4>;    // 128 x  64
 using TileL = Tile<2, 4, 1, 2, 1, 128, 2, 2>;    // 128 x 128
 
@@ -73,7 +73,7 @@ constexpr int kOutside = 0x70000000;   // byte offset behind any matrix these ke
 template <class G_, bool kAligned, bool kCut = true>   // G::kFast: a chunk advances along the row, otherwise along the rows
 struct DenseOperand {
   using G = G_;
-  static constexpr bool kFast = G::kFast;
+  static constexpr bool kFast = G::kFast, kPairs = !kAligned;
   struct Raw {
     v4i lo, hi;   // hi: unused when the rows are aligned
   };
@@ -183,7 +183,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
   // Fragments are read LOOK steps ahead of their products; `meanwhile` (the loads of a later chunk and their addresses) runs
   // behind the first reads.  One step at a time, a chunk took an LDS round trip per step: 64 x 64 tiles walked a long
   // reduction in 0.75 us per 256 steps.
-  constexpr int LOOK = T::LOOK;
+  constexpr int LOOK = OpA::kPairs && T::LOOK > 2 ? 2 : T::LOOK;   // registers: granule pairs take twice as many
   constexpr int READS = (TA ? 2 : 1) * T::TM + (TB ? 1 : 2) * T::TN;   // of one step
   v2i alo[LOOK][T::TM], ahi[LOOK][T::TM], blo[LOOK][T::TN], bhi[LOOK][T::TN];
   v4i av[LOOK][T::TM], bv[LOOK][T::TN];
@@ -312,6 +312,12 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
   // loads of an array behind stores to it: one trip to memory per group otherwise)
   v4i rnd[G];
   uint32_t wold[G];
+  constexpr bool kUnpool = MODE == kRequant && G <= 4;   // the launches that use it have these tiles
+  uint32_t window[kUnpool ? G : 1][4];
+  auto window_at = [&](int row, int col) {
+    const int image = g.by_map.of(row), rest = row - image * (g.map_h * g.map_w), h = g.by_map_w.of(rest), w = rest - h * g.map_w;
+    return (static_cast<long long>(image * 2 * g.map_h + 2 * h) * (2 * g.map_w) + 2 * w) * g.n + col;
+  };
   if (MODE != kInt32) {
 #pragma unroll
     for (int i = 0; i < G; ++i) {
@@ -324,6 +330,13 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
       if (g.method == NITI_ROUND_STOCHASTIC) __builtin_memcpy(&rnd[i], g.rand + at, 16);
       if (MODE == kUpdate) __builtin_memcpy(&wold[i], g.w + at, 4);
       if (MODE == kRequant && g.mask != nullptr) __builtin_memcpy(&wold[i], g.mask + at, 4);
+      if constexpr (kUnpool) {
+        if (g.unpool != nullptr) {
+          const int8_t* const from = g.pool_x + window_at(row, col);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) __builtin_memcpy(&window[i][q], from + ((q >> 1) * 2 * g.map_w + (q & 1)) * static_cast<long long>(g.n), 4);
+        }
+      }
     }
   }
 #pragma unroll
@@ -356,6 +369,21 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
         for (int e = 0; e < here; ++e) mk |= static_cast<uint32_t>(static_cast<uint8_t>(g.mask[at + e])) << (8 * e);
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[e] = static_cast<int8_t>((mk >> (8 * e)) & 0xFFu) > 0 ? r[e] : 0;
+    }
+    if constexpr (kUnpool) {
+      if (g.unpool != nullptr) {   // channels are a multiple of 16 here
+        const uint32_t v = pack4_i8(r[0], r[1], r[2], r[3]);
+        int8_t* const to = g.unpool + window_at(row, col);
+        uint32_t taken = 0;        // bytes that an earlier position of the window (scan order) already received
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t eq = equal_bytes(window[i][q], wold[i]);
+          const uint32_t put = v & (g.ties_all != 0 ? eq : eq & ~taken);
+          taken |= eq;
+          __builtin_memcpy(to + ((q >> 1) * 2 * g.map_w + (q & 1)) * static_cast<long long>(g.n), &put, 4);
+        }
+        continue;
+      }
     }
     if (here == 4) {
       const uint32_t packed = pack4_i8(r[0], r[1], r[2], r[3]);

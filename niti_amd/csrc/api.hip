@@ -642,6 +642,80 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
                                 dw_out, w_prepared, workspace, static_cast<hipStream_t>(stream));
 }
 
+// Whether both gradients in one launch are the faster way.  Outside the 3x3 kernels' maps they are wherever they fit; there the
+// data gradient's own kernel (its stages of 32 channels, longer on the wider maps) and the weight gradient's are estimated.
+static bool backward_together(const ConvShape& s) {
+  const char* e = getenv("NITI_BACKWARD_TOGETHER");   // 0 / 1 pins (tests)
+  if (e != nullptr) return e[0] != '0';
+  const double us = conv_backward_us(s);
+  if (us == 0.0) return false;
+  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad)) {
+    const double stage = s.H >= 32 ? 1.25 : s.H == 16 ? 1.05 : 0.62;
+    return us < 0.8 * (3.5 + stage * ((s.K + 31) / 32) + wgrad3x3_us(s.N, s.H, s.C, s.K));
+  }
+  const double d = conv_any_dgrad_us(s), w = conv_any_wgrad_us(s);
+  return d == 0.0 || us < d + w;
+}
+
+extern "C" size_t niti_conv2d_i8_backward_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad) {
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || pad < 0) return 0;
+  const ConvShape s{N, H, W, C, K, R, S, 1, pad};
+  return backward_together(s) ? conv_backward_words(s) : 0;
+}
+
+extern "C" size_t niti_conv2d_i8_backward_workspace(int N, int H, int W, int C, int K, int R, int S, int pad) {
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || pad < 0) return 0;
+  return round256(conv_backward_workspace({N, H, W, C, K, R, S, 1, pad}));
+}
+
+extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+                                       int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
+                                       const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
+                                       size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
+                                       const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
+                                       int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  const char* who = "conv_backward";
+  int st = check_conv_dims(who, N, H, W, C, K, R, S, 1, pad);
+  if (st == NITI_OK) st = check_flags(who, flags, NITI_EPI_F32_ROUNDTRIP | NITI_CONV_SHIFT_HINT);
+  if (st != NITI_OK) return st;
+  if (err == nullptr || act == nullptr || w == nullptr || dx8 == nullptr || sync == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: null pointer", who);
+  for (const void* p : {static_cast<const void*>(err), static_cast<const void*>(act), static_cast<const void*>(w), static_cast<const void*>(dx8),
+                        static_cast<const void*>(err_rand), static_cast<const void*>(relu_mask), static_cast<const void*>(pool_in),
+                        static_cast<const void*>(g8_out), static_cast<const void*>(w_prepared)})
+    if (!aligned16(p)) return fail(NITI_ERR_INVALID_ARG, "%s: pointers must be 16-byte aligned", who);
+  if (err_bits < 1 || err_bits > 7 || grad_bits < 1 || grad_bits > 7)
+    return fail(NITI_ERR_INVALID_ARG, "%s: target bits %d, %d outside 1..7", who, err_bits, grad_bits);
+  if (err_method != NITI_ROUND_NEAREST && err_method != NITI_ROUND_PSEUDO_STOCHASTIC && !(err_method == NITI_ROUND_STOCHASTIC && err_rand != nullptr && pool_in == nullptr))
+    return fail(NITI_ERR_INVALID_ARG, "%s: error rounding method %d", who, err_method);
+  if (grad_method != NITI_ROUND_NEAREST && grad_method != NITI_ROUND_PSEUDO_STOCHASTIC)
+    return fail(NITI_ERR_UNSUPPORTED, "%s: gradient rounding method %d needs random input", who, grad_method);
+  if (div_mode != NITI_DIV_FLOOR && div_mode != NITI_DIV_TRUNC) return fail(NITI_ERR_INVALID_ARG, "%s: div_mode=%d", who, div_mode);
+  if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
+  if (pool_in != nullptr && (relu_mask == nullptr || (ties != NITI_TIES_FIRST && ties != NITI_TIES_ALL)))
+    return fail(NITI_ERR_INVALID_ARG, "%s: pool_in needs the pooled map as relu_mask; ties=%d", who, ties);
+  const ConvShape s{N, H, W, C, K, R, S, 1, pad};
+  if (w_prepared != nullptr && filter_copy_kind(N, H, W, C, K, R, S, 1, pad, 0) != 2)
+    return fail(NITI_ERR_UNSUPPORTED, "%s: w_prepared needs a shape whose forward pass uses a kernel-ready filter copy", who);
+  const size_t need = conv_backward_words(s), bytes = conv_backward_workspace(s);
+  if (need == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: the workgroups of both gradients do not fit on the device at once", who);
+  if (sync_words < need) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, need, sync_words);
+  if (bytes > 0 && (workspace == nullptr || workspace_bytes < bytes || !aligned16(workspace)))
+    return fail(NITI_ERR_WORKSPACE, "%s: needs %zu workspace bytes (16-byte aligned), got %zu", who, bytes, workspace_bytes);
+  RequantSpec rq{err_bits, err_method, div_mode == NITI_DIV_TRUNC, bw_mode, 0u, sync_spin_limit(), timeout_word(), err_shift_out, exp_err, exp_w, err_exp_out,
+                 relu_mask, nullptr};
+  rq.rand = err_method == NITI_ROUND_STOCHASTIC ? err_rand : nullptr;
+  if (pool_in != nullptr) {
+    rq.pool_x = pool_in;
+    rq.unpool = dx8;
+    rq.ties_all = ties == NITI_TIES_ALL ? 1 : 0;
+  }
+  RequantSpec grad{grad_bits, grad_method, div_mode == NITI_DIV_TRUNC, bw_mode, (flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u, sync_spin_limit(),
+                   timeout_word(), grad_shift_out, nullptr, exp_act, grad_exp_out, nullptr, nullptr};
+  return launch_conv_backward(s, err, act, w, dx8, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, grad, g8_out, w_prepared, workspace,
+                              static_cast<hipStream_t>(stream));
+}
+
 extern "C" size_t niti_gemm_i8_workspace(int trans_a, int trans_b, int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   if (gemm_kmajor_shape(trans_a, trans_b, m, n, k) && gemm_any_shape(m, n, k)) return gemm_lines_workspace(trans_a, trans_b, m, n, k);   // read as stored; partial sums of a split reduction

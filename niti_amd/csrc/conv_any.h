@@ -18,6 +18,7 @@ bool conv_any_shape(ConvPass pass, const ConvShape& s);   // extents and channel
 int launch_conv_any(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int32_t* y, bool roundtrip, uint32_t* absmax, hipStream_t stream);
 // the same rounded to int8 in the launch: sync words, 0 when no tile's grid is resident at once
 size_t conv_any_requant_words(ConvPass pass, const ConvShape& s);
+double conv_any_dgrad_us(const ConvShape& s);   // estimated time of the data gradient with rounding, 0: does not run
 int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int8_t* y, bool roundtrip, uint32_t* sync,
                             const RequantSpec& rq, hipStream_t stream);
 // weight gradient (stride 1)
@@ -28,5 +29,13 @@ int launch_conv_any_wgrad(const ConvShape& s, const int8_t* act, const int8_t* e
 size_t conv_any_wgrad_update_words(const ConvShape& s);
 int launch_conv_any_wgrad_update(const ConvShape& s, const int8_t* act, const int8_t* err, int8_t* w, int w_channels, bool roundtrip, uint32_t* sync,
                                  const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, void* workspace, hipStream_t stream);
+
+// Data gradient and weight gradient with update as one launch (conv_backward.hip; stride 1).  The gradient's exponent builds on
+// the error's: grad.exp_a is not read.  words 0: not resident together.
+double conv_backward_us(const ConvShape& s);   // estimated time
+size_t conv_backward_words(const ConvShape& s);
+size_t conv_backward_workspace(const ConvShape& s);
+int launch_conv_backward(const ConvShape& s, const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx, bool roundtrip, uint32_t* sync, const RequantSpec& rq,
+                         const RequantSpec& grad, int8_t* g8, int8_t* wprep, void* workspace, hipStream_t stream);
 
 }  // namespace niti

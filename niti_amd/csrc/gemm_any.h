@@ -33,6 +33,12 @@ struct AnyArgs {
   int channels = 0;
   Reciprocal by_channels{};
   const int8_t* mask = nullptr;   // laid out like out8: results are zero where it is not positive (not for the weight update)
+  // with a mask: the result is the gradient of a 2x2 / stride-2 max-pool's output (= mask, [rows][map_h][map_w][n]) and goes to
+  // the position(s) of each window of the pool's input pool_x that hold the maximum, in unpool; out8 is not written
+  const int8_t* pool_x = nullptr;
+  int8_t* unpool = nullptr;
+  int ties_all = 0, map_h = 0, map_w = 0;
+  Reciprocal by_map{}, by_map_w{};
   const int32_t* rand = nullptr;
   uint32_t* sync = nullptr;
   int target_bits = 7, method = 0, trunc = 0, bw_mode = 0;

@@ -350,64 +350,37 @@ PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// layer_dgrad(fuse, err, w, stride, pad, f32, bits, method, div, bw, shift state, exp_a, exp_b, forward copy, mask, pool_in,
-//             ties, rand) -> (error, exponent, unpooled?)
-// TiConv2d.backward's data gradient: err_calc(conv_dgrad(err, w)), zeroed where `mask` (the layer's input) is not positive,
+struct DataGradient {
+  at::Tensor y, e;
+  bool unpooled = false;
+};
+// TiConv2d.backward's data gradient: err_calc(conv_dgrad(err, w)), zeroed where `f.mask` (the layer's input) is not positive,
 // and - `pool_in` given - routed through the 2x2 max-pool in front of the layer, one launch where the kernels cover it.
-PyObject* layer_dgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return guarded([&]() -> PyObject* {
-    Args a(args, n, 18, "conv layer data gradient");
-    const bool fuse = a.flag();
-    const at::Tensor& err = a.tensor();
-    const at::Tensor& w = a.tensor();
-    Fused f;
-    f.dgrad = true;
-    f.stride = a.i();
-    f.pad = a.i();
-    f.f32 = a.flag();
-    f.r = rounding_of(a);
-    f.shift = a.opt();
-    f.hint = f.shift != nullptr;
-    f.exp_a = a.opt();
-    f.exp_b = a.opt();
-    f.prepared = a.opt();
-    f.mask = a.opt();
-    Opt pool_in = a.opt();
-    f.ties = a.i();
-    f.rand = a.opt();
-    const Dims d = gradient_dims(err, w, f.pad, "conv layer");
-    // the forward pass's copy serves the data gradient only where both run the 3x3 kernel
-    f.forward_copy = f.prepared != nullptr;
-    if (f.forward_copy && niti_conv2d_i8_forward_copy_ok(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad) == 0) {
-      f.forward_copy = false;
-      f.prepared = nullptr;
-    }
-    at::Tensor y, shift, e = scalar32(err);
-    f.exp_out = &e;
-    PyObject* unpooled = Py_False;
-    bool done = false;
-    if (fuse && pool_in != nullptr && d.H == d.W && d.H <= 32 && (d.H & (d.H - 1)) == 0) {
-      f.pool_in = pool_in;
-      done = conv_requant(err, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant_unpool");
-      if (done) unpooled = Py_True;
-      f.pool_in = nullptr;
-    }
-    if (fuse && !done) done = conv_requant(err, w, d, f, true, &y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant");
-    if (!done) {
-      uint32_t* am = arena_take(1, err, nullptr);
-      at::Tensor dx = dgrad_i32(err, w, f.stride, f.pad, f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u, am, f.prepared, f.forward_copy);
-      y = requant_i32(dx, am, f.r, f.rand, false, nullptr, f.exp_a, f.exp_b, ptr<int32_t>(e));
-      if (f.mask != nullptr)
-        check(niti_relu_i8_bwd(ptr<int8_t>(*f.mask), ptr<int8_t>(y), ptr<int8_t>(y), y.numel(), stream_of(err)), "niti_relu_i8_bwd");
-    }
-    PyObject* out = PyTuple_New(3);
-    if (out == nullptr) throw python_error();
-    PyTuple_SET_ITEM(out, 0, wrap(y));
-    PyTuple_SET_ITEM(out, 1, wrap(e));
-    Py_INCREF(unpooled);
-    PyTuple_SET_ITEM(out, 2, unpooled);
-    return out;
-  });
+void data_gradient(bool fuse, const at::Tensor& err, const at::Tensor& w, Fused f, Opt pool_in, DataGradient* r) {
+  const Dims d = gradient_dims(err, w, f.pad, "conv layer");
+  // the forward pass's copy serves the data gradient only where both run the 3x3 kernel
+  f.forward_copy = f.prepared != nullptr;
+  if (f.forward_copy && niti_conv2d_i8_forward_copy_ok(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad) == 0) {
+    f.forward_copy = false;
+    f.prepared = nullptr;
+  }
+  at::Tensor shift;
+  f.exp_out = &r->e;
+  bool done = false;
+  if (fuse && pool_in != nullptr && d.H == d.W && d.H <= 32 && (d.H & (d.H - 1)) == 0) {
+    f.pool_in = pool_in;
+    done = conv_requant(err, w, d, f, true, &r->y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant_unpool");
+    r->unpooled = done;
+    f.pool_in = nullptr;
+  }
+  if (fuse && !done) done = conv_requant(err, w, d, f, true, &r->y, &shift, nullptr, "niti_conv2d_i8_dgrad_requant");
+  if (!done) {
+    uint32_t* am = arena_take(1, err, nullptr);
+    at::Tensor dx = dgrad_i32(err, w, f.stride, f.pad, f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u, am, f.prepared, f.forward_copy);
+    r->y = requant_i32(dx, am, f.r, f.rand, false, nullptr, f.exp_a, f.exp_b, ptr<int32_t>(r->e));
+    if (f.mask != nullptr)
+      check(niti_relu_i8_bwd(ptr<int8_t>(*f.mask), ptr<int8_t>(r->y), ptr<int8_t>(r->y), r->y.numel(), stream_of(err)), "niti_relu_i8_bwd");
+  }
 }
 
 struct Update {
@@ -469,10 +442,95 @@ PyObject* wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
+struct WeightGradient {
+  bool want_grad = false, want_dw = false;
+  Rounding r{};
+  unsigned flags = 0;
+  Opt shift = nullptr, exp_a = nullptr, exp_b = nullptr, prepared = nullptr, rand = nullptr;
+};
+// TiConv2d.backward's weight gradient, grad_calc and update of w in place; returns whether one call did it all.  Without a
+// one-call form the int32 gradient (its zero-padded channels dropped) is rounded and applied in a second step and returned.
+bool weight_gradient(bool fuse, const at::Tensor& act, const at::Tensor& err, const at::Tensor& w, int stride, int pad, const WeightGradient& g, Update* u,
+                     const at::Tensor& e) {
+  const bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, g.flags | NITI_CONV_ANY_KERNEL | (g.shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), g.r,
+                                              g.want_grad, g.want_dw, nullptr, g.shift, g.exp_a, g.exp_b, ptr<int32_t>(e), nullptr, g.prepared, true, u, nullptr);
+  if (one) {
+    if (g.want_dw && u->dw.size(3) != w.size(3)) u->dw = u->dw.slice(3, 0, w.size(3)).contiguous();
+    return true;
+  }
+  uint32_t* am = arena_take(1, act, nullptr);
+  u->dw = wgrad_i32(act, err, static_cast<int>(w.size(1)), static_cast<int>(w.size(2)), stride, pad, g.flags, am, nullptr);
+  // zero-padded input channels give zero gradient columns (they cannot raise the range)
+  if (u->dw.size(3) != w.size(3)) u->dw = u->dw.slice(3, 0, w.size(3)).contiguous();
+  if (g.rand != nullptr && (g.rand->scalar_type() != at::kInt || g.rand->numel() != u->dw.numel()))
+    refuse("grad_update: rand must be int32 with one entry per element");
+  if (g.want_grad) u->g8 = empty8(w.sizes(), w);
+  u->shift = scalar32(w);
+  check(niti_grad_update_i8(ptr<int32_t>(u->dw), ptr<int8_t>(w), u->dw.numel(), am, g.r.bits, g.r.method, g.r.div, g.r.bw, ptr<int32_t>(g.rand),
+                            g.want_grad ? ptr<int8_t>(u->g8) : nullptr, ptr<int32_t>(u->shift), ptr<int32_t>(g.exp_a), ptr<int32_t>(g.exp_b), ptr<int32_t>(e),
+                            stream_of(act)),
+        "niti_grad_update_i8");
+  return false;
+}
+
+// both in one call where niti_conv2d_i8_backward covers them
+bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tensor& w, const Fused& f, Opt pool_in, const WeightGradient& g, DataGradient* r,
+                    Update* u, const at::Tensor& e) {
+  if (f.stride != 1 || g.want_dw || g.rand != nullptr || g.r.method == NITI_ROUND_STOCHASTIC || act.size(3) != w.size(3)) return false;
+  if (!is_i8(act) || !is_i8(err) || !is_i8(w)) return false;
+  for (Opt t : {&act, &err, &w, f.mask, f.rand, pool_in, g.prepared})
+    if (t != nullptr && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
+  const Dims d = gradient_dims(err, w, f.pad, "conv layer");
+  if (!has_shape(act, {d.N, d.H, d.W, d.C}) || d.R != d.S) return false;
+  const bool sto = f.r.method == NITI_ROUND_STOCHASTIC;
+  std::vector<int64_t> shape{d.N, d.H, d.W, d.C};
+  if (f.mask != nullptr && (!is_i8(*f.mask) || !has_shape(*f.mask, shape))) return false;
+  if (sto && (f.rand == nullptr || f.rand->scalar_type() != at::kInt || !has_shape(*f.rand, shape))) return false;
+  if (pool_in != nullptr) {
+    shape = {d.N, 2LL * d.H, 2LL * d.W, d.C};
+    if (sto || f.mask == nullptr || !is_i8(*pool_in) || !has_shape(*pool_in, shape)) pool_in = nullptr, shape = {d.N, d.H, d.W, d.C};
+  }
+  const size_t words = niti_conv2d_i8_backward_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
+  if (words == 0) return false;
+  const size_t bytes = niti_conv2d_i8_backward_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
+  at::Tensor ws;
+  if (bytes > 0) ws = scratch(bytes, act);
+  uint32_t* sync = arena_take(static_cast<long>(words), act, nullptr);
+  r->y = empty8(shape, act);
+  if (g.want_grad) u->g8 = empty8(w.sizes(), w);
+  u->shift = g.shift != nullptr ? *g.shift : scalar32(w);
+  const int rc = niti_conv2d_i8_backward(
+      ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), ptr<int8_t>(r->y), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad,
+      g.flags | (g.shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), f.r.bits, f.r.method, sto ? ptr<int32_t>(f.rand) : nullptr, ptr<int8_t>(f.mask),
+      ptr<int8_t>(pool_in), f.ties, g.r.bits, g.r.method, f.r.div, f.r.bw, sync, words, g.want_grad ? ptr<int8_t>(u->g8) : nullptr, ptr<int8_t>(g.prepared),
+      ptr<int32_t>(f.shift), ptr<int32_t>(u->shift), ptr<int32_t>(f.exp_a), ptr<int32_t>(f.exp_b), ptr<int32_t>(g.exp_b), ptr<int32_t>(r->e), ptr<int32_t>(e),
+      bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(act));
+  if (!check_fits(rc, "niti_conv2d_i8_backward")) return false;
+  r->unpooled = pool_in != nullptr;
+  return true;
+}
+
+PyObject* put_all(std::initializer_list<PyObject*> items) {   // takes the references over
+  PyObject* out = PyTuple_New(static_cast<Py_ssize_t>(items.size()));
+  if (out == nullptr) throw python_error();
+  Py_ssize_t k = 0;
+  for (PyObject* o : items) PyTuple_SET_ITEM(out, k++, o);
+  return out;
+}
+PyObject* boolean(bool b) {
+  PyObject* o = b ? Py_True : Py_False;
+  Py_INCREF(o);
+  return o;
+}
+
+void take_weight_gradient(Args& a, WeightGradient* g) {
+  g->want_grad = a.flag();
+  g->want_dw = a.flag();
+  g->shift = a.opt();
+}
+
 // layer_wgrad_update(fuse, act, err, w, stride, pad, f32, mu, method, div, bw, want_grad, want_dw, shift state, exp_a, exp_b,
-//                    prepared, rand) -> (g8, dw, shift, exponent, one call?)
-// TiConv2d.backward's weight gradient, grad_calc and update of w in place; without a one-call form the int32 gradient (its
-// zero-padded channels dropped) is rounded and applied in a second step and returned.
+//                    prepared, rand) -> (g8, dw, shift, exponent, one call?): the first layer's backward pass
 PyObject* layer_wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Args a(args, n, 18, "conv layer weight gradient");
@@ -481,40 +539,67 @@ PyObject* layer_wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const at::Tensor& err = a.tensor();
     const at::Tensor& w = a.tensor();
     const int stride = a.i(), pad = a.i();
-    const unsigned flags = a.flag() ? NITI_EPI_F32_ROUNDTRIP : 0u;
-    const Rounding r = rounding_of(a);
-    const bool want_grad = a.flag(), want_dw = a.flag();
-    Opt shift = a.opt(), exp_a = a.opt(), exp_b = a.opt(), prepared = a.opt(), rand = a.opt();
+    WeightGradient g;
+    g.flags = a.flag() ? NITI_EPI_F32_ROUNDTRIP : 0u;
+    g.r = rounding_of(a);
+    take_weight_gradient(a, &g);
+    g.exp_a = a.opt();
+    g.exp_b = a.opt();
+    g.prepared = a.opt();
+    g.rand = a.opt();
     at::Tensor e = scalar32(act);
     Update u;
-    bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, flags | NITI_CONV_ANY_KERNEL | (shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), r, want_grad, want_dw,
-                                          nullptr, shift, exp_a, exp_b, ptr<int32_t>(e), nullptr, prepared, true, &u, nullptr);
-    if (one) {
-      if (want_dw && u.dw.size(3) != w.size(3)) u.dw = u.dw.slice(3, 0, w.size(3)).contiguous();
-    } else {
-      uint32_t* am = arena_take(1, act, nullptr);
-      u.dw = wgrad_i32(act, err, static_cast<int>(w.size(1)), static_cast<int>(w.size(2)), stride, pad, flags, am, nullptr);
-      // zero-padded input channels give zero gradient columns (they cannot raise the range)
-      if (u.dw.size(3) != w.size(3)) u.dw = u.dw.slice(3, 0, w.size(3)).contiguous();
-      if (rand != nullptr && (rand->scalar_type() != at::kInt || rand->numel() != u.dw.numel()))
-        refuse("grad_update: rand must be int32 with one entry per element");
-      if (want_grad) u.g8 = empty8(w.sizes(), w);
-      u.shift = scalar32(w);
-      check(niti_grad_update_i8(ptr<int32_t>(u.dw), ptr<int8_t>(w), u.dw.numel(), am, r.bits, r.method, r.div, r.bw, ptr<int32_t>(rand),
-                                want_grad ? ptr<int8_t>(u.g8) : nullptr, ptr<int32_t>(u.shift), ptr<int32_t>(exp_a), ptr<int32_t>(exp_b),
-                                ptr<int32_t>(e), stream_of(act)),
-            "niti_grad_update_i8");
+    const bool one = weight_gradient(fuse, act, err, w, stride, pad, g, &u, e);
+    return put_all({wrap(u.g8), wrap(u.dw), wrap(u.shift), wrap(e), boolean(one)});
+  });
+}
+
+// layer_backward(fuse, err, act, w, stride, pad, f32, error bits, method, div, bw, error shift state, exp_err, exp_w, forward copy, mask,
+//                pool_in, ties, error rand, mu, gradient method, want_grad, want_dw, gradient shift state, exp_act, prepared, gradient rand)
+//   -> (error, exponent, unpooled?, g8, dw, shift, exponent, one call?)
+// TiConv2d.backward: both gradients in one launch where that is the faster way, one after the other otherwise.
+PyObject* layer_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a(args, n, 27, "conv layer backward");
+    const bool fuse = a.flag();
+    const at::Tensor& err = a.tensor();
+    const at::Tensor& act = a.tensor();
+    const at::Tensor& w = a.tensor();
+    Fused f;
+    f.dgrad = true;
+    f.stride = a.i();
+    f.pad = a.i();
+    f.f32 = a.flag();
+    f.r = rounding_of(a);
+    f.shift = a.opt();
+    f.hint = f.shift != nullptr;
+    f.exp_a = a.opt();
+    f.exp_b = a.opt();
+    f.prepared = a.opt();
+    f.mask = a.opt();
+    Opt pool_in = a.opt();
+    f.ties = a.i();
+    f.rand = a.opt();
+    WeightGradient g;
+    g.flags = f.f32 ? NITI_EPI_F32_ROUNDTRIP : 0u;
+    g.r = f.r;
+    g.r.bits = a.i();
+    g.r.method = a.i();
+    take_weight_gradient(a, &g);
+    g.exp_b = a.opt();
+    g.prepared = a.opt();
+    g.rand = a.opt();
+    DataGradient r;
+    r.e = scalar32(err);
+    at::Tensor e = scalar32(act);
+    Update u;
+    bool one = fuse && both_gradients(act, err, w, f, pool_in, g, &r, &u, e);
+    if (!one) {
+      data_gradient(fuse, err, w, f, pool_in, &r);
+      g.exp_a = &r.e;
+      one = weight_gradient(fuse && g.rand == nullptr, act, err, w, f.stride, f.pad, g, &u, e);
     }
-    PyObject* out = PyTuple_New(5);
-    if (out == nullptr) throw python_error();
-    PyTuple_SET_ITEM(out, 0, wrap(u.g8));
-    PyTuple_SET_ITEM(out, 1, wrap(u.dw));
-    PyTuple_SET_ITEM(out, 2, wrap(u.shift));
-    PyTuple_SET_ITEM(out, 3, wrap(e));
-    PyObject* b = one ? Py_True : Py_False;
-    Py_INCREF(b);
-    PyTuple_SET_ITEM(out, 4, b);
-    return out;
+    return put_all({wrap(r.y), wrap(r.e), boolean(r.unpooled), wrap(u.g8), wrap(u.dw), wrap(u.shift), wrap(e), boolean(one)});
   });
 }
 
@@ -528,7 +613,7 @@ PyMethodDef kConvMethods[] = {{"conv_fprop", FAST(fprop)},
                               {"conv_fprop_requant", FAST(fprop_requant)},
                               {"conv_dgrad_requant", FAST(dgrad_requant)},
                               {"conv_layer_forward", FAST(layer_forward)},
-                              {"conv_layer_dgrad", FAST(layer_dgrad)},
+                              {"conv_layer_backward", FAST(layer_backward)},
                               {"conv_wgrad_update", FAST(wgrad_update)},
                               {"conv_layer_wgrad_update", FAST(layer_wgrad_update)},
                               {nullptr, nullptr, 0, nullptr}};

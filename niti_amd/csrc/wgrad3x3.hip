@@ -1122,14 +1122,23 @@ size_t wgrad3x3_workspace(int N, int H, int C, int K) {
 // against 11.7 us, 24 images 25.8 / 21.0, 80 images 33.5 / 37.2 (a fifth is kept as margin: operands that the launch before
 // has just written cost its many tiles more).  NITI_WGRAD_ANY=0 / 1 pins the choice (tests), as do the other
 // pins of this file.
+static double nine_tap_us(int N, int H, int C, int K) {
+  const int splits = pick_splits(N, H, C, K), bands = (N * H * H + 255) / 256;
+  return 14.5 + 1.55 * ((bands + splits - 1) / splits) + 0.3e-6 * static_cast<double>(wgrad3x3_workspace(N, H, C, K));
+}
 bool wgrad3x3_prefers_any(int N, int H, int C, int K) {
   const char* e = getenv("NITI_WGRAD_ANY");
   const double any = conv_any_wgrad_us({N, H, H, C, K, 3, 3, 1, 1});
   if (any == 0.0) return false;
   if (e != nullptr) return e[0] != '0';
   if (getenv("NITI_WGRAD_ONE_LAUNCH") != nullptr || getenv("NITI_WGRAD_BLOCKS") != nullptr || !use_narrow_arrangement(N, H)) return false;
-  const int splits = pick_splits(N, H, C, K), bands = (N * H * H + 255) / 256;
-  return any < 0.8 * (14.5 + 1.55 * ((bands + splits - 1) / splits) + 0.3e-6 * static_cast<double>(wgrad3x3_workspace(N, H, C, K)));
+  return any < 0.8 * nine_tap_us(N, H, C, K);
+}
+
+// estimated time of the gradient with update, whichever kernel takes it
+double wgrad3x3_us(int N, int H, int C, int K) {
+  if (wgrad_small_supported(N, H, C, K, C)) return 9.5 + 3.3e-3 * N * H * H + 7.6e-6 * C * K;
+  return wgrad3x3_prefers_any(N, H, C, K) ? conv_any_wgrad_us({N, H, H, C, K, 3, 3, 1, 1}) : nine_tap_us(N, H, C, K);
 }
 
 static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N, int H, int C, int K, int Cp, void* workspace,

@@ -223,6 +223,19 @@ def conv2d_wgrad_update(act, err, w, stride=1, padding=1, f32_epilogue=False, mu
                                       want_grad, want_dw, shift_out, exp_a, exp_b, exp_out, workspace, prepared_filter)
 
 
+def conv2d_backward(err, act, w, padding=1, f32_epilogue=False, err_bits=7, err_method="round", mu=5, grad_method="psto", div_mode="floor",
+                    bw_mode="int", relu_mask=None, pool_in=None, ties="first", err_rand=None, want_grad=False, exp_err=None, exp_w=None,
+                    exp_act=None, prepared_filter=None, err_shift=None, grad_shift=None):
+    """TiConv2d.backward (ti_torch.py:404-437), stride 1: err [N,P,Q,K], act [N,H,W,C], w [K,R,S,C] int8, w updated in place behind the
+    data gradient that reads it; both gradients in one launch where that is the faster way.  ``pool_in``: relu_mask is the output of
+    a 2x2 / stride-2 max-pool on it, the error comes back at its size (element 2 of the result says whether it did).
+    ``err_shift`` / ``grad_shift``: predicted shifts, overwritten with the actual ones.
+    Returns (error, its exponent, unpooled?, int8 gradient or None, int32 gradient or None, gradient shift, gradient exponent, one call?)."""
+    return L.host().conv_layer_backward(True, err, act, w, 1, padding, f32_epilogue, err_bits, L.ROUND[err_method], L.DIV[div_mode], L.BW[bw_mode],
+                                        err_shift, exp_err, exp_w, prepared_filter, relu_mask, pool_in, L.TIES[ties], err_rand, mu,
+                                        L.ROUND[grad_method], want_grad, False, grad_shift, exp_act, prepared_filter, None)
+
+
 def gemm(a, b, trans_a=False, trans_b=False, absmax=None, out=None, f32_epilogue=False):
     """c[m,n] = op(a) @ op(b), int8 x int8 -> int32.  trans_a: a stored [k,m]; trans_b: b stored [n,k].
     f32_epilogue: every sum takes the int32 -> float32 -> int32 round trip of the reference's convolution epilogue."""

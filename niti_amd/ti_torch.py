@@ -439,19 +439,21 @@ class TiConv2d(UpdateWeight):
                 rand = _sto_rand(method, rand, (N, P - 2 * self.padding + R - 1, Q - 2 * self.padding + S - 1, C), dev)
             elif rand is not None:
                 rand = None
-            err_out, new_exp, unpooled = host.conv_layer_dgrad(
-                FUSE_CONV_REQUANT, err_in, weight, self.stride, self.padding, F32_EPILOGUE, BITWIDTH, method, div, bw,
-                self._shift_state("err", dev), d["err_exp_in"], self._wexp(),
-                prepared if act16.shape[3] == weight.shape[3] else None, mask, pool_in, _lib.TIES[POOL_TIES], rand)
+        g_method = _method_code(GRAD_ROUND_METHOD)
+        grad_rand = _sto_rand(g_method, grad_rand, tuple(weight.shape), dev)
+        if self.first_layer:
+            d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"], one = host.conv_layer_wgrad_update(
+                FUSE_CONV_REQUANT and grad_rand is None, act16, err_in, weight, self.stride, self.padding, False, GRAD_BITWIDTH, g_method, div, bw,
+                self.keep_grad, KEEP_INT32_GRAD, self._shift_state("grad", dev), d["err_exp"], _exp_tensor(d["act_in_exp"], dev), prepared,
+                grad_rand)
+        else:
+            err_out, d["err_exp"], unpooled, d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"], one = host.conv_layer_backward(
+                FUSE_CONV_REQUANT, err_in, act16, weight, self.stride, self.padding, F32_EPILOGUE, BITWIDTH, method, div, bw,
+                self._shift_state("err", dev), d["err_exp_in"], self._wexp(), prepared if act16.shape[3] == weight.shape[3] else None, mask,
+                pool_in, _lib.TIES[POOL_TIES], rand, GRAD_BITWIDTH, g_method, self.keep_grad, KEEP_INT32_GRAD, self._shift_state("grad", dev),
+                _exp_tensor(d["act_in_exp"], dev), prepared, grad_rand)
             if unpooled:
                 pool.__dict__["bwd_done"] = err_out
-            d["err_exp"] = new_exp
-        method = _method_code(GRAD_ROUND_METHOD)
-        grad_rand = _sto_rand(method, grad_rand, tuple(weight.shape), dev)
-        d["grad"], d["grad_int32acc"], d["grad_shift"], d["grad_exp"], one = host.conv_layer_wgrad_update(
-            FUSE_CONV_REQUANT and grad_rand is None, act16, err_in, weight, self.stride, self.padding,
-            F32_EPILOGUE and not self.first_layer, GRAD_BITWIDTH, method, div, bw, self.keep_grad, KEEP_INT32_GRAD,
-            self._shift_state("grad", dev), d["err_exp"], _exp_tensor(d["act_in_exp"], dev), prepared, grad_rand)
         if not one:
             d["_wprep_key"] = None      # any kernel-ready copy of the old weights is stale now
         if not self.first_layer:

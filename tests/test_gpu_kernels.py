@@ -1365,3 +1365,61 @@ def test_linear_backward_together(dev, case, tile, monkeypatch):
         assert torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh and int(ge.cpu()) == gsh + dsh - 7 + 2
         assert torch.equal(wd.cpu(), po.weight_update(w, gref))
     assert not ops.sync_arena.timed_out(dev)
+
+
+# (N, H, W, C, K, filter, padding): edges of the tiles of both gradients, maps of the 3x3 kernels and others
+TOGETHER = [(1, 1, 1, 16, 16, 3, 1), (3, 7, 9, 32, 48, 3, 1), (2, 4, 6, 128, 144, 5, 2), (5, 13, 6, 48, 32, 1, 0), (2, 6, 6, 16, 64, 5, 0), (9, 14, 14, 96, 160, 3, 1),
+            (1, 8, 8, 512, 64, 3, 1), (7, 8, 8, 48, 208, 3, 1), (2, 16, 16, 64, 96, 3, 1), (5, 4, 4, 128, 64, 3, 1), (1, 32, 32, 32, 48, 3, 1)]
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", "3", ""])
+@pytest.mark.parametrize("case", TOGETHER)
+def test_conv_backward_together(dev, case, tile, monkeypatch):
+    """Both gradients of a convolution as one launch, the reduction over the pixels whole and cut: the error comes from the old
+    weights, is masked and routed through the max-pool below, the exponents add up, the filter copy follows."""
+    from niti_amd import _lib, ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, H, W, C, K, R, pad = case
+    if tile:
+        monkeypatch.setenv("NITI_ANY_TILE", tile)
+    monkeypatch.setenv("NITI_BACKWARD_TOGETHER", "1")
+    _say("conv_backward_together", case, tile)
+    g = torch.Generator().manual_seed(9900 + N + H + C + K)
+    x, w = ri8(g, N, H, W, C), ri8(g, K, R, R, C)
+    e = ri8(g, N, H + 2 * pad - R + 1, W + 2 * pad - R + 1, K, lo=-40, hi=40)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    dacc, wacc = co.conv_dgrad(e, w, H, W, 1, pad), co.conv_wgrad(x, e, R, R, 1, pad)
+    gref, gsh = po.grad_calc(wacc, 5, "psto")
+    whole = ri8(g, N, 2 * H, 2 * W, C, lo=-3, hi=4)      # few values: ties in most windows
+    pooled = po.maxpool_fwd(whole)
+    rand = torch.randint(0, 1 << 20, dacc.shape, generator=g, dtype=torch.int32)
+    ran = False
+    for slices in ("1", "3", ""):
+        monkeypatch.setenv("NITI_ANY_SLICES", slices) if slices else monkeypatch.delenv("NITI_ANY_SLICES")
+        if _lib.lib().niti_conv2d_i8_backward_sync_words(N, H, W, C, K, R, R, pad) == 0:
+            continue       # the pinned tiles are not resident together
+        ran = True
+        for kind in ("plain", "mask", "first", "all", "sto"):
+            method = "sto" if kind == "sto" else "round"
+            dref, dsh = po.err_calc(dacc, method, rand=rand % (1 << max(po.RangeEstimate(dacc, "int") - 7, 0)))
+            wd = w.to(dev)
+            prepared = ops.conv_filter_prepare(wd, N, H, W, 1, pad)
+            guess = [scalar(dsh), scalar(gsh + 1)]
+            dx, de, unpooled, g8, _, sh, ge, one = ops.conv2d_backward(
+                e.to(dev), x.to(dev), wd, pad, err_method=method, relu_mask=None if kind in ("plain", "sto") else (x if kind == "mask" else pooled).to(dev),
+                pool_in=whole.to(dev) if kind in ("first", "all") else None, ties=kind if kind in ("first", "all") else "first",
+                err_rand=rand.to(dev) if kind == "sto" else None, want_grad=True, exp_err=scalar(-4), exp_w=scalar(-3), exp_act=scalar(2),
+                prepared_filter=prepared, err_shift=guess[0], grad_shift=guess[1])
+            if kind == "mask":
+                dref = dref * (x > 0)
+            elif kind in ("first", "all"):
+                dref = po.maxpool_bwd(pooled, dref * (pooled > 0), whole, ties=kind)
+            assert one and unpooled == (kind in ("first", "all"))
+            assert torch.equal(dx.cpu(), dref) and int(de.cpu()) == dsh - 7 and int(guess[0].cpu()) == dsh, (kind, slices)
+            assert torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh and int(ge.cpu()) == gsh + dsh - 7 + 2, (kind, slices)
+            assert torch.equal(wd.cpu(), po.weight_update(w, gref))
+            if prepared is not None:
+                assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, H, W, 1, pad))
+    assert ran or tile
+    assert not ops.sync_arena.timed_out(dev)
