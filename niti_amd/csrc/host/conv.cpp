@@ -216,10 +216,13 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
     flags |= NITI_CONV_FILTER_PREPARED | (f.forward_copy ? NITI_CONV_FILTER_FORWARD_COPY : 0u);
     wp = ptr<int8_t>(*f.prepared);
   } else {
-    bytes = niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
-    ws = empty8({static_cast<int64_t>(bytes > 16 ? bytes : 16)}, x);
+    // only the 3x3 kernels, whose maps are squares of a power of two, read a copy of the filter
+    if (!any || (d.R == 3 && d.S == 3 && d.H == d.W && (d.H & (d.H - 1)) == 0)) {
+      bytes = niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
+      ws = empty8({static_cast<int64_t>(bytes > 16 ? bytes : 16)}, x);
+    }
   }
-  void* wsp = f.prepared != nullptr ? nullptr : ws.data_ptr();
+  void* wsp = ws.defined() ? ws.data_ptr() : nullptr;
   const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u) | (any ? NITI_RQ_ANY_SHAPE : 0u);
   const int8_t* xp = ptr<int8_t>(x);
   int8_t* yp = ptr<int8_t>(*y);

@@ -27,6 +27,8 @@ struct Arena {
   size_t chunk = 0;
   long pos = 0;
   std::vector<std::pair<size_t, long>> taken;   // slices since the reset
+  at::Tensor scalars;                           // block that scalar32 cuts from, and what is left of it
+  int scalars_left = 0;
   unsigned long long capture = 0, used = 0;
 };
 std::map<std::pair<int, void*>, Arena> g_arenas;
@@ -39,8 +41,7 @@ unsigned long long capture_id(hipStream_t s) {
   return id + 1;
 }
 
-Arena& arena_of(int device) {
-  hipStream_t s = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+Arena& arena_of(int device, hipStream_t s) {
   const auto key = std::make_pair(device, static_cast<void*>(s));
   auto it = g_arenas.find(key);
   if (it == g_arenas.end()) {
@@ -62,11 +63,27 @@ void arena_restart(Arena& a) {
   a.taken.clear();
 }
 
+// The arena of the tensor's device and current stream.  Where a capture has begun or ended since its last use it starts
+// afresh: its memory has to be the graph's, and filled inside it.
+Arena& arena_now(const at::Tensor& like) {
+  hipStream_t s = static_cast<hipStream_t>(stream_of(like));
+  Arena& a = arena_of(like.device().index(), s);
+  const unsigned long long id = capture_id(s);
+  if (id != a.capture) {
+    a.chunks.clear();
+    arena_restart(a);
+    a.scalars = at::Tensor();
+    a.scalars_left = 0;
+    a.capture = id;
+  }
+  return a;
+}
+
 PyObject* arena_reset(PyObject*, PyObject* arg) {
   return guarded([&]() -> PyObject* {
     const long device = PyLong_AsLong(arg);
     if (device < 0) refuse("arena_reset: device index expected");
-    arena_restart(arena_of(static_cast<int>(device)));
+    arena_restart(arena_of(static_cast<int>(device), c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream()));
     Py_RETURN_NONE;
   });
 }
@@ -247,7 +264,7 @@ PyObject* quantize_input(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     at::Tensor y = out != nullptr ? *out : empty8({N, H, W, cpad}, x);
     at::Tensor e = exp_given != nullptr ? *exp_given : scalar32(x);
-    at::Tensor parts = empty32({256}, x);
+    at::Tensor parts = scratch(256 * sizeof(int32_t), x);
     check(niti_quantize_batch_f32_i8(ptr<float>(x), ptr<int8_t>(y), static_cast<int>(N), static_cast<int>(C), static_cast<int>(H),
                                      static_cast<int>(W), static_cast<int>(cpad), bits, ptr<uint32_t>(parts), ptr<int32_t>(e),
                                      ptr<int64_t>(target), ptr<int64_t>(target_out), static_cast<int>(targets), stream_of(x)),
@@ -290,15 +307,24 @@ at::Tensor gemm(const at::Tensor& a, const at::Tensor& b, bool ta, bool tb, uint
   return gemm_out(a, b, ta, tb, absmax, nullptr, 0u);
 }
 
-uint32_t* arena_take(long words, const at::Tensor& like, at::Tensor* view) {
-  Arena& a = arena_of(like.device().index());
-  hipStream_t s = static_cast<hipStream_t>(stream_of(like));
-  const unsigned long long id = capture_id(s);
-  if (id != a.capture) {   // a capture has begun or ended: its chunks are the graph's, and filled inside it
-    a.chunks.clear();
-    arena_restart(a);
-    a.capture = id;
+at::Tensor scalar32(const at::Tensor& like) {
+  constexpr int kBlock = 128;
+  Arena& a = arena_now(like);
+  if (a.scalars_left == 0) {
+    a.scalars = empty32({kBlock}, like);
+    a.scalars_left = kBlock;
   }
+  at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(a.scalars.storage()), a.scalars.key_set(), a.scalars.dtype());
+  c10::TensorImpl* const impl = t.unsafeGetTensorImpl();
+  impl->set_storage_offset(kBlock - a.scalars_left);
+  impl->set_sizes_contiguous({1});
+  if (--a.scalars_left == 0) a.scalars = at::Tensor();
+  return t;
+}
+
+uint32_t* arena_take(long words, const at::Tensor& like, at::Tensor* view) {
+  Arena& a = arena_now(like);
+  hipStream_t s = static_cast<hipStream_t>(stream_of(like));
   if (a.chunks.empty()) a.chunks.push_back(empty32({words > kChunkWords ? words : kChunkWords}, like));
   while (a.pos + words > a.chunks[a.chunk].numel()) {
     a.chunk += 1;

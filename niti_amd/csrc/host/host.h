@@ -91,7 +91,9 @@ inline at::Tensor empty(at::IntArrayRef shape, at::ScalarType type, const at::Te
 }
 inline at::Tensor empty8(at::IntArrayRef shape, const at::Tensor& like) { return empty(shape, at::kChar, like); }
 inline at::Tensor empty32(at::IntArrayRef shape, const at::Tensor& like) { return empty(shape, at::kInt, like); }
-inline at::Tensor scalar32(const at::Tensor& like) { return empty32({1}, like); }
+// An uninitialised int32 tensor of one element: exponents and shifts, of which a layer returns several per call.  They are cut
+// from blocks of 128 (an allocation takes longer than everything else about such a tensor); no element is handed out twice.
+at::Tensor scalar32(const at::Tensor& like);
 
 inline void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 

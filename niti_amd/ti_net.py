@@ -3,9 +3,16 @@ import collections
 
 import torch
 from torch.nn.modules import Module
+from torch.nn.modules import module as _module
 
 from . import ops, ti_torch
 from .ti_loss import TiLoss
+
+
+def _plain(module):
+    """Whether calling ``module`` is calling its forward method: no hooks, nothing compiled or traced in between."""
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or module._compiled_call_impl is not None)
 
 
 class TiNet(Module):
@@ -94,8 +101,16 @@ class TiNet(Module):
             self._head.next_target = None
             if target is not None and ti_torch.TRAINING and target.dtype == torch.int64 and target.is_contiguous() and target.is_cuda:
                 self._head.next_target = (target, loss_rand)
-        self.out, self.out_exp = self.forward_layers((x_data, x_exp))
-        return self.out, self.out_exp
+        d = self.__dict__       # plain attributes: Module.__setattr__ looks for parameters first
+        layers, x = self.forward_layers, (x_data, x_exp)
+        if type(layers) is torch.nn.Sequential and _plain(layers) and not _module._has_any_global_hook() and torch._C._get_tracing_state() is None:
+            # the container's loop without Module.__call__'s checks per layer (a third of an evaluation step's host time)
+            for layer in layers._modules.values():
+                x = layer.forward(x) if _plain(layer) else layer(x)
+        else:
+            x = layers(x)
+        d["out"], d["out_exp"] = x
+        return d["out"], d["out_exp"]
 
     @property
     def out_bits(self):
@@ -115,7 +130,8 @@ class TiNet(Module):
 
     def backward_from(self, x):
         """Back-propagate a given (int8 error, exponent) pair through the layers in reverse."""
-        for layer in reversed(self.forward_layers):
+        layers = self.forward_layers
+        for layer in reversed(list(layers._modules.values()) if type(layers) is torch.nn.Sequential else layers):
             if isinstance(layer, torch.nn.Sequential):
                 for block in reversed(layer):
                     x = block.backward(x)
