@@ -47,6 +47,8 @@ enum {
 #define NITI_RQ_RELU 1u /* clamp the int8 result at 0 (TiReLU.forward, ti_torch.py:272-279) */
 #define NITI_RQ_ANY_SHAPE 4u /* niti_conv2d_i8_*_requant*: also run what niti_conv2d_i8_requant_sync_words does not cover but
                                 niti_conv2d_i8_requant_sync_words_any does (sync sized by that) */
+#define NITI_RQ_ANY_KERNEL 8u /* niti_conv2d_i8_fprop_requant*: the kernel for any shape, on w as stored (sync sized by
+                                 niti_conv2d_i8_fprop_small_sync_words) */
 #define NITI_RQ_SHIFT_HINT 2u /* niti_conv2d_i8_*_requant: *shift_out holds a predicted shift on entry (the same
                                  tensor's shift of the previous training step).  The kernels store results before the
                                  tensor's range is final and store again if the shift turns out different; a good
@@ -158,6 +160,8 @@ int niti_conv2d_i8_dgrad(const int8_t* err, const int8_t* w, int32_t* dx, int N,
  * equal to the pooled maximum.
  */
 size_t niti_conv2d_i8_requant_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad);
+/* sync words of a forward pass with NITI_RQ_ANY_KERNEL; 0 unless the batch is small enough for that to be the faster kernel */
+size_t niti_conv2d_i8_fprop_small_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 /* the same for calls with NITI_RQ_ANY_SHAPE: batches that are no whole tiles of 256 pixels are covered too */
 size_t niti_conv2d_i8_requant_sync_words_any(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad);
 int niti_conv2d_i8_fprop_requant(const int8_t* x, const int8_t* w, int8_t* y8, int N, int H, int W, int C, int K, int R,

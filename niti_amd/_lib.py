@@ -78,6 +78,7 @@ SIGNATURES = {
     "niti_linear_i8_fwd_requant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _u, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "niti_linear_i8_dgrad_requant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "niti_linear_i8_wgrad_update": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "niti_conv2d_i8_fprop_small_sync_words": (_sz, [_i] * 9),
     "niti_conv2d_i8_backward_sync_words": (_sz, [_i] * 8),
     "niti_conv2d_i8_backward_workspace": (_sz, [_i] * 8),
     "niti_conv2d_i8_backward": (_i, [_vp] * 4 + [_i] * 8 + [_u, _i, _i, _vp, _vp, _vp] + [_i] * 5 + [_vp, _sz] + [_vp] * 10 + [_sz, _vp]),

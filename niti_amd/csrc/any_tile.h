@@ -314,6 +314,16 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
   uint32_t wold[G];
   constexpr bool kUnpool = MODE == kRequant && G <= 4;   // the launches that use it have these tiles
   uint32_t window[kUnpool ? G : 1][4];
+  constexpr bool kPool = MODE == kRequant && T::BN <= 64;      // a window's four rows lie in one wavefront
+  auto place = [&](int row, int col) {                         // of a result
+    if constexpr (kPool) {
+      if (g.pool != nullptr) {
+        const int image = g.by_map.of(row), rest = row - image * (g.map_h * g.map_w), window = rest >> 2, wh = g.by_map_w.of(window);
+        row = image * (g.map_h * g.map_w) + (2 * wh + ((rest >> 1) & 1)) * g.map_w + 2 * (window - wh * (g.map_w >> 1)) + (rest & 1);
+      }
+    }
+    return static_cast<long long>(row) * g.n + col;
+  };
   auto window_at = [&](int row, int col) {
     const int image = g.by_map.of(row), rest = row - image * (g.map_h * g.map_w), h = g.by_map_w.of(rest), w = rest - h * g.map_w;
     return (static_cast<long long>(image * 2 * g.map_h + 2 * h) * (2 * g.map_w) + 2 * w) * g.n + col;
@@ -326,7 +336,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
       rnd[i] = v4i{0, 0, 0, 0};
       wold[i] = 0;
       if ((GROUPS < 512 && t >= GROUPS) || row >= g.m || col + 4 > g.n) continue;
-      const long long at = static_cast<long long>(row) * g.n + col;
+      const long long at = place(row, col);
       if (g.method == NITI_ROUND_STOCHASTIC) __builtin_memcpy(&rnd[i], g.rand + at, 16);
       if (MODE == kUpdate) __builtin_memcpy(&wold[i], g.w + at, 4);
       if (MODE == kRequant && g.mask != nullptr) __builtin_memcpy(&wold[i], g.mask + at, 4);
@@ -345,7 +355,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
     if (GROUPS < 512 && t >= GROUPS) continue;
     const int row = m0 + t / (T::BN / 4), col = n0 + t % (T::BN / 4) * 4;
     if (row >= g.m || col >= g.n) continue;
-    const long long at = static_cast<long long>(row) * g.n + col;
+    const long long at = place(row, col);
     const int here = min(4, g.n - col);
     if (MODE == kInt32) {
       if (here == 4) {
@@ -387,6 +397,13 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
     }
     if (here == 4) {
       const uint32_t packed = pack4_i8(r[0], r[1], r[2], r[3]);
+      if constexpr (kPool) {
+        if (g.pool != nullptr) {     // whole windows are inside the result or outside, columns a multiple of 4
+          uint32_t mx = max_i8x4(packed, static_cast<uint32_t>(__shfl_xor(static_cast<int>(packed), T::BN / 4)));
+          mx = max_i8x4(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), T::BN / 2)));
+          if ((row & 3) == 0) __builtin_memcpy(g.pool + static_cast<long long>(row >> 2) * g.n + col, &mx, 4);
+        }
+      }
       if (MODE == kUpdate) {
         const uint32_t old = wold[i];
         int wn4[4];

@@ -319,6 +319,20 @@ extern "C" size_t niti_conv2d_i8_requant_sync_words_any(int N, int H, int W, int
   return nb > 0 ? conv3x3_halo_sync_words(nb) : conv_any_requant_words(dgrad ? kConvDgrad : kConvForward, {N, H, W, C, K, R, S, stride, pad});
 }
 
+// Few images on the 3x3 kernels' maps: their workgroups of 256 pixels leave most of the chip idle and walk all input channels
+// (stages of 32, longer on the wider maps), where the kernel for any shape has 32 x 32 tiles.  One image: 32 x 32, 128 -> 128
+// 8.3 against 6.2 us, 16 x 16, 256 -> 256 11.3 / 7.0, 8 x 8, 512 -> 512 12.9 / 8.6; 24 images of the latter 13.4 / 15.5.
+extern "C" size_t niti_conv2d_i8_fprop_small_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
+  if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0 || K % 4 != 0) return 0;
+  const ConvShape s{N, H, W, C, K, R, S, stride, pad};
+  const char* e = getenv("NITI_FPROP_SMALL");   // 0 / 1 pins (tests)
+  if (e != nullptr) return e[0] != '0' ? conv_any_requant_words(kConvForward, s) : 0;
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0, true);
+  if (nb == 0 || nb > 256) return 0;
+  const double us = conv_any_forward_us(s), stage = H >= 32 ? 1.25 : H == 16 ? 1.05 : 0.62;
+  return us > 0.0 && us < 0.9 * (3.5 + stage * ((C + 31) / 32)) ? conv_any_requant_words(kConvForward, s) : 0;
+}
+
 static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_t* w, int8_t* y8, int N, int H, int W, int C,
                         int K, int R, int S, int stride, int pad, unsigned flags, int target_bits, int method, int div_mode,
                         int bw_mode, unsigned rq_flags, const int8_t* relu_mask, uint32_t* sync, size_t sync_words,
@@ -338,9 +352,11 @@ static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_
   if (rand != nullptr && !aligned16(rand)) return fail(NITI_ERR_INVALID_ARG, "%s: rand must be 16-byte aligned", who);
   if (div_mode != NITI_DIV_FLOOR && div_mode != NITI_DIV_TRUNC) return fail(NITI_ERR_INVALID_ARG, "%s: div_mode=%d", who, div_mode);
   if (bw_mode != NITI_BW_INT && bw_mode != NITI_BW_F32) return fail(NITI_ERR_INVALID_ARG, "%s: bw_mode=%d", who, bw_mode);
-  if ((rq_flags & ~(NITI_RQ_RELU | NITI_RQ_SHIFT_HINT | NITI_RQ_ANY_SHAPE)) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
-  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, (rq_flags & NITI_RQ_ANY_SHAPE) != 0u);
-  if (nb == 0 && (rq_flags & NITI_RQ_ANY_SHAPE) != 0u && pool_out == nullptr && pool_x == nullptr && (!dgrad || (flags & NITI_CONV_FILTER_PREPARED) == 0u)) {
+  if ((rq_flags & ~(NITI_RQ_RELU | NITI_RQ_SHIFT_HINT | NITI_RQ_ANY_SHAPE | NITI_RQ_ANY_KERNEL)) != 0u) return fail(NITI_ERR_INVALID_ARG, "%s: rq_flags=%#x", who, rq_flags);
+  const bool any_kernel = (rq_flags & NITI_RQ_ANY_KERNEL) != 0u;
+  const int nb = any_kernel ? 0 : fused_blocks(N, H, W, C, K, R, S, stride, pad, dgrad, (rq_flags & NITI_RQ_ANY_SHAPE) != 0u);
+  if (nb == 0 && (any_kernel || (rq_flags & NITI_RQ_ANY_SHAPE) != 0u) && (pool_out == nullptr || any_kernel) && pool_x == nullptr &&
+      ((!dgrad && !any_kernel) || (flags & NITI_CONV_FILTER_PREPARED) == 0u)) {
     // every other shape, read as stored
     const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
     const ConvPass pass = dgrad ? kConvDgrad : kConvForward;
@@ -348,7 +364,7 @@ static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_
     if (words != 0) {
       if (sync_words < words) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, words, sync_words);
       RequantSpec rq{target_bits, method, div_mode == NITI_DIV_TRUNC, bw_mode, rq_flags, sync_spin_limit(), timeout_word(), shift_out, exp_a, exp_b, exp_out,
-                     relu_mask, nullptr};
+                     relu_mask, pool_out};
       rq.rand = method == NITI_ROUND_STOCHASTIC ? rand : nullptr;
       return launch_conv_any_requant(pass, shape, x, w, y8, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, static_cast<hipStream_t>(stream));
     }

@@ -202,6 +202,16 @@ size_t conv_any_requant_words(ConvPass pass, const ConvShape& s) {
   return words_for(tiles_with(t, m, n));
 }
 
+double conv_any_forward_us(const ConvShape& s) {
+  if (conv_any_requant_words(kConvForward, s) == 0) return 0.0;
+  int m, n, k;
+  product_of(kConvForward, s, &m, &n, &k);
+  const int t = requant_tile(kConvForward, s);
+  if (t > 1) return 1e9;   // the wide tiles: not for the few workgroups this is asked for
+  const double chunks = t == 0 ? (k + TileS::BK - 1) / TileS::BK : (k + TileM::BK - 1) / TileM::BK;
+  return (t == 0 ? 4.9 + 0.42 * chunks : 5.6 + 0.58 * chunks) * (tiles_with(t, m, n) > 256 ? 1.5 : 1.0);
+}
+
 double conv_any_dgrad_us(const ConvShape& s) {
   if (conv_any_requant_words(kConvDgrad, s) == 0) return 0.0;
   constexpr double kChunk[4] = {0.58, 0.58, 0.47, 0.68};
@@ -216,7 +226,16 @@ int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* x, 
   ConvAnyArgs a = args_of(pass, s, x, w, roundtrip);
   set_rounding(a.g, rq, sync);
   a.g.out8 = y;
+  if (rq.pool != nullptr) {
+    a.g.pool = rq.pool;
+    a.g.map_h = a.P;
+    a.g.map_w = a.Q;
+    a.g.by_map = a.by_pq;
+    a.g.by_map_w = Reciprocal(a.Q / 2);
+  }
   const int t = requant_tile(pass, s);
+  if (rq.pool != nullptr && (t == 3 || pass != kConvForward || a.P % 2 != 0 || a.Q % 2 != 0 || s.K % 4 != 0))
+    return fail(NITI_ERR_UNSUPPORTED, "conv_any: this launch's tiles do not fit whole pooling windows");
   if (t < 0) return fail(NITI_ERR_UNSUPPORTED, "conv_any: the workgroups of a %d x %d result do not fit on the device at once", a.g.m, a.g.n);
   return pass == kConvForward ? launch_tile<kConvForward, kRequant>(t, a, 1, stream) : launch_tile<kConvDgrad, kRequant>(t, a, 1, stream);
 }

@@ -44,7 +44,15 @@ struct PixelRows {
     for (int i = 0; i < G::N; ++i) {
       const int m = first + G::row(i);
       const int n = a.by_pq.of(m), pq = m - n * (a.P * a.Q);
-      const int p = a.by_q.of(pq), q = pq - p * a.Q;
+      int p, q;
+      if (a.g.pool == nullptr) {
+        p = a.by_q.of(pq);
+        q = pq - p * a.Q;
+      } else {               // window by window
+        const int window = pq >> 2, wp = a.g.by_map_w.of(window);
+        p = 2 * wp + ((pq >> 1) & 1);
+        q = 2 * (window - wp * (a.Q >> 1)) + (pq & 1);
+      }
       h[i] = m < a.pixels ? p * a.stride - a.pad : -0x20000000;   // no tap of it is inside
       w[i] = q * a.stride - a.pad;
       at[i] = ((n * a.H + p * a.stride - a.pad) * a.W + w[i]) * a.C;

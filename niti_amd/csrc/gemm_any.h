@@ -35,6 +35,9 @@ struct AnyArgs {
   const int8_t* mask = nullptr;   // laid out like out8: results are zero where it is not positive (not for the weight update)
   // with a mask: the result is the gradient of a 2x2 / stride-2 max-pool's output (= mask, [rows][map_h][map_w][n]) and goes to
   // the position(s) of each window of the pool's input pool_x that hold the maximum, in unpool; out8 is not written
+  // pool: rows come window by window (2 x 2 pixels of the [map_h][map_w] result, by_map_w divides by map_w / 2) and the maximum of
+  // each window goes there as well
+  int8_t* pool = nullptr;
   const int8_t* pool_x = nullptr;
   int8_t* unpool = nullptr;
   int ties_all = 0, map_h = 0, map_w = 0;

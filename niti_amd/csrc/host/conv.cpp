@@ -163,6 +163,7 @@ PyObject* wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // ---- results rounded to int8 in the launch -------------------------------------------------------------------------
 struct Fused {
+  bool current = false;   // forward: w holds the filter itself (next to `prepared`)
   bool dgrad = false, f32 = false, relu = false, hint = false, forward_copy = false, any_shape = false;
   int stride = 1, pad = 1, ties = 0;
   Rounding r{};
@@ -197,7 +198,9 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
   }
   if (!is_i8(x) || !is_i8(w)) refuse(std::string(who) + ": int8 tensors expected");
   const bool any = soft || f.any_shape;
-  const size_t words = any ? niti_conv2d_i8_requant_sync_words_any(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg)
+  // few images: the kernel for any shape, which reads the filter as stored
+  const size_t small = soft && f.current ? niti_conv2d_i8_fprop_small_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad) : 0;
+  const size_t words = small > 0 ? small : any ? niti_conv2d_i8_requant_sync_words_any(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg)
                            : niti_conv2d_i8_requant_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.stride, f.pad, dg);
   if (words == 0) {
     if (soft) return false;
@@ -212,7 +215,9 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
   at::Tensor ws;
   size_t bytes = 0;
   const int8_t* wp = ptr<int8_t>(w);
-  if (f.prepared != nullptr) {
+  if (small > 0) {
+    // nothing to prepare
+  } else if (f.prepared != nullptr) {
     flags |= NITI_CONV_FILTER_PREPARED | (f.forward_copy ? NITI_CONV_FILTER_FORWARD_COPY : 0u);
     wp = ptr<int8_t>(*f.prepared);
   } else {
@@ -223,7 +228,7 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
     }
   }
   void* wsp = ws.defined() ? ws.data_ptr() : nullptr;
-  const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u) | (any ? NITI_RQ_ANY_SHAPE : 0u);
+  const unsigned rq = (f.relu ? NITI_RQ_RELU : 0u) | (f.hint ? NITI_RQ_SHIFT_HINT : 0u) | (any ? NITI_RQ_ANY_SHAPE : 0u) | (small > 0 ? NITI_RQ_ANY_KERNEL : 0u);
   const int8_t* xp = ptr<int8_t>(x);
   int8_t* yp = ptr<int8_t>(*y);
   int32_t* sp = ptr<int32_t>(*shift);
@@ -308,13 +313,14 @@ PyObject* requant_op(PyObject* const* args, Py_ssize_t n, bool dg) {
 PyObject* fprop_requant(PyObject*, PyObject* const* args, Py_ssize_t n) { return requant_op(args, n, false); }
 PyObject* dgrad_requant(PyObject*, PyObject* const* args, Py_ssize_t n) { return requant_op(args, n, true); }
 
-// layer_forward(fuse, x, w, stride, pad, f32, bits, method, div, bw, relu, shift state, exp_a, exp_b, prepared, pool, rand)
+// layer_forward(fuse, x, w, stride, pad, f32, bits, method, div, bw, relu, shift state, exp_a, exp_b, prepared, pool, rand,
+//               w current?)
 //   -> (y, exponent, pooled map or None)
 // TiConv2d.forward: convolution, act_calc and where asked the ReLU and the 2x2 max-pool behind it (`pool`), in one launch
 // where the single-launch kernels cover the shape; otherwise convolution, then requantisation (nothing pooled).
 PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    Args a(args, n, 17, "conv layer forward");
+    Args a(args, n, 18, "conv layer forward");
     const bool fuse = a.flag();
     const at::Tensor& x = a.tensor();
     const at::Tensor& w = a.tensor();
@@ -331,6 +337,7 @@ PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     f.prepared = a.opt();
     const bool pool = a.flag();
     f.rand = a.opt();
+    f.current = a.flag();
     const Dims d = forward_dims(x, w, "conv layer");
     at::Tensor y, shift, pooled, e = scalar32(x);
     f.exp_out = &e;

@@ -401,7 +401,7 @@ class TiConv2d(UpdateWeight):
         y, exp_out, pooled = _lib.host().conv_layer_forward(
             FUSE_CONV_REQUANT, act16, w16, self.stride, self.padding, F32_EPILOGUE, BITWIDTH, method, _lib.DIV[DIV_MODE], _lib.BW[BW_MODE],
             self.fuse_relu, self._shift_state("act", dev), _exp_tensor(act_exp, dev), self._wexp(), d["_wprep"],
-            self.pool_after is not None, rand)
+            self.pool_after is not None, rand, not shape_only)
         if pooled is not None:      # the pooling layer finds its result ready when it sees this tensor
             self.pool_after.__dict__["preset"] = (y, pooled)
         return y, exp_out

@@ -1423,3 +1423,27 @@ def test_conv_backward_together(dev, case, tile, monkeypatch):
                 assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, H, W, 1, pad))
     assert ran or tile
     assert not ops.sync_arena.timed_out(dev)
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", ""])
+@pytest.mark.parametrize("case", [(1, 8, 512, 64), (3, 8, 48, 208), (2, 16, 64, 96), (1, 32, 16, 48), (5, 4, 128, 32), (7, 2, 32, 64)])
+def test_small_batch_forward(dev, case, tile, monkeypatch):
+    """3x3 layers of few images on the kernel for any shape: rounding, ReLU and the 2x2 max-pool behind the layer."""
+    from niti_amd import _lib, ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    if tile:
+        monkeypatch.setenv("NITI_ANY_TILE", tile)
+    monkeypatch.setenv("NITI_FPROP_SMALL", "1")
+    _say("small_batch_forward", case, tile)
+    g = torch.Generator().manual_seed(12100 + N + Q + C)
+    x, w = ri8(g, N, Q, Q, C), ri8(g, K, 3, 3, C)
+    ref = torch.clamp(po.act_calc(co.conv_fprop(x, w, 1, 1), 0)[0], min=0)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    for pool in (False, True):
+        y, e, pooled = _lib.host().conv_layer_forward(True, x.to(dev), w.to(dev), 1, 1, True, 7, _lib.ROUND["round"], _lib.DIV["floor"], _lib.BW["int"],
+                                                      True, scalar(0), scalar(-3), scalar(1), None, pool, None, True)
+        assert torch.equal(y.cpu(), ref) and int(e.cpu()) == po.act_calc(co.conv_fprop(x, w, 1, 1), -2)[1]
+        assert (pooled is not None) == pool and (not pool or torch.equal(pooled.cpu(), po.maxpool_fwd(ref)))
+    assert not ops.sync_arena.timed_out(dev)
