@@ -369,6 +369,11 @@ int niti_quantize_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, 
 int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
                                int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, void* stream);
 
+/* the same, clearing zero[0 .. zero_words) as well (16-byte aligned, a multiple of four words) */
+int niti_quantize_batch_zero_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
+                                    int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, uint32_t* zero,
+                                    int zero_words, void* stream);
+
 /* Display metrics of a step (main.py:156-163, meters.py:56-70) in one launch: sums[0..2] (double) += n x { mean cross entropy of
    softmax(out_val 2^out_exp), top-1 %, top-5 % }.  out_val: [n,classes] int8, target: int64 [n], classes >= 5.  Ties count as
    torch.topk orders them. */

@@ -67,6 +67,7 @@ SIGNATURES = {
     "niti_mask_features_i8": (_i, [_vp, _vp, _vp, _i64, _i, _vp, _vp, _i, _vp]),
     "niti_quantize_f32_i8": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "niti_quantize_batch_f32_i8": (_i, [_vp, _vp] + [_i] * 6 + [_vp, _vp, _vp, _vp, _i, _vp]),
+    "niti_quantize_batch_zero_f32_i8": (_i, [_vp, _vp] + [_i] * 6 + [_vp, _vp, _vp, _vp, _i, _vp, _i, _vp]),
     "niti_batch_metrics_i8": (_i, [_vp, _vp, _vp, _i, _i, _vp, _vp]),
     "niti_maxpool_i8_fwd": (_i, [_vp, _vp] + [_i] * 7 + [_vp]),
     "niti_maxpool_i8_bwd": (_i, [_vp, _vp, _vp, _vp] + [_i] * 8 + [_vp]),

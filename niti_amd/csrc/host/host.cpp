@@ -29,6 +29,7 @@ struct Arena {
   std::vector<std::pair<size_t, long>> taken;   // slices since the reset
   at::Tensor scalars;                           // block that scalar32 cuts from, and what is left of it
   int scalars_left = 0;
+  bool cleared = false;                         // the first chunk was cleared for the period that has just begun
   unsigned long long capture = 0, used = 0;
 };
 std::map<std::pair<int, void*>, Arena> g_arenas;
@@ -74,6 +75,7 @@ Arena& arena_now(const at::Tensor& like) {
     arena_restart(a);
     a.scalars = at::Tensor();
     a.scalars_left = 0;
+    a.cleared = false;
     a.capture = id;
   }
   return a;
@@ -242,10 +244,10 @@ PyObject* maxpool_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---- input quantiser ---------------------------------------------------------------------------------------------
-// quantize_input(x, bits, cpad, out, exp_out, target, target_out) -> (y, exponent)
+// quantize_input(x, bits, cpad, out, exp_out, target, target_out, step begins?) -> (y, exponent)
 PyObject* quantize_input(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    Args a(args, n, 7, "quantize_input");
+    Args a(args, n, 8, "quantize_input");
     const at::Tensor& x = a.tensor();
     const int bits = a.i();
     int64_t cpad = a.integer();
@@ -265,9 +267,20 @@ PyObject* quantize_input(PyObject*, PyObject* const* args, Py_ssize_t n) {
     at::Tensor y = out != nullptr ? *out : empty8({N, H, W, cpad}, x);
     at::Tensor e = exp_given != nullptr ? *exp_given : scalar32(x);
     at::Tensor parts = scratch(256 * sizeof(int32_t), x);
-    check(niti_quantize_batch_f32_i8(ptr<float>(x), ptr<int8_t>(y), static_cast<int>(N), static_cast<int>(C), static_cast<int>(H),
+    uint32_t* zero = nullptr;
+    int zero_words = 0;
+    if (a.flag()) {   // a step begins: its first launch clears the sync words
+      Arena& arena = arena_now(x);
+      arena_restart(arena);
+      if (arena.chunks.empty()) arena.chunks.push_back(empty32({kChunkWords}, x));
+      zero = ptr<uint32_t>(arena.chunks[0]);
+      zero_words = static_cast<int>(arena.chunks[0].numel());
+      if (zero_words > kChunkWords) zero = nullptr, zero_words = 0;   // an unusually long one: left to its own fill
+      arena.cleared = zero != nullptr;
+    }
+    check(niti_quantize_batch_zero_f32_i8(ptr<float>(x), ptr<int8_t>(y), static_cast<int>(N), static_cast<int>(C), static_cast<int>(H),
                                      static_cast<int>(W), static_cast<int>(cpad), bits, ptr<uint32_t>(parts), ptr<int32_t>(e),
-                                     ptr<int64_t>(target), ptr<int64_t>(target_out), static_cast<int>(targets), stream_of(x)),
+                                     ptr<int64_t>(target), ptr<int64_t>(target_out), static_cast<int>(targets), zero, zero_words, stream_of(x)),
           "niti_quantize_batch_f32_i8");
     return tuple_of({y, e});
   });
@@ -341,7 +354,10 @@ uint32_t* arena_take(long words, const at::Tensor& like, at::Tensor* view) {
   }
   at::Tensor& c = a.chunks[a.chunk];
   uint32_t* base = static_cast<uint32_t*>(c.data_ptr());
-  if (a.pos == 0) check(niti_fill_u32(base, c.numel(), 0u, s), "niti_fill_u32");
+  if (a.pos == 0) {
+    if (a.chunk != 0 || !a.cleared) check(niti_fill_u32(base, c.numel(), 0u, s), "niti_fill_u32");
+    if (a.chunk == 0) a.cleared = false;
+  }
   const long at = a.pos;
   a.pos += (words + 31) / 32 * 32;
   a.taken.emplace_back(a.chunk, at);

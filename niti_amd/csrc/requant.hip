@@ -176,10 +176,19 @@ __global__ __launch_bounds__(256) void absmax_parts_f32_kernel(const float* __re
 // channels zero-padded to cpad; exp_out = bw - bits.  The product and the rounding are the reference's float32 operations.
 // r = the largest of nparts partial maxima (one word: the caller's absmax_bits); nparts == 0 (a batch of a few images):
 // every workgroup takes the maximum over the whole batch itself, which saves the launch in front of this one.
+// The last kZeroBlocks workgroups clear `zero` where asked (the words that the launches behind this one exchange their ranges
+// through: one launch less).
+constexpr int kZeroBlocks = 16;
 __global__ __launch_bounds__(256) void quantize_f32_i8_kernel(const float* __restrict__ x, int8_t* __restrict__ y, int64_t pixels,
                                                               int C, int HW, int cpad, const uint32_t* __restrict__ parts, int nparts,
                                                               int32_t* exp_out, int bits, const int64_t* __restrict__ t_in,
-                                                              int64_t* __restrict__ t_out, int nt) {
+                                                              int64_t* __restrict__ t_out, int nt, v4i* __restrict__ zero, int zero_quads) {
+  if (static_cast<int>(blockIdx.x) >= static_cast<int>(gridDim.x) - (zero_quads > 0 ? kZeroBlocks : 0)) {
+    const v4i nothing = {0, 0, 0, 0};
+    for (int i = (static_cast<int>(blockIdx.x) - static_cast<int>(gridDim.x) + kZeroBlocks) * 256 + static_cast<int>(threadIdx.x); i < zero_quads; i += kZeroBlocks * 256)
+      zero[i] = nothing;
+    return;
+  }
   __shared__ uint32_t wmax[4];
   uint32_t m = 0;
   if (nparts > 0) {
@@ -220,7 +229,7 @@ __global__ __launch_bounds__(256) void quantize_f32_i8_kernel(const float* __res
     return word;
   };
   const bool wide = cpad % 16 == 0 && aligned16_dev(y);
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x - (zero_quads > 0 ? kZeroBlocks : 0)) * blockDim.x;
   for (int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < pixels; p += stride) {
     const int64_t n = p / HW, hw = p - n * HW;
     const float* src = x + n * C * HW + hw;
@@ -396,18 +405,21 @@ extern "C" int niti_quantize_f32_i8(const float* x, int8_t* y, int N, int C, int
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(absmax_f32_kernel, dim3(grid_for(n, 256, 1024)), dim3(256), 0, s, x, n, absmax_bits);
   hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad, absmax_bits, 1,
-                     exp_out, bits, static_cast<const int64_t*>(nullptr), static_cast<int64_t*>(nullptr), 0);
+                     exp_out, bits, static_cast<const int64_t*>(nullptr), static_cast<int64_t*>(nullptr), 0, static_cast<v4i*>(nullptr), 0);
   return check_launch("quantize");
 }
 
-extern "C" int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
-                                          int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, void* stream) {
+extern "C" int niti_quantize_batch_zero_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
+                                               int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, uint32_t* zero,
+                                               int zero_words, void* stream) {
   clear_error();
   if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || cpad < C || cpad % 4 != 0 || bits < 1 || bits > 7 || targets < 0)
     return fail(NITI_ERR_INVALID_ARG, "quantize_batch: N=%d C=%d H=%d W=%d cpad=%d bits=%d targets=%d", N, C, H, W, cpad, bits, targets);
   if (x == nullptr || y == nullptr || parts == nullptr || (targets > 0 && (target_in == nullptr || target_out == nullptr)))
     return fail(NITI_ERR_INVALID_ARG, "quantize_batch: null pointer");
   if (reinterpret_cast<uintptr_t>(y) % 4 != 0) return fail(NITI_ERR_INVALID_ARG, "quantize_batch: output must be 4-byte aligned");
+  if (zero_words < 0 || zero_words % 4 != 0 || (zero_words > 0 && (zero == nullptr || !aligned16(zero))))
+    return fail(NITI_ERR_INVALID_ARG, "quantize_batch: words to clear must be whole, aligned groups of four");
   const int64_t pixels = static_cast<int64_t>(N) * H * W, n = pixels * C;
   hipStream_t s = static_cast<hipStream_t>(stream);
   // up to 12 Ki values (four CIFAR images, 48 loads a thread) a workgroup reads the batch in less time than a launch takes
@@ -417,9 +429,14 @@ extern "C" int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int 
     nparts = grid_for((n + 3) / 4, 1024, kQuantParts);
     hipLaunchKernelGGL(absmax_parts_f32_kernel, dim3(nparts), dim3(256), 0, s, x, n, parts, target_in, target_out, targets);
   }
-  hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad, parts, nparts,
-                     exp_out, bits, target_in, target_out, solo ? targets : 0);
+  hipLaunchKernelGGL(quantize_f32_i8_kernel, dim3(grid_for(pixels, 256) + (zero_words > 0 ? kZeroBlocks : 0)), dim3(256), 0, s, x, y, pixels, C, H * W, cpad,
+                     parts, nparts, exp_out, bits, target_in, target_out, solo ? targets : 0, reinterpret_cast<v4i*>(zero), zero_words / 4);
   return check_launch("quantize_batch");
+}
+
+extern "C" int niti_quantize_batch_f32_i8(const float* x, int8_t* y, int N, int C, int H, int W, int cpad, int bits, uint32_t* parts,
+                                          int32_t* exp_out, const int64_t* target_in, int64_t* target_out, int targets, void* stream) {
+  return niti_quantize_batch_zero_f32_i8(x, y, N, C, H, W, cpad, bits, parts, exp_out, target_in, target_out, targets, nullptr, 0, stream);
 }
 
 extern "C" int niti_mask_features_i8(const int8_t* x, const int8_t* mask, int8_t* y, int64_t rows, int features,

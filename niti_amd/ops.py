@@ -295,11 +295,11 @@ def relu_fwd(x):
     return y
 
 
-def quantize_input(x, bits=7, cpad=16, out=None, exp_out=None, target=None, target_out=None):
+def quantize_input(x, bits=7, cpad=16, out=None, exp_out=None, target=None, target_out=None, start_step=False):
     """Float NCHW batch -> (int8 NHWC batch with the channels zero-padded to ``cpad``, exponent as a 1-element int32
     tensor): the reference's input quantiser and the layout change behind it in two launches (one for a few images).
     ``out`` / ``exp_out``: tensors to write instead of new ones; ``target`` (int64) is copied to ``target_out`` on the way."""
-    return L.host().quantize_input(x, bits, cpad, out, exp_out, target, target_out)
+    return L.host().quantize_input(x, bits, cpad, out, exp_out, target, target_out, start_step)
 
 
 def batch_metrics(out_val, out_exp, target, sums):

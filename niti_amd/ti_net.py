@@ -79,7 +79,10 @@ class TiNet(Module):
         """ti_net.py:17-23: float NCHW batch -> (int8 logits, exponent).  ``target`` (not in the reference): the
         class indices that backward() will be called with; the classifier's forward launch then computes the loss
         gradient as well and backward(target) with the same tensor starts from it."""
-        x_data, x_exp = self.quantize_input(x)
+        if type(self).quantize_input is TiNet.quantize_input:
+            x_data, x_exp = self._quantize(x, True)
+        else:
+            x_data, x_exp = self.quantize_input(x)
         return self.forward_int8(x_data, x_exp, target)
 
     @staticmethod
@@ -88,9 +91,14 @@ class TiNet(Module):
         the GPU takes the library's two launches (channels come zero-padded to 16, which the first convolution
         would do next anyway); anything else - and BW_MODE "f32", whose range exponent is the reference's float32
         ``ceil(log2(r))`` rather than the exact one - the reference's tensor operations."""
+        return TiNet._quantize(x, False)
+
+    @staticmethod
+    def _quantize(x, start_step):
+        """``start_step``: the launch also clears the range-exchange words of the step that follows (forward_int8)."""
         x = x.to(ti_torch.GPU)
         if x.dtype == torch.float32 and x.dim() == 4 and x.is_contiguous() and x.is_cuda and ti_torch.BW_MODE == "int":
-            return ops.quantize_input(x, ti_torch.BITWIDTH)
+            return ops.quantize_input(x, ti_torch.BITWIDTH, start_step=start_step)
         x_data, x_exp = ti_torch.TiFloatToInt8(x)
         return x_data.permute(0, 2, 3, 1).contiguous(), x_exp
 

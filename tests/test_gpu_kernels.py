@@ -1447,3 +1447,20 @@ def test_small_batch_forward(dev, case, tile, monkeypatch):
         assert torch.equal(y.cpu(), ref) and int(e.cpu()) == po.act_calc(co.conv_fprop(x, w, 1, 1), -2)[1]
         assert (pooled is not None) == pool and (not pool or torch.equal(pooled.cpu(), po.maxpool_fwd(ref)))
     assert not ops.sync_arena.timed_out(dev)
+
+
+@pytest.mark.parametrize("n", [1, 5, 80])
+def test_quantiser_clears_the_steps_words(dev, n):
+    """The quantiser's launch that begins a step leaves the exchange words zero and the batch as it is without."""
+    from niti_amd import ops
+    x = torch.randn((n, 3, 32, 32), device=dev)
+    want = ops.quantize_input(x)
+    for _ in range(3):
+        got = ops.quantize_input(x, start_step=True)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        words = ops.sync_arena.take(4096, x.device)
+        rest = ops.sync_arena.take(61440, x.device)
+        assert not words.any() and not rest.any()
+        words.fill_(7)
+        rest.fill_(7)
+        ops.sync_arena.reset(x.device)
