@@ -709,7 +709,18 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
     constexpr int LPP = NWF * 2;       // lanes (16-byte pieces) per pixel
     constexpr int PPI = 64 / LPP;      // pixels per store instruction
     const int prow = lane / LPP, piece = lane % LPP;
-    const int ch = chbase + piece * 16;
+    // With the max-pool's backward pass folded in, the two wavefronts that share pixels exchange halves of their patches: each
+    // then writes the windows of 32 pixels at the tile's full width.  At its own width a wavefront wrote every line of the
+    // four times larger result in pieces of 32 (64) bytes, and the lines left the cache half written (16 x 16 -> 32 x 32, 128
+    // channels, 256 images: 46.9 us, 24.7 of them without the folded pass).
+    constexpr bool kPairs = !G::TWO && KT != 32;
+    const bool pairs = kPairs && a.unpool != nullptr;
+    constexpr int LPU = KT / 16, PPU = 64 / LPU;
+    const int mfirst = pairs ? pixbase + wp_ * 64 + wc * 32 + lane / LPU : pixwave + prow;
+    const int mstep = pairs ? PPU : PPI;
+    const int ch = pairs ? kt * KT + lane % LPU * 16 : chbase + piece * 16;
+    const int8_t* const from = pairs ? smem + (wp_ + 4 * (lane % LPU / (KT / 32))) * (32 * PT * PROW) + (wc * 32 + lane / LPU) * PROW + lane % LPU % (KT / 32) * 16
+                                     : patch + prow * PROW + piece * 16;
     if (rt) {   // once, in place: the values are rounded up to twice below
 #pragma unroll
       for (int i = 0; i < NWF; ++i)
@@ -730,14 +741,14 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
     v4i mkpre[MKD];
     auto mask_request = [&](int t) {
       const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.mask), 0, a.y8_bytes, 0x00020000);
-      const int m = pixwave + t * PPI + prow;
+      const int m = mfirst + t * mstep;
       const int off = (m < total_pix && ch < a.K) ? m * a.K + ch : kOob;
       mkpre[t % MKD] = __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0);
     };
     // the same for the pooling windows of the folded max-pool backward, one piece ahead
     v4i xwpre[kMaskAhead ? 4 : 1];
     auto window_offsets = [&](int t, int (&wo)[4]) {
-      const int m = pixwave + t * PPI + prow;
+      const int m = mfirst + t * mstep;
       const bool in = m < total_pix && ch < a.K;
       const int n = m / (Q * Q), rem = m - n * (Q * Q);
       const int pp = rem / Q, pq = rem - pp * Q;
@@ -812,11 +823,11 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
       if (fast) round_tiles(std::true_type{});
       else round_tiles(std::false_type{});
       // same wavefront reads back what it wrote: LDS operations of one wavefront complete in order
+      if (pairs) __syncthreads();
 #pragma unroll
       for (int t = 0; t < 32 * PT / PPI; ++t) {
-        const int pl = t * PPI + prow;
-        v4i v = *reinterpret_cast<const v4i*>(patch + pl * PROW + piece * 16);
-        const int m = pixwave + pl;
+        v4i v = *reinterpret_cast<const v4i*>(from + t * mstep * PROW);
+        const int m = mfirst + t * mstep;
         const int off = (m < total_pix && ch < a.K) ? m * a.K + ch : kOob;
         v4i mk;
         if (a.mask != nullptr) {  // ReLU backward of the layer below, folded in: its output is this layer's input
@@ -1217,8 +1228,7 @@ int compute_units() {
   return cus;
 }
 
-// Channel tile of a launch: 128 unless that leaves fewer workgroups than the device runs at once while
-// a tile of 64 would give it more to do.
+// Channel tile of a launch: 128 unless that leaves compute units idle to which narrower tiles would give something to do.
 int halo_ktile(long long pix, int K, int H, int C) {
   const long long ptiles = (pix + 255) / 256;
   const int cus = compute_units();
@@ -1226,17 +1236,17 @@ int halo_ktile(long long pix, int K, int H, int C) {
   const int forced = e != nullptr ? atoi(e) : 0;
   if (forced == 128 || forced == 64) return forced;
   if (forced == 32 && H <= 16) return 32;
-  // fewer 64-channel tiles than compute units on the small maps: tiles of 32 channels, twice as many workgroups
-  if (forced == 0 && H <= 8 && K > 32 && ptiles * ((K + 63) / 64) < cus) return 32;
-  // exactly one 64-channel tile per compute unit and a short reduction: two 32-channel workgroups per unit overlap
-  // each other's fill and epilogue (measured per launch: 128 -> 256 at 16 x 16 data gradient 14.5 -> 13.9 us, 256 -> 512
-  // at 8 x 8 forward 13.9 -> 12.7 us; with 512 input channels the narrower tile's longer loop loses more than that)
-  if (forced == 0 && H <= 16 && K > 32 && C <= 256 && ptiles * ((K + 63) / 64) == cus) return 32;
+  // one 32-channel tile per compute unit at most: twice as many workgroups as with 64 channels, each half as long (24 images of
+  // 16 x 16, 256 -> 256: 12.3 -> 9.3 us, 60 of 8 x 8, 512 -> 512: 18.8 -> 16.6).  Two of them on a unit are slower than one
+  // 64-channel tile (50 images of the former 16.7 / 12.8 us, 120 of the latter 27.8 / 22.6).
+  if (forced == 0 && H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
   if (K <= 64) return 64;   // nothing to gain from computing 128 channels
   // one slice of reduction (the first layer): the launch is all output stores, and the 64-channel tile's workgroups -
   // 512 pixels each where 256-pixel ones would not all fit - spread them better (3 -> 128 at 32 x 32: 9.9 -> 9.5 us)
   if (forced == 0 && C <= 32 && H == 32 && pix % 512 == 0) return 64;
   const long long b128 = ptiles * ((K + 127) / 128);
+  // (One 128-channel tile per unit beats two of 64 channels by 7% on operands that lie in the caches, and loses 10 to 25% inside a
+  // training step, where the second workgroup hides the trips to memory.)
   return (b128 < 2LL * cus && K > 64) ? 64 : 128;
 }
 
