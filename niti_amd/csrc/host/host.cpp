@@ -269,19 +269,20 @@ PyObject* quantize_input(PyObject*, PyObject* const* args, Py_ssize_t n) {
     at::Tensor parts = scratch(256 * sizeof(int32_t), x);
     uint32_t* zero = nullptr;
     int zero_words = 0;
-    if (a.flag()) {   // a step begins: its first launch clears the sync words
-      Arena& arena = arena_now(x);
-      arena_restart(arena);
-      if (arena.chunks.empty()) arena.chunks.push_back(empty32({kChunkWords}, x));
-      zero = ptr<uint32_t>(arena.chunks[0]);
-      zero_words = static_cast<int>(arena.chunks[0].numel());
+    Arena* const arena = a.flag() ? &arena_now(x) : nullptr;
+    if (arena != nullptr) {   // a step begins: its first launch clears the sync words
+      arena_restart(*arena);
+      arena->cleared = false;
+      if (arena->chunks.empty()) arena->chunks.push_back(empty32({kChunkWords}, x));
+      zero = ptr<uint32_t>(arena->chunks[0]);
+      zero_words = static_cast<int>(arena->chunks[0].numel());
       if (zero_words > kChunkWords) zero = nullptr, zero_words = 0;   // an unusually long one: left to its own fill
-      arena.cleared = zero != nullptr;
     }
     check(niti_quantize_batch_zero_f32_i8(ptr<float>(x), ptr<int8_t>(y), static_cast<int>(N), static_cast<int>(C), static_cast<int>(H),
                                      static_cast<int>(W), static_cast<int>(cpad), bits, ptr<uint32_t>(parts), ptr<int32_t>(e),
                                      ptr<int64_t>(target), ptr<int64_t>(target_out), static_cast<int>(targets), zero, zero_words, stream_of(x)),
           "niti_quantize_batch_f32_i8");
+    if (arena != nullptr) arena->cleared = zero != nullptr;   // behind the check: a refused call has launched nothing
     return tuple_of({y, e});
   });
 }

@@ -1464,3 +1464,17 @@ def test_quantiser_clears_the_steps_words(dev, n):
         words.fill_(7)
         rest.fill_(7)
         ops.sync_arena.reset(x.device)
+
+
+def test_refused_quantiser_leaves_the_words_to_a_fill(dev):
+    """A quantiser call that the library refuses has cleared nothing: words taken behind it, without a call that begins a step
+    in between, are zero all the same."""
+    from niti_amd import ops
+    x = torch.randn((3, 3, 8, 8), device=dev)
+    for bad, bits in ((x[:0], 7), (x, 0), (x, 8)):
+        ops.sync_arena.reset(x.device)
+        ops.sync_arena.take(65536, x.device).fill_(7)
+        with pytest.raises(RuntimeError):
+            ops.quantize_input(bad, bits, start_step=True)
+        assert not ops.sync_arena.take(65536, x.device).any(), (tuple(bad.shape), bits)
+    ops.sync_arena.reset(x.device)
