@@ -165,18 +165,21 @@ constexpr unsigned long long kTopkFirst = 0x1231300031112230ULL;
 // Per sample: cross entropy of softmax(v 2^e) (main.py:156-157), whether the target is the first and whether it is among
 // the five largest (meters.py:56-70); added up and folded into sums[3] = {loss, top-1 %, top-5 %} x samples.  One workgroup:
 // the work is a few kilobytes, the tensor-library sequence it replaces is 22 launches (85 us of a 540 us step).
+// A target of -100 is left out of the loss's mean and hits nothing, as in F.cross_entropy's default (no sample left: NaN).  Any
+// other target outside the classes, which F.cross_entropy refuses, makes all three sums NaN.
+constexpr long long kIgnoredTarget = -100;
 __global__ __launch_bounds__(1024) void batch_metrics_kernel(const int8_t* __restrict__ out, const int32_t* __restrict__ out_exp,
                                                              const int64_t* __restrict__ target, int n, int classes, double* sums) {
-  __shared__ double red[3][16];
+  __shared__ double red[5][16];
   __shared__ int8_t stage[kMetricsStage];   // the logits of up to 1024 samples: each is looked at twice, one after the other
   const float scale = ldexpf(1.0f, *out_exp);
-  double loss = 0.0, hit1 = 0.0, hit5 = 0.0;
+  double loss = 0.0, hit1 = 0.0, hit5 = 0.0, counted = 0.0, outside = 0.0;
   const bool staged = classes <= kMetricsStage / 64;
   const int rows = staged && kMetricsStage / classes < 1024 ? kMetricsStage / classes : 1024;
   for (int base = 0; base < n; base += rows) {
     const int8_t* src = out + static_cast<long long>(base) * classes;
     const int here = n - base < rows ? n - base : rows;
-    const long long t = static_cast<int>(threadIdx.x) < here ? target[base + threadIdx.x] : -1;
+    const long long t = static_cast<int>(threadIdx.x) < here ? target[base + threadIdx.x] : kIgnoredTarget;
     if (staged) {
       __syncthreads();
       for (int i = threadIdx.x; i < here * classes; i += 1024) stage[i] = src[i];
@@ -216,21 +219,29 @@ __global__ __launch_bounds__(1024) void batch_metrics_kernel(const int8_t* __res
       loss += static_cast<double>(logf(sum) - (static_cast<float>(v[t]) * scale - fmx));
       hit1 += tpos == static_cast<int>((kTopkFirst >> (4 * pattern)) & 15u) ? 1.0 : 0.0;
       hit5 += tpos >= 0 ? 1.0 : 0.0;
+      counted += 1.0;
+    } else if (t != kIgnoredTarget) {
+      outside += 1.0;
     }
   }
-  double part[3] = {loss, hit1, hit5};
+  double part[5] = {loss, hit1, hit5, counted, outside};
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
+  for (int k = 0; k < 5; ++k) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) part[k] += __shfl_xor(part[k], off, 64);
     if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = part[k];
   }
   __syncthreads();
   if (threadIdx.x < 3) {
-    double s = 0.0;
-    for (int i = 0; i < 16; ++i) s += red[threadIdx.x][i];
+    double s = 0.0, valid = 0.0, bad = 0.0;
+    for (int i = 0; i < 16; ++i) {
+      s += red[threadIdx.x][i];
+      valid += red[3][i];
+      bad += red[4][i];
+    }
     // the mean over the batch as a float32 value, times the batch size in double: the order of the tensor operations
-    const float mean = threadIdx.x == 0 ? static_cast<float>(s / n) : static_cast<float>(s) * (100.0f / static_cast<float>(n));
+    float mean = threadIdx.x == 0 ? static_cast<float>(s / valid) : static_cast<float>(s) * (100.0f / static_cast<float>(n));
+    if (bad > 0.0) mean = __builtin_nanf("");
     sums[threadIdx.x] += static_cast<double>(mean) * n;
   }
 }

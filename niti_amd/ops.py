@@ -304,7 +304,8 @@ def quantize_input(x, bits=7, cpad=16, out=None, exp_out=None, target=None, targ
 
 def batch_metrics(out_val, out_exp, target, sums):
     """sums (float64 [3]) += batch size x (display loss, top-1 %, top-5 %) of int8 logits [n, classes >= 5] with exponent
-    ``out_exp`` (1-element int32 device tensor), in one launch."""
+    ``out_exp`` (1-element int32 device tensor), in one launch.  Targets of -100 are left out of the loss's mean and hit
+    nothing; any other target outside the classes makes all three sums NaN."""
     _chk_dev(out_val, out_exp, target, sums)
     n, classes = out_val.shape
     if (out_val.dtype != torch.int8 or out_exp.dtype != torch.int32 or target.dtype != torch.int64 or target.numel() != n

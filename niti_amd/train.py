@@ -48,13 +48,22 @@ def _add_metrics(output, output_exp, target, sums):
     network, the same as tensor operations for anything else."""
     if (output.is_cuda and output.dtype == torch.int8 and output.dim() == 2 and output.size(0) > 0 and output.size(1) >= 5
             and output.is_contiguous() and isinstance(output_exp, torch.Tensor) and output_exp.dtype == torch.int32
-            and output_exp.numel() == 1 and output_exp.is_cuda and target.dtype == torch.int64 and target.is_contiguous()):
+            and output_exp.numel() == 1 and output_exp.is_cuda and target.dtype == torch.int64 and target.is_contiguous()
+            and target.is_cuda and tuple(target.shape) == (output.size(0),)
+            and sums.dtype == torch.float64 and sums.is_cuda and sums.is_contiguous() and tuple(sums.shape) == (3,)):
         ops.batch_metrics(output, output_exp.reshape(1), target, sums)
         return
     scale = torch.exp2(torch.as_tensor(output_exp, device=output.device).float().reshape(()))
     loss = F.cross_entropy(output.float() * scale, target)
     prec1, prec5 = accuracy(output.detach(), target, topk=(1, 5))
     sums += torch.stack([loss.double(), prec1.double(), prec5.double()]) * target.size(0)
+
+
+def _check_targets(sums):
+    """Raises where a class index outside the logits' classes reached ``_add_metrics``: F.cross_entropy refuses such a target
+    (-100, which it ignores, aside), the launch that stands in for it leaves NaN in every sum."""
+    if sums[1] != sums[1]:
+        raise IndexError("target out of bounds: a batch of this pass holds class indices outside the network's classes")
 
 
 def _one_step(model, training, inputs, target, sums):
@@ -163,6 +172,7 @@ def run_epoch(data_loader, model, training, log_interval=0, epoch=0, use_graph=F
         count += inputs.size(0)
         if training and log_interval and i % log_interval == 0:
             s = (sums / count).tolist()
+            _check_targets(s)
             logging.info('[%d][%3d] loss %.3f @1 %.3f', epoch, i, s[0], s[1])
         # A shared device makes every grid-wide wait run into its limit and every step round with wrong shifts: find out
         # after the first steps and whenever the host reads the device anyway, not at the end of a pass that looked hung
@@ -170,8 +180,9 @@ def run_epoch(data_loader, model, training, log_interval=0, epoch=0, use_graph=F
             check_waits(dev)
     if count == 0:
         return 0.0, 0.0, 0.0
-    loss_avg, top1, top5 = (sums / count).tolist()
+    loss_avg, top1, top5 = s = (sums / count).tolist()
     check_waits(dev)
+    _check_targets(s)
     return loss_avg, top1, top5
 
 

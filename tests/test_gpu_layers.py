@@ -551,3 +551,52 @@ def test_batch_metrics(tt, n, classes):
         prec1, prec5 = train.accuracy(out, target, topk=(1, 5))
         ref = torch.stack([loss.double(), prec1.double(), prec5.double()]) * n + 7.0
         assert torch.allclose(sums, ref, rtol=1e-6, atol=1e-6), (hi, e, sums.tolist(), ref.tolist())
+
+
+def test_batch_metrics_targets_outside_the_classes(tt):
+    """Targets of -100 leave the mean of the loss, as in F.cross_entropy (none left: NaN); a target that F.cross_entropy refuses
+    makes every sum NaN, and a pass over such a batch raises."""
+    from niti_amd import ops, train
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(5)
+    exp = torch.tensor([-3], dtype=torch.int32, device=dev)
+    for n, ignored in ((1, 0), (37, 5), (1100, 700), (8, 8)):
+        out = ri8(g, n, 10).to(dev)
+        target = torch.randint(0, 10, (n,), generator=g)
+        target[:ignored] = -100
+        target = target.to(dev)
+        sums = torch.zeros(3, dtype=torch.float64, device=dev)
+        ops.batch_metrics(out, exp, target, sums)
+        loss = torch.nn.functional.cross_entropy(out.float() * 2.0 ** -3, target)
+        prec1, prec5 = train.accuracy(out, target, topk=(1, 5))
+        ref = torch.stack([loss.double(), prec1.double(), prec5.double()]) * n
+        assert torch.allclose(sums, ref, rtol=1e-6, atol=1e-6, equal_nan=True), (n, sums.tolist(), ref.tolist())
+        assert bool(sums[0].isnan()) == (ignored == n)
+    out = ri8(g, 6, 10).to(dev)
+    for bad in (-1, 10, -101, 1 << 40):
+        target = torch.tensor([1, 2, bad, 4, -100, 5], device=dev)
+        sums = torch.zeros(3, dtype=torch.float64, device=dev)
+        ops.batch_metrics(out, exp, target, sums)
+        assert bool(sums.isnan().all()), (bad, sums.tolist())
+        with pytest.raises(IndexError):
+            train.run_epoch([(out, target)], lambda x, t: (x, exp), False)
+    assert train.run_epoch([(out, target.clamp(0, 9))], lambda x, t: (x, exp), False)[2] >= 0.0
+
+
+def test_metrics_take_what_the_tensor_operations_take(tt):
+    """Sums and targets that the one-launch form does not take go through the tensor operations: float32 sums are added to,
+    targets of another shape than one index per sample are refused by the loss."""
+    from niti_amd import train
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(6)
+    out, exp = ri8(g, 50, 10).to(dev), torch.tensor([-4], dtype=torch.int32, device=dev)
+    target = torch.randint(0, 10, (50,), generator=g).to(dev)
+    want = torch.zeros(3, dtype=torch.float64, device=dev)
+    train._add_metrics(out, exp, target, want)
+    got = torch.zeros(3, dtype=torch.float32, device=dev)
+    train._add_metrics(out, exp, target, got)
+    assert torch.allclose(got.double(), want, rtol=1e-6)
+    with pytest.raises((RuntimeError, ValueError)):
+        train._add_metrics(out, exp, target.view(50, 1), want)
+    with pytest.raises((RuntimeError, ValueError)):
+        train._add_metrics(out, exp, target[:49], want)
