@@ -376,7 +376,7 @@ int niti_quantize_batch_zero_f32_i8(const float* x, int8_t* y, int N, int C, int
 
 /* Display metrics of a step (main.py:156-163, meters.py:56-70) in one launch: sums[0..2] (double) += n x { mean cross entropy of
    softmax(out_val 2^out_exp), top-1 %, top-5 % }.  out_val: [n,classes] int8, target: int64 [n], classes >= 5.  Ties count as
-   torch.topk orders them.  A target of -100 is left out of the loss's mean and hits nothing; any other target outside the
+   torch.topk (2.10) orders them up to 1000 classes.  A target of -100 is left out of the loss's mean and hits nothing; any other target outside the
    classes makes the three sums NaN. */
 int niti_batch_metrics_i8(const int8_t* out_val, const int32_t* out_exp, const int64_t* target, int n, int classes, double* sums,
                           void* stream);

@@ -43,10 +43,16 @@ def apply_regime(regime, epoch):
             break
 
 
+# Which of several equal logits torch.topk lists first is defined nowhere.  ops.batch_metrics reproduces what this release does for
+# up to this many classes (a single row of 10000 already comes out in another order); anything else asks torch.topk.
+TOPK_RELEASE, TOPK_CLASSES = "2.10.", 1000
+
+
 def _add_metrics(output, output_exp, target, sums):
     """Adds batch size x (display loss, top-1, top-5) to ``sums`` (main.py:156-163): one launch for the integer logits of a
     network, the same as tensor operations for anything else."""
-    if (output.is_cuda and output.dtype == torch.int8 and output.dim() == 2 and output.size(0) > 0 and output.size(1) >= 5
+    if (output.is_cuda and output.dtype == torch.int8 and output.dim() == 2 and output.size(0) > 0 and 5 <= output.size(1) <= TOPK_CLASSES
+            and torch.__version__.startswith(TOPK_RELEASE)
             and output.is_contiguous() and isinstance(output_exp, torch.Tensor) and output_exp.dtype == torch.int32
             and output_exp.numel() == 1 and output_exp.is_cuda and target.dtype == torch.int64 and target.is_contiguous()
             and target.is_cuda and tuple(target.shape) == (output.size(0),)

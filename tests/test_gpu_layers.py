@@ -600,3 +600,25 @@ def test_metrics_take_what_the_tensor_operations_take(tt):
         train._add_metrics(out, exp, target.view(50, 1), want)
     with pytest.raises((RuntimeError, ValueError)):
         train._add_metrics(out, exp, target[:49], want)
+
+
+@pytest.mark.parametrize("classes", [5, 6, 7, 10, 11, 32, 33, 100, 257, 512, 1000, 1001, 10000])
+def test_metrics_order_ties_as_topk_does(tt, monkeypatch, classes):
+    """Each of the five entries torch.topk lists as the target, few distinct logits: the hit is counted where torch.topk has it,
+    also for class counts and torch releases that the one-launch form does not cover."""
+    from niti_amd import train
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(classes)
+    exp = torch.tensor([0], dtype=torch.int32, device=dev)
+    for release in (train.TOPK_RELEASE, "0."):
+        monkeypatch.setattr(train, "TOPK_RELEASE", release)
+        for n in (1, 15, 30, 60, 300, 3000):
+            if n * classes > 3000000:
+                continue
+            for hi in (0, 1, 2):
+                out = torch.randint(-hi, hi + 1, (n, classes), generator=g, dtype=torch.int8).to(dev)
+                listed = out.topk(5, 1, True, True)[1]
+                for k in range(5):
+                    sums = torch.zeros(3, dtype=torch.float64, device=dev)
+                    train._add_metrics(out, exp, listed[:, k].contiguous(), sums)
+                    assert abs(float(sums[1]) / n - (100.0 if k == 0 else 0.0)) < 1e-3 and abs(float(sums[2]) / n - 100.0) < 1e-3, (n, hi, k)
