@@ -9,10 +9,20 @@ from . import ops, ti_torch
 from .ti_loss import TiLoss
 
 
+_MODULE_CALL = Module.__call__      # as defined: torch.fx replaces it while it traces
+
+
 def _plain(module):
-    """Whether calling ``module`` is calling its forward method: no hooks, nothing compiled or traced in between."""
-    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-                or module._compiled_call_impl is not None)
+    """Whether calling ``module`` is calling its forward method: no call of its own, no hooks, nothing compiled or traced in
+    between."""
+    return type(module).__call__ is _MODULE_CALL and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+        or module._compiled_call_impl is not None)
+
+
+def own_quantiser(model):
+    """Whether ``model`` quantises its input itself: a subclass's method, one set on the object, or a replacement of TiNet's."""
+    return model.quantize_input is not _QUANTIZE_INPUT
 
 
 class TiNet(Module):
@@ -79,10 +89,10 @@ class TiNet(Module):
         """ti_net.py:17-23: float NCHW batch -> (int8 logits, exponent).  ``target`` (not in the reference): the
         class indices that backward() will be called with; the classifier's forward launch then computes the loss
         gradient as well and backward(target) with the same tensor starts from it."""
-        if type(self).quantize_input is TiNet.quantize_input:
-            x_data, x_exp = self._quantize(x, True)
-        else:
+        if own_quantiser(self):
             x_data, x_exp = self.quantize_input(x)
+        else:
+            x_data, x_exp = self._quantize(x, True)
         return self.forward_int8(x_data, x_exp, target)
 
     @staticmethod
@@ -111,7 +121,8 @@ class TiNet(Module):
                 self._head.next_target = (target, loss_rand)
         d = self.__dict__       # plain attributes: Module.__setattr__ looks for parameters first
         layers, x = self.forward_layers, (x_data, x_exp)
-        if type(layers) is torch.nn.Sequential and _plain(layers) and not _module._has_any_global_hook() and torch._C._get_tracing_state() is None:
+        if (type(layers) is torch.nn.Sequential and _plain(layers) and "forward" not in layers.__dict__ and not _module._has_any_global_hook()
+                and torch._C._get_tracing_state() is None):
             # the container's loop without Module.__call__'s checks per layer (a third of an evaluation step's host time)
             for layer in layers._modules.values():
                 x = layer.forward(x) if _plain(layer) else layer(x)
@@ -165,3 +176,6 @@ class TiNet(Module):
                 prefix = "layers." + str(idx) + "."
                 l.weight = state_dict[prefix + "weight"].to(ti_torch.GPU).contiguous()
                 l.weight_exp = state_dict[prefix + "weight_exp"]
+
+
+_QUANTIZE_INPUT = TiNet.quantize_input

@@ -21,7 +21,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ops, ti_torch
-from .ti_net import TiNet
+from .ti_net import own_quantiser
 from .ti_vgg import TiVGG_cifar
 
 
@@ -92,8 +92,7 @@ class StepGraph:
         self.model, self.training = model, training
         x_data, _ = model.quantize_input(inputs)
         self.x8 = torch.empty_like(x_data)                                               # quantised batch, NHWC
-        # the library's quantiser can write it: the network has no quantiser of its own, and the layout is that one's
-        self.direct = type(model).quantize_input is TiNet.quantize_input and x_data.dim() == 4 and x_data.shape[3] % 16 == 0
+        self.direct = x_data.dim() == 4 and x_data.shape[3] % 16 == 0      # the library's quantiser can write it: the layout is that one's
         self.x_exp = torch.empty(1, dtype=torch.int32, device=inputs.device)
         self.target = torch.empty_like(target)
         self.graph, self.failed, self.eager_left = None, False, eager_steps
@@ -106,7 +105,7 @@ class StepGraph:
             self.model.backward(self.target)
 
     def __call__(self, inputs, target, sums):
-        if (self.direct and inputs.is_cuda and inputs.dtype == torch.float32 and inputs.is_contiguous() and ti_torch.BW_MODE == "int"
+        if (self.direct and not own_quantiser(self.model) and inputs.is_cuda and inputs.dtype == torch.float32 and inputs.is_contiguous() and ti_torch.BW_MODE == "int"
                 and target.is_cuda and target.dtype == torch.int64 and target.is_contiguous()):
             # ti_net.py:17-19 straight into the step's own buffers
             ops.quantize_input(inputs, ti_torch.BITWIDTH, out=self.x8, exp_out=self.x_exp, target=target, target_out=self.target)

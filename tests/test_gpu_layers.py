@@ -622,3 +622,32 @@ def test_metrics_order_ties_as_topk_does(tt, monkeypatch, classes):
                     sums = torch.zeros(3, dtype=torch.float64, device=dev)
                     train._add_metrics(out, exp, listed[:, k].contiguous(), sums)
                     assert abs(float(sums[1]) / n - (100.0 if k == 0 else 0.0)) < 1e-3 and abs(float(sums[2]) / n - 100.0) < 1e-3, (n, hi, k)
+
+
+def test_step_runner_asks_an_overridden_quantiser(tt):
+    """StepGraph quantises with what the network says at each call, eager or replayed, also where that changed behind its
+    construction."""
+    from niti_amd import train
+    from niti_amd.ti_net import TiNet
+    from niti_amd.ti_vgg import TiVGG_cifar
+    dev = torch.device("cuda:0")
+    torch.manual_seed(8)
+    tt.TRAINING = False
+    model = TiVGG_cifar(depth=7)
+    x, target = torch.randn(8, 3, 32, 32, device=dev), torch.zeros(8, dtype=torch.int64, device=dev)
+    sums = torch.zeros(3, dtype=torch.float64, device=dev)
+    runner = train.StepGraph(model, False, x, target, eager_steps=1)
+    for calls in range(3):
+        runner(x, target, sums)
+    assert runner.graph is not None
+    asked = []
+    model.quantize_input = lambda batch: asked.append(1) or TiNet.quantize_input(-batch)
+    runner(x, target, sums)
+    got = model.out.clone()
+    runner = train.StepGraph(model, False, x, target, eager_steps=1)
+    for calls in range(3):
+        runner(x, target, sums)
+        assert torch.equal(model.out, got)
+    assert len(asked) == 1 + 1 + 3       # the replay, the runner's construction, its three steps
+    del model.quantize_input
+    assert torch.equal(model(-x)[0], got)

@@ -3,7 +3,7 @@ import os
 
 import torch
 
-from niti_amd import ti_torch, train
+from niti_amd import ops, ti_net, ti_torch, train
 
 
 def test_accuracy_known_answers():
@@ -90,3 +90,57 @@ def test_quantisers_follow_bw_mode():
         assert float(ti_torch._ceil_log2(torch.tensor(16.0))) == 4.0 and float(ti_torch._ceil_log2(torch.tensor(17.0))) == 5.0
     finally:
         ti_torch.BW_MODE = old
+
+
+class _Add(torch.nn.Module):
+    """A layer of the networks below: adds to the activations."""
+
+    def __init__(self, n):
+        super().__init__()
+        self.n = n
+
+    def forward(self, x):
+        return x[0] + self.n, x[1]
+
+
+class _Counted(_Add):
+    """... with a call of its own around forward."""
+
+    def __call__(self, x):
+        return super().__call__((x[0] * 10, x[1]))
+
+
+def _net(*layers):
+    net = ti_net.TiNet()
+    net.forward_layers = torch.nn.Sequential(*layers)
+    return net
+
+
+def test_overrides_on_objects_are_called(monkeypatch):
+    """What a program replaces on a network, its container or a layer is what runs: a quantiser set on the object, a subclass's or
+    one that takes TiNet's place, a forward set on the container or a layer, a layer class with a call of its own, hooks."""
+    monkeypatch.setattr(ops.sync_arena, "reset", lambda device: None, raising=False)
+    monkeypatch.setattr(ti_net.TiNet, "_quantize", staticmethod(lambda x, start_step: (x, 0)))
+    x = torch.ones(2)
+    run = lambda net: float(net(x)[0][0])
+    assert run(_net(_Add(1), _Add(2))) == 4.0
+    net = _net(_Add(1))
+    net.quantize_input = lambda t: (t * 5, 0)
+    assert run(net) == 6.0 and ti_net.own_quantiser(net)
+    own = type("Own", (ti_net.TiNet,), {"quantize_input": staticmethod(lambda t: (t * 7, 0))})()
+    own.forward_layers = torch.nn.Sequential(_Add(1))
+    assert run(own) == 8.0 and ti_net.own_quantiser(own)
+    with monkeypatch.context() as m:
+        m.setattr(ti_net.TiNet, "quantize_input", staticmethod(lambda t: (t * 3, 0)))
+        assert run(_net(_Add(1))) == 4.0
+    assert not ti_net.own_quantiser(_net())
+    assert run(_net(_Add(1), _Counted(2))) == 22.0
+    net = _net(_Add(1), _Add(2))
+    net.forward_layers.forward = lambda x: (x[0] * 100, x[1])
+    assert run(net) == 100.0
+    net = _net(_Add(1), _Add(2))
+    net.forward_layers[1].forward = lambda x: (x[0] * 100, x[1])
+    assert run(net) == 200.0
+    net = _net(_Add(1), _Add(2))
+    net.forward_layers[0].register_forward_hook(lambda mod, args, out: (out[0] * 10, out[1]))
+    assert run(net) == 22.0
