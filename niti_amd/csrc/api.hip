@@ -545,6 +545,18 @@ extern "C" int niti_conv2d_i8_dgrad_requant_unpool(const int8_t* err, const int8
                       workspace_bytes, stream, nullptr, pool_in, ties);
 }
 
+// bytes of both operands re-laid with the batch index fast (the general weight gradient's workspace)
+static size_t wgrad_copies(int N, int H, int W, int C, int K, int P, int Q) {
+  const size_t np = static_cast<size_t>(round16(N));
+  return round256(static_cast<size_t>(C) * H * W * np) + round256(static_cast<size_t>(K) * P * Q * np);
+}
+// Batches of the 3x3 maps that are no whole bands of 128 (4 x 4 and 2 x 2 maps: 256) pixels also take operands that do not start
+// on 16-byte boundaries: those are re-laid.
+static bool wgrad_ragged(int N, int H) {
+  const long long pix = static_cast<long long>(N) * H * H;
+  return pix % (H <= 4 ? 256 : 128) != 0;
+}
+
 extern "C" size_t niti_conv2d_i8_wgrad_workspace(int N, int H, int W, int C, int K, int R, int S, int pad) {
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || pad < 0) return 0;
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
@@ -552,10 +564,10 @@ extern "C" size_t niti_conv2d_i8_wgrad_workspace(int N, int H, int W, int C, int
   if (wgrad3x3_supported(N, H, W, C, K, R, S, 1, pad)) {
     const size_t own = wgrad3x3_workspace(N, H, C, K);
     const size_t any = wgrad3x3_prefers_any(N, H, C, K) ? conv_any_wgrad_workspace({N, H, W, C, K, R, S, 1, pad}) : 0;
-    return round256(any > own ? any : own);
+    const size_t fast = round256(any > own ? any : own), copies = wgrad_ragged(N, H) ? wgrad_copies(N, H, W, C, K, P, Q) : 0;
+    return fast > copies ? fast : copies;
   }
-  const size_t np = static_cast<size_t>(round16(N));
-  const size_t copies = round256(static_cast<size_t>(C) * H * W * np) + round256(static_cast<size_t>(K) * P * Q * np);
+  const size_t copies = wgrad_copies(N, H, W, C, K, P, Q);
   const size_t slices = round256(conv_any_wgrad_workspace({N, H, W, C, K, R, S, 1, pad}));
   return slices > copies ? slices : copies;
 }
@@ -573,14 +585,14 @@ extern "C" int niti_conv2d_i8_wgrad(const int8_t* act, const int8_t* err, int32_
   if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))
     return fail(NITI_ERR_WORKSPACE, "conv_wgrad: needs %zu workspace bytes (16-byte aligned), got %zu", need, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad)) {
-    if (!aligned16(act) || !aligned16(err) || !aligned16(dw))
-      return fail(NITI_ERR_INVALID_ARG, "conv_wgrad: pointers must be 16-byte aligned");
+  const bool aligned = aligned16(act) && aligned16(err) && aligned16(dw);
+  if (wgrad3x3_supported(N, H, W, C, K, R, S, stride, pad) && (aligned || !wgrad_ragged(N, H))) {
+    if (!aligned) return fail(NITI_ERR_INVALID_ARG, "conv_wgrad: pointers must be 16-byte aligned");
     return launch_wgrad3x3(act, err, dw, N, H, C, K, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
   }
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
   const ConvShape shape{N, H, W, C, K, R, S, stride, pad};
-  if (conv_any_shape(kConvWgrad, shape) && aligned16(act) && aligned16(err) && aligned16(dw))
+  if (conv_any_shape(kConvWgrad, shape) && aligned)
     return launch_conv_any_wgrad(shape, act, err, dw, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
   const int np = round16(N);
   int8_t* act_t = static_cast<int8_t*>(workspace);                                 // [C][H*W][np]

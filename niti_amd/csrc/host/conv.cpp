@@ -43,6 +43,7 @@ Rounding rounding_of(Args& a) {
 }
 
 bool is_i8(const at::Tensor& t) { return t.scalar_type() == at::kChar; }
+bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
 // ---- int32 results -----------------------------------------------------------------------------------------------
 at::Tensor fprop_i32(const at::Tensor& x, const at::Tensor& w, int stride, int pad, unsigned flags, uint32_t* absmax, Opt prepared) {
@@ -462,7 +463,8 @@ struct WeightGradient {
 // one-call form the int32 gradient (its zero-padded channels dropped) is rounded and applied in a second step and returned.
 bool weight_gradient(bool fuse, const at::Tensor& act, const at::Tensor& err, const at::Tensor& w, int stride, int pad, const WeightGradient& g, Update* u,
                      const at::Tensor& e) {
-  const bool one = fuse && wgrad_update_fused(act, err, w, stride, pad, g.flags | NITI_CONV_ANY_KERNEL | (g.shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), g.r,
+  // the one-call kernels load 16 bytes at a time; operands that start elsewhere are re-laid by the int32 gradient
+  const bool one = fuse && aligned16(act) && aligned16(err) && wgrad_update_fused(act, err, w, stride, pad, g.flags | NITI_CONV_ANY_KERNEL | (g.shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), g.r,
                                               g.want_grad, g.want_dw, nullptr, g.shift, g.exp_a, g.exp_b, ptr<int32_t>(e), nullptr, g.prepared, true, u, nullptr);
   if (one) {
     if (g.want_dw && u->dw.size(3) != w.size(3)) u->dw = u->dw.slice(3, 0, w.size(3)).contiguous();
@@ -489,7 +491,7 @@ bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tens
   if (f.stride != 1 || g.want_dw || g.rand != nullptr || g.r.method == NITI_ROUND_STOCHASTIC || act.size(3) != w.size(3)) return false;
   if (!is_i8(act) || !is_i8(err) || !is_i8(w)) return false;
   for (Opt t : {&act, &err, &w, f.mask, f.rand, pool_in, g.prepared})
-    if (t != nullptr && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
+    if (t != nullptr && !aligned16(*t)) return false;
   const Dims d = gradient_dims(err, w, f.pad, "conv layer");
   if (!has_shape(act, {d.N, d.H, d.W, d.C}) || d.R != d.S) return false;
   const bool sto = f.r.method == NITI_ROUND_STOCHASTIC;

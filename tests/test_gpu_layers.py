@@ -651,3 +651,34 @@ def test_step_runner_asks_an_overridden_quantiser(tt):
     assert len(asked) == 1 + 1 + 3       # the replay, the runner's construction, its three steps
     del model.quantize_input
     assert torch.equal(model(-x)[0], got)
+
+
+# (N, H, W, C, K, filter, padding): an odd batch of the 3x3 maps, the first layer's three channels, other maps and filters
+@pytest.mark.parametrize("case", [(3, 8, 8, 16, 32, 3, 1), (5, 8, 8, 3, 48, 3, 1), (7, 4, 4, 32, 16, 3, 1), (5, 2, 2, 16, 16, 3, 1), (2, 7, 9, 48, 32, 3, 1),
+                                  (3, 10, 6, 3, 16, 5, 2), (2, 6, 6, 32, 10, 3, 0)])
+def test_first_layer_takes_errors_that_start_anywhere(tt, case):
+    """The first layer's weight gradient and update from an error map (contiguous) that does not start on a 16-byte boundary."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    dev = torch.device("cuda:0")
+    N, H, W, C, K, R, pad = case
+    _say("unaligned errors", case)
+    g = torch.Generator().manual_seed(600 + N + C + K)
+    x, w = ri8(g, N, H, W, C), ri8(g, K, R, R, C)
+    e = ri8(g, N, H + 2 * pad - R + 1, W + 2 * pad - R + 1, K, lo=-40, hi=40)
+    padded = torch.nn.functional.pad(x, (0, -C % 16))
+    acc = co.conv_wgrad(padded, e, R, R, 1, pad)
+    g8, _ = po.grad_calc(acc[..., :C].contiguous(), 5, "psto")
+    for offset in (0, 1, 4):
+        flat = torch.zeros(e.numel() + 16, dtype=torch.int8, device=dev)
+        err = flat[offset:offset + e.numel()].view(e.shape)
+        err.copy_(e)
+        assert err.is_contiguous() and err.data_ptr() % 16 == offset
+        layer = tt.TiConv2d(C, K, kernel_size=R, padding=pad, first_layer=True)
+        layer.weight = w.to(dev)
+        layer.forward((x.to(dev), 0))
+        layer.backward((err, -4))
+        assert torch.equal(layer.weight.cpu(), po.weight_update(w, g8)), offset
+        am = ops.new_scalar_u32(dev)
+        assert torch.equal(ops.conv2d_wgrad(padded.to(dev), err, R, R, 1, pad, absmax=am).cpu(), acc) and int(am.cpu()) == po.absmax(acc), offset
