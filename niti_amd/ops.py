@@ -38,15 +38,25 @@ def _flags(f32_epilogue: bool) -> int:
     return L.EPI_F32_ROUNDTRIP if f32_epilogue else 0
 
 
-def conv_filter_prepare(w, N, H, W, stride=1, padding=1, dgrad=False):
-    """Kernel-ready copy of the [K,R,S,C] filter for a convolution over an [N,H,W,*] input (forward) or
-    the data gradient of one (dgrad=True).  Returns None when the kernels read the filter as stored."""
-    _chk_dev(w)
+def conv_filter_bytes(w, N, H, W, stride=1, padding=1, dgrad=False) -> int:
+    """Bytes of conv_filter_prepare's copy, 0 when the kernels read the filter as stored.  The forward copy's layout depends on
+    the filter alone: one copy serves every [N,H,W] for which this is not 0."""
     K, R, S, C = w.shape
-    nbytes = L.lib().niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, padding, int(dgrad))
+    return L.lib().niti_conv2d_i8_filter_workspace(N, H, W, C, K, R, S, stride, padding, int(dgrad))
+
+
+def conv_filter_prepare(w, N, H, W, stride=1, padding=1, dgrad=False, out=None):
+    """Kernel-ready copy of the [K,R,S,C] filter for a convolution over an [N,H,W,*] input (forward) or
+    the data gradient of one (dgrad=True).  Returns None when the kernels read the filter as stored.  ``out``: int8 tensor of
+    conv_filter_bytes bytes to write instead of a new one."""
+    _chk_dev(w, out)
+    K, R, S, C = w.shape
+    nbytes = conv_filter_bytes(w, N, H, W, stride, padding, dgrad)
     if nbytes == 0:
         return None
-    dst = torch.empty(nbytes, dtype=torch.int8, device=w.device)
+    if out is not None and (out.dtype != torch.int8 or out.numel() != nbytes or out.device != w.device):
+        raise RuntimeError("conv_filter_prepare: out must be an int8 tensor of %d bytes next to the filter" % nbytes)
+    dst = torch.empty(nbytes, dtype=torch.int8, device=w.device) if out is None else out
     st = L.lib().niti_conv2d_i8_filter_prepare(_ptr(w), _ptr(dst), nbytes, N, H, W, C, K, R, S, stride, padding,
                                                int(dgrad), _stream(w))
     L.check(st, "niti_conv2d_i8_filter_prepare")

@@ -348,7 +348,10 @@ class UpdateWeight(Module):
         self.grad, self.grad_shift = ops.grad_update(
             g, self.weight, absmax, GRAD_BITWIDTH, method, DIV_MODE, BW_MODE, rand, want_grad=self.keep_grad,
             exp_a=_exp_tensor(self.err_exp, g.device), exp_b=_exp_tensor(self.act_in_exp, g.device), exp_out=self.grad_exp)
-        self._wprep_key = None      # any kernel-ready copy of the old weights is stale now
+        self._weights_changed()
+
+    def _weights_changed(self):
+        """The weights have been updated by a call that kept no copy of them in step."""
 
 
 class TiConv2d(UpdateWeight):
@@ -385,10 +388,7 @@ class TiConv2d(UpdateWeight):
             shape_only = fresh and d.get("_wprep") is not None and d.get("_w16_kept") is not None
             w16 = d["_w16_kept"] = self._w16_kept if shape_only else _pad_channels16(weight).contiguous()
         if not fresh:
-            # kernel-ready copy of the filter: made when the weight tensor was replaced or modified through torch; the
-            # fused weight update keeps it in step with its own changes
-            N, H, W, _ = act16.shape
-            d["_wprep"] = ops.conv_filter_prepare(w16, N, H, W, self.stride, self.padding)
+            d["_wprep"] = self._filter_copy(w16, act16.shape)
             d["_wprep_key"] = key
         method = _method_code(ACT_ROUND_METHOD)
         if method == _STO:
@@ -454,10 +454,41 @@ class TiConv2d(UpdateWeight):
                 _exp_tensor(d["act_in_exp"], dev), prepared, grad_rand)
             if unpooled:
                 pool.__dict__["bwd_done"] = err_out
-        if not one:
-            d["_wprep_key"] = None      # any kernel-ready copy of the old weights is stale now
+        if not one or prepared is not d.get("_wprep_kept"):
+            self._weights_changed()
         if not self.first_layer:
             return err_out, d["err_exp"]
+
+    def _filter_copy(self, w16, shape):
+        """Kernel-ready copy of the filter for activations of ``shape``, None where the kernels read it as stored.  The layer keeps
+        one buffer, whatever batches and maps come along: captured steps hold its address.  It is written here when the weight
+        tensor was replaced or modified through torch; the one-call update keeps it in step with its own changes, and
+        _weights_changed follows every other update."""
+        d, (N, H, W, _), weight = self.__dict__, shape, self.weight
+        nbytes = ops.conv_filter_bytes(w16, N, H, W, self.stride, self.padding)
+        if nbytes == 0:
+            return None
+        kept = d.get("_wprep_kept")
+        if kept is None or kept.numel() != nbytes or kept.device != w16.device:
+            kept = d["_wprep_kept"] = torch.empty(nbytes, dtype=torch.int8, device=w16.device)
+            d["_wprep_of"] = None
+        made_of = (weight.data_ptr(), weight._version)
+        if d["_wprep_of"] != made_of:
+            ops.conv_filter_prepare(w16, N, H, W, self.stride, self.padding, out=kept)
+            d["_wprep_of"], d["_wprep_for"] = made_of, (N, H, W)
+        return kept
+
+    def _weights_changed(self):
+        d = self.__dict__
+        kept = d.get("_wprep_kept")
+        if kept is None:
+            return
+        w16 = _pad_channels16(self.weight).contiguous()
+        if w16.device != kept.device or ops.conv_filter_bytes(w16, *d["_wprep_for"], self.stride, self.padding) != kept.numel():
+            d["_wprep_kept"] = d["_wprep_key"] = None      # another filter has taken the place of the one it was made for
+            return
+        ops.conv_filter_prepare(w16, *d["_wprep_for"], self.stride, self.padding, out=kept)
+        d["_wprep_of"] = (self.weight.data_ptr(), self.weight._version)
 
     def _shift_state(self, which, device):
         """1-element int32 device tensor that keeps the requantisation shift of this layer's activations ("act") or

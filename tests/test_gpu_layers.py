@@ -682,3 +682,76 @@ def test_first_layer_takes_errors_that_start_anywhere(tt, case):
         assert torch.equal(layer.weight.cpu(), po.weight_update(w, g8)), offset
         am = ops.new_scalar_u32(dev)
         assert torch.equal(ops.conv2d_wgrad(padded.to(dev), err, R, R, 1, pad, absmax=am).cpu(), acc) and int(am.cpu()) == po.absmax(acc), offset
+
+
+def test_captures_that_follow_each_other(tt):
+    """Three graphs captured in turn (the later ones on the stream handles and words of the earlier): each replays to its own
+    results, several times, with eager layers between the replays."""
+    import gc
+    from niti_amd import ops
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(9)
+    conv, linear = tt.TiConv2d(32, 48), tt.TiLinear(48 * 64, 72)
+
+    def step(x):
+        ops.sync_arena.reset(dev)
+        y, e = conv.forward((x, 0))
+        return [y, e, *linear.forward((y.view(y.shape[0], -1), e))]
+    batches = [ri8(g, n, 8, 8, 32).to(dev) for n in (4, 7, 4)]
+    want = [[t.clone() for t in step(x)] for x in batches]
+    graphs, outs = [], []
+    gc.collect()
+    gc.disable()         # a collection may free tensors, which a capturing process may not
+    try:
+        for x in batches:
+            step(x)      # the filter copy for this batch's shape is made outside the graph
+            torch.cuda.synchronize()
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1]):
+                outs.append(step(x))
+    finally:
+        gc.enable()
+    for turn in range(4):
+        for k in (0, 1, 2) if turn % 2 == 0 else (2, 1, 0):
+            for t in outs[k]:
+                t.zero_()
+            graphs[k].replay()
+            eager = step(batches[(k + turn) % 3])
+            torch.cuda.synchronize()
+            assert all(torch.equal(p, q) for p, q in zip(outs[k], want[k])), (turn, k)
+            assert all(torch.equal(p, q) for p, q in zip(eager, want[(k + turn) % 3])), (turn, k)
+    assert not ops.sync_timeouts(dev)
+
+
+@pytest.mark.parametrize("sto", [False, True])
+def test_replays_behind_other_batches(tt, sto):
+    """Passes whose last batch is smaller, training and evaluation: the captured steps of the whole batches are replayed behind
+    eager steps of other shapes and end where the same passes issued launch by launch end (also with gradients rounded in
+    a second call, which keeps no filter copy in step)."""
+    from niti_amd import train
+    from niti_amd.ti_vgg import TiVGG_cifar
+    _say("replays behind other batches", sto)
+    g = torch.Generator().manual_seed(41)
+    x, y = torch.randn(6 * 32 + 21, 3, 32, 32, generator=g), torch.randint(0, 10, (6 * 32 + 21,), generator=g)
+    tt.GRAD_ROUND_METHOD = tt.StoShift if sto else tt.PstoShift
+
+    def passes(use_graph):
+        torch.manual_seed(42)
+        torch.cuda.manual_seed(42)
+        model = TiVGG_cifar(depth=7)
+        model.regime = [{'epoch': 0, 'gb': 5}]
+        hist = train.fit(model, train.TensorLoader(x, y, 32), train.TensorLoader(x[:6 * 32 - 5], y[:6 * 32 - 5], 32), epochs=3, use_graph=use_graph)
+        return model, hist
+    model, hist = passes(True)
+    whole = [r for k, r in model.__dict__["_step_graphs"].items() if k[1][0] == 32]
+    assert len(whole) == 2 and all(r.graph is not None and not r.failed for r in whole)
+    twin, hist2 = passes(False)
+    if sto:     # the random integers of the rounding come from torch's generator, which a capture advances otherwise
+        for layer in model.forward_layers:
+            if isinstance(layer, tt.TiConv2d) and layer.__dict__.get("_wprep_kept") is not None:
+                w16 = tt._pad_channels16(layer.weight).contiguous()
+                assert torch.equal(layer._wprep_kept, tt.ops.conv_filter_prepare(w16, *layer._wprep_for))
+        return
+    assert hist2 == hist
+    for a, b in zip(model.state_dict().values(), twin.state_dict().values()):
+        assert torch.equal(a, b)
