@@ -475,7 +475,8 @@ class TiConv2d(UpdateWeight):
         made_of = (weight.data_ptr(), weight._version)
         if d["_wprep_of"] != made_of:
             ops.conv_filter_prepare(w16, N, H, W, self.stride, self.padding, out=kept)
-            d["_wprep_of"], d["_wprep_for"] = made_of, (N, H, W)
+            # the alias keeps the weights' memory from being given to another tensor, which their address would not tell apart
+            d["_wprep_of"], d["_wprep_for"], d["_wprep_weight"] = made_of, (N, H, W), weight.detach()
         return kept
 
     def _weights_changed(self):
@@ -488,7 +489,7 @@ class TiConv2d(UpdateWeight):
             d["_wprep_kept"] = d["_wprep_key"] = None      # another filter has taken the place of the one it was made for
             return
         ops.conv_filter_prepare(w16, *d["_wprep_for"], self.stride, self.padding, out=kept)
-        d["_wprep_of"] = (self.weight.data_ptr(), self.weight._version)
+        d["_wprep_of"], d["_wprep_weight"] = (self.weight.data_ptr(), self.weight._version), self.weight.detach()
 
     def _shift_state(self, which, device):
         """1-element int32 device tensor that keeps the requantisation shift of this layer's activations ("act") or

@@ -755,3 +755,21 @@ def test_replays_behind_other_batches(tt, sto):
     assert hist2 == hist
     for a, b in zip(model.state_dict().values(), twin.state_dict().values()):
         assert torch.equal(a, b)
+
+
+def test_conv_layer_sees_weights_at_an_address_it_knew(tt):
+    """Weights replaced several times between two forward passes: the allocator hands out addresses again, the filter copy must
+    not be taken for one of them."""
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(15)
+    layer = tt.TiConv2d(32, 48)
+    x = ri8(g, 4, 8, 8, 32)
+    for _ in range(4):
+        for _ in range(3):
+            layer.weight = None
+            w = ri8(g, 48, 3, 3, 32)
+            layer.weight = w.to(dev)
+        y, _ = layer.forward((x.to(dev), 0))
+        assert torch.equal(y.cpu(), po.act_calc(co.conv_fprop(x, w, 1, 1), 0)[0])
