@@ -160,7 +160,8 @@ def scratch(nbytes: int, device) -> torch.Tensor:
     """One grow-only int8 buffer per stream for kernel workspaces that live only inside a call.  Calls on one
     stream run in order, so they can all use the same memory - which also keeps the partial sums of
     consecutive weight-gradient launches in the same cache-resident region instead of walking through fresh
-    allocations.  Under graph capture: memory of the graph."""
+    allocations.  Under graph capture: memory of the graph.  The buffers of the sixteen streams used last are kept.  A buffer for
+    each stream does not make it safe to run layers on several streams at once: see _SyncArena."""
     return L.host().scratch(nbytes, _index(device))
 
 
@@ -172,7 +173,12 @@ class _SyncArena:
     chunk it uses.  Slices are handed out once per reset, so a kernel never sees words another kernel of the
     same step wrote.  An arena that runs out (or was never reset) grows by another chunk; ``timed_out`` covers every
     slice handed out since the last reset.  Every stream, and every stream capture, has an arena of its own
-    (csrc/host/host.cpp); reset and take work on the current stream's."""
+    (csrc/host/host.cpp; those of the sixteen streams used last are kept); reset and take work on the current stream's.
+
+    Not for several streams at once: a launch that exchanges its range waits for all of its workgroups, so it must have the
+    device to itself.  Two such launches that run side by side can each hold compute units that the other's workgroups wait
+    for; both then give up at the wait limit (2 s) with wrong shifts, which ``timed_out`` and ``sync_timeouts`` report.
+    Streams that take turns (an event or wait_stream between them) are fine."""
 
     def reset(self, device):
         L.host().arena_reset(_index(device))

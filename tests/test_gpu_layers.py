@@ -773,3 +773,36 @@ def test_conv_layer_sees_weights_at_an_address_it_knew(tt):
             layer.weight = w.to(dev)
         y, _ = layer.forward((x.to(dev), 0))
         assert torch.equal(y.cpu(), po.act_calc(co.conv_fprop(x, w, 1, 1), 0)[0])
+
+
+def _layers_once(tt, dev, seed):
+    """A convolution and a linear layer, forward and backward on fresh weights: every result."""
+    g = torch.Generator().manual_seed(seed)
+    x, e, w = ri8(g, 6, 8, 8, 32).to(dev), ri8(g, 6, 8, 8, 48, lo=-40, hi=40).to(dev), ri8(g, 48, 3, 3, 32).to(dev)
+    a, f, v = ri8(g, 20, 200).to(dev), ri8(g, 20, 72, lo=-40, hi=40).to(dev), ri8(g, 72, 200).to(dev)
+    conv, linear = tt.TiConv2d(32, 48), tt.TiLinear(200, 72)
+    conv.weight, conv.weight_exp, linear.weight, linear.weight_exp = w, torch.tensor(-7.0), v, torch.tensor(-7.0)
+    return [*conv.forward((x, 0)), *conv.backward((e, -4)), conv.weight, *linear.forward((a, 0)), *linear.backward((f, -4)), linear.weight]
+
+
+def test_streams_one_after_another(tt):
+    """More streams than the front end keeps words and scratch memory for, each waiting for the one before, with and without a
+    step's reset: the same results on each, and again on the first ones, whose memory has been given back."""
+    from niti_amd import ops
+    dev = torch.device("cuda:0")
+    want = [_layers_once(tt, dev, s) for s in (1, 2)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    assert len({s.cuda_stream for s in streams}) > 16
+    last, got = torch.cuda.current_stream(), []
+    for i, s in enumerate(streams + streams[:6]):
+        s.wait_stream(last)
+        with torch.cuda.stream(s):
+            if i % 3 == 0:
+                ops.sync_arena.reset(dev)
+            got.append((i, _layers_once(tt, dev, 1 + i % 2)))
+        last = s
+    torch.cuda.synchronize()
+    for i, results in got:
+        assert all(torch.equal(p, q) for p, q in zip(results, want[i % 2])), i
+    assert not ops.sync_timeouts(dev)
