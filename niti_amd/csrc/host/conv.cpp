@@ -30,6 +30,12 @@ Dims gradient_dims(const at::Tensor& err, const at::Tensor& w, int pad, const ch
               static_cast<int>(w.size(3)), static_cast<int>(w.size(0)), R, S};
 }
 
+// a kernel-ready filter copy that a launch reads (or, forward, keeps in step)
+void want_copy(Opt prepared, const Dims& d, int stride, int pad, int dgrad, const char* who) {
+  if (prepared == nullptr) return;
+  want_bytes(*prepared, static_cast<int64_t>(niti_conv2d_i8_filter_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, stride, pad, dgrad)), who, "a prepared filter");
+}
+
 struct Rounding {
   int bits, method, div, bw;
 };
@@ -54,6 +60,7 @@ at::Tensor fprop_i32(const at::Tensor& x, const at::Tensor& w, int stride, int p
   at::Tensor ws;
   size_t bytes = 0;
   const int8_t* wp = prepared != nullptr ? ptr<int8_t>(*prepared) : ptr<int8_t>(w);
+  want_copy(prepared, d, stride, pad, 0, who);
   if (prepared != nullptr) {
     flags |= NITI_CONV_FILTER_PREPARED;
   } else {
@@ -70,6 +77,7 @@ at::Tensor fprop_i32(const at::Tensor& x, const at::Tensor& w, int stride, int p
 at::Tensor dgrad_i32(const at::Tensor& err, const at::Tensor& w, int stride, int pad, unsigned flags, uint32_t* absmax, Opt prepared,
                      bool forward_copy) {
   const Dims d = gradient_dims(err, w, pad, "conv2d_dgrad");
+  want_copy(prepared, d, stride, pad, forward_copy ? 0 : 1, "conv2d_dgrad");
   if (d.H < 0 || d.W < 0) refuse("conv2d_dgrad: filter larger than the padded input");
   at::Tensor dx = empty32({d.N, d.H, d.W, d.C}, err);
   at::Tensor ws;
@@ -92,6 +100,7 @@ at::Tensor wgrad_i32(const at::Tensor& act, const at::Tensor& err, int R, int S,
   if (act.dim() != 4 || err.dim() != 4) refuse("conv2d_wgrad: [N,H,W,C] and [N,P,Q,K] tensors expected");
   const int N = static_cast<int>(act.size(0)), H = static_cast<int>(act.size(1)), W = static_cast<int>(act.size(2)),
             C = static_cast<int>(act.size(3)), K = static_cast<int>(err.size(3));
+  want_bytes(err, static_cast<int64_t>(N) * out_extent(H, R, 1, pad) * out_extent(W, S, 1, pad) * K, "conv2d_wgrad", "an error map");
   const size_t bytes = niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, pad);
   at::Tensor ws = workspace != nullptr ? *workspace : scratch(bytes, act);
   if (static_cast<size_t>(ws.numel()) < bytes)
@@ -219,6 +228,7 @@ bool conv_requant(const at::Tensor& x, const at::Tensor& w, const Dims& d, const
   if (small > 0) {
     // nothing to prepare
   } else if (f.prepared != nullptr) {
+    want_copy(f.prepared, d, f.stride, f.pad, f.dgrad && !f.forward_copy ? 1 : 0, who);
     flags |= NITI_CONV_FILTER_PREPARED | (f.forward_copy ? NITI_CONV_FILTER_FORWARD_COPY : 0u);
     wp = ptr<int8_t>(*f.prepared);
   } else {
@@ -413,6 +423,7 @@ bool wgrad_update_fused(const at::Tensor& act, const at::Tensor& err, const at::
     refuse_niti("conv2d_wgrad_update: shape not covered by the single-pass path");
   }
   if (!has_shape(err, {N, out_extent(H, R, 1, pad), out_extent(W, S, 1, pad), K})) refuse("conv2d_wgrad_update: error map does not match the activations");
+  want_copy(prepared, Dims{N, H, W, C, K, R, S}, stride, pad, 0, "conv2d_wgrad_update");
   size_t have = 0;
   uint32_t* sp = sync_words(sync, words, act, sync_view, &have, "conv2d_wgrad_update");
   const size_t bytes = niti_conv2d_i8_wgrad_workspace(N, H, W, C, K, R, S, pad);
@@ -504,6 +515,7 @@ bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tens
   }
   const size_t words = niti_conv2d_i8_backward_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
   if (words == 0) return false;
+  want_copy(g.prepared, d, 1, f.pad, 0, "conv layer");
   const size_t bytes = niti_conv2d_i8_backward_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
   at::Tensor ws;
   if (bytes > 0) ws = scratch(bytes, act);

@@ -139,6 +139,7 @@ at::Tensor gemm_out(const at::Tensor& a, const at::Tensor& b, bool ta, bool tb, 
   if (a.dim() != 2 || b.dim() != 2) refuse("gemm: matrices expected");
   const int64_t m = a.size(ta ? 1 : 0), k = a.size(ta ? 0 : 1), n = b.size(tb ? 0 : 1), k2 = b.size(tb ? 1 : 0);
   if (k != k2) refuse("gemm: inner extents differ (" + std::to_string(k) + " vs " + std::to_string(k2) + ")");
+  if (out != nullptr) want_bytes(*out, 4 * m * n, "gemm", "an int32 result");
   at::Tensor c = out != nullptr ? *out : empty32({m, n}, a);
   const size_t bytes = niti_gemm_i8_workspace(ta, tb, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
   at::Tensor ws;
@@ -203,6 +204,12 @@ PyObject* absmax_i32(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---- pooling -----------------------------------------------------------------------------------------------------
+int64_t pooled_side(int64_t v, int ks, int stride, int pad) {
+  const int64_t t = v + 2 * pad - ks;   // rounded down like Python's //
+  const int64_t q = stride > 0 ? (t >= 0 ? t / stride : -((-t + stride - 1) / stride)) + 1 : 0;
+  return q > 0 ? q : 0;
+}
+
 // maxpool_fwd(x, kernel, stride, padding) -> y
 PyObject* maxpool_fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
@@ -212,12 +219,7 @@ PyObject* maxpool_fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     want_i8(x, "maxpool_fwd");
     if (x.dim() != 4) refuse("maxpool_fwd: [N,H,W,C] tensor expected");
     const int64_t N = x.size(0), H = x.size(1), W = x.size(2), C = x.size(3);
-    auto side = [&](int64_t v) {
-      const int64_t t = v + 2 * pad - ks;   // rounded down like Python's //
-      const int64_t q = stride > 0 ? (t >= 0 ? t / stride : -((-t + stride - 1) / stride)) + 1 : 0;
-      return q > 0 ? q : 0;
-    };
-    at::Tensor y = empty8({N, side(H), side(W), C}, x);
+    at::Tensor y = empty8({N, pooled_side(H, ks, stride, pad), pooled_side(W, ks, stride, pad), C}, x);
     check(niti_maxpool_i8_fwd(ptr<int8_t>(x), ptr<int8_t>(y), static_cast<int>(N), static_cast<int>(H), static_cast<int>(W),
                               static_cast<int>(C), ks, stride, pad, stream_of(x)),
           "niti_maxpool_i8_fwd");
@@ -234,6 +236,9 @@ PyObject* maxpool_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const at::Tensor& x = a.tensor();
     const int ks = a.i(), stride = a.i(), pad = a.i(), ties = a.i();
     if (x.dim() != 4) refuse("maxpool_bwd: [N,H,W,C] tensor expected");
+    const int64_t pooled = x.size(0) * pooled_side(x.size(1), ks, stride, pad) * pooled_side(x.size(2), ks, stride, pad) * x.size(3);
+    want_bytes(y, pooled, "maxpool_bwd", "a pooled map");
+    want_bytes(dy, pooled, "maxpool_bwd", "an error map");
     at::Tensor dx = empty(x.sizes(), x.scalar_type(), x);
     check(niti_maxpool_i8_bwd(ptr<int8_t>(y), ptr<int8_t>(dy), ptr<int8_t>(x), ptr<int8_t>(dx), static_cast<int>(x.size(0)),
                               static_cast<int>(x.size(1)), static_cast<int>(x.size(2)), static_cast<int>(x.size(3)), ks, stride, pad, ties,

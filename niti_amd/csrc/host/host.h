@@ -98,6 +98,11 @@ at::Tensor scalar32(const at::Tensor& like);
 inline void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 inline bool has_shape(const at::Tensor& t, at::IntArrayRef shape) { return t.sizes() == shape; }
+// a launch reads or writes `bytes` of t: a tensor of other extents than the rest of the call's must not be smaller
+inline void want_bytes(const at::Tensor& t, int64_t bytes, const char* who, const char* what) {
+  if (static_cast<int64_t>(t.nbytes()) < bytes)
+    refuse(std::string(who) + ": " + what + " of " + std::to_string(bytes) + " bytes expected, got " + std::to_string(t.nbytes()));
+}
 inline void want_i8(const at::Tensor& t, const char* who) {
   if (t.scalar_type() != at::kChar) refuse(std::string(who) + ": int8 tensor expected");
 }

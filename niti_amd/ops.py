@@ -297,8 +297,15 @@ def grad_update(g, w, absmax, mu, method="psto", div_mode="floor", bw_mode="int"
     return g8, shift_out
 
 
+def _chk_bytes(t, nbytes, who):
+    """A launch reads ``nbytes`` of ``t``."""
+    if t.numel() * t.element_size() < nbytes:
+        raise RuntimeError("%s: a tensor of %d bytes expected, got %d" % (who, nbytes, t.numel() * t.element_size()))
+
+
 def weight_update(w, g):
     _chk_dev(w, g)
+    _chk_bytes(g, w.numel(), "weight_update")
     st = L.lib().niti_weight_update_i8(_ptr(w), _ptr(g), w.numel(), _stream(w))
     L.check(st, "niti_weight_update_i8")
     return w
@@ -346,6 +353,7 @@ def mask_features(x, mask, exp_in=None, exp_add=None):
 
 def relu_bwd(act, dy):
     _chk_dev(act, dy)
+    _chk_bytes(act, dy.numel(), "relu_bwd")
     dx = torch.empty_like(dy)
     L.check(L.lib().niti_relu_i8_bwd(_ptr(act), _ptr(dy), _ptr(dx), dy.numel(), _stream(dy)), "niti_relu_i8_bwd")
     return dx
@@ -447,6 +455,12 @@ def _linear_sync(which, M, O, F, sync, device, who):
     return sync
 
 
+def _chk_linear(rows, inner, w, who):
+    """Rows [M,features] against weights [O,F] along whose dimension ``inner`` they are multiplied."""
+    if rows.dim() != 2 or w.dim() != 2 or rows.shape[1] != w.shape[inner]:
+        raise RuntimeError("%s: rows %s do not go with weights %s" % (who, tuple(rows.shape), tuple(w.shape)))
+
+
 def _chk_rand(rand, shape, who):
     if rand is not None and (rand.dtype != torch.int32 or tuple(rand.shape) != tuple(shape) or not rand.is_contiguous()):
         raise RuntimeError("%s: rand must be a contiguous int32 tensor shaped like the output" % who)
@@ -457,6 +471,7 @@ def linear_fwd_requant(act, w, target_bits=7, method="round", div_mode="floor", 
     """act_calc(act @ w^T) in one launch for a layer of any width: act [M,F] int8, w [O,F] int8 -> ([M,O] int8, shift,
     sync).  ``rand`` (int32 [M,O]) for method "sto"."""
     _chk_dev(act, w, rand, sync, shift_out, exp_a, exp_b, exp_out)
+    _chk_linear(act, 1, w, "linear_fwd_requant")
     M, F = act.shape
     O = w.shape[0]
     _chk_rand(rand, (M, O), "linear_fwd_requant")
@@ -475,6 +490,7 @@ def linear_dgrad_requant(err, w, target_bits=7, method="round", div_mode="floor"
                          shift_out=None, exp_a=None, exp_b=None, exp_out=None):
     """err_calc(err @ w) in one launch: err [M,O] int8, w [O,F] int8 -> ([M,F] int8, shift, sync)."""
     _chk_dev(err, w, rand, sync, shift_out, exp_a, exp_b, exp_out)
+    _chk_linear(err, 0, w, "linear_dgrad_requant")
     M, O = err.shape
     F = w.shape[1]
     _chk_rand(rand, (M, F), "linear_dgrad_requant")
@@ -493,6 +509,10 @@ def linear_wgrad_update(err, act, w, mu=5, method="psto", div_mode="floor", bw_m
     """grad_calc(err^T @ act) and the weight update in one launch: err [M,O], act [M,F], w [O,F] int8 updated in place.
     Returns (int8 gradient or None, shift, sync)."""
     _chk_dev(err, act, w, rand, sync, shift_out, exp_a, exp_b, exp_out)
+    _chk_linear(err, 0, w, "linear_wgrad_update")
+    _chk_linear(act, 1, w, "linear_wgrad_update")
+    if act.shape[0] != err.shape[0]:
+        raise RuntimeError("linear_wgrad_update: %d errors for %d rows of activations" % (err.shape[0], act.shape[0]))
     M, O = err.shape
     F = act.shape[1]
     _chk_rand(rand, (O, F), "linear_wgrad_update")

@@ -1478,3 +1478,29 @@ def test_refused_quantiser_leaves_the_words_to_a_fill(dev):
             ops.quantize_input(bad, bits, start_step=True)
         assert not ops.sync_arena.take(65536, x.device).any(), (tuple(bad.shape), bits)
     ops.sync_arena.reset(x.device)
+
+
+def test_tensors_too_small_for_the_call_are_refused(dev):
+    """Operands whose extents do not go together raise before anything is launched."""
+    from niti_amd import ops
+    i8 = lambda *shape: torch.zeros(shape, dtype=torch.int8, device=dev)
+    x, w, e = i8(4, 8, 8, 32), i8(48, 3, 3, 32), i8(4, 8, 8, 48)
+    copy = ops.conv_filter_prepare(w, 4, 8, 8)
+    calls = [lambda: ops.gemm(i8(8, 16), i8(16, 8), out=torch.zeros(63, dtype=torch.int32, device=dev)),
+             lambda: ops.maxpool_bwd(i8(2, 4, 4, 16), i8(2, 4, 3, 16), i8(2, 8, 8, 16)),
+             lambda: ops.maxpool_bwd(i8(2, 4, 4, 8), i8(2, 4, 4, 16), i8(2, 8, 8, 16)),
+             lambda: ops.relu_bwd(i8(15), i8(16)),
+             lambda: ops.weight_update(i8(16), i8(15)),
+             lambda: ops.linear_fwd_requant(i8(8, 64), i8(32, 48)),
+             lambda: ops.linear_dgrad_requant(i8(8, 64), i8(32, 48)),
+             lambda: ops.linear_wgrad_update(i8(8, 32), i8(7, 48), i8(32, 48)),
+             lambda: ops.linear_wgrad_update(i8(8, 32), i8(8, 48), i8(32, 32)),
+             lambda: ops.conv2d_wgrad(x, e[:3], 3, 3), lambda: ops.conv2d_wgrad(x, e[:, :7].contiguous(), 3, 3),
+             lambda: ops.conv2d_fprop(x, w, prepared_filter=copy[:-16]), lambda: ops.conv2d_dgrad(e, w, forward_filter=copy[:-16]),
+             lambda: ops.conv2d_fprop_requant(x, w, prepared_filter=copy[:-16]),
+             lambda: ops.conv2d_wgrad_update(x, e, w, prepared_filter=copy[:-16]),
+             lambda: ops.conv2d_backward(e, x, w, prepared_filter=copy[:-16])]
+    for i, call in enumerate(calls):
+        with pytest.raises(RuntimeError):
+            call()
+            pytest.fail("call %d was taken" % i)
