@@ -15,9 +15,9 @@ _MODULE_CALL = Module.__call__      # as defined: torch.fx replaces it while it 
 def _plain(module):
     """Whether calling ``module`` is calling its forward method: no call of its own, no hooks, nothing compiled or traced in
     between."""
+    d = module.__dict__      # the hooks' dictionaries, without the attribute look-up on the class first
     return type(module).__call__ is _MODULE_CALL and not (
-        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-        or module._compiled_call_impl is not None)
+        d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or module._compiled_call_impl is not None)
 
 
 def own_quantiser(model):
@@ -123,9 +123,16 @@ class TiNet(Module):
         layers, x = self.forward_layers, (x_data, x_exp)
         if (type(layers) is torch.nn.Sequential and _plain(layers) and "forward" not in layers.__dict__ and not _module._has_any_global_hook()
                 and torch._C._get_tracing_state() is None):
-            # the container's loop without Module.__call__'s checks per layer (a third of an evaluation step's host time)
+            # the container's loop without Module.__call__'s checks per layer (a third of an evaluation step's host time); _plain
+            # written out, for its call takes as long as what it checks
             for layer in layers._modules.values():
-                x = layer.forward(x) if _plain(layer) else layer(x)
+                m = layer.__dict__
+                if type(layer).__call__ is _MODULE_CALL and not (
+                        m["_forward_hooks"] or m["_forward_pre_hooks"] or m["_backward_hooks"] or m["_backward_pre_hooks"]
+                        or layer._compiled_call_impl is not None):
+                    x = layer.forward(x)
+                else:
+                    x = layer(x)
         else:
             x = layers(x)
         d["out"], d["out_exp"] = x
