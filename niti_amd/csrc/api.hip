@@ -48,6 +48,17 @@ int fail(int status, const char* fmt, ...) {
 }
 void clear_error() { g_err[0] = 0; }
 
+int compute_units() {
+  static int of[kDeviceSlots] = {};
+  int& cus = of[device_slot()];
+  if (cus == 0) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      cus = 256;
+  }
+  return cus;
+}
+
 }  // namespace niti
 
 using namespace niti;
@@ -328,9 +339,9 @@ extern "C" size_t niti_conv2d_i8_fprop_small_sync_words(int N, int H, int W, int
   const char* e = getenv("NITI_FPROP_SMALL");   // 0 / 1 pins (tests)
   if (e != nullptr) return e[0] != '0' ? conv_any_requant_words(kConvForward, s) : 0;
   const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0, true);
-  if (nb == 0 || nb > 256) return 0;
-  const double us = conv_any_forward_us(s), stage = H >= 32 ? 1.25 : H == 16 ? 1.05 : 0.62;
-  return us > 0.0 && us < 0.9 * (3.5 + stage * ((C + 31) / 32)) ? conv_any_requant_words(kConvForward, s) : 0;
+  if (nb == 0 || nb > compute_units()) return 0;
+  const double us = conv_any_forward_us(s);
+  return us > 0.0 && us < 0.9 * conv3x3_halo_us(H, C) ? conv_any_requant_words(kConvForward, s) : 0;
 }
 
 static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_t* w, int8_t* y8, int N, int H, int W, int C,
@@ -677,10 +688,8 @@ static bool backward_together(const ConvShape& s) {
   if (e != nullptr) return e[0] != '0';
   const double us = conv_backward_us(s);
   if (us == 0.0) return false;
-  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad)) {
-    const double stage = s.H >= 32 ? 1.25 : s.H == 16 ? 1.05 : 0.62;
-    return us < 0.8 * (3.5 + stage * ((s.K + 31) / 32) + wgrad3x3_us(s.N, s.H, s.C, s.K));
-  }
+  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad))
+    return us < 0.8 * (conv3x3_halo_us(s.H, s.K) + wgrad3x3_us(s.N, s.H, s.C, s.K));
   const double d = conv_any_dgrad_us(s), w = conv_any_wgrad_us(s);
   return d == 0.0 || us < d + w;
 }
@@ -746,7 +755,7 @@ extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int
 
 extern "C" size_t niti_gemm_i8_workspace(int trans_a, int trans_b, int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  if (gemm_kmajor_shape(trans_a, trans_b, m, n, k) && gemm_any_shape(m, n, k)) return gemm_lines_workspace(trans_a, trans_b, m, n, k);   // read as stored; partial sums of a split reduction
+  if (gemm_in_place_shape(trans_a, trans_b, m, n, k) && gemm_any_shape(m, n, k)) return gemm_lines_workspace(trans_a, trans_b, m, n, k);   // read as stored; partial sums of a split reduction
   const size_t kp = static_cast<size_t>(round16(k));
   size_t bytes = 0;
   if (trans_a || k % 16 != 0) bytes += round256(static_cast<size_t>(m) * kp);
@@ -766,7 +775,7 @@ extern "C" int niti_gemm_i8(int trans_a, int trans_b, const int8_t* a, const int
     return fail(NITI_ERR_WORKSPACE, "gemm: needs %zu workspace bytes (16-byte aligned), got %zu", need, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // whole-line kernel: few, long rows of tiles (gemm_lines.hip says where it is the faster one)
-  if (gemm_lines_shape(trans_a, trans_b, m, n, k) && aligned16(a) && aligned16(b))
+  if (gemm_lines_shape(trans_a, trans_b, m, n, k) && aligned16(a) && aligned16(b) && workspace_bytes >= gemm_lines_workspace(trans_a, trans_b, m, n, k))
     return launch_gemm_lines(trans_b, a, b, c, m, n, k, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, absmax, workspace, s);
   // Operands with the reduction index fast in both and 16-byte rows are implicit-GEMM tiles as they stand; on results that
   // fill the chip that kernel's LDS-DMA ring is the faster one (4000 x 2000 x 8192 85 us against 97)

@@ -26,6 +26,9 @@ inline int device_slot() {
 }
 
 
+// compute units of the current device
+int compute_units();
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -195,7 +198,7 @@ int launch_conv_igemm(const ConvProblem& p, hipStream_t stream);
 
 // int32 GEMM of operands with a slow reduction index, staged as whole lines (gemm_lines.hip): NN (b as [k][n]) or TT (a as [k][m],
 // b as [n][k])
-bool gemm_kmajor_shape(int trans_a, int trans_b, int m, int n, int k);   // shapes read as stored since before gemm_any.hip: no copies in the workspace
+bool gemm_in_place_shape(int trans_a, int trans_b, int m, int n, int k);   // niti_gemm_i8_workspace counts no copies of the operands
 bool gemm_lines_shape(int trans_a, int trans_b, int m, int n, int k);
 size_t gemm_lines_workspace(int trans_a, int trans_b, int m, int n, int k);   // partial sums of a reduction split over workgroups
 int launch_gemm_lines(int trans_b, const int8_t* a, const int8_t* b, int32_t* c, int m, int n, int k, bool roundtrip, uint32_t* absmax,
@@ -220,6 +223,7 @@ int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, in
 // 3x3 / stride 1 / pad 1 forward kernel with LDS-resident activation halo (conv3x3_halo.hip)
 bool conv3x3_halo_supported(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 size_t conv3x3_halo_filter_bytes(int C, int K);
+double conv3x3_halo_us(int H, int C);   // estimated time with rounding of a launch of at most one workgroup per compute unit
 int launch_halo_filter_prepare(const int8_t* w, int8_t* dst, int kout, int cin, int mode, hipStream_t stream);
 int launch_conv3x3_halo(const int8_t* x, const int8_t* wp, int32_t* y, int N, int H, int C, int K, unsigned flags,
                         uint32_t* absmax, hipStream_t stream);
@@ -246,6 +250,9 @@ long long sync_spin_limit();
 // this device's word that every grid-wide wait sets when it gives up (api.hip); nullptr if it cannot be looked up
 uint32_t* timeout_word();
 int wgrad_finish_blocks(long long elements);
+// elements from one slice of partial sums to the next: the same element of consecutive slices falls into different memory channels
+// (a stride that is a multiple of 64 KB would put them all into one)
+inline long long slice_stride(long long elements) { return (elements + 1023) / 1024 * 1024 + 1088; }
 int wgrad3x3_finish_blocks(int C, int K);
 // partial sums in slices [K][R][S][C] -> int32 gradient, or -> rounded gradient -> updated weights (sync words: slots of
 // wgrad_finish_blocks workgroups)

@@ -109,10 +109,7 @@ struct Split {
   double us;               // estimated time
 };
 int chunk_of(int tile) { return tile == 0 ? TileS::BK : tile == 1 ? TileM::BK : TileL::BK; }
-long long slice_of(const ConvShape& s) {
-  const long long n = static_cast<long long>(s.K) * s.R * s.S * s.C;
-  return (n + 1023) / 1024 * 1024 + 1088;   // the same element of consecutive slices in different memory channels
-}
+long long slice_of(const ConvShape& s) { return slice_stride(static_cast<long long>(s.K) * s.R * s.S * s.C); }
 // The tile and the number of slices with the least estimated time.  A compute unit's time is its rounds of workgroups times
 // their chunks; a tile costs its prologue and epilogue, and cutting the reduction costs the finishing launch and the partial
 // sums' way through memory.  The constants are a least-squares fit (13% rms) to 46 layers, 0.1 to 23 GOP, each with every tile
@@ -122,22 +119,22 @@ Split estimate_split(const ConvShape& s) {
   constexpr double kFinish = 2.0, kMillionSums = 1.6;
   int m, n, k;
   product_of(kConvWgrad, s, &m, &n, &k);
-  const int pin = pinned_tile();
+  const int pin = pinned_tile(), cus = compute_units();
   const char* e = getenv("NITI_ANY_SLICES");   // pins the number of slices (tests, measurements)
   Split best{0, 0, 0, 0};
   for (int t = 0; t < 4; ++t) {
     if (pin >= 0 && t != pin) continue;
     const long long tiles = tiles_with(t, m, n);
     const int chunks = (k + chunk_of(t) - 1) / chunk_of(t);
-    for (int round = 0; round <= 4; ++round) {   // one workgroup per tile; 192, 256, 512, 768 workgroups
-      long long want = e != nullptr ? atoi(e) : round == 0 ? 1 : (round == 1 ? 192 : 256 * (round - 1)) / tiles;
+    for (int round = 0; round <= 4; ++round) {   // one workgroup per tile; as many as 3/4, 1, 2, 3 times the compute units
+      long long want = e != nullptr ? atoi(e) : round == 0 ? 1 : (round == 1 ? cus * 3 / 4 : cus * (round - 1)) / tiles;
       if (want < 1 || (want == 1 && round > 0 && e == nullptr)) continue;
       if (want > chunks) want = chunks;
       const int per = static_cast<int>((chunks + want - 1) / want), slices = (chunks + per - 1) / per;
       const double blocks = static_cast<double>(tiles) * slices;
-      const double rounds = blocks > 512 ? blocks / 256 : blocks > 256 ? 2 : 1;
+      const double rounds = blocks > 2 * cus ? blocks / cus : blocks > cus ? 2 : 1;
       double us = kTile[t] + rounds * per * kChunk[t] + (rounds - 1) * kRound[t];
-      if (slices > 1 || blocks > 512) us += kFinish + kMillionSums * 1e-6 * slices * static_cast<double>(m) * n;
+      if (slices > 1 || blocks > 2 * cus) us += kFinish + kMillionSums * 1e-6 * slices * static_cast<double>(m) * n;
       if (best.slices == 0 || us < best.us) best = Split{t, slices, per, us};
     }
   }
@@ -148,11 +145,11 @@ Split estimate_split(const ConvShape& s) {
 Split pick_split(const ConvShape& s) {
   if (getenv("NITI_ANY_TILE") != nullptr || getenv("NITI_ANY_SLICES") != nullptr) return estimate_split(s);
   struct Entry {
-    int key[6];
+    int key[7];
     Split split;
   };
   static thread_local Entry kept[16] = {};
-  const int key[6] = {s.N, s.H * 65536 + s.W, s.C, s.K, s.R * 65536 + s.S, s.pad};
+  const int key[7] = {s.N, s.H * 65536 + s.W, s.C, s.K, s.R * 65536 + s.S, s.pad, device_slot()};
   unsigned h = 0;
   for (int v : key) h = h * 31u + static_cast<unsigned>(v);
   Entry& e = kept[(h ^ (h >> 8)) & 15u];
@@ -209,7 +206,7 @@ double conv_any_forward_us(const ConvShape& s) {
   const int t = requant_tile(kConvForward, s);
   if (t > 1) return 1e9;   // the wide tiles: not for the few workgroups this is asked for
   const double chunks = t == 0 ? (k + TileS::BK - 1) / TileS::BK : (k + TileM::BK - 1) / TileM::BK;
-  return (t == 0 ? 4.9 + 0.42 * chunks : 5.6 + 0.58 * chunks) * (tiles_with(t, m, n) > 256 ? 1.5 : 1.0);
+  return (t == 0 ? 4.9 + 0.42 * chunks : 5.6 + 0.58 * chunks) * (tiles_with(t, m, n) > compute_units() ? 1.5 : 1.0);
 }
 
 double conv_any_dgrad_us(const ConvShape& s) {
@@ -218,7 +215,7 @@ double conv_any_dgrad_us(const ConvShape& s) {
   int m, n, k;
   product_of(kConvDgrad, s, &m, &n, &k);
   const int t = requant_tile(kConvDgrad, s), block = t == 0 ? TileS::BK : t == 1 ? TileM::BK : TileL::BK;
-  return 5.5 + (tiles_with(t, m, n) > 256 ? 1.5 : 1.0) * kChunk[t] * ((k + block - 1) / block);
+  return 5.5 + (tiles_with(t, m, n) > compute_units() ? 1.5 : 1.0) * kChunk[t] * ((k + block - 1) / block);
 }
 
 int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* x, const int8_t* w, int8_t* y, bool roundtrip, uint32_t* sync,

@@ -71,6 +71,7 @@ Plan estimate(const ConvShape& s) {
   const char* te = getenv("NITI_ANY_TILE");
   const char* se = getenv("NITI_ANY_SLICES");
   const int pin = te != nullptr && te[0] >= '0' && te[0] <= '3' ? te[0] - '0' : -1, pin_slices = se != nullptr ? atoi(se) : 0;
+  const int cus = compute_units();
   int dm, dn, dk, wm, wn, wk;
   product_of(kConvDgrad, s, &dm, &dn, &dk);
   product_of(kConvWgrad, s, &wm, &wn, &wk);
@@ -79,19 +80,19 @@ Plan estimate(const ConvShape& s) {
     if (pin >= 0 && td != (pin < 3 ? pin : 2)) continue;
     const long long nd = with_tile(td, [&](auto t) { return tiles_of<decltype(t)>(dm, dn); });
     const int cd = (dk + kBlock[td] - 1) / kBlock[td];
-    if (nd > 512) continue;
+    if (nd > 2 * cus) continue;
     for (int tw = 0; tw < 4; ++tw) {
       if (pin >= 0 && tw != pin) continue;
       const long long tiles = with_tile(tw, [&](auto t) { return tiles_of<decltype(t)>(wm, wn); });
       const int cw = (wk + kBlock[tw] - 1) / kBlock[tw];
-      for (int round = 0; round < 4; ++round) {   // whole; as many workgroups as the data gradient leaves of 256, 384, 512
-        long long want = pin_slices > 0 ? pin_slices : round == 0 ? 1 : (128 * (round + 1) - nd) / tiles;
+      for (int round = 0; round < 4; ++round) {   // whole; as many workgroups as the data gradient leaves of 1, 1.5, 2 per compute unit
+        long long want = pin_slices > 0 ? pin_slices : round == 0 ? 1 : (cus / 2 * (round + 1) - nd) / tiles;
         if (want < 1 || (want == 1 && round > 0 && pin_slices == 0)) continue;
         if (want > cw) want = cw;
         const int per = static_cast<int>((cw + want - 1) / want), slices = (cw + per - 1) / per;
         const long long nw = tiles * slices;
-        if (nd + nw > 512 || (slices > 1 && wgrad_finish_blocks(static_cast<long long>(wm) * wn) == 0)) continue;
-        const double chain_d = cd * kChunkD[td], chain_w = per * kChunkW[tw], all = (nd * chain_d + nw * chain_w) / 256;
+        if (nd + nw > 2 * cus || (slices > 1 && wgrad_finish_blocks(static_cast<long long>(wm) * wn) == 0)) continue;
+        const double chain_d = cd * kChunkD[td], chain_w = per * kChunkW[tw], all = (nd * chain_d + nw * chain_w) / cus;
         double us = kBase + (chain_d > chain_w ? (chain_d > all ? chain_d : all) : (chain_w > all ? chain_w : all));
         if (slices > 1) us += kFinish + kMillionSums * 1e-6 * slices * static_cast<double>(wm) * wn;
         if (best.nd != 0 && us >= best.us) continue;
@@ -128,10 +129,7 @@ size_t words_of(const ConvShape& s, const Plan& p) {
   const long long second = p.slices > 1 ? wgrad_finish_blocks(static_cast<long long>(s.K) * s.R * s.S * s.C) : p.nw;
   return 2 * static_cast<size_t>(kSlot0) + slot_words(static_cast<int>(p.nd)) + slot_words(static_cast<int>(second));
 }
-long long slice_of(const ConvShape& s) {
-  const long long n = static_cast<long long>(s.K) * s.R * s.S * s.C;
-  return (n + 1023) / 1024 * 1024 + 1088;   // the same element of consecutive slices in different memory channels
-}
+long long slice_of(const ConvShape& s) { return slice_stride(static_cast<long long>(s.K) * s.R * s.S * s.C); }
 
 }  // namespace
 

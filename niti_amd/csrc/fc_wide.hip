@@ -657,8 +657,7 @@ long long plan(int which, int M, int O, int F, int* tiles) {
   const char* e = getenv("NITI_FC_TILES");
   const int pin = e != nullptr ? atoi(e) : 0;
   const bool fwd = which == NITI_FC_FORWARD;
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+  const int cus = compute_units();
   long long best = 0;
   for (int t = 1; t <= 4; t *= 2) {
     if (pin != 0 && t != pin) continue;

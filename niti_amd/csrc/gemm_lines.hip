@@ -139,8 +139,9 @@ LnPlan lines_plan(int m, int n, int k) {
 
 }  // namespace
 
-// Products whose operands were always read as stored: niti_gemm_i8_workspace counts no copies of them.
-bool gemm_kmajor_shape(int trans_a, int trans_b, int m, int n, int k) {
+// Extents that every kernel which may take the product reads as stored: niti_gemm_i8_workspace counts no copies of the operands.
+// (gemm_any.hip reads all others as stored as well, but the workspace stays what callers have been told.)
+bool gemm_in_place_shape(int trans_a, int trans_b, int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 32 != 0) return false;
   if (trans_b != 0) return trans_a != 0 && m % 32 == 0 && (n + 127) / 128 <= 65535;   // TT = NN of (b, a), transposed
   if (n % 32 != 0) return false;
@@ -152,7 +153,7 @@ bool gemm_kmajor_shape(int trans_a, int trans_b, int m, int n, int k) {
 // so - 512 x 4096 x 2048 12.0 / 18.2, 128 x 8192 x 1024 6.0 / 6.1; with the reduction split (two launches) a reduction of 8192
 // steps, 128 x 1024 x 8192 9.9 / 18.0, but not one of 4096, 32 x 4096 x 4096 8.5 / 7.6, or 512, 512^3 7.5 / 3.5.
 bool gemm_lines_shape(int trans_a, int trans_b, int m, int n, int k) {
-  if ((trans_a != 0) != (trans_b != 0) || !gemm_kmajor_shape(trans_a, trans_b, m, n, k)) return false;
+  if ((trans_a != 0) != (trans_b != 0) || !gemm_in_place_shape(trans_a, trans_b, m, n, k)) return false;
   if (gemm_any_large(m, n)) return false;
   const LnPlan p = trans_b != 0 ? lines_plan(n, m, k) : lines_plan(m, n, k);
   return p.parts == 1 ? k >= 512 : p.parts > 1 && k > 6000;

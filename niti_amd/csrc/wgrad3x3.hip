@@ -1001,12 +1001,7 @@ __global__ __launch_bounds__(NW * 64, 4) void wgrad_finish_kernel(const FinishAr
   finish_columns<NW, kFinishV>(a, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), sh, predicted_raw);
 }
 
-// Slices are spaced so that the same element of consecutive slices falls into different memory
-// channels (a stride that is a multiple of 64 KB would put them all into one).
-long long slice_stride_for(int C, int K) {
-  const long long n = static_cast<long long>(K) * 9 * C;
-  return (n + 1023) / 1024 * 1024 + 1088;
-}
+long long slice_stride_for(int C, int K) { return slice_stride(static_cast<long long>(K) * 9 * C); }
 
 // The narrow-tile arrangement takes any batch (pixels behind the last image read as zeros).  NITI_WGRAD_NARROW=0 pins the wide
 // one, which needs whole bands of 128 pixels (tests).
