@@ -1,0 +1,164 @@
+"""Kernel variants that the dispatch picks by itself and that the sizes of the other tests do not reach: pairs of different tiles
+in the combined backward launches, the stochastic forms of every channel tile, the wide linear kernels' ends of range, the
+general convolution kernel behind a prepared data-gradient filter and behind the re-laid weight gradient."""
+import ctypes
+
+import pytest
+import torch
+
+import test_gpu_kernels as base
+
+pytestmark = pytest.mark.gpu
+ri8 = base.ri8
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+# data gradient on 32 x 32 tiles with an update on 64 x 64 and 128 x 128 ones, on 64 x 64 with 32 x 32 and 128 x 128; rows that
+# start on 16-byte boundaries and others
+@pytest.mark.parametrize("case", [(20, 320, 1024), (20, 300, 1000), (20, 1024, 2560), (20, 1030, 2300), (1024, 16, 512), (1030, 20, 510),
+                                  (512, 1024, 2560)])
+def test_linear_backward_of_two_tiles(dev, case, monkeypatch):
+    base.test_linear_backward_together(dev, case, "", monkeypatch)
+
+
+# N, H, W, C, K, filter, padding: the data gradient on 32 x 32 tiles with slices of the weight gradient on 64 x 64, 128 x 128; on
+# 64 x 64 with 32 x 32; on 128 x 64 with 32 x 32, with 64 x 64, and with whole 64 x 64
+@pytest.mark.parametrize("case", [(123, 5, 5, 16, 16, 3, 1), (9, 26, 26, 16, 80, 5, 2), (13, 27, 27, 16, 16, 3, 1), (41, 26, 26, 16, 16, 1, 0),
+                                  (56, 19, 19, 16, 16, 1, 0), (60, 33, 33, 16, 48, 1, 0)])
+def test_conv_backward_of_two_tiles(dev, case, monkeypatch):
+    base.test_conv_backward_together(dev, case, "", monkeypatch)
+
+
+# N, side, C, K with the channel tile pinned: every map's 128-channel tile, 64 channels of 4 x 4 maps, workgroups of 512 pixels
+# of 16 x 16 maps (forward and data gradient)
+@pytest.mark.parametrize("tile,case", [("128", (2, 32, 16, 160)), ("128", (2, 16, 32, 144)), ("128", (4, 8, 32, 144)), ("128", (16, 4, 16, 144)),
+                                       ("64", (16, 4, 32, 128)), ("64", (260, 16, 16, 128)), ("64", (260, 16, 128, 16))])
+def test_conv_sto_tiles(dev, tile, case, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_KT", tile)
+    base.test_conv_requant_sto(dev, case, "floor")
+
+
+@pytest.mark.parametrize("case", [(3, 2, 32, 48), (1, 16, 48, 32)])
+def test_conv_dgrad_i32_from_the_forward_copy(dev, case):
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    N, Q, C, K = case
+    g = torch.Generator().manual_seed(31 + N)
+    e, w = ri8(g, N, Q, Q, K), ri8(g, K, 3, 3, C)
+    got = ops.conv2d_dgrad(e.to(dev), w.to(dev), forward_filter=ops.conv_filter_prepare(w.to(dev), N, Q, Q))
+    assert torch.equal(got.cpu(), co.conv_dgrad(e, w, Q, Q, 1, 1))
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2"])
+@pytest.mark.parametrize("case", [(33, 48, 80), (65, 16, 208), (130, 80, 144)])
+def test_linear_dgrad_of_aligned_rows(dev, case, tile, monkeypatch):
+    """Widths that are multiples of 16 and not of 32: the kernel for any extents, rows on 16-byte boundaries."""
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    monkeypatch.setenv("NITI_ANY_TILE", tile)
+    M, O, F = case
+    g = torch.Generator().manual_seed(M)
+    err, w = ri8(g, M, O, lo=-60, hi=60), ri8(g, O, F)
+    for method in ("round", "psto"):
+        y, sh, sync = ops.linear_dgrad_requant(err.to(dev), w.to(dev), 7, method)
+        ref, sh_ref = po.err_calc(po.int8mm(err, w), method, "floor")
+        assert torch.equal(y.cpu(), ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_gemm_f32_epilogue_of_a_split_reduction(dev, ta, tb):
+    """The whole-line kernel with the reduction split over workgroups: the round trip happens where the parts are added."""
+    base.test_gemm_f32_epilogue_above_2_24(dev, ta, tb, (128, 128, 8192))
+
+
+# M, O, F: layers whose update would be more 128 x 128 tiles than are resident at once - few outputs and very many features, one
+# with as many workgroups as are resident, a ragged last tile, the widest square of them
+@pytest.mark.parametrize("case", [(5, 32, 131072), (7, 16, 100000), (3, 1024, 8192)])
+def test_linear_update_of_wide_layers(dev, case):
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    M, O, F = case
+    base._say("linear_update_of_wide_layers", case)
+    g = torch.Generator().manual_seed(O)
+    err, act, w = ri8(g, M, O, lo=-60, hi=60), ri8(g, M, F), ri8(g, O, F)
+    assert ops.linear_sync_words("wgrad", M, O, F) > 0
+    acc = po.int8mm(err.t().contiguous(), act)
+    rand = torch.randint(0, 1 << 24, acc.shape, generator=g, dtype=torch.int32)
+    for method in ("psto", "sto"):
+        low = rand & ((1 << max(po.bitwidth_int(po.absmax(acc)) - 5, 0)) - 1)
+        wd = w.to(dev)
+        g8, sh, sync = ops.linear_wgrad_update(err.to(dev), act.to(dev), wd, 5, method, rand=rand.to(dev) if method == "sto" else None, want_grad=True)
+        ref, sh_ref = po.grad_calc(acc, 5, method, "floor", rand=low if method == "sto" else None)
+        assert torch.equal(g8.cpu(), ref) and int(sh.cpu()) == sh_ref and int(sync.cpu()[1]) == 0, method
+        assert torch.equal(wd.cpu(), po.weight_update(w, ref)), method
+
+
+def test_linear_forward_of_two_sample_tiles(dev):
+    """128 rows, a reduction that is no multiple of 128: two tiles of 16 samples per workgroup."""
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    M, O, F = 128, 1024, 144
+    g = torch.Generator().manual_seed(77)
+    act, w = ri8(g, M, F), ri8(g, O, F)
+    y, sh, sync = ops.linear_fwd_requant(act.to(dev), w.to(dev))
+    ref, _ = po.act_calc(po.int8mm(act, w.t().contiguous()), 0)
+    assert torch.equal(y.cpu(), ref) and int(sync.cpu()[1]) == 0
+
+
+# N, H, W, C, K, filter, padding: whole 128-byte steps of one tap; 512- and 256-pixel tiles; a filter of more than 32 taps
+@pytest.mark.parametrize("case", [(2, 9, 9, 32, 128, 3, 1), (128, 30, 30, 32, 16, 3, 1), (32, 30, 30, 144, 16, 3, 1), (1, 9, 9, 16, 16, 7, 3)])
+def test_conv_dgrad_from_its_own_copy(dev, case):
+    """The data gradient from a filter flipped beforehand, on maps outside the 3 x 3 kernels': the general convolution kernel."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, H, W, C, K, R, pad = case
+    base._say("conv_dgrad_from_its_own_copy", case)
+    g = torch.Generator().manual_seed(51 + N)
+    e, w = ri8(g, N, H + 2 * pad - R + 1, W + 2 * pad - R + 1, K), ri8(g, K, R, R, C)
+    ref = co.conv_dgrad(e, w, H, W, 1, pad)
+    copy = ops.conv_filter_prepare(w.to(dev), N, H, W, 1, pad, dgrad=True)
+    am = ops.new_scalar_u32(dev)
+    assert torch.equal(ops.conv2d_dgrad(e.to(dev), w.to(dev), 1, pad, absmax=am, prepared_filter=copy).cpu(), ref)
+    assert int(am.cpu()) == po.absmax(ref)
+
+
+# N, H, W, C, K: filters that are no multiple of 16, so both operands are re-laid; batches of whole 128-byte steps with few and many
+# channels, shorter ones with 256- and 512-row tiles
+@pytest.mark.parametrize("case", [(128, 4, 4, 16, 10), (128, 4, 4, 1600, 10), (64, 4, 4, 3200, 10), (16, 4, 4, 6400, 10)])
+def test_conv_wgrad_re_laid(dev, case):
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, H, W, C, K = case
+    base._say("conv_wgrad_re_laid", case)
+    g = torch.Generator().manual_seed(61 + C)
+    a, e = ri8(g, N, H, W, C), ri8(g, N, H, W, K, lo=-40, hi=40)
+    ref = co.conv_wgrad(a, e, 3, 3, 1, 1)
+    am = ops.new_scalar_u32(dev)
+    assert torch.equal(ops.conv2d_wgrad(a.to(dev), e.to(dev), 3, 3, absmax=am).cpu(), ref) and int(am.cpu()) == po.absmax(ref)
+
+
+def test_quantiser_entries_of_the_c_abi(dev):
+    """The two entries that the front end does not call, against the one it does."""
+    from niti_amd import _lib as L
+    from niti_amd import ops
+    x = torch.randn((9, 3, 16, 16), generator=torch.Generator().manual_seed(4)).to(dev)
+    want, exp = ops.quantize_input(x)
+    N, C, H, W = x.shape
+    stream = torch.cuda.current_stream().cuda_stream
+    y, e = torch.full_like(want, 55), torch.full_like(exp, 55)
+    word = torch.zeros(1, dtype=torch.int32, device=dev)
+    L.check(L.lib().niti_quantize_f32_i8(x.data_ptr(), y.data_ptr(), N, C, H, W, 16, 7, word.data_ptr(), e.data_ptr(), stream), "quantize")
+    assert torch.equal(y, want) and torch.equal(e, exp)
+    y.fill_(55), e.fill_(55)
+    parts = torch.empty(256, dtype=torch.int32, device=dev)
+    target = torch.arange(9, device=dev)
+    copied = torch.zeros_like(target)
+    L.check(L.lib().niti_quantize_batch_f32_i8(x.data_ptr(), y.data_ptr(), N, C, H, W, 16, 7, parts.data_ptr(), e.data_ptr(), target.data_ptr(),
+                                               copied.data_ptr(), 9, ctypes.c_void_p(stream)), "quantize_batch")
+    assert torch.equal(y, want) and torch.equal(e, exp) and torch.equal(copied, target)
