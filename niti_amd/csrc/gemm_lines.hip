@@ -149,14 +149,19 @@ bool gemm_in_place_shape(int trans_a, int trans_b, int m, int n, int k) {
   return (m + 127) / 128 <= 65535;
 }
 
-// Where this kernel is the faster one (us, this / gemm_any.hip): rows of tiles that fill the device without 128 x 128 tiles doing
-// so - 512 x 4096 x 2048 12.0 / 18.2, 128 x 8192 x 1024 6.0 / 6.1; with the reduction split (two launches) a reduction of 8192
-// steps, 128 x 1024 x 8192 9.9 / 18.0, but not one of 4096, 32 x 4096 x 4096 8.5 / 7.6, or 512, 512^3 7.5 / 3.5.
+// Where this kernel is the faster one (us, this / gemm_any.hip, measured at 128 ... 16384 steps for twelve results each):
+//   rows of tiles that fill the device without 128 x 128 tiles doing so.  NN between 512 and 5120 steps while b stays in the caches:
+//   512 x 2048 at 512 4.8 / 5.0, 3072 11.1 / 14.3, 5120 17.6 / 21.0, 6144 26.9 / 24.4; 128 x 8192 at 3072 11.1 / 14.4, 4096
+//   21.5 / 17.6.  TT, whose stores are columns, up to 1024: 384 x 2048 at 512 4.4 / 4.6, 1024 5.6 / 5.7, 2048 8.1 / 7.7, 4096
+//   17.9 / 11.7;
+//   the reduction split (two launches), from about 6000 steps on: NN 128 x 1024 at 4096 8.4 / 7.5, 5120 8.6 / 8.3, 6144 8.9 / 9.4, 8192
+//   9.5 / 17.5; TT of it 5120 8.4 / 7.9, 6144 8.8 / 8.8, 8192 9.4 / 11.2; 128 x 128 at 4096 6.7 / 6.6, 6144 6.8 / 8.5.
 bool gemm_lines_shape(int trans_a, int trans_b, int m, int n, int k) {
   if ((trans_a != 0) != (trans_b != 0) || !gemm_in_place_shape(trans_a, trans_b, m, n, k)) return false;
   if (gemm_any_large(m, n)) return false;
   const LnPlan p = trans_b != 0 ? lines_plan(n, m, k) : lines_plan(m, n, k);
-  return p.parts == 1 ? k >= 512 : p.parts > 1 && k > 6000;
+  if (p.parts > 1) return k > 6000;
+  return p.parts == 1 && k >= 512 && (trans_b != 0 ? k <= 1024 : k <= 5120 && static_cast<long long>(k) * n <= (24 << 20));
 }
 
 // bytes of partial results the whole-line kernel wants for this product (0: none)
