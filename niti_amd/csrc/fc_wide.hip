@@ -19,6 +19,8 @@
 // slot of its own and reads all slots (all workgroups resident - checked by the host - wait bounded by a wall clock).
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "gemm_any.h"
 #include "grid_range.h"
@@ -588,10 +590,9 @@ int fwd_lds_resident(int mt) {
   return resident_cached(c2, fcw_fwd_lds_kernel<2>, 512, fwd_lds_bytes(2));
 }
 int fwd_resident(int mt) {
-  static int c1[kDeviceSlots] = {}, c2[kDeviceSlots] = {}, c4[kDeviceSlots] = {};
+  static int c1[kDeviceSlots] = {}, c2[kDeviceSlots] = {};
   if (mt == 1) return resident_cached(c1, fcw_fwd_kernel<1>, 1024, fwd_lds(1));
-  if (mt == 2) return resident_cached(c2, fcw_fwd_kernel<2>, 1024, fwd_lds(2));
-  return resident_cached(c4, fcw_fwd_kernel<4>, 1024, fwd_lds(4));
+  return resident_cached(c2, fcw_fwd_kernel<2>, 1024, fwd_lds(2));
 }
 int wgrad_resident(int t) {
   static int c1[kDeviceSlots] = {}, c2[kDeviceSlots] = {}, c4[kDeviceSlots] = {};
@@ -640,10 +641,8 @@ long long plan(int which, int M, int O, int F, int* tiles) {
   *tiles = 0;
   if (!shape_ok(which, M, O, F)) return 0;
   // Where both sets of kernels cover the shape the ones for any extents take every weight gradient they fit (they share a
-  // 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512 8.6 -> 7.1) and the
-  // forward passes of large batches (512 x 4096 -> 1024 15.2 -> 13.0 us; 128 x 8192 -> 1024 takes them 12.3 instead of 8.3)
+  // 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512 8.6 -> 7.1)
   if (which == NITI_FC_WGRAD && any_blocks(which, M, O, F) > 0) return 0;
-  if (which == NITI_FC_FORWARD && M > 160 && any_blocks(which, M, O, F) > 0) return 0;
   if (which == NITI_FC_DGRAD) {
     if (const long long nl = dgrad_lds_blocks(M, O, F)) {
       *tiles = 1;
@@ -659,17 +658,25 @@ long long plan(int which, int M, int O, int F, int* tiles) {
   const bool fwd = which == NITI_FC_FORWARD;
   const int cus = compute_units();
   long long best = 0;
-  for (int t = 1; t <= 4; t *= 2) {
+  for (int t = 1; t <= (fwd ? 2 : 4); t *= 2) {
     if (pin != 0 && t != pin) continue;
     const long long nb = fwd ? static_cast<long long>((O + 15) / 16) * ((M + 16 * t - 1) / (16 * t))
                              : static_cast<long long>((F + 255) / 256) * ((O + 32 * t - 1) / (32 * t));
     if (nb > kMaxSlots || nb > (fwd ? fwd_resident(t) : wgrad_resident(t))) continue;
-    // forward: more sample tiles per workgroup re-read the weights less often, as long as every compute unit still
-    // gets a workgroup (measured on 128 x 8192 x 1024: 21.7 / 15.9 / 23.3 us for 1 / 2 / 4 tiles)
+    // forward: two sample tiles per workgroup read the weights half as often, as long as every compute unit still gets a workgroup
     if (best == 0 || (fwd && nb >= cus)) {
       best = nb;
       *tiles = t;
     }
+  }
+  // Forward: as long as a compute unit has at most one workgroup the launch is as long as one walk along F; behind that the kernels
+  // for any extents are the faster ones.  These / any extents, us: 8192 -> 1024 with 128 rows 8.5 / 13.7, 144 22.8 / 14.2, 256
+  // 23.3 / 17.1; 2048 -> 512 with 128 5.3 / 6.3, 144 6.6 / 6.4, 256 (two sample tiles) 5.6 / 6.5, 320 9.4 / 6.5; 2048 -> 2048 with 64
+  // 5.7 / 6.5, 96 9.9 / 6.8; 1008 -> 1000 with 64 5.7 / 6.0, 96 6.8 / 6.0; 4096 -> 64 with 512 5.4 / 7.8.  Of 117 shapes, 9 layers
+  // with 32 ... 512 rows, only 1024 -> 4096 with 32 goes against it (6.7 / 5.7).
+  if (fwd && pin == 0 && best > cus && any_blocks(which, M, O, F) > 0) {
+    *tiles = 0;
+    return 0;
   }
   return best;
 }
@@ -702,7 +709,8 @@ using namespace niti;
 extern "C" size_t niti_linear_i8_sync_words(int which, int M, int O, int F) {
   int tiles = 0;
   long long nb = plan(which, M, O, F, &tiles);
-  if (nb == 0) nb = any_blocks(which, M, O, F);
+  // a forward pass whose pointers do not start on 16-byte boundaries goes to the kernels for any extents
+  if (nb == 0 || which == NITI_FC_FORWARD) nb = std::max(nb, any_blocks(which, M, O, F));
   return nb == 0 ? 0 : static_cast<size_t>(kSlot0) + slot_words(static_cast<int>(nb));
 }
 
@@ -757,22 +765,23 @@ extern "C" int niti_linear_i8_fwd_requant(const int8_t* act, const int8_t* w, in
   a.rq_flags = rq_flags;
   a.kchunk = fwd_chunk(F);
   int mt = 0;
-  if (plan(NITI_FC_FORWARD, M, O, F, &mt) == 0) return launch_any(kAnyForward, a, act, w, M, O, F, static_cast<hipStream_t>(stream));
-  if (!aligned16(act) || !aligned16(w) || !aligned16(rand) || reinterpret_cast<uintptr_t>(out8) % 4 != 0)
+  const bool aligned = aligned16(act) && aligned16(w) && aligned16(rand) && reinterpret_cast<uintptr_t>(out8) % 4 == 0;
+  if (plan(NITI_FC_FORWARD, M, O, F, &mt) == 0 || (!aligned && any_blocks(NITI_FC_FORWARD, M, O, F) > 0))
+    return launch_any(kAnyForward, a, act, w, M, O, F, static_cast<hipStream_t>(stream));
+  if (!aligned)
     return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   const dim3 grid((O + 15) / 16, (M + 16 * mt - 1) / (16 * mt));
   hipStream_t s = static_cast<hipStream_t>(stream);
   // whole lines through LDS where the rows are whole lines (NITI_FC_LDS=0 pins the direct-fragment kernel)
   const char* e = getenv("NITI_FC_LDS");
-  if (F % 128 == 0 && mt <= 2 && (e == nullptr || e[0] != '0') && static_cast<long long>(grid.x) * grid.y <= fwd_lds_resident(mt)) {
+  if (F % 128 == 0 && (e == nullptr || e[0] != '0') && static_cast<long long>(grid.x) * grid.y <= fwd_lds_resident(mt)) {
     a.kchunk = ((F + 7) / 8 + 127) / 128 * 128;
     if (mt == 1) hipLaunchKernelGGL(fcw_fwd_lds_kernel<1>, grid, dim3(512), fwd_lds_bytes(1), s, a);
     else hipLaunchKernelGGL(fcw_fwd_lds_kernel<2>, grid, dim3(512), fwd_lds_bytes(2), s, a);
     return check_launch(who);
   }
   if (mt == 1) hipLaunchKernelGGL(fcw_fwd_kernel<1>, grid, dim3(1024), fwd_lds(1), s, a);
-  else if (mt == 2) hipLaunchKernelGGL(fcw_fwd_kernel<2>, grid, dim3(1024), fwd_lds(2), s, a);
-  else hipLaunchKernelGGL(fcw_fwd_kernel<4>, grid, dim3(1024), fwd_lds(4), s, a);
+  else hipLaunchKernelGGL(fcw_fwd_kernel<2>, grid, dim3(1024), fwd_lds(2), s, a);
   return check_launch(who);
 }
 

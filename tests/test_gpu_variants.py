@@ -109,6 +109,26 @@ def test_linear_forward_of_two_sample_tiles(dev):
     assert torch.equal(y.cpu(), ref) and int(sync.cpu()[1]) == 0
 
 
+# M, O, F on both sides of one workgroup per compute unit, with whole lines and without
+@pytest.mark.parametrize("case", [(64, 1024, 256), (65, 1024, 256), (128, 1024, 256), (129, 1024, 256), (64, 1000, 144), (80, 1000, 144)])
+def test_linear_forward_of_operands_that_start_anywhere(dev, case):
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    M, O, F = case
+    g = torch.Generator().manual_seed(M + F)
+    act, w = ri8(g, M, F), ri8(g, O, F)
+    ref, _ = po.act_calc(po.int8mm(act, w.t().contiguous()), 0)
+
+    def placed(t, offset):
+        flat = torch.zeros(t.numel() + 16, dtype=torch.int8, device=dev)
+        view = flat[offset:offset + t.numel()].view(t.shape)
+        view.copy_(t)
+        return view
+    for a, b in ((0, 0), (1, 0), (0, 4), (8, 3)):
+        y, sh, sync = ops.linear_fwd_requant(placed(act, a), placed(w, b))
+        assert torch.equal(y.cpu(), ref) and int(sync.cpu()[1]) == 0, (a, b)
+
+
 # N, H, W, C, K, filter, padding: whole 128-byte steps of one tap; 512- and 256-pixel tiles; a filter of more than 32 taps
 @pytest.mark.parametrize("case", [(2, 9, 9, 32, 128, 3, 1), (128, 30, 30, 32, 16, 3, 1), (32, 30, 30, 144, 16, 3, 1), (1, 9, 9, 16, 16, 7, 3)])
 def test_conv_dgrad_from_its_own_copy(dev, case):
