@@ -343,8 +343,8 @@ PyObject* layer_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     f.relu = a.flag();
     f.shift = a.opt();
     f.hint = f.shift != nullptr;
-    f.exp_a = a.opt();
-    f.exp_b = a.opt();
+    f.exp_a = a.exponent();
+    f.exp_b = a.exponent();
     f.prepared = a.opt();
     const bool pool = a.flag();
     f.rand = a.opt();
@@ -567,8 +567,8 @@ PyObject* layer_wgrad_update(PyObject*, PyObject* const* args, Py_ssize_t n) {
     g.flags = a.flag() ? NITI_EPI_F32_ROUNDTRIP : 0u;
     g.r = rounding_of(a);
     take_weight_gradient(a, &g);
-    g.exp_a = a.opt();
-    g.exp_b = a.opt();
+    g.exp_a = a.exponent();
+    g.exp_b = a.exponent();
     g.prepared = a.opt();
     g.rand = a.opt();
     at::Tensor e = scalar32(act);
@@ -597,8 +597,8 @@ PyObject* layer_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     f.r = rounding_of(a);
     f.shift = a.opt();
     f.hint = f.shift != nullptr;
-    f.exp_a = a.opt();
-    f.exp_b = a.opt();
+    f.exp_a = a.exponent();
+    f.exp_b = a.exponent();
     f.prepared = a.opt();
     f.mask = a.opt();
     Opt pool_in = a.opt();
@@ -610,7 +610,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     g.r.bits = a.i();
     g.r.method = a.i();
     take_weight_gradient(a, &g);
-    g.exp_b = a.opt();
+    g.exp_b = a.exponent();
     g.prepared = a.opt();
     g.rand = a.opt();
     DataGradient r;

@@ -59,6 +59,11 @@ class Args {
     if (!THPVariable_Check(o)) refuse("niti_amd: tensor or None expected");
     return &use(THPVariable_Unpack(o));
   }
+  Opt exponent() {   // one value, as a layer hands it on
+    Opt t = opt();
+    if (t != nullptr && (t->numel() != 1 || t->scalar_type() != at::kInt)) refuse("niti_amd: an exponent is one int32 value");
+    return t;
+  }
   long integer() {
     const long v = PyLong_AsLong(a_[i_++]);
     if (v == -1 && PyErr_Occurred()) throw python_error();

@@ -37,7 +37,7 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const at::Tensor& act = a.tensor();
     const at::Tensor& w = a.tensor();
     const int bits = a.i(), method = a.i(), div = a.i(), bw = a.i();
-    Opt ea = a.opt(), eb = a.opt(), rand = a.opt();
+    Opt ea = a.exponent(), eb = a.exponent(), rand = a.opt();
     const Shape s = shape_of(act, w, 1, "linear_forward");
     check_rand(rand, static_cast<int64_t>(s.M) * s.O, "linear_forward");
     at::Tensor y, e = scalar32(act);
@@ -133,7 +133,7 @@ PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     re.div = rg.div = a.i();
     re.bw = rg.bw = a.i();
     const bool want_grad = a.flag(), keep = a.flag();
-    Opt exp_err = a.opt(), exp_w = a.opt(), exp_act = a.opt();
+    Opt exp_err = a.exponent(), exp_w = a.exponent(), exp_act = a.exponent();
     re.rand = a.opt();
     rg.rand = a.opt();
     const Shape s = shape_of(err, w, 0, "linear_backward");
@@ -169,7 +169,7 @@ PyObject* head_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int bits = a.i(), method = a.i(), div = a.i(), bw = a.i(), dropout = a.i();
     Opt mask_given = a.opt(), rng = a.opt();
     const int exp_bias = a.i();
-    Opt target = a.opt(), loss_rand = a.opt(), ea = a.opt(), eb = a.opt();
+    Opt target = a.opt(), loss_rand = a.opt(), ea = a.exponent(), eb = a.exponent();
     const Shape s = shape_of(act, w, 1, "head_forward");
     const size_t words = niti_head_i8_sync_words(0, s.M, s.O, s.F);
     if (words == 0) Py_RETURN_NONE;
@@ -203,7 +203,7 @@ PyObject* head_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int eb = a.i(), em = a.i(), gb = a.i(), gm = a.i(), div = a.i(), bw = a.i();
     Opt mask = a.opt();
     const bool want_grad = a.flag();
-    Opt exp_err = a.opt(), exp_w = a.opt(), exp_act = a.opt();
+    Opt exp_err = a.exponent(), exp_w = a.exponent(), exp_act = a.exponent();
     const int bias = a.i();
     Opt pool_in = a.opt();
     const int pool_flags = a.i();

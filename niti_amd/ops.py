@@ -344,6 +344,8 @@ def mask_features(x, mask, exp_in=None, exp_add=None):
     _chk_dev(x, mask, exp_in)
     if x.dtype != torch.int8 or mask.dtype != torch.int8 or x.dim() != 2 or mask.numel() != x.shape[1]:
         raise RuntimeError("mask_features: int8 [rows, F] tensor and int8 [F] mask expected")
+    if exp_in is not None and exp_in.numel() != 1:
+        raise RuntimeError("mask_features: an exponent is one value")
     y = torch.empty_like(x)
     exp_out = torch.empty(1, dtype=torch.int32, device=x.device) if exp_add is not None else None
     L.check(L.lib().niti_mask_features_i8(_ptr(x), _ptr(mask), _ptr(y), x.shape[0], x.shape[1], _ptr(exp_in), _ptr(exp_out),

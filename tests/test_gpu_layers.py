@@ -806,3 +806,22 @@ def test_streams_one_after_another(tt):
     for i, results in got:
         assert all(torch.equal(p, q) for p, q in zip(results, want[i % 2])), i
     assert not ops.sync_timeouts(dev)
+
+
+def test_layers_refuse_exponents_of_several_values(tt):
+    """An exponent tensor of more than one element is an error in every pass of the layers, not its first element."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(2)
+    two = torch.zeros(2, dtype=torch.int32, device=dev)
+    conv, first, linear, few = tt.TiConv2d(32, 48), tt.TiConv2d(16, 48, first_layer=True), tt.TiLinear(200, 72), tt.TiLinear(64, 10)
+    x, x1, a, b = (ri8(g, *s).to(dev) for s in ((2, 8, 8, 32), (2, 8, 8, 16), (20, 200), (20, 64)))
+    e, f, h = (ri8(g, *s).to(dev) for s in ((2, 8, 8, 48), (20, 72), (20, 10)))
+    for layer, inp, err in ((conv, x, e), (first, x1, e), (linear, a, f), (few, b, h)):
+        with pytest.raises(RuntimeError):
+            layer.forward((inp, two))
+        layer.forward((inp, 0))
+        with pytest.raises(RuntimeError):
+            layer.backward((err, two))
+        layer.backward((err, torch.zeros((), dtype=torch.int32, device=dev)))
+    with pytest.raises(RuntimeError):
+        tt.TiDropout().forward((b, two))
