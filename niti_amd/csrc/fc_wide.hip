@@ -636,13 +636,18 @@ long long any_blocks(int which, int M, int O, int F) {
 }
 
 // Workgroups of the launch on the current device and the per-workgroup tile count (MT / T); 0 when the shape is outside
-// the kernels or no variant's grid fits on the device at once.
-long long plan(int which, int M, int O, int F, int* tiles) {
+// the kernels, no variant's grid fits on the device at once, or the kernels for any extents take it.  any: their workgroups, where
+// they come into question.
+long long plan(int which, int M, int O, int F, int* tiles, long long* any) {
   *tiles = 0;
-  if (!shape_ok(which, M, O, F)) return 0;
+  *any = which == NITI_FC_DGRAD ? 0 : any_blocks(which, M, O, F);
+  if (!shape_ok(which, M, O, F)) {
+    if (which == NITI_FC_DGRAD) *any = any_blocks(which, M, O, F);
+    return 0;
+  }
   // Where both sets of kernels cover the shape the ones for any extents take every weight gradient they fit (they share a
   // 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512 8.6 -> 7.1)
-  if (which == NITI_FC_WGRAD && any_blocks(which, M, O, F) > 0) return 0;
+  if (which == NITI_FC_WGRAD && *any > 0) return 0;
   if (which == NITI_FC_DGRAD) {
     if (const long long nl = dgrad_lds_blocks(M, O, F)) {
       *tiles = 1;
@@ -650,7 +655,9 @@ long long plan(int which, int M, int O, int F, int* tiles) {
     }
     const long long nb = static_cast<long long>(F / 32) * ((M + 127) / 128);
     *tiles = 1;
-    return (nb <= kMaxSlots && nb <= dgrad_resident(O)) ? nb : 0;
+    if (nb <= kMaxSlots && nb <= dgrad_resident(O)) return nb;
+    *any = any_blocks(which, M, O, F);
+    return 0;
   }
   // NITI_FC_TILES pins the tiles per workgroup (measurements); otherwise the smallest count whose grid fits
   const char* e = getenv("NITI_FC_TILES");
@@ -670,11 +677,13 @@ long long plan(int which, int M, int O, int F, int* tiles) {
     }
   }
   // Forward: as long as a compute unit has at most one workgroup the launch is as long as one walk along F; behind that the kernels
-  // for any extents are the faster ones.  These / any extents, us: 8192 -> 1024 with 128 rows 8.5 / 13.7, 144 22.8 / 14.2, 256
-  // 23.3 / 17.1; 2048 -> 512 with 128 5.3 / 6.3, 144 6.6 / 6.4, 256 (two sample tiles) 5.6 / 6.5, 320 9.4 / 6.5; 2048 -> 2048 with 64
-  // 5.7 / 6.5, 96 9.9 / 6.8; 1008 -> 1000 with 64 5.7 / 6.0, 96 6.8 / 6.0; 4096 -> 64 with 512 5.4 / 7.8.  Of 117 shapes, 9 layers
-  // with 32 ... 512 rows, only 1024 -> 4096 with 32 goes against it (6.7 / 5.7).
-  if (fwd && pin == 0 && best > cus && any_blocks(which, M, O, F) > 0) {
+  // for any extents are the faster ones, for long rows only where the workgroups that stage whole lines are not all resident.  These /
+  // any extents, us: 8192 -> 1024 with 128 rows 8.5 / 13.7, 144 22.8 / 14.2, 256 23.3 / 17.1; 2048 -> 512 with 128 5.3 / 6.3, 256 (two
+  // sample tiles) 5.6 / 6.5, 320 9.4 / 6.5; 2048 -> 2048 with 64 5.7 / 6.5, 96 9.9 / 6.8; 4096 -> 64 with 512 5.4 / 7.8; a layer's
+  // forward and backward pass with one and a half to two workgroups per unit: 8192 -> 1024 with 96 37.8 / 41.2, 4096 -> 512 with 160
+  // 27.1 / 28.2, 2048 -> 1024 with 96 27.4 / 27.4, 1024 -> 768 with 128 20.0 / 18.8, 512 -> 256 with 480 15.1 / 14.3.
+  const bool lines = F % 128 == 0 && F >= 4096;
+  if (fwd && pin == 0 && best > (lines ? fwd_lds_resident(*tiles) : cus) && *any > 0) {
     *tiles = 0;
     return 0;
   }
@@ -708,9 +717,9 @@ using namespace niti;
 
 extern "C" size_t niti_linear_i8_sync_words(int which, int M, int O, int F) {
   int tiles = 0;
-  long long nb = plan(which, M, O, F, &tiles);
+  long long any = 0, nb = plan(which, M, O, F, &tiles, &any);
   // a forward pass whose pointers do not start on 16-byte boundaries goes to the kernels for any extents
-  if (nb == 0 || which == NITI_FC_FORWARD) nb = std::max(nb, any_blocks(which, M, O, F));
+  if (nb == 0 || which == NITI_FC_FORWARD) nb = std::max(nb, any);
   return nb == 0 ? 0 : static_cast<size_t>(kSlot0) + slot_words(static_cast<int>(nb));
 }
 
@@ -765,8 +774,9 @@ extern "C" int niti_linear_i8_fwd_requant(const int8_t* act, const int8_t* w, in
   a.rq_flags = rq_flags;
   a.kchunk = fwd_chunk(F);
   int mt = 0;
+  long long any = 0;
   const bool aligned = aligned16(act) && aligned16(w) && aligned16(rand) && reinterpret_cast<uintptr_t>(out8) % 4 == 0;
-  if (plan(NITI_FC_FORWARD, M, O, F, &mt) == 0 || (!aligned && any_blocks(NITI_FC_FORWARD, M, O, F) > 0))
+  if (plan(NITI_FC_FORWARD, M, O, F, &mt, &any) == 0 || (!aligned && any > 0))
     return launch_any(kAnyForward, a, act, w, M, O, F, static_cast<hipStream_t>(stream));
   if (!aligned)
     return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
@@ -799,7 +809,8 @@ extern "C" int niti_linear_i8_dgrad_requant(const int8_t* err, const int8_t* w, 
   a.w = const_cast<int8_t*>(w);
   a.out8 = dx8;
   int tiles = 0;
-  if (plan(NITI_FC_DGRAD, M, O, F, &tiles) == 0) return launch_any(kAnyDgrad, a, err, w, M, F, O, static_cast<hipStream_t>(stream));
+  long long any = 0;
+  if (plan(NITI_FC_DGRAD, M, O, F, &tiles, &any) == 0) return launch_any(kAnyDgrad, a, err, w, M, F, O, static_cast<hipStream_t>(stream));
   if (!aligned16(err) || !aligned16(w) || !aligned16(rand) || reinterpret_cast<uintptr_t>(dx8) % 4 != 0)
     return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   if (dgrad_lds_blocks(M, O, F) != 0) {
@@ -828,7 +839,8 @@ extern "C" int niti_linear_i8_wgrad_update(const int8_t* err, const int8_t* act,
   a.w = w;
   a.out8 = g8_out;
   int t_use = 0;
-  if (plan(NITI_FC_WGRAD, M, O, F, &t_use) == 0) return launch_any(kAnyUpdate, a, err, act, O, F, M, static_cast<hipStream_t>(stream));
+  long long any = 0;
+  if (plan(NITI_FC_WGRAD, M, O, F, &t_use, &any) == 0) return launch_any(kAnyUpdate, a, err, act, O, F, M, static_cast<hipStream_t>(stream));
   if (!aligned16(err) || !aligned16(act) || !aligned16(w) || !aligned16(g8_out) || !aligned16(rand))
     return fail(NITI_ERR_INVALID_ARG, "%s: misaligned pointer", who);
   const dim3 grid((F + 255) / 256, (O + 32 * t_use - 1) / (32 * t_use));
