@@ -149,19 +149,21 @@ bool gemm_in_place_shape(int trans_a, int trans_b, int m, int n, int k) {
   return (m + 127) / 128 <= 65535;
 }
 
-// Where this kernel is the faster one (us, this / gemm_any.hip, measured at 128 ... 16384 steps for twelve results each):
-//   rows of tiles that fill the device without 128 x 128 tiles doing so.  NN between 512 and 5120 steps while b stays in the caches:
-//   512 x 2048 at 512 4.8 / 5.0, 3072 11.1 / 14.3, 5120 17.6 / 21.0, 6144 26.9 / 24.4; 128 x 8192 at 3072 11.1 / 14.4, 4096
-//   21.5 / 17.6.  TT, whose stores are columns, up to 1024: 384 x 2048 at 512 4.4 / 4.6, 1024 5.6 / 5.7, 2048 8.1 / 7.7, 4096
-//   17.9 / 11.7;
-//   the reduction split (two launches), from about 6000 steps on: NN 128 x 1024 at 4096 8.4 / 7.5, 5120 8.6 / 8.3, 6144 8.9 / 9.4, 8192
-//   9.5 / 17.5; TT of it 5120 8.4 / 7.9, 6144 8.8 / 8.8, 8192 9.4 / 11.2; 128 x 128 at 4096 6.7 / 6.6, 6144 6.8 / 8.5.
+// Where this kernel is the faster one: this / gemm_any.hip, us, the same operands again and again (they lie in the caches) and new
+// ones at every call (they do not), at 512 ... 8192 steps for eight results in each form.
+//   Rows of tiles that fill the device without 128 x 128 tiles doing so: 512 x 2048 NN at 512 steps 4.8 / 5.0 and new 5.0 / 5.4, 1024
+//   6.1 / 6.2 and 6.9 / 7.1, 3072 11.1 / 14.3 and 20.3 / 17.0, 5120 17.6 / 21.0 and 33.0 / 27.2, 6144 26.9 / 24.4 and 38.4 / 31.7:
+//   taken up to 5120 while b stays in the caches (128 x 8192 at 3072 11.1 / 14.4, 4096 21.5 / 17.6).  TT, whose stores are columns:
+//   384 x 2048 at 512 4.4 / 4.6 and 4.6 / 4.7, 1024 5.6 / 5.7 and 6.6 / 6.0, 2048 8.1 / 7.7 and 10.4 / 8.4, 4096 17.9 / 11.7.
+//   The reduction split over workgroups (two launches): 128 x 1024 NN at 3072 8.0 / 6.4 and 8.3 / 9.1, 4096 8.4 / 7.5 and 8.8 / 11.1, 5120
+//   8.6 / 8.3 and 9.5 / 13.1, 6144 8.9 / 9.4 and 10.7 / 17.2, 8192 9.5 / 17.5; TT of it 5120 8.4 / 7.9 and 9.2 / 11.8; 128 x 128 NN at
+//   4096 6.7 / 6.6 and 6.7 / 9.3; 512 x 512 at 5120 10.2 / 10.2 and 11.8 / 11.9.
 bool gemm_lines_shape(int trans_a, int trans_b, int m, int n, int k) {
   if ((trans_a != 0) != (trans_b != 0) || !gemm_in_place_shape(trans_a, trans_b, m, n, k)) return false;
   if (gemm_any_large(m, n)) return false;
   const LnPlan p = trans_b != 0 ? lines_plan(n, m, k) : lines_plan(m, n, k);
-  if (p.parts > 1) return k > 6000;
-  return p.parts == 1 && k >= 512 && (trans_b != 0 ? k <= 1024 : k <= 5120 && static_cast<long long>(k) * n <= (24 << 20));
+  if (p.parts > 1) return k > 5000;
+  return p.parts == 1 && k >= 512 && (trans_b != 0 ? k < 1024 : k <= 5120 && static_cast<long long>(k) * n <= (24 << 20));
 }
 
 // bytes of partial results the whole-line kernel wants for this product (0: none)
