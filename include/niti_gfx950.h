@@ -430,9 +430,11 @@ int niti_fc_i8_wgrad_update(const int8_t* err, const int8_t* act, int8_t* w, int
  * act [M][F], w [O][F], err [M][O], int8; no operand is re-laid and no int32 product is written to memory.
  * Rounding: NITI_ROUND_NEAREST, NITI_ROUND_PSEUDO_STOCHASTIC, or NITI_ROUND_STOCHASTIC with `rand` (one int32 per
  * OUTPUT element - [M][O], [M][F], [O][F] - low `shift` bits used, as in niti_requant_i32_i8; NULL otherwise).
- * Any shape; operands of forward F % 16 == 0, O % 4 == 0, dgrad O % 32 == 0, F % 32 == 0 and wgrad O % 16 == 0, F % 16 == 0
- * must be 16-byte aligned, others need no alignment.  niti_linear_i8_sync_words returns 0 for results whose workgroups the
- * current device does not hold at once (about 8 M values; then use niti_gemm_i8 + niti_requant_i32_i8 / niti_grad_update_i8).
+ * Any shape.  16-byte alignment is asked of operands and `rand` of dgrad with O % 32 == 0, F % 32 == 0 and of wgrad with O % 16 == 0,
+ * F % 16 == 0 and more than about 4 M results; the kernels that take everything else read any alignment (a misaligned forward is refused
+ * only where its result is too large for them).  niti_linear_i8_sync_words returns 0 for results whose workgroups the current
+ * device does not hold at once (from 4 to 8 M values on, by pass and extents; then use niti_gemm_i8 + niti_requant_i32_i8 /
+ * niti_grad_update_i8).
  * sync, shift_out, exp_* as in niti_fc_i8_*.
  */
 size_t niti_linear_i8_sync_words(int which, int M, int O, int F);

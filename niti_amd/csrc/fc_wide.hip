@@ -398,8 +398,9 @@ __global__ __launch_bounds__(512) void fcw_dgrad_lds_kernel(const FcwArgs a) {
 }
 
 // ---- weight gradient + update -------------------------------------------------------------------------------
-// grid.x = 256-feature tiles, grid.y = groups of T 32-row tiles of the weight matrix.  Samples are walked in chunks of
-// 128.  MFMA A = 32 features x 32 samples (activation columns), B = 32 output features x 32 samples (error columns):
+// For results whose 64- and 128-row tiles are not all resident at once (more than 256 tiles of 128 x 128, 4.2 M values); the others
+// are gemm_any.hip's.  grid.x = 256-feature tiles, grid.y = groups of T 32-row tiles of the weight matrix.  Samples are walked in
+// chunks of 128.  MFMA A = 32 features x 32 samples (activation columns), B = 32 output features x 32 samples (error columns):
 // result element 4 g + e of a lane is feature 8 g + 4 (lane / 32) + e of output feature lane % 32.
 constexpr int kWgActPitch = 256 + 16;   // bytes between samples of the activation tile: eight consecutive samples of
                                         // one 8-byte column fall into eight different bank groups
@@ -645,8 +646,9 @@ long long plan(int which, int M, int O, int F, int* tiles, long long* any) {
     if (which == NITI_FC_DGRAD) *any = any_blocks(which, M, O, F);
     return 0;
   }
-  // Where both sets of kernels cover the shape the ones for any extents take every weight gradient they fit (they share a
-  // 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512 8.6 -> 7.1)
+  // Where both sets of kernels cover the shape the ones for any extents take every weight gradient they fit (up to 256
+  // tiles of 128 x 128; they share a 64- or 128-row tile's staging: 1000 x 1024 -> 2000 with StoShift 23.6 -> 15.8 us, 200 x 2048 -> 512
+  // 8.6 -> 7.1)
   if (which == NITI_FC_WGRAD && *any > 0) return 0;
   if (which == NITI_FC_DGRAD) {
     if (const long long nl = dgrad_lds_blocks(M, O, F)) {
