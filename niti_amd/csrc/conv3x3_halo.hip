@@ -26,27 +26,19 @@
 // this removes 8 of the 9 bytes moved per output element.  The same epilogue can leave the 2x2 / stride-2
 // maximum of its output next to it (the max-pool that follows the layer).
 //
+// Input channels that fill whole slices of 64 have a faster form of the same kernel (conv3x3_k64.h); this one is left with the
+// first layer and other counts whose last slice of 64 would be half empty.
+//
 // Launches the device cannot hold at once: the 64-channel tile takes 512 pixels per workgroup where that
 // is enough (HGeom::TWO); otherwise the launch runs twice without waiting (kRqNoWait, kRqSettle below).
 // Maps of 2 x 2 pixels have a kernel of their own at the end of this file (conv3x3_map2_kernel).
 #include <stdlib.h>
 
-#include "common.h"
-#include "lds_asm.h"
-#include "requant_math.h"
+#include "conv3x3_epilogue.h"
 
 namespace niti {
 namespace {
 
-constexpr int kOob = -1;
-constexpr int kOobFar = static_cast<int>(0x80000000u);   // out of range whatever scalar offset below 2^31 is added
-
-// s_waitcnt vmcnt(N) with the other counters left alone
-template <int N>
-__device__ inline void hc_wait_vmcnt() {
-  static_assert(N >= 0 && N <= 15);
-  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
-}
 // the same for a wavefront that has N loads in flight if it issues the full number of filter loads per stage and
 // N - 1 if it issues one fewer (the count is an immediate, so the choice is a branch on a wavefront-uniform flag)
 template <int N>
@@ -56,12 +48,6 @@ __device__ inline void hc_wait_vmcnt_pair(bool full) {
   else
     hc_wait_vmcnt<N - 1>();
 }
-__device__ inline void hc_sync() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // The four dwords of a fragment, each lane taking its right-hand neighbour's (kLeft: wave_shl:1) or its left-hand
 // neighbour's (wave_shr:1) value - zero where there is none - and-ed with keep.  The shift rides on the AND as its DPP
 // modifier: one instruction per dword where a DPP move followed by the AND would be two.  The compiler does not see
@@ -91,52 +77,6 @@ __device__ inline v4i shifted_and4(v4i x, int keep) {
   return v4i{r0, r1, r2, r3};
 }
 
-struct HaloArgs {
-  const int8_t* x;    // [N,Q,Q,C]
-  const int8_t* wp;   // prepared filter: [ceil(K/64)][cslices][9][64][32], rows XOR-swizzled
-  int32_t* y;         // [N,Q,Q,K]
-  uint32_t* absmax;
-  int N, C, K;
-  int cslices;        // ceil(C / 32)
-  int src_cslices;    // kWT only: 32-channel slices of the forward filter copy read as the data gradient's filter
-  long long x_bytes, wp_bytes, y_bytes;
-  unsigned flags;
-  // requantising variant only
-  int8_t* y8;         // [N,Q,Q,K] int8
-  const int8_t* mask; // optional [N,Q,Q,K] int8: outputs whose mask byte is not positive are stored as zero
-  uint32_t* sync;     // word 0: max |sum| of the launch (output), word 1: set when the wait gave up,
-                      // words kSyncSlot0..: one slot per workgroup, max + 1; all zero on entry
-  long long y8_bytes;
-  int8_t* pool;       // optional [N,Q/2,Q/2,K] int8: 2x2 / stride-2 maximum of y8 (the max-pool that follows the layer)
-  long long pool_bytes;
-  // data gradient through a 2x2 / stride-2 max-pool in front of the layer: `mask` is the pooled map (this launch's
-  // result is the gradient with respect to it), pool_x the pooling's input [N,2Q,2Q,K]; the rounded, masked result
-  // goes to the position(s) of each window that equal the pooled value, into unpool [N,2Q,2Q,K], and y8 is not written
-  const int8_t* pool_x;
-  int8_t* unpool;
-  long long unpool_bytes;
-  int ties_all;
-  int target_bits, method, trunc, bw_mode;
-  const int32_t* rand;   // NITI_ROUND_STOCHASTIC: one random integer per output element [N,Q,Q,K], low `shift` bits used
-  unsigned rq_flags;
-  long long spin_limit;  // wall-clock ticks (100 MHz) the wait may last
-  uint32_t* sticky;      // device-wide word set when the wait gives up, may be null
-  int32_t* shift_out;
-  const int32_t* exp_a;
-  const int32_t* exp_b;
-  int32_t* exp_out;
-};
-constexpr int kSyncSlot0 = 16;
-// A grid with more workgroups than the device holds at once cannot wait for itself.  It runs as two launches of the
-// same kernel instead (set by the launcher in rq_flags, not part of the interface):
-//   kRqNoWait  every workgroup fills its slot (largest magnitude + 1, and next to it the shift it used), stores its
-//              tile rounded with the predicted shift or what its own sums need, and ends;
-//   kRqSettle  every workgroup first reads all slots - final after the first launch -, and ends at once if its tile
-//              was stored with the final shift; otherwise it computes its tile again and stores it with that shift.
-// With a good prediction (the previous training step's shift) the second launch does nothing but look.
-constexpr unsigned kRqNoWait = 1u << 30, kRqSettle = 1u << 31;
-static_assert(kSlotStride >= 2, "the two-launch form keeps the shift a tile was stored with in the word behind its slot");
-constexpr int kMaxSlots = 4096;
 
 // Q: image width = height; BR: output rows of one image per workgroup; NI: images per workgroup; BR*NI*Q == 256.
 // The halo tile is NI*(BR+2) rows of Q slots of 32 bytes; for Q a multiple of 8 the bank of a slot depends on its
@@ -172,6 +112,12 @@ struct HGeom {
   static_assert(NI == 1 || BR == Q, "several images per workgroup only as whole images");
 };
 
+// which four sums of a 32 x 32 product tile a register quad holds
+struct Layout32 {
+  static __device__ int channel(int g, int lane) { return 8 * g + 4 * (lane >> 5); }
+  static __device__ int pixel(int, int lane) { return lane & 31; }
+};
+
 // kWT: the filter operand is the FORWARD copy of the filter of the convolution whose data gradient this launch
 // computes (input channels of this launch = that filter's output channels and vice versa, taps flipped); its
 // 32 x 32 byte blocks are staged as they are and transposed by ds_read_b64_tr_b8 when the fragments are read.
@@ -197,50 +143,16 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
 
   int settle_shift = -1;   // kRqSettle: the final shift, when this workgroup has to store its tile again
   if constexpr (kFused) {
-    if ((a.rq_flags & kRqSettle) != 0) {
-      uint32_t* const slots = a.sync + kSyncSlot0;
-      uint32_t* const words = reinterpret_cast<uint32_t*>(dump);
-      const int nb = gridDim.x * gridDim.y;
-      const int b = blockIdx.y * gridDim.x + blockIdx.x;
-      uint32_t m = 0;
-      for (int i = tid; i < nb; i += 512) m = max(m, __hip_atomic_load(slot_word(slots, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      m = wave_max_u32(m);
-      if (lane == 0) words[wave] = m;
-      __syncthreads();
-      uint32_t g = words[0];
-#pragma unroll
-      for (int w = 1; w < 8; ++w) g = max(g, words[w]);
-      const uint32_t gmax = g != 0u ? g - 1u : 0u;
-      const int fshift = max(bitwidth_of(gmax, a.bw_mode) - a.target_bits, 0);
-      const int used = static_cast<int>(slot_word(slots, b)[1]);
-      if (b == 0 && tid == 0) {
-        a.sync[0] = gmax;
-        if (a.shift_out != nullptr) *a.shift_out = fshift;
-        if (a.exp_out != nullptr) *a.exp_out = fshift + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
-      }
-      if (used == fshift) return;
-      settle_shift = fshift;
-      __syncthreads();   // the words are written again below
-    }
+    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, dump, settle_shift)) return;
   }
+
 
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.x), 0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.wp), 0, a.wp_bytes, 0x00020000);
 
-  // NITI_RQ_SHIFT_HINT: *shift_out holds the caller's prediction (the previous training step's shift of this tensor).
-  // Read here, a whole main loop before it is needed; workgroup (0, 0) overwrites the word only after all slots are
-  // filled, i.e. after every workgroup has passed this line.
-  // The load is unconditional (from the range word when there is no prediction), its address looks lane-dependent to
-  // the compiler and its result is not looked at before the epilogue: a load inside a branch, or one whose result the
-  // compiler knows to be the same in all lanes (and moves to a scalar register at once), would be waited for on the
-  // spot - a trip to memory in front of the first stage's loads.
-  bool hinted = false;
-  int predicted_raw = 0;
-  if constexpr (kFused) {
-    hinted = (a.rq_flags & NITI_RQ_SHIFT_HINT) != 0 && a.shift_out != nullptr && settle_shift < 0;
-    const int32_t* const src = hinted ? a.shift_out : reinterpret_cast<const int32_t*>(a.sync);
-    predicted_raw = __hip_atomic_load(src + opaque_zero(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  ShiftHint hint{false, 0};
+  if constexpr (kFused) hint = halo_shift_hint(a, settle_shift);
+
 
   // ---- activation staging: an instruction fills 32 consecutive slots; lane -> (slot lane/2, half lane%2).
   // A lane's offset is split into a part fixed for the whole launch (vector register) and the slice's 32 * cs
@@ -584,348 +496,18 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
 
   // ---- epilogue: acc[i][j][4g+e] = channel kt*KT + wc*(KT/2) + i*32 + 8g + 4*lk + e of pixel pixbase+wp_*64+j*32+lr
   __builtin_amdgcn_s_setprio(0);
-  const bool roundtrip = (a.flags & NITI_EPI_F32_ROUNDTRIP) != 0;
-  int vmax = 0, vmin = 0;
+  v4i q[NWF * PT * 4];
 #pragma unroll
   for (int i = 0; i < NWF; ++i)
 #pragma unroll
     for (int j = 0; j < PT; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; e += 2) {
-        vmax = max(vmax, max(acc[i][j][e], acc[i][j][e + 1]));
-        vmin = min(vmin, min(acc[i][j][e], acc[i][j][e + 1]));
-      }
-  // The fp32 round trip is the identity up to 2^24, so it is applied (wavefront-uniformly) only beyond; it is
-  // monotonic and odd, so the range after it follows from the extreme values alone, and the sums themselves
-  // are converted where they are consumed below instead of in a second copy of the accumulators.
-  bool rt = false;
-  if (roundtrip) rt = wave_max_u32(max(static_cast<uint32_t>(vmax), 0u - static_cast<uint32_t>(vmin))) > (1u << 24);
-  if (rt) {
-    vmax = f32_roundtrip(vmax);
-    vmin = f32_roundtrip(vmin);
-  }
-  const uint32_t lmax = max(static_cast<uint32_t>(vmax), 0u - static_cast<uint32_t>(vmin));
-  const long long total_pix = static_cast<long long>(a.N) * Q * Q;
-  const int chbase = G::TWO ? kt * KT : kt * KT + wc * (KT / 2);
-  const int pixwave = pixbase + (G::TWO ? wc * 256 : 0) + wp_ * (32 * PT);   // first pixel of this wavefront
-  uint32_t* const red = reinterpret_cast<uint32_t*>(dump);  // behind the tiles, clear of the patches below
-  if constexpr (!kFused) {
-    hc_sync();  // all wavefronts are done with the tiles: reuse LDS as per-wavefront transposition patches
-    constexpr int ROWB = 32 * 4 + 16;  // one 32-channel tile row of int32, padded
-    int8_t* patch = smem + wave * (32 * ROWB);
-    const int rrow = lane >> 3, rcol = lane & 7;  // 8 lanes x 16 bytes = one 32-channel row
-    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
-#pragma unroll
-    for (int j = 0; j < PT; ++j) {
-      const int mrow = pixwave + j * 32 + rrow;
-#pragma unroll
-      for (int i = 0; i < NWF; ++i) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          v4i v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-          if (rt) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = f32_roundtrip(v[e]);
-          }
-          *reinterpret_cast<v4i*>(patch + lr * ROWB + (g * 8 + lk * 4) * 4) = v;
-        }
-        // same wavefront reads back what it wrote: LDS operations of one wavefront complete in order
-        const int ch = chbase + i * 32 + rcol * 4;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const v4i v = *reinterpret_cast<const v4i*>(patch + (t * 8 + rrow) * ROWB + rcol * 16);
-          const int m = mrow + t * 8;
-          const int off = (m < total_pix && ch < a.K) ? (m * a.K + ch) * 4 : kOob;
-          __builtin_amdgcn_raw_buffer_store_b128(v, ry, off, 0, 2);
-        }
-      }
-    }
-    // one atomic per workgroup at most: same-address atomics serialise in the memory system
-    if (a.absmax != nullptr) {
-      const uint32_t wmax = wave_max_u32(lmax);
-      if (lane == 0) red[wave] = wmax;
-      __syncthreads();
-      if (wave == 0) fold_absmax(a.absmax, lane < 8 ? red[lane] : 0u);
-    }
-  } else {
-    // ---- tensor-wide range: workgroup maximum -> own slot -> maximum over the slots of all workgroups.
-    // Results are stored before the range is final: the slots filled so far (read before this workgroup's own
-    // maximum is known, so the latency hides behind that reduction) and the own maximum give a shift that is the
-    // final one unless another workgroup raises the bit width; the int8 stores of all workgroups then overlap the
-    // wait for the last slots instead of following it in one burst.  When the final shift differs, the sums (still
-    // in registers) are rounded and stored once more.
-    const int nb = gridDim.x * gridDim.y;
-    uint32_t* const slots = a.sync + kSyncSlot0;
-    constexpr int kLook = 8;   // slots a lane reads with its loads in flight together
-    const bool nowait = (a.rq_flags & kRqNoWait) != 0;
-    const bool settled = settle_shift >= 0;
-    // Without a prediction, a hint: the first 64 * kLook slots as they are now.  With one the look would only put a
-    // trip to memory between the last product and the first store.
-    uint32_t early[kLook];
-#pragma unroll
-    for (int u = 0; u < kLook; ++u) {
-      const int i = u * 64 + lane;
-      early[u] = (wave == 0 && i < nb && !nowait && !settled && !hinted) ? __hip_atomic_load(slot_word(slots, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-    }
-    const uint32_t wmax = wave_max_u32(lmax);
-    __syncthreads();  // the tiles are dead from here on
-    if (lane == 0) red[wave] = wmax;
-    __syncthreads();
-    if (wave == 0 && !settled) {
-      uint32_t bmax = lane < 8 ? red[lane] : 0u;
-      bmax = wave_max_u32(bmax);
-      const int b = blockIdx.y * gridDim.x + blockIdx.x;
-      if (lane == 0) __hip_atomic_store(slot_word(slots, b), bmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      uint32_t g = bmax + 1u;
-#pragma unroll
-      for (int u = 0; u < kLook; ++u) g = early[u] > g ? early[u] : g;
-      g = wave_max_u32(g);
-      if (lane == 0) {
-        red[8] = g - 1u;
-        red[9] = nb == 1 ? 1u : 0u;
-      }
-    }
-    __syncthreads();
-    // a shift below 1 means "no shift" whatever its value; the prediction counts unless this workgroup's own sums or
-    // the slots seen so far already need more (or the range is final already)
-    int shift = max(bitwidth_of(red[8], a.bw_mode) - a.target_bits, 0);
-    bool final_range = red[9] != 0u;
-    if (!final_range && hinted) shift = max(shift, predicted_raw);
-    if (settled) shift = settle_shift;
-    if (nowait) {   // the shift this tile is stored with, for the settling launch
-      if (tid == 0) slot_word(slots, blockIdx.y * gridDim.x + blockIdx.x)[1] = static_cast<uint32_t>(shift);
-    }
-    final_range = final_range || nowait || settled;
-    const bool trunc = a.trunc != 0;
-    const bool relu = (a.rq_flags & NITI_RQ_RELU) != 0;
-    const bool psto = a.method == NITI_ROUND_PSEUDO_STOCHASTIC;
-    // StoShift: the caller's random integer of each output element decides its rounding step; a tile that is rounded
-    // twice (final shift unlike the first) takes the low bits of the same integers for the other shift
-    constexpr bool sto = kSto;
-    const __amdgpu_buffer_rsrc_t rrand = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(a.rand), 0, sto ? a.y8_bytes * 4 : 0, 0x00020000);
-    constexpr int PROW = NWF * 32 + 16;  // the wavefront's channels of one pixel, padded
-    int8_t* patch = smem + wave * (32 * PT * PROW);
-    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(a.y8, 0, a.y8_bytes, 0x00020000);
-    constexpr int LPP = NWF * 2;       // lanes (16-byte pieces) per pixel
-    constexpr int PPI = 64 / LPP;      // pixels per store instruction
-    const int prow = lane / LPP, piece = lane % LPP;
-    // With the max-pool's backward pass folded in, the two wavefronts that share pixels exchange halves of their patches: each
-    // then writes the windows of 32 pixels at the tile's full width.  At its own width a wavefront wrote every line of the
-    // four times larger result in pieces of 32 (64) bytes, and the lines left the cache half written (16 x 16 -> 32 x 32, 128
-    // channels, 256 images: 46.9 us, 24.7 of them without the folded pass).
-    constexpr bool kPairs = !G::TWO && KT != 32;
-    const bool pairs = kPairs && a.unpool != nullptr;
-    constexpr int LPU = KT / 16, PPU = 64 / LPU;
-    const int mfirst = pairs ? pixbase + wp_ * 64 + wc * 32 + lane / LPU : pixwave + prow;
-    const int mstep = pairs ? PPU : PPI;
-    const int ch = pairs ? kt * KT + lane % LPU * 16 : chbase + piece * 16;
-    const int8_t* const from = pairs ? smem + (wp_ + 4 * (lane % LPU / (KT / 32))) * (32 * PT * PROW) + (wc * 32 + lane / LPU) * PROW + lane % LPU % (KT / 32) * 16
-                                     : patch + prow * PROW + piece * 16;
-    if (rt) {   // once, in place: the values are rounded up to twice below
-#pragma unroll
-      for (int i = 0; i < NWF; ++i)
-#pragma unroll
-        for (int j = 0; j < PT; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] = f32_roundtrip(acc[i][j][e]);
-    }
-    // The mask bytes (ReLU backward of the layer below / the pooled map) do not depend on the rounding: the first two
-    // of the wavefront's pieces are requested here and each later one two pieces ahead of its use, so that they have
-    // arrived when the stores below need them - requested where it is used, every piece would be a trip to memory
-    // between two stores.
-    // (Only where registers allow: the wavefronts with four accumulator tiles are at the 128-register limit of two
-    // workgroups per CU and fetch each piece where it is used.)
-    constexpr int NPIECE = 32 * PT / PPI;
-    constexpr bool kMaskAhead = NWF * PT <= 2;
-    constexpr int MKD = !kMaskAhead ? 1 : (NPIECE < 2 ? NPIECE : 2);
-    v4i mkpre[MKD];
-    auto mask_request = [&](int t) {
-      const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.mask), 0, a.y8_bytes, 0x00020000);
-      const int m = mfirst + t * mstep;
-      const int off = (m < total_pix && ch < a.K) ? m * a.K + ch : kOob;
-      mkpre[t % MKD] = __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0);
-    };
-    // the same for the pooling windows of the folded max-pool backward, one piece ahead
-    v4i xwpre[kMaskAhead ? 4 : 1];
-    auto window_offsets = [&](int t, int (&wo)[4]) {
-      const int m = mfirst + t * mstep;
-      const bool in = m < total_pix && ch < a.K;
-      const int n = m / (Q * Q), rem = m - n * (Q * Q);
-      const int pp = rem / Q, pq = rem - pp * Q;
-      const int rowb = 2 * Q * a.K;
-      const int base = ((n * 2 * Q + 2 * pp) * 2 * Q + 2 * pq) * a.K + ch;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) wo[k] = in ? base + (k >> 1) * rowb + (k & 1) * a.K : kOob;
-    };
-    auto window_request = [&](int t) {
-      if constexpr (kMaskAhead) {
-        const __amdgpu_buffer_rsrc_t rxp = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.pool_x), 0, a.unpool_bytes, 0x00020000);
-        int wo[4];
-        window_offsets(t, wo);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) xwpre[k] = __builtin_amdgcn_raw_buffer_load_b128(rxp, wo[k], 0, 0);
-      }
-    };
-    if (kMaskAhead && a.mask != nullptr) {
-#pragma unroll
-      for (int t = 0; t < MKD; ++t) mask_request(t);
-      if (a.unpool != nullptr) window_request(0);
-    }
-#pragma nounroll
-    for (int pass = 0; pass < 2; ++pass) {
-      // the sums look modified to the compiler in every pass: nothing derived from them (magnitudes, signs) is
-      // computed ahead of the loop and kept in 64 more registers
-#pragma unroll
-      for (int i = 0; i < NWF; ++i)
-#pragma unroll
-        for (int j = 0; j < PT; ++j) asm volatile("" : "+v"(acc[i][j]));
-      // round, pack four channels per dword, transpose through a per-wavefront patch, store 16-byte pieces; the
-      // common rounding mode gets a short form
-      // The shift is the same in every lane but has come through LDS, which the compiler cannot know: made a scalar
-      // here, the choice between the two forms below is ONE scalar branch.  (Left inside the loops as a per-lane
-      // condition it cost every value both forms' set-up under execution masks and a taken branch.)
-      const int ushift = __builtin_amdgcn_readfirstlane(shift);
-      const bool fast = ushift >= 1 && !trunc && !psto && !sto;
-      const int sm1 = ushift - 1, lo = relu ? 0 : -127;
-      auto round_tiles = [&](auto fastc) {
-        constexpr bool kFast = decltype(fastc)::value;
-#pragma unroll
-        for (int j = 0; j < PT; ++j)
-#pragma unroll
-          for (int i = 0; i < NWF; ++i)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              uint32_t packed;
-              if constexpr (kFast) {
-                packed = round4_nearest_floor_fast(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3], sm1, lo);
-              } else {
-                int r[4];
-                v4i u = {0, 0, 0, 0};
-                if (sto) {   // the four values are consecutive channels of one pixel
-                  const int m = pixwave + j * 32 + lr, c0 = chbase + i * 32 + 8 * g + 4 * lk;
-                  u = __builtin_amdgcn_raw_buffer_load_b128(rrand, (m < total_pix && c0 < a.K) ? (m * a.K + c0) * 4 : kOob, 0, 0);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  const int x = acc[i][j][4 * g + e];
-                  if (ushift >= 1)
-                    r[e] = sto    ? round_sto32(x, ushift, trunc, u[e])
-                           : psto ? round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(x, ushift, trunc)
-                                  : round_one32<NITI_ROUND_NEAREST>(x, ushift, trunc);
-                  else r[e] = wrap_to_i8(x);
-                  if (relu && r[e] < 0) r[e] = 0;
-                }
-                packed = pack4_i8(r[0], r[1], r[2], r[3]);
-              }
-              *reinterpret_cast<uint32_t*>(patch + (j * 32 + lr) * PROW + (i * 8 + 2 * g + lk) * 4) = packed;
-            }
-      };
-      if (fast) round_tiles(std::true_type{});
-      else round_tiles(std::false_type{});
-      // same wavefront reads back what it wrote: LDS operations of one wavefront complete in order
-      if (pairs) __syncthreads();
-#pragma unroll
-      for (int t = 0; t < 32 * PT / PPI; ++t) {
-        v4i v = *reinterpret_cast<const v4i*>(from + t * mstep * PROW);
-        const int m = mfirst + t * mstep;
-        const int off = (m < total_pix && ch < a.K) ? m * a.K + ch : kOob;
-        v4i mk;
-        if (a.mask != nullptr) {  // ReLU backward of the layer below, folded in: its output is this layer's input
-          if constexpr (kMaskAhead) {
-            mk = mkpre[t % MKD];
-            if (t + MKD < NPIECE) mask_request(t + MKD);
-          } else {
-            const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.mask), 0, a.y8_bytes, 0x00020000);
-            mk = __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0);
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] &= static_cast<int>(positive_bytes(static_cast<uint32_t>(mk[q])));
-        }
-        if (a.unpool != nullptr) {
-          // max-pool backward folded in (mk holds the pooled values): the window of pooled pixel m in the pooling's input
-          const __amdgpu_buffer_rsrc_t rxp = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.pool_x), 0, a.unpool_bytes, 0x00020000);
-          const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(a.unpool, 0, a.unpool_bytes, 0x00020000);
-          int wo[4];
-          window_offsets(t, wo);
-          v4i xw[4], ow[4];
-          if constexpr (kMaskAhead) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) xw[k] = xwpre[k];
-            if (t + 1 < NPIECE) window_request(t + 1);
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) xw[k] = __builtin_amdgcn_raw_buffer_load_b128(rxp, wo[k], 0, 0);
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            uint32_t taken = 0;   // bytes whose gradient an earlier position of the window (scan order) already received
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const uint32_t eq = equal_bytes(static_cast<uint32_t>(xw[k][q]), static_cast<uint32_t>(mk[q]));
-              const uint32_t keep = a.ties_all != 0 ? eq : eq & ~taken;
-              ow[k][q] = static_cast<int>(static_cast<uint32_t>(v[q]) & keep);
-              taken |= eq;
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) __builtin_amdgcn_raw_buffer_store_b128(ow[k], ru, wo[k], 0, 0);
-        } else {
-          // the 128-channel tile writes 64 bytes per pixel and wavefront: streaming stores start the write-back of the
-          // 16 MiB result while the kernel still runs (measured 2 us per launch); the 32-byte pieces of the 64-channel
-          // tile are slower that way
-          __builtin_amdgcn_raw_buffer_store_b128(v, ry, off, 0, NWF == 2 ? 2 : 0);
-        }
-      }
-      if (a.pool != nullptr) {
-        // The max-pool behind this layer, from the rounded values still in the patch: the wavefront's 64 pixels are a
-        // strip of whole image rows (or whole images), i.e. 16 whole 2 x 2 windows; a lane takes 16 channels of one.
-        constexpr int PC = Q / 2;   // pooled pixels per row
-        const int pq = lane / LPP;
-        if (pq < 8 * PT) {
-          const int l0 = 2 * (pq / PC) * Q + 2 * (pq % PC);   // upper left pixel of the window inside the strip
-          const int8_t* src = patch + l0 * PROW + piece * 16;
-          const v4i p00 = *reinterpret_cast<const v4i*>(src), p01 = *reinterpret_cast<const v4i*>(src + PROW);
-          const v4i p10 = *reinterpret_cast<const v4i*>(src + Q * PROW), p11 = *reinterpret_cast<const v4i*>(src + (Q + 1) * PROW);
-          v4i mx;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            mx[q] = static_cast<int>(max_i8x4(max_i8x4(static_cast<uint32_t>(p00[q]), static_cast<uint32_t>(p01[q])),
-                                              max_i8x4(static_cast<uint32_t>(p10[q]), static_cast<uint32_t>(p11[q]))));
-          const int m0 = pixwave + l0;
-          const int n = m0 / (Q * Q), rem = m0 - n * (Q * Q);
-          const int pr = rem / Q, pcol = rem - pr * Q;
-          const int pix2 = (n * PC + (pr >> 1)) * PC + (pcol >> 1);
-          const int off = (m0 < total_pix && ch < a.K) ? pix2 * a.K + ch : kOob;
-          const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(a.pool, 0, a.pool_bytes, 0x00020000);
-          __builtin_amdgcn_raw_buffer_store_b128(mx, rp, off, 0, 0);
-        }
-      }
-      if (final_range) break;
-      // ---- wait for the slots of all workgroups; the maximum over them is the tensor's range
-      if (wave == 0) {
-        const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
-        if (lane == 0) red[8] = g != 0u ? g - 1u : 0u;
-      }
-      __syncthreads();
-      final_range = true;
-      const int fshift = max(bitwidth_of(red[8], a.bw_mode) - a.target_bits, 0);
-      if (fshift == shift) break;
-      shift = fshift;
-      __builtin_amdgcn_s_waitcnt(0);   // the stores of the first pass leave before those that replace them
-      if (kMaskAhead && a.mask != nullptr) {
-#pragma unroll
-        for (int t = 0; t < MKD; ++t) mask_request(t);
-        if (a.unpool != nullptr) window_request(0);
-      }
-    }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0 && !nowait && !settled) {
-      const int sh = shift > 0 ? shift : 0;
-      a.sync[0] = red[8];
-      if (a.shift_out != nullptr) *a.shift_out = sh;
-      if (a.exp_out != nullptr)
-        *a.exp_out = sh + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
-    }
-  }
+      for (int g = 0; g < 4; ++g)
+        q[(i * PT + j) * 4 + g] = v4i{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+  const HaloPieces<Q, KT, G::TWO, NWF, PT, false> pieces(a, pixbase, kt, wp_, wc);
+  HaloAhead<Q, KT, G::TWO, NWF, PT, false> ahead;
+  halo_epilogue<Q, KT, G::TWO, NWF, PT, kFused, kSto, false, Layout32>(a, q, smem, reinterpret_cast<uint32_t*>(dump), pixbase, kt, wp_, wc, settle_shift, hint,
+                                                                       pieces, ahead);
 }
 
 // ---- 2 x 2 maps -----------------------------------------------------------------------------------------
@@ -1239,12 +821,45 @@ int halo_ktile(long long pix, int K, int H, int C) {
   return (b128 < 2LL * cus && K > 64) ? 64 : 128;
 }
 
+// The kernel of 64-channel slices (conv3x3_k64.h) multiplies a whole number of them: not where the last would be half empty
+// (C up to 32, the first layer, among them).  NITI_HALO_K64=0 pins the kernel of 32-channel slices (tests).
+bool halo_k64(int C) {
+  const char* e = getenv("NITI_HALO_K64");
+  return (C + 31) / 32 % 2 == 0 && (e == nullptr || e[0] != '0');
+}
+
 // The 64-channel tile with 512 pixels per workgroup: where 256-pixel workgroups would be more than the device holds
 // at once (a condition of the requantising variant), on the large maps where such launches occur.
 bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
   if (ktile != 64 || (H != 32 && H != 16)) return false;
   const int cus = compute_units();
   return (pix + 255) / 256 * ((K + 63) / 64) > 2LL * cus;
+}
+
+// Channel tile of the kernel of 64-channel slices: the narrowest that leaves one workgroup on a compute unit at most, which
+// spreads the work over the most units; 128 where even 64-channel workgroups are more than the units.  (128 images, 512 -> 512
+// channels at 8 x 8: 32 / 64 / 128 channels 22.0 / 18.7 / 25.6 us; 256 -> 256 at 16 x 16: 27.2 / 20.2 / 17.4.)
+int k64_ktile(long long pix, int K, int H) {
+  const long long ptiles = (pix + 255) / 256;
+  const int cus = compute_units();
+  const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
+  const int forced = e != nullptr ? atoi(e) : 0;
+  if (forced == 128 || forced == 64 || (forced == 32 && H <= 16)) return forced;
+  if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
+  return K <= 64 || ptiles * ((K + 63) / 64) <= cus ? 64 : 128;
+}
+
+// Which kernel takes a launch, and the pixels and channels of its workgroups.
+struct HaloTile {
+  int channels, pixels;
+  bool k64;
+};
+HaloTile halo_tile(long long pix, int K, int H, int C, bool fused) {
+  const bool k64 = halo_k64(C);
+  const int ktile = k64 ? k64_ktile(pix, K, H) : halo_ktile(pix, K, H, C);
+  // (at 64 channels and more of such workgroups than the device holds, one launch of the other kernel's 512 pixels instead of two)
+  if (fused && halo_two_pixel_tiles(pix, K, H, ktile)) return {ktile, 512, false};
+  return {ktile, 256, k64};
 }
 
 template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto = false>
@@ -1254,40 +869,8 @@ int launch_halo(const HaloArgs& a, hipStream_t stream) {
   static_assert(8 * 32 * (32 * 4 + 16) <= G::TILE_BYTES, "int32 patches must stay clear of the reduction words");
   static_assert(8 * 32 * G::PT * (G::NWF * 32 + 16) <= G::TILE_BYTES, "int8 patches must stay clear of the reduction words");
   static_assert(2 * lds <= 160 * 1024, "two workgroups per compute unit");
-  auto k = conv3x3_halo_kernel<Q, BR, NI, KT, kFused, kWT, kSto>;
-  static bool attr_set_of[kDeviceSlots] = {};   // function attributes are per device
-  static int resident_of[kDeviceSlots] = {};     // workgroups the device holds at once
-  const int slot = device_slot();
-  bool& attr_set = attr_set_of[slot];
-  int& resident = resident_of[slot];
-  if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-      return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot reserve %zu bytes of LDS", lds);
-    if (kFused) {
-      int dev = 0, cus = 0, per_cu = 0;
-      if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k), 512, lds) != hipSuccess)
-        return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot query occupancy");
-      resident = cus * per_cu;
-    }
-    attr_set = true;
-  }
-  const long long pix = static_cast<long long>(a.N) * Q * Q;
-  dim3 grid(static_cast<unsigned>((pix + G::PX - 1) / G::PX), (a.K + KT - 1) / KT);
-  if (kFused && static_cast<long long>(grid.x) * grid.y > resident) {
-    // more workgroups than the device holds at once: nobody waits; a second launch settles the tiles stored with
-    // another shift than the final one
-    if (static_cast<long long>(grid.x) * grid.y > kMaxSlots)
-      return fail(NITI_ERR_UNSUPPORTED, "conv3x3_halo: %u workgroups exceed the %d range slots", grid.x * grid.y, kMaxSlots);
-    HaloArgs b = a;
-    b.rq_flags = a.rq_flags | kRqNoWait;
-    hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, b);
-    b.rq_flags = a.rq_flags | kRqSettle;
-    hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, b);
-    return check_launch("conv3x3_halo");
-  }
-  hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, a);
-  return check_launch("conv3x3_halo");
+  static HaloLaunch state;
+  return launch_halo_kernel<kFused>(conv3x3_halo_kernel<Q, BR, NI, KT, kFused, kWT, kSto>, state, lds, G::PX, KT, Q, a, stream);
 }
 
 inline int map2_blocks(int N, int K) { return ((N + 31) / 32) * ((K + 31) / 32); }
@@ -1335,7 +918,12 @@ int launch_map2(const HaloArgs& a, hipStream_t stream) {
 template <bool kFused, bool kWT, bool kSto = false>
 int launch_halo_tiles(const HaloArgs& a, int H, hipStream_t stream) {
   if (H == 2) return launch_map2<kFused, kWT>(a, stream);
-  const int ktile = halo_ktile(static_cast<long long>(a.N) * H * H, a.K, H, a.C);
+  const HaloTile tile = halo_tile(static_cast<long long>(a.N) * H * H, a.K, H, a.C, kFused);
+  const int ktile = tile.channels;
+  if (tile.k64) {
+    if (!kFused) return launch_conv3x3_k64_int32(a, H, ktile, stream);
+    return kSto ? launch_conv3x3_k64_sto(a, H, ktile, stream) : launch_conv3x3_k64_requant(a, H, ktile, stream);
+  }
   if (ktile == 128) {
     if (H == 32) return launch_halo<32, 8, 1, 128, kFused, kWT, kSto>(a, stream);
     if (H == 16) return launch_halo<16, 16, 1, 128, kFused, kWT, kSto>(a, stream);
@@ -1348,7 +936,7 @@ int launch_halo_tiles(const HaloArgs& a, int H, hipStream_t stream) {
     return launch_halo<4, 4, 16, 32, kFused, kWT, kSto>(a, stream);
   }
   if constexpr (kFused) {
-    if (halo_two_pixel_tiles(static_cast<long long>(a.N) * H * H, a.K, H, ktile)) {
+    if (tile.pixels == 512) {
       if (H == 32) return launch_halo<32, 16, 1, 64, kFused, kWT, kSto>(a, stream);
       return launch_halo<16, 16, 2, 64, kFused, kWT, kSto>(a, stream);
     }
@@ -1429,9 +1017,8 @@ int launch_conv3x3_halo(const int8_t* x, const int8_t* wp, int32_t* y, int N, in
 int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
   if (!conv3x3_halo_supported(N, H, W, C, K, R, S, stride, pad) || K % 16 != 0) return 0;
   const long long pix = static_cast<long long>(N) * H * W;
-  const int ktile = halo_ktile(pix, K, H, C);
-  const long long px = halo_two_pixel_tiles(pix, K, H, ktile) ? 512 : 256;
-  const long long nb = H == 2 ? map2_blocks(N, K) : ((pix + px - 1) / px) * ((K + ktile - 1) / ktile);
+  const HaloTile tile = halo_tile(pix, K, H, C, true);
+  const long long nb = H == 2 ? map2_blocks(N, K) : ((pix + tile.pixels - 1) / tile.pixels) * ((K + tile.channels - 1) / tile.channels);
   return nb <= kMaxSlots ? static_cast<int>(nb) : 0;  // more than the device holds at once run as two launches
 }
 

@@ -42,6 +42,28 @@ def test_conv_sto_tiles(dev, tile, case, monkeypatch):
     base.test_conv_requant_sto(dev, case, "floor")
 
 
+# N, side, C, K: the kernel of 64-channel slices in each of its forms (channel tile, workgroups per compute unit it is made for) on
+# every map: one to five slices, a last one of 48 channels, a last tile of 16 outputs, batches that end inside a tile (five more
+# images); int32, rounded, both filter copies, the mask and the pooling's backward pass, StoShift
+@pytest.mark.parametrize("tile,per_cu", [("32", "1"), ("64", "1"), ("64", "2"), ("128", "1"), ("128", "2")])
+@pytest.mark.parametrize("case", [(2, 32, 64, 144), (1, 32, 304, 64), (3, 16, 112, 80), (4, 8, 256, 192), (16, 4, 64, 272), (32, 4, 192, 128)])
+def test_conv_slices_of_64(dev, case, tile, per_cu, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_KT", tile)
+    monkeypatch.setenv("NITI_HALO_PER_CU", per_cu)
+    N, Q, C, K = case
+    base.test_conv_halo_tiles(dev, case, tile)
+    if Q < 32:
+        base.test_conv_dgrad_requant_unpool(dev, (N, Q, K, C))
+    base.test_conv_requant_sto(dev, case, "floor")
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    g = torch.Generator().manual_seed(N)
+    x, w = ri8(g, N + 5, Q, Q, C), ri8(g, K, 3, 3, C)
+    ref, sh_ref = po.act_calc(po.conv2d_fprop_i32(x, w, 1, 1), 0)
+    y8, sh, sync = ops.conv2d_fprop_requant(x.to(dev), w.to(dev), relu=True, any_shape=True)
+    assert int(sync.cpu()[1]) == 0 and torch.equal(y8.cpu(), ref.clamp(min=0)) and int(sh.cpu()) == sh_ref
+
+
 @pytest.mark.parametrize("case", [(3, 2, 32, 48), (1, 16, 48, 32)])
 def test_conv_dgrad_i32_from_the_forward_copy(dev, case):
     from niti_amd import ops
