@@ -452,8 +452,8 @@ int niti_linear_i8_wgrad_update(const int8_t* err, const int8_t* act, int8_t* w,
  * TiLinear.backward (ti_torch.py:249-266) as one launch: dx8 = err_calc(err @ w) with the weights as they are on entry, then
  * w = clip(w - grad_calc(err^T @ act)).  err_exp_out = error shift + exp_err + exp_w, grad_exp_out = gradient shift +
  * err_exp_out + exp_act.  Roundings as above, the random integers of the error [M][F] and of the gradient [O][F].  Any
- * alignment; niti_linear_i8_backward_sync_words returns 0 where the workgroups of both do not fit on the current device at
- * once (then: the two entry points above).
+ * alignment, 16 bytes for weights of more than 256 tiles of 128 x 128; niti_linear_i8_backward_sync_words returns 0 where the
+ * workgroups of both do not fit on the current device at once (then: the two entry points above).
  */
 size_t niti_linear_i8_backward_sync_words(int M, int O, int F);
 int niti_linear_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int M, int O, int F, int err_bits,

@@ -119,6 +119,35 @@ def test_linear_update_of_wide_layers(dev, case):
         assert torch.equal(wd.cpu(), po.weight_update(w, ref)), method
 
 
+# M, O, F: both gradients as one launch of a workgroup per compute unit - one tile of dx for a quarter of the workgroups, ragged last
+# tiles of both, as many tiles of dx as workgroups (the second with two chunks of samples); one row more: two launches
+@pytest.mark.parametrize("case", [(1, 1024, 8192), (40, 1152, 6272), (128, 1024, 8192), (256, 2048, 4096), (129, 1024, 8192)])
+def test_linear_backward_of_wide_layers(dev, case):
+    from niti_amd import _lib, ops
+    from oracle import niti_oracle as po
+    M, O, F = case
+    base._say("linear_backward_of_wide_layers", case)
+    assert (_lib.lib().niti_linear_i8_backward_sync_words(M, O, F) > 0) == (M != 129)
+    g = torch.Generator().manual_seed(O + M)
+    err, act, w = ri8(g, M, O, lo=-60, hi=60), ri8(g, M, F), ri8(g, O, F)
+    exps = [torch.tensor([e], dtype=torch.int32, device=dev) for e in (-3, -9, -2)]
+    acc_e, acc_g = po.int8mm(err, w), po.int8mm(err.t().contiguous(), act)
+    for err_method, grad_method, div in (("round", "psto", "floor"), ("sto", "sto", "trunc")):
+        drawn = []
+        for acc, bits, method in ((acc_e, 7, err_method), (acc_g, 5, grad_method)):   # wide integers, their low bits for the oracle
+            u = torch.randint(0, 1 << 24, acc.shape, generator=g, dtype=torch.int32)
+            low = u & ((1 << max(po.bitwidth_int(po.absmax(acc)) - bits, 0)) - 1)
+            drawn.append((u.to(dev), low) if method == "sto" else (None, None))
+        wd = w.to(dev)
+        dx, ee, g8, _, sh, ge = ops.linear_backward(err.to(dev), act.to(dev), wd, 7, err_method, 5, grad_method, div, err_rand=drawn[0][0],
+                                                    grad_rand=drawn[1][0], want_grad=True, exp_err=exps[0], exp_w=exps[1], exp_act=exps[2])
+        e_ref, e_shift = po.err_calc(acc_e, err_method, div, rand=drawn[0][1])
+        g_ref, g_shift = po.grad_calc(acc_g, 5, grad_method, div, rand=drawn[1][1])
+        assert torch.equal(dx.cpu(), e_ref) and int(ee.cpu()) == e_shift - 12, err_method
+        assert torch.equal(g8.cpu(), g_ref) and int(sh.cpu()) == g_shift and int(ge.cpu()) == g_shift + e_shift - 14, grad_method
+        assert torch.equal(wd.cpu(), po.weight_update(w, g_ref)), grad_method
+
+
 def test_linear_forward_of_two_sample_tiles(dev):
     """128 rows, a reduction that is no multiple of 128: two tiles of 16 samples per workgroup."""
     from niti_amd import ops
