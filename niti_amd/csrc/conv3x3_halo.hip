@@ -839,14 +839,20 @@ bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
 // Channel tile of the kernel of 64-channel slices: the narrowest that leaves one workgroup on a compute unit at most, which
 // spreads the work over the most units; 128 where even 64-channel workgroups are more than the units.  (128 images, 512 -> 512
 // channels at 8 x 8: 32 / 64 / 128 channels 22.0 / 18.7 / 25.6 us; 256 -> 256 at 16 x 16: 27.2 / 20.2 / 17.4.)
-int k64_ktile(long long pix, int K, int H) {
+// With few slices to walk and wide results two 64-channel workgroups on a unit, which hide each other's way to the first stage and to
+// memory at the end, beat one of 128 channels inside a training step (64 / 128 channels: 128 -> 256 at 16 x 16, 80 and 128
+// images 12.8 / 14.6 and 13.5 / 15.3 us; 256 -> 256, 80 images 19.8 / 20.0, data gradient 19.8 / 20.7; 256 -> 512 at 8 x 8, 256 images
+// 19.6 / 22.8), with eight slices they do not (512 -> 512 at 8 x 8, 256 images 31.1 / 29.6), nor where 128 channels are all there
+// are (the folded pooling's backward pass then writes half lines: 42.6 / 32.6).
+int k64_ktile(long long pix, int K, int H, int C) {
   const long long ptiles = (pix + 255) / 256;
   const int cus = compute_units();
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
   if (forced == 128 || forced == 64 || (forced == 32 && H <= 16)) return forced;
   if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
-  return K <= 64 || ptiles * ((K + 63) / 64) <= cus ? 64 : 128;
+  const long long b64 = ptiles * ((K + 63) / 64);
+  return K <= 64 || b64 <= cus || (C <= 256 && K >= 256 && b64 <= 2LL * cus) ? 64 : 128;
 }
 
 // Which kernel takes a launch, and the pixels and channels of its workgroups.
@@ -856,7 +862,7 @@ struct HaloTile {
 };
 HaloTile halo_tile(long long pix, int K, int H, int C, bool fused) {
   const bool k64 = halo_k64(C);
-  const int ktile = k64 ? k64_ktile(pix, K, H) : halo_ktile(pix, K, H, C);
+  const int ktile = k64 ? k64_ktile(pix, K, H, C) : halo_ktile(pix, K, H, C);
   // (at 64 channels and more of such workgroups than the device holds, one launch of the other kernel's 512 pixels instead of two)
   if (fused && halo_two_pixel_tiles(pix, K, H, ktile)) return {ktile, 512, false};
   return {ktile, 256, k64};
