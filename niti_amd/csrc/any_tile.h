@@ -133,7 +133,7 @@ struct DenseOperand {
 
 // An operand's load(c, raw) is called for c = first, first + 1, ... in turn, piece(raw, i, c, last) once for each of its pieces.
 // Chunks first .. chunks - 1 of the tile at (m0, n0) of the [g.m][g.n] result; int32 sums go to `out`.  shift_of(largest
-// magnitude of the lane, 32 words of LDS): the shift, for the modes that round.
+// magnitude of the lane, 32 words of LDS, requests to send while it waits): the shift, for the modes that round.
 template <class T, class OpA, class OpB, int MODE, class ShiftOf>
 __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, OpA oa, OpB ob, const int m0, const int n0, const int first,
                                          const int chunks, int8_t* const smem, ShiftOf shift_of) {
@@ -296,8 +296,13 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
     }
   }
   // What the rounding reads besides the sums - random integers, old weights, mask, windows - is requested for all of the thread's
-  // results in front of the range exchange: the trip to memory runs while the launch waits for its range (100 x 1000 -> 300
-  // forward and backward pass 14.7 -> 14.4 us).
+  // results behind the workgroup's own slot and in front of the looks at the others': the trip to memory runs while the launch waits
+  // for its range, and neither the requests nor the work on their addresses keep the other workgroups waiting for this slot.  Device
+  // times, us, operands that are in no cache / in the caches, requests behind the exchange -> in front of the slot -> here:
+  //   100 x 1000 -> 300, forward + backward      18.56 / 17.36 -> 17.72 / 16.84 -> 17.76 / 16.84
+  //   the same, StoShift                         19.32 / 17.36 -> 17.60 / 16.72 -> 17.60 / 16.40
+  //   300 x 2000 -> 1000                         41.88 / 38.16 -> 42.23 / 38.39 -> 40.47 / 36.76
+  //   one image through 7 layers (nothing to request)  71.3 / 56.2 -> 72.3 / 57.1 -> 71.0 / 55.6
   v4i rnd[G];
   uint32_t wold[G];
   constexpr bool kUnpool = MODE == kRequant && G <= 4;   // the launches that use it have these tiles
@@ -316,7 +321,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
     const int image = g.by_map.of(row), rest = row - image * (g.map_h * g.map_w), h = g.by_map_w.of(rest), w = rest - h * g.map_w;
     return (static_cast<long long>(image * 2 * g.map_h + 2 * h) * (2 * g.map_w) + 2 * w) * g.n + col;
   };
-  if (MODE != kInt32) {
+  auto request = [&] {
 #pragma unroll
     for (int i = 0; i < G; ++i) {
       const int t = tid + i * 512;
@@ -336,7 +341,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
         }
       }
     }
-  }
+  };
   uint32_t* const words = reinterpret_cast<uint32_t*>(smem + any_lds_bytes<T, OpA, OpB>() - 32 * 4);
   int shift = 0;
   if (MODE == kInt32) {
@@ -347,7 +352,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
       if (wave == 0) fold_absmax(g.absmax, lane < 8 ? words[lane] : 0u);
     }
   } else {
-    shift = shift_of(lmax, words);
+    shift = shift_of(lmax, words, request);
   }
   const bool trunc = g.trunc != 0, relu = (g.rq_flags & NITI_RQ_RELU) != 0;
 #pragma unroll

@@ -26,7 +26,7 @@ template <class T, ConvPass PASS, int MODE>
 __global__ __launch_bounds__(512) void conv_any_kernel(const ConvAnyArgs a) {
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   conv_any_tile<T, PASS, MODE>(a, (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, gridDim.x, gridDim.y, gridDim.z, smem,
-                               [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(a.g, lmax, words, words + 8); });
+                               [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift<8>(a.g, lmax, words, words + 8, meanwhile); });
 }
 
 // workgroups of this kernel the device holds at once; 0: cannot be launched

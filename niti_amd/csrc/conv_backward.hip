@@ -19,11 +19,11 @@ __global__ __launch_bounds__(512, 4) void conv_backward_kernel(const ConvAnyArgs
   const int id = blockIdx.x;
   if (id < nd) {
     conv_any_tile<TD, kConvDgrad, kRequant>(d, id, (d.g.n + TD::BN - 1) / TD::BN, (d.g.m + TD::BM - 1) / TD::BM, 1, smem,
-                                            [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(d.g, lmax, words, words + 8, id, nd); });
+                                            [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift<8>(d.g, lmax, words, words + 8, id, nd, meanwhile); });
   } else {
     const int nw = static_cast<int>(gridDim.x) - nd;
     conv_any_tile<TW, kConvWgrad, MODE>(w, id - nd, (w.g.n + TW::BN - 1) / TW::BN, (w.g.m + TW::BM - 1) / TW::BM, slices, smem,
-                                        [&](uint32_t lmax, uint32_t* words) { return grid_shift_behind<8>(w.g, d.g, nd, lmax, words, words + 8, id - nd, nw); });
+                                        [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift_behind<8>(w.g, d.g, nd, lmax, words, words + 8, id - nd, nw, meanwhile); });
   }
 }
 

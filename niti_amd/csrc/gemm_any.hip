@@ -38,7 +38,7 @@ template <class T, bool TA, bool TB, int MODE, bool kAligned>
 __global__ __launch_bounds__(512) void gemm_any_kernel(const AnyArgs g) {
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   gemm_any_tile<T, TA, TB, MODE, kAligned>(g, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y, smem,
-                                           [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(g, lmax, words, words + 8); });
+                                           [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift<8>(g, lmax, words, words + 8, meanwhile); });
 }
 
 // TiLinear's backward pass as one launch: the first `nd` workgroups take the data gradient, the others the weight gradient and
@@ -51,11 +51,11 @@ __global__ __launch_bounds__(512, kAligned || TW::BM < 128 ? 4 : 2) void gemm_ba
   const int id = blockIdx.x;
   if (id < nd) {
     gemm_any_tile<TD, false, false, kRequant, kAligned>(d, id, (d.n + TD::BN - 1) / TD::BN, (d.m + TD::BM - 1) / TD::BM, smem,
-                                                        [&](uint32_t lmax, uint32_t* words) { return grid_shift<8>(d, lmax, words, words + 8, id, nd); });
+                                                        [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift<8>(d, lmax, words, words + 8, id, nd, meanwhile); });
   } else {
     const int nw = static_cast<int>(gridDim.x) - nd;
     gemm_any_tile<TW, true, false, kUpdate, kAligned>(w, id - nd, (w.n + TW::BN - 1) / TW::BN, (w.m + TW::BM - 1) / TW::BM, smem,
-                                                      [&](uint32_t lmax, uint32_t* words) { return grid_shift_behind<8>(w, d, nd, lmax, words, words + 8, id - nd, nw); });
+                                                      [&](uint32_t lmax, uint32_t* words, auto meanwhile) { return grid_shift_behind<8>(w, d, nd, lmax, words, words + 8, id - nd, nw, meanwhile); });
   }
 }
 

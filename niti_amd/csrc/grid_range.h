@@ -41,10 +41,15 @@ __device__ inline void write_scalars(const Args& a, uint32_t gmax, int shift) {
   if (a.exp_out != nullptr) *a.exp_out = sh + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
 }
 
+struct Nothing {
+  __device__ void operator()() const {}
+};
+
 // The workgroup's shift from every wavefront's largest magnitude: wmax[] holds one word per wavefront, gshare the result.
-// `block` of `blocks` workgroups take part.
-template <int NWAVES, class Args>
-__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare, int block, int blocks) {
+// `block` of `blocks` workgroups take part.  meanwhile(): called by every wavefront behind the workgroup's own slot and in front of
+// the looks at the others', for requests whose trip to memory may run beside the exchange.
+template <int NWAVES, class Args, class Meanwhile = Nothing>
+__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare, int block, int blocks, Meanwhile meanwhile = {}) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   lmax = wave_max_u32(lmax);
@@ -53,6 +58,9 @@ __device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, u
   if (wave == 0) {
     const uint32_t b = wave_max_u32(lane < NWAVES ? wmax[lane] : 0u);
     if (lane == 0) __hip_atomic_store(slot_word(a.sync + kSlot0, block), b + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  meanwhile();
+  if (wave == 0) {
     const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &a.sync[1], a.sticky);
     if (lane == 0) *gshare = g != 0u ? g - 1u : 0u;
   }
@@ -62,17 +70,17 @@ __device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, u
   if (block == 0 && threadIdx.x == 0) write_scalars(a, gmax, shift);
   return shift;
 }
-template <int NWAVES, class Args>
-__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare) {
-  return grid_shift<NWAVES>(a, lmax, wmax, gshare, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+template <int NWAVES, class Args, class Meanwhile = Nothing>
+__device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, uint32_t* gshare, Meanwhile meanwhile = {}) {
+  return grid_shift<NWAVES>(a, lmax, wmax, gshare, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y, meanwhile);
 }
 
 // A weight update next to the data gradient `first` that reads the old weights, in one launch: the update's workgroups wait for
 // both ranges - a workgroup of the data gradient fills its slot when it has read its weights - and the gradient's exponent
-// builds on the error's that comes out of this launch.  share: two words.
-template <int NWAVES, class Args>
+// builds on the error's that comes out of this launch.  share: two words.  meanwhile(): see grid_shift.
+template <int NWAVES, class Args, class Meanwhile>
 __device__ inline int grid_shift_behind(const Args& a, const Args& first, int first_blocks, uint32_t lmax, uint32_t* wmax, uint32_t* share, int block,
-                                        int blocks) {
+                                        int blocks, Meanwhile meanwhile) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   lmax = wave_max_u32(lmax);
@@ -81,6 +89,9 @@ __device__ inline int grid_shift_behind(const Args& a, const Args& first, int fi
   if (wave == 0) {
     const uint32_t b = wave_max_u32(lane < NWAVES ? wmax[lane] : 0u);
     if (lane == 0) __hip_atomic_store(slot_word(a.sync + kSlot0, block), b + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  meanwhile();
+  if (wave == 0) {
     const uint32_t f = wait_slots(first.sync + kSlot0, first_blocks, a.spin_limit, &a.sync[1], a.sticky);
     const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &a.sync[1], a.sticky);
     if (lane == 0) {
