@@ -64,6 +64,74 @@ def test_conv_slices_of_64(dev, case, tile, per_cu, monkeypatch):
     assert int(sync.cpu()[1]) == 0 and torch.equal(y8.cpu(), ref.clamp(min=0)) and int(sh.cpu()) == sh_ref
 
 
+# N, side, C, K: more workgroups of the same kernel than the device holds at once, two launches of which the second settles the shift
+# (tiles of 128 channels, of 64 on small maps; the layers' data gradients where the forward pass has an odd number of 32-channel
+# slices): right, wrong and absurd predictions, StoShift, and nearly every tile stored again
+TWO_LAUNCHES = [(65, 32, 64, 144), (172, 16, 272, 64), (2052, 8, 64, 64)]
+
+
+@pytest.mark.parametrize("case", TWO_LAUNCHES)
+def test_conv_slices_of_64_on_a_grid_larger_than_the_device(dev, case):
+    base.test_conv_requant_predicted_shift(dev, case)
+
+
+@pytest.mark.parametrize("case", TWO_LAUNCHES)
+def test_conv_slices_of_64_on_a_grid_larger_than_the_device_sto(dev, case):
+    base.test_conv_requant_sto(dev, case, "floor")
+
+
+# N, side of the pooled map, channels, reduction
+@pytest.mark.parametrize("case", [(172, 16, 272, 64), (2052, 8, 64, 64)])
+def test_conv_slices_of_64_unpooling_on_a_grid_larger_than_the_device(dev, case):
+    base.test_conv_dgrad_requant_unpool(dev, case)
+
+
+@pytest.mark.parametrize("forward", [True, False])
+def test_conv_slices_of_64_stored_again(dev, forward):
+    """One image with large values among images of tiny ones: the settling launch computes nearly every tile again, with the pooled
+    output, with the mask of a ReLU below and from both filter copies."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = 65, 32, 64, 144
+    base._say("conv_slices_of_64_stored_again", forward)
+    g = torch.Generator().manual_seed(6161)
+    x = ri8(g, N, Q, Q, C, lo=-1, hi=1)
+    x[31] = ri8(g, Q, Q, C)
+    if forward:
+        w = ri8(g, K, 3, 3, C)
+        acc = po.conv2d_fprop_i32(x, w, 1, 1)
+        ref, sh_ref = po.act_calc(acc, 0)
+        pooled = torch.empty((N, Q // 2, Q // 2, K), dtype=torch.int8, device=dev)
+        y, sh, sync = ops.conv2d_fprop_requant(x.to(dev), w.to(dev), relu=True, pool_out=pooled)
+        assert int(sync.cpu()[1]) == 0 and int(sync.cpu()[0]) == po.absmax(acc) and int(sh.cpu()) == sh_ref
+        assert torch.equal(y.cpu(), ref.clamp(min=0)) and torch.equal(pooled.cpu(), po.maxpool_fwd(ref.clamp(min=0)))
+        return
+    w = ri8(g, C, 3, 3, K)          # the error map has C channels, the result K
+    acc = co.conv_dgrad(x, w, Q, Q, 1, 1)
+    ref, sh_ref = po.err_calc(acc)
+    mask = ri8(g, N, Q, Q, K)
+    wf = ops.conv_filter_prepare(w.to(dev), N, Q, Q)
+    for kw in (dict(), dict(forward_filter=wf)):
+        y, sh, sync = ops.conv2d_dgrad_requant(x.to(dev), w.to(dev), relu_mask=mask.to(dev), **kw)
+        assert int(sync.cpu()[1]) == 0 and int(sh.cpu()) == sh_ref
+        assert torch.equal(y.cpu(), torch.where(mask > 0, ref, torch.zeros_like(ref)))
+
+
+# the kernel of 32-channel slices on an even number of them, which the dispatch gives to the other one
+@pytest.mark.parametrize("tile", ["auto", "32", "64", "128"])
+@pytest.mark.parametrize("case", [(2, 32, 64, 144), (3, 16, 128, 80), (8, 8, 256, 64), (16, 4, 64, 272)])
+def test_conv_slices_of_32_in_pairs(dev, case, tile, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "0")
+    if tile != "auto":
+        monkeypatch.setenv("NITI_HALO_KT", tile)
+    N, Q, C, K = case
+    base.test_conv_halo_tiles(dev, case, tile)
+    if Q < 32:
+        base.test_conv_dgrad_requant_unpool(dev, (N, Q, K, C))
+    base.test_conv_requant_sto(dev, case, "trunc")
+
+
 @pytest.mark.parametrize("case", [(3, 2, 32, 48), (1, 16, 48, 32)])
 def test_conv_dgrad_i32_from_the_forward_copy(dev, case):
     from niti_amd import ops
