@@ -822,7 +822,11 @@ int halo_ktile(long long pix, int K, int H, int C) {
 }
 
 // The kernel of 64-channel slices (conv3x3_k64.h) multiplies a whole number of them: not where the last would be half empty
-// (C up to 32, the first layer, among them).  NITI_HALO_K64=0 pins the kernel of 32-channel slices (tests).
+// (C up to 32, the first layer, among them).  Its time with a whole slice more, i.e. at most what a half-empty one would cost, against the
+// kernel of 32-channel slices at 3 / 5 / 7 / 9 of those (16 to 256 images of 8 x 8 to 32 x 32, 64 to 512 filters): that kernel takes 0.86 /
+// 0.97 / 1.01 / 1.04 of it at the median (0.78 to 0.94, 0.93 to 1.09, 0.96 to 1.10, 0.98 to 1.11; data gradients 0.02 more), so up to five
+// slices it is the faster one and from seven on little is lost.  At 4 / 6 / 8 / 10 slices the kernel of 64-channel slices takes 0.99 / 0.95 /
+// 0.93 / 0.92 of the other's time.  NITI_HALO_K64=0 pins the kernel of 32-channel slices (tests).
 bool halo_k64(int C) {
   const char* e = getenv("NITI_HALO_K64");
   return (C + 31) / 32 % 2 == 0 && (e == nullptr || e[0] != '0');
@@ -837,13 +841,21 @@ bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
 }
 
 // Channel tile of the kernel of 64-channel slices: the narrowest that leaves one workgroup on a compute unit at most, which
-// spreads the work over the most units; 128 where even 64-channel workgroups are more than the units.  (128 images, 512 -> 512
-// channels at 8 x 8: 32 / 64 / 128 channels 22.0 / 18.7 / 25.6 us; 256 -> 256 at 16 x 16: 27.2 / 20.2 / 17.4.)
-// With few slices to walk and wide results two 64-channel workgroups on a unit, which hide each other's way to the first stage and to
-// memory at the end, beat one of 128 channels inside a training step (64 / 128 channels: 128 -> 256 at 16 x 16, 80 and 128
-// images 12.8 / 14.6 and 13.5 / 15.3 us; 256 -> 256, 80 images 19.8 / 20.0, data gradient 19.8 / 20.7; 256 -> 512 at 8 x 8, 256 images
-// 19.6 / 22.8), with eight slices they do not (512 -> 512 at 8 x 8, 256 images 31.1 / 29.6), nor where 128 channels are all there
-// are (the folded pooling's backward pass then writes half lines: 42.6 / 32.6).
+// spreads the work over the most units.  (128 images, 512 -> 512 channels at 8 x 8: 32 / 64 / 128 channels 22.0 / 18.7 / 25.6 us;
+// 256 -> 256 at 16 x 16: 27.2 / 20.2 / 17.4.)  Where even 64-channel workgroups are more than the units:
+//  - 64 channels, two on a unit, where 128-channel ones would be more than the units too.  Then the last of them are half empty
+//    (64 K filters by an odd number), and two on a unit walk in turn what one and a half would: 64 / 128 channels, C from 64 to 512,
+//    162 images of 16 x 16 to 160 filters 0.86 to 0.73 of the time (448 -> 160 30.9 / 42.5 us), 192 and 320 filters 0.89 to 0.72, the same
+//    at 8 x 8 and 32 x 32, data gradients alike.  With 128-channel workgroups on two thirds of the units the two are within 8%.
+//  - Otherwise 128.  Alone, on operands that a copy has just written, one such workgroup per unit beats two of 64 channels by 2 to 13%
+//    (data gradients 7 to 30%) over C = 64 .. 512, K = 128 .. 512.  Inside a training step the two of 64 hide each other's way to the
+//    first stage and to memory: with few slices and wide results they are ahead there (128 -> 256 at 16 x 16, 80 and 128 images 12.8 / 14.6
+//    and 13.5 / 15.3 us; 256 -> 512 at 8 x 8, 256 images 19.6 / 22.8).  Chains of eight layers stepped as a graph, us a launch that the
+//    64-channel tile takes longer than the other, 1.3 and 1.95 workgroups of 64 channels per unit: to 256 filters at 16 x 16, C = 64 -0.9 -0.3,
+//    128 -0.5 -0.1, 256 -1.0 -0.5, 320 0.0 -0.5, 384 -0.3 +2.6; to 512 at 8 x 8, C = 64 -2.0 -1.6, 128 -1.2 0.0, 256 -0.2 -0.5, 320 -0.2 +3.8,
+//    384 +0.4 +2.0, 512 +1.0 +0.2; to 256 at 32 x 32, C = 64 -1.2 -0.3, 128 -1.6 +0.2, 256 -1.4 +0.4; to 128 filters at 16 x 16, C = 128 +0.1 +2.9,
+//    256 -1.5 +0.8; single figures repeat within 0.7.  128 channels are also all there are where the folded pooling's backward pass
+//    would write half lines (42.6 / 32.6).
 int k64_ktile(long long pix, int K, int H, int C) {
   const long long ptiles = (pix + 255) / 256;
   const int cus = compute_units();
@@ -852,7 +864,8 @@ int k64_ktile(long long pix, int K, int H, int C) {
   if (forced == 128 || forced == 64 || (forced == 32 && H <= 16)) return forced;
   if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
   const long long b64 = ptiles * ((K + 63) / 64);
-  return K <= 64 || b64 <= cus || (C <= 256 && K >= 256 && b64 <= 2LL * cus) ? 64 : 128;
+  const long long b128 = ptiles * ((K + 127) / 128);
+  return K <= 64 || b64 <= cus || (b64 <= 2LL * cus && (b128 > cus || (C <= 256 && K >= 256))) ? 64 : 128;
 }
 
 // Which kernel takes a launch, and the pixels and channels of its workgroups.

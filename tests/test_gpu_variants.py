@@ -118,6 +118,13 @@ def test_conv_slices_of_64_stored_again(dev, forward):
         assert torch.equal(y.cpu(), torch.where(mask > 0, ref, torch.zeros_like(ref)))
 
 
+# more 128-channel workgroups than compute units, fewer 64-channel ones than twice those: an odd number of 64-channel groups, the last
+# of 32 and of 64 channels; forward, then data gradient
+@pytest.mark.parametrize("case", [(130, 16, 64, 160), (130, 16, 160, 64), (344, 8, 64, 320)])
+def test_conv_slices_of_64_two_workgroups_per_unit(dev, case):
+    base.test_conv_halo_tiles(dev, case, "auto")
+
+
 # the kernel of 32-channel slices on an even number of them, which the dispatch gives to the other one
 @pytest.mark.parametrize("tile", ["auto", "32", "64", "128"])
 @pytest.mark.parametrize("case", [(2, 32, 64, 144), (3, 16, 128, 80), (8, 8, 256, 64), (16, 4, 64, 272)])
