@@ -307,13 +307,13 @@ extern "C" int niti_sync_timeouts(uint32_t* flag_out, int clear, void* stream) {
 }
 
 // `any`: also batches that are no whole tiles (the entry points refuse those unless NITI_RQ_ANY_SHAPE asks for them)
-static int fused_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad, bool any) {
+static int fused_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, int dgrad, bool any, double* us = nullptr) {
   if (halo_off()) return 0;
   if (!any && !(H == 2 && W == 2) && static_cast<long long>(N) * H * W % 256 != 0) return 0;
-  if (!dgrad) return conv3x3_halo_requant_blocks(N, H, W, C, K, R, S, stride, pad);
+  if (!dgrad) return conv3x3_halo_requant_blocks(N, H, W, C, K, R, S, stride, pad, us);
   if (stride != 1 || R != S || pad > R - 1) return 0;
   const int P = H + 2 * pad - R + 1, Q = W + 2 * pad - S + 1;
-  return conv3x3_halo_requant_blocks(N, P, Q, K, C, R, S, 1, R - 1 - pad);
+  return conv3x3_halo_requant_blocks(N, P, Q, K, C, R, S, 1, R - 1 - pad, us);
 }
 
 extern "C" size_t niti_conv2d_i8_requant_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad,
@@ -330,18 +330,22 @@ extern "C" size_t niti_conv2d_i8_requant_sync_words_any(int N, int H, int W, int
   return nb > 0 ? conv3x3_halo_sync_words(nb) : conv_any_requant_words(dgrad ? kConvDgrad : kConvForward, {N, H, W, C, K, R, S, stride, pad});
 }
 
-// Few images on the 3x3 kernels' maps: their workgroups of 256 pixels leave most of the chip idle and walk all input channels
-// (stages of 32, longer on the wider maps), where the kernel for any shape has 32 x 32 tiles.  One image: 32 x 32, 128 -> 128
-// 8.3 against 6.2 us, 16 x 16, 256 -> 256 11.3 / 7.0, 8 x 8, 512 -> 512 12.9 / 8.6; 24 images of the latter 13.4 / 15.5.
+// Few images on the 3x3 kernels' maps: their workgroups of 256 pixels leave most of the chip idle and walk all input channels, where the
+// kernel for any shape has 32 x 32 tiles.  Both are estimated.  Measured (that kernel / the 3x3 one, us, eight layers in a graph): one image
+// of 32 x 32, 128 -> 128 7.1 / 9.0; 16 x 16, 256 -> 256 9.0 / 9.1; 8 x 8, 512 -> 512 11.0 / 12.3; 24 images of the latter 18.1 / 14.1.  Over 700 drawn
+// layers of 4 x 4 to 32 x 32 (16 to 512 channels, at most one workgroup per unit) the estimate's choice is 0.3% off the faster of the two on
+// the geometric mean and 12% at most (400 further ones: 0.3 and 10%); always the 3x3 kernel 8%.
 extern "C" size_t niti_conv2d_i8_fprop_small_sync_words(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
   if (N <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || R <= 0 || S <= 0 || stride <= 0 || pad < 0 || K % 4 != 0) return 0;
   const ConvShape s{N, H, W, C, K, R, S, stride, pad};
   const char* e = getenv("NITI_FPROP_SMALL");   // 0 / 1 pins (tests)
   if (e != nullptr) return e[0] != '0' ? conv_any_requant_words(kConvForward, s) : 0;
-  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0, true);
+  double own = 0.0;
+  const int nb = fused_blocks(N, H, W, C, K, R, S, stride, pad, 0, true, &own);
   if (nb == 0 || nb > compute_units()) return 0;
-  const double us = conv_any_forward_us(s);
-  return us > 0.0 && us < 0.9 * conv3x3_halo_us(H, C) ? conv_any_requant_words(kConvForward, s) : 0;
+  size_t words = 0;
+  const double us = conv_any_forward_us(s, &words);
+  return us > 0.0 && us < own ? words : 0;
 }
 
 static int conv_requant(const char* who, int dgrad, const int8_t* x, const int8_t* w, int8_t* y8, int N, int H, int W, int C,
@@ -682,14 +686,17 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
 }
 
 // Whether both gradients in one launch are the faster way.  Outside the 3x3 kernels' maps they are wherever they fit; there the
-// data gradient's own kernel (its stages of 32 channels, longer on the wider maps) and the weight gradient's are estimated.
+// data gradient's own kernel and the weight gradient's are estimated.  0.8: the one launch's estimate is 0.85 of its measured time on the
+// average (0.14 rms), the other two's 1.04 (0.09).  Over 500 drawn layers of 4 x 4 to 32 x 32 (16 to 512 channels) the choice is 0.2% off the
+// faster way on the geometric mean (300 further ones: 0.6%, seven by 10 to 26%); 0.75 / 0.85 / 0.9: 0.6 / 0.3 / 0.5%.
 static bool backward_together(const ConvShape& s) {
   const char* e = getenv("NITI_BACKWARD_TOGETHER");   // 0 / 1 pins (tests)
   if (e != nullptr) return e[0] != '0';
   const double us = conv_backward_us(s);
   if (us == 0.0) return false;
-  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad))
-    return us < 0.8 * (conv3x3_halo_us(s.H, s.K) + wgrad3x3_us(s.N, s.H, s.C, s.K));
+  double dgrad = 0.0;
+  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad))
+    return us < 0.8 * (dgrad + wgrad3x3_us(s.N, s.H, s.C, s.K));
   const double d = conv_any_dgrad_us(s), w = conv_any_wgrad_us(s);
   return d == 0.0 || us < d + w;
 }

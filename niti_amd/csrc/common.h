@@ -223,7 +223,6 @@ int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, in
 // 3x3 / stride 1 / pad 1 forward kernel with LDS-resident activation halo (conv3x3_halo.hip)
 bool conv3x3_halo_supported(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 size_t conv3x3_halo_filter_bytes(int C, int K);
-double conv3x3_halo_us(int H, int C);   // estimated time with rounding of a launch of at most one workgroup per compute unit
 int launch_halo_filter_prepare(const int8_t* w, int8_t* dst, int kout, int cin, int mode, hipStream_t stream);
 int launch_conv3x3_halo(const int8_t* x, const int8_t* wp, int32_t* y, int N, int H, int C, int K, unsigned flags,
                         uint32_t* absmax, hipStream_t stream);
@@ -276,7 +275,7 @@ bool wgrad_small_shape(int N, int H, int W, int C, int K, int R, int S, int stri
 bool wgrad_small_supported(int N, int H, int C, int K, int w_channels);
 int launch_wgrad_small_update(const int8_t* act, const int8_t* err, int8_t* w, int N, int H, int C, int K, bool roundtrip,
                               uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream);
-int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
+int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, double* us = nullptr);
 size_t conv3x3_halo_sync_words(int blocks);
 int launch_conv3x3_halo_requant(const int8_t* x, const int8_t* wp, int8_t* y8, int N, int H, int C, int K, unsigned flags,
                                 uint32_t* sync, const RequantSpec& rq, hipStream_t stream);

@@ -991,6 +991,22 @@ void fill_common(HaloArgs& a, const int8_t* x, const int8_t* wp, int N, int H, i
   a.flags = flags;
 }
 
+// Estimated time of a launch with rounding: start, a slice's walk times the slices (in turns where a compute unit has several
+// workgroups), and what more workgroups on the device cost (their range, lines and stores).  Least squares over 700 launches in replayed
+// graphs of eight layers, 1 to 256 images of 4 x 4 to 32 x 32, 16 to 512 channels on both sides: 4% rms, from 0.90 to 1.21 of the measured
+// time; 2 x 2 maps 150 launches, 0.5 us rms.  (The 128-channel tile of the kernel of 32-channel slices is taken as two of 64: its launches
+// are far from every line this decides.)
+double requant_us(const HaloTile& tile, int blocks, int H, int C) {
+  constexpr double kStart64[3] = {5.4, 5.6, 4.5}, kSlice64[3] = {0.93, 1.44, 3.02}, kFill64[3] = {3.1, 3.5, 6.0};   // 32, 64, 128 channels
+  constexpr double kStart32[3] = {4.5, 4.8, 4.8}, kSlice32[3] = {0.69, 0.96, 1.92}, kFill32[3] = {2.8, 2.8, 5.6};
+  const double fill = static_cast<double>(blocks) / compute_units();
+  if (H == 2) return 5.7 + 0.24 * ((C + 31) / 32) + 3.6 * fill;
+  const double turns = fill <= 1.0 ? 1.0 : fill <= 2.0 ? 2.0 : fill;
+  const int i = tile.channels == 32 ? 0 : tile.channels == 64 ? 1 : 2;
+  if (tile.k64) return kStart64[i] + kSlice64[i] * turns * ((C + 63) / 64) + kFill64[i] * fill;
+  return kStart32[i] + kSlice32[i] * turns * (tile.pixels / 256) * ((C + 31) / 32) + kFill32[i] * fill;
+}
+
 }  // namespace
 
 bool conv3x3_halo_supported(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
@@ -1004,10 +1020,6 @@ bool conv3x3_halo_supported(int N, int H, int W, int C, int K, int R, int S, int
   if (conv3x3_halo_filter_bytes(C, K) >= 0x7fffffffULL) return false;
   return true;
 }
-
-// A workgroup walks the input channels in stages of 32, whose length the map's width decides: within 6% of the launches of 1 and 24
-// images listed beside niti_conv2d_i8_fprop_small_sync_words (api.hip).
-double conv3x3_halo_us(int H, int C) { return 3.5 + (H >= 32 ? 1.25 : H == 16 ? 1.05 : 0.62) * ((C + 31) / 32); }
 
 size_t conv3x3_halo_filter_bytes(int C, int K) {
   return static_cast<size_t>((K + 63) / 64) * ((C + 31) / 32) * 9 * 64 * 32;
@@ -1032,12 +1044,13 @@ int launch_conv3x3_halo(const int8_t* x, const int8_t* wp, int32_t* y, int N, in
   return launch_halo_any<false>(a, H, stream);
 }
 
-// Workgroups of a launch of the requantising variant (= sync slots), or 0 when the variant cannot run the shape.
-int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad) {
+// Workgroups of a launch of the requantising variant (= sync slots), or 0 when the variant cannot run the shape.  us: its estimated time.
+int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S, int stride, int pad, double* us) {
   if (!conv3x3_halo_supported(N, H, W, C, K, R, S, stride, pad) || K % 16 != 0) return 0;
   const long long pix = static_cast<long long>(N) * H * W;
   const HaloTile tile = halo_tile(pix, K, H, C, true);
   const long long nb = H == 2 ? map2_blocks(N, K) : ((pix + tile.pixels - 1) / tile.pixels) * ((K + tile.channels - 1) / tile.channels);
+  if (us != nullptr) *us = nb <= kMaxSlots ? requant_us(tile, static_cast<int>(nb), H, C) : 0.0;
   return nb <= kMaxSlots ? static_cast<int>(nb) : 0;  // more than the device holds at once run as two launches
 }
 

@@ -18,7 +18,7 @@ bool conv_any_shape(ConvPass pass, const ConvShape& s);   // extents and channel
 int launch_conv_any(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int32_t* y, bool roundtrip, uint32_t* absmax, hipStream_t stream);
 // the same rounded to int8 in the launch: sync words, 0 when no tile's grid is resident at once
 size_t conv_any_requant_words(ConvPass pass, const ConvShape& s);
-double conv_any_forward_us(const ConvShape& s);   // estimated time of the forward pass with rounding, 0: does not run
+double conv_any_forward_us(const ConvShape& s, size_t* words);   // estimated time of the forward pass with rounding and its sync words, 0: does not run
 double conv_any_dgrad_us(const ConvShape& s);   // estimated time of the data gradient with rounding, 0: does not run
 int launch_conv_any_requant(ConvPass pass, const ConvShape& s, const int8_t* a, const int8_t* b, int8_t* y, bool roundtrip, uint32_t* sync,
                             const RequantSpec& rq, hipStream_t stream);

@@ -199,14 +199,21 @@ size_t conv_any_requant_words(ConvPass pass, const ConvShape& s) {
   return words_for(tiles_with(t, m, n));
 }
 
-double conv_any_forward_us(const ConvShape& s) {
-  if (conv_any_requant_words(kConvForward, s) == 0) return 0.0;
+// The walk of a workgroup, longer the more of them there are; from one per compute unit on, units have two.  Least squares over 642
+// launches of the 3 x 3 maps that requant_us (conv3x3_halo.hip) is fitted to: 5% rms, from 0.84 to 1.21 of the measured time.
+double conv_any_forward_us(const ConvShape& s, size_t* words) {
+  *words = 0;
+  if (!conv_any_shape(kConvForward, s)) return 0.0;
+  const int t = requant_tile(kConvForward, s);
+  if (t < 0) return 0.0;
   int m, n, k;
   product_of(kConvForward, s, &m, &n, &k);
-  const int t = requant_tile(kConvForward, s);
+  *words = words_for(tiles_with(t, m, n));
   if (t > 1) return 1e9;   // the wide tiles: not for the few workgroups this is asked for
   const double chunks = t == 0 ? (k + TileS::BK - 1) / TileS::BK : (k + TileM::BK - 1) / TileM::BK;
-  return (t == 0 ? 4.9 + 0.42 * chunks : 5.6 + 0.58 * chunks) * (tiles_with(t, m, n) > compute_units() ? 1.5 : 1.0);
+  const double fill = static_cast<double>(tiles_with(t, m, n)) / compute_units();
+  if (t == 0) return fill <= 1.0 ? 5.1 + 0.55 * chunks + 0.8 * fill : 4.9 + (0.64 + 0.35 * fill) * chunks + 0.6 * fill;
+  return fill <= 1.0 ? 5.4 + 0.69 * chunks + 0.5 * fill : 6.0 + (0.44 + 0.40 * fill) * chunks + 1.2 * fill;
 }
 
 double conv_any_dgrad_us(const ConvShape& s) {

@@ -125,6 +125,30 @@ def test_conv_slices_of_64_two_workgroups_per_unit(dev, case):
     base.test_conv_halo_tiles(dev, case, "auto")
 
 
+# one to three 512-step chunks, 32 x 32 and 64 x 64 tiles, more tiles than compute units
+@pytest.mark.parametrize("case", [(1, 8, 64, 64), (2, 16, 112, 48), (40, 4, 160, 32), (9, 32, 32, 64), (40, 2, 64, 96)])
+def test_few_images_sto(dev, case, monkeypatch):
+    """StoShift on supplied integers in a forward pass of few images, with the pooling behind the layer, by both kernels that the
+    estimate chooses between."""
+    from niti_amd import _lib
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    g = torch.Generator().manual_seed(12200 + N + Q + C)
+    x, w = ri8(g, N, Q, Q, C), ri8(g, K, 3, 3, C)
+    acc = co.conv_fprop(x, w, 1, 1)
+    u = torch.randint(0, 2 ** max(po.RangeEstimate(acc) - 7, 1), acc.shape, generator=g, dtype=torch.int32)
+    ref = torch.clamp(po.act_calc(acc, 0, "sto", "floor", u)[0], min=0)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    for pin in ("0", "1"):
+        monkeypatch.setenv("NITI_FPROP_SMALL", pin)
+        for pool in (False, True):
+            y, _, pooled = _lib.host().conv_layer_forward(True, x.to(dev), w.to(dev), 1, 1, True, 7, _lib.ROUND["sto"], _lib.DIV["floor"], _lib.BW["int"],
+                                                          True, scalar(0), scalar(-3), scalar(1), None, pool, u.to(dev), True)
+            assert torch.equal(y.cpu(), ref), (pin, pool)
+            assert pooled is None or torch.equal(pooled.cpu(), po.maxpool_fwd(ref)), pin
+
+
 # the kernel of 32-channel slices on an even number of them, which the dispatch gives to the other one
 @pytest.mark.parametrize("tile", ["auto", "32", "64", "128"])
 @pytest.mark.parametrize("case", [(2, 32, 64, 144), (3, 16, 128, 80), (8, 8, 256, 64), (16, 4, 64, 272)])
