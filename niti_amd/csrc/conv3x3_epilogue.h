@@ -474,11 +474,11 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
       // ---- wait for the slots of all workgroups; the maximum over them is the tensor's range
       if (wave == 0) {
         const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
-        if (lane == 0) red[8] = g != 0u ? g - 1u : 0u;
+        if (lane == 0) red[9] = g != 0u ? g - 1u : 0u;   // (not red[8]: no barrier has passed since the others read that)
       }
       __syncthreads();
       final_range = true;
-      gmax = red[8];
+      gmax = red[9];
       const int fshift = max(bitwidth_of(gmax, a.bw_mode) - a.target_bits, 0);
       if (fshift == shift) break;
       shift = fshift;
