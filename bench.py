@@ -368,7 +368,8 @@ def _avg_us(fn, reps=20, warm=3):
 def mfma_probe(dev):
     """What the matrix units sustain in a register-resident MFMA loop (no LDS, no memory traffic) for constant and for
     uniform random int8 operands: the shader clock follows the multipliers' power draw, so the second figure - not the
-    datasheet peak - is the ceiling of kernels that multiply random data."""
+    datasheet peak - is the ceiling of kernels that multiply random data.  Both instructions that the kernels use: 16x16x64 (the
+    convolutions; it moves half the accumulator bytes per operation, so its rate is the higher one and the ceiling) and 32x32x32."""
     import torch
     from niti_amd import ops
     g = torch.Generator().manual_seed(4321)
@@ -377,20 +378,20 @@ def mfma_probe(dev):
     zero = torch.zeros(1 << 20, dtype=torch.int8, device=dev)
     ops.mfma_probe(const)                              # clocks up
     # one workgroup (8 wavefronts) per compute unit: two wavefronts per SIMD, each issuing its run of products back to
-    # back.  With two workgroups per compute unit the same loop reaches two thirds of this (four wavefronts of equal
-    # priority take turns on a SIMD's matrix unit, and the changes of wavefront cost it idle clocks).
-    one = dict(workgroups=256, iters=2400)
-    zt, zg = ops.mfma_probe(zero, **one)
-    ct, cg = ops.mfma_probe(const, **one)
-    rt, rg = ops.mfma_probe(rnd, **one)
-    rt2, rg2 = ops.mfma_probe(rnd)
-    return {"zero_operands_tops": round(zt, 1), "zero_operands_clock_ghz": round(zg, 2),
-            "constant_operands_tops": round(ct, 1), "constant_operands_clock_ghz": round(cg, 2),
-            "random_operands_tops": round(rt, 1), "random_operands_clock_ghz": round(rg, 2),
-            "random_operands_two_workgroups_per_cu_tops": round(rt2, 1), "random_operands_two_workgroups_per_cu_clock_ghz": round(rg2, 2),
-            "note": "256 workgroups (one per compute unit) x 8 wavefronts x 2400 x 12 v_mfma_i32_32x32x32_i8 on register operands; "
-                    "clock = shader cycle counter against the 100 MHz wall clock inside the loop; the last pair is the same loop "
-                    "with 512 workgroups x 1200"}
+    # back.  With two workgroups per compute unit four wavefronts of equal priority take turns on a SIMD's matrix unit; the
+    # changes of wavefront cost 32x32x32 a third of its rate and 16x16x64 nothing.
+    out = {}
+    for shape, suffix in (("16x16x64", ""), ("32x32x32", "_32x32x32")):
+        for name, operands, wgs in (("zero_operands", zero, 256), ("constant_operands", const, 256), ("random_operands", rnd, 256),
+                                    ("random_operands_two_workgroups_per_cu", rnd, 512)):
+            # launches of about 5 ms: the clock takes some ten to settle behind another load (2400 rounds read up to 15% less)
+            tops, ghz = ops.mfma_probe(operands, workgroups=wgs, iters=12000 * 256 // wgs, shape=shape)
+            out[name + suffix + "_tops"] = round(tops, 1)
+            out[name + suffix + "_clock_ghz"] = round(ghz, 2)
+    out["note"] = ("256 workgroups (one per compute unit) x 8 wavefronts x 12000 rounds of 786432 operations on register operands, v_mfma_i32_16x16x64_i8 "
+                   "and (suffix _32x32x32) v_mfma_i32_32x32x32_i8; clock = shader cycle counter against the 100 MHz wall clock inside the loop; "
+                   "two_workgroups_per_cu is the same loop with 512 workgroups x 6000")
+    return out
 
 
 def side_workloads(dev):

@@ -577,6 +577,10 @@ int niti_group_conv_i8_f32(const int8_t* x, const int8_t* w, float* y, int N, in
  */
 int niti_mfma_probe_i8(const int8_t* operands, size_t operand_bytes, int workgroups, int iters, int32_t* out,
                        int64_t* clocks, void* stream);
+/* The same loop on v_mfma_i32_16x16x64_i8, which the convolution kernel of 64-channel slices uses: 24 MFMAs of half the size per
+ * round, i.e. as many operations. */
+int niti_mfma_probe_i8_16x16x64(const int8_t* operands, size_t operand_bytes, int workgroups, int iters, int32_t* out,
+                                int64_t* clocks, void* stream);
 
 #ifdef __cplusplus
 }

@@ -2,9 +2,9 @@
 // v_mfma_i32_16x16x64_i8: 64 input channels per product instead of 32.
 //
 // Why this instruction: the matrix units are power-limited on random operands, and a 16 x 16 x 64 product moves half
-// the accumulator bytes of a 32 x 32 x 32 one per operation.  A register-resident loop sustains 4.2 POP/s at 2.1 GHz on uniform
-// random int8 where the 32 x 32 x 32 form sustains 3.5 at 1.77, and with two workgroups on a compute unit (four wavefronts per
-// matrix unit taking turns) 4.2 against 3.1.
+// the accumulator bytes of a 32 x 32 x 32 one per operation.  A register-resident loop (probe.hip) sustains 3.9 to 4.1 POP/s at 2.0 GHz on
+// uniform random int8 where the 32 x 32 x 32 form sustains 3.5 at 1.75, and with two workgroups on a compute unit (four wavefronts per
+// matrix unit taking turns) 3.9 to 4.1 against 2.5 to 3.0.
 //
 // A workgroup owns 256 consecutive output pixels x KT output channels (128, 64 or 32) and walks over the input channels in
 // slices of 64.  8 wavefronts: 4 pixel groups of 64 x 2 channel groups of KT/2 (KT = 32: 8 pixel groups of 32).  Of 32
@@ -130,6 +130,8 @@ __device__ inline v4i neighbour4(v4i x, int keep) {
 __device__ inline void mfma64(v4i& d, v4i a, v4i b) { asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b)); }
 __device__ inline void mfma_settle() { asm volatile("s_nop 15\n\ts_nop 15"); }
 
+// (What is left: the StoShift instances for two workgroups per unit spill 6 registers at 64 channels and 17 or 18 at 128, none of them inside
+// the loop; no other instance spills.)
 // kWT: the filter operand is the forward copy of the filter of the convolution whose data gradient this launch computes; its
 // blocks of 64 reduction channels x 32 outputs are transposed by ds_read_b64_tr_b8 when the fragments are read.
 // kSto: StoShift on random integers read in the epilogue.

@@ -730,10 +730,12 @@ def head_backward(err, act, w, err_bits=7, err_method="psto", grad_bits=5, grad_
     return dx, g8, shifts[0:1], shifts[1:2], sync
 
 
-def mfma_probe(operands, workgroups=512, iters=1200):
-    """Times the library's register-resident int8 MFMA loop over the given operand bytes (int8 tensor, >= 128 bytes).
+def mfma_probe(operands, workgroups=512, iters=1200, shape="32x32x32"):
+    """Times the library's register-resident int8 MFMA loop over the given operand bytes (int8 tensor, >= 128 bytes), on the
+    instruction of ``shape`` ("32x32x32" or "16x16x64").
     Returns (tera-operations per second, shader clock in GHz during the loop): the matrix-unit ceiling for operands
     with these values."""
+    name = {"32x32x32": "niti_mfma_probe_i8", "16x16x64": "niti_mfma_probe_i8_16x16x64"}[shape]
     _chk_dev(operands)
     if operands.dtype != torch.int8 or not operands.is_contiguous():
         raise RuntimeError("mfma_probe: contiguous int8 tensor expected")
@@ -742,8 +744,7 @@ def mfma_probe(operands, workgroups=512, iters=1200):
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
 
     def launch():
-        L.check(L.lib().niti_mfma_probe_i8(_ptr(operands), operands.numel(), workgroups, iters, _ptr(out), _ptr(clocks),
-                                           _stream(operands)), "niti_mfma_probe_i8")
+        L.check(getattr(L.lib(), name)(_ptr(operands), operands.numel(), workgroups, iters, _ptr(out), _ptr(clocks), _stream(operands)), name)
     for _ in range(3):
         launch()
     e0.record()
