@@ -856,7 +856,10 @@ bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
 //    384 +0.4 +2.0, 512 +1.0 +0.2; to 256 at 32 x 32, C = 64 -1.2 -0.3, 128 -1.6 +0.2, 256 -1.4 +0.4; to 128 filters at 16 x 16, C = 128 +0.1 +2.9,
 //    256 -1.5 +0.8; single figures repeat within 0.7.  128 channels are also all there are where the folded pooling's backward pass
 //    would write half lines (42.6 / 32.6).
-int k64_ktile(long long pix, int K, int H, int C) {
+//  - int32 results are four times the stores, which the second workgroup hides: C <= 256 to 96 and 128 filters, 1.3 to 2 workgroups of 64
+//    channels per unit, maps of 8 x 8 to 32 x 32: 64 channels take 0.85 to 1.01 of the time of 128 (220 images of 16 x 16, 128 -> 128: 12.3 /
+//    13.7 us); at 384 and 512 0.93 to 1.05, on 4 x 4 maps 1.00 to 1.12.
+int k64_ktile(long long pix, int K, int H, int C, bool fused) {
   const long long ptiles = (pix + 255) / 256;
   const int cus = compute_units();
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
@@ -865,7 +868,7 @@ int k64_ktile(long long pix, int K, int H, int C) {
   if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
   const long long b64 = ptiles * ((K + 63) / 64);
   const long long b128 = ptiles * ((K + 127) / 128);
-  return K <= 64 || b64 <= cus || (b64 <= 2LL * cus && (b128 > cus || (C <= 256 && K >= 256))) ? 64 : 128;
+  return K <= 64 || b64 <= cus || (b64 <= 2LL * cus && (b128 > cus || (C <= 256 && (K >= 256 || (!fused && H >= 8))))) ? 64 : 128;
 }
 
 // Which kernel takes a launch, and the pixels and channels of its workgroups.
@@ -875,7 +878,7 @@ struct HaloTile {
 };
 HaloTile halo_tile(long long pix, int K, int H, int C, bool fused) {
   const bool k64 = halo_k64(C);
-  const int ktile = k64 ? k64_ktile(pix, K, H, C) : halo_ktile(pix, K, H, C);
+  const int ktile = k64 ? k64_ktile(pix, K, H, C, fused) : halo_ktile(pix, K, H, C);
   // (at 64 channels and more of such workgroups than the device holds, one launch of the other kernel's 512 pixels instead of two)
   if (fused && halo_two_pixel_tiles(pix, K, H, ktile)) return {ktile, 512, false};
   return {ktile, 256, k64};

@@ -125,6 +125,12 @@ def test_conv_slices_of_64_two_workgroups_per_unit(dev, case):
     base.test_conv_halo_tiles(dev, case, "auto")
 
 
+# two slices whose int32 results come from two narrow workgroups per unit, forward and data gradient
+@pytest.mark.parametrize("case", [(130, 16, 128, 128), (130, 16, 192, 96), (130, 16, 96, 192)])
+def test_conv_slices_of_64_int32_from_narrow_workgroups(dev, case):
+    base.test_conv_halo_tiles(dev, case, "auto")
+
+
 # one to three 512-step chunks, 32 x 32 and 64 x 64 tiles, more tiles than compute units
 @pytest.mark.parametrize("case", [(1, 8, 64, 64), (2, 16, 112, 48), (40, 4, 160, 32), (9, 32, 32, 64), (40, 2, 64, 96)])
 def test_few_images_sto(dev, case, monkeypatch):
