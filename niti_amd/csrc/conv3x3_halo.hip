@@ -26,8 +26,8 @@
 // this removes 8 of the 9 bytes moved per output element.  The same epilogue can leave the 2x2 / stride-2
 // maximum of its output next to it (the max-pool that follows the layer).
 //
-// Input channels that fill whole slices of 64 have a faster form of the same kernel (conv3x3_k64.h); this one is left with the
-// first layer and other counts whose last slice of 64 would be half empty.
+// Input channels that fill two or more whole slices of 64 have a faster form of the same kernel (conv3x3_k64.h); this one is left with
+// the first layer, most launches of a single such slice and other counts whose last slice of 64 would be half empty.
 //
 // Launches the device cannot hold at once: the 64-channel tile takes 512 pixels per workgroup where that
 // is enough (HGeom::TWO); otherwise the launch runs twice without waiting (kRqNoWait, kRqSettle below).
@@ -821,17 +821,6 @@ int halo_ktile(long long pix, int K, int H, int C) {
   return (b128 < 2LL * cus && K > 64) ? 64 : 128;
 }
 
-// The kernel of 64-channel slices (conv3x3_k64.h) multiplies a whole number of them: not where the last would be half empty
-// (C up to 32, the first layer, among them).  Its time with a whole slice more, i.e. at most what a half-empty one would cost, against the
-// kernel of 32-channel slices at 3 / 5 / 7 / 9 of those (16 to 256 images of 8 x 8 to 32 x 32, 64 to 512 filters): that kernel takes 0.86 /
-// 0.97 / 1.01 / 1.04 of it at the median (0.78 to 0.94, 0.93 to 1.09, 0.96 to 1.10, 0.98 to 1.11; data gradients 0.02 more), so up to five
-// slices it is the faster one and from seven on little is lost.  At 4 / 6 / 8 / 10 slices the kernel of 64-channel slices takes 0.99 / 0.95 /
-// 0.93 / 0.92 of the other's time.  NITI_HALO_K64=0 pins the kernel of 32-channel slices (tests).
-bool halo_k64(int C) {
-  const char* e = getenv("NITI_HALO_K64");
-  return (C + 31) / 32 % 2 == 0 && (e == nullptr || e[0] != '0');
-}
-
 // The 64-channel tile with 512 pixels per workgroup: where 256-pixel workgroups would be more than the device holds
 // at once (a condition of the requantising variant), on the large maps where such launches occur.
 bool halo_two_pixel_tiles(long long pix, int K, int H, int ktile) {
@@ -871,17 +860,38 @@ int k64_ktile(long long pix, int K, int H, int C, bool fused) {
   return K <= 64 || b64 <= cus || (b64 <= 2LL * cus && (b128 > cus || (C <= 256 && (K >= 256 || (!fused && H >= 8))))) ? 64 : 128;
 }
 
-// Which kernel takes a launch, and the pixels and channels of its workgroups.
+// Which kernel takes a launch, and the pixels and channels of its workgroups.  The kernel of 64-channel slices multiplies a whole number
+// of them: not where the last would be half empty (the first layer among them).  Its time with a whole slice more, i.e. at most what a
+// half-empty one would cost, against the kernel of 32-channel slices at 3 / 5 / 7 / 9 of those (16 to 256 images of 8 x 8 to 32 x 32, 64 to 512
+// filters): that kernel takes 0.86 / 0.97 / 1.01 / 1.04 of it at the median (0.78 to 0.94, 0.93 to 1.09, 0.96 to 1.10, 0.98 to 1.11; data
+// gradients 0.02 more), so up to five slices it is the faster one and from seven on little is lost.
+// At 4 / 6 / 8 / 10 slices the kernel of 64-channel slices takes 0.99 / 0.95 / 0.93 / 0.92 of the other's time (at 4 and at most one workgroup
+// per unit 1.03 forward, 1.01 of the data gradient, 0.97 with the pooling folded in).  A single slice of 64 channels is over before its
+// longer way to the first product is made up for.  Over 105 layers of 16 to 1000 images of 4 x 4 to 32 x 32, 32 to 512 filters, replayed in
+// graphs, it takes 1.07 to 1.10 of the other's time forward, 1.05 to 1.08 of the data gradient, 1.07 to 1.08 of int32 results with at
+// most one workgroup per unit (64 images of 32 x 32, 64 -> 64: 7.7 / 7.1 us), and 1.02 / 0.97 / 1.06 with more.  It keeps, of the rounded launches:
+//  - one workgroup of 128 channels on a unit, none of them half empty, where the other kernel has two of 64: 0.86 to 1.04 forward, 0.77 to
+//    0.92 of the data gradient (256 images of 16 x 16, 64 -> 128: 10.1 / 9.7 and 10.1 / 12.5 us);
+//  - grids that fit on the device where the other's do not: 0.66 (1000 images of 8 x 8, 64 -> 256: 14.3 / 21.8 us).
+// NITI_HALO_K64 = 0 / 1 pins the kernel of 32-channel / 64-channel slices, the second where they are whole (tests).
 struct HaloTile {
   int channels, pixels;
   bool k64;
 };
 HaloTile halo_tile(long long pix, int K, int H, int C, bool fused) {
-  const bool k64 = halo_k64(C);
-  const int ktile = k64 ? k64_ktile(pix, K, H, C, fused) : halo_ktile(pix, K, H, C);
+  const char* e = getenv("NITI_HALO_K64");
+  const bool whole = (C + 31) / 32 % 2 == 0 && (e == nullptr || e[0] != '0');
+  const auto blocks = [&](int ktile) { return (pix + 255) / 256 * ((K + ktile - 1) / ktile); };
+  const int cus = compute_units();
+  const int wide = whole ? k64_ktile(pix, K, H, C, fused) : 0;
   // (at 64 channels and more of such workgroups than the device holds, one launch of the other kernel's 512 pixels instead of two)
+  if (whole && fused && halo_two_pixel_tiles(pix, K, H, wide)) return {wide, 512, false};
+  if (whole && (C > 64 || e != nullptr)) return {wide, 256, true};
+  const int ktile = halo_ktile(pix, K, H, C);
+  if (whole && fused && wide == 128 && K % 128 == 0 && blocks(128) <= cus) return {wide, 256, true};
   if (fused && halo_two_pixel_tiles(pix, K, H, ktile)) return {ktile, 512, false};
-  return {ktile, 256, k64};
+  if (whole && fused && blocks(ktile) > 2LL * cus && blocks(wide) <= 2LL * cus) return {wide, 256, true};
+  return {ktile, 256, false};
 }
 
 template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto = false>

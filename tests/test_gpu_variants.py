@@ -43,11 +43,14 @@ def test_conv_sto_tiles(dev, tile, case, monkeypatch):
 
 
 # N, side, C, K: the kernel of 64-channel slices in each of its forms (channel tile, workgroups per compute unit it is made for) on
-# every map: one to five slices, a last one of 48 channels, a last tile of 16 outputs, batches that end inside a tile (five more
-# images); int32, rounded, both filter copies, the mask and the pooling's backward pass, StoShift
+# every map (tiles of 32 channels: of at most 16 x 16): one to five slices, a last one of 48 channels, a last tile of 16 outputs,
+# batches that end inside a tile (five more images); int32, rounded, the mask, both filter copies and the pooling's backward pass where the
+# outputs are an even number of 32-channel slices too, StoShift
 @pytest.mark.parametrize("tile,per_cu", [("32", "1"), ("64", "1"), ("64", "2"), ("128", "1"), ("128", "2")])
-@pytest.mark.parametrize("case", [(2, 32, 64, 144), (1, 32, 304, 64), (3, 16, 112, 80), (4, 8, 256, 192), (16, 4, 64, 272), (32, 4, 192, 128)])
+@pytest.mark.parametrize("case", [(2, 32, 64, 144), (1, 32, 304, 64), (3, 16, 112, 80), (3, 16, 112, 64), (2, 16, 64, 192), (4, 8, 256, 192), (16, 4, 64, 272),
+                                  (32, 4, 192, 128)])
 def test_conv_slices_of_64(dev, case, tile, per_cu, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     monkeypatch.setenv("NITI_HALO_KT", tile)
     monkeypatch.setenv("NITI_HALO_PER_CU", per_cu)
     N, Q, C, K = case
@@ -71,28 +74,32 @@ TWO_LAUNCHES = [(65, 32, 64, 144), (172, 16, 272, 64), (2052, 8, 64, 64)]
 
 
 @pytest.mark.parametrize("case", TWO_LAUNCHES)
-def test_conv_slices_of_64_on_a_grid_larger_than_the_device(dev, case):
+def test_conv_slices_of_64_on_a_grid_larger_than_the_device(dev, case, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_requant_predicted_shift(dev, case)
 
 
 @pytest.mark.parametrize("case", TWO_LAUNCHES)
-def test_conv_slices_of_64_on_a_grid_larger_than_the_device_sto(dev, case):
+def test_conv_slices_of_64_on_a_grid_larger_than_the_device_sto(dev, case, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_requant_sto(dev, case, "floor")
 
 
 # N, side of the pooled map, channels, reduction
 @pytest.mark.parametrize("case", [(172, 16, 272, 64), (2052, 8, 64, 64)])
-def test_conv_slices_of_64_unpooling_on_a_grid_larger_than_the_device(dev, case):
+def test_conv_slices_of_64_unpooling_on_a_grid_larger_than_the_device(dev, case, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_dgrad_requant_unpool(dev, case)
 
 
 @pytest.mark.parametrize("forward", [True, False])
-def test_conv_slices_of_64_stored_again(dev, forward):
+def test_conv_slices_of_64_stored_again(dev, forward, monkeypatch):
     """One image with large values among images of tiny ones: the settling launch computes nearly every tile again, with the pooled
     output, with the mask of a ReLU below and from both filter copies."""
     from niti_amd import ops
     from oracle import c_oracle as co
     from oracle import niti_oracle as po
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     N, Q, C, K = 65, 32, 64, 144
     base._say("conv_slices_of_64_stored_again", forward)
     g = torch.Generator().manual_seed(6161)
@@ -122,6 +129,14 @@ def test_conv_slices_of_64_stored_again(dev, forward):
 # of 32 and of 64 channels; forward, then data gradient
 @pytest.mark.parametrize("case", [(130, 16, 64, 160), (130, 16, 160, 64), (344, 8, 64, 320)])
 def test_conv_slices_of_64_two_workgroups_per_unit(dev, case):
+    base.test_conv_halo_tiles(dev, case, "auto")
+
+
+# a single slice of 64 channels, the last sixteen of one channel count empty: at most one workgroup per unit, more of them, one of 128
+# channels where two of 64 would be on a unit (also as the reduction of a data gradient), a grid that fits on the device with 128 channels
+# only
+@pytest.mark.parametrize("case", [(3, 16, 48, 64), (129, 16, 48, 96), (130, 16, 64, 128), (130, 16, 128, 64), (520, 8, 64, 256)])
+def test_conv_single_slice_of_64(dev, case):
     base.test_conv_halo_tiles(dev, case, "auto")
 
 
