@@ -128,7 +128,8 @@ def test_conv_slices_of_64_stored_again(dev, forward, monkeypatch):
 # more 128-channel workgroups than compute units, fewer 64-channel ones than twice those: an odd number of 64-channel groups, the last
 # of 32 and of 64 channels; forward, then data gradient
 @pytest.mark.parametrize("case", [(130, 16, 64, 160), (130, 16, 160, 64), (344, 8, 64, 320)])
-def test_conv_slices_of_64_two_workgroups_per_unit(dev, case):
+def test_conv_slices_of_64_two_workgroups_per_unit(dev, case, monkeypatch):
+    monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_halo_tiles(dev, case, "auto")
 
 
