@@ -686,17 +686,23 @@ extern "C" int niti_conv2d_i8_wgrad_update(const int8_t* act, const int8_t* err,
 }
 
 // Whether both gradients in one launch are the faster way.  Outside the 3x3 kernels' maps they are wherever they fit; there the
-// data gradient's own kernel and the weight gradient's are estimated.  0.8: the one launch's estimate is 0.85 of its measured time on the
-// average (0.14 rms), the other two's 1.04 (0.09).  Over 500 drawn layers of 4 x 4 to 32 x 32 (16 to 512 channels) the choice is 0.2% off the
-// faster way on the geometric mean (300 further ones: 0.6%, seven by 10 to 26%); 0.75 / 0.85 / 0.9: 0.6 / 0.3 / 0.5%.
+// data gradient's own kernel and the weight gradient's are estimated.  The factors are the one launch's estimated time to the other two's
+// at which the two ways took the same time inside training steps (226 pairs: layers of VGG-7 and VGG-13, 8 to 128 images, each
+// layer stepped either way) and of layers by themselves (42 of 64 to 512 channels whose weight gradient is the nine-tap kernel's): 0.28 us a
+// pair lost to the faster way, 0.48 with 0.8 for both, 0.77 with the 3x3 kernels priced by the map's width alone.  Against the nine-tap kernel
+// the line lies lower: 256 -> 256 at 16 x 16, 48 images, in a VGG-7 step 312 us as one launch, 304 as two; 128 -> 256 at 16 x 16, 56 images, whose
+// weight gradient is not that kernel's, 310 / 313.
 static bool backward_together(const ConvShape& s) {
   const char* e = getenv("NITI_BACKWARD_TOGETHER");   // 0 / 1 pins (tests)
   if (e != nullptr) return e[0] != '0';
   const double us = conv_backward_us(s);
   if (us == 0.0) return false;
   double dgrad = 0.0;
-  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad))
-    return us < 0.8 * (dgrad + wgrad3x3_us(s.N, s.H, s.C, s.K));
+  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) > 0 && wgrad3x3_supported(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad)) {
+    bool nine_tap = false;
+    const double wgrad = wgrad3x3_us(s.N, s.H, s.C, s.K, &nine_tap);
+    return us < (nine_tap ? 0.7 : 0.84) * (dgrad + wgrad);
+  }
   const double d = conv_any_dgrad_us(s), w = conv_any_wgrad_us(s);
   return d == 0.0 || us < d + w;
 }

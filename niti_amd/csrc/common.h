@@ -215,7 +215,7 @@ int launch_post_i32(int32_t* v, int64_t n, bool roundtrip, uint32_t* absmax, hip
 // native 3x3 / stride 1 / pad 1 weight gradient (wgrad3x3.hip)
 bool wgrad3x3_supported(int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 size_t wgrad3x3_workspace(int N, int H, int C, int K);
-double wgrad3x3_us(int N, int H, int C, int K);   // estimated time with update
+double wgrad3x3_us(int N, int H, int C, int K, bool* nine_tap);   // estimated time with update
 bool wgrad3x3_prefers_any(int N, int H, int C, int K);   // few pixels: conv_any.hip's kernel is the faster one
 int launch_wgrad3x3(const int8_t* act, const int8_t* err, int32_t* dw, int N, int H, int C, int K, bool roundtrip,
                     uint32_t* absmax, void* workspace, hipStream_t stream);

@@ -1130,10 +1130,12 @@ bool wgrad3x3_prefers_any(int N, int H, int C, int K) {
   return any < 0.8 * nine_tap_us(N, H, C, K);
 }
 
-// estimated time of the gradient with update, whichever kernel takes it
-double wgrad3x3_us(int N, int H, int C, int K) {
+// estimated time of the gradient with update, whichever kernel takes it; *nine_tap: the one of this file's nine-tap sums
+double wgrad3x3_us(int N, int H, int C, int K, bool* nine_tap) {
+  *nine_tap = false;
   if (wgrad_small_supported(N, H, C, K, C)) return 9.5 + 3.3e-3 * N * H * H + 7.6e-6 * C * K;
-  return wgrad3x3_prefers_any(N, H, C, K) ? conv_any_wgrad_us({N, H, H, C, K, 3, 3, 1, 1}) : nine_tap_us(N, H, C, K);
+  *nine_tap = !wgrad3x3_prefers_any(N, H, C, K);
+  return *nine_tap ? nine_tap_us(N, H, C, K) : conv_any_wgrad_us({N, H, H, C, K, 3, 3, 1, 1});
 }
 
 static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N, int H, int C, int K, int Cp, void* workspace,
