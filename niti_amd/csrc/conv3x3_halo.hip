@@ -27,7 +27,9 @@
 // maximum of its output next to it (the max-pool that follows the layer).
 //
 // Input channels that fill two or more whole slices of 64 have a faster form of the same kernel (conv3x3_k64.h); this one is left with
-// the first layer, most launches of a single such slice and other counts whose last slice of 64 would be half empty.
+// the first layer, most launches of a single such slice and other counts whose last slice of 64 would be half empty.  Of its instances the
+// StoShift ones for 64 channels spill 4 registers, those for 128 or for 512 pixels 15 to 19, and the data gradients for 512 pixels one;
+// no other does.
 //
 // Launches the device cannot hold at once: the 64-channel tile takes 512 pixels per workgroup where that
 // is enough (HGeom::TWO); otherwise the launch runs twice without waiting (kRqNoWait, kRqSettle below).
