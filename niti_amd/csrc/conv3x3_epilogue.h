@@ -135,7 +135,9 @@ __device__ inline ShiftHint halo_shift_hint(const HaloArgs& a, int settle_shift)
 // requests them, in the place of the loads that have nothing left to fetch, and all stay in registers (without a mask or a
 // pooling the requests are out of range: zeros, no memory traffic).  Otherwise the first two
 // mask pieces and the first window are requested in front of the range reduction and later ones two (one) pieces ahead of
-// their use; the wavefronts with four accumulator tiles in 128 registers fetch each piece where it is used.
+// their use; the wavefronts with four accumulator tiles in 128 registers request two mask pieces behind the rounding, later ones two
+// pieces ahead, and windows where they are used (256 images of 16 x 16, 256 -> 256, data gradient with every mask piece where it is used
+// 36.2 us, so 35.7; of 32 x 32, 128 -> 128 44.9 / 43.8; through the pooling 57.9 / 55.5).
 template <int Q, int KT, bool kTwo, int NWF, int PT, bool kRegs256>
 struct HaloPieces {
   static constexpr int LPP = NWF * 2;       // lanes (16-byte pieces) per pixel
@@ -349,6 +351,9 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
     }
 #pragma nounroll
     for (int pass = 0; pass < 2; ++pass) {
+      // addresses are worked out in every pass rather than kept in registers that the wavefronts with four accumulator tiles do not have
+      P pieces = pc;
+      if constexpr (!kMaskAhead) asm volatile("" : "+v"(pieces.mfirst));
       // the sums look modified to the compiler in every pass: nothing derived from them (magnitudes, signs) is
       // computed ahead of the loop and kept in 64 more registers
 #pragma unroll
@@ -398,18 +403,25 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
       if (fast) round_tiles(std::true_type{});
       else round_tiles(std::false_type{});
       // same wavefront reads back what it wrote: LDS operations of one wavefront complete in order
+      // without room for them earlier: two mask pieces at a time from here on (all four: 1 to 3 us more a launch for what they spill)
+      v4i mask_of[2];
+      if (!kMaskAhead && a.mask != nullptr) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) mask_of[t] = pieces.mask(a, t);
+      }
       if (pc.pairs) __syncthreads();
 #pragma unroll
       for (int t = 0; t < 32 * PT / PPI; ++t) {
         v4i v = *reinterpret_cast<const v4i*>(from + t * mstep * PROW);
-        const int off = pc.offset(a, t);
+        const int off = pieces.offset(a, t);
         v4i mk;
         if (a.mask != nullptr) {  // ReLU backward of the layer below, folded in: its output is this layer's input
           if constexpr (kMaskAhead) {
             mk = ahead.mk[t % MKD];
-            if (t + MKD < NPIECE) ahead.mk[t % MKD] = pc.mask(a, t + MKD);
+            if (t + MKD < NPIECE) ahead.mk[t % MKD] = pieces.mask(a, t + MKD);
           } else {
-            mk = pc.mask(a, t);
+            mk = mask_of[t % 2];
+            if (t + 2 < NPIECE) mask_of[t % 2] = pieces.mask(a, t + 2);
           }
 #pragma unroll
           for (int d = 0; d < 4; ++d) v[d] &= static_cast<int>(positive_bytes(static_cast<uint32_t>(mk[d])));
@@ -418,14 +430,14 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
           // max-pool backward folded in (mk holds the pooled values): the window of pooled pixel m in the pooling's input
           const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(a.unpool, 0, a.unpool_bytes, 0x00020000);
           int wo[4];
-          pc.window_offsets(a, t, wo);
+          pieces.window_offsets(a, t, wo);
           v4i xw[4], ow[4];
           if constexpr (kMaskAhead) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) xw[k] = ahead.xw[t % P::XWD][k];
-            if (t + P::XWD < NPIECE) pc.windows(a, t + P::XWD, ahead.xw[t % P::XWD]);
+            if (t + P::XWD < NPIECE) pieces.windows(a, t + P::XWD, ahead.xw[t % P::XWD]);
           } else {
-            pc.windows(a, t, xw);
+            pieces.windows(a, t, xw);
           }
 #pragma unroll
           for (int d = 0; d < 4; ++d) {
