@@ -485,6 +485,22 @@ int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int
                             int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The same as two launches, for 3x3 / pad 1 layers whose gradients are larger: the weight gradient's sums, then the data gradient
+ * with the update beside it.  w_prepared must be given: the data gradient reads the copy, which then receives the updated weights.
+ * err_method NITI_ROUND_NEAREST or NITI_ROUND_PSEUDO_STOCHASTIC.  NITI_CONV_SHIFT_HINT: *err_shift_out holds a predicted shift on entry.
+ * workspace: niti_conv2d_i8_backward_pair_workspace bytes.  niti_conv2d_i8_backward_pair_sync_words returns 0 where the kernels do
+ * not fit or another way is the faster (niti_conv2d_i8_backward; niti_conv2d_i8_dgrad_requant, niti_conv2d_i8_wgrad_update).
+ */
+size_t niti_conv2d_i8_backward_pair_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad);
+size_t niti_conv2d_i8_backward_pair_workspace(int N, int H, int W, int C, int K, int R, int S, int pad);
+int niti_conv2d_i8_backward_pair(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+                                 int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
+                                 const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
+                                 size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
+                                 const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
+                                 int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Integer cross-entropy gradient, TiLoss.forward (ti_loss.py:5-36), as one launch: out_val [n][classes] int8 logits
  * with exponent *out_exp (device scalar), target [n] int64 class indices, rand [n][classes] int32 random integers
  * (the low four bits stand in for the reference's torch.randint(0, 16)) -> grad [n][classes] int8 with exponent 0.

@@ -83,6 +83,9 @@ SIGNATURES = {
     "niti_conv2d_i8_backward_sync_words": (_sz, [_i] * 8),
     "niti_conv2d_i8_backward_workspace": (_sz, [_i] * 8),
     "niti_conv2d_i8_backward": (_i, [_vp] * 4 + [_i] * 8 + [_u, _i, _i, _vp, _vp, _vp] + [_i] * 5 + [_vp, _sz] + [_vp] * 10 + [_sz, _vp]),
+    "niti_conv2d_i8_backward_pair": (_i, [_vp] * 4 + [_i] * 8 + [_u, _i, _i, _vp, _vp, _vp] + [_i] * 5 + [_vp, _sz] + [_vp] * 10 + [_sz, _vp]),
+    "niti_conv2d_i8_backward_pair_sync_words": (_sz, [_i] * 8),
+    "niti_conv2d_i8_backward_pair_workspace": (_sz, [_i] * 8),
     "niti_linear_i8_backward_sync_words": (_sz, [_i] * 3),
     "niti_linear_i8_backward": (_i, [_vp, _vp, _vp, _vp] + [_i] * 9 + [_vp, _vp, _vp, _sz] + [_vp] * 9),
     "niti_loss_grad_i8": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),

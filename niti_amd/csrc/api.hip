@@ -721,14 +721,43 @@ extern "C" size_t niti_conv2d_i8_backward_workspace(int N, int H, int W, int C, 
   return round256(conv_backward_workspace({N, H, W, C, K, R, S, 1, pad}));
 }
 
-extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+// The pair of launches of larger 3x3 layers against the faster other way, as estimated.  Over the same 420 layers, each stepped all three ways
+// (as a pair, as one launch, one gradient after the other), the choice is 0.6% off the fastest on the geometric mean, 21% at most; without the
+// pair it was 7% and 44%, and with the pair only where the nine-tap kernel already was the weight gradient's 2.3% and 33%.  The factor
+// is what gives that: estimates of one launch are below what it takes in such graphs.  (80 images of 8 x 8, 256 -> 512 as
+// one launch 42.2 us, as a pair 33.7; 24 of 16 x 16, 128 -> 128 20.2 / 22.3; 128 of 32 x 32, 128 -> 128 one after the other 60.3 / 54.3.)
+static bool backward_as_pair(const ConvShape& s) {
+  const char* e = getenv("NITI_BACKWARD_PAIR");   // 0 / 1 pins (tests)
+  if (e != nullptr) return e[0] != '0';
+  const char* together = getenv("NITI_BACKWARD_TOGETHER");
+  if (together != nullptr && together[0] != '0') return false;
+  double dgrad = 0.0;
+  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) == 0) return false;
+  bool nine_tap = false;
+  const double us = conv_pair_us(s.N, s.H, s.C, s.K, dgrad);
+  const double other = backward_together(s) ? conv_backward_us(s) : dgrad + wgrad3x3_us(s.N, s.H, s.C, s.K, &nine_tap);
+  return us > 0.0 && us < 1.3 * other;
+}
+
+extern "C" size_t niti_conv2d_i8_backward_pair_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad) {
+  if (N <= 0 || H <= 0 || C <= 0 || K <= 0 || R != 3 || S != 3 || pad != 1 || H != W || halo_off()) return 0;
+  const size_t words = conv_pair_words(N, H, C, K);
+  return words > 0 && backward_as_pair({N, H, W, C, K, R, S, 1, pad}) ? words : 0;
+}
+
+extern "C" size_t niti_conv2d_i8_backward_pair_workspace(int N, int H, int W, int C, int K, int R, int S, int pad) {
+  if (N <= 0 || H <= 0 || C <= 0 || K <= 0 || R != 3 || S != 3 || pad != 1 || H != W || halo_off()) return 0;
+  return round256(conv_pair_workspace(N, H, C, K));
+}
+
+// together: one launch for both gradients; otherwise the weight gradient's sums, then the data gradient with the update beside it
+static int conv_backward(const char* who, bool together, const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
                                        int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
                                        const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
                                        size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
                                        const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
                                        int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
-  const char* who = "conv_backward";
   int st = check_conv_dims(who, N, H, W, C, K, R, S, 1, pad);
   if (st == NITI_OK) st = check_flags(who, flags, NITI_EPI_F32_ROUNDTRIP | NITI_CONV_SHIFT_HINT);
   if (st != NITI_OK) return st;
@@ -750,8 +779,12 @@ extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int
   const ConvShape s{N, H, W, C, K, R, S, 1, pad};
   if (w_prepared != nullptr && filter_copy_kind(N, H, W, C, K, R, S, 1, pad, 0) != 2)
     return fail(NITI_ERR_UNSUPPORTED, "%s: w_prepared needs a shape whose forward pass uses a kernel-ready filter copy", who);
-  const size_t need = conv_backward_words(s), bytes = conv_backward_workspace(s);
-  if (need == 0) return fail(NITI_ERR_UNSUPPORTED, "%s: the workgroups of both gradients do not fit on the device at once", who);
+  if (!together && (R != 3 || S != 3 || pad != 1 || H != W || halo_off())) return fail(NITI_ERR_UNSUPPORTED, "%s: shape not covered", who);
+  if (!together && w_prepared == nullptr) return fail(NITI_ERR_INVALID_ARG, "%s: the kernel-ready filter copy is read and written", who);
+  if (!together && err_method == NITI_ROUND_STOCHASTIC) return fail(NITI_ERR_UNSUPPORTED, "%s: stochastic rounding of the error", who);
+  const size_t need = together ? conv_backward_words(s) : conv_pair_words(N, H, C, K);
+  const size_t bytes = together ? conv_backward_workspace(s) : round256(conv_pair_workspace(N, H, C, K));
+  if (need == 0) return fail(NITI_ERR_UNSUPPORTED, together ? "%s: the workgroups of both gradients do not fit on the device at once" : "%s: shape not covered", who);
   if (sync_words < need) return fail(NITI_ERR_WORKSPACE, "%s: needs %zu zeroed sync words, got %zu", who, need, sync_words);
   if (bytes > 0 && (workspace == nullptr || workspace_bytes < bytes || !aligned16(workspace)))
     return fail(NITI_ERR_WORKSPACE, "%s: needs %zu workspace bytes (16-byte aligned), got %zu", who, bytes, workspace_bytes);
@@ -765,8 +798,31 @@ extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int
   }
   RequantSpec grad{grad_bits, grad_method, div_mode == NITI_DIV_TRUNC, bw_mode, (flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u, sync_spin_limit(),
                    timeout_word(), grad_shift_out, nullptr, exp_act, grad_exp_out, nullptr, nullptr};
+  if (!together) {
+    rq.flags = (flags & NITI_CONV_SHIFT_HINT) ? NITI_RQ_SHIFT_HINT : 0u;
+    return launch_conv_pair(err, act, w, dx8, N, H, C, K, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, grad, g8_out, w_prepared, workspace,
+                            static_cast<hipStream_t>(stream));
+  }
   return launch_conv_backward(s, err, act, w, dx8, (flags & NITI_EPI_F32_ROUNDTRIP) != 0, sync, rq, grad, g8_out, w_prepared, workspace,
                               static_cast<hipStream_t>(stream));
+}
+
+extern "C" int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+                                       int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
+                                       const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
+                                       size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
+                                       const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
+                                       int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream) {
+  return conv_backward("conv_backward", true, err, act, w, dx8, N, H, W, C, K, R, S, pad, flags, err_bits, err_method, err_rand, relu_mask, pool_in, ties, grad_bits, grad_method, div_mode, bw_mode, sync, sync_words, g8_out, w_prepared, err_shift_out, grad_shift_out, exp_err, exp_w, exp_act, err_exp_out, grad_exp_out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int niti_conv2d_i8_backward_pair(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx8, int N, int H, int W, int C, int K, int R, int S,
+                                       int pad, unsigned flags, int err_bits, int err_method, const int32_t* err_rand, const int8_t* relu_mask,
+                                       const int8_t* pool_in, int ties, int grad_bits, int grad_method, int div_mode, int bw_mode, uint32_t* sync,
+                                       size_t sync_words, int8_t* g8_out, int8_t* w_prepared, int32_t* err_shift_out, int32_t* grad_shift_out,
+                                       const int32_t* exp_err, const int32_t* exp_w, const int32_t* exp_act, int32_t* err_exp_out,
+                                       int32_t* grad_exp_out, void* workspace, size_t workspace_bytes, void* stream) {
+  return conv_backward("conv_backward_pair", false, err, act, w, dx8, N, H, W, C, K, R, S, pad, flags, err_bits, err_method, err_rand, relu_mask, pool_in, ties, grad_bits, grad_method, div_mode, bw_mode, sync, sync_words, g8_out, w_prepared, err_shift_out, grad_shift_out, exp_err, exp_w, exp_act, err_exp_out, grad_exp_out, workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t niti_gemm_i8_workspace(int trans_a, int trans_b, int m, int n, int k) {

@@ -60,7 +60,19 @@ int launch_conv3x3_k64_int32(const HaloArgs& a, int H, int ktile, hipStream_t st
 int launch_conv3x3_k64_requant(const HaloArgs& a, int H, int ktile, hipStream_t stream);
 int launch_conv3x3_k64_sto(const HaloArgs& a, int H, int ktile, hipStream_t stream);
 
+// the arguments of a launch of the requantising variant (conv3x3_halo.hip)
+int halo_requant_args(HaloArgs& a, const int8_t* x, const int8_t* wp, int8_t* y8, int N, int H, int C, int K, unsigned flags, uint32_t* sync,
+                      const RequantSpec& rq);
+
 namespace {
+
+// Which of the convolution's workgroups this is: x along the pixels, y along the channel tiles, of nx * ny.  (A launch may hold others.)
+struct HaloPlace {
+  int x, y, nx, ny;
+  __device__ int block() const { return y * nx + x; }
+  __device__ int blocks() const { return nx * ny; }
+};
+__device__ inline HaloPlace halo_grid_place() { return {static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(gridDim.x), static_cast<int>(gridDim.y)}; }
 
 constexpr int kOob = -1;
 constexpr int kOobFar = static_cast<int>(0x80000000u);   // out of range whatever scalar offset below 2^31 is added
@@ -79,15 +91,15 @@ __device__ inline void hc_sync() {
 
 // The settling launch (kRqSettle), called before anything else: false if this workgroup's tile already has the final shift and
 // it is done; otherwise settle_shift is the shift to store it with.
-__device__ inline bool halo_settle(const HaloArgs& a, int8_t* dump, int& settle_shift) {
+__device__ inline bool halo_settle(const HaloArgs& a, const HaloPlace at, int8_t* dump, int& settle_shift) {
   settle_shift = -1;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint32_t* const slots = a.sync + kSyncSlot0;
   uint32_t* const words = reinterpret_cast<uint32_t*>(dump);
-  const int nb = gridDim.x * gridDim.y;
-  const int b = blockIdx.y * gridDim.x + blockIdx.x;
+  const int nb = at.blocks();
+  const int b = at.block();
   uint32_t m = 0;
   for (int i = tid; i < nb; i += 512) m = max(m, __hip_atomic_load(slot_word(slots, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   m = wave_max_u32(m);
@@ -194,15 +206,24 @@ struct HaloAhead {
   v4i xw[P::XWD][4];
 };
 
+// What a workgroup does besides: see SumsAlong (wgrad_finish.h).
+struct NothingAlong {
+  __device__ void begin() {}
+  __device__ void publish() {}
+  __device__ void guess() {}
+  __device__ void wait() const {}
+  __device__ void update(int, const int32_t*, const int32_t*) const {}
+};
+
 // Results of a workgroup: 8 wavefronts of PT x 32 pixels x NWF x 32 channels (wp_: pixel group, wc: channel group; kTwo: wc is
 // the 256-pixel half, all wavefronts have the same 64 channels).  q[(i * PT + j) * 4 + g]: four consecutive channels of one pixel
 // of the 32-channel tile i and 32-pixel tile j; L says which: channel L::channel(g, lane) .. + 3 of the tile, pixel
 // L::pixel(g, lane).  smem: the main loop's tiles, dead once every wavefront is here; red: 16 words
 // that no load of the main loop writes.
-template <int Q, int KT, bool kTwo, int NWF, int PT, bool kFused, bool kSto, bool kRegs256, class L>
-__device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * PT * 4], int8_t* const smem, uint32_t* const red, const int pixbase,
+template <int Q, int KT, bool kTwo, int NWF, int PT, bool kFused, bool kSto, bool kRegs256, class L, class Along>
+__device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace at, v4i (&q)[NWF * PT * 4], int8_t* const smem, uint32_t* const red, const int pixbase,
                                               const int kt, const int wp_, const int wc, const int settle_shift, const ShiftHint hint,
-                                              const HaloPieces<Q, KT, kTwo, NWF, PT, kRegs256>& pc, HaloAhead<Q, KT, kTwo, NWF, PT, kRegs256>& ahead) {
+                                              const HaloPieces<Q, KT, kTwo, NWF, PT, kRegs256>& pc, HaloAhead<Q, KT, kTwo, NWF, PT, kRegs256>& ahead, Along& along) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -275,7 +296,7 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
     // final one unless another workgroup raises the bit width; the int8 stores of all workgroups then overlap the
     // wait for the last slots instead of following it in one burst.  When the final shift differs, the sums (still
     // in registers) are rounded and stored once more.
-    const int nb = gridDim.x * gridDim.y;
+    const int nb = at.blocks();
     uint32_t* const slots = a.sync + kSyncSlot0;
     constexpr int kLook = 8;   // slots a lane reads with its loads in flight together
     const bool nowait = (a.rq_flags & kRqNoWait) != 0;
@@ -314,7 +335,8 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
     uint32_t gmax = red[0];
 #pragma unroll
     for (int w = 1; w < 8; ++w) gmax = max(gmax, red[w]);
-    if (tid == 0 && !settled) __hip_atomic_store(slot_word(slots, blockIdx.y * gridDim.x + blockIdx.x), gmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0 && !settled) __hip_atomic_store(slot_word(slots, at.block()), gmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    along.publish();
     if (nb > 1 && !nowait && !settled && !hinted) {
       if (wave == 0) {
         uint32_t g = gmax + 1u;
@@ -333,7 +355,7 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
     if (!final_range && hinted) shift = max(shift, predicted_raw);
     if (settled) shift = settle_shift;
     if (nowait) {   // the shift this tile is stored with, for the settling launch
-      if (tid == 0) slot_word(slots, blockIdx.y * gridDim.x + blockIdx.x)[1] = static_cast<uint32_t>(shift);
+      if (tid == 0) slot_word(slots, at.block())[1] = static_cast<uint32_t>(shift);
     }
     final_range = final_range || nowait || settled;
     const bool trunc = a.trunc != 0;
@@ -483,21 +505,24 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, v4i (&q)[NWF * 
         }
       }
       if (final_range) break;
+      along.guess();
       // ---- wait for the slots of all workgroups; the maximum over them is the tensor's range
       if (wave == 0) {
         const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
         if (lane == 0) red[9] = g != 0u ? g - 1u : 0u;   // (not red[8]: no barrier has passed since the others read that)
       }
+      along.wait();
       __syncthreads();
       final_range = true;
       gmax = red[9];
       const int fshift = max(bitwidth_of(gmax, a.bw_mode) - a.target_bits, 0);
+      along.update(fshift, a.exp_a, a.exp_b);
       if (fshift == shift) break;
       shift = fshift;
       __builtin_amdgcn_s_waitcnt(0);   // the stores of the first pass leave before those that replace them
       request_first();
     }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0 && !nowait && !settled) {
+    if (at.block() == 0 && tid == 0 && !nowait && !settled) {
       const int sh = shift > 0 ? shift : 0;
       a.sync[0] = gmax;
       if (a.shift_out != nullptr) *a.shift_out = sh;

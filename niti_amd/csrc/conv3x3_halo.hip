@@ -145,7 +145,7 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
 
   int settle_shift = -1;   // kRqSettle: the final shift, when this workgroup has to store its tile again
   if constexpr (kFused) {
-    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, dump, settle_shift)) return;
+    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, halo_grid_place(), dump, settle_shift)) return;
   }
 
 
@@ -508,8 +508,9 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
         q[(i * PT + j) * 4 + g] = v4i{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
   const HaloPieces<Q, KT, G::TWO, NWF, PT, false> pieces(a, pixbase, kt, wp_, wc);
   HaloAhead<Q, KT, G::TWO, NWF, PT, false> ahead;
-  halo_epilogue<Q, KT, G::TWO, NWF, PT, kFused, kSto, false, Layout32>(a, q, smem, reinterpret_cast<uint32_t*>(dump), pixbase, kt, wp_, wc, settle_shift, hint,
-                                                                       pieces, ahead);
+  NothingAlong along;
+  halo_epilogue<Q, KT, G::TWO, NWF, PT, kFused, kSto, false, Layout32>(a, halo_grid_place(), q, smem, reinterpret_cast<uint32_t*>(dump), pixbase, kt, wp_, wc, settle_shift, hint,
+                                                                       pieces, ahead, along);
 }
 
 // ---- 2 x 2 maps -----------------------------------------------------------------------------------------
@@ -1071,9 +1072,8 @@ int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S,
 
 size_t conv3x3_halo_sync_words(int blocks) { return static_cast<size_t>(kSyncSlot0) + slot_words(blocks); }
 
-int launch_conv3x3_halo_requant(const int8_t* x, const int8_t* wp, int8_t* y8, int N, int H, int C, int K, unsigned flags,
-                                uint32_t* sync, const RequantSpec& rq, hipStream_t stream) {
-  HaloArgs a;
+int halo_requant_args(HaloArgs& a, const int8_t* x, const int8_t* wp, int8_t* y8, int N, int H, int C, int K, unsigned flags, uint32_t* sync,
+                      const RequantSpec& rq) {
   fill_common(a, x, wp, N, H, C, K, flags);
   a.y8 = y8;
   a.mask = rq.mask;
@@ -1106,7 +1106,14 @@ int launch_conv3x3_halo_requant(const int8_t* x, const int8_t* wp, int8_t* y8, i
   a.exp_a = rq.exp_a;
   a.exp_b = rq.exp_b;
   a.exp_out = rq.exp_out;
-  return launch_halo_any<true>(a, H, stream);
+  return NITI_OK;
+}
+
+int launch_conv3x3_halo_requant(const int8_t* x, const int8_t* wp, int8_t* y8, int N, int H, int C, int K, unsigned flags,
+                                uint32_t* sync, const RequantSpec& rq, hipStream_t stream) {
+  HaloArgs a;
+  const int st = halo_requant_args(a, x, wp, y8, N, H, C, K, flags, sync, rq);
+  return st != NITI_OK ? st : launch_halo_any<true>(a, H, stream);
 }
 
 }  // namespace niti

@@ -135,26 +135,27 @@ __device__ inline void mfma_settle() { asm volatile("s_nop 15\n\ts_nop 15"); }
 // kWT: the filter operand is the forward copy of the filter of the convolution whose data gradient this launch computes; its
 // blocks of 64 reduction channels x 32 outputs are transposed by ds_read_b64_tr_b8 when the fragments are read.
 // kSto: StoShift on random integers read in the epilogue.
-template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto>
-__global__ __launch_bounds__(512, 2 * PER_CU) void conv3x3_k64_kernel(const HaloArgs a) {
+template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto, class Along>
+__device__ __forceinline__ void k64_tile(const HaloArgs& a, const HaloPlace at, int8_t* const smem, Along& along) {
   static_assert(kFused || !kSto);
   using G = KGeom<Q, BR, NI, KT, PER_CU>;
   constexpr int PT = G::PT, NWF = G::NWF, TPS = G::TPS, S = G::S, R = G::R, WL = G::WL;
-  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t* const dump = smem + G::TILE_BYTES;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pixbase = blockIdx.x * G::PX;  // first output pixel of this workgroup in [N*Q*Q]
-  const int kt = blockIdx.y;
+  const int pixbase = at.x * G::PX;  // first output pixel of this workgroup in [N*Q*Q]
+  const int kt = at.y;
   const int n0 = pixbase / (Q * Q);
   const int p0 = (pixbase - n0 * (Q * Q)) / Q;
 
   int settle_shift = -1;   // kRqSettle: the final shift, when this workgroup has to store its tile again
   if constexpr (kFused) {
-    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, dump, settle_shift)) return;
+    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, at, dump, settle_shift)) return;
   }
+
+  along.begin();
 
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.x), 0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.wp), 0, a.wp_bytes, 0x00020000);
@@ -446,7 +447,13 @@ __global__ __launch_bounds__(512, 2 * PER_CU) void conv3x3_k64_kernel(const Halo
 #pragma unroll
   for (int t = 0; t < NWF * PT * 4; ++t) asm volatile("" : "+v"(acc[t]));   // not read in front of that wait
   __builtin_amdgcn_s_setprio(0);
-  halo_epilogue<Q, KT, false, NWF, PT, kFused, kSto, PER_CU == 1, Layout16>(a, acc, smem, reinterpret_cast<uint32_t*>(dump + 1024), pixbase, kt, wp_, wc, settle_shift, hint, pieces, ahead);
+  halo_epilogue<Q, KT, false, NWF, PT, kFused, kSto, PER_CU == 1, Layout16>(a, at, acc, smem, reinterpret_cast<uint32_t*>(dump + 1024), pixbase, kt, wp_, wc, settle_shift, hint, pieces, ahead, along);
+}
+template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto>
+__global__ __launch_bounds__(512, 2 * PER_CU) void conv3x3_k64_kernel(const HaloArgs a) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  NothingAlong along;
+  k64_tile<Q, BR, NI, KT, PER_CU, kFused, kWT, kSto>(a, halo_grid_place(), smem, along);
 }
 
 template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto>

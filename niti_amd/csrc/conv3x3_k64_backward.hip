@@ -1,0 +1,158 @@
+// Both gradients of a 3x3 layer whose weight gradient is the nine-tap kernel's, in two launches (ti_torch.py:404-437): the weight
+// gradient's main loop, which leaves its partial sums in memory, then the data gradient, along with which they are added and the weights
+// updated.
+//
+// Added by its own launch, the partial sums (24 to 28 MB whatever the layer) cost it an arrival wait, their way back from memory and a
+// range exchange of its own, with the matrix units idle.  Here the next launch's start is the arrival, the sums come in while others
+// multiply, and the two ranges are exchanged at the same time.  The copy of the filter that the data gradient reads is written behind the
+// last of its slots.
+//
+// Both launches in replayed graphs against the data gradient's and the one-launch weight gradient's (us): 128 images of 32 x 32, 128 -> 128
+// 59.6 -> 54.3, of 16 x 16, 128 -> 256 40.0 -> 34.5, 256 -> 256 55.8 -> 48.3, of 8 x 8, 256 -> 512 41.7 -> 36.2, 512 -> 512 53.9 -> 50.2;
+// 80 of 16 x 16, 128 -> 256 41.3 -> 29.2.  Of the weight gradient's launch its main loop and the way out are left (25.5 -> 16.5 us at
+// 16 x 16, 128 -> 256); the data gradient's grows by 3 to 7 us.  Timestamps of that layer: the slices are in at 9.5 us, their range known
+// at 13.3, the error's at 14.4, the copy written at 15.6; the products end at 11.0.  What bounds it: the slices' way from memory beside the
+// stages' loads, then one exchange.
+#include <stdlib.h>
+
+#include "conv3x3_k64.h"
+#include "conv_any.h"
+#include "wgrad_finish.h"
+
+namespace niti {
+namespace {
+
+constexpr int kBesideItems = 5, kWithinItems = 1;   // (two workgroups on a unit that multiply leave registers for one)
+constexpr int per_cu_geometry(int ktile) { return ktile == 32 ? 1 : 2; }   // the 32-channel tile fits twice as it is
+
+// The first nx x ny workgroups are the data gradient's.  kBeside: the others finish the weight gradient; otherwise the last work.nblocks
+// of them do so as well.
+template <int Q, int BR, int NI, int KT, bool kBeside>
+__global__ __launch_bounds__(512, 4) void conv3x3_k64_backward_kernel(const HaloArgs a, const FinishArgs f, const AlongWork work, const int nx, const int ny) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  constexpr int kPer = per_cu_geometry(KT);
+  const int id = blockIdx.x, first = nx * ny;
+  const HaloPlace at{id % nx, id / nx, nx, ny};
+  if constexpr (kBeside) {
+    if (id < first) {
+      NothingAlong along;
+      k64_tile<Q, BR, NI, KT, kPer, true, true, false>(a, at, smem, along);
+    } else {
+      finish_beside(SumsAlong<kBesideItems, (KT < 128)>(f, work, id - first, smem), a, a.sync + kSyncSlot0, first);
+    }
+  } else {
+    SumsAlong<kWithinItems, false> along(f, work, id - (first - work.nblocks), smem + KGeom<Q, BR, NI, KT, kPer>::LDS_BYTES);
+    k64_tile<Q, BR, NI, KT, kPer, true, true, false>(a, at, smem, along);
+  }
+}
+
+struct PairPlan {
+  int ktile;    // channel tile of the data gradient
+  int nx, ny;   // its workgroups, 0: not this way
+  bool beside;
+  AlongWork work;
+};
+
+// calls f(width, rows, images, channel tile, beside?) with the plan's numbers as types
+template <class F>
+auto with_geometry(int H, const PairPlan& p, F f) {
+  using std::integral_constant;
+  const auto tiles = [&](auto q, auto br, auto ni) {
+    if constexpr (decltype(q)::value <= 16) {
+      if (p.ktile == 32) return f(q, br, ni, integral_constant<int, 32>{}, std::true_type{});
+    }
+    if (p.ktile == 64) return p.beside ? f(q, br, ni, integral_constant<int, 64>{}, std::true_type{}) : f(q, br, ni, integral_constant<int, 64>{}, std::false_type{});
+    return p.beside ? f(q, br, ni, integral_constant<int, 128>{}, std::true_type{}) : f(q, br, ni, integral_constant<int, 128>{}, std::false_type{});
+  };
+  if (H == 32) return tiles(integral_constant<int, 32>{}, integral_constant<int, 8>{}, integral_constant<int, 1>{});
+  if (H == 16) return tiles(integral_constant<int, 16>{}, integral_constant<int, 16>{}, integral_constant<int, 1>{});
+  return tiles(integral_constant<int, 8>{}, integral_constant<int, 8>{}, integral_constant<int, 4>{});
+}
+
+constexpr size_t kHalfLds = 80 * 1024;   // two workgroups on a unit
+
+// Whether two of the plan's workgroups fit on a compute unit, in LDS for its chunks and in registers
+bool fits_twice(int H, const PairPlan& p) {
+  return with_geometry(H, p, [&](auto q, auto br, auto ni, auto kt, auto beside) {
+    constexpr int Q = decltype(q)::value, BR = decltype(br)::value, NI = decltype(ni)::value, KT = decltype(kt)::value;
+    constexpr bool kBeside = decltype(beside)::value;
+    using G = KGeom<Q, BR, NI, KT, per_cu_geometry(KT)>;
+    static_assert(G::LDS_BYTES <= kHalfLds, "two workgroups on a unit");
+    static_assert(8 * 32 * G::PT * (G::NWF * 32 + 16) <= G::TILE_BYTES, "int8 patches must stay clear of the reduction words");
+    if (p.work.own > 8 * (kBeside ? kBesideItems : kWithinItems) || along_lds(p.work.own) + (kBeside ? 0 : G::LDS_BYTES) > kHalfLds) return false;
+    static bool of[kDeviceSlots] = {};
+    bool& twice = of[device_slot()];
+    if (!twice) {
+      auto k = conv3x3_k64_backward_kernel<Q, BR, NI, KT, kBeside>;
+      int per_cu = 0;
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfLds) != hipSuccess ||
+          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k), 512, kHalfLds) != hipSuccess)
+        return false;
+      twice = per_cu >= 2;
+    }
+    return twice;
+  });
+}
+
+PairPlan pair_plan(int N, int H, int C, int K) {
+  PairPlan p{};
+  if (H != 8 && H != 16 && H != 32) return p;
+  if (C % 64 != 0 || K <= 64 || (K + 31) / 32 % 2 != 0 || !conv3x3_halo_supported(N, H, H, K, C, 3, 3, 1, 1)) return p;   // the data gradient: K -> C
+  const int slices = wgrad3x3_planes_blocks(N, H, C, K) / (((K + 127) / 128) * (C / 32));
+  if (slices == 0) return p;
+  const int cus = compute_units();
+  const long long ptiles = (static_cast<long long>(N) * H * H + 255) / 256, units = static_cast<long long>(K) * 9 * C / 4;
+  const auto blocks = [&](int ktile) { return ptiles * ((C + ktile - 1) / ktile); };
+  p.ktile = H <= 16 && blocks(32) <= cus ? 32 : C == 64 || blocks(64) <= cus ? 64 : 128;
+  const long long nb = blocks(p.ktile);
+  if (nb < 2 || nb > 2LL * cus) return PairPlan{};
+  p.nx = static_cast<int>(ptiles);
+  p.ny = (C + p.ktile - 1) / p.ktile;
+  const int room = static_cast<int>(2LL * cus - nb);
+  p.beside = room >= cus / 4;
+  // Where those that multiply fill the device, the later ones of the two on each unit add the slices before their first stage: their
+  // neighbours have the matrix units to themselves meanwhile (128 images of 32 x 32, 128 -> 128: 8.5 us, of which 4 show).
+  p.work = along_work(units, slices, p.beside && room < cus ? room : cus);
+  return fits_twice(H, p) ? p : PairPlan{};
+}
+
+size_t finish_words(const PairPlan& p) { return static_cast<size_t>(kFinishSlot0) + slot_words(p.work.nblocks); }
+
+}  // namespace
+
+size_t conv_pair_words(int N, int H, int C, int K) {
+  const PairPlan p = pair_plan(N, H, C, K);
+  if (p.nx == 0) return 0;
+  return conv3x3_halo_sync_words(p.nx * p.ny) + finish_words(p) + static_cast<size_t>(wgrad3x3_planes_blocks(N, H, C, K)) + 1;
+}
+// Least squares over 420 layers of 64 to 512 channels, 2 to 300 images of 8 x 8 to 32 x 32, in replayed graphs: 7% rms.
+double conv_pair_us(int N, int H, int C, int K, double dgrad_us) {
+  int bands = 0;
+  if (wgrad3x3_planes_blocks(N, H, C, K, &bands) == 0) return 0.0;
+  return 9.5 + 1.85 * bands + 0.2e-6 * static_cast<double>(wgrad3x3_workspace(N, H, C, K)) + 0.85 * dgrad_us;
+}
+size_t conv_pair_workspace(int N, int H, int C, int K) { return pair_plan(N, H, C, K).nx == 0 ? 0 : wgrad3x3_workspace(N, H, C, K); }
+
+int launch_conv_pair(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx, int N, int H, int C, int K, bool roundtrip, uint32_t* sync,
+                     const RequantSpec& rq, const RequantSpec& grad, int8_t* g8, int8_t* wprep, void* workspace, hipStream_t stream) {
+  const PairPlan p = pair_plan(N, H, C, K);
+  if (p.nx == 0) return fail(NITI_ERR_UNSUPPORTED, "conv_backward_pair: shape not covered");
+  HaloArgs a;
+  int st = halo_requant_args(a, err, wprep, dx, N, H, K, C, (roundtrip ? NITI_EPI_F32_ROUNDTRIP : 0u) | NITI_CONV_FILTER_FORWARD_COPY, sync, rq);
+  if (st != NITI_OK) return st;
+  uint32_t* const sync_w = sync + conv3x3_halo_sync_words(p.nx * p.ny);
+  FinishArgs f;
+  st = launch_wgrad3x3_planes(act, err, w, N, H, C, K, roundtrip, sync_w, sync_w + finish_words(p), grad, g8, wprep, workspace, &f, stream);
+  if (st != NITI_OK) return st;
+  return with_geometry(H, p, [&](auto q, auto br, auto ni, auto kt, auto beside) {
+    constexpr int Q = decltype(q)::value, BR = decltype(br)::value, NI = decltype(ni)::value, KT = decltype(kt)::value;
+    constexpr bool kBeside = decltype(beside)::value;
+    constexpr size_t own = KGeom<Q, BR, NI, KT, per_cu_geometry(KT)>::LDS_BYTES;
+    const size_t sums = along_lds(p.work.own), lds = kBeside ? (own > sums ? own : sums) : own + sums;
+    hipLaunchKernelGGL((conv3x3_k64_backward_kernel<Q, BR, NI, KT, kBeside>), dim3(p.nx * p.ny + (kBeside ? p.work.nblocks : 0)), dim3(512), lds, stream, a, f, p.work, p.nx,
+                       p.ny);
+    return check_launch("conv3x3_k64_backward");
+  });
+}
+
+}  // namespace niti

@@ -39,4 +39,12 @@ size_t conv_backward_workspace(const ConvShape& s);
 int launch_conv_backward(const ConvShape& s, const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx, bool roundtrip, uint32_t* sync, const RequantSpec& rq,
                          const RequantSpec& grad, int8_t* g8, int8_t* wprep, void* workspace, hipStream_t stream);
 
+// Both gradients of a 3x3 layer on H x H maps as the weight gradient's sums and the data gradient with the update beside it
+// (conv3x3_k64_backward.hip); wprep is the filter copy that the data gradient reads.  words 0: not a shape of these kernels.
+size_t conv_pair_words(int N, int H, int C, int K);
+double conv_pair_us(int N, int H, int C, int K, double dgrad_us);   // estimated time, dgrad_us the data gradient's by itself
+size_t conv_pair_workspace(int N, int H, int C, int K);
+int launch_conv_pair(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx, int N, int H, int C, int K, bool roundtrip, uint32_t* sync,
+                     const RequantSpec& rq, const RequantSpec& grad, int8_t* g8, int8_t* wprep, void* workspace, hipStream_t stream);
+
 }  // namespace niti

@@ -496,7 +496,7 @@ bool weight_gradient(bool fuse, const at::Tensor& act, const at::Tensor& err, co
   return false;
 }
 
-// both in one call where niti_conv2d_i8_backward covers them
+// both in one call where niti_conv2d_i8_backward or niti_conv2d_i8_backward_pair covers them
 bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tensor& w, const Fused& f, Opt pool_in, const WeightGradient& g, DataGradient* r,
                     Update* u, const at::Tensor& e) {
   if (f.stride != 1 || g.want_dw || g.rand != nullptr || g.r.method == NITI_ROUND_STOCHASTIC || act.size(3) != w.size(3)) return false;
@@ -513,23 +513,27 @@ bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tens
     shape = {d.N, 2LL * d.H, 2LL * d.W, d.C};
     if (sto || f.mask == nullptr || !is_i8(*pool_in) || !has_shape(*pool_in, shape)) pool_in = nullptr, shape = {d.N, d.H, d.W, d.C};
   }
-  const size_t words = niti_conv2d_i8_backward_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
+  size_t words = 0;
+  if (!sto && f.prepared != nullptr && g.prepared != nullptr && f.prepared->data_ptr() == g.prepared->data_ptr())
+    words = niti_conv2d_i8_backward_pair_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
+  const bool pair = words != 0;
+  if (!pair) words = niti_conv2d_i8_backward_sync_words(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
   if (words == 0) return false;
   want_copy(g.prepared, d, 1, f.pad, 0, "conv layer");
-  const size_t bytes = niti_conv2d_i8_backward_workspace(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
+  const size_t bytes = (pair ? niti_conv2d_i8_backward_pair_workspace : niti_conv2d_i8_backward_workspace)(d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad);
   at::Tensor ws;
   if (bytes > 0) ws = scratch(bytes, act);
   uint32_t* sync = arena_take(static_cast<long>(words), act, nullptr);
   r->y = empty8(shape, act);
   if (g.want_grad) u->g8 = empty8(w.sizes(), w);
   u->shift = g.shift != nullptr ? *g.shift : scalar32(w);
-  const int rc = niti_conv2d_i8_backward(
+  const int rc = (pair ? niti_conv2d_i8_backward_pair : niti_conv2d_i8_backward)(
       ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), ptr<int8_t>(r->y), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad,
-      g.flags | (g.shift != nullptr ? NITI_CONV_SHIFT_HINT : 0u), f.r.bits, f.r.method, sto ? ptr<int32_t>(f.rand) : nullptr, ptr<int8_t>(f.mask),
+      g.flags | ((pair ? f.shift : g.shift) != nullptr ? NITI_CONV_SHIFT_HINT : 0u), f.r.bits, f.r.method, sto ? ptr<int32_t>(f.rand) : nullptr, ptr<int8_t>(f.mask),
       ptr<int8_t>(pool_in), f.ties, g.r.bits, g.r.method, f.r.div, f.r.bw, sync, words, g.want_grad ? ptr<int8_t>(u->g8) : nullptr, ptr<int8_t>(g.prepared),
       ptr<int32_t>(f.shift), ptr<int32_t>(u->shift), ptr<int32_t>(f.exp_a), ptr<int32_t>(f.exp_b), ptr<int32_t>(g.exp_b), ptr<int32_t>(r->e), ptr<int32_t>(e),
       bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(act));
-  if (!check_fits(rc, "niti_conv2d_i8_backward")) return false;
+  if (!check_fits(rc, pair ? "niti_conv2d_i8_backward_pair" : "niti_conv2d_i8_backward")) return false;
   r->unpooled = pool_in != nullptr;
   return true;
 }

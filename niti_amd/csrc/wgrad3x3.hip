@@ -19,7 +19,8 @@
 // over gridDim.z workgroups; each writes its partial sums to a workspace slice and a second
 // kernel adds the slices (integer addition: any split gives the same result).  The arrangement with
 // 128 x 32 tiles (wgrad3x3_narrow_kernel) can also add the slices itself, at the end of the same
-// launch, once all of its workgroups - resident together - have written theirs.
+// launch, once all of its workgroups - resident together - have written theirs, or leave them to the data gradient's launch
+// (conv3x3_k64_backward.hip).
 #include <stdlib.h>
 
 #include <type_traits>
@@ -28,6 +29,7 @@
 #include "conv_any.h"
 #include "lds_asm.h"
 #include "requant_math.h"
+#include "wgrad_finish.h"
 
 namespace niti {
 namespace {
@@ -327,322 +329,6 @@ __global__ __launch_bounds__(512, 1) void wgrad3x3_kernel(const WgradArgs a) {
   }
 }
 
-// Partial sums -> rounded gradient -> updated weights in one launch (the int32 gradient is not stored unless
-// asked for).  A workgroup owns kFinishV x 64 int4 columns at a grid-wide stride; its NW wavefronts each add every
-// NW-th slice of every column (no barrier in between, so all those loads are in flight together), column v is
-// then completed through LDS by wavefront v % NW, which keeps the sums in registers.  The workgroup publishes its
-// largest magnitude in its slot and waits for the slots of all workgroups (all resident: the host sizes the grid
-// for that; the wait is bounded by a wall-clock limit), derives the shift from the maximum over the slots, and
-// every wavefront applies w = clip(w - round(sum >> shift)) to its columns.  NW = 16 serves the launches with
-// many slices and few columns, NW = 4 the others.
-constexpr int kFinishV = 16;
-constexpr int kFusedV = 48;         // columns per lane in the one-launch form (8 wavefronts: six each)
-constexpr int kArriveSlots = 256;   // workgroups of the one-launch form at most
-constexpr uint32_t kPartialBias = 1u << 23;   // added to the partial sums of the one-launch form before they are cut to 24 bits
-constexpr int kFinishSlot0 = 16;
-struct FinishArgs {
-  const int32_t* partial;
-  long long slice_stride;
-  int splits;
-  long long nv;        // int4 columns of the gradient: K*9*C / 4
-  int C, Cw;           // channels per gradient row / per weight row (Cw <= C; the rest is channel padding)
-  int8_t* w;           // [K][9][Cw], updated in place
-  int8_t* g8;          // optional rounded gradient, laid out like w
-  int32_t* dw;         // optional int32 gradient [K][9][C]
-  int8_t* wprep;       // optional: the halo convolution kernel's forward copy of the [K][9][C] filter, kept in step with w
-  uint32_t* sync;      // word 0: max |sum| (output); word 1: wait gave up; words kFinishSlot0..: slots, zero on entry
-  int roundtrip, target_bits, method, trunc, bw_mode;
-  int predict;         // *shift_out holds a predicted shift on entry
-  long long spin_limit;
-  uint32_t* sticky;    // device-wide word set when the wait gives up, may be null
-  int32_t* shift_out;
-  const int32_t* exp_a;
-  const int32_t* exp_b;
-  int32_t* exp_out;
-  uint32_t* arrive;    // one-launch form only: a slot per workgroup, zero on entry, filled when its partial sums are in memory
-  // one-launch form only.  A slice then holds, per group of four consecutive output channels kg, tap t and input channel
-  // c (unit u = (kg * 9 + t) * C + c), three planes: bits 0..15 of the four sums (8 bytes at 8u), bits 16..23 (4 bytes at
-  // units * 8 + 4u) and bits 24..31 (4 bytes at units * 12 + 4u).  The third plane is written only by a workgroup whose
-  // sums do not fit 24 bits; it says so in wide[tile + tiles * slice] (zero on entry) and in the value of its arrival slot.
-  uint32_t* wide;
-  int tiles_k, tiles_c;
-};
-
-typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-
-template <int NW>
-struct FinishShared {
-  v4i part[2][NW][64];
-  uint32_t wmax[NW];
-  uint32_t gshare;
-};
-
-// The finishing pass of workgroup `block` out of `nblocks` (V = int4 columns per lane it may own, NW its wavefronts).
-// predicted_raw: the word read from a.shift_out (or anything when there is no prediction) at kernel start.
-// any_wide (uniform): some workgroup wrote the third plane (top bytes) of its part of its slice.
-// kCoherent: the partial sums were written by this same launch (by other dies' workgroups, with write-through stores): they
-// are read with loads that do not hit a line another die may have changed (byte offsets then fit 31 bits: host check).
-template <int NW, int V, bool kCoherent = false>
-__device__ __forceinline__ void finish_columns(const FinishArgs& a, const int block, const int nblocks, FinishShared<NW>& sh,
-                                               const int predicted_raw, const bool any_wide = false) {
-  const __amdgpu_buffer_rsrc_t rpart =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(a.partial), 0, kCoherent ? static_cast<int>(a.slice_stride * a.splits * 4) : 0, 0x00020000);
-  constexpr int kSc1 = 16;   // cache policy bit: coherent across the dies' L2 caches
-  const int units = static_cast<int>(a.nv);   // kCoherent: a column is a unit (four output channels), not four input channels
-  // kMixed = false: no workgroup wrote a third plane, every sum is the sign-extended 24-bit value
-  auto slice_col = [&](auto mixed, int z, long long col) -> v4i {
-    if constexpr (kCoherent) {
-      const int zoff = __builtin_amdgcn_readfirstlane(static_cast<int>(z * a.slice_stride * 4));   // z is the same in all lanes
-      const v2u lo = __builtin_amdgcn_raw_buffer_load_b64(rpart, static_cast<int>(col) * 8, zoff, kSc1);
-      const uint32_t mid = __builtin_amdgcn_raw_buffer_load_b32(rpart, units * 8 + static_cast<int>(col) * 4, zoff, kSc1);
-      v4i r;   // biased sums, 24 bits each
-      r[0] = static_cast<int>(__builtin_amdgcn_perm(mid, lo[0], 0x0C040100u));   // 0, mid.b0, lo.b1, lo.b0
-      r[1] = static_cast<int>(__builtin_amdgcn_perm(mid, lo[0], 0x0C050302u));
-      r[2] = static_cast<int>(__builtin_amdgcn_perm(mid, lo[1], 0x0C060100u));
-      r[3] = static_cast<int>(__builtin_amdgcn_perm(mid, lo[1], 0x0C070302u));
-      if constexpr (decltype(mixed)::value) {   // rare: the writer of this column's tile in slice z tells whether it wrote top bytes
-        const uint32_t rt = static_cast<uint32_t>(col) / static_cast<uint32_t>(a.C);   // kg * 9 + t
-        const uint32_t tile = (rt / 9u >> 5) + static_cast<uint32_t>(a.tiles_k) * ((static_cast<uint32_t>(col) - rt * static_cast<uint32_t>(a.C)) >> 5);
-        const bool wide = __hip_atomic_load(a.wide + tile + static_cast<uint32_t>(a.tiles_k * a.tiles_c) * static_cast<uint32_t>(z), __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT) != 0u;
-        uint32_t hi = 0;
-        if (wide) hi = __builtin_amdgcn_raw_buffer_load_b32(rpart, units * 12 + static_cast<int>(col) * 4, zoff, kSc1);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = static_cast<int>(static_cast<uint32_t>(r[e]) | ((hi >> (8 * e)) << 24));
-      }
-      return r;
-    } else {
-      return reinterpret_cast<const v4i*>(a.partial + z * a.slice_stride)[col];
-    }
-  };
-  constexpr int OWN = V / NW > 0 ? V / NW : 1;   // columns a wavefront completes
-  constexpr int VS = V < NW ? V : NW;            // columns a workgroup has when the slices are shared (fewer rounds than wavefronts)
-  auto& part = sh.part;
-  auto& wmax = sh.wmax;
-  uint32_t& gshare = sh.gshare;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool has_prediction = a.predict != 0 && a.shift_out != nullptr;
-  const bool trunc = a.trunc != 0;
-  const bool psto = a.method == NITI_ROUND_PSEUDO_STOCHASTIC;
-  const bool same_layout = a.Cw == a.C;
-  const uint32_t C = static_cast<uint32_t>(a.C), Cw = static_cast<uint32_t>(a.Cw);
-  // division by the channel count: a shift for the usual powers of two (a 32-bit division is some forty instructions,
-  // and this part of the launch runs few wavefronts)
-  const int c_log2 = (C & (C - 1u)) == 0u ? 31 - __builtin_clz(C) : -1;
-  auto div_c = [&](uint32_t x) -> uint32_t { return c_log2 >= 0 ? x >> c_log2 : x / C; };
-  auto out_col = [&](long long col) -> long long {
-    if constexpr (kCoherent) {
-      const uint32_t rt = div_c(static_cast<uint32_t>(col)), c = static_cast<uint32_t>(col) - rt * C, kg = rt / 9u, tap = rt - kg * 9u;
-      return static_cast<long long>(((kg * 4u + (c & 3u)) * 9u + tap) * (C >> 2) + (c >> 2));
-    } else {
-      return col;
-    }
-  };
-  // the old weights are requested first: they depend on nothing and are wanted right after the sums
-  uint32_t wold[OWN];
-#pragma unroll
-  for (int j = 0; j < OWN; ++j) {
-    const int v = j * NW + wave;
-    const long long col = (static_cast<long long>(v) * nblocks + block) * 64 + lane;
-    wold[j] = (same_layout && v < V && col < a.nv) ? reinterpret_cast<const uint32_t*>(a.w)[out_col(col)] : 0u;
-  }
-  v4i fin[OWN];
-  uint32_t lmax = 0;
-  // Every wavefront has columns of its own at least in the first round (uniform over the grid): then each adds all
-  // slices of its own columns and nothing goes through LDS.  With fewer columns than wavefronts the slices are
-  // shared instead (phases 1 and 2 below), so that no wavefront idles while another walks over all slices.
-  const bool direct = a.nv >= static_cast<long long>(NW) * nblocks * 64;
-  // the whole gathering phase exists twice, so that the usual case (no third plane anywhere) has no branch between
-  // its loads and keeps them all in flight
-  const int bias_total = kCoherent ? static_cast<int>(static_cast<uint32_t>(a.splits) * kPartialBias) : 0;   // modulo 2^32, as the sums
-  auto gather = [&](auto mixed) {
-  if (direct) {
-#pragma unroll
-    for (int j = 0; j < OWN; ++j) {
-      const int v = j * NW + wave;
-      const long long col = (static_cast<long long>(v) * nblocks + block) * 64 + lane;
-      v4i s = {0, 0, 0, 0};
-      if (v < V && col < a.nv) {
-        int z = 0;
-        for (; z + 3 < a.splits; z += 4) {
-          const v4i v0 = slice_col(mixed, z + 0, col);
-          const v4i v1 = slice_col(mixed, z + 1, col);
-          const v4i v2 = slice_col(mixed, z + 2, col);
-          const v4i v3 = slice_col(mixed, z + 3, col);
-          s += (v0 + v1) + (v2 + v3);
-        }
-        for (; z < a.splits; ++z) s += slice_col(mixed, z, col);
-        s -= bias_total;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (a.roundtrip) s[e] = f32_roundtrip(s[e]);
-        const uint32_t u = uabs(s[e]);
-        lmax = u > lmax ? u : lmax;
-      }
-      fin[j] = s;
-    }
-  } else {
-  v4i sum[VS];
-  // phase 1: every wavefront adds its share of the slices for all of the workgroup's columns
-#pragma unroll
-  for (int v = 0; v < VS; ++v) {
-    const long long col = (static_cast<long long>(v) * nblocks + block) * 64 + lane;
-    v4i s = {0, 0, 0, 0};
-    if (col < a.nv) {
-      int z = wave;
-      for (; z + 3 * NW < a.splits; z += 4 * NW) {
-        const v4i v0 = slice_col(mixed, z + 0 * NW, col);
-        const v4i v1 = slice_col(mixed, z + 1 * NW, col);
-        const v4i v2 = slice_col(mixed, z + 2 * NW, col);
-        const v4i v3 = slice_col(mixed, z + 3 * NW, col);
-        s += (v0 + v1) + (v2 + v3);
-      }
-      for (; z < a.splits; z += NW) s += slice_col(mixed, z, col);
-    }
-    sum[v] = s;
-  }
-  // phase 2: column v is completed by wavefront v % NW (two LDS buffers in turn: one barrier per column)
-#pragma unroll
-  for (int v = 0; v < VS; ++v) {
-    if (static_cast<long long>(v) * nblocks * 64 >= a.nv) continue;  // uniform over the grid: nothing at this stride
-    part[v & 1][wave][lane] = sum[v];
-    __syncthreads();
-    if (wave == v % NW) {
-      v4i s = part[v & 1][0][lane];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) s += part[v & 1][w][lane];
-      if ((static_cast<long long>(v) * nblocks + block) * 64 + lane < a.nv) s -= bias_total;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (a.roundtrip) s[e] = f32_roundtrip(s[e]);
-        const uint32_t u = uabs(s[e]);
-        lmax = u > lmax ? u : lmax;
-      }
-      fin[v / NW] = s;
-    }
-  }
-  }
-  };
-  if (kCoherent && any_wide) gather(std::true_type{});
-  else gather(std::false_type{});
-  // kCoherent: a lane holds four output channels of one input channel, its quad four consecutive input channels: a
-  // 4 x 4 transposition inside the quad (two rounds of swaps) gives every lane four input channels of one output
-  // channel, the form of the weights in memory, and out_col the column that is (quads lie inside one row: C % 4 == 0)
-  if constexpr (kCoherent) {
-    const bool odd1 = (lane & 1) != 0, odd2 = (lane & 2) != 0;
-#pragma unroll
-    for (int j = 0; j < OWN; ++j) {
-      v4i s = fin[j], x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_mov_dpp(s[e ^ 1], 0xB1, 0xf, 0xf, true);   // quad_perm:[1,0,3,2]
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = (((e & 1) != 0) == odd1) ? s[e] : x[e];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_mov_dpp(s[e ^ 2], 0x4E, 0xf, 0xf, true);   // quad_perm:[2,3,0,1]
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = (((e & 2) != 0) == odd2) ? s[e] : x[e];
-      fin[j] = s;
-    }
-  }
-  lmax = wave_max_u32(lmax);
-  if (lane == 0) wmax[wave] = lmax;
-  __syncthreads();
-  uint32_t bmax = 0;   // the workgroup's largest magnitude, in every wavefront
-#pragma unroll
-  for (int w = 0; w < NW; ++w) bmax = max(bmax, wmax[w]);
-  if (wave == 0 && lane == 0)
-    __hip_atomic_store(slot_word(a.sync + kFinishSlot0, block), bmax + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-
-  // phase 3: every wavefront rounds its columns and updates their weights (element counts fit 31 bits: host check).
-  // With a predicted shift (a.predict) the update is applied before the range is final, so that its stores overlap
-  // the wait for the other workgroups, and applied once more from the same old weights if the final shift differs.
-  // shift: the same in every lane, but it has come through LDS or memory, which the compiler cannot know - as a scalar
-  // the choices below are scalar branches instead of both sides under execution masks
-  auto apply = [&](int shift_any, bool first) {
-    const int shift = __builtin_amdgcn_readfirstlane(shift_any);
-#pragma unroll
-    for (int j = 0; j < OWN; ++j) {
-      const int v = j * NW + wave;
-      if (v >= V) continue;
-      const long long gcol = (static_cast<long long>(v) * nblocks + block) * 64 + lane;
-      if (gcol >= a.nv) continue;
-      const long long col = out_col(gcol);
-      const v4i s = fin[j];
-      if (first && a.dw != nullptr) reinterpret_cast<v4i*>(a.dw)[col] = s;
-      int r[4];
-      if (shift < 1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = wrap_to_i8(s[e]);
-      } else if (psto) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(s[e], shift, trunc);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_NEAREST>(s[e], shift, trunc);
-      }
-      const uint32_t e0 = static_cast<uint32_t>(col) * 4u;
-      const uint32_t rt = div_c(e0);            // k * 9 + tap
-      const uint32_t c0 = e0 - rt * C;
-      uint32_t wnew = 0;   // the four updated weights (zero where the gradient column is channel padding)
-      if (same_layout) {
-        uint32_t gp = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int wo = static_cast<int>(static_cast<int8_t>((wold[j] >> (8 * e)) & 0xFFu));
-          wnew |= (static_cast<uint32_t>(clip127(wo - r[e])) & 0xFFu) << (8 * e);
-          gp |= (static_cast<uint32_t>(r[e]) & 0xFFu) << (8 * e);
-        }
-        reinterpret_cast<uint32_t*>(a.w)[col] = wnew;
-        if (a.g8 != nullptr) reinterpret_cast<uint32_t*>(a.g8)[col] = gp;
-      } else {   // applied once only (the old weights are read here)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (c0 + e < Cw) {
-            const uint32_t wi = rt * Cw + c0 + e;
-            const int wn = clip127(static_cast<int>(a.w[wi]) - r[e]);
-            a.w[wi] = static_cast<int8_t>(wn);
-            wnew |= (static_cast<uint32_t>(wn) & 0xFFu) << (8 * e);
-            if (a.g8 != nullptr) a.g8[wi] = static_cast<int8_t>(r[e]);
-          }
-        }
-      }
-      if (a.wprep != nullptr) {
-        // [64-channel group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
-        const uint32_t k = rt / 9u, tap = rt - k * 9u;
-        const uint32_t row = k & 63u, cs = c0 >> 5;
-        const uint32_t half = ((c0 >> 4) & 1u) ^ ((row >> 3) & 1u);
-        const uint32_t dst = (((((k >> 6) * ((C + 31u) >> 5) + cs) * 9u + tap) * 64u + row) << 5) + half * 16u + (c0 & 15u);
-        *reinterpret_cast<uint32_t*>(a.wprep + dst) = wnew;
-      }
-    }
-  };
-  const bool speculate = a.predict != 0 && same_layout && nblocks > 1;
-  int applied = -1;
-  if (speculate) {
-    applied = max(max(bitwidth_of(bmax, a.bw_mode) - a.target_bits, 0), has_prediction ? predicted_raw : 0);
-    apply(applied, true);
-  }
-  if (wave == 0) {
-    const uint32_t g = wait_slots(a.sync + kFinishSlot0, nblocks, a.spin_limit, &a.sync[1], a.sticky);
-    if (lane == 0) gshare = g != 0u ? g - 1u : 0u;
-  }
-  __syncthreads();
-  const uint32_t gmax = gshare;
-  const int shift = max(bitwidth_of(gmax, a.bw_mode) - a.target_bits, 0);
-  if (block == 0 && threadIdx.x == 0) {
-    a.sync[0] = gmax;
-    if (a.shift_out != nullptr) *a.shift_out = shift;
-    if (a.exp_out != nullptr)
-      *a.exp_out = shift + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
-  }
-  if (shift != applied) {
-    if (applied >= 0) __builtin_amdgcn_s_waitcnt(0);   // the first update's stores leave before those that replace them
-    apply(shift, applied < 0);
-  }
-}
-
 // ---- the same computation with half the partial-sum traffic ------------------------------------------------
 // The kernel above leaves 128 x 64 x 9 partial sums (295 KB) per workgroup in memory; with about one workgroup
 // per compute unit that is almost 60 MB per launch, written and read again, whatever the layer - more time than
@@ -672,15 +358,22 @@ struct NGeom {
   static_assert(LDS_BYTES <= 160 * 1024, "stages must fit in LDS");
 };
 
+// What becomes of a workgroup's sums
+enum NarrowMode {
+  kSlicesOut,    // int32 slices, added by another launch
+  kFinishHere,   // planes, added by the same launch
+  kPlanesOut,    // planes, added beside the data gradient that follows (conv3x3_k64_backward.hip)
+};
+
 // kHalfK (at most 64 output channels): the wavefronts are 2 channel quarters x 4 pixel quarters instead of 4 x 2, so
 // that none multiplies channels that do not exist.
-template <int Q, int BR, int NI, bool kFinish, bool kHalfK>
+template <int Q, int BR, int NI, int kMode, bool kHalfK>
 __global__ __launch_bounds__(512, 1) void wgrad3x3_narrow_kernel(const WgradArgs a, const FinishArgs f) {
   using G = NGeom<Q, BR, NI>;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t* const dump = smem + G::LDS_BYTES - 1024;
   int predicted_raw = 0;
-  if constexpr (kFinish) {
+  if constexpr (kMode == kFinishHere) {
     // read at kernel start, looked at in the finishing part (see wgrad_finish_kernel)
     const bool has_prediction = f.predict != 0 && f.shift_out != nullptr;
     predicted_raw = __hip_atomic_load((has_prediction ? f.shift_out : reinterpret_cast<const int32_t*>(f.sync)) + opaque_zero(),
@@ -849,7 +542,7 @@ __global__ __launch_bounds__(512, 1) void wgrad3x3_narrow_kernel(const WgradArgs
   __syncthreads();
   // partial sums: acc[t][4g+e] = dw[k0+wk*32+8g+4*lk+e][tap t][c0+(lane&31)]
   const int c = c0 + (lane & 31);
-  if constexpr (!kFinish) {
+  if constexpr (kMode == kSlicesOut) {
     if (ph == 0) {
       int32_t* out = a.partial + static_cast<long long>(item.z) * a.slice_stride;
 #pragma unroll
@@ -876,7 +569,7 @@ __global__ __launch_bounds__(512, 1) void wgrad3x3_narrow_kernel(const WgradArgs
     // reader adds zero-extended 24-bit numbers and takes the bias off once per column.
     const __amdgpu_buffer_rsrc_t rout =
         __builtin_amdgcn_make_buffer_rsrc(a.partial, 0, static_cast<int>(a.slice_stride * f.splits * 4), 0x00020000);
-    constexpr int kSc1 = 16;   // written through to memory
+    constexpr int kSc1 = 16;   // written through to memory (for the next launch it is faster as well: 0.3 - 1.1 us a pair of launches)
     const int zoff = static_cast<int>(item.z * a.slice_stride * 4);
     const int units = static_cast<int>(f.nv);
     uint32_t over = 0;   // bits above the 24 of any biased value
@@ -927,6 +620,10 @@ __global__ __launch_bounds__(512, 1) void wgrad3x3_narrow_kernel(const WgradArgs
           __builtin_amdgcn_raw_buffer_store_b32(h01 | h23, rout, live ? units * 12 + u * 4 : kOob, zoff, kSc1);
         }
       }
+    }
+    if constexpr (kMode == kPlanesOut) {
+      if (wide && tid == 0) f.wide[item.x + f.tiles_k * (item.y + f.tiles_c * item.z)] = f.wide[f.tiles_k * f.tiles_c * f.splits] = 1u;
+      return;
     }
     const int nblocks = static_cast<int>(gridDim.x * gridDim.y * gridDim.z);
     const int block = static_cast<int>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
@@ -1030,20 +727,20 @@ int pick_splits(int N, int Q, int C, int K) {
   return (bands + per - 1) / per;
 }
 
-// f != nullptr: the one-launch form (main loop + finishing pass); returns NITI_ERR_UNSUPPORTED without launching when its
+// kFinishHere: the one-launch form (main loop + finishing pass); returns NITI_ERR_UNSUPPORTED without launching when its
 // grid would not be resident at once, and the caller then runs the pair of launches.
-template <int Q, int BR, int NI, bool kFinish, bool kHalfK>
+template <int Q, int BR, int NI, int kMode, bool kHalfK>
 int launch_narrow_geom_as(const WgradArgs& a, int splits, hipStream_t stream, const FinishArgs& f) {
   using G = NGeom<Q, BR, NI>;
   constexpr size_t lds = G::LDS_BYTES;
-  auto k = wgrad3x3_narrow_kernel<Q, BR, NI, kFinish, kHalfK>;
+  auto k = wgrad3x3_narrow_kernel<Q, BR, NI, kMode, kHalfK>;
   static bool attr_set_of[kDeviceSlots] = {};   // function attributes are per device
   static int resident_of[kDeviceSlots] = {};    // workgroups of this kernel the device holds at once
   bool& attr_set = attr_set_of[device_slot()];
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return fail(NITI_ERR_LAUNCH, "wgrad: cannot reserve %zu bytes of LDS", lds);
-    if (kFinish) {
+    if (kMode == kFinishHere) {
       int dev = 0, cus = 0, per = 0;
       if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k), 512, lds) != hipSuccess)
@@ -1053,7 +750,7 @@ int launch_narrow_geom_as(const WgradArgs& a, int splits, hipStream_t stream, co
     attr_set = true;
   }
   dim3 grid((a.K + 127) / 128, (a.C + 31) / 32, splits);
-  if (kFinish) {
+  if (kMode == kFinishHere) {
     const long long nblocks = static_cast<long long>(grid.x) * grid.y * grid.z;
     if (nblocks > resident_of[device_slot()] || nblocks > kArriveSlots || f.nv > nblocks * kFusedV * 64 ||
         f.slice_stride * f.splits * 4 >= 0x7fffffffLL)
@@ -1064,16 +761,17 @@ int launch_narrow_geom_as(const WgradArgs& a, int splits, hipStream_t stream, co
 }
 
 template <int Q, int BR, int NI>
-int launch_narrow_geom(const WgradArgs& a, int splits, hipStream_t stream, const FinishArgs* f) {
+int launch_narrow_geom(const WgradArgs& a, int splits, hipStream_t stream, const FinishArgs* f, NarrowMode mode) {
   if constexpr (Q >= 8) {
     const bool half_k = a.K <= 64;   // two channel quarters x four pixel quarters
-    if (f != nullptr)
-      return half_k ? launch_narrow_geom_as<Q, BR, NI, true, true>(a, splits, stream, *f) : launch_narrow_geom_as<Q, BR, NI, true, false>(a, splits, stream, *f);
-    return half_k ? launch_narrow_geom_as<Q, BR, NI, false, true>(a, splits, stream, FinishArgs{})
-                  : launch_narrow_geom_as<Q, BR, NI, false, false>(a, splits, stream, FinishArgs{});
+    if (mode == kFinishHere)
+      return half_k ? launch_narrow_geom_as<Q, BR, NI, kFinishHere, true>(a, splits, stream, *f) : launch_narrow_geom_as<Q, BR, NI, kFinishHere, false>(a, splits, stream, *f);
+    if (mode == kPlanesOut) return launch_narrow_geom_as<Q, BR, NI, kPlanesOut, false>(a, splits, stream, *f);
+    return half_k ? launch_narrow_geom_as<Q, BR, NI, kSlicesOut, true>(a, splits, stream, FinishArgs{})
+                  : launch_narrow_geom_as<Q, BR, NI, kSlicesOut, false>(a, splits, stream, FinishArgs{});
   } else {
-    if (f != nullptr) return NITI_ERR_UNSUPPORTED;
-    return launch_narrow_geom_as<Q, BR, NI, false, false>(a, splits, stream, FinishArgs{});
+    if (mode != kSlicesOut) return NITI_ERR_UNSUPPORTED;
+    return launch_narrow_geom_as<Q, BR, NI, kSlicesOut, false>(a, splits, stream, FinishArgs{});
   }
 }
 
@@ -1139,7 +837,7 @@ double wgrad3x3_us(int N, int H, int C, int K, bool* nine_tap) {
 }
 
 static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N, int H, int C, int K, int Cp, void* workspace,
-                                    WgradArgs& a, int& splits, hipStream_t stream, FinishArgs* finish = nullptr) {
+                                    WgradArgs& a, int& splits, hipStream_t stream, FinishArgs* finish = nullptr, NarrowMode mode = kSlicesOut) {
   a.act = act;
   a.err = err;
   a.partial = static_cast<int32_t*>(workspace);
@@ -1163,11 +861,11 @@ static int launch_wgrad3x3_partials(const int8_t* act, const int8_t* err, int N,
     finish->tiles_c = (C + 31) / 32;
   }
   if (narrow) {
-    if (H == 32) return launch_narrow_geom<32, 8, 1>(a, splits, stream, finish);
-    if (H == 16) return launch_narrow_geom<16, 16, 1>(a, splits, stream, finish);
-    if (H == 8) return launch_narrow_geom<8, 8, 4>(a, splits, stream, finish);
-    if (H == 4) return launch_narrow_geom<4, 4, 16>(a, splits, stream, finish);
-    return launch_narrow_geom<2, 2, 64>(a, splits, stream, finish);
+    if (H == 32) return launch_narrow_geom<32, 8, 1>(a, splits, stream, finish, mode);
+    if (H == 16) return launch_narrow_geom<16, 16, 1>(a, splits, stream, finish, mode);
+    if (H == 8) return launch_narrow_geom<8, 8, 4>(a, splits, stream, finish, mode);
+    if (H == 4) return launch_narrow_geom<4, 4, 16>(a, splits, stream, finish, mode);
+    return launch_narrow_geom<2, 2, 64>(a, splits, stream, finish, mode);
   }
   if (H == 32) return launch_geom<32, 4, 1>(a, splits, stream);
   if (H == 16) return launch_geom<16, 8, 1>(a, splits, stream);
@@ -1267,6 +965,24 @@ int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int spli
   return launch_finish(f, partial, slice_stride, splits, stream);
 }
 
+int wgrad3x3_planes_blocks(int N, int H, int C, int K, int* bands) {
+  if (H < 8 || K <= 64 || !wgrad3x3_supported(N, H, H, C, K, 3, 3, 1, 1) || !use_narrow_arrangement(N, H)) return 0;
+  if (static_cast<long long>(wgrad3x3_workspace(N, H, C, K)) >= 0x7fffffffLL) return 0;
+  const int splits = pick_splits(N, H, C, K);
+  if (bands != nullptr) *bands = ((N * H * H + 255) / 256 + splits - 1) / splits;
+  return ((K + 127) / 128) * ((C + 31) / 32) * splits;
+}
+
+int launch_wgrad3x3_planes(const int8_t* act, const int8_t* err, int8_t* w, int N, int H, int C, int K, bool roundtrip, uint32_t* sync, uint32_t* wide,
+                           const RequantSpec& rq, int8_t* g8, int8_t* wprep, void* workspace, FinishArgs* finish, hipStream_t stream) {
+  *finish = finish_args(static_cast<long long>(K) * 9 * C, C, w, C, roundtrip, sync, rq, g8, nullptr);
+  finish->wprep = wprep;
+  finish->wide = wide;
+  WgradArgs a;
+  int splits = 1;
+  return launch_wgrad3x3_partials(act, err, N, H, C, K, C, workspace, a, splits, stream, finish, kPlanesOut);
+}
+
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
                            bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep,
                            void* workspace, hipStream_t stream) {
@@ -1304,7 +1020,7 @@ int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int 
     // main loop and finishing pass as one launch where its grid is resident at once (NITI_WGRAD_ONE_LAUNCH=0 pins the pair)
     const char* e = getenv("NITI_WGRAD_ONE_LAUNCH");
     if (e == nullptr || e[0] != '0') {
-      const int st1 = launch_wgrad3x3_partials(act, err, N, H, C, K, Cp, workspace, a, splits, stream, &f);
+      const int st1 = launch_wgrad3x3_partials(act, err, N, H, C, K, Cp, workspace, a, splits, stream, &f, kFinishHere);
       if (st1 != NITI_ERR_UNSUPPORTED) return st1;
     }
   }

@@ -354,3 +354,100 @@ def test_quantiser_entries_of_the_c_abi(dev):
     L.check(L.lib().niti_quantize_batch_f32_i8(x.data_ptr(), y.data_ptr(), N, C, H, W, 16, 7, parts.data_ptr(), e.data_ptr(), target.data_ptr(),
                                                copied.data_ptr(), 9, ctypes.c_void_p(stream)), "quantize_batch")
     assert torch.equal(y, want) and torch.equal(e, exp) and torch.equal(copied, target)
+
+
+# N, side, C, K of layers whose two gradients run as a pair of launches.  Update beside the data gradient: its tiles of 32, 64 and 128
+# channels on every map; one slice of partial sums and 67, three input-channel groups of 64, batches that end inside a tile; some
+# workgroups for the update fewer than the device has units.  Update by workgroups that multiply as well: 64 and 128 channels.
+PAIRS = [(3, 16, 64, 128), (5, 8, 192, 128), (2, 8, 256, 512), (5, 32, 64, 128), (70, 16, 128, 128), (70, 8, 512, 128), (36, 32, 128, 192), (70, 16, 256, 128),
+         (300, 8, 256, 128), (97, 32, 128, 128), (115, 32, 64, 128), (115, 32, 128, 128), (230, 16, 256, 128), (900, 8, 256, 128)]
+
+
+@pytest.mark.parametrize("case", PAIRS)
+def test_conv_backward_pair(dev, case, monkeypatch):
+    """Both gradients of a 3x3 layer as the weight gradient's sums and the data gradient along with the update: error, mask and
+    pooling as in the one launch, exponents, weights, filter copy, with right, wrong and no predicted shifts."""
+    from niti_amd import _lib, ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    monkeypatch.setenv("NITI_BACKWARD_PAIR", "1")
+    base._say("conv_backward_pair", case)
+    assert _lib.lib().niti_conv2d_i8_backward_pair_sync_words(N, Q, Q, C, K, 3, 3, 1) > 0
+    g = torch.Generator().manual_seed(9800 + N + Q + C + K)
+    x, w, e = ri8(g, N, Q, Q, C), ri8(g, K, 3, 3, C), ri8(g, N, Q, Q, K, lo=-40, hi=40)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    dacc, wacc = co.conv_dgrad(e, w, Q, Q, 1, 1), co.conv_wgrad(x, e, 3, 3, 1, 1)
+    whole = ri8(g, N, 2 * Q, 2 * Q, C, lo=-3, hi=4)      # few values: ties in most windows
+    pooled = po.maxpool_fwd(whole)
+    for kind, err_method, grad_method, off in (("plain", "round", "psto", None), ("mask", "round", "psto", 0), ("mask", "psto", "round", 1), ("first", "round", "psto", -1)):
+        dref, dsh = po.err_calc(dacc, err_method)
+        gref, gsh = po.grad_calc(wacc, 5, grad_method)
+        if kind == "mask":
+            dref = dref * (x > 0)
+        elif kind == "first":
+            dref = po.maxpool_bwd(pooled, dref * (pooled > 0), whole, ties=kind)
+        wd = w.to(dev)
+        prepared = ops.conv_filter_prepare(wd, N, Q, Q, 1, 1)
+        guess = [None, None] if off is None else [scalar(dsh + off), scalar(gsh + off)]
+        dx, de, unpooled, g8, _, sh, ge, one = ops.conv2d_backward(
+            e.to(dev), x.to(dev), wd, err_method=err_method, grad_method=grad_method, relu_mask=None if kind == "plain" else (pooled if kind == "first" else x).to(dev),
+            pool_in=whole.to(dev) if kind == "first" else None, want_grad=True, exp_err=scalar(-4), exp_w=scalar(-3), exp_act=scalar(2), prepared_filter=prepared,
+            err_shift=guess[0], grad_shift=guess[1])
+        assert one and unpooled == (kind == "first")
+        assert torch.equal(dx.cpu(), dref) and int(de.cpu()) == dsh - 7, (kind, off)
+        assert torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh and int(ge.cpu()) == gsh + dsh - 7 + 2, (kind, off)
+        assert off is None or (int(guess[0].cpu()), int(guess[1].cpu())) == (dsh, gsh)
+        assert torch.equal(wd.cpu(), po.weight_update(w, gref)), (kind, off)
+        assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1)), (kind, off)
+    assert not ops.sync_arena.timed_out(dev)
+
+
+@pytest.mark.parametrize("case", [(12, 16, 128, 128), (115, 32, 64, 128)])
+def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
+    """Partial sums that need more than 24 bits, from some workgroups of the weight gradient and not from others."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    monkeypatch.setenv("NITI_BACKWARD_PAIR", "1")
+    monkeypatch.setenv("NITI_WGRAD_BLOCKS", "16")
+    base._say("conv_backward_pair, partial sums > 2^23", case)
+    g = torch.Generator().manual_seed(4500 + Q)
+    act, err, w = ri8(g, N, Q, Q, C, lo=-20, hi=20), ri8(g, N, Q, Q, K, lo=-20, hi=20), ri8(g, K, 3, 3, C)
+    n_hot = N // 4
+    act[:n_hot, :, :, :32] = 127
+    err[:n_hot] = 127
+    err[:n_hot, :, :, 1::2] = -127
+    dw = co.conv_wgrad(act, err, 3, 3, 1, 1)
+    assert int(dw.abs().max()) > 2 ** 23 and int(dw[:, :, :, 32:].abs().max()) < 2 ** 22
+    gref, gsh = po.grad_calc(dw, 5, "psto")
+    wd = w.to(dev)
+    prepared = ops.conv_filter_prepare(wd, N, Q, Q, 1, 1)
+    g8, sh = ops.conv2d_backward(err.to(dev), act.to(dev), wd, want_grad=True, prepared_filter=prepared)[3:6:2]
+    assert torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh and torch.equal(wd.cpu(), po.weight_update(w, gref))
+    assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
+
+
+@pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 128, 128)])
+def test_conv_backward_pair_gives_up(case):
+    """Waits with a limit of zero: the launch ends and the device-wide word says so."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import torch
+from niti_amd import ops
+N, Q, C, K = %r
+dev = torch.device("cuda:0")
+ri = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device=dev)
+w = ri(K, 3, 3, C)
+ops.conv2d_backward(ri(N, Q, Q, K), ri(N, Q, Q, C), w, prepared_filter=ops.conv_filter_prepare(w, N, Q, Q, 1, 1))
+torch.cuda.synchronize()
+print("STICKY", int(ops.sync_timeouts(dev)))
+""" % (case,)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, NITI_SYNC_TIMEOUT_MS="0", NITI_BACKWARD_PAIR="1")
+    out = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stderr[-2000:]
+    assert "STICKY 1" in out.stdout
