@@ -140,9 +140,8 @@ int niti_conv2d_i8_dgrad(const int8_t* err, const int8_t* w, int32_t* dx, int N,
  * Covered: 3x3, stride 1, pad 1, square inputs of side 2, 4, 8, 16 or 32, N*H*W % 256 == 0 (side 2: any N), input
  * channels % 16 == 0, output channels % 16 == 0, rounding NITI_ROUND_NEAREST or NITI_ROUND_PSEUDO_STOCHASTIC, and a
  * launch of at most 4096 workgroups (N*H*W/256 x ceil(out channels/128 or 64); side 2: ceil(N/32) x ceil(out
- * channels/32), which must fit on the device at once).  Launches of the other sides that do not fit on the device at
- * once run as two launches that do not wait (the second one settles tiles stored with another shift than the final
- * one).  niti_conv2d_i8_requant_sync_words returns 0 for shapes outside that (then use the two-pass entry points); the
+ * channels/32), which must fit on the device at once).  Of the other sides a workgroup takes several of these tiles in turn where they
+ * do not all fit on the device at once.  niti_conv2d_i8_requant_sync_words returns 0 for shapes outside that (then use the two-pass entry points); the
  * entry points return NITI_ERR_UNSUPPORTED for them.
  *
  * sync: niti_conv2d_i8_requant_sync_words(...) uint32 words that are ZERO on entry (niti_fill_u32).  On return

@@ -1,6 +1,8 @@
 // What the 3x3 convolution kernels on 4 ... 32 pixel wide maps share: their arguments, the grid-wide range exchange around
 // their main loops and the epilogue that turns a workgroup's int32 sums into int32 or rounded int8 results.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "lds_asm.h"
 #include "requant_math.h"
@@ -43,15 +45,7 @@ struct HaloArgs {
   int32_t* exp_out;
 };
 constexpr int kSyncSlot0 = 16;
-// A grid with more workgroups than the device holds at once cannot wait for itself.  It runs as two launches of the
-// same kernel instead (set by the launcher in rq_flags, not part of the interface):
-//   kRqNoWait  every workgroup fills its slot (largest magnitude + 1, and next to it the shift it used), stores its
-//              tile rounded with the predicted shift or what its own sums need, and ends;
-//   kRqSettle  every workgroup first reads all slots - final after the first launch -, and ends at once if its tile
-//              was stored with the final shift; otherwise it computes its tile again and stores it with that shift.
-// With a good prediction (the previous training step's shift) the second launch does nothing but look.
-constexpr unsigned kRqNoWait = 1u << 30, kRqSettle = 1u << 31;
-static_assert(kSlotStride >= 2, "the two-launch form keeps the shift a tile was stored with in the word behind its slot");
+static_assert(kSlotStride >= 2, "workgroups with several tiles keep the shift a tile was stored with in the word behind its slot");
 constexpr int kMaxSlots = 4096;
 
 // The same convolution on products of 64 channels (conv3x3_k64.h); the filter copy must hold a whole number of 64-channel
@@ -66,7 +60,7 @@ int halo_requant_args(HaloArgs& a, const int8_t* x, const int8_t* wp, int8_t* y8
 
 namespace {
 
-// Which of the convolution's workgroups this is: x along the pixels, y along the channel tiles, of nx * ny.  (A launch may hold others.)
+// Which of the convolution's tiles this is: x along the pixels, y along the channel tiles, of nx * ny.
 struct HaloPlace {
   int x, y, nx, ny;
   __device__ int block() const { return y * nx + x; }
@@ -89,42 +83,9 @@ __device__ inline void hc_sync() {
   asm volatile("" ::: "memory");
 }
 
-// The settling launch (kRqSettle), called before anything else: false if this workgroup's tile already has the final shift and
-// it is done; otherwise settle_shift is the shift to store it with.
-__device__ inline bool halo_settle(const HaloArgs& a, const HaloPlace at, int8_t* dump, int& settle_shift) {
-  settle_shift = -1;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint32_t* const slots = a.sync + kSyncSlot0;
-  uint32_t* const words = reinterpret_cast<uint32_t*>(dump);
-  const int nb = at.blocks();
-  const int b = at.block();
-  uint32_t m = 0;
-  for (int i = tid; i < nb; i += 512) m = max(m, __hip_atomic_load(slot_word(slots, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  m = wave_max_u32(m);
-  if (lane == 0) words[wave] = m;
-  __syncthreads();
-  uint32_t g = words[0];
-#pragma unroll
-  for (int w = 1; w < 8; ++w) g = max(g, words[w]);
-  const uint32_t gmax = g != 0u ? g - 1u : 0u;
-  const int fshift = max(bitwidth_of(gmax, a.bw_mode) - a.target_bits, 0);
-  const int used = static_cast<int>(slot_word(slots, b)[1]);
-  if (b == 0 && tid == 0) {
-    a.sync[0] = gmax;
-    if (a.shift_out != nullptr) *a.shift_out = fshift;
-    if (a.exp_out != nullptr) *a.exp_out = fshift + (a.exp_a != nullptr ? *a.exp_a : 0) + (a.exp_b != nullptr ? *a.exp_b : 0);
-  }
-  if (used == fshift) return false;
-  settle_shift = fshift;
-  __syncthreads();   // the words are written again below
-  return true;
-}
-
 // NITI_RQ_SHIFT_HINT: *shift_out holds the caller's prediction (the previous training step's shift of this tensor).
-// Read at kernel start, a whole main loop before it is needed; workgroup (0, 0) overwrites the word only after all slots are
-// filled, i.e. after every workgroup has passed this line.
+// Read at a tile's start, a whole main loop before it is needed; tile 0 overwrites the word only after all slots are filled, i.e. after
+// this line has been passed for every tile.
 // The load is unconditional (from the range word when there is no prediction), its address looks lane-dependent to
 // the compiler and its result is not looked at before the epilogue: a load inside a branch, or one whose result the
 // compiler knows to be the same in all lanes (and moves to a scalar register at once), would be waited for on the
@@ -166,8 +127,7 @@ struct HaloPieces {
   static constexpr int LPU = KT / 16, PPU = 64 / LPU;
   bool pairs;
   int mfirst, mstep, ch;
-  __device__ HaloPieces(const HaloArgs& a, int pixbase, int kt, int wp_, int wc) {
-    const int lane = threadIdx.x & 63;
+  __device__ HaloPieces(const HaloArgs& a, int pixbase, int kt, int wp_, int wc, int lane) {
     pairs = kPairs && a.unpool != nullptr;
     mfirst = pixbase + (kTwo ? wc * 256 : 0) + wp_ * (32 * PT) + (pairs ? wc * (16 * PT) + lane / LPU : lane / LPP);
     mstep = pairs ? PPU : PPI;
@@ -206,8 +166,14 @@ struct HaloAhead {
   v4i xw[P::XWD][4];
 };
 
+// A workgroup's only tile; see Turns
+struct OneTile {
+  __device__ int thread() const { return threadIdx.x; }
+  __device__ int again() const { return -1; }       // the final shift, when the tile is stored again with it
+  __device__ bool early() const { return false; }   // stored by the shift as it looks from here; nobody waits
+};
 // What a workgroup does besides: see SumsAlong (wgrad_finish.h).
-struct NothingAlong {
+struct NothingAlong : OneTile {
   __device__ void begin() {}
   __device__ void publish() {}
   __device__ void guess() {}
@@ -224,7 +190,7 @@ template <int Q, int KT, bool kTwo, int NWF, int PT, bool kFused, bool kSto, boo
 __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace at, v4i (&q)[NWF * PT * 4], int8_t* const smem, uint32_t* const red, const int pixbase,
                                               const int kt, const int wp_, const int wc, const int settle_shift, const ShiftHint hint,
                                               const HaloPieces<Q, KT, kTwo, NWF, PT, kRegs256>& pc, HaloAhead<Q, KT, kTwo, NWF, PT, kRegs256>& ahead, Along& along) {
-  const int tid = threadIdx.x;
+  const int tid = along.thread();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool hinted = hint.hinted;
@@ -299,7 +265,7 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace
     const int nb = at.blocks();
     uint32_t* const slots = a.sync + kSyncSlot0;
     constexpr int kLook = 8;   // slots a lane reads with its loads in flight together
-    const bool nowait = (a.rq_flags & kRqNoWait) != 0;
+    const bool nowait = along.early();
     const bool settled = settle_shift >= 0;
     constexpr int PROW = NWF * 32 + 16;  // the wavefront's channels of one pixel, padded
     int8_t* patch = smem + wave * (32 * PT * PROW);
@@ -354,8 +320,8 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace
     bool final_range = nb == 1;
     if (!final_range && hinted) shift = max(shift, predicted_raw);
     if (settled) shift = settle_shift;
-    if (nowait) {   // the shift this tile is stored with, for the settling launch
-      if (tid == 0) slot_word(slots, at.block())[1] = static_cast<uint32_t>(shift);
+    if (nowait) {   // the shift this tile is stored with: see tiles_in_turns
+      if (tid == 0) __hip_atomic_store(slot_word(slots, at.block()) + 1, static_cast<uint32_t>(shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     final_range = final_range || nowait || settled;
     const bool trunc = a.trunc != 0;
@@ -532,43 +498,114 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace
   }
 }
 
+// ---- more tiles than the device holds workgroups at once: every workgroup takes several in turn, the last of them (number blockIdx.x) as
+// always.  The earlier ones are stored by the predicted shift, or what their own sums need, and leave a slot each; behind the wait of the
+// last one, when the final shift is known, those that were stored with another are computed again and stored with it.
+// One launch for all tiles without waiting and a second one that computed every tile again unless its shift was right took, with
+// predictions that fail (as about half of those inside a training step do) and with good ones (us): 256 images of 32 x 32, 128 -> 128
+// 67.4 / 44.1, so 57.5 / 42.1; data gradient 73.1 / 48.2, 62.6 / 46.6; 192 images 55.6 / 36.4, 47.6 / 35.2; 136 images 50.1 / 33.1, 43.2 / 33.5;
+// 256 of 16 x 16, 256 -> 512 121.1 / 64.4, 96.1 / 63.6; 256 of 32 x 32, 256 -> 256 (four tiles each) 242 / 125, 223 / 129.  What bounds it:
+// the first stage of each tile waits for its loads behind the stores of the one before.
+struct Turns : NothingAlong {
+  int final_shift = 0, settle_shift = -1;
+  bool is_early = false;
+  // (a new value to the compiler in every turn, like the arguments: what follows from them is worked out again rather than kept in registers)
+  __device__ int thread() const {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  }
+  __device__ int again() const { return settle_shift; }
+  __device__ bool early() const { return is_early; }
+  __device__ void update(int shift, const int32_t*, const int32_t*) { final_shift = shift; }
+};
+// tile(args, at, along), in a kernel whose first argument is its HaloArgs and whose grid has at most as many workgroups as there are tiles (nx * ny)
+template <class F>
+__device__ __forceinline__ void tiles_in_turns(const int nx, const int ny, F tile) {
+  using Args = const __attribute__((address_space(4))) HaloArgs;
+  const int step = gridDim.x, own = blockIdx.x;
+  Turns along;
+  const auto take = [&](int id) {
+    const HaloPlace at{id % nx, id / nx, nx, ny};
+    Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    tile(*(const HaloArgs*)args, at, along);
+  };
+  // ids: own + n * step, .., own + step, own, then own + step, .. again
+  const int last = own + (nx * ny - 1 - own) / step * step;
+  bool back = false;
+  for (int id = last;;) {
+    along.is_early = !back && id != own;
+    bool stored = false;
+    if (back) {
+      Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+      // (written in front of the own tile's loads, which have been waited for since)
+      stored = static_cast<int>(__hip_atomic_load(slot_word(args->sync + kSyncSlot0, id) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == along.settle_shift;
+    }
+    if (!stored) take(id);
+    back = back || id == own;
+    if (back) {
+      id += step;
+      if (id > last) return;
+      along.settle_shift = __builtin_amdgcn_readfirstlane(along.final_shift);
+    } else {
+      id -= step;
+    }
+    __syncthreads();   // the tile before has left LDS
+  }
+}
+
 // what a kernel's launches remember per device
 struct HaloLaunch {
   bool attr_set[kDeviceSlots] = {};   // function attributes are per device
   int resident[kDeviceSlots] = {};    // workgroups the device holds at once
 };
-
-// grid: ceil(pixels / px) x ceil(K / ktile)
-template <bool kFused, class Kernel>
-int launch_halo_kernel(Kernel k, HaloLaunch& state, size_t lds, int px, int ktile, int Q, const HaloArgs& a, hipStream_t stream) {
+template <class Kernel>
+int halo_attributes(Kernel k, HaloLaunch& state, size_t lds, bool count) {
   const int slot = device_slot();
-  if (!state.attr_set[slot]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-      return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot reserve %zu bytes of LDS", lds);
-    if (kFused) {
-      int dev = 0, cus = 0, per_cu = 0;
-      if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k), 512, lds) != hipSuccess)
-        return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot query occupancy");
-      state.resident[slot] = cus * per_cu;
-    }
-    state.attr_set[slot] = true;
+  if (state.attr_set[slot]) return NITI_OK;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot reserve %zu bytes of LDS", lds);
+  if (count) {
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k), 512, lds) != hipSuccess)
+      return fail(NITI_ERR_LAUNCH, "conv3x3_halo: cannot query occupancy");
+    state.resident[slot] = cus * per_cu;
   }
+  state.attr_set[slot] = true;
+  return NITI_OK;
+}
+
+// A launch of ceil(pixels / px) x ceil(K / ktile) tiles by kernel `one`, or by kernel `several` where they are more than the device holds of
+// its workgroups (the same kernel twice: a tile that is not chosen for such launches).
+template <class Kernel>
+struct HaloKernel {
+  Kernel k;
+  size_t lds;
+};
+template <class Kernel>
+HaloKernel(Kernel, size_t) -> HaloKernel<Kernel>;
+template <bool kFused, class One, class Several>
+int launch_halo_kernel(HaloKernel<One> one, HaloKernel<Several> several, HaloLaunch (&state)[2], int px, int ktile, int Q, const HaloArgs& a, hipStream_t stream) {
+  int st = halo_attributes(one.k, state[0], one.lds, kFused);
+  if (st != NITI_OK) return st;
   const long long pix = static_cast<long long>(a.N) * Q * Q;
-  dim3 grid(static_cast<unsigned>((pix + px - 1) / px), (a.K + ktile - 1) / ktile);
-  if (kFused && static_cast<long long>(grid.x) * grid.y > state.resident[slot]) {
-    // more workgroups than the device holds at once: nobody waits; a second launch settles the tiles stored with
-    // another shift than the final one
-    if (static_cast<long long>(grid.x) * grid.y > kMaxSlots)
-      return fail(NITI_ERR_UNSUPPORTED, "conv3x3_halo: %u workgroups exceed the %d range slots", grid.x * grid.y, kMaxSlots);
-    HaloArgs b = a;
-    b.rq_flags = a.rq_flags | kRqNoWait;
-    hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, b);
-    b.rq_flags = a.rq_flags | kRqSettle;
-    hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, b);
-    return check_launch("conv3x3_halo");
+  const dim3 grid(static_cast<unsigned>((pix + px - 1) / px), (a.K + ktile - 1) / ktile);
+  const long long tiles = static_cast<long long>(grid.x) * grid.y;
+  if (kFused && tiles > state[0].resident[device_slot()]) {
+    if constexpr (std::is_same_v<One, Several>) {
+      return fail(NITI_ERR_UNSUPPORTED, "conv3x3_halo: %lld workgroups of this tile do not fit on the device at once", tiles);
+    } else {
+      if (tiles > kMaxSlots) return fail(NITI_ERR_UNSUPPORTED, "conv3x3_halo: %lld tiles exceed the %d range slots", tiles, kMaxSlots);
+      st = halo_attributes(several.k, state[1], several.lds, true);
+      if (st != NITI_OK) return st;
+      const long long fit = state[1].resident[device_slot()];
+      hipLaunchKernelGGL(several.k, dim3(static_cast<unsigned>(tiles < fit ? tiles : fit)), dim3(512), several.lds, stream, a, static_cast<int>(grid.x), static_cast<int>(grid.y));
+      return check_launch("conv3x3_halo");
+    }
   }
-  hipLaunchKernelGGL(k, grid, dim3(512), lds, stream, a);
+  hipLaunchKernelGGL(one.k, grid, dim3(512), one.lds, stream, a);
   return check_launch("conv3x3_halo");
 }
 

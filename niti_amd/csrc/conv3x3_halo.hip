@@ -28,11 +28,11 @@
 //
 // Input channels that fill two or more whole slices of 64 have a faster form of the same kernel (conv3x3_k64.h); this one is left with
 // the first layer, most launches of a single such slice and other counts whose last slice of 64 would be half empty.  Of its instances the
-// StoShift ones for 64 channels spill 4 registers, those for 128 or for 512 pixels 15 to 19, and the data gradients for 512 pixels one;
-// no other does.
+// StoShift ones for 64 channels spill 4 registers, those for 128 or for 512 pixels 15 to 19, the data gradients for 512 pixels one, and
+// the ones that take several tiles in turn 1 to 4 (StoShift or 512 pixels 3 to 19); no other does.
 //
 // Launches the device cannot hold at once: the 64-channel tile takes 512 pixels per workgroup where that
-// is enough (HGeom::TWO); otherwise the launch runs twice without waiting (kRqNoWait, kRqSettle below).
+// is enough (HGeom::TWO); otherwise every workgroup takes several tiles in turn (tiles_in_turns).
 // Maps of 2 x 2 pixels have a kernel of their own at the end of this file (conv3x3_map2_kernel).
 #include <stdlib.h>
 
@@ -125,29 +125,24 @@ struct Layout32 {
 // 32 x 32 byte blocks are staged as they are and transposed by ds_read_b64_tr_b8 when the fragments are read.
 // kSto: the requantising variant with StoShift (random integers read in the epilogue); instances of their own so that the
 // others keep their register allocation.
-template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto = false>
-__global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) {
+template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto, class Along>
+__device__ __forceinline__ void halo_tile(const HaloArgs& a, const HaloPlace at, int8_t* const smem, Along& along) {
   static_assert(kFused || !kSto);
   using G = HGeom<Q, BR, NI, KT>;
   constexpr int NWF = G::NWF;
-  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t* const act_buf = smem;                         // 2 x ACT_BYTES
   int8_t* const w_buf = smem + 2 * G::ACT_BYTES;        // WSTAGES x W_BYTES
   int8_t* const dump = smem + G::TILE_BYTES;
 
-  const int tid = threadIdx.x;
+  const int tid = along.thread();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pixbase = blockIdx.x * G::PX;  // first output pixel of this workgroup in [N*Q*Q]
-  const int kt = blockIdx.y;
+  const int pixbase = at.x * G::PX;  // first output pixel of this workgroup in [N*Q*Q]
+  const int kt = at.y;
   const int n0 = pixbase / (Q * Q);
   const int p0 = (pixbase - n0 * (Q * Q)) / Q;
 
-  int settle_shift = -1;   // kRqSettle: the final shift, when this workgroup has to store its tile again
-  if constexpr (kFused) {
-    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, halo_grid_place(), dump, settle_shift)) return;
-  }
-
+  const int settle_shift = along.again();   // the final shift, when this workgroup has to store its tile again
 
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.x), 0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.wp), 0, a.wp_bytes, 0x00020000);
@@ -506,11 +501,22 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         q[(i * PT + j) * 4 + g] = v4i{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-  const HaloPieces<Q, KT, G::TWO, NWF, PT, false> pieces(a, pixbase, kt, wp_, wc);
+  const HaloPieces<Q, KT, G::TWO, NWF, PT, false> pieces(a, pixbase, kt, wp_, wc, lane);
   HaloAhead<Q, KT, G::TWO, NWF, PT, false> ahead;
+  halo_epilogue<Q, KT, G::TWO, NWF, PT, kFused, kSto, false, Layout32>(a, at, q, smem, reinterpret_cast<uint32_t*>(dump), pixbase, kt, wp_, wc, settle_shift, hint, pieces,
+                                                                       ahead, along);
+}
+template <int Q, int BR, int NI, int KT, bool kFused, bool kWT, bool kSto = false>
+__global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   NothingAlong along;
-  halo_epilogue<Q, KT, G::TWO, NWF, PT, kFused, kSto, false, Layout32>(a, halo_grid_place(), q, smem, reinterpret_cast<uint32_t*>(dump), pixbase, kt, wp_, wc, settle_shift, hint,
-                                                                       pieces, ahead, along);
+  halo_tile<Q, BR, NI, KT, kFused, kWT, kSto>(a, halo_grid_place(), smem, along);
+}
+// the same for launches with more tiles than the device holds workgroups
+template <int Q, int BR, int NI, int KT, bool kWT, bool kSto>
+__global__ __launch_bounds__(512, 4) void conv3x3_halo_turns_kernel(const HaloArgs, const int nx, const int ny) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  tiles_in_turns(nx, ny, [&](const HaloArgs& a, const HaloPlace at, Turns& along) { halo_tile<Q, BR, NI, KT, true, kWT, kSto>(a, at, smem, along); });
 }
 
 // ---- 2 x 2 maps -----------------------------------------------------------------------------------------
@@ -809,7 +815,7 @@ int halo_ktile(long long pix, int K, int H, int C) {
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
   if (forced == 128 || forced == 64) return forced;
-  if (forced == 32 && H <= 16) return 32;
+  if (forced == 32 && H <= 16 && ptiles * ((K + 31) / 32) <= 2LL * cus) return 32;
   // one 32-channel tile per compute unit at most: twice as many workgroups as with 64 channels, each half as long (24 images of
   // 16 x 16, 256 -> 256: 12.3 -> 9.3 us, 60 of 8 x 8, 512 -> 512: 18.8 -> 16.6).  Two of them on a unit are slower than one
   // 64-channel tile (50 images of the former 16.7 / 12.8 us, 120 of the latter 27.8 / 22.6).
@@ -856,7 +862,7 @@ int k64_ktile(long long pix, int K, int H, int C, bool fused) {
   const int cus = compute_units();
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
-  if (forced == 128 || forced == 64 || (forced == 32 && H <= 16)) return forced;
+  if (forced == 128 || forced == 64 || (forced == 32 && H <= 16 && ptiles * ((K + 31) / 32) <= 2LL * cus)) return forced;
   if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
   const long long b64 = ptiles * ((K + 63) / 64);
   const long long b128 = ptiles * ((K + 127) / 128);
@@ -887,7 +893,8 @@ HaloTile halo_tile(long long pix, int K, int H, int C, bool fused) {
   const auto blocks = [&](int ktile) { return (pix + 255) / 256 * ((K + ktile - 1) / ktile); };
   const int cus = compute_units();
   const int wide = whole ? k64_ktile(pix, K, H, C, fused) : 0;
-  // (at 64 channels and more of such workgroups than the device holds, one launch of the other kernel's 512 pixels instead of two)
+  // (at 64 channels and more of such workgroups than the device holds, the other kernel's 512 pixels instead of several tiles in turn: 256
+  // images of 32 x 32, 128 -> 64 28.2 / 30.8 us, with a prediction that fails 29.9 / 41.6; 32 -> 64 12.6 / 19.2 and 14.7 / 25.2)
   if (whole && fused && halo_two_pixel_tiles(pix, K, H, wide)) return {wide, 512, false};
   if (whole && (C > 64 || e != nullptr)) return {wide, 256, true};
   const int ktile = halo_ktile(pix, K, H, C);
@@ -904,8 +911,10 @@ int launch_halo(const HaloArgs& a, hipStream_t stream) {
   static_assert(8 * 32 * (32 * 4 + 16) <= G::TILE_BYTES, "int32 patches must stay clear of the reduction words");
   static_assert(8 * 32 * G::PT * (G::NWF * 32 + 16) <= G::TILE_BYTES, "int8 patches must stay clear of the reduction words");
   static_assert(2 * lds <= 160 * 1024, "two workgroups per compute unit");
-  static HaloLaunch state;
-  return launch_halo_kernel<kFused>(conv3x3_halo_kernel<Q, BR, NI, KT, kFused, kWT, kSto>, state, lds, G::PX, KT, Q, a, stream);
+  static HaloLaunch state[2];
+  const HaloKernel one{conv3x3_halo_kernel<Q, BR, NI, KT, kFused, kWT, kSto>, lds};
+  if constexpr (kFused && KT != 32) return launch_halo_kernel<true>(one, HaloKernel{conv3x3_halo_turns_kernel<Q, BR, NI, KT, kWT, kSto>, lds}, state, G::PX, KT, Q, a, stream);
+  else return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: at most one workgroup on a unit)
 }
 
 inline int map2_blocks(int N, int K) { return ((N + 31) / 32) * ((K + 31) / 32); }
@@ -1067,7 +1076,7 @@ int conv3x3_halo_requant_blocks(int N, int H, int W, int C, int K, int R, int S,
   const HaloTile tile = halo_tile(pix, K, H, C, true);
   const long long nb = H == 2 ? map2_blocks(N, K) : ((pix + tile.pixels - 1) / tile.pixels) * ((K + tile.channels - 1) / tile.channels);
   if (us != nullptr) *us = nb <= kMaxSlots ? requant_us(tile, static_cast<int>(nb), H, C) : 0.0;
-  return nb <= kMaxSlots ? static_cast<int>(nb) : 0;  // more than the device holds at once run as two launches
+  return nb <= kMaxSlots ? static_cast<int>(nb) : 0;  // (more than the device holds at once: see tiles_in_turns)
 }
 
 size_t conv3x3_halo_sync_words(int blocks) { return static_cast<size_t>(kSyncSlot0) + slot_words(blocks); }

@@ -130,8 +130,8 @@ __device__ inline v4i neighbour4(v4i x, int keep) {
 __device__ inline void mfma64(v4i& d, v4i a, v4i b) { asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b)); }
 __device__ inline void mfma_settle() { asm volatile("s_nop 15\n\ts_nop 15"); }
 
-// (What is left: the StoShift instances for two workgroups per unit spill 6 registers at 64 channels and 17 or 18 at 128, none of them inside
-// the loop; no other instance spills.)
+// (What is left: the StoShift instances for two workgroups per unit spill 6 registers at 64 channels and 17 or 18 at 128, and those that take
+// several tiles in turn 2 to 11 (StoShift 7 to 25), none of them inside the loop; no other instance spills.)
 // kWT: the filter operand is the forward copy of the filter of the convolution whose data gradient this launch computes; its
 // blocks of 64 reduction channels x 32 outputs are transposed by ds_read_b64_tr_b8 when the fragments are read.
 // kSto: StoShift on random integers read in the epilogue.
@@ -142,7 +142,7 @@ __device__ __forceinline__ void k64_tile(const HaloArgs& a, const HaloPlace at, 
   constexpr int PT = G::PT, NWF = G::NWF, TPS = G::TPS, S = G::S, R = G::R, WL = G::WL;
   int8_t* const dump = smem + G::TILE_BYTES;
 
-  const int tid = threadIdx.x;
+  const int tid = along.thread();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pixbase = at.x * G::PX;  // first output pixel of this workgroup in [N*Q*Q]
@@ -150,11 +150,7 @@ __device__ __forceinline__ void k64_tile(const HaloArgs& a, const HaloPlace at, 
   const int n0 = pixbase / (Q * Q);
   const int p0 = (pixbase - n0 * (Q * Q)) / Q;
 
-  int settle_shift = -1;   // kRqSettle: the final shift, when this workgroup has to store its tile again
-  if constexpr (kFused) {
-    if ((a.rq_flags & kRqSettle) != 0 && !halo_settle(a, at, dump, settle_shift)) return;
-  }
-
+  const int settle_shift = along.again();   // the final shift, when this workgroup has to store its tile again
   along.begin();
 
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.x), 0, a.x_bytes, 0x00020000);
@@ -271,7 +267,7 @@ __device__ __forceinline__ void k64_tile(const HaloArgs& a, const HaloPlace at, 
   // results' mask bytes and pooling windows: requested in the last slice (PER_CU == 1), see HaloPieces
   constexpr bool kAhead = kFused && PER_CU == 1;
   using Pieces = HaloPieces<Q, KT, false, NWF, PT, PER_CU == 1>;
-  const Pieces pieces(a, pixbase, kt, wp_, wc);
+  const Pieces pieces(a, pixbase, kt, wp_, wc, lane);
   HaloAhead<Q, KT, false, NWF, PT, PER_CU == 1> ahead;
   constexpr int kSpare = G::ACT_LOADS + S * WL;   // loads of the last slice, none of which has anything to fetch (R > S)
   static_assert(!kAhead || (R > S && kSpare >= Pieces::NPIECE));
@@ -456,14 +452,26 @@ __global__ __launch_bounds__(512, 2 * PER_CU) void conv3x3_k64_kernel(const Halo
   k64_tile<Q, BR, NI, KT, PER_CU, kFused, kWT, kSto>(a, halo_grid_place(), smem, along);
 }
 
+// the same for launches with more tiles than the device holds workgroups
+template <int Q, int BR, int NI, int KT, bool kWT, bool kSto>
+__global__ __launch_bounds__(512, 4) void conv3x3_k64_turns_kernel(const HaloArgs, const int nx, const int ny) {
+  extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+  tiles_in_turns(nx, ny, [&](const HaloArgs& a, const HaloPlace at, Turns& along) { k64_tile<Q, BR, NI, KT, 2, true, kWT, kSto>(a, at, smem, along); });
+}
+
 template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto>
 int launch_k64(const HaloArgs& a, hipStream_t stream) {
   using G = KGeom<Q, BR, NI, KT, PER_CU>;
-  constexpr size_t lds = G::LDS_BYTES;
   static_assert(8 * 32 * (32 * 4 + 16) <= G::TILE_BYTES, "int32 patches must stay clear of the reduction words");
   static_assert(8 * 32 * G::PT * (G::NWF * 32 + 16) <= G::TILE_BYTES, "int8 patches must stay clear of the reduction words");
-  static HaloLaunch state;
-  return launch_halo_kernel<kFused>(conv3x3_k64_kernel<Q, BR, NI, KT, PER_CU, kFused, kWT, kSto>, state, lds, G::PX, KT, Q, a, stream);
+  static HaloLaunch state[2];
+  const HaloKernel one{conv3x3_k64_kernel<Q, BR, NI, KT, PER_CU, kFused, kWT, kSto>, G::LDS_BYTES};
+  if constexpr (kFused && KT != 32) {
+    const HaloKernel several{conv3x3_k64_turns_kernel<Q, BR, NI, KT, kWT, kSto>, KGeom<Q, BR, NI, KT, 2>::LDS_BYTES};
+    return launch_halo_kernel<true>(one, several, state, G::PX, KT, Q, a, stream);
+  } else {
+    return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: at most one workgroup on a unit)
+  }
 }
 
 // One workgroup per compute unit as long as the launch has no more of them; NITI_HALO_PER_CU pins the choice (tests).

@@ -25,6 +25,10 @@ namespace {
 constexpr int kBesideItems = 5, kWithinItems = 1;   // (two workgroups on a unit that multiply leave registers for one)
 constexpr int per_cu_geometry(int ktile) { return ktile == 32 ? 1 : 2; }   // the 32-channel tile fits twice as it is
 
+struct SumsWithin : SumsAlong<kWithinItems, false>, OneTile {
+  using SumsAlong::SumsAlong;
+};
+
 // The first nx x ny workgroups are the data gradient's.  kBeside: the others finish the weight gradient; otherwise the last work.nblocks
 // of them do so as well.
 template <int Q, int BR, int NI, int KT, bool kBeside>
@@ -41,7 +45,7 @@ __global__ __launch_bounds__(512, 4) void conv3x3_k64_backward_kernel(const Halo
       finish_beside(SumsAlong<kBesideItems, (KT < 128)>(f, work, id - first, smem), a, a.sync + kSyncSlot0, first);
     }
   } else {
-    SumsAlong<kWithinItems, false> along(f, work, id - (first - work.nblocks), smem + KGeom<Q, BR, NI, KT, kPer>::LDS_BYTES);
+    SumsWithin along(f, work, id - (first - work.nblocks), smem + KGeom<Q, BR, NI, KT, kPer>::LDS_BYTES);
     k64_tile<Q, BR, NI, KT, kPer, true, true, false>(a, at, smem, along);
   }
 }

@@ -125,6 +125,40 @@ def test_conv_slices_of_64_stored_again(dev, forward, monkeypatch):
         assert torch.equal(y.cpu(), torch.where(mask > 0, ref, torch.zeros_like(ref)))
 
 
+# N, side, C, K: two to five tiles for a workgroup, some with one fewer, the last tile of channels ragged, with 64 and 128 channels
+# and 256 and 512 pixels, by the kernels of 64-channel and of 32-channel slices
+@pytest.mark.parametrize("case", [(2052, 8, 64, 192), (151, 32, 64, 400), (601, 32, 96, 64), (259, 16, 32, 512), (4112, 4, 128, 272)])
+def test_conv_tiles_in_turns(dev, case):
+    """Predictions that fit, that fit no tile and that fit some, and none: forward with the pooled output, data gradient from both filter
+    copies with a mask, against the int32 results rounded by the oracle."""
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    base._say("conv_tiles_in_turns", case)
+    g = torch.Generator().manual_seed(N + K)
+    x, w = ri8(g, N, Q, Q, C).to(dev), ri8(g, K, 3, 3, C).to(dev)
+    x[N // 2:] //= 4          # the later images need two bits fewer
+    e, mask = ri8(g, N, Q, Q, C).to(dev), ri8(g, N, Q, Q, K).to(dev)
+    wb = ri8(g, C, 3, 3, K).to(dev)
+    acc, dacc = ops.conv2d_fprop(x, w, 1, 1).cpu(), ops.conv2d_dgrad(e, wb, 1, 1).cpu()
+    (ref, sh_ref), (dref, dsh) = po.act_calc(acc, 0), po.err_calc(dacc)
+    dref = torch.where(mask.cpu() > 0, dref, torch.zeros_like(dref))
+    wf = ops.conv_filter_prepare(wb, N, Q, Q)
+    for off in (None, 0, 3, -2):
+        def state(right):
+            return {} if off is None else dict(shift_out=torch.tensor([max(right + off, 0)], dtype=torch.int32, device=dev), shift_hint=True)
+        pooled = torch.empty((N, Q // 2, Q // 2, K), dtype=torch.int8, device=dev)
+        y, sh, sync = ops.conv2d_fprop_requant(x, w, relu=True, pool_out=pooled, **state(sh_ref))
+        assert int(sync.cpu()[1]) == 0 and int(sync.cpu()[0]) == po.absmax(acc) and int(sh.cpu()) == sh_ref
+        assert torch.equal(y.cpu(), ref.clamp(min=0)) and torch.equal(pooled.cpu(), po.maxpool_fwd(ref.clamp(min=0)))
+        for kw in (dict(), dict(forward_filter=wf)):
+            d, sh, sync = ops.conv2d_dgrad_requant(e, wb, relu_mask=mask, **kw, **state(dsh))
+            assert int(sync.cpu()[1]) == 0 and int(sh.cpu()) == dsh and torch.equal(d.cpu(), dref)
+    y, sh, sync = ops.conv2d_fprop_requant(x[:-1].contiguous(), w, relu=True, any_shape=True)   # the last tile of pixels not full
+    ref, sh_ref = po.act_calc(acc[:-1], 0)
+    assert int(sync.cpu()[1]) == 0 and int(sh.cpu()) == sh_ref and torch.equal(y.cpu(), ref.clamp(min=0))
+
+
 # more 128-channel workgroups than compute units, fewer 64-channel ones than twice those: an odd number of 64-channel groups, the last
 # of 32 and of 64 channels; forward, then data gradient
 @pytest.mark.parametrize("case", [(130, 16, 64, 160), (130, 16, 160, 64), (344, 8, 64, 320)])
