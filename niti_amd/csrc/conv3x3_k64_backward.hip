@@ -15,6 +15,8 @@
 // stages' loads, then one exchange.
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "conv3x3_k64.h"
 #include "conv_any.h"
 #include "wgrad_finish.h"
@@ -116,7 +118,11 @@ PairPlan pair_plan(int N, int H, int C, int K) {
   p.beside = room >= cus / 4;
   // Where those that multiply fill the device, the later ones of the two on each unit add the slices before their first stage: their
   // neighbours have the matrix units to themselves meanwhile (128 images of 32 x 32, 128 -> 128: 8.5 us, of which 4 show).
-  p.work = along_work(units, slices, p.beside && room < cus ? room : cus);
+  // More than one of them per unit take part where that leaves none with more chunks than it has room for (both launches against the
+  // data gradient's and the one-launch weight gradient's: 16 x 16, 256 -> 256 at 160 / 192 / 256 images 68.8 -> 60.3, 73.4 -> 65.3, 83.3 -> 80.4 us;
+  // 200 images 256 -> 320 119.3 -> 109.7; five eighths or all of the workgroups instead of half 0 to 2 us slower).
+  const long long least = ((units + 63) / 64 + 8 * kWithinItems - 1) / (8 * kWithinItems);
+  p.work = along_work(units, slices, p.beside ? std::min(room, cus) : static_cast<int>(std::min(std::max<long long>(least, cus), nb)));
   return fits_twice(H, p) ? p : PairPlan{};
 }
 

@@ -392,9 +392,10 @@ def test_quantiser_entries_of_the_c_abi(dev):
 
 # N, side, C, K of layers whose two gradients run as a pair of launches.  Update beside the data gradient: its tiles of 32, 64 and 128
 # channels on every map; one slice of partial sums and 67, three input-channel groups of 64, batches that end inside a tile; some
-# workgroups for the update fewer than the device has units.  Update by workgroups that multiply as well: 64 and 128 channels.
+# workgroups for the update fewer than the device has units.  Update by workgroups that multiply as well: 64 and 128 channels, and
+# more of them than the device has units.
 PAIRS = [(3, 16, 64, 128), (5, 8, 192, 128), (2, 8, 256, 512), (5, 32, 64, 128), (70, 16, 128, 128), (70, 8, 512, 128), (36, 32, 128, 192), (70, 16, 256, 128),
-         (300, 8, 256, 128), (97, 32, 128, 128), (115, 32, 64, 128), (115, 32, 128, 128), (230, 16, 256, 128), (900, 8, 256, 128)]
+         (300, 8, 256, 128), (97, 32, 128, 128), (115, 32, 64, 128), (115, 32, 128, 128), (230, 16, 256, 128), (900, 8, 256, 128), (150, 16, 256, 256)]
 
 
 @pytest.mark.parametrize("case", PAIRS)
