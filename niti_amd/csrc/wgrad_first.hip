@@ -5,14 +5,19 @@
 // pixels - a gradient of 3 456 numbers, one MFMA column block wide.  Run through the general kernel pair (the input
 // padded to 16 channels, 256 workgroups of partial sums, a finishing launch) it takes two launches at their floor.
 //
-// One workgroup per image.  The 3 channel planes of the image sit in LDS with a border of zeros; the error map arrives
+// One workgroup per image or per half of one.  The 3 channel planes of the image sit in LDS with a border of zeros; the error map arrives
 // in pieces of 8 image rows ([pixel][K], buffer_load ... lds, two buffers).  A reduction step is one image row of 32
 // pixels: A = 32 output channels x 32 pixels by transposing LDS reads of the error tile, B = 32 columns (tap, channel) x
 // 32 pixels, where a column's 16 pixels per lane are 16 consecutive bytes of a plane row, shifted by the tap's
-// horizontal offset.  The workgroup adds its 32 K sums into one accumulation buffer with integer atomics (3 456 per
+// horizontal offset.  The workgroup adds its 32 K sums into an accumulation buffer with integer atomics (3 456 per
 // image instead of 37 K partial sums per workgroup); the workgroup that arrives last holds the whole gradient and
 // finishes alone - range, rounding, w = clip(w - g), the forward pass's filter copy - without any wait between
 // workgroups.
+//
+// What bounds it, 128 filters, replayed graphs, 4 / 80 / 128 / 256 images 10.5 / 13.4 / 15.3 / 19.8 us: the way of 128 KB an image to one
+// compute unit, about 10 ns of additions a workgroup, and the last one's trips to memory, which are one for all of its words (one after
+// the other they took 1.3 us more).  Two accumulation buffers that the workgroups share out halve the additions that wait for
+// each other (one 12.1 / 13.9 / 16.2 / 21.4; four 12.2 / 13.8 / 15.7 / 20.0); 64-bit additions of two sums are no faster.
 #include "common.h"
 #include "lds_asm.h"
 #include "requant_math.h"
@@ -24,7 +29,14 @@ constexpr int kWfPitch = 48;                          // bytes per plane row: ze
 constexpr int kWfPlane = 34 * kWfPitch;               // image rows -1 .. 32
 constexpr int kWfXBytes = 3 * kWfPlane + 64;
 constexpr int kWfCounter = 2;                         // sync word that counts the workgroups that are done
-constexpr int kWfCols = 32;                           // accumulation buffer: [K][32] words, column = tap * Cw + c
+constexpr int kWfCols = 32;                           // accumulation buffers: [K][32] words, column = tap * Cw + c
+constexpr int kWfCopies = 2;
+
+constexpr int wf_buffers(int K, int P) { return K <= 128 || 4 / P <= 2 ? 4 / P : 2; }
+constexpr size_t wf_lds(int K, int P) {   // (the wavefronts' sums are parked across the error tiles at the end: 32 KB)
+  const size_t tiles = static_cast<size_t>(wf_buffers(K, P)) * 256 * K;
+  return static_cast<size_t>(kWfXBytes) + (tiles > 32768 ? tiles : 32768);
+}
 
 struct WfArgs {
   const int8_t* act;   // [N][32][32][16], channels >= Cw are padding
@@ -34,7 +46,7 @@ struct WfArgs {
   int32_t* dw;         // optional int32 gradient [K][9][16]
   int8_t* wprep;       // optional kernel-ready forward filter copy (16-channel layout)
   uint32_t* sync;      // word 0 range out, word kWfCounter arrivals
-  int32_t* accum;      // [K][32] zeroed words
+  int32_t* accum;      // [kWfCopies][K][32] zeroed words
   int N, K, Cw;
   long long err_bytes;
   int roundtrip, target_bits, method, trunc, bw_mode;
@@ -54,8 +66,8 @@ __device__ inline void wf_sync() {
   asm volatile("" ::: "memory");
 }
 
-// KB = K / 32 blocks of output channels; the 8 wavefronts are KB blocks x (8 / KB) groups of image rows
-template <int KB>
+// KB = K / 32 blocks of output channels; the 8 wavefronts are KB blocks x (8 / KB) groups of image rows.  P workgroups share an image.
+template <int KB, int P>
 __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
   constexpr int K = KB * 32;
   constexpr int G = 8 / KB;              // row groups
@@ -63,9 +75,9 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
   constexpr int PP = K / 16;             // 16-byte pieces per pixel of the error tile
   constexpr int SWZ = PP >= 8 ? 7 : PP - 1;
   constexpr int PPI = 1024 / K;          // pixels per staging instruction
-  constexpr int NBUF = K <= 128 ? 4 : 2;                   // error tiles of 8 rows in LDS
-  constexpr int BUF = 256 * K;                             // the wavefronts' sums are parked across them at the end (32 KB)
-  static_assert(NBUF * BUF >= 32768, "room for the parked sums");
+  constexpr int PIECES = 4 / P;
+  constexpr int NBUF = wf_buffers(K, P);                   // error tiles of 8 rows in LDS
+  constexpr int BUF = 256 * K;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t* const planes = smem;
   int8_t* const ebuf = smem + kWfXBytes;
@@ -75,7 +87,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kb = wave % KB, pg = wave / KB;
-  const int n = blockIdx.x;
+  const int n = blockIdx.x / P, first = blockIdx.x % P * PIECES;   // image, first of its pieces
 
   // the image's pixels (the first dword of each holds the channels), requested ahead of the error tiles
   uint32_t xv[2];
@@ -104,7 +116,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
       const int q = wave + 8 * i;                         // instruction of this piece: pixels q * PPI ..
       const int pix = q * PPI + lane / PP;
       const int slot = lane % PP;
-      const int off = ((n * 1024 + piece8 * 256 + pix) * K) + ((slot ^ ((pix >> 1) & SWZ)) << 4);
+      const int off = ((n * 1024 + (first + piece8) * 256 + pix) * K) + ((slot ^ ((pix >> 1) & SWZ)) << 4);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rerr, NITI_LDS(ebuf + buf * BUF + q * 1024), 16, off, 0, 0, 0);
     }
   };
@@ -130,9 +142,9 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0;
   // all four pieces of the image are requested at once where they fit (one memory latency instead of four)
-  if (NBUF == 4) {
+  if (NBUF == PIECES) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) issue(q, q);
+    for (int q = 0; q < PIECES; ++q) issue(q, q);
   } else {
     issue(0, 0);
   }
@@ -147,12 +159,12 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
     for (int c = 0; c < 3; ++c)
       if (c < a.Cw) planes[c * kWfPlane + at] = static_cast<int8_t>((xv[h] >> (8 * c)) & 0xFFu);
   }
-  static_for<4>([&](auto piecec) {
+  static_for<PIECES>([&](auto piecec) {
     constexpr int piece8 = decltype(piecec)::value;
-    if (NBUF == 4) wf_wait_vmcnt<(3 - piece8) * KB>();     // this piece has landed (loads complete in order)
+    if (NBUF == PIECES) wf_wait_vmcnt<(PIECES - 1 - piece8) * KB>();     // this piece has landed (loads complete in order)
     else wf_wait_vmcnt<0>();
     wf_sync();                                             // ... for every wavefront, and the other buffer has been read
-    if (NBUF != 4 && piece8 + 1 < 4) issue(piece8 + 1, (piece8 + 1) & 1);
+    if (NBUF != PIECES && piece8 + 1 < PIECES) issue(piece8 + 1, (piece8 + 1) & 1);
     const unsigned ebase = lds0 + static_cast<unsigned>(kWfXBytes + (piece8 % NBUF) * BUF);
 #pragma unroll
     for (int i = 0; i < RW; ++i) {
@@ -160,7 +172,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
       const unsigned ea = ebase + static_cast<unsigned>(r * 32 * K);
       const v2i alo = lds_read_tr8<0>(ea + a_off[0]);
       const v2i ahi = lds_read_tr8<0>(ea + a_off[1]);
-      const unsigned ba = lds0 + b_off + static_cast<unsigned>((piece8 * 8 + r) * kWfPitch);
+      const unsigned ba = lds0 + b_off + static_cast<unsigned>(((first + piece8) * 8 + r) * kWfPitch);
       const v4i d = lds_read_b128(ba);
       int d4;
       asm volatile("ds_read_b32 %0, %1 offset:16" : "=v"(d4) : "v"(ba));
@@ -186,6 +198,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
     for (int e = 0; e < 16; ++e) park[(wave * 16 + e) * 64 + lane] = acc[e];
   }
   __syncthreads();
+  int32_t* const accum = a.accum + (blockIdx.x & (kWfCopies - 1)) * (K * kWfCols);
   if (pg == 0 && live) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -193,7 +206,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
 #pragma unroll
       for (int q = 1; q < G; ++q) s += park[((q * KB + kb) * 16 + e) * 64 + lane];
       const int k = kb * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
-      if (s != 0) __hip_atomic_fetch_add(a.accum + k * kWfCols + col, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (s != 0) __hip_atomic_fetch_add(accum + k * kWfCols + col, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // this lane's additions have been performed
@@ -209,18 +222,26 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
   int s[PER];
   uint32_t lmax = 0;
   const int total = K * ncols;
+  int word[PER];   // of the accumulation buffer
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int idx = i * 512 + tid;
-    int v = 0;
-    if (idx < total) {
-      const int k = idx / ncols, c = idx - k * ncols;
-      v = __hip_atomic_load(a.accum + k * kWfCols + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (a.roundtrip) v = f32_roundtrip(v);
-    }
-    s[i] = v;
-    const uint32_t u = uabs(v);
-    lmax = u > lmax ? u : lmax;
+    const int idx = min(i * 512 + tid, total - 1), k = idx / ncols;
+    word[i] = k * kWfCols + idx - k * ncols;
+    s[i] = 0;
+  }
+#pragma unroll
+  for (int q = 0; q < kWfCopies; ++q) {
+    int v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = __hip_atomic_load(a.accum + q * (K * kWfCols) + word[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) s[i] += v[i];
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    if (i * 512 + tid >= total) s[i] = 0;
+    if (a.roundtrip) s[i] = f32_roundtrip(s[i]);
+    lmax = max(lmax, uabs(s[i]));
   }
   lmax = wave_max_u32(lmax);
   if (lane == 0) wmax[wave] = lmax;
@@ -260,7 +281,7 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
       int v = 0;
       if (c < a.Cw) {
         const int k = kt / 9, t9 = kt - 9 * k;
-        v = __hip_atomic_load(a.accum + k * kWfCols + t9 * a.Cw + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int q = 0; q < kWfCopies; ++q) v += __hip_atomic_load(a.accum + q * (K * kWfCols) + k * kWfCols + t9 * a.Cw + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a.roundtrip) v = f32_roundtrip(v);
       }
       a.dw[idx] = v;
@@ -268,11 +289,10 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
   }
 }
 
-template <int KB>
+template <int KB, int P>
 int wf_launch(const WfArgs& a, hipStream_t stream) {
-  constexpr int K = KB * 32;
-  constexpr size_t lds = static_cast<size_t>(kWfXBytes) + static_cast<size_t>(K <= 128 ? 4 : 2) * 256 * K;
-  auto k = wgrad_first_kernel<KB>;
+  constexpr size_t lds = wf_lds(KB * 32, P);
+  auto k = wgrad_first_kernel<KB, P>;
   static bool attr_set_of[kDeviceSlots] = {};   // function attributes are per device
   bool& attr_set = attr_set_of[device_slot()];
   if (!attr_set) {
@@ -280,7 +300,7 @@ int wf_launch(const WfArgs& a, hipStream_t stream) {
       return fail(NITI_ERR_LAUNCH, "wgrad_first: cannot reserve %zu bytes of LDS", lds);
     attr_set = true;
   }
-  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(a.N)), dim3(512), lds, stream, a);
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(a.N * P)), dim3(512), lds, stream, a);
   return check_launch("wgrad_first");
 }
 
@@ -290,7 +310,7 @@ int wf_launch(const WfArgs& a, hipStream_t stream) {
 size_t wgrad_first_extra_words(int H, int C, int K) {
   if (H != 32 || C != 16) return 0;
   if (K != 32 && K != 64 && K != 128 && K != 256) return 0;
-  return static_cast<size_t>(K) * kWfCols;
+  return static_cast<size_t>(kWfCopies) * K * kWfCols;
 }
 
 bool wgrad_first_supported(int N, int H, int C, int K, int w_channels) {
@@ -323,10 +343,14 @@ int launch_wgrad_first_update(const int8_t* act, const int8_t* err, int8_t* w, i
   a.exp_a = rq.exp_a;
   a.exp_b = rq.exp_b;
   a.exp_out = rq.exp_out;
-  if (K == 32) return wf_launch<1>(a, stream);
-  if (K == 64) return wf_launch<2>(a, stream);
-  if (K == 128) return wf_launch<4>(a, stream);
-  return wf_launch<8>(a, stream);
+  // Half an image for a workgroup as long as that is a third of the device: the unit's share arrives sooner, but there are twice as many
+  // additions (128 filters, 4 / 32 / 48 / 80 images 10.5 / 11.2 / 11.8 / 14.3 us, 11.8 / 12.0 / 12.2 / 13.4 with whole ones; 256 filters, 4 / 32 / 64
+  // images 15.9 / 17.3 / 20.7, 18.5 / 18.2 / 19.5; 32 filters, 4 / 32 / 64 images 7.4 / 7.8 / 8.7, 7.6 / 7.8 / 8.2)
+  const bool halves = N <= compute_units() / 6;
+  if (K == 32) return halves ? wf_launch<1, 2>(a, stream) : wf_launch<1, 1>(a, stream);
+  if (K == 64) return halves ? wf_launch<2, 2>(a, stream) : wf_launch<2, 1>(a, stream);
+  if (K == 128) return halves ? wf_launch<4, 2>(a, stream) : wf_launch<4, 1>(a, stream);
+  return halves ? wf_launch<8, 2>(a, stream) : wf_launch<8, 1>(a, stream);
 }
 
 }  // namespace niti

@@ -390,6 +390,34 @@ def test_quantiser_entries_of_the_c_abi(dev):
     assert torch.equal(y, want) and torch.equal(e, exp) and torch.equal(copied, target)
 
 
+# batches on both sides of the line between workgroups of half an image and of a whole one, every number of filters and of channels
+@pytest.mark.parametrize("case", [(1, 32, 3), (42, 32, 1), (43, 64, 3), (42, 64, 2), (42, 128, 3), (43, 128, 3), (2, 256, 3), (43, 256, 1)])
+def test_first_layer_wgrad_by_images(dev, case):
+    """The first layer's weight gradient and update, sums of both signs beyond the float32 mantissa among them."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, K, Cw = case
+    base._say("first_layer_wgrad", case)
+    g = torch.Generator().manual_seed(N + K)
+    act, err, w = torch.zeros(N, 32, 32, 16, dtype=torch.int8), ri8(g, N, 32, 32, K), ri8(g, K, 3, 3, Cw)
+    act[..., :Cw] = ri8(g, N, 32, 32, Cw)
+    act[..., 0], err[..., ::2], err[..., 1::2] = 127, 127, -127
+    dw = co.conv_wgrad(act, err, 3, 3, 1, 1)
+    gref, sh_ref = po.grad_calc(dw, 5, "psto")
+    for want_dw in (False, True):
+        wd = w.to(dev)
+        wide = torch.zeros(K, 3, 3, 16, dtype=torch.int8, device=dev)
+        wide[..., :Cw] = wd
+        prepared = ops.conv_filter_prepare(wide, N, 32, 32, 1, 1)
+        g8, d, sh, sync = ops.conv2d_wgrad_update(act.to(dev), err.to(dev), wd, want_grad=True, want_dw=want_dw, prepared_filter=prepared)
+        assert int(sync.cpu()[0]) == po.absmax(dw) and int(sh.cpu()) == sh_ref
+        assert torch.equal(g8.cpu(), gref[..., :Cw]) and torch.equal(wd.cpu(), po.weight_update(w, gref[..., :Cw].contiguous()))
+        wide[..., :Cw] = wd
+        assert torch.equal(prepared, ops.conv_filter_prepare(wide, N, 32, 32, 1, 1))
+        assert not want_dw or torch.equal(d.cpu(), dw)
+
+
 # N, side, C, K of layers whose two gradients run as a pair of launches.  Update beside the data gradient: its tiles of 32, 64 and 128
 # channels on every map; one slice of partial sums and 67, three input-channel groups of 64, batches that end inside a tile; some
 # workgroups for the update fewer than the device has units.  Update by workgroups that multiply as well: 64 and 128 channels, and
