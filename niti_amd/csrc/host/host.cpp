@@ -19,7 +19,7 @@ PyObject* g_niti_error = nullptr;   // niti_amd._lib.NitiError
 // since the reset is taken: one fill for the words of a whole step, contained in a graph that captures the step.  One
 // arena per stream, so steps on different streams do not share words, and one per stream capture: its chunks come from
 // the memory of the graph being captured.
-constexpr long kChunkWords = 1L << 16;
+constexpr long kChunkWords = 1L << 17;
 constexpr size_t kMaxChunks = 8;    // a caller that never resets starts over behind this many
 constexpr size_t kMaxArenas = 16;   // streams remembered; the least recently used one is given back
 struct Arena {
