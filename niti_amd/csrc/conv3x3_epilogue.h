@@ -519,17 +519,16 @@ struct Turns : NothingAlong {
   __device__ bool early() const { return is_early; }
   __device__ void update(int shift, const int32_t*, const int32_t*) { final_shift = shift; }
 };
-// tile(args, at, along), in a kernel whose first argument is its HaloArgs and whose grid has at most as many workgroups as there are tiles (nx * ny)
-template <class F>
-__device__ __forceinline__ void tiles_in_turns(const int nx, const int ny, F tile) {
+// tile(args, at), with `along` (Turns), in a kernel whose first argument is its HaloArgs and whose grid has at most as many workgroups as there are tiles (nx * ny)
+template <class Along, class F>
+__device__ __forceinline__ void tiles_in_turns(const int nx, const int ny, Along& along, F tile) {
   using Args = const __attribute__((address_space(4))) HaloArgs;
   const int step = gridDim.x, own = blockIdx.x;
-  Turns along;
   const auto take = [&](int id) {
     const HaloPlace at{id % nx, id / nx, nx, ny};
     Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
-    tile(*(const HaloArgs*)args, at, along);
+    tile(*(const HaloArgs*)args, at);
   };
   // ids: own + n * step, .., own + step, own, then own + step, .. again
   const int last = own + (nx * ny - 1 - own) / step * step;

@@ -516,7 +516,8 @@ __global__ __launch_bounds__(512, 4) void conv3x3_halo_kernel(const HaloArgs a) 
 template <int Q, int BR, int NI, int KT, bool kWT, bool kSto>
 __global__ __launch_bounds__(512, 4) void conv3x3_halo_turns_kernel(const HaloArgs, const int nx, const int ny) {
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-  tiles_in_turns(nx, ny, [&](const HaloArgs& a, const HaloPlace at, Turns& along) { halo_tile<Q, BR, NI, KT, true, kWT, kSto>(a, at, smem, along); });
+  Turns along;
+  tiles_in_turns(nx, ny, along, [&](const HaloArgs& a, const HaloPlace at) { halo_tile<Q, BR, NI, KT, true, kWT, kSto>(a, at, smem, along); });
 }
 
 // ---- 2 x 2 maps -----------------------------------------------------------------------------------------

@@ -456,7 +456,8 @@ __global__ __launch_bounds__(512, 2 * PER_CU) void conv3x3_k64_kernel(const Halo
 template <int Q, int BR, int NI, int KT, bool kWT, bool kSto>
 __global__ __launch_bounds__(512, 4) void conv3x3_k64_turns_kernel(const HaloArgs, const int nx, const int ny) {
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-  tiles_in_turns(nx, ny, [&](const HaloArgs& a, const HaloPlace at, Turns& along) { k64_tile<Q, BR, NI, KT, 2, true, kWT, kSto>(a, at, smem, along); });
+  Turns along;
+  tiles_in_turns(nx, ny, along, [&](const HaloArgs& a, const HaloPlace at) { k64_tile<Q, BR, NI, KT, 2, true, kWT, kSto>(a, at, smem, along); });
 }
 
 template <int Q, int BR, int NI, int KT, int PER_CU, bool kFused, bool kWT, bool kSto>

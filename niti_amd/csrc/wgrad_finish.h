@@ -400,8 +400,8 @@ struct SumsAlong {
   int guessed;
   uint32_t wnew[kItems];
 
-  __device__ SumsAlong(const FinishArgs& args, const AlongWork& w, int block_, int8_t* lds_)
-      : a(args), work(w), block(block_), lds(lds_), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
+  __device__ SumsAlong(const FinishArgs& args, const AlongWork& w, int block_, int8_t* lds_, int thread = threadIdx.x)
+      : a(args), work(w), block(block_), lds(lds_), lane(thread & 63), wave(__builtin_amdgcn_readfirstlane(thread >> 6)) {}
 
   __device__ int* sums(int l, int e, int unit) const { return reinterpret_cast<int*>(lds + 64) + (l * 4 + e) * 64 + unit; }   // [chunk][output channel of the unit][unit]
   // 0 largest magnitude, 1 wavefronts that have folded theirs in, 2 range, 3 the data gradient's range, 4 predicted shift

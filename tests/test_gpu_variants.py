@@ -421,9 +421,10 @@ def test_first_layer_wgrad_by_images(dev, case):
 # N, side, C, K of layers whose two gradients run as a pair of launches.  Update beside the data gradient: its tiles of 32, 64 and 128
 # channels on every map; one slice of partial sums and 67, three input-channel groups of 64, batches that end inside a tile; some
 # workgroups for the update fewer than the device has units.  Update by workgroups that multiply as well: 64 and 128 channels, and
-# more of them than the device has units.
+# more of them than the device has units; by some that multiply several tiles.
 PAIRS = [(3, 16, 64, 128), (5, 8, 192, 128), (2, 8, 256, 512), (5, 32, 64, 128), (70, 16, 128, 128), (70, 8, 512, 128), (36, 32, 128, 192), (70, 16, 256, 128),
-         (300, 8, 256, 128), (97, 32, 128, 128), (115, 32, 64, 128), (115, 32, 128, 128), (230, 16, 256, 128), (900, 8, 256, 128), (150, 16, 256, 256)]
+         (300, 8, 256, 128), (97, 32, 128, 128), (115, 32, 64, 128), (115, 32, 128, 128), (230, 16, 256, 128), (900, 8, 256, 128), (150, 16, 256, 256),
+         (135, 32, 128, 128), (1030, 8, 192, 128)]
 
 
 @pytest.mark.parametrize("case", PAIRS)
@@ -492,7 +493,7 @@ def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
     assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
 
 
-@pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 128, 128)])
+@pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 128, 128), (135, 32, 128, 128)])
 def test_conv_backward_pair_gives_up(case):
     """Waits with a limit of zero: the launch ends and the device-wide word says so."""
     import os
