@@ -731,6 +731,10 @@ static bool backward_as_pair(const ConvShape& s) {
   if (e != nullptr) return e[0] != '0';
   const char* together = getenv("NITI_BACKWARD_TOGETHER");
   if (together != nullptr && together[0] != '0') return false;
+  // Smaller layers than any that the estimates give to the pair (64 to 512 channels on maps of 8 to 32: from 2880 pixels and 115e6 products of
+  // pixels and filter elements on): not worth the microsecond that asking takes, which bounds steps of small batches
+  const long long pixels = static_cast<long long>(s.N) * s.H * s.H;
+  if (s.C % 64 != 0 || s.K <= 64 || pixels < 2816 || pixels * s.C * s.K < 110000000LL) return false;
   double dgrad = 0.0;
   if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) == 0) return false;
   bool nine_tap = false;
@@ -741,8 +745,7 @@ static bool backward_as_pair(const ConvShape& s) {
 
 extern "C" size_t niti_conv2d_i8_backward_pair_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad) {
   if (N <= 0 || H <= 0 || C <= 0 || K <= 0 || R != 3 || S != 3 || pad != 1 || H != W || halo_off()) return 0;
-  const size_t words = conv_pair_words(N, H, C, K);
-  return words > 0 && backward_as_pair({N, H, W, C, K, R, S, 1, pad}) ? words : 0;
+  return backward_as_pair({N, H, W, C, K, R, S, 1, pad}) ? conv_pair_words(N, H, C, K) : 0;
 }
 
 extern "C" size_t niti_conv2d_i8_backward_pair_workspace(int N, int H, int W, int C, int K, int R, int S, int pad) {
