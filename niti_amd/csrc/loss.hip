@@ -172,8 +172,11 @@ constexpr long long kIgnoredTarget = -100;
 __global__ __launch_bounds__(1024) void batch_metrics_kernel(const int8_t* __restrict__ out, const int32_t* __restrict__ out_exp,
                                                              const int64_t* __restrict__ target, int n, int classes, double* sums) {
   __shared__ double red[5][16];
-  __shared__ int8_t stage[kMetricsStage];   // the logits of up to 1024 samples: each is looked at twice, one after the other
+  __shared__ __attribute__((aligned(16))) int8_t stage[kMetricsStage];   // the logits of up to 1024 samples: each is looked at twice, one after the other
+  // What bounds the kernel are its trips to memory one after the other: the exponent, the sums so far, the targets and the logits (as words
+  // where they start on one) are on their way together (128 / 256 samples 5.9 / 6.3 us; with the logits byte by byte and the sums at the end 6.6 / 7.6).
   const float scale = ldexpf(1.0f, *out_exp);
+  const double before = threadIdx.x < 3 ? sums[threadIdx.x] : 0.0;
   double loss = 0.0, hit1 = 0.0, hit5 = 0.0, counted = 0.0, outside = 0.0;
   const bool staged = classes <= kMetricsStage / 64;
   const int rows = staged && kMetricsStage / classes < 1024 ? kMetricsStage / classes : 1024;
@@ -183,7 +186,9 @@ __global__ __launch_bounds__(1024) void batch_metrics_kernel(const int8_t* __res
     const long long t = static_cast<int>(threadIdx.x) < here ? target[base + threadIdx.x] : kIgnoredTarget;
     if (staged) {
       __syncthreads();
-      for (int i = threadIdx.x; i < here * classes; i += 1024) stage[i] = src[i];
+      const int bytes = here * classes, words = reinterpret_cast<uintptr_t>(src) % 4 == 0 ? bytes / 4 : 0;
+      for (int i = threadIdx.x; i < words; i += 1024) reinterpret_cast<uint32_t*>(stage)[i] = reinterpret_cast<const uint32_t*>(src)[i];
+      for (int i = 4 * words + threadIdx.x; i < bytes; i += 1024) stage[i] = src[i];
       __syncthreads();
     }
     if (static_cast<int>(threadIdx.x) >= here) continue;
@@ -243,7 +248,7 @@ __global__ __launch_bounds__(1024) void batch_metrics_kernel(const int8_t* __res
     // the mean over the batch as a float32 value, times the batch size in double: the order of the tensor operations
     float mean = threadIdx.x == 0 ? static_cast<float>(s / valid) : static_cast<float>(s) * (100.0f / static_cast<float>(n));
     if (bad > 0.0) mean = __builtin_nanf("");
-    sums[threadIdx.x] += static_cast<double>(mean) * n;
+    sums[threadIdx.x] = before + static_cast<double>(mean) * n;
   }
 }
 }  // namespace
