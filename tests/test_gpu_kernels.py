@@ -110,7 +110,7 @@ FUSED_CASES = [(4, 8, 16, 16), (4, 8, 64, 128), (8, 8, 80, 144), (1, 16, 16, 48)
                (5, 2, 48, 16), (33, 2, 16, 80), (256, 2, 160, 96), (1, 2, 96, 32),
                # more than 512 tiles of 256 pixels x 64 channels: workgroups of 512 pixels
                (256, 32, 16, 64), (1024, 16, 32, 48), (144, 32, 48, 64),
-               # more workgroups than the device holds at once: two launches, the second one settling the shift
+               # more tiles than the device holds workgroups at once: several of them in turn
                (264, 16, 16, 272), (600, 32, 16, 48)]
 
 
@@ -206,7 +206,7 @@ def test_conv_fprop_requant(dev, case, method, div_mode):
 
 STO_CASES = [(4, 8, 16, 16), (8, 8, 80, 144), (3, 16, 192, 272), (2, 32, 16, 64), (8, 32, 128, 128), (16, 4, 64, 128),
              (256, 32, 16, 64),      # workgroups of 512 pixels
-             (264, 16, 16, 272)]     # two launches, the second one settling the shift
+             (264, 16, 16, 272)]     # several tiles for a workgroup, in turn
 
 
 @pytest.mark.parametrize("div_mode", ["floor", "trunc"])
@@ -642,7 +642,7 @@ def test_conv_requant_rejects_what_it_does_not_cover(dev):
     e = torch.zeros((3, 7, 9, 32), dtype=torch.int8, device=dev)
     with pytest.raises(NitiError):
         ops.conv2d_dgrad(e, torch.zeros((32, 3, 3, 16), dtype=torch.int8, device=dev), forward_filter=torch.zeros(64, dtype=torch.int8, device=dev))
-    # a launch that would not be resident at once runs as two launches that do not wait for each other
+    # tiles that would not be resident at once: a workgroup takes several in turn
     from oracle import niti_oracle as po
     N = 2048                                                          # 2048 tiles of 256 pixels
     assert ops.conv_requant_sync_words(N, 16, 16, 16, 16) > 0

@@ -114,8 +114,8 @@ def test_conv_layer_sto_runs_in_the_single_launch_kernels(tt):
 
 
 def test_conv_layer_on_a_grid_larger_than_the_device(tt):
-    """A layer whose convolutions have more workgroups than the device holds at once (136 images of 32 x 32, 80 -> 144
-    channels: 1088 and 544 tiles): forward and data gradient run as two launches that do not wait.  Two training
+    """A layer whose convolutions have more tiles than the device holds workgroups at once (136 images of 32 x 32, 80 -> 144
+    channels: 1088 and 544 tiles): in forward and data gradient workgroups take several tiles in turn.  Two training
     steps in a row, the second one predicting its shifts from the first."""
     from oracle import niti_model_oracle as mo
     dev = torch.device("cuda:0")

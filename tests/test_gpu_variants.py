@@ -67,7 +67,7 @@ def test_conv_slices_of_64(dev, case, tile, per_cu, monkeypatch):
     assert int(sync.cpu()[1]) == 0 and torch.equal(y8.cpu(), ref.clamp(min=0)) and int(sh.cpu()) == sh_ref
 
 
-# N, side, C, K: more workgroups of the same kernel than the device holds at once, two launches of which the second settles the shift
+# N, side, C, K: more tiles of the same kernel than the device holds workgroups at once, which take several of them in turn
 # (tiles of 128 channels, of 64 on small maps; the layers' data gradients where the forward pass has an odd number of 32-channel
 # slices): right, wrong and absurd predictions, StoShift, and nearly every tile stored again
 TWO_LAUNCHES = [(65, 32, 64, 144), (172, 16, 272, 64), (2052, 8, 64, 64)]
@@ -94,7 +94,7 @@ def test_conv_slices_of_64_unpooling_on_a_grid_larger_than_the_device(dev, case,
 
 @pytest.mark.parametrize("forward", [True, False])
 def test_conv_slices_of_64_stored_again(dev, forward, monkeypatch):
-    """One image with large values among images of tiny ones: the settling launch computes nearly every tile again, with the pooled
+    """One image with large values among images of tiny ones: nearly every tile that is stored before the range is known is computed again, with the pooled
     output, with the mask of a ReLU below and from both filter copies."""
     from niti_amd import ops
     from oracle import c_oracle as co
