@@ -74,7 +74,7 @@ int niti_bitwidth(uint32_t r, int bw_mode);
 
 /*
  * Grid-wide waits that gave up.  Every single-launch kernel with a tensor-wide range (niti_conv2d_i8_*_requant,
- * niti_conv2d_i8_wgrad_update, niti_fc_i8_*) flags a wait that ran into its time limit in word 1 of its own sync words
+ * niti_conv2d_i8_wgrad_update, niti_fc_i8_*) flags a wait that ran into its time limit in word 1 of the sync words its call was given
  * AND in one word per device inside the library, which stays set until cleared here - so a driver whose sync words are
  * zeroed again every step can look once per epoch, and before it writes a checkpoint.  Copies that word to *flag_out
  * (host memory) after everything queued on `stream` so far has run (the call blocks), and zeroes it if clear != 0.

@@ -128,12 +128,15 @@ inline size_t slot_words(int blocks) { return static_cast<size_t>((blocks + 15) 
 // Called by a whole wavefront: waits until all nb slots are filled and returns the largest value.  512 slots at a
 // time, eight per lane with the loads in flight together (one trip to memory per look); a lane reads a slot again
 // only while it is still empty, so the reads of the waiting workgroups die down as the slots fill.  Gives up after
-// spin_limit ticks of the 100 MHz clock: `code` is or-ed into *timed_out (the launch's own flag: 1 = a wait for the
-// tensor-wide range, 2 = the one-launch weight gradient's wait for the partial sums), *sticky (the device-wide word
+// spin_limit ticks of the 100 MHz clock: `code` is or-ed into *timed_out (word 1 of the sync words that the call was given,
+// whichever part of them the slots lie in), *sticky (the device-wide word
 // that niti_sync_timeouts reads, may be null) is set to 1 and the largest value seen so far is returned.  A limit of
 // zero gives up after the first look whatever it saw (tests of this path: every waiting wavefront then takes it).
+constexpr uint32_t kWaitRange = 1;    // for the tensor-wide range
+constexpr uint32_t kWaitPlanes = 2;   // the one-launch weight gradient's for the partial sums
+constexpr uint32_t kWaitUpdate = 4;   // those of a weight update in a call that computes the data gradient as well
 __device__ inline uint32_t wait_slots(uint32_t* slots, int nb, long long spin_limit, uint32_t* timed_out, uint32_t* sticky,
-                                      uint32_t code = 1u) {
+                                      uint32_t code = kWaitRange) {
   constexpr int kLook = 8;
   const int lane = threadIdx.x & 63;
   const long long t0 = wall_clock64();
@@ -258,7 +261,8 @@ int wgrad3x3_finish_blocks(int C, int K);
 int launch_wgrad_reduce(const int32_t* partial, long long slice_stride, int splits, int32_t* dw, int64_t n, bool roundtrip, uint32_t* absmax,
                         hipStream_t stream);
 int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
-                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream);
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream,
+                        uint32_t* data_gradient_sync = nullptr);   // of the call's data gradient, if sync are not the call's first words
 size_t wgrad3x3_sync_words(int blocks);
 int launch_wgrad3x3_update(const int8_t* act, const int8_t* err, int8_t* w, int w_channels, int N, int H, int C, int K,
                            bool roundtrip, uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep,

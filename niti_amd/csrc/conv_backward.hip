@@ -189,7 +189,7 @@ int launch_conv_backward(const ConvShape& s, const int8_t* err, const int8_t* ac
   RequantSpec behind = grad;
   behind.exp_a = rq.exp_out;
   return launch_wgrad_finish(static_cast<const int32_t*>(workspace), slice_of(s), p.slices, static_cast<long long>(s.K) * s.R * s.S * s.C, s.C, w, s.C, roundtrip,
-                             sync_w, behind, g8, nullptr, wprep, stream);
+                             sync_w, behind, g8, nullptr, wprep, stream, sync);
 }
 
 }  // namespace niti

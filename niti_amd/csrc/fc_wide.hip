@@ -637,7 +637,7 @@ __global__ __launch_bounds__(512) void fcw_backward_kernel(const FcwArgs d, cons
   }
   if (wave == 0) {
     const uint32_t r = wait_slots(d.sync + kSlot0, nd, d.spin_limit, &d.sync[1], d.sticky);
-    const uint32_t s = wait_slots(g.sync + kSlot0, nw, g.spin_limit, &g.sync[1], g.sticky);
+    const uint32_t s = wait_slots(g.sync + kSlot0, nw, g.spin_limit, &d.sync[1], g.sticky, kWaitUpdate);
     if (lane == 0) {
       words[16] = r != 0u ? r - 1u : 0u;
       words[17] = s != 0u ? s - 1u : 0u;

@@ -77,7 +77,8 @@ __device__ inline int grid_shift(const Args& a, uint32_t lmax, uint32_t* wmax, u
 
 // A weight update next to the data gradient `first` that reads the old weights, in one launch: the update's workgroups wait for
 // both ranges - a workgroup of the data gradient fills its slot when it has read its weights - and the gradient's exponent
-// builds on the error's that comes out of this launch.  share: two words.  meanwhile(): see grid_shift.
+// builds on the error's that comes out of this launch.  Waits that give up say so in the data gradient's words, the first of the
+// call's.  share: two words.  meanwhile(): see grid_shift.
 template <int NWAVES, class Args, class Meanwhile>
 __device__ inline int grid_shift_behind(const Args& a, const Args& first, int first_blocks, uint32_t lmax, uint32_t* wmax, uint32_t* share, int block,
                                         int blocks, Meanwhile meanwhile) {
@@ -92,8 +93,8 @@ __device__ inline int grid_shift_behind(const Args& a, const Args& first, int fi
   }
   meanwhile();
   if (wave == 0) {
-    const uint32_t f = wait_slots(first.sync + kSlot0, first_blocks, a.spin_limit, &a.sync[1], a.sticky);
-    const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &a.sync[1], a.sticky);
+    const uint32_t f = wait_slots(first.sync + kSlot0, first_blocks, a.spin_limit, &first.sync[1], a.sticky, kWaitUpdate);
+    const uint32_t g = wait_slots(a.sync + kSlot0, blocks, a.spin_limit, &first.sync[1], a.sticky, kWaitUpdate);
     if (lane == 0) {
       share[0] = g != 0u ? g - 1u : 0u;
       share[1] = f != 0u ? f - 1u : 0u;

@@ -639,7 +639,7 @@ __global__ __launch_bounds__(512, 1) void wgrad3x3_narrow_kernel(const WgradArgs
       __hip_atomic_store(slot_word(f.arrive, block), wide ? 2u : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (wave == 0) {
-      const uint32_t seen = wait_slots(f.arrive, nblocks, f.spin_limit, &f.sync[1], f.sticky, 2u);
+      const uint32_t seen = wait_slots(f.arrive, nblocks, f.spin_limit, f.flag, f.sticky, kWaitPlanes);
       if (lane == 0) wgm[8] = seen;
     }
     __syncthreads();
@@ -919,6 +919,8 @@ static FinishArgs finish_args(long long elements, int C, int8_t* w, int w_channe
   f.g8 = g8;
   f.dw = dw;
   f.sync = sync;
+  f.flag = sync + 1;
+  f.flag_code = kWaitRange;
   f.roundtrip = roundtrip ? 1 : 0;
   f.target_bits = rq.target_bits;
   f.method = rq.method;
@@ -959,9 +961,13 @@ static int launch_finish(FinishArgs f, const int32_t* partial, long long slice_s
 }
 
 int launch_wgrad_finish(const int32_t* partial, long long slice_stride, int splits, long long elements, int C, int8_t* w, int w_channels, bool roundtrip,
-                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream) {
+                        uint32_t* sync, const RequantSpec& rq, int8_t* g8, int32_t* dw, int8_t* wprep, hipStream_t stream, uint32_t* data_gradient_sync) {
   FinishArgs f = finish_args(elements, C, w, w_channels, roundtrip, sync, rq, g8, dw);
   f.wprep = wprep;
+  if (data_gradient_sync != nullptr) {
+    f.flag = data_gradient_sync + 1;
+    f.flag_code = kWaitUpdate;
+  }
   return launch_finish(f, partial, slice_stride, splits, stream);
 }
 

@@ -31,7 +31,9 @@ struct FinishArgs {
   int8_t* g8;          // optional rounded gradient, laid out like w
   int32_t* dw;         // optional int32 gradient [K][9][C]
   int8_t* wprep;       // optional: the halo convolution kernel's forward copy of the [K][9][C] filter, kept in step with w
-  uint32_t* sync;      // word 0: max |sum| (output); word 1: wait gave up; words kFinishSlot0..: slots, zero on entry
+  uint32_t* sync;      // word 0: max |sum| (output); words kFinishSlot0..: slots, zero on entry
+  uint32_t* flag;      // a wait gave up: word 1 of the call's sync words, into which flag_code is or-ed
+  uint32_t flag_code;
   int roundtrip, target_bits, method, trunc, bw_mode;
   int predict;         // *shift_out holds a predicted shift on entry
   long long spin_limit;
@@ -338,7 +340,7 @@ __device__ __forceinline__ void finish_columns(const FinishArgs& a, const int bl
     cols.update(applied, true);
   }
   if (cols.wave == 0) {
-    const uint32_t g = wait_slots(a.sync + kFinishSlot0, nblocks, a.spin_limit, &a.sync[1], a.sticky);
+    const uint32_t g = wait_slots(a.sync + kFinishSlot0, nblocks, a.spin_limit, a.flag, a.sticky, a.flag_code);
     if (cols.lane == 0) sh.gshare = g != 0u ? g - 1u : 0u;
   }
   __syncthreads();
@@ -595,7 +597,7 @@ struct SumsAlong {
   // A wavefront's wait for the gradient's range; a barrier follows.
   __device__ __forceinline__ void wait(int waiter) const {
     if (block < 0 || wave != waiter) return;
-    const uint32_t g = wait_slots(a.sync + kFinishSlot0, work.nblocks, a.spin_limit, &a.sync[1], a.sticky);
+    const uint32_t g = wait_slots(a.sync + kFinishSlot0, work.nblocks, a.spin_limit, a.flag, a.sticky, a.flag_code);
     if (lane == 0) words()[2] = g != 0u ? g - 1u : 0u;
   }
   // Behind it: the weights are right.
@@ -644,8 +646,8 @@ __device__ __forceinline__ void finish_beside(SumsAlong<kItems, kStream> along, 
   along.settle();
   if (along.wave == 0) {
     // one slot at first: the others are looked at when the data gradient is about to end
-    wait_slots(slot_word(first_slots, along.block % first_blocks), 1, along.a.spin_limit, &along.a.sync[1], along.a.sticky);
-    const uint32_t f = wait_slots(first_slots, first_blocks, along.a.spin_limit, &along.a.sync[1], along.a.sticky);
+    wait_slots(slot_word(first_slots, along.block % first_blocks), 1, along.a.spin_limit, along.a.flag, along.a.sticky, along.a.flag_code);
+    const uint32_t f = wait_slots(first_slots, first_blocks, along.a.spin_limit, along.a.flag, along.a.sticky, along.a.flag_code);
     if (along.lane == 0) along.words()[3] = f != 0u ? f - 1u : 0u;
   }
   __syncthreads();

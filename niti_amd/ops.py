@@ -243,7 +243,7 @@ def conv2d_backward(err, act, w, padding=1, f32_epilogue=False, err_bits=7, err_
                     bw_mode="int", relu_mask=None, pool_in=None, ties="first", err_rand=None, want_grad=False, exp_err=None, exp_w=None,
                     exp_act=None, prepared_filter=None, err_shift=None, grad_shift=None):
     """TiConv2d.backward (ti_torch.py:404-437), stride 1: err [N,P,Q,K], act [N,H,W,C], w [K,R,S,C] int8, w updated in place behind the
-    data gradient that reads it; both gradients in one launch where that is the faster way.  ``pool_in``: relu_mask is the output of
+    data gradient that reads it; both gradients in one call of the library where that is the faster way.  ``pool_in``: relu_mask is the output of
     a 2x2 / stride-2 max-pool on it, the error comes back at its size (element 2 of the result says whether it did).
     ``err_shift`` / ``grad_shift``: predicted shifts, overwritten with the actual ones.
     Returns (error, its exponent, unpooled?, int8 gradient or None, int32 gradient or None, gradient shift, gradient exponent, one call?)."""

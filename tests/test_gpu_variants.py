@@ -493,6 +493,55 @@ def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
     assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
 
 
+def test_updates_waits_are_flagged_in_the_words_of_the_call():
+    """Waits with a limit of zero in every call that updates weights beside a data gradient: the update's waits have a bit of their own
+    in the flag word that sync_arena.timed_out looks at, that of the slice the call was given."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import os
+import torch
+from niti_amd import _lib, ops
+dev = torch.device("cuda:0")
+ri = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device=dev)
+
+def flags(name, call, **env):
+    os.environ.update(env)
+    ops.sync_arena.reset(dev)
+    call()
+    torch.cuda.synchronize()
+    seen = 0
+    for t in _lib.host().arena_flags(0):
+        seen |= int(t.item())
+    print("FLAGS", name, seen, int(ops.sync_arena.timed_out(dev)), flush=True)
+    for k in env:
+        del os.environ[k]
+
+def conv(N, Q, C, K):
+    w = ri(K, 3, 3, C)
+    assert ops.conv2d_backward(ri(N, Q, Q, K), ri(N, Q, Q, C), w, prepared_filter=ops.conv_filter_prepare(w, N, Q, Q, 1, 1))[-1]
+
+def linear(M, O, F):
+    assert _lib.lib().niti_linear_i8_backward_sync_words(M, O, F) > 0
+    ops.linear_backward(ri(M, O), ri(M, F), ri(O, F))
+
+for case in ((3, 16, 64, 128), (115, 32, 128, 128), (135, 32, 128, 128)):
+    flags("pair%d" % case[0], lambda: conv(*case), NITI_BACKWARD_PAIR="1")
+for slices in "14":
+    flags("together" + slices, lambda: conv(3, 16, 64, 128), NITI_BACKWARD_PAIR="0", NITI_BACKWARD_TOGETHER="1", NITI_ANY_SLICES=slices)
+flags("linear_wide", lambda: linear(128, 1024, 8192))
+flags("linear_any", lambda: linear(100, 300, 1000))
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", code], cwd=root, env=dict(os.environ, NITI_SYNC_TIMEOUT_MS="0"), capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stderr[-2000:]
+    lines = [line.split()[1:] for line in out.stdout.splitlines() if line.startswith("FLAGS")]
+    assert len(lines) == 7
+    for name, seen, timed_out in lines:
+        assert int(seen) & 4 and timed_out == "1", out.stdout
+
+
 @pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 128, 128), (135, 32, 128, 128)])
 def test_conv_backward_pair_gives_up(case):
     """Waits with a limit of zero: the launch ends and the device-wide word says so."""
