@@ -486,7 +486,8 @@ int niti_conv2d_i8_backward(const int8_t* err, const int8_t* act, int8_t* w, int
 /*
  * The same as two launches, for 3x3 / pad 1 layers whose gradients are larger: the weight gradient's sums, then the data gradient
  * with the update beside it.  w_prepared must be given: the data gradient reads the copy, which then receives the updated weights.
- * err_method NITI_ROUND_NEAREST or NITI_ROUND_PSEUDO_STOCHASTIC.  NITI_CONV_SHIFT_HINT: *err_shift_out holds a predicted shift on entry.
+ * err_method NITI_ROUND_NEAREST or NITI_ROUND_PSEUDO_STOCHASTIC.  NITI_CONV_SHIFT_HINT: *err_shift_out and *grad_shift_out, where they
+ * are given, both hold a predicted shift on entry (set it only if they do).
  * workspace: niti_conv2d_i8_backward_pair_workspace bytes.  niti_conv2d_i8_backward_pair_sync_words returns 0 where the kernels do
  * not fit or another way is the faster (niti_conv2d_i8_backward; niti_conv2d_i8_dgrad_requant, niti_conv2d_i8_wgrad_update).
  */

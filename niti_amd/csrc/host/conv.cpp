@@ -527,9 +527,11 @@ bool both_gradients(const at::Tensor& act, const at::Tensor& err, const at::Tens
   r->y = empty8(shape, act);
   if (g.want_grad) u->g8 = empty8(w.sizes(), w);
   u->shift = g.shift != nullptr ? *g.shift : scalar32(w);
+  // the pair's flag speaks of both words, one of which is fresh where only the other tensor has a prediction
+  const bool hint = g.shift != nullptr && (!pair || f.shift != nullptr);
   const int rc = (pair ? niti_conv2d_i8_backward_pair : niti_conv2d_i8_backward)(
       ptr<int8_t>(err), ptr<int8_t>(act), ptr<int8_t>(w), ptr<int8_t>(r->y), d.N, d.H, d.W, d.C, d.K, d.R, d.S, f.pad,
-      g.flags | ((pair ? f.shift : g.shift) != nullptr ? NITI_CONV_SHIFT_HINT : 0u), f.r.bits, f.r.method, sto ? ptr<int32_t>(f.rand) : nullptr, ptr<int8_t>(f.mask),
+      g.flags | (hint ? NITI_CONV_SHIFT_HINT : 0u), f.r.bits, f.r.method, sto ? ptr<int32_t>(f.rand) : nullptr, ptr<int8_t>(f.mask),
       ptr<int8_t>(pool_in), f.ties, g.r.bits, g.r.method, f.r.div, f.r.bw, sync, words, g.want_grad ? ptr<int8_t>(u->g8) : nullptr, ptr<int8_t>(g.prepared),
       ptr<int32_t>(f.shift), ptr<int32_t>(u->shift), ptr<int32_t>(f.exp_a), ptr<int32_t>(f.exp_b), ptr<int32_t>(g.exp_b), ptr<int32_t>(r->e), ptr<int32_t>(e),
       bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(act));

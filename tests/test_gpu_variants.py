@@ -493,6 +493,30 @@ def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
     assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
 
 
+@pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 64, 128), (135, 32, 128, 128)])
+def test_conv_backward_pair_with_one_prediction(dev, case, monkeypatch):
+    """A predicted shift for one of the two gradients only, right and absurd: the other one is as without any."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    monkeypatch.setenv("NITI_BACKWARD_PAIR", "1")
+    base._say("conv_backward_pair, one prediction", case)
+    g = torch.Generator().manual_seed(7700 + N)
+    x, w, e = ri8(g, N, Q, Q, C), ri8(g, K, 3, 3, C), ri8(g, N, Q, Q, K, lo=-40, hi=40)
+    dref, dsh = po.err_calc(co.conv_dgrad(e, w, Q, Q, 1, 1))
+    gref, gsh = po.grad_calc(co.conv_wgrad(x, e, 3, 3, 1, 1), 5, "psto")
+    for which, right in (("err_shift", dsh), ("grad_shift", gsh)):
+        for guess in (right, right + 9, -3):
+            word = torch.tensor([guess], dtype=torch.int32, device=dev)
+            wd = w.to(dev)
+            prepared = ops.conv_filter_prepare(wd, N, Q, Q, 1, 1)
+            dx, _, _, g8, _, sh, _, one = ops.conv2d_backward(e.to(dev), x.to(dev), wd, want_grad=True, prepared_filter=prepared, **{which: word})
+            assert one and torch.equal(dx.cpu(), dref) and torch.equal(g8.cpu(), gref) and int(sh.cpu()) == gsh, (which, guess)
+            assert int(word.cpu()) == right and torch.equal(wd.cpu(), po.weight_update(w, gref)), (which, guess)
+    assert not ops.sync_arena.timed_out(dev) and not ops.sync_timeouts(dev)
+
+
 def test_updates_waits_are_flagged_in_the_words_of_the_call():
     """Waits with a limit of zero in every call that updates weights beside a data gradient: the update's waits have a bit of their own
     in the flag word that sync_arena.timed_out looks at, that of the slice the call was given."""
