@@ -809,6 +809,9 @@ __global__ __launch_bounds__(256) void halo_filter_prepare_kernel(const int8_t* 
   }
 }
 
+// Whether a launch may be pinned to the 32-channel tile, whose workgroups, of either kernel, fit twice on a unit and take no tiles in turn
+bool halo_narrow_fits(long long ptiles, int K, int H) { return H <= 16 && ptiles * ((K + 31) / 32) <= 2LL * compute_units(); }
+
 // Channel tile of a launch: 128 unless that leaves compute units idle to which narrower tiles would give something to do.
 int halo_ktile(long long pix, int K, int H, int C) {
   const long long ptiles = (pix + 255) / 256;
@@ -816,7 +819,7 @@ int halo_ktile(long long pix, int K, int H, int C) {
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
   if (forced == 128 || forced == 64) return forced;
-  if (forced == 32 && H <= 16 && ptiles * ((K + 31) / 32) <= 2LL * cus) return 32;
+  if (forced == 32 && halo_narrow_fits(ptiles, K, H)) return 32;
   // one 32-channel tile per compute unit at most: twice as many workgroups as with 64 channels, each half as long (24 images of
   // 16 x 16, 256 -> 256: 12.3 -> 9.3 us, 60 of 8 x 8, 512 -> 512: 18.8 -> 16.6).  Two of them on a unit are slower than one
   // 64-channel tile (50 images of the former 16.7 / 12.8 us, 120 of the latter 27.8 / 22.6).
@@ -863,7 +866,7 @@ int k64_ktile(long long pix, int K, int H, int C, bool fused) {
   const int cus = compute_units();
   const char* e = getenv("NITI_HALO_KT");  // tests and tuning runs pin the tile
   const int forced = e != nullptr ? atoi(e) : 0;
-  if (forced == 128 || forced == 64 || (forced == 32 && H <= 16 && ptiles * ((K + 31) / 32) <= 2LL * cus)) return forced;
+  if (forced == 128 || forced == 64 || (forced == 32 && halo_narrow_fits(ptiles, K, H))) return forced;
   if (H <= 16 && K > 32 && ptiles * ((K + 31) / 32) <= cus) return 32;
   const long long b64 = ptiles * ((K + 63) / 64);
   const long long b128 = ptiles * ((K + 127) / 128);
@@ -915,7 +918,7 @@ int launch_halo(const HaloArgs& a, hipStream_t stream) {
   static HaloLaunch state[2];
   const HaloKernel one{conv3x3_halo_kernel<Q, BR, NI, KT, kFused, kWT, kSto>, lds};
   if constexpr (kFused && KT != 32) return launch_halo_kernel<true>(one, HaloKernel{conv3x3_halo_turns_kernel<Q, BR, NI, KT, kWT, kSto>, lds}, state, G::PX, KT, Q, a, stream);
-  else return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: at most one workgroup on a unit)
+  else return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: see halo_narrow_fits)
 }
 
 inline int map2_blocks(int N, int K) { return ((N + 31) / 32) * ((K + 31) / 32); }

@@ -465,13 +465,14 @@ int launch_k64(const HaloArgs& a, hipStream_t stream) {
   using G = KGeom<Q, BR, NI, KT, PER_CU>;
   static_assert(8 * 32 * (32 * 4 + 16) <= G::TILE_BYTES, "int32 patches must stay clear of the reduction words");
   static_assert(8 * 32 * G::PT * (G::NWF * 32 + 16) <= G::TILE_BYTES, "int8 patches must stay clear of the reduction words");
+  static_assert(KT != 32 || 2 * G::LDS_BYTES <= 160 * 1024, "two 32-channel workgroups on a unit where a launch is pinned to them");
   static HaloLaunch state[2];
   const HaloKernel one{conv3x3_k64_kernel<Q, BR, NI, KT, PER_CU, kFused, kWT, kSto>, G::LDS_BYTES};
   if constexpr (kFused && KT != 32) {
     const HaloKernel several{conv3x3_k64_turns_kernel<Q, BR, NI, KT, kWT, kSto>, KGeom<Q, BR, NI, KT, 2>::LDS_BYTES};
     return launch_halo_kernel<true>(one, several, state, G::PX, KT, Q, a, stream);
   } else {
-    return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: at most one workgroup on a unit)
+    return launch_halo_kernel<kFused>(one, one, state, G::PX, KT, Q, a, stream);   // (32 channels: see halo_narrow_fits)
   }
 }
 

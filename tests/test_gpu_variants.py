@@ -219,6 +219,23 @@ def test_conv_slices_of_32_in_pairs(dev, case, tile, monkeypatch):
     base.test_conv_requant_sto(dev, case, "trunc")
 
 
+# more 32-channel tiles than the device has units, and more than it holds at once (the pin is left aside), by both kernels
+@pytest.mark.parametrize("k64", ["0", "1"])
+@pytest.mark.parametrize("case", [(100, 16, 64, 128), (150, 16, 64, 128)])
+def test_conv_pinned_to_the_narrowest_tile(dev, case, k64, monkeypatch):
+    from niti_amd import ops
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    monkeypatch.setenv("NITI_HALO_KT", "32")
+    monkeypatch.setenv("NITI_HALO_K64", k64)
+    monkeypatch.setenv("NITI_HALO_PER_CU", "1")
+    g = torch.Generator().manual_seed(N)
+    x, w = ri8(g, N, Q, Q, C).to(dev), ri8(g, K, 3, 3, C).to(dev)
+    ref, sh_ref = po.act_calc(ops.conv2d_fprop(x, w, 1, 1).cpu(), 0)
+    y, sh, sync = ops.conv2d_fprop_requant(x, w)
+    assert int(sync.cpu()[1]) == 0 and int(sh.cpu()) == sh_ref and torch.equal(y.cpu(), ref)
+
+
 @pytest.mark.parametrize("case", [(3, 2, 32, 48), (1, 16, 48, 32)])
 def test_conv_dgrad_i32_from_the_forward_copy(dev, case):
     from niti_amd import ops
