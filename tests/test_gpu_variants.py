@@ -510,6 +510,48 @@ def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
     assert torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
 
 
+# the update beside the data gradient, by workgroups that multiply one tile as well, by those that multiply several; filters that leave
+# part of the last 64 and of the last 128 empty
+@pytest.mark.parametrize("options", [dict(), dict(pool="all", div="trunc", bw="f32", want_grad=False), dict(pool="first", f32=False)])
+@pytest.mark.parametrize("case", [(12, 16, 128, 112), (40, 8, 192, 240), (115, 32, 64, 112), (115, 32, 128, 240), (135, 32, 128, 176)])
+def test_conv_backward_pair_options(dev, case, options, monkeypatch):
+    """Partial sums beyond 24 bits from some workgroups, whole sums beyond the float32 mantissa, through the float32 epilogue and not;
+    both divisions and bit widths, both tie rules of the pooling's backward pass, with and without the int8 gradient."""
+    from niti_amd import ops
+    from oracle import c_oracle as co
+    from oracle import niti_oracle as po
+    N, Q, C, K = case
+    f32, div, bw, pool, want_grad = (options.get(k, v) for k, v in (("f32", True), ("div", "floor"), ("bw", "int"), ("pool", None), ("want_grad", True)))
+    monkeypatch.setenv("NITI_BACKWARD_PAIR", "1")
+    monkeypatch.setenv("NITI_WGRAD_BLOCKS", "16")
+    base._say("conv_backward_pair options", case, options)
+    g = torch.Generator().manual_seed(5600 + N + K)
+    act, err, w = ri8(g, N, Q, Q, C, lo=-20, hi=20), ri8(g, N, Q, Q, K, lo=-20, hi=20), ri8(g, K, 3, 3, C)
+    act[:N // 2, :, :, :32], err[:N // 2], err[:N // 2, :, :, 1::2] = 127, 127, -127
+    dacc, wacc = co.conv_dgrad(err, w, Q, Q, 1, 1), co.conv_wgrad(act, err, 3, 3, 1, 1)
+    assert int(wacc.abs().max()) > 2 ** 24 and int(wacc[:, :, :, 32:].abs().max()) < 2 ** 23 and not torch.equal(wacc, po.f32_roundtrip(wacc))
+    if f32:
+        dacc, wacc = po.f32_roundtrip(dacc), po.f32_roundtrip(wacc)
+    (dref, dsh), (gref, gsh) = po.err_calc(dacc, div_mode=div, bw_mode=bw), po.grad_calc(wacc, 5, "psto", div_mode=div, bw_mode=bw)
+    kw = {}
+    if pool is not None:
+        whole = ri8(g, N, 2 * Q, 2 * Q, C, lo=-3, hi=4)
+        pooled = po.maxpool_fwd(whole)
+        dref = po.maxpool_bwd(pooled, dref * (pooled > 0), whole, ties=pool)
+        kw = dict(relu_mask=pooled.to(dev), pool_in=whole.to(dev), ties=pool)
+    wd = w.to(dev)
+    prepared = ops.conv_filter_prepare(wd, N, Q, Q, 1, 1)
+    scalar = lambda v: torch.tensor([v], dtype=torch.int32, device=dev)
+    dx, de, unpooled, g8, _, sh, ge, one = ops.conv2d_backward(
+        err.to(dev), act.to(dev), wd, f32_epilogue=f32, div_mode=div, bw_mode=bw, want_grad=want_grad, prepared_filter=prepared,
+        exp_err=scalar(-4), exp_w=scalar(-3), exp_act=scalar(2), **kw)
+    assert one and unpooled == (pool is not None) and (g8 is not None) == want_grad
+    assert torch.equal(dx.cpu(), dref) and int(de.cpu()) == dsh - 7
+    assert int(sh.cpu()) == gsh and int(ge.cpu()) == gsh + dsh - 7 + 2 and (g8 is None or torch.equal(g8.cpu(), gref))
+    assert torch.equal(wd.cpu(), po.weight_update(w, gref)) and torch.equal(prepared, ops.conv_filter_prepare(wd, N, Q, Q, 1, 1))
+    assert not ops.sync_arena.timed_out(dev) and not ops.sync_timeouts(dev)
+
+
 @pytest.mark.parametrize("case", [(3, 16, 64, 128), (115, 32, 64, 128), (135, 32, 128, 128)])
 def test_conv_backward_pair_with_one_prediction(dev, case, monkeypatch):
     """A predicted shift for one of the two gradients only, right and absurd: the other one is as without any."""
