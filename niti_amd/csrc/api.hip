@@ -731,16 +731,18 @@ static bool backward_as_pair(const ConvShape& s) {
   if (e != nullptr) return e[0] != '0';
   const char* together = getenv("NITI_BACKWARD_TOGETHER");
   if (together != nullptr && together[0] != '0') return false;
-  // Smaller layers than any that the estimates give to the pair (64 to 512 channels on maps of 8 to 32: from 2880 pixels and 115e6 products of
-  // pixels and filter elements on): not worth the microsecond that asking takes, which bounds steps of small batches
-  const long long pixels = static_cast<long long>(s.N) * s.H * s.H;
-  if (s.C % 64 != 0 || s.K <= 64 || pixels < 2816 || pixels * s.C * s.K < 110000000LL) return false;
-  double dgrad = 0.0;
-  if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) == 0) return false;
-  bool nine_tap = false;
-  const double us = conv_pair_us(s.N, s.H, s.C, s.K, dgrad);
-  const double other = backward_together(s) ? conv_backward_us(s) : dgrad + wgrad3x3_us(s.N, s.H, s.C, s.K, &nine_tap);
-  return us > 0.0 && us < 1.3 * other;
+  if (s.C % 64 != 0 || s.K <= 64) return false;
+  const auto faster = [&] {
+    double dgrad = 0.0;
+    if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) == 0) return false;
+    bool nine_tap = false;
+    const double us = conv_pair_us(s.N, s.H, s.C, s.K, dgrad);
+    const double other = backward_together(s) ? conv_backward_us(s) : dgrad + wgrad3x3_us(s.N, s.H, s.C, s.K, &nine_tap);
+    return us > 0.0 && us < 1.3 * other;
+  };
+  if (together != nullptr) return faster();
+  static thread_local KeptPerShape<bool> kept;   // (0.9 us to work out, asked for on every call)
+  return kept.get(s, 0, faster);
 }
 
 extern "C" size_t niti_conv2d_i8_backward_pair_sync_words(int N, int H, int W, int C, int K, int R, int S, int pad) {

@@ -188,12 +188,9 @@ bool fits_twice(int H, const PairPlan& p) {
   });
 }
 
-PairPlan pair_plan(int N, int H, int C, int K) {
+PairPlan plan_for(int N, int H, int C, int K, int slices) {
   PairPlan p{};
-  if (H != 8 && H != 16 && H != 32) return p;
   if (C % 64 != 0 || K <= 64 || (K + 31) / 32 % 2 != 0 || !conv3x3_halo_supported(N, H, H, K, C, 3, 3, 1, 1)) return p;   // the data gradient: K -> C
-  const int slices = wgrad3x3_planes_blocks(N, H, C, K) / (((K + 127) / 128) * (C / 32));
-  if (slices == 0) return p;
   const int cus = compute_units();
   const long long ptiles = (static_cast<long long>(N) * H * H + 255) / 256, units = static_cast<long long>(K) * 9 * C / 4;
   const auto blocks = [&](int ktile) { return ptiles * ((C + ktile - 1) / ktile); };
@@ -213,6 +210,14 @@ PairPlan pair_plan(int N, int H, int C, int K) {
   p.work = along_work(units, slices, p.way == kBeside ? std::min(room, cus) : static_cast<int>(std::min<long long>(std::max<long long>(least, cus), held)));
   p.blocks = held + (p.way == kBeside ? p.work.nblocks : 0);
   return fits_twice(H, p) ? p : PairPlan{};
+}
+
+PairPlan pair_plan(int N, int H, int C, int K) {
+  if ((H != 8 && H != 16 && H != 32) || C % 64 != 0 || K <= 0) return PairPlan{};
+  const int slices = wgrad3x3_planes_blocks(N, H, C, K) / (((K + 127) / 128) * (C / 32));
+  if (slices == 0) return PairPlan{};
+  static thread_local KeptPerShape<PairPlan> kept;
+  return kept.get({N, H, H, C, K, 3, 3, 1, 1}, slices, [&] { return plan_for(N, H, C, K, slices); });
 }
 
 size_t finish_words(const PairPlan& p) { return static_cast<size_t>(kFinishSlot0) + slot_words(p.work.nblocks); }

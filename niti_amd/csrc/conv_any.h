@@ -1,5 +1,7 @@
 // int8 convolutions of any map, filter and channel count (multiples of 16 where stated), read as stored (conv_any.hip).
 #pragma once
+#include <string.h>
+
 #include "common.h"
 
 namespace niti {
@@ -38,6 +40,33 @@ size_t conv_backward_words(const ConvShape& s);
 size_t conv_backward_workspace(const ConvShape& s);
 int launch_conv_backward(const ConvShape& s, const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx, bool roundtrip, uint32_t* sync, const RequantSpec& rq,
                          const RequantSpec& grad, int8_t* g8, int8_t* wprep, void* workspace, hipStream_t stream);
+
+// What a thread last worked out for a few layers, for answers that are asked for several times per call.  `extra`: whatever else the answer
+// hangs on.
+template <class T>
+class KeptPerShape {
+ public:
+  template <class F>
+  const T& get(const ConvShape& s, int extra, F make) {
+    const int key[kKey] = {s.N, s.H, s.W, s.C, s.K, s.R, s.S, s.stride, s.pad, device_slot() + 1, extra};   // (never all zero)
+    unsigned h = 0;
+    for (int v : key) h = h * 31u + static_cast<unsigned>(v);
+    Entry& e = kept_[(h ^ (h >> 8)) & 15u];
+    if (memcmp(e.key, key, sizeof(key)) != 0) {
+      e.value = make();
+      memcpy(e.key, key, sizeof(key));
+    }
+    return e.value;
+  }
+
+ private:
+  static constexpr int kKey = 11;
+  struct Entry {
+    int key[kKey];
+    T value;
+  };
+  Entry kept_[16] = {};
+};
 
 // Both gradients of a 3x3 layer on H x H maps as the weight gradient's sums and the data gradient with the update beside it
 // (conv3x3_k64_backward.hip); wprep is the filter copy that the data gradient reads.  words 0: not a shape of these kernels.

@@ -6,7 +6,6 @@
 // reduction over the pixels is not cut the weights are updated in the same launch, behind the last read of the old ones; where
 // it is cut the partial sums go to memory and the finishing launch of wgrad3x3.hip follows.
 #include <stdlib.h>
-#include <string.h>
 
 #include "conv_operands.h"
 
@@ -109,20 +108,8 @@ Plan estimate(const ConvShape& s) {
 Plan plan_of(const ConvShape& s) {
   if (!conv_any_shape(kConvDgrad, s) || !conv_any_shape(kConvWgrad, s)) return Plan{};
   if (getenv("NITI_ANY_TILE") != nullptr || getenv("NITI_ANY_SLICES") != nullptr) return estimate(s);
-  struct Entry {   // asked for several times per call: each thread keeps the last few
-    int key[7];
-    Plan plan;
-  };
-  static thread_local Entry kept[16] = {};
-  const int key[7] = {s.N, s.H * 65536 + s.W, s.C, s.K, s.R * 65536 + s.S, s.pad, device_slot()};
-  unsigned h = 0;
-  for (int v : key) h = h * 31u + static_cast<unsigned>(v);
-  Entry& e = kept[(h ^ (h >> 8)) & 15u];
-  if (memcmp(e.key, key, sizeof(key)) != 0) {
-    memcpy(e.key, key, sizeof(key));
-    e.plan = estimate(s);
-  }
-  return e.plan;
+  static thread_local KeptPerShape<Plan> kept;
+  return kept.get(s, 0, [&] { return estimate(s); });
 }
 
 size_t words_of(const ConvShape& s, const Plan& p) {
