@@ -705,7 +705,7 @@ def main():
     roofline_wgrad = {"bound": "mfma", "achieved": round(w_achieved, 2), "peak": INT8_MFMA_PEAK_TOPS, "unit": "TFLOP/s",
                       "frac": round(w_achieved / INT8_MFMA_PEAK_TOPS, 4), "traffic": wgrad_traffic,
                       "traffic_source": traffic_source,
-                      "kernel": "wgrad3x3_narrow_kernel<..., true> (weight gradient + gradient rounding + weight update + "
+                      "kernel": "wgrad3x3_narrow_kernel<..., kFinishHere, *> (weight gradient + gradient rounding + weight update + "
                                 "filter copy, one launch; layers 2-6)",
                       "launches": len(wsel), "avg_launch_us": round(w_ms * 1e3 / max(len(wsel), 1), 2),
                       "ops_per_launch_avg": w_ops / max(len(wsel), 1), "algorithmic_bytes_per_launch_avg": int(w_alg_bytes),

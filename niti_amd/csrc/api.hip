@@ -726,6 +726,9 @@ extern "C" size_t niti_conv2d_i8_backward_workspace(int N, int H, int W, int C, 
 // pair it was 7% and 44%, and with the pair only where the nine-tap kernel already was the weight gradient's 2.3% and 33%.  The factor
 // is what gives that: estimates of one launch are below what it takes in such graphs.  (80 images of 8 x 8, 256 -> 512 as
 // one launch 42.2 us, as a pair 33.7; 24 of 16 x 16, 128 -> 128 20.2 / 22.3; 128 of 32 x 32, 128 -> 128 one after the other 60.3 / 54.3.)
+// Through the front end, launch by launch, 300 other layers that the pair can take: taken for 167, slower there than the faster other way by more
+// than 2% for 4 (66 images of 8 x 8, 448 -> 448 43.4 / 41.0; 149 of 16 x 16, 192 -> 448 100.7 / 96.0; 202 of 8 x 8, 128 -> 128 22.9 / 21.9).  The larger
+// losses are layers left to the other ways: 51 images of 8 x 8, 384 -> 512 42.8 / 32.2; 13 of 16 x 16, 512 -> 384 41.5 / 31.6.
 static bool backward_as_pair(const ConvShape& s) {
   const char* e = getenv("NITI_BACKWARD_PAIR");   // 0 / 1 pins (tests)
   if (e != nullptr) return e[0] != '0';

@@ -504,8 +504,10 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace
 // One launch for all tiles without waiting and a second one that computed every tile again unless its shift was right took, with
 // predictions that fail (as about half of those inside a training step do) and with good ones (us): 256 images of 32 x 32, 128 -> 128
 // 67.4 / 44.1, so 57.5 / 42.1; data gradient 73.1 / 48.2, 62.6 / 46.6; 192 images 55.6 / 36.4, 47.6 / 35.2; 136 images 50.1 / 33.1, 43.2 / 33.5;
-// 256 of 16 x 16, 256 -> 512 121.1 / 64.4, 96.1 / 63.6; 256 of 32 x 32, 256 -> 256 (four tiles each) 242 / 125, 223 / 129.  What bounds it:
-// the first stage of each tile waits for its loads behind the stores of the one before.
+// 256 of 16 x 16, 256 -> 512 121.1 / 64.4, 96.1 / 63.6; 256 of 32 x 32, 256 -> 256 (four tiles each) 242 / 125, 223 / 129.  So with
+// four tiles each and predictions that hold it is the slower way by about 2% (through the layer 123.4 / 125.5), with two it is not (136 to 256 images,
+// 128 -> 128, 32.1 ... 41.7 / 31.0 ... 40.8).  It waits for its whole grid, which the two launches did not: it wants the device to itself, as
+// the launches that fit at once do.  What bounds it: the first stage of each tile waits for its loads behind the stores of the one before.
 struct Turns : NothingAlong {
   int final_shift = 0, settle_shift = -1;
   bool is_early = false;

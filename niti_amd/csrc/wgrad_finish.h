@@ -360,7 +360,7 @@ __device__ __forceinline__ void finish_columns(const FinishArgs& a, const int bl
 
 // ---- the same along with the data gradient ---------------------------------------------------------------------
 // (conv3x3_k64_backward.hip) `nblocks` workgroups of the data gradient's launch add the slices and update the weights: workgroups of
-// their own that share the units with those that multiply, or where these fill the device the later half of them, before their first stage.
+// their own that share the units with those that multiply, or where these fill the device the later ones of them (pair_plan), before their first stage.
 // Loads on a unit that multiplies wait behind its stages' (36 loads a wavefront in batches of eight took 10 to 15 us, where a trip to
 // memory is 2): a lane takes two units of a slice at a time (16 + 8 bytes) and has its loads - 9 to 12 at the usual 9216 unit slices
 // per workgroup - in flight together.  The sums are added up in LDS.  A half-wave works on a chunk of 64 units, the sixteen of them on

@@ -6,7 +6,7 @@
 // padded to 16 channels, 256 workgroups of partial sums, a finishing launch) it takes two launches at their floor.
 //
 // One workgroup per image or per half of one.  The 3 channel planes of the image sit in LDS with a border of zeros; the error map arrives
-// in pieces of 8 image rows ([pixel][K], buffer_load ... lds, two buffers).  A reduction step is one image row of 32
+// in pieces of 8 image rows ([pixel][K], buffer_load ... lds, all of them at once where they fit, else two buffers).  A reduction step is one image row of 32
 // pixels: A = 32 output channels x 32 pixels by transposing LDS reads of the error tile, B = 32 columns (tap, channel) x
 // 32 pixels, where a column's 16 pixels per lane are 16 consecutive bytes of a plane row, shifted by the tap's
 // horizontal offset.  The workgroup adds its 32 K sums into an accumulation buffer with integer atomics (3 456 per

@@ -397,8 +397,8 @@ def test_conv_requant_predicted_shift(dev, case):
 
 
 def test_conv_requant_oversubscribed_range_set_by_one_tile(dev):
-    """Two-launch form (more workgroups than fit at once): one image with large values among images of tiny ones makes
-    nearly every workgroup of the second launch compute and store its tile again; with the mask of a ReLU below and
+    """More tiles than workgroups fit at once: one image with large values among images of tiny ones makes
+    nearly every workgroup compute and store its earlier tiles again; with the mask of a ReLU below and
     with the pooled output."""
     from niti_amd import ops
     from oracle import c_oracle as co
@@ -1086,7 +1086,7 @@ def test_linear_any_width(dev, case, div_mode):
 
 
 @pytest.mark.parametrize("case", [(4, 8, 16, 32), (8, 16, 128, 64), (2, 16, 48, 80), (16, 4, 64, 128), (8, 32, 32, 16), (1024, 16, 48, 32),
-                                  (264, 16, 16, 272), (64, 2, 64, 128), (40, 2, 48, 80)])   # N, Q (pooled map), C, K; 512-pixel tiles, two-launch form, 2 x 2 maps
+                                  (264, 16, 16, 272), (64, 2, 64, 128), (40, 2, 48, 80)])   # N, Q (pooled map), C, K; 512-pixel tiles, several tiles in turn, 2 x 2 maps
 def test_conv_dgrad_requant_unpool(dev, case):
     """Data gradient + err_calc + ReLU mask + the backward pass of the 2x2 max-pool in front of the layer in one launch,
     against the oracle's three steps; windows with several equal maxima under both tie rules."""

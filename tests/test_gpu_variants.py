@@ -70,16 +70,16 @@ def test_conv_slices_of_64(dev, case, tile, per_cu, monkeypatch):
 # N, side, C, K: more tiles of the same kernel than the device holds workgroups at once, which take several of them in turn
 # (tiles of 128 channels, of 64 on small maps; the layers' data gradients where the forward pass has an odd number of 32-channel
 # slices): right, wrong and absurd predictions, StoShift, and nearly every tile stored again
-TWO_LAUNCHES = [(65, 32, 64, 144), (172, 16, 272, 64), (2052, 8, 64, 64)]
+MORE_THAN_FIT = [(65, 32, 64, 144), (172, 16, 272, 64), (2052, 8, 64, 64)]
 
 
-@pytest.mark.parametrize("case", TWO_LAUNCHES)
+@pytest.mark.parametrize("case", MORE_THAN_FIT)
 def test_conv_slices_of_64_on_a_grid_larger_than_the_device(dev, case, monkeypatch):
     monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_requant_predicted_shift(dev, case)
 
 
-@pytest.mark.parametrize("case", TWO_LAUNCHES)
+@pytest.mark.parametrize("case", MORE_THAN_FIT)
 def test_conv_slices_of_64_on_a_grid_larger_than_the_device_sto(dev, case, monkeypatch):
     monkeypatch.setenv("NITI_HALO_K64", "1")
     base.test_conv_requant_sto(dev, case, "floor")
