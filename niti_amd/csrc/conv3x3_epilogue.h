@@ -177,7 +177,7 @@ struct NothingAlong : OneTile {
   __device__ void begin() {}
   __device__ void publish() {}
   __device__ void guess() {}
-  __device__ void wait() const {}
+  __device__ void wait(const HaloArgs&) const {}
   __device__ void update(int, const int32_t*, const int32_t*) const {}
 };
 
@@ -477,7 +477,7 @@ __device__ __forceinline__ void halo_epilogue(const HaloArgs& a, const HaloPlace
         const uint32_t g = wait_slots(slots, nb, a.spin_limit, &a.sync[1], a.sticky);
         if (lane == 0) red[9] = g != 0u ? g - 1u : 0u;   // (not red[8]: no barrier has passed since the others read that)
       }
-      along.wait();
+      along.wait(a);
       __syncthreads();
       final_range = true;
       gmax = red[9];

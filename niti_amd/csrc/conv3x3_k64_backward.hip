@@ -92,7 +92,7 @@ struct SumsInTurns : Turns {
 #pragma unroll
     for (int i = 0; i < kWithinItems; ++i) wnew[i] = s.wnew[i];
   }
-  __device__ __forceinline__ void wait() { sums().wait(); }
+  __device__ __forceinline__ void wait(const HaloArgs& a) { sums().wait(a); }
   __device__ __forceinline__ void update(int shift, const int32_t* exp_a, const int32_t* exp_b) {
     Turns::update(shift, exp_a, exp_b);
     SumsWithin s = sums();
@@ -113,7 +113,7 @@ struct SumsInTurns : Turns {
     if (threadIdx.x == 0) __hip_atomic_store(slot_word(done, blockIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     SumsWithin s = sums();
     if (s.block < 0) return;
-    if (s.wave == 0) wait_slots(done, gridDim.x, args.a.spin_limit, args.f.flag, args.f.sticky, args.f.flag_code);
+    if (s.wave == 0) wait_slots(done, gridDim.x, args.a.spin_limit, &args.a.sync[1], args.a.sticky, kWaitUpdate);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kWithinItems; ++i) s.wnew[i] = wnew[i];
@@ -248,8 +248,6 @@ int launch_conv_pair(const int8_t* err, const int8_t* act, int8_t* w, int8_t* dx
   FinishArgs f;
   st = launch_wgrad3x3_planes(act, err, w, N, H, C, K, roundtrip, sync_w, sync_w + finish_words(p), grad, g8, wprep, workspace, &f, stream);
   if (st != NITI_OK) return st;
-  f.flag = sync + 1;
-  f.flag_code = kWaitUpdate;
   return with_geometry(H, p, [&](auto q, auto br, auto ni, auto kt, auto way) {
     constexpr int Q = decltype(q)::value, BR = decltype(br)::value, NI = decltype(ni)::value, KT = decltype(kt)::value;
     constexpr PairWay kWay = decltype(way)::value;
