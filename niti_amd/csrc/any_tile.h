@@ -417,11 +417,10 @@ __device__ __forceinline__ void any_tile(const AnyArgs& g, int32_t* const out, O
         for (int e = 0; e < 4; ++e) wn4[e] = clip127(static_cast<int>(static_cast<int8_t>((old >> (8 * e)) & 0xFFu)) - r[e]);
         const uint32_t fresh = pack4_i8(wn4[0], wn4[1], wn4[2], wn4[3]);
         __builtin_memcpy(g.w + at, &fresh, 4);
-        if (g.wprep != nullptr) {   // [64-filter group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
+        if (g.wprep != nullptr) {
           const int tap = g.by_channels.of(col), ch = col - tap * g.channels;
-          const int half = ((ch >> 4) & 1) ^ ((row >> 3) & 1);
-          const int to = (((((row >> 6) * ((g.channels + 31) >> 5) + (ch >> 5)) * 9 + tap) * 64 + (row & 63)) << 5) + half * 16 + (ch & 15);
-          *reinterpret_cast<uint32_t*>(g.wprep + to) = fresh;
+          const int block = ((row >> 6) * ((g.channels + 31) >> 5) + (ch >> 5)) * 9 + tap;
+          *reinterpret_cast<uint32_t*>(g.wprep + filter_copy_at(static_cast<uint32_t>(block), static_cast<uint32_t>(row) & 63u, static_cast<uint32_t>(ch))) = fresh;
         }
       }
       if (MODE == kRequant || g.out8 != nullptr) __builtin_memcpy(g.out8 + at, &packed, 4);

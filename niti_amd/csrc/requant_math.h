@@ -158,4 +158,10 @@ __device__ inline uint32_t max_i8x4(uint32_t a, uint32_t b) {
 // shift < 1: the reference converts int32 to int8 by keeping the low byte
 __device__ inline int wrap_to_i8(int x) { return static_cast<int>(static_cast<int8_t>(static_cast<uint32_t>(x) & 0xFFu)); }
 
+// Where the weight of channel c in row `row` of a block of the 3x3 kernels' filter copy lies (bytes):
+// [64-filter group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd; block: (group * slices + slice) * 9 + tap.
+__device__ __forceinline__ uint32_t filter_copy_at(uint32_t block, uint32_t row, uint32_t c) {
+  return ((block * 64u + row) << 5) + ((((c >> 4) ^ (row >> 3)) & 1u) << 4) + (c & 15u);
+}
+
 }  // namespace niti

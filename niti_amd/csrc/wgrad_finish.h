@@ -65,6 +65,34 @@ namespace {
 
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
+// Four sums of a gradient -> the rounded gradient; shift: a scalar
+__device__ __forceinline__ v4i rounded4(const v4i s, const int shift, const bool psto, const bool trunc) {
+  v4i r;
+  if (shift < 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = wrap_to_i8(s[e]);
+  } else if (psto) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(s[e], shift, trunc);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_NEAREST>(s[e], shift, trunc);
+  }
+  return r;
+}
+// Four weights and their rounded gradient, as words: the updated weights; gp: the gradient's word
+__device__ __forceinline__ uint32_t updated4(const uint32_t wold, const v4i r, uint32_t& gp) {
+  uint32_t wnew = 0;
+  gp = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int wo = static_cast<int>(static_cast<int8_t>((wold >> (8 * e)) & 0xFFu));
+    wnew |= (static_cast<uint32_t>(clip127(wo - r[e])) & 0xFFu) << (8 * e);
+    gp |= (static_cast<uint32_t>(r[e]) & 0xFFu) << (8 * e);
+  }
+  return wnew;
+}
+
 template <int NW>
 struct FinishShared {
   v4i part[2][NW][64];
@@ -258,15 +286,11 @@ struct FinishColumns {
     return bmax;
   }
 
-  // where the four weights of column `col` lie in the forward copy:
-  // [64-channel group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
+  // where the four weights of column `col` lie in the forward copy
   __device__ uint32_t* copy_word(long long col) const {
     const uint32_t e0 = static_cast<uint32_t>(col) * 4u, rt = div_c(e0), c0 = e0 - rt * C;
     const uint32_t k = rt / 9u, tap = rt - k * 9u;
-    const uint32_t row = k & 63u, cs = c0 >> 5;
-    const uint32_t half = ((c0 >> 4) & 1u) ^ ((row >> 3) & 1u);
-    const uint32_t dst = (((((k >> 6) * ((C + 31u) >> 5) + cs) * 9u + tap) * 64u + row) << 5) + half * 16u + (c0 & 15u);
-    return reinterpret_cast<uint32_t*>(a.wprep + dst);
+    return reinterpret_cast<uint32_t*>(a.wprep + filter_copy_at(((k >> 6) * ((C + 31u) >> 5) + (c0 >> 5)) * 9u + tap, k & 63u, c0));
   }
 
   // Every wavefront rounds its columns and updates their weights (element counts fit 31 bits: host check).  dw is stored the first time only.
@@ -286,25 +310,10 @@ struct FinishColumns {
       const v4i s = fin[j];
       if (first && a.dw != nullptr) reinterpret_cast<v4i*>(a.dw)[col] = s;
       uint32_t wnew = 0;   // the four updated weights (zero where the gradient column is channel padding)
-      int r[4];
-      if (shift < 1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = wrap_to_i8(s[e]);
-      } else if (psto) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(s[e], shift, trunc);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_NEAREST>(s[e], shift, trunc);
-      }
+      const v4i r = rounded4(s, shift, psto, trunc);
       if (same_layout) {
-        uint32_t gp = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int wo = static_cast<int>(static_cast<int8_t>((wold[j] >> (8 * e)) & 0xFFu));
-          wnew |= (static_cast<uint32_t>(clip127(wo - r[e])) & 0xFFu) << (8 * e);
-          gp |= (static_cast<uint32_t>(r[e]) & 0xFFu) << (8 * e);
-        }
+        uint32_t gp;
+        wnew = updated4(wold[j], r, gp);
         reinterpret_cast<uint32_t*>(a.w)[col] = wnew;
         if (a.g8 != nullptr) reinterpret_cast<uint32_t*>(a.g8)[col] = gp;
       } else {   // applied once only (the old weights are read here)
@@ -431,11 +440,11 @@ struct SumsAlong {
     const Place p = place(item_chunk(j));
     return (((p.k + (static_cast<uint32_t>(lane) >> 4)) * 9u + p.tap) * static_cast<uint32_t>(a.C) + p.c >> 2) + (static_cast<uint32_t>(lane) & 15u);
   }
-  __device__ uint32_t* item_copy(int j) const {   // in the forward copy: [64-channel group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
+  __device__ uint32_t* item_copy(int j) const {   // in the forward copy
     const Place p = place(item_chunk(j));
     const uint32_t q = static_cast<uint32_t>(lane) & 15u, row = (p.k & 63u) + (static_cast<uint32_t>(lane) >> 4);
     const uint32_t block64 = ((p.k >> 6) * (static_cast<uint32_t>(a.C) >> 5) + (p.c >> 5) + (q >> 3)) * 9u + p.tap;
-    return reinterpret_cast<uint32_t*>(a.wprep + ((block64 * 64u + row) << 5) + ((((q >> 2) ^ (row >> 3)) & 1u) << 4) + (q & 3u) * 4u);
+    return reinterpret_cast<uint32_t*>(a.wprep + filter_copy_at(block64, row, q * 4u));
   }
   __device__ v4i item(int j) const {
     v4i s = *reinterpret_cast<const v4i*>(sums(item_own(j), lane >> 4, 4 * (lane & 15))) - static_cast<int>(static_cast<uint32_t>(a.splits) * kPartialBias);   // modulo 2^32
@@ -563,25 +572,9 @@ struct SumsAlong {
       wnew[j] = 0;
       if (j * 8 >= work.own || !has_item(j)) continue;   // uniform
       const v4i s = item(j);
-      int r[4];
-      if (shift < 1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = wrap_to_i8(s[e]);
-      } else if (psto) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_PSEUDO_STOCHASTIC>(s[e], shift, trunc);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = round_one32<NITI_ROUND_NEAREST>(s[e], shift, trunc);
-      }
-      const uint32_t wold = *old_word(j);
-      uint32_t gp = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int wo = static_cast<int>(static_cast<int8_t>((wold >> (8 * e)) & 0xFFu));
-        wnew[j] |= (static_cast<uint32_t>(clip127(wo - r[e])) & 0xFFu) << (8 * e);
-        gp |= (static_cast<uint32_t>(r[e]) & 0xFFu) << (8 * e);
-      }
+      const v4i r = rounded4(s, shift, psto, trunc);
+      uint32_t gp;
+      wnew[j] = updated4(*old_word(j), r, gp);
       const uint32_t word = item_word(j);
       reinterpret_cast<uint32_t*>(a.w)[word] = wnew[j];
       if (a.g8 != nullptr) reinterpret_cast<uint32_t*>(a.g8)[word] = gp;

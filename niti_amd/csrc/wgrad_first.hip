@@ -269,10 +269,8 @@ __global__ __launch_bounds__(512) void wgrad_first_kernel(const WfArgs a) {
     a.w[idx] = static_cast<int8_t>(wn);
     if (a.g8 != nullptr) a.g8[idx] = static_cast<int8_t>(r);
     if (a.wprep != nullptr) {
-      // [64-channel group][one 32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
-      const uint32_t row = static_cast<uint32_t>(k) & 63u;
-      const uint32_t dst = ((((static_cast<uint32_t>(k) >> 6) * 9u + static_cast<uint32_t>(t9)) * 64u + row) << 5) + ((row >> 3) & 1u) * 16u + static_cast<uint32_t>(c);
-      a.wprep[dst] = static_cast<int8_t>(wn);
+      const uint32_t block = (static_cast<uint32_t>(k) >> 6) * 9u + static_cast<uint32_t>(t9);   // (one slice of channels, and of its first half)
+      a.wprep[filter_copy_at(block, static_cast<uint32_t>(k) & 63u, 0u) + static_cast<uint32_t>(c)] = static_cast<int8_t>(wn);
     }
   }
   if (a.dw != nullptr) {

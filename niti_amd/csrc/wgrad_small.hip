@@ -195,13 +195,9 @@ __global__ __launch_bounds__(576) void wgrad_small_kernel(const WsArgs a) {
     if (a.g8 != nullptr) *reinterpret_cast<uint32_t*>(a.g8 + at) = gp;
     if (a.dw != nullptr) *reinterpret_cast<v4i*>(a.dw + at) = v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
     if (a.wprep != nullptr) {
-      // [64-channel group][32-channel slice][tap][64 rows][32 bytes], 16-byte halves swapped where (row >> 3) is odd
       const uint32_t c = static_cast<uint32_t>(8 * g + 4 * lk);             // inside the slice
-      const uint32_t row = static_cast<uint32_t>(k) & 63u;
-      const uint32_t half = ((c >> 4) & 1u) ^ ((row >> 3) & 1u);
-      const uint32_t slices = static_cast<uint32_t>(a.C) >> 5;
-      const uint32_t dst = ((((static_cast<uint32_t>(k) >> 6) * slices + blockIdx.x) * 9u + static_cast<uint32_t>(tap)) * 64u + row) * 32u + half * 16u + (c & 15u);
-      *reinterpret_cast<uint32_t*>(a.wprep + dst) = wnew;
+      const uint32_t block = ((static_cast<uint32_t>(k) >> 6) * (static_cast<uint32_t>(a.C) >> 5) + blockIdx.x) * 9u + static_cast<uint32_t>(tap);
+      *reinterpret_cast<uint32_t*>(a.wprep + filter_copy_at(block, static_cast<uint32_t>(k) & 63u, c)) = wnew;
     }
   }
 }
