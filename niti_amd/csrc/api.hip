@@ -734,7 +734,11 @@ static bool backward_as_pair(const ConvShape& s) {
   if (e != nullptr) return e[0] != '0';
   const char* together = getenv("NITI_BACKWARD_TOGETHER");
   if (together != nullptr && together[0] != '0') return false;
-  if (s.C % 64 != 0 || s.K <= 64) return false;
+  // The estimates are those of 64 to 512 channels and give the pair to none smaller than this; to some of more channels they do, and those are the
+  // slower for it (60 layers of 576 to 2048 channels below the line: 1.024 of the other way on the geometric mean, 0.85 to 1.31: 37 images of 8 x 8,
+  // 1792 -> 128 39.2 / 32.9 us; 220 above it 0.897, 0.72 to 1.21)
+  const long long pixels = static_cast<long long>(s.N) * s.H * s.H;
+  if (s.C % 64 != 0 || s.K <= 64 || pixels < 2816 || pixels * s.C * s.K < 110000000LL) return false;
   const auto faster = [&] {
     double dgrad = 0.0;
     if (fused_blocks(s.N, s.H, s.W, s.C, s.K, s.R, s.S, 1, s.pad, 1, true, &dgrad) == 0) return false;

@@ -484,6 +484,17 @@ def test_conv_backward_pair(dev, case, monkeypatch):
     assert not ops.sync_arena.timed_out(dev)
 
 
+# few pixels or short sums of many channels, on either side of the lines
+@pytest.mark.parametrize("case,pair", [((37, 8, 1792, 128), False), ((43, 8, 768, 320), False), ((9, 16, 1728, 128), False), ((44, 8, 448, 576), True),
+                                       ((128, 8, 576, 128), True), ((128, 32, 128, 128), True)])
+def test_conv_backward_pair_rule(dev, case, pair, monkeypatch):
+    from niti_amd import _lib
+    N, Q, C, K = case
+    for name in ("NITI_BACKWARD_PAIR", "NITI_BACKWARD_TOGETHER"):
+        monkeypatch.delenv(name, raising=False)
+    assert (_lib.lib().niti_conv2d_i8_backward_pair_sync_words(N, Q, Q, C, K, 3, 3, 1) > 0) == pair
+
+
 @pytest.mark.parametrize("case", [(12, 16, 128, 128), (115, 32, 64, 128)])
 def test_conv_backward_pair_sums_beyond_2_23(dev, case, monkeypatch):
     """Partial sums that need more than 24 bits, from some workgroups of the weight gradient and not from others."""
