@@ -55,7 +55,7 @@ __global__ __launch_bounds__(512, 4) void conv3x3_k64_backward_kernel(const Halo
 // More tiles of the data gradient than the device holds workgroups: several in turn, and the sums in front of the first of them.  Both
 // launches against the data gradient's and the one-launch weight gradient's (us): 32 x 32, 128 -> 128 at 136 / 160 / 192 / 256 images
 // 76.6 -> 69.9, 75.4 -> 70.0, 81.7 -> 75.5, 98.6 -> 91.6; 256 images of 16 x 16, 384 -> 256 153.1 -> 146.7, 512 -> 128 87.6 -> 87.6.  What bounds it: the
-// tiles; the wait in front of the copy of the filter costs the 2 us of an exchange.  (15 registers spill, outside the loop.)
+// tiles; the wait in front of the copy of the filter costs the 2 us of an exchange.  (15 or 16 registers spill, outside the loop.)
 struct PairArgs {
   HaloArgs a;   // (first: tiles_in_turns)
   FinishArgs f;
